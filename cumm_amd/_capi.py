@@ -67,6 +67,7 @@ SYMBOLS = {
     "cumm_hip_sparse_conv": (C.c_int, [C.POINTER(ConvDesc), C.POINTER(SparseConvArgs), _VP]),
     "cumm_hip_sparse_conv_static_ws": (C.c_int, [C.POINTER(ConvDesc), C.POINTER(SparseConvArgs), _VP]),
     "cumm_hip_query_gemm_workspace": (C.c_int64, [C.POINTER(GemmDesc), C.c_int, C.c_int, C.c_int, C.c_int]),
+    "cumm_hip_query_gemm_optional_workspace": (C.c_int64, [C.POINTER(GemmDesc), C.c_int, C.c_int, C.c_int]),
     "cumm_hip_query_conv_workspace": (C.c_int64, [C.POINTER(ConvDesc), C.c_int, C.c_int, C.c_int, C.c_int, C.c_int]),
     "cumm_hip_query_wgrad_ordered_workspace": (C.c_int64, [C.c_int, C.c_int, C.c_int, C.c_int, C.c_int]),
     "cumm_hip_list_gemm_algos": (C.c_int, [C.POINTER(GemmDesc), C.c_int]),
@@ -115,6 +116,9 @@ SYMBOLS = {
                                  [C.c_int, _VP, _VP, _VP, _VP, _VP, _VP, C.c_size_t, _VP]),
     "cumm_hip_pair_lists_workspace": (C.c_size_t, [C.c_int, C.c_int]),
     "cumm_hip_pair_lists": (C.c_int, [_VP, C.c_int, C.c_int, _VP, _VP, _VP, _VP, C.c_size_t, _VP]),
+    "cumm_hip_wgrad_pairs_workspace": (C.c_int64, [_VP, C.c_int, C.c_int, C.c_int]),
+    "cumm_hip_wgrad_pairs": (C.c_int, [_VP, _VP, _VP, _VP, _VP, _VP, C.c_int, C.c_int64, C.c_int, C.c_int, C.c_int, C.c_int,
+                                       C.c_int, _VP, C.c_size_t, _VP]),
     "cumm_hip_finish_rows": (C.c_int, [_VP, C.c_int, _VP, _VP, C.c_int64, C.c_int, C.c_float, C.c_float, C.c_int,
                                        C.c_float, _VP]),
     "cumm_hip_relu_backward": (C.c_int, [_VP, _VP, _VP, C.c_size_t, C.c_int, _VP]),

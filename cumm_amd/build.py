@@ -38,6 +38,8 @@ def _units():
         units.append(("rowgemm_" + name, os.path.join(CSRC, "rowgemm_inst.hip"), defs))
         extra = ["-DCUMM_NO_WGRAD_ATOMIC"] if tag == "S8" else []   # no s8 backward pass
         units.append(("tilegemm_" + name, os.path.join(CSRC, "tilegemm_inst.hip"), defs + extra))
+        if tag != "S8":
+            units.append(("wgrad_pairs_" + name, os.path.join(CSRC, "wgrad_pairs_inst.hip"), defs))
         # the same kernels with four-byte outputs (s8 -> s32, f16 / bf16 -> f32)
         units.append(("rowgemm_wide_" + name, os.path.join(CSRC, "rowgemm_inst.hip"), defs + ["-DCUMM_WIDE=1"]))
         units.append(("tilegemm_wide_" + name, os.path.join(CSRC, "tilegemm_inst.hip"), defs + ["-DCUMM_WIDE=1"]))
@@ -188,7 +190,7 @@ def check_asm_hazards(force=False, jobs=None):
     """Compile every translation unit to device assembly (kept beside the objects, redone when a
     source is newer) and look for the hazard described above; returns the findings."""
     os.makedirs(OBJ, exist_ok=True)
-    units = [u for u in _units() if u[0].startswith(("rowgemm", "tilegemm"))]   # the units with asm loads
+    units = [u for u in _units() if u[0].startswith(("rowgemm", "tilegemm", "wgrad"))]   # the units with asm loads
     jobs = jobs or min(len(units), max(1, (os.cpu_count() or 2)), 8)
     with ThreadPoolExecutor(jobs) as pool:
         files = list(pool.map(lambda u: _device_asm(u, force), units))

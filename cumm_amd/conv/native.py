@@ -14,7 +14,6 @@ Forward and backward-input accumulate all offsets in an fp32 image (the f16 / bf
 and round once at the end (``cumm_hip_finish_rows``, with bias and activation): one rounding, as
 the mask-based kernels make, instead of one per offset.
 """
-import ctypes
 from typing import Optional
 
 import numpy as np
@@ -164,105 +163,72 @@ def backward_input(dout: tv.Tensor, weight: tv.Tensor, dinp: tv.Tensor, lists, *
     plan_backward_input(dout, weight, dinp, lists, stream=stream, acc=acc)()
 
 
-_NO_PAIR = {}
-
-
 class _WeightPlan:
-    """The per-offset launches of backward-weight, validated once (the first run goes through the
-    operator's prelude, a hundred microseconds of Python per offset) and then replayed straight at
-    the C entry point - on the same tensors, or on others of the same shapes and types whose
-    addresses ``rebind`` writes into the argument blocks."""
+    """Backward-weight of all kernel offsets in one call of the library (``cumm_hip_wgrad_pairs``),
+    validated once: run on the tensors it was made for, or through ``rebind`` on others of the same
+    shapes and types by address."""
 
-    def __init__(self, steps, dout, inp, dweight):
-        self.steps = steps
-        self._tensors = (dout, inp, dweight)     # kept alive with the blocks that point at them
-        self._blocks = None
+    def __init__(self, dout, inp, dweight, lists, stream):
+        self._tensors, self._lists, self._stream = (dout, inp, dweight), lists, stream
+        self._workspace = None
+        lib = _capi.lib()
+        kv, k_out, c_in = dweight.dim(1), dweight.dim(0), dweight.dim(2)
+        self._fn = lib.cumm_hip_wgrad_pairs
+        self._counts = np.ascontiguousarray(lists.counts, np.int32)
+        counts = self._counts.ctypes.data
+        self._pairs = (lists.pair_out.byte_pointer(), lists.pair_in.byte_pointer(), counts, kv, lists.pair_in.dim(1))
+        self._sizes = (dout.dim(0), inp.dim(0), k_out, c_in, dweight.dtype)
+        #: bytes of workspace that a run needs
+        self.workspace_bytes = int(lib.cumm_hip_wgrad_pairs_workspace(counts, kv, k_out, c_in))
+        if self.workspace_bytes < 0:
+            raise RuntimeError("at most 128 kernel offsets, channel counts multiples of 8")
 
     def __call__(self) -> None:
-        for p in self.steps:
-            GemmMainUnitTest.matmul2(p)
-        if self._blocks is None:
-            base = self._tensors[2].byte_pointer()
-            self._blocks = []
-            for p in self.steps:
-                prep = p.__dict__.get("_prepared")
-                if prep is None:
-                    raise RuntimeError("the operator call left no validated argument block")
-                args = prep[5]
-                self._blocks.append((prep[1], prep[2], prep[3], args, int(args.ptr_C) - base, int(args.ptr_D or 0) - base))
+        if self._tensors is None:
+            raise RuntimeError("the plan has released its tensors: use rebind")
+        dout, inp, dweight = self._tensors
+        self.rebind(dout.byte_pointer(), inp.byte_pointer(), dweight.byte_pointer(), self._stream)
 
-    def rebind(self, dout_ptr: int, inp_ptr: int, dweight_ptr: int, stream: int) -> None:
-        """Run on other tensors of the same shapes (device addresses), on ``stream``."""
-        if self._blocks is None:
-            raise RuntimeError("the plan has not run yet")
-        for fn, cdesc_ref, args_ref, args, c_delta, d_delta in self._blocks:
-            args.ptr_A, args.ptr_B = dout_ptr, inp_ptr
-            args.ptr_C = dweight_ptr + c_delta
-            if args.ptr_D:
-                args.ptr_D = dweight_ptr + d_delta
-            status = fn(cdesc_ref, args_ref, stream)
-            if status:
-                _capi.check(status)
+    def rebind(self, dout_ptr: int, inp_ptr: int, dweight_ptr: int, stream: int, workspace_ptr: Optional[int] = None) -> None:
+        """Run on other tensors of the same shapes (device addresses), on ``stream``.  Without a
+        workspace (``workspace_bytes`` bytes) the plan's own is used: one run at a time then."""
+        if workspace_ptr is None:
+            if self._workspace is None:
+                self._workspace = tv.empty([max(self.workspace_bytes, 16)], tv.uint8, 0)
+            workspace_ptr = self._workspace.byte_pointer()
+        status = self._fn(dweight_ptr, dout_ptr, inp_ptr, *self._pairs, *self._sizes, workspace_ptr, self.workspace_bytes, stream)
+        if status:
+            _capi.check(status)
 
     def release(self) -> None:
-        """Forget the tensors of the first run (a caller that goes on through ``rebind`` with its
-        own): the argument blocks hold addresses only, the pair lists belong to their owner."""
-        if self._blocks is None:
-            raise RuntimeError("the plan has not run yet")
-        self.steps, self._tensors = [], None
+        """Forget the tensors of the first run (a caller that goes on through ``rebind`` with its own);
+        the pair lists stay."""
+        self._tensors = None
 
     @property
     def launches(self) -> int:
-        return len(self._blocks) if self._blocks is not None else len(self.steps)
+        """Products the plan makes: one per kernel offset (they share the launches of one call)."""
+        return self._pairs[3]
 
 
 def plan_backward_weight(dout: tv.Tensor, inp: tv.Tensor, dweight: tv.Tensor, lists, *, stream: int = 0) -> _WeightPlan:
-    """Backward-weight as a reusable plan: one gathered GEMM per kernel offset into its slice of
-    ``dweight`` [K, kv, C] (an offset without pairs writes zeros)."""
-    kv = _check(inp, dweight, lists, dout.dim(0))
-    if dout.dim(1) != dweight.dim(0) or dout.dtype != inp.dtype:
+    """Backward-weight as a reusable plan: dweight[:, k, :] of every kernel offset (zeros for an
+    offset without pairs)."""
+    _check(inp, dweight, lists, dout.dim(0))
+    if dout.dim(1) != dweight.dim(0) or dout.dtype != inp.dtype or dweight.dim(2) != inp.dim(1):
         raise RuntimeError("error")
-    steps = []
-    for k in range(kv):
-        cnt = int(lists.counts[k])
-        p = GemmParams()
-        p.algo_desp = _find(inp.dtype, inp.dtype, ShuffleStrideType.ShuffleAB, 64, 64, True, False).copy()
-        p.a, p.b, p.c = dout, inp, dweight.select(1, k)
-        if cnt > 0:
-            p.a_inds = lists.pair_out.select(0, k).slice_first_axis(0, cnt)
-            p.b_inds = lists.pair_in.select(0, k).slice_first_axis(0, cnt)
-        else:
-            dev = inp.device
-            if dev not in _NO_PAIR:
-                _NO_PAIR[dev] = tv.from_numpy(np.full(32, -1, np.int32)).cuda()
-            p.a_inds = p.b_inds = _NO_PAIR[dev]
-        p.stream = stream
-        steps.append(p)
-    return _WeightPlan(steps, dout, inp, dweight)
+    for t in (dout, inp, dweight):
+        if t.device < 0 or not t.is_contiguous():
+            raise ValueError("operands must be contiguous device tensors")
+    return _WeightPlan(dout, inp, dweight, lists, stream)
 
 
 def backward_weight(dout: tv.Tensor, inp: tv.Tensor, dweight: tv.Tensor, lists, *, split_k_slices: int = 1,
                     stream: int = 0, workspace: Optional[tv.Tensor] = None) -> None:
-    """dweight[:, k, :] = dout[pair_out[k]].T @ inp[pair_in[k]] for every offset (zero without pairs)."""
-    kv = _check(inp, dweight, lists, dout.dim(0))
-    if dout.dim(1) != dweight.dim(0) or dout.dtype != inp.dtype:
-        raise RuntimeError("error")
-    for k in range(kv):
-        cnt = int(lists.counts[k])
-        p = GemmParams()
-        p.algo_desp = _find(inp.dtype, inp.dtype, ShuffleStrideType.ShuffleAB, 64, 64, True, False).copy()
-        p.a, p.b, p.c = dout, inp, dweight.select(1, k)
-        if cnt > 0:
-            p.a_inds = lists.pair_out.select(0, k).slice_first_axis(0, cnt)
-            p.b_inds = lists.pair_in.select(0, k).slice_first_axis(0, cnt)
-        else:
-            # an offset without pairs: one step of absent rows (index -1) writes the zeros
-            dev = inp.device
-            if dev not in _NO_PAIR:
-                _NO_PAIR[dev] = tv.from_numpy(np.full(32, -1, np.int32)).cuda()
-            p.a_inds = p.b_inds = _NO_PAIR[dev]
-        p.split_k_slices = split_k_slices if cnt >= 4096 * split_k_slices else 1
-        if workspace is not None:
-            p.workspace = workspace
-        p.stream = stream
-        GemmMainUnitTest.matmul2(p)
+    """dweight[:, k, :] = dout[pair_out[k]].T @ inp[pair_in[k]] for every offset (zero without pairs).
+    ``split_k_slices`` is what a caller of the per-offset products would pass; the pairs are spread
+    over the device in any case.  ``workspace`` is used when it is large enough."""
+    plan = plan_backward_weight(dout, inp, dweight, lists, stream=stream)
+    if workspace is not None and not workspace.empty() and workspace.nbytes >= plan.workspace_bytes:
+        plan._workspace = workspace
+    plan()      # (a workspace of its own goes away with the plan: freeing device memory waits for it)

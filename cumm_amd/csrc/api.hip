@@ -347,6 +347,74 @@ OrderedLayout ordered_layout(int N, int C, int K, int kv, int mask_width) {
   return l;
 }
 
+// ---- weight gradients over pair lists (wgrad_pairs.h)
+// The stream of 32-pair steps is cut into one share per compute unit and channel block (one workgroup
+// fits a unit): more shares only mean more partial tiles to add up.
+struct WgradPairsPlan {
+  int kblocks, cblocks, wgs, per_wg, most_slots;
+  int64_t steps;
+  size_t bytes;        // of slots
+};
+int compute_units() {
+  static std::atomic<int> known[kMaxDevices];
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 256;
+  if ((cus = known[dev].load()) > 0) return cus;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) {
+    (void)hipGetLastError();
+    return 256;
+  }
+  known[dev].store(cus);
+  return cus;
+}
+WgradPairsPlan wgrad_pairs_plan(const int32_t *counts, int lists, int K, int C, int32_t *step0) {
+  WgradPairsPlan l;
+  l.kblocks = (K + 63) / 64; l.cblocks = (C + 63) / 64;
+  const int combos = l.kblocks * l.cblocks;
+  l.steps = 0;
+  for (int r = 0; r < lists; ++r) l.steps += ((int64_t)counts[r] + 31) / 32;
+  int shares = compute_units() / combos;
+  if (shares < 1) shares = 1;
+  // (a step for each of the four waves at least, and as many for each)
+  const int64_t per = (l.steps + shares - 1) / shares;
+  l.per_wg = (int)(per < 4 ? 4 : (per + 3) / 4 * 4);
+  l.wgs = (int)((l.steps + l.per_wg - 1) / l.per_wg);
+  l.bytes = (size_t)(l.wgs + lists) * combos * kWgradPairsSlotFloats * sizeof(float);
+  l.most_slots = 0;
+  int64_t at = 0;
+  for (int r = 0; r < lists; ++r) {
+    if (step0) step0[r] = (int32_t)at;
+    const int64_t end = at + ((int64_t)counts[r] + 31) / 32;
+    const int slots = end > at ? (int)((end - 1) / l.per_wg - at / l.per_wg + 1) : 0;
+    if (slots > l.most_slots) l.most_slots = slots;
+    at = end;
+  }
+  if (step0) step0[lists] = (int32_t)at;
+  return l;
+}
+
+hipError_t run_wgrad_pairs(WgradPairsParams *w, WgradPairsFinalizeParams *f, const WgradPairsPlan &l, int lists, int K, int C, int dt,
+                           bool wide, void *workspace, hipStream_t stream) {
+  w->slots = reinterpret_cast<float *>(workspace);
+  w->K = f->K = K; w->C = f->C = C; w->lists = f->lists = lists;
+  w->kblocks = f->kblocks = l.kblocks; w->cblocks = f->cblocks = l.cblocks;
+  w->wgs = l.wgs; w->per_wg = f->per_wg = l.per_wg;
+  f->slots = w->slots;
+  std::memcpy(f->step0, w->step0, sizeof(int32_t) * (lists + 1));
+  return dt == CUMM_HIP_F16 ? launch_wgrad_pairs_f16(*w, *f, wide, l.most_slots, stream)
+                            : launch_wgrad_pairs_bf16(*w, *f, wide, l.most_slots, stream);
+}
+
+// ShuffleAB products of two-byte operands with one slice whose pairs are many against their output
+// take the pair-list kernel: from kWgradPairsMin pairs on (its two launches take 8.0 us for 256 pairs of
+// 64 x 64 channels, the tiled kernel's one 9.4 us; for 192 pairs that one takes 7.6 us) and while the
+// output is not itself enough tiles to fill the device.
+constexpr int kWgradPairsMin = 256;
+bool wgrad_pairs_serves(const CummHipGemmDesc &d, int m, int n, int k) {
+  return d.shuffle_type == CUMM_HIP_SHUFFLE_AB && is_float16_like(d.dtype_a) && k >= kWgradPairsMin && m % 8 == 0 && n % 8 == 0 &&
+         (int64_t)((m + 63) / 64) * ((n + 63) / 64) <= 256;
+}
+
 }  // namespace
 
 extern "C" {
@@ -366,6 +434,13 @@ int64_t cumm_hip_query_gemm_workspace(const CummHipGemmDesc *desc, int m, int n,
   if (desc->split_k_serial) return (int64_t)sizeof(int32_t) * tiles_m * tiles_n;
   if (desc->split_k_parallel) return (int64_t)4 * m * n * split_k_slices;   // (accumulators are 4 bytes: f32 or s32)
   return -1;
+}
+
+int64_t cumm_hip_query_gemm_optional_workspace(const CummHipGemmDesc *desc, int m, int n, int k) {
+  if (!desc || m < 0 || n < 0 || k < 0) return -1;
+  if (gemm_family(*desc) == 0 || !wgrad_pairs_serves(*desc, m, n, k)) return 0;
+  const int32_t count = k;
+  return (int64_t)wgrad_pairs_plan(&count, 1, m, n, nullptr).bytes;
 }
 
 int64_t cumm_hip_query_conv_workspace(const CummHipConvDesc *desc, int m, int n, int k, int split_k_slices,
@@ -604,6 +679,26 @@ int cumm_hip_gemm(const CummHipGemmDesc *desc, const CummHipGemmArgs *a, void *s
     yk = false; xk = false;
     p.y_gather = a->indiceA; p.x_gather = a->indiceBorC;
     p.rows_y = a->rows_A; p.rows_x = a->rows_B;
+    uint32_t a_bytes = 0, b_bytes = 0;
+    if (a->split_k_slices == 1 && a->workspace && a->rows_A > 0 && a->rows_B > 0 && wgrad_pairs_serves(d, m, n, a->k) &&
+        extent32(a->rows_A, lda, m, 2, &a_bytes) && extent32(a->rows_B, ldb, n, 2, &b_bytes) && (int64_t)a->k * 4 < (int64_t)1 << 31) {
+      WgradPairsParams w;
+      std::memset(&w, 0, sizeof(w));
+      const int32_t count = a->k;
+      const WgradPairsPlan l = wgrad_pairs_plan(&count, 1, m, n, w.step0);
+      if (a->workspace_bytes >= l.bytes && aligned16(a->workspace)) {
+        w.dout = A; w.inp = B; w.pair_out = a->indiceA; w.pair_in = a->indiceBorC;
+        w.ldy = lda; w.ldx = ldb; w.rows_y = a->rows_A; w.rows_x = a->rows_B;
+        WgradPairsFinalizeParams f;
+        std::memset(&f, 0, sizeof(f));
+        f.dw = a->ptr_C; f.src = ptr_D; f.ldw = a->stride_C; f.lds = ldd;
+        f.alpha = a->alpha; f.beta = a->beta; f.act_alpha = a->act_alpha; f.act = a->act_type;
+        w.count[0] = count;
+        const hipError_t e = run_wgrad_pairs(&w, &f, l, 1, m, n, dt, wide, a->workspace, stream);
+        if (e == hipSuccess) return CUMM_HIP_OK;
+        if (e != hipErrorNotSupported) return hip_fail(e, "pair-list weight gradient launch");
+      }
+    }
   } else {
     yk = !ta;  // A stored [m, k]
     xk = tb;   // B stored [n, k]
@@ -1351,6 +1446,55 @@ int cumm_hip_pair_lists(const int32_t *indices, int kv, int n, int32_t *pair_in,
   p.kv = kv; p.n = n; p.chunks = (n + kPairListChunk - 1) / kPairListChunk;
   hipError_t e = launch_pair_lists(p, reinterpret_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "pair list launch");
+  return CUMM_HIP_OK;
+}
+
+// ---- weight gradients of the per-offset convolution, all offsets in one launch
+static bool wgrad_pairs_args(const int32_t *counts, int lists, int K, int C) {
+  if (!counts || lists < 1 || lists > kWgradPairsMaxLists || K <= 0 || C <= 0 || K % 8 || C % 8) return false;
+  int64_t steps = 0;
+  for (int r = 0; r < lists; ++r) {
+    if (counts[r] < 0) return false;
+    steps += ((int64_t)counts[r] + 31) / 32;
+  }
+  return steps < (int64_t)1 << 30 && (int64_t)((K + 63) / 64) * ((C + 63) / 64) < 4096;
+}
+int64_t cumm_hip_wgrad_pairs_workspace(const int32_t *counts, int lists, int K, int C) {
+  return wgrad_pairs_args(counts, lists, K, C) ? (int64_t)wgrad_pairs_plan(counts, lists, K, C, nullptr).bytes : -1;
+}
+
+int cumm_hip_wgrad_pairs(void *dw, const void *dout, const void *inp, const int32_t *pair_out, const int32_t *pair_in,
+                         const int32_t *counts, int lists, int64_t list_stride, int rows_out, int rows_in, int K, int C,
+                         int dtype, void *workspace, size_t workspace_bytes, void *stream) {
+  if (!is_float16_like(dtype)) return fail(CUMM_HIP_EINVAL, "dtype must be f16 or bf16");
+  if (!wgrad_pairs_args(counts, lists, K, C) || rows_out < 0 || rows_in < 0)
+    return fail(CUMM_HIP_EINVAL, "1 to %d pair lists with counts on the host, channels multiples of 8", kWgradPairsMaxLists);
+  WgradPairsParams w;
+  WgradPairsFinalizeParams f;
+  std::memset(&w, 0, sizeof(w));
+  std::memset(&f, 0, sizeof(f));
+  const WgradPairsPlan l = wgrad_pairs_plan(counts, lists, K, C, w.step0);
+  uint32_t y_bytes = 0, x_bytes = 0;
+  if (!dw || !aligned16(dw)) return fail(CUMM_HIP_EINVAL, "dw must be 16-byte aligned and not empty");
+  if (l.steps > 0) {
+    if (!dout || !inp || !pair_out || !pair_in || !aligned16(dout) || !aligned16(inp))
+      return fail(CUMM_HIP_EINVAL, "dout, inp (16-byte aligned) and the pair lists must not be empty");
+    for (int r = 0; r < lists; ++r)
+      if (counts[r] > list_stride && lists > 1) return fail(CUMM_HIP_EINVAL, "a list is longer than list_stride");
+    if (rows_out < 1 || rows_in < 1) return fail(CUMM_HIP_EINVAL, "pairs without rows");
+    if (!extent32(rows_out, K, K, 2, &y_bytes) || !extent32(rows_in, C, C, 2, &x_bytes))
+      return fail(CUMM_HIP_ERUNTIME, "your data exceed int32 range.");
+    if (!workspace || workspace_bytes < l.bytes) return fail(CUMM_HIP_ERUNTIME, "workspace at least %zu bytes.", l.bytes);
+    if (!aligned16(workspace)) return fail(CUMM_HIP_EINVAL, "workspace must be 16-byte aligned");
+  }
+  w.dout = dout; w.inp = inp; w.pair_out = pair_out; w.pair_in = pair_in;
+  w.ldy = K; w.ldx = C; w.list_stride = list_stride; w.rows_y = rows_out; w.rows_x = rows_in;
+  std::memcpy(w.count, counts, sizeof(int32_t) * lists);
+  f.dw = dw; f.src = dw; f.ldw = f.lds = (int64_t)lists * C; f.ldr = C; f.alpha = 1.0f;
+  const hipError_t e = run_wgrad_pairs(&w, &f, l, lists, K, C, dtype, false, workspace, reinterpret_cast<hipStream_t>(stream));
+  if (e == hipErrorNotSupported)
+    return fail(CUMM_HIP_ERUNTIME, "the pair-list kernel of this build uses scratch memory, which its hand-counted waits do not allow");
+  if (e != hipSuccess) return hip_fail(e, "pair-list weight gradient launch");
   return CUMM_HIP_OK;
 }
 

@@ -4,6 +4,7 @@
 #include "rowgemm.h"
 #include "tilegemm.h"
 #include "wgrad_atomic.h"
+#include "wgrad_pairs.h"
 
 namespace cummhip {
 
@@ -58,6 +59,11 @@ int wgrad_ordered_resident_f16(bool wide);
 int wgrad_ordered_resident_bf16(bool wide);
 hipError_t launch_wgrad_ordered_f16(const WgradParams &p, const WgradPrepareParams &pre, const WgradOrderedParams &f, bool wide, int wgs, hipStream_t s);
 hipError_t launch_wgrad_ordered_bf16(const WgradParams &p, const WgradPrepareParams &pre, const WgradOrderedParams &f, bool wide, int wgs, hipStream_t s);
+
+// weight gradients over explicit pair lists (f16 / bf16 operands; wide: f32 result); most_slots = slots
+// of the list with most of them
+hipError_t launch_wgrad_pairs_f16(const WgradPairsParams &p, const WgradPairsFinalizeParams &f, bool wide, int most_slots, hipStream_t s);
+hipError_t launch_wgrad_pairs_bf16(const WgradPairsParams &p, const WgradPairsFinalizeParams &f, bool wide, int most_slots, hipStream_t s);
 
 // tile shapes the tables above hold
 inline bool rowgemm_has_tile(int tm, int tn) {

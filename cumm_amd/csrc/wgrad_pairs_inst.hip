@@ -1,0 +1,35 @@
+// Instantiations of the pair-list weight gradient for one element type (selected with -DCUMM_ELEM=...).
+#include "launch.h"
+
+namespace cummhip {
+
+#define CUMM_CAT_(a, b) a##b
+#define CUMM_CAT(a, b) CUMM_CAT_(a, b)
+
+template <class T, bool WIDE>
+static hipError_t finalize(const WgradPairsFinalizeParams &f, int most_slots, hipStream_t s) {
+  const uint32_t groups = (uint32_t)f.K * (uint32_t)(f.C / 4);
+  const auto grid = [&](uint32_t g) { return dim3((groups * g + 255) / 256, (unsigned)f.lists); };
+  // Lanes per element: enough for one or two batches of eight loads on a lane of the longest list; with
+  // many lists, most of which have a few slots, eight lanes at most (125 lists, the longest of 81 slots,
+  // 64 x 64 channels: 34.4 us with 32 lanes)
+  if (most_slots <= 16) hipLaunchKernelGGL((wgrad_pairs_finalize_kernel<T, 2, WIDE>), grid(2), dim3(256), 0, s, f);
+  else if (most_slots <= 64 || f.lists > 8) hipLaunchKernelGGL((wgrad_pairs_finalize_kernel<T, 8, WIDE>), grid(8), dim3(256), 0, s, f);
+  else hipLaunchKernelGGL((wgrad_pairs_finalize_kernel<T, 32, WIDE>), grid(32), dim3(256), 0, s, f);
+  return hipGetLastError();
+}
+
+hipError_t CUMM_CAT(launch_wgrad_pairs_, CUMM_NAME)(const WgradPairsParams &p, const WgradPairsFinalizeParams &f, bool wide,
+                                                    int most_slots, hipStream_t s) {
+  using T = CUMM_ELEM;
+  if (!counted_waits_hold<wgrad_pairs_kernel<T>>()) return hipErrorNotSupported;
+  const unsigned grid = (unsigned)((p.wgs + 7) / 8 * 8) * (unsigned)(p.kblocks * p.cblocks);
+  if (grid) {
+    hipLaunchKernelGGL(wgrad_pairs_kernel<T>, dim3(grid), dim3(256), 0, s, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return wide ? finalize<T, true>(f, most_slots, s) : finalize<T, false>(f, most_slots, s);
+}
+
+}  // namespace cummhip

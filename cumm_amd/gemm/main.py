@@ -253,6 +253,13 @@ class GemmMainUnitTest:
                     raise RuntimeError("workspace at least %d bytes." % workspace_size)
             else:
                 workspace = empty([workspace_size], uint8, 0)
+        else:
+            # one slice needs no workspace (the caller's, which other calls may share, stays unused); where
+            # the library can use one all the same it is kept with the validated arguments
+            workspace = Tensor()
+            optional = int(_capi.lib().cumm_hip_query_gemm_optional_workspace(ctypes.byref(desp_to_c(desp)), m, n, k))
+            if optional > 0:
+                workspace = empty([optional], uint8, 0)
 
         args = _capi.GemmArgs()
         args.m, args.n, args.k = m, n, k

@@ -308,20 +308,19 @@ class _SparseConvFunction(torch.autograd.Function):
                 ConvMainUnitTest.implicit_gemm2(p)
                 g._launches[key] = _Launch(p, {"input": grad_in, "weight": weight, "output": grad_out})
         if ctx.needs_input_grad[1] and g.words > 1:
-            # no mask kernel for this pass: one gathered GEMM per kernel offset, straight into its
-            # slice of the gradient (an offset without pairs writes zeros)
+            # no mask kernel for this pass: the products of all kernel offsets over their pair lists, in
+            # one call (an offset without pairs writes zeros)
             from .conv import native
             grad_w = torch.empty_like(weight)
-            key = ("wgrad_per_offset", dtype, tuple(weight.shape), tuple(features.shape), tuple(grad_out.shape))
+            key = ("wgrad_pairs", dtype, tuple(weight.shape), tuple(features.shape), tuple(grad_out.shape))
             plan = g._launches.get(key)
-            if plan is None:      # validated once (the prelude costs 0.1 ms of Python per offset), replayed after
+            if plan is None:
                 plan = native.plan_backward_weight(torch2tensor(grad_out), torch2tensor(features), torch2tensor(grad_w),
                                                    g.lists, stream=stream)
-                plan()
-                plan.release()      # (later calls bring their own tensors)
+                plan.release()      # (every call brings its own tensors)
                 g._launches[key] = plan
-            else:
-                plan.rebind(grad_out.data_ptr(), features.data_ptr(), grad_w.data_ptr(), stream)
+            ws = torch.empty(max(plan.workspace_bytes, 16), dtype=torch.uint8, device=grad_out.device)
+            plan.rebind(grad_out.data_ptr(), features.data_ptr(), grad_w.data_ptr(), stream, ws.data_ptr())
         elif ctx.needs_input_grad[1]:
             grad_w = torch.empty_like(weight)
             # torch's switch for reproducible results selects the fixed-order sum of the partial blocks

@@ -191,6 +191,13 @@ int64_t cumm_hip_query_gemm_workspace(const CummHipGemmDesc *desc, int m, int n,
 int64_t cumm_hip_query_conv_workspace(const CummHipConvDesc *desc, int m, int n, int k, int split_k_slices,
                                       int kernel_volume);
 
+/* Bytes of workspace with which a launch with split_k_slices == 1, which needs none, is faster: a
+ * product with few outputs and a long contraction (ShuffleAB of two-byte elements) is then cut
+ * along the contraction, its partial sums kept in fp32 and rounded once.  0 = none is of use, -1
+ * for bad arguments.  (No counterpart in the reference, which splits only into slices that the
+ * caller asks for.) */
+int64_t cumm_hip_query_gemm_optional_workspace(const CummHipGemmDesc *desc, int m, int n, int k);
+
 /* Bytes of workspace with which the fixed-order backward-weight (CummHipSparseConvArgs.deterministic)
  * runs at full width; 256-byte aligned.  With less it uses fewer workgroups, down to a minimum it
  * names in its error.  -1 for arguments it does not take.  (No counterpart in the reference: its
@@ -354,6 +361,19 @@ int cumm_hip_conv_pairs_fill(const int32_t *coords, int n_in, int batch_size, co
 size_t cumm_hip_pair_lists_workspace(int kv, int n);
 int cumm_hip_pair_lists(const int32_t *indices, int kv, int n, int32_t *pair_in, int32_t *pair_out, int32_t *counts,
                         void *workspace, size_t workspace_bytes, void *stream);
+
+/* Backward-weight of the per-offset convolution for all offsets at once:
+ *   dw[:, r, :] = sum over i < counts[r] of dout[pair_out[r][i]]^T inp[pair_in[r][i]]
+ * dw [K, lists, C], dout [rows_out, K], inp [rows_in, C] (f16 / bf16, fp32 sums in a fixed order, rounded
+ * once); pair_out / pair_in [lists, list_stride] on the device, counts [lists] on the HOST; at most 128
+ * lists; an offset without pairs gets zeros; row numbers outside the tensors contribute nothing.  What
+ * a caller of the reference does with one ShuffleAB matmul2 per offset
+ * (cumm/conv/main_real_spconv.py:375-403).  workspace: cumm_hip_wgrad_pairs_workspace bytes (-1 for
+ * arguments that are not taken), 16-byte aligned. */
+int64_t cumm_hip_wgrad_pairs_workspace(const int32_t *counts, int lists, int K, int C);
+int cumm_hip_wgrad_pairs(void *dw, const void *dout, const void *inp, const int32_t *pair_out, const int32_t *pair_in,
+                         const int32_t *counts, int lists, int64_t list_stride, int rows_out, int rows_in, int K, int C,
+                         int dtype, void *workspace, size_t workspace_bytes, void *stream);
 
 /* Masks of a pair table, any kernel volume up to 128: mask [n, words], words = ceil(kv / 32), bit b of
  * word w of output o set wherever indices[32 w + b][o] >= 0 (the layout a dynamic_mask descriptor takes;

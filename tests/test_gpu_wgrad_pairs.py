@@ -1,0 +1,89 @@
+"""The pair-list weight gradient (wgrad_pairs.h) where its cuts fall: one step and less, one pair more
+than a step, shares of the stream that end inside a list, empty lists, channel blocks with remainders,
+row numbers out of range - against fp32 products of the same operands in numpy."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from cumm_amd import _capi
+from cumm_amd import tensorview as tv
+from cumm_amd.gemm.main import GemmMainUnitTest, desp_to_c
+from cumm_amd.tensorview.gemm import GemmParams, ShuffleStrideType
+import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+# the result is rounded once from fp32 sums: half a unit in the last place of the largest element, and
+# the sums themselves to about 1e-5
+TOL = {"f16": 2.0 ** -11 + 1e-4, "bf16": 2.0 ** -8 + 1e-4}
+
+
+def _data(rng, shape, dtype):
+    return H.to_storage(rng.normal(0, 1, size=shape).astype(np.float32), dtype)
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("counts,k_out,c_in", [
+    ([1], 8, 8), ([32], 64, 64), ([33, 0, 31], 72, 16), ([0, 0, 127, 128, 129], 64, 136), ([0], 16, 24),
+    ([40000], 64, 64), ([9000, 0, 1, 20000, 5], 128, 72), ([300] * 125, 24, 40), ([2000] * 128, 64, 8)])
+def test_pair_lists(counts, k_out, c_in, dtype):
+    print("case wgrad_pairs", counts[:6], len(counts), k_out, c_in, dtype, flush=True)
+    rng = np.random.default_rng(sum(counts) + k_out)
+    lists, stride = len(counts), max(max(counts), 1) + 3
+    rows_out, rows_in = 777, 1234
+    dout, inp = _data(rng, (rows_out, k_out), dtype), _data(rng, (rows_in, c_in), dtype)
+    po = rng.integers(0, rows_out, size=(lists, stride)).astype(np.int32)
+    pi = rng.integers(0, rows_in, size=(lists, stride)).astype(np.int32)
+    po[:, ::17], pi[:, 5::29] = -1, rows_in        # absent rows
+    lib = _capi.lib()
+    cnt = np.array(counts, np.int32)
+    need = int(lib.cumm_hip_wgrad_pairs_workspace(cnt.ctypes.data, lists, k_out, c_in))
+    ws = H.dev(np.full(max(need // 4, 4), np.nan, np.float32), "f32")
+    dw = H.dev(_data(rng, (k_out, lists, c_in), dtype), dtype)
+    d_out, d_in, d_po, d_pi = H.dev(dout, dtype), H.dev(inp, dtype), H.dev(po, "i32"), H.dev(pi, "i32")
+    got = []
+    for _ in range(2):
+        _capi.check(lib.cumm_hip_wgrad_pairs(dw.byte_pointer(), d_out.byte_pointer(), d_in.byte_pointer(), d_po.byte_pointer(),
+                                             d_pi.byte_pointer(), cnt.ctypes.data, lists, stride, rows_out, rows_in, k_out, c_in,
+                                             H.TV_DTYPE[dtype], ws.byte_pointer(), ws.nbytes, 0))
+        got.append(H.as_f32(H.host(dw), dtype))
+    f_out, f_in = H.as_f32(dout, dtype), H.as_f32(inp, dtype)
+    ref = np.zeros((k_out, lists, c_in), np.float32)
+    for r, n in enumerate(counts):
+        ok = (po[r, :n] >= 0) & (pi[r, :n] < rows_in)
+        ref[:, r] = f_out[po[r, :n][ok]].T @ f_in[pi[r, :n][ok]]
+    assert np.array_equal(got[0], got[1])          # a fixed order of the sums
+    scale = max(np.abs(ref).max(), 1.0)
+    assert np.abs(got[0] - ref).max() <= TOL[dtype] * scale
+    for r, n in enumerate(counts):
+        if n == 0:
+            assert not got[0][:, r].any()
+
+
+@pytest.mark.parametrize("pairs", [255, 256, 1000, 33000])
+@pytest.mark.parametrize("dtype,out", [("f16", "f16"), ("bf16", "f32")])
+def test_shuffle_ab_epilogue_on_either_side_of_the_dispatch(pairs, dtype, out):
+    """alpha, beta with a separate D, rows wider than the operand, ReLU, f32 results: the tiled kernel
+    below 256 pairs, the pair-list kernel from there on."""
+    from cumm_amd.tensorview.gemm import Activation
+    print("case shuffle_ab", pairs, dtype, out, flush=True)
+    rng = np.random.default_rng(pairs)
+    rows, m, n = 5000, 72, 136
+    a, b = _data(rng, (rows, m), dtype), _data(rng, (rows, n), dtype)
+    ai, bi = (rng.integers(0, rows, size=pairs).astype(np.int32) for _ in range(2))
+    d = _data(rng, (m, n), out) if out != "f32" else rng.normal(0, 1, size=(m, n)).astype(np.float32)
+    p = GemmParams()
+    p.algo_desp = H.find_gemm_desp(dtype, ShuffleStrideType.ShuffleAB, 64, 64, True, False, dtype_c=out)
+    p.a, p.b = H.dev(a, dtype), H.dev(b, dtype)
+    p.c = tv.zeros([m, n], H.TV_DTYPE[out], 0)
+    p.d = H.dev(d, out)
+    p.a_inds, p.b_inds = H.dev(ai, "i32"), H.dev(bi, "i32")
+    p.alpha, p.beta, p.act_type = 0.25, 2.0, Activation.ReLU
+    GemmMainUnitTest.matmul2(p)
+    ref = np.maximum(0.25 * (H.as_f32(a, dtype)[ai].T @ H.as_f32(b, dtype)[bi]) + 2.0 * (H.as_f32(d, out) if out != "f32" else d), 0)
+    got = H.host(p.c) if out == "f32" else H.as_f32(H.host(p.c), out)
+    tol = 1e-5 * np.sqrt(pairs) if out == "f32" else TOL[out]
+    assert np.abs(got - ref).max() <= tol * max(np.abs(ref).max(), 1.0)
+    cd = desp_to_c(p.algo_desp)
+    assert (int(_capi.lib().cumm_hip_query_gemm_optional_workspace(ctypes.byref(cd), m, n, pairs)) > 0) == (pairs >= 256)
