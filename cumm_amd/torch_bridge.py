@@ -100,45 +100,72 @@ def _desp_like(dtype, op, parallel=False, dynamic=False):
     return _DESP_LIKE[key].copy()
 
 
+_PTRS = ("ptr_A", "ptr_B", "ptr_C", "ptr_D", "bias_pointer", "workspace")
+
+
 class _Launch:
     """The validated argument block of one operator call, replayed with other tensors of the same
-    shapes: the first call goes through the operator's prelude (and the tuner), a repeat patches the
-    pointers of the tensors that change from call to call into the block and calls the C entry
-    point - a layer of a network makes the same call every iteration, and the prelude costs several
-    times what the kernel does."""
+    shapes - and on other geometries: the first call of its kind goes through the operator's prelude
+    and the tuner (close to a millisecond of Python), a repeat copies the block, patches the pointers
+    that change from call to call into it and calls the C entry point.  A copy per call, so that
+    threads can share a geometry."""
 
-    _FIELDS = ("ptr_A", "ptr_B", "ptr_C", "ptr_D", "bias_pointer", "workspace")
+    __slots__ = ("fn", "cdesc", "args", "fields", "tile_m", "_call")
 
-    def __init__(self, params: ConvParams, roles):
+    def __init__(self, fn, cdesc, args, fields, tile_m):
+        self.fn, self.cdesc, self.args, self.fields, self.tile_m = fn, cdesc, args, fields, tile_m
+        self._call = ctypes.byref(cdesc)
+
+    @classmethod
+    def of(cls, params: ConvParams, roles) -> "_Launch":
         prep = params.__dict__.get("_prepared")
         if prep is None:
             raise RuntimeError("the operator call left no validated argument block")
-        self.fn, self.cdesc, self.args = prep[1], prep[4], prep[5]
-        self.params = params       # keeps the geometry's tensors alive
-        self.fields = {}
+        args = _copy(prep[5])
+        fields = {}
         for role, t in roles.items():
             ptr = t.data_ptr()
-            if t.numel() == 0:     # an empty tensor has no address to find in the block: nothing to patch
-                self.fields[role] = []
-                continue
-            self.fields[role] = [f for f in self._FIELDS if ptr and getattr(self.args, f) == ptr]
-            if not self.fields[role]:
+            # (an empty tensor has no address to find in the block: nothing to patch)
+            fields[role] = tuple(f for f in _PTRS if ptr and t.numel() and getattr(args, f) == ptr)
+            if t.numel() and not fields[role]:
                 raise RuntimeError("the argument block does not point at the %s tensor" % role)
-        # the tensors of the first call are replaced by the caller's on every replay: only the
-        # geometry's stay referenced here (a backward-weight workspace can be tens of megabytes)
-        from .tensorview import Tensor as _T
-        for name in ("input", "weight", "output", "bias", "workspace"):
-            if name in roles:
-                params.__dict__[name] = _T()
+        return cls(prep[1], prep[4], args, fields, int(params.conv_algo_desp.tile_shape[0]))
 
-    def __call__(self, stream: int, **tensors) -> None:
+    def on(self, n_pos, rows_in, rows_out, indices, mask, argsort, mask_out) -> "_Launch":
+        """The same call on another geometry (device addresses)."""
+        args = _copy(self.args)
+        args.N, args.rows_in, args.rows_out = n_pos, rows_in, rows_out
+        args.indice_ptr, args.mask_ptr, args.mask_argsort_ptr, args.mask_out_ptr = indices, mask, argsort, mask_out
+        return _Launch(self.fn, self.cdesc, args, self.fields, self.tile_m)
+
+    def __call__(self, stream: int, workspace_bytes: int = 0, **tensors) -> None:
+        args = _copy(self.args)
         for role, t in tensors.items():
             ptr = t.data_ptr()
             for f in self.fields[role]:
-                setattr(self.args, f, ptr)
-        status = self.fn(ctypes.byref(self.cdesc), ctypes.byref(self.args), stream)
+                setattr(args, f, ptr)
+        if workspace_bytes:
+            args.workspace_bytes = workspace_bytes
+        status = self.fn(self._call, ctypes.byref(args), stream)
         if status:
             _capi.check(status)
+
+
+def _copy(args: _capi.SparseConvArgs) -> _capi.SparseConvArgs:
+    return _capi.SparseConvArgs.from_buffer_copy(args)
+
+
+# validated calls by kind (pass, types, channels, kernel volume, epilogue, size class): what _Launch.on
+# moves to the next geometry.  Bounded by the kinds of layers a program has.
+_KINDS = {}
+
+
+def _size_class(n: int) -> int:
+    return max(n - 1, 0).bit_length()      # (the tuner's bucket of the position count)
+
+
+def _bytes(n: int, device) -> torch.Tensor:
+    return torch.empty(max(int(n), 256), dtype=torch.uint8, device=device)
 
 
 class SparseConvGeometry:
@@ -146,79 +173,162 @@ class SparseConvGeometry:
     every layer (and every pass) that uses it.  Kernel volumes up to 32 have one mask word per
     position; above that (up to 128, e.g. 5 x 5 x 5) the masks have ``ceil(kv / 32)`` words, forward
     and backward-input run on the ``dynamic_mask`` descriptors, and backward-weight - which has no
-    such kernel, in the reference neither - goes offset by offset over the pair lists."""
+    such kernel, in the reference neither - goes over the pair lists of all offsets.
+
+    All tables lie in one block from torch's caching allocator (a new cloud per iteration then
+    allocates nothing from the driver); ``indices_fwd`` and the other tables are views of it."""
+
+    _TABLES = ("indices_fwd", "indices_bwd", "mask_fwd", "order_fwd", "mask_bwd", "order_bwd", "indices_fwd_pos", "indices_bwd_pos")
 
     def __init__(self, coords: torch.Tensor, spatial_shape: Sequence[int], ksize=(3, 3, 3), stride=None,
                  padding=(1, 1, 1), dilation=(1, 1, 1), batch_size: int = 1):
         if coords.dtype != torch.int32 or not coords.is_cuda or coords.dim() != 2 or coords.shape[1] != 4:
             raise ValueError("coords must be a cuda int32 tensor [N, 4] of (batch, z, y, x)")
         coords = coords.contiguous()
-        stream = current_stream()
-        c_tv = torch2tensor(coords)
+        self._stream = s = current_stream()
+        self._device = dev = coords.device
         self.subm = stride is None
-        self.n_in = int(coords.shape[0])
-        self.kv = int(ksize[0]) * int(ksize[1]) * int(ksize[2])
-        if self.subm:
-            t = pairs.subm_pairs_device(c_tv, spatial_shape, ksize, dilation, stream=stream)
-            self.out_coords, self.out_shape = coords, tuple(int(s) for s in spatial_shape)
-        else:
-            t = pairs.sparse_conv_pairs_device(c_tv, spatial_shape, ksize, stride, padding, dilation,
-                                               batch_size=batch_size, stream=stream)
-            self.out_coords, self.out_shape = tensor2torch(t.out_coords, clone=False), t.out_shape
-        self.indices_fwd, self.indices_bwd = t.indices_fwd, t.indices_bwd
-        self.n_out = int(t.indices_fwd.dim(1))
-        self.words = (self.kv + 31) // 32
+        self.n_in = n_in = int(coords.shape[0])
+        self.kv = kv = int(ksize[0]) * int(ksize[1]) * int(ksize[2])
+        self.words = words = (kv + 31) // 32
         self.lists = None
-        if self.kv > 32:
-            # the builders give no masks for these volumes: made from the tables, sorted by offset
-            # count and word pattern; the per-offset lists serve backward-weight
-            mf = pairs.masks_from_pairs_device(t.indices_fwd, stream=stream)
-            self.mask_fwd, self.order_fwd = pairs.sort_by_mask_words_device(mf, stream=stream)
-            if self.subm:
-                self.mask_bwd, self.order_bwd = self.mask_fwd, self.order_fwd
-            else:
-                mb = pairs.masks_from_pairs_device(t.indices_bwd, stream=stream)
-                self.mask_bwd, self.order_bwd = pairs.sort_by_mask_words_device(mb, stream=stream)
-            self.lists = pairs.pair_lists_device(t.indices_fwd, stream=stream)
-            self.light_fwd = self.light_bwd = 0
-            self.indices_fwd_pos = pairs.pairs_by_position_device(self.indices_fwd, self.order_fwd, stream=stream)
-            self.indices_bwd_pos = pairs.pairs_by_position_device(self.indices_bwd, self.order_bwd, stream=stream)
-            self._reduced = {}
-            self._launches = {}
+        # (how far the light end of each sorted order reaches - the hint of the forward and backward-input
+        # launches - stays on the device: the sort leaves it in the library's table under the sorted
+        # array's address and the launches look it up there; 0 = not given here)
+        self.light_fwd = self.light_bwd = 0
+        self._reduced = {}
+        self._launches = {}      # calls of the layers on this geometry, see _Launch
+        self._tensors = {}
+        lib, arr3 = _capi.lib(), ctypes.c_int32 * 3
+        shape, ks, pad, dil = (arr3(*[int(v) for v in a]) for a in (spatial_shape, ksize, padding, dilation))
+        masks = words == 1       # (the builders make masks of one word)
+        if self.subm:
+            pairs._check_odd_ksize(ksize)
+            self.n_out = n_out = n_in
+            self.out_coords, self.out_shape = coords, tuple(int(v) for v in spatial_shape)
+            self._allocate()
+            ws = _bytes(lib.cumm_hip_subm_pairs_workspace(n_in), dev)
+            _capi.check(lib.cumm_hip_subm_pairs(
+                coords.data_ptr(), n_in, shape, ks, dil, self._ptr["indices_fwd"], self._ptr["indices_bwd"],
+                self._ptr["raw_fwd"] if masks else None, self._ptr["raw_bwd"] if masks else None, ws.data_ptr(), ws.numel(), s))
+        else:
+            st = arr3(*[int(v) for v in stride])
+            geo = (shape, ks, st, pad, dil)
+            need = int(lib.cumm_hip_conv_pairs_workspace(n_in, int(batch_size), *geo))
+            if need == 0:
+                raise ValueError("bad geometry (kernel volume 1..128, non-empty output grid) or too many voxels")
+            ws = _bytes(need, dev)
+            out_shape, found = arr3(), ctypes.c_int32(0)
+            _capi.check(lib.cumm_hip_conv_pairs_sites(coords.data_ptr(), n_in, int(batch_size), *geo, out_shape,
+                                                      ctypes.byref(found), ws.data_ptr(), ws.numel(), s))
+            self.n_out = n_out = int(found.value)
+            self.out_shape = tuple(int(v) for v in out_shape)
+            self.out_coords = torch.empty((n_out, 4), dtype=torch.int32, device=dev)
+            self._allocate()
+            _capi.check(lib.cumm_hip_conv_pairs_fill(
+                coords.data_ptr(), n_in, int(batch_size), *geo, n_out, self.out_coords.data_ptr(), self._ptr["indices_fwd"],
+                self._ptr["indices_bwd"], self._ptr["raw_fwd"] if masks else None, self._ptr["raw_bwd"] if masks else None,
+                ws.data_ptr(), ws.numel(), s))
+        for side, n in (("fwd", n_out), ("bwd", n_in)):
+            if side == "fwd" or not self.subm:
+                self._sort(side, n)
+            # the pair tables once more in the order of the sorted positions: what forward and
+            # backward-input read (a tile's entries for one offset are then consecutive in memory);
+            # backward-weight keeps the table by row
+            _capi.check(lib.cumm_hip_pairs_by_position(self._ptr["indices_" + side], self._ptr["order_" + side], kv, n,
+                                                       self._ptr["indices_%s_pos" % side], s))
+        if not masks:
+            self._make_lists()
+
+    def _allocate(self) -> None:
+        n_out, n_in, kv, words = self.n_out, self.n_in, self.kv, self.words
+        mask = [self.n_out] if words == 1 else [n_out, words]
+        spec = [("indices_fwd", [kv, n_out], tv.int32), ("indices_bwd", [kv, n_in], tv.int32),
+                ("indices_fwd_pos", [kv, n_out], tv.int32), ("indices_bwd_pos", [kv, n_in], tv.int32),
+                ("mask_fwd", mask, tv.uint32), ("order_fwd", [n_out], tv.int32), ("raw_fwd", mask, tv.uint32)]
+        mask = [n_in] if words == 1 else [n_in, words]
+        if not self.subm:
+            spec += [("mask_bwd", mask, tv.uint32), ("order_bwd", [n_in], tv.int32)]
+        spec.append(("raw_bwd", mask, tv.uint32))
+        self._spec, at = {}, 0
+        for name, dims, dtype in spec:
+            self._spec[name] = (at, dims, dtype)
+            size = 4
+            for d in dims:
+                size *= d
+            at += (size + 255) // 256 * 256
+        self._block = _bytes(at, self._device)
+        base = self._block.data_ptr()
+        self._ptr = {name: base + v[0] for name, v in self._spec.items()}
+        if self.subm:      # the forward masks serve the backward-input pass, bit-reversed in the kernel
+            for name in ("mask", "order"):
+                self._spec[name + "_bwd"], self._ptr[name + "_bwd"] = self._spec[name + "_fwd"], self._ptr[name + "_fwd"]
+
+    def _sort(self, side: str, n: int) -> None:
+        lib, p, s = _capi.lib(), self._ptr, self._stream
+        if self.words > 1:
+            # the builders give no masks for these volumes: made from the tables, sorted by offset count
+            # and word pattern
+            _capi.check(lib.cumm_hip_masks_from_pairs(p["indices_" + side], self.kv, n, p["raw_" + side], s))
+            ws = _bytes(lib.cumm_hip_sort_by_mask_words_workspace(n), self._device)
+            _capi.check(lib.cumm_hip_sort_by_mask_words(p["raw_" + side], n, self.words, p["mask_" + side], p["order_" + side],
+                                                        ws.data_ptr(), ws.numel(), s))
             return
         # (a mask has one bit per kernel offset: a filter of that width spares the sort the passes over
-        # the bits above it)
+        # the bits above it; the library's order by offset count where the masks leave room for the
+        # count: same rows, lighter tiles, and the few many-offset tiles in a short run at the end)
         bits = (1 << self.kv) - 1 if self.kv < 32 else 0xFFFFFFFF
-        # (the library's order by offset count where the masks leave room for the count: same rows,
-        # lighter tiles, and the few many-offset tiles in a short run at the end)
-        by_count = self.kv <= 27
-        self.mask_fwd, self.order_fwd = pairs.sort_by_mask_device(t.mask_fwd, mask_filter=bits, stream=stream,
-                                                                  by_offset_count=by_count)
-        if self.subm:      # the forward masks serve the backward-input pass, bit-reversed in the kernel
-            self.mask_bwd, self.order_bwd = self.mask_fwd, self.order_fwd
-        else:
-            self.mask_bwd, self.order_bwd = pairs.sort_by_mask_device(t.mask_bwd, mask_filter=bits, stream=stream,
-                                                                      by_offset_count=by_count)
-        # (how far the light end of each sorted order reaches - the hint of the forward and
-        # backward-input launches - stays on the device: the sort leaves it in the library's table
-        # under the sorted array's address and the launches look it up there; 0 = not given here)
-        self.light_fwd = self.light_bwd = 0
-        # the pair tables once more in the order of the sorted positions: what forward and
-        # backward-input read (a tile's entries for one offset are then consecutive in memory);
-        # backward-weight keeps the table by row
-        self.indices_fwd_pos = pairs.pairs_by_position_device(self.indices_fwd, self.order_fwd, stream=stream)
-        self.indices_bwd_pos = pairs.pairs_by_position_device(self.indices_bwd, self.order_bwd, stream=stream)
-        self._reduced = {}
-        self._launches = {}      # validated calls of the layers on this geometry, see _Launch
+        ws = _bytes(lib.cumm_hip_sort_by_mask_workspace(n), self._device)
+        _capi.check(lib.cumm_hip_sort_by_mask_ordered(p["raw_" + side], n, bits, 1 if self.kv <= 27 else 0, p["mask_" + side],
+                                                      p["order_" + side], ws.data_ptr(), ws.numel(), s))
+
+    def _make_lists(self) -> None:
+        """The per-offset pair lists of backward-weight; their counts come to the host."""
+        n, kv, lib = self.n_out, self.kv, _capi.lib()
+        lists = torch.empty((2, kv, n), dtype=torch.int32, device=self._device)
+        counts = torch.empty(kv, dtype=torch.int32, device=self._device)
+        need = int(lib.cumm_hip_pair_lists_workspace(kv, n))
+        ws = _bytes(need, self._device)
+        _capi.check(lib.cumm_hip_pair_lists(self._ptr["indices_fwd"], kv, n, lists[0].data_ptr(), lists[1].data_ptr(),
+                                            counts.data_ptr(), ws.data_ptr(), ws.numel(), self._stream))
+        self.lists = pairs.DevicePairLists(torch2tensor(lists[0]), torch2tensor(lists[1]), counts.cpu().numpy())
+        self._list_block = lists
+
+    def __getattr__(self, name: str):
+        if name not in SparseConvGeometry._TABLES or "_spec" not in self.__dict__:
+            raise AttributeError(name)
+        t = self._tensors.get(name)
+        if t is None:
+            _, dims, dtype = self._spec[name]
+            t = self._tensors[name] = tv.from_blob(self._ptr[name], dims, dtype, self._device.index, keepalive=self._block)
+        return t
+
+    def used_on(self, stream: int) -> None:
+        """Tell torch's allocator that ``stream`` - the current one - reads the tables."""
+        if stream != self._stream:
+            current = torch.cuda.current_stream()
+            self._block.record_stream(current)
+            for buf in self._reduced.values():
+                buf.record_stream(current)
+            if self.lists is not None:
+                self._list_block.record_stream(current)
+
+    def reduced_mask(self, width: int) -> torch.Tensor:
+        """One word per run of ``width`` sorted output positions: the forward launch writes (all of) the
+        OR of the run's masks here (its ``mask_output``), and backward-weight reads it."""
+        buf = self._reduced.get(width)
+        if buf is None:
+            tiles = (self.n_out + width - 1) // width
+            buf = self._reduced[width] = torch.empty(max(tiles, 1), dtype=torch.int32, device=self._device)
+        return buf
 
     def reduced_mask_buffer(self, width: int) -> tv.Tensor:
-        """One word per run of ``width`` sorted output positions: the forward launch writes the
-        OR of the run's masks here (its ``mask_output``), and backward-weight reads it."""
-        if width not in self._reduced:
-            tiles = (self.n_out + width - 1) // width
-            buf = torch.zeros(max(tiles, 1), dtype=torch.int32, device=self.out_coords.device)
-            self._reduced[width] = (torch2tensor(buf).type_view(tv.uint32), buf)
-        return self._reduced[width][0]
+        return torch2tensor(self.reduced_mask(width)).type_view(tv.uint32)
+
+
+def _same_device(*tensors) -> None:
+    if any(t.device != tensors[0].device for t in tensors):
+        raise ValueError("all tensors must be on the same device")
 
 
 class _SparseConvFunction(torch.autograd.Function):
@@ -230,46 +340,18 @@ class _SparseConvFunction(torch.autograd.Function):
             raise ValueError("features must be [%d, C]: one row per input site of the geometry" % geometry.n_in)
         if weight.dim() != 3 or weight.shape[1] != geometry.kv or weight.shape[2] != features.shape[1]:
             raise ValueError("weight must be [K, %d, %d]" % (geometry.kv, features.shape[1]))
-        dtype = _TORCH_TO_TV[features.dtype]
         out = torch.empty((geometry.n_out, weight.shape[0]), dtype=features.dtype, device=features.device)
-        if bias is not None:
-            bias = bias.contiguous()
-        key = ("fwd", dtype, weight.dtype, tuple(features.shape), tuple(weight.shape),
-               None if bias is None else (bias.dtype, tuple(bias.shape)), relu)
-        hit = geometry._launches.get(key)
-        if hit is not None:
-            launch, tile_m = hit
-            if bias is not None:
-                launch(current_stream(), input=features, weight=weight, output=out, bias=bias)
-            else:
-                launch(current_stream(), input=features, weight=weight, output=out)
-            ctx.geometry, ctx.relu, ctx.has_bias, ctx.tile_m = geometry, relu, bias is not None, tile_m
-            ctx.save_for_backward(features, weight, out if relu else None)
-            return out
-        p = ConvParams(3, ConvOpType.Forward)
-        p.conv_algo_desp = _desp_like(dtype, ConvOpType.Forward, dynamic=geometry.words > 1)
-        p.input, p.weight, p.output = torch2tensor(features), torch2tensor(weight), torch2tensor(out)
-        p.indices, p.mask, p.mask_argsort = geometry.indices_fwd_pos, geometry.mask_fwd, geometry.order_fwd
-        p.indices_by_position = True
-        p.mask_int_count = geometry.words
-        p.light_prefix = geometry.light_fwd
-        if bias is not None:
-            p.bias, p.beta = torch2tensor(bias), 1.0
-        if relu:
-            p.act_type = Activation.ReLU
-        p.stream = current_stream()
-        _TUNER.tune_conv(p)
-        # the tile masks the forward launch computes anyway are what backward-weight needs
-        # (not for several mask words: that backward-weight walks the pair lists)
-        tile_m = int(p.conv_algo_desp.tile_shape[0])
-        if geometry.words == 1:
-            p.mask_output = geometry.reduced_mask_buffer(tile_m)
-        ConvMainUnitTest.implicit_gemm2(p)
         roles = {"input": features, "weight": weight, "output": out}
         if bias is not None:
-            roles["bias"] = bias
-        geometry._launches[key] = (_Launch(p, roles), tile_m)
-        ctx.geometry, ctx.relu, ctx.has_bias, ctx.tile_m = geometry, relu, bias is not None, tile_m
+            roles["bias"] = bias = bias.contiguous()
+        stream = current_stream()
+        geometry.used_on(stream)
+        key = ("fwd", features.dtype, weight.dtype, weight.shape, None if bias is None else (bias.dtype, bias.shape), relu)
+        launch = geometry._launches.get(key)
+        if launch is None:
+            launch = _forward_launch(geometry, key, roles, relu, stream)
+        launch(stream, **roles)
+        ctx.geometry, ctx.relu, ctx.has_bias, ctx.tile_m = geometry, relu, bias is not None, launch.tile_m
         ctx.save_for_backward(features, weight, out if relu else None)
         return out
 
@@ -280,6 +362,7 @@ class _SparseConvFunction(torch.autograd.Function):
         grad_out = grad_out.contiguous()
         dtype = _TORCH_TO_TV[features.dtype]
         stream = current_stream()
+        g.used_on(stream)
         lib = _capi.lib()
         if ctx.relu:       # the gradient passes where the fused ReLU let the output through
             gated = torch.empty_like(grad_out)
@@ -290,74 +373,140 @@ class _SparseConvFunction(torch.autograd.Function):
         if ctx.needs_input_grad[0]:
             # inputs that feed no output site sit in tiles the kernel skips (mask 0): zero them
             grad_in = torch.empty_like(features) if g.subm else torch.zeros_like(features)
-            key = ("dgrad", dtype, tuple(weight.shape))
+            roles = {"input": grad_in, "weight": weight, "output": grad_out}
+            key = ("dgrad", dtype, weight.shape)
             launch = g._launches.get(key)
-            if launch is not None:
-                launch(stream, input=grad_in, weight=weight, output=grad_out)
-            else:
-                p = ConvParams(3, ConvOpType.BackwardInput)
-                p.conv_algo_desp = _desp_like(dtype, ConvOpType.BackwardInput, dynamic=g.words > 1)
-                p.input, p.weight, p.output = torch2tensor(grad_in), torch2tensor(weight), torch2tensor(grad_out)
-                p.indices, p.mask, p.mask_argsort = g.indices_bwd_pos, g.mask_bwd, g.order_bwd
-                p.indices_by_position = True
-                p.mask_int_count = g.words
-                p.reverse_mask = g.subm
-                p.light_prefix = g.light_bwd
-                p.stream = stream
-                _TUNER.tune_conv(p)
-                ConvMainUnitTest.implicit_gemm2(p)
-                g._launches[key] = _Launch(p, {"input": grad_in, "weight": weight, "output": grad_out})
+            if launch is None:
+                launch = _backward_input_launch(g, key, roles, dtype, stream)
+            launch(stream, **roles)
         if ctx.needs_input_grad[1] and g.words > 1:
             # no mask kernel for this pass: the products of all kernel offsets over their pair lists, in
             # one call (an offset without pairs writes zeros)
             from .conv import native
             grad_w = torch.empty_like(weight)
-            key = ("wgrad_pairs", dtype, tuple(weight.shape), tuple(features.shape), tuple(grad_out.shape))
+            key = ("wgrad_pairs", dtype, weight.shape)
             plan = g._launches.get(key)
             if plan is None:
                 plan = native.plan_backward_weight(torch2tensor(grad_out), torch2tensor(features), torch2tensor(grad_w),
                                                    g.lists, stream=stream)
                 plan.release()      # (every call brings its own tensors)
                 g._launches[key] = plan
-            ws = torch.empty(max(plan.workspace_bytes, 16), dtype=torch.uint8, device=grad_out.device)
+            ws = _bytes(plan.workspace_bytes, grad_out.device)
             plan.rebind(grad_out.data_ptr(), features.data_ptr(), grad_w.data_ptr(), stream, ws.data_ptr())
         elif ctx.needs_input_grad[1]:
             grad_w = torch.empty_like(weight)
             # torch's switch for reproducible results selects the fixed-order sum of the partial blocks
             deterministic = bool(torch.are_deterministic_algorithms_enabled())
-            key = ("wgrad", dtype, tuple(weight.shape), ctx.tile_m, deterministic)
+            key = ("wgrad", dtype, weight.shape, ctx.tile_m, deterministic)
             hit = g._launches.get(key)
-            if hit is not None:
-                launch, need = hit
-                # the workspace comes from torch's caching allocator (the prelude's own would be a
-                # device allocation per call)
-                ws = torch.empty(need, dtype=torch.uint8, device=grad_out.device)
-                launch(stream, input=features, weight=grad_w, output=grad_out, workspace=ws)
-            else:
-                p = ConvParams(3, ConvOpType.BackwardWeight)
-                p.conv_algo_desp = _desp_like(dtype, ConvOpType.BackwardWeight, parallel=True)
-                p.input, p.weight, p.output = torch2tensor(features), torch2tensor(grad_w), torch2tensor(grad_out)
-                p.indices, p.mask, p.mask_argsort = g.indices_fwd, g.reduced_mask_buffer(ctx.tile_m), g.order_fwd
-                p.mask_width, p.split_k_slices = ctx.tile_m, 32
-                p.deterministic = deterministic
-                n_pos, k_out, kv, c_in = int(grad_out.shape[0]), int(weight.shape[0]), int(weight.shape[1]), int(weight.shape[2])
-                need = p.conv_algo_desp.query_conv_workspace_size(k_out, kv * c_in, n_pos, p.split_k_slices, kv)
-                if deterministic:
-                    need = max(need, int(lib.cumm_hip_query_wgrad_ordered_workspace(n_pos, c_in, k_out, kv, ctx.tile_m)))
-                need = max(int(need), 256)
-                ws = torch.empty(need, dtype=torch.uint8, device=grad_out.device)
-                p.workspace = torch2tensor(ws)
-                p.stream = stream
-                ConvMainUnitTest.implicit_gemm2(p)
-                g._launches[key] = (_Launch(p, {"input": features, "weight": grad_w, "output": grad_out, "workspace": ws}), need)
+            if hit is None:
+                hit = g._launches[key] = _backward_weight_launch(g, key, features, weight, grad_w, grad_out, dtype, stream)
+            launch, need = hit
+            # the workspace comes from torch's caching allocator (the prelude's own would be a
+            # device allocation per call)
+            ws = _bytes(need, grad_out.device)
+            launch(stream, need, input=features, weight=grad_w, output=grad_out, workspace=ws)
         if ctx.has_bias and ctx.needs_input_grad[2]:
             rows, k_out = int(grad_out.shape[0]), int(grad_out.shape[1])
             grad_b = torch.empty(k_out, dtype=grad_out.dtype, device=grad_out.device)
             need = int(lib.cumm_hip_column_sum_workspace(rows, k_out))
-            ws = torch.empty(max(need, 4), dtype=torch.uint8, device=grad_out.device)
+            ws = _bytes(need, grad_out.device)
             _capi.check(lib.cumm_hip_column_sum(grad_b.data_ptr(), grad_out.data_ptr(), rows, k_out, dtype,
-                                                ws.data_ptr(), need, stream))
+                                                ws.data_ptr(), ws.numel(), stream))
         return grad_in, grad_w, grad_b, None, None
+
+
+def _kind(g: SparseConvGeometry, key, n_pos: int, *tensors):
+    """The key of a call in _KINDS; the tensors of a first call are checked here for what the operator's
+    prelude checks and a moved call does not (types and shapes are in the key)."""
+    _same_device(*tensors)
+    return key + (g.kv, g.subm, _size_class(n_pos), tensors[0].device.index)
+
+
+def _forward_launch(g: SparseConvGeometry, key, roles, relu, stream) -> _Launch:
+    features, weight, out, bias = roles["input"], roles["weight"], roles["output"], roles.get("bias")
+    kind = _kind(g, key, g.n_out, *roles.values())
+    known = _KINDS.get(kind)
+    if known is not None and features.numel() and out.numel():
+        launch = known.on(g.n_out, g.n_in, g.n_out, g._ptr["indices_fwd_pos"], g._ptr["mask_fwd"], g._ptr["order_fwd"],
+                          g.reduced_mask(known.tile_m).data_ptr() if g.words == 1 else None)
+        g._launches[key] = launch
+        return launch
+    p = ConvParams(3, ConvOpType.Forward)
+    dtype = _TORCH_TO_TV[features.dtype]
+    p.conv_algo_desp = _desp_like(dtype, ConvOpType.Forward, dynamic=g.words > 1)
+    p.input, p.weight, p.output = torch2tensor(features), torch2tensor(weight), torch2tensor(out)
+    p.indices, p.mask, p.mask_argsort = g.indices_fwd_pos, g.mask_fwd, g.order_fwd
+    p.indices_by_position = True
+    p.mask_int_count = g.words
+    p.light_prefix = g.light_fwd
+    if bias is not None:
+        p.bias, p.beta = torch2tensor(bias), 1.0
+    if relu:
+        p.act_type = Activation.ReLU
+    p.stream = stream
+    _TUNER.tune_conv(p)
+    # the tile masks the forward launch computes anyway are what backward-weight needs
+    # (not for several mask words: that backward-weight walks the pair lists)
+    if g.words == 1:
+        p.mask_output = g.reduced_mask_buffer(int(p.conv_algo_desp.tile_shape[0]))
+    ConvMainUnitTest.implicit_gemm2(p)
+    launch = g._launches[key] = _Launch.of(p, roles)
+    _KINDS[kind] = launch
+    return launch
+
+
+def _backward_input_launch(g: SparseConvGeometry, key, roles, dtype, stream) -> _Launch:
+    grad_in, weight, grad_out = roles["input"], roles["weight"], roles["output"]
+    kind = _kind(g, key, g.n_in, *roles.values())
+    known = _KINDS.get(kind)
+    if known is not None and grad_in.numel() and grad_out.numel():
+        launch = known.on(g.n_in, g.n_in, g.n_out, g._ptr["indices_bwd_pos"], g._ptr["mask_bwd"], g._ptr["order_bwd"], None)
+        g._launches[key] = launch
+        return launch
+    p = ConvParams(3, ConvOpType.BackwardInput)
+    p.conv_algo_desp = _desp_like(dtype, ConvOpType.BackwardInput, dynamic=g.words > 1)
+    p.input, p.weight, p.output = torch2tensor(grad_in), torch2tensor(weight), torch2tensor(grad_out)
+    p.indices, p.mask, p.mask_argsort = g.indices_bwd_pos, g.mask_bwd, g.order_bwd
+    p.indices_by_position = True
+    p.mask_int_count = g.words
+    p.reverse_mask = g.subm
+    p.light_prefix = g.light_bwd
+    p.stream = stream
+    _TUNER.tune_conv(p)
+    ConvMainUnitTest.implicit_gemm2(p)
+    launch = g._launches[key] = _Launch.of(p, roles)
+    _KINDS[kind] = launch
+    return launch
+
+
+def _backward_weight_launch(g: SparseConvGeometry, key, features, weight, grad_w, grad_out, dtype, stream):
+    """(call, bytes of workspace)"""
+    tile_m, deterministic = key[3], key[4]
+    n_pos, k_out, kv, c_in = int(grad_out.shape[0]), int(weight.shape[0]), int(weight.shape[1]), int(weight.shape[2])
+    desp = _desp_like(dtype, ConvOpType.BackwardWeight, parallel=True)
+    slices = 32
+    need = desp.query_conv_workspace_size(k_out, kv * c_in, n_pos, slices, kv)
+    if deterministic:
+        need = max(need, int(_capi.lib().cumm_hip_query_wgrad_ordered_workspace(n_pos, c_in, k_out, kv, tile_m)))
+    need = max(int(need), 256)
+    kind = _kind(g, key, n_pos, grad_out, features, grad_w)
+    known = _KINDS.get(kind)
+    if known is not None and features.numel() and grad_out.numel():
+        return known.on(n_pos, g.n_in, g.n_out, g._ptr["indices_fwd"], g.reduced_mask(tile_m).data_ptr(), g._ptr["order_fwd"],
+                        None), need
+    p = ConvParams(3, ConvOpType.BackwardWeight)
+    p.conv_algo_desp = desp
+    p.input, p.weight, p.output = torch2tensor(features), torch2tensor(grad_w), torch2tensor(grad_out)
+    p.indices, p.mask, p.mask_argsort = g.indices_fwd, g.reduced_mask_buffer(tile_m), g.order_fwd
+    p.mask_width, p.split_k_slices = tile_m, slices
+    p.deterministic = deterministic
+    ws = _bytes(need, grad_out.device)
+    p.workspace = torch2tensor(ws)
+    p.stream = stream
+    ConvMainUnitTest.implicit_gemm2(p)
+    launch = _KINDS[kind] = _Launch.of(p, {"input": features, "weight": grad_w, "output": grad_out, "workspace": ws})
+    return launch, need
 
 
 def sparse_conv(features: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
