@@ -60,6 +60,11 @@ class SparseConvArgs(C.Structure):
                 ("ungated_rows", C.c_int32), ("indices_by_position", C.c_int32), ("mask_int_count", C.c_int32)]
 
 
+class OrderSide(C.Structure):
+    _fields_ = [("indices", C.c_void_p), ("n", C.c_int32), ("sorted_mask", C.c_void_p), ("argsort", C.c_void_p),
+                ("by_position", C.c_void_p), ("by_position_reversed", C.c_void_p)]
+
+
 # every symbol include/cumm_hip.h declares: name -> (restype, argtypes)
 _VP, _PVP = C.c_void_p, C.POINTER(C.c_void_p)
 SYMBOLS = {
@@ -116,6 +121,8 @@ SYMBOLS = {
                                  [C.c_int, _VP, _VP, _VP, _VP, _VP, _VP, C.c_size_t, _VP]),
     "cumm_hip_pair_lists_workspace": (C.c_size_t, [C.c_int, C.c_int]),
     "cumm_hip_pair_lists": (C.c_int, [_VP, C.c_int, C.c_int, _VP, _VP, _VP, _VP, C.c_size_t, _VP]),
+    "cumm_hip_order_pairs_workspace": (C.c_size_t, [C.POINTER(OrderSide), C.c_int, C.c_int]),
+    "cumm_hip_order_pairs": (C.c_int, [C.POINTER(OrderSide), C.c_int, C.POINTER(C.c_int32), _VP, C.c_size_t, _VP]),
     "cumm_hip_wgrad_pairs_workspace": (C.c_int64, [_VP, C.c_int, C.c_int, C.c_int]),
     "cumm_hip_wgrad_pairs": (C.c_int, [_VP, _VP, _VP, _VP, _VP, _VP, C.c_int, C.c_int64, C.c_int, C.c_int, C.c_int, C.c_int,
                                        C.c_int, _VP, C.c_size_t, _VP]),

@@ -32,7 +32,8 @@ def _units():
              ("pairs", os.path.join(CSRC, "pairs_inst.hip"), []),
              ("gather", os.path.join(CSRC, "gather_inst.hip"), []),
              ("elementwise", os.path.join(CSRC, "elementwise_inst.hip"), []),
-             ("sort", os.path.join(CSRC, "sort_inst.hip"), [])]
+             ("sort", os.path.join(CSRC, "sort_inst.hip"), []),
+             ("order", os.path.join(CSRC, "order_inst.hip"), [])]
     for tag, name in ELEMS:
         defs = ["-DCUMM_ELEM=%s" % tag, "-DCUMM_NAME=%s" % name]
         units.append(("rowgemm_" + name, os.path.join(CSRC, "rowgemm_inst.hip"), defs))

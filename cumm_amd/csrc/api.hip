@@ -1449,6 +1449,49 @@ int cumm_hip_pair_lists(const int32_t *indices, int kv, int n, int32_t *pair_in,
   return CUMM_HIP_OK;
 }
 
+// ---- masks, order and tables by position
+size_t cumm_hip_order_pairs_workspace(const CummHipOrderSide *sides, int n_sides, int kv) {
+  if (!sides || n_sides < 1 || n_sides > 2 || kv < 1 || kv > kMaxKernelVolume) return 0;
+  size_t bytes = 0;
+  for (int i = 0; i < n_sides; ++i) bytes += order_pairs_workspace_bytes(sides[i].n, (kv + 31) / 32);
+  return bytes;
+}
+
+int cumm_hip_order_pairs(const CummHipOrderSide *sides, int n_sides, const int32_t *ksize, void *workspace,
+                         size_t workspace_bytes, void *stream) {
+  if (!sides || !ksize || n_sides < 1 || n_sides > 2) return fail(CUMM_HIP_EINVAL, "one or two tables");
+  const int64_t kv = (int64_t)ksize[0] * ksize[1] * ksize[2];
+  if (ksize[0] < 1 || ksize[1] < 1 || ksize[2] < 1 || kv > kMaxKernelVolume)
+    return fail(CUMM_HIP_EINVAL, "kernel volume must be 1..%d", kMaxKernelVolume);
+  OrderPairsSide s[2];
+  bool any = false;
+  for (int i = 0; i < n_sides; ++i) {
+    const CummHipOrderSide &d = sides[i];
+    if (d.n < 0) return fail(CUMM_HIP_EINVAL, "bad arguments");
+    // (the entries are fetched through a 32-bit descriptor whose upper half means "absent")
+    if (kv * d.n * 4 >= (int64_t)1 << 31) return fail(CUMM_HIP_ERUNTIME, "your data exceed int32 range.");
+    if (d.n > 0 && (!d.indices || !d.sorted_mask || !d.argsort || !d.by_position))
+      return fail(CUMM_HIP_EINVAL, "indices, sorted_mask, argsort and by_position must not be empty");
+    if (d.n > 0 && (d.by_position == d.indices || d.by_position_reversed == d.indices))
+      return fail(CUMM_HIP_EINVAL, "by_position must not be the table itself");
+    any = any || d.n > 0;
+    s[i].indices = d.indices; s[i].n = d.n; s[i].sorted = d.sorted_mask; s[i].order = d.argsort;
+    s[i].by_pos = d.by_position; s[i].by_pos_rev = d.by_position_reversed;
+    s[i].hint_slot = d.n > 0 ? light_hint_slot_ptr(d.sorted_mask) : nullptr;
+  }
+  if (!any) return CUMM_HIP_OK;
+  // (the two tables' hints may hash to one slot: the second one's then stand)
+  if (n_sides == 2 && s[0].hint_slot == s[1].hint_slot) s[0].hint_slot = nullptr;
+  const size_t need = cumm_hip_order_pairs_workspace(sides, n_sides, (int)kv);
+  if (!workspace || workspace_bytes < need) return fail(CUMM_HIP_ERUNTIME, "workspace at least %zu bytes.", need);
+  if (reinterpret_cast<uintptr_t>(workspace) & 255u) return fail(CUMM_HIP_EINVAL, "workspace must be 256-byte aligned");
+  int32_t *status = nullptr;
+  if (int rc = async_status_ptr(&status)) return rc;
+  const hipError_t e = launch_order_pairs(s, n_sides, (int)kv, ksize, workspace, status + 1, reinterpret_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "pair order launch");
+  return CUMM_HIP_OK;
+}
+
 // ---- weight gradients of the per-offset convolution, all offsets in one launch
 static bool wgrad_pairs_args(const int32_t *counts, int lists, int K, int C) {
   if (!counts || lists < 1 || lists > kWgradPairsMaxLists || K <= 0 || C <= 0 || K % 8 || C % 8) return false;

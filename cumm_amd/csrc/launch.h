@@ -140,6 +140,19 @@ hipError_t launch_light_prefix(const uint32_t *sorted, int n, uint32_t filter, i
 hipError_t launch_sort_by_mask(const uint32_t *mask, int n, uint32_t filter, uint32_t *sorted, int32_t *argsort,
                                void *workspace, int32_t *give_ups, int32_t *hint_slot, int order, hipStream_t s);
 
+// masks, their order, masks and table(s) in that order (order_inst.hip); up to two tables at once
+struct OrderPairsSide {
+  const int32_t *indices;      // [kv, n]
+  int32_t n;
+  uint32_t *sorted;            // [n, words]
+  int32_t *order;              // [n]
+  int32_t *by_pos, *by_pos_rev;   // [kv, n]; by_pos_rev[kv - 1 - k] = by_pos[k], or NULL
+  int32_t *hint_slot;
+};
+size_t order_pairs_workspace_bytes(int n, int words);      // per table
+hipError_t launch_order_pairs(const OrderPairsSide *sides, int n_sides, int kv, const int32_t *ksize, void *workspace,
+                              int32_t *give_ups, hipStream_t s);
+
 // per-offset lists of (input row, output row) out of a pair table [kv, n] (pairs_inst.hip)
 struct PairListsParams {
   const int32_t *indices;   // [kv, n]: input row of output o at offset k, -1 = none

@@ -1,0 +1,487 @@
+// From finished pair tables to what the mask-based kernels read: the masks, an order of the positions
+// in which a tile's masks share their bits, the masks and the table in that order, and the launch
+// hints - for one table or for the two of a strided layer in the same launches.  (The reference's
+// callers take masks and sort from spconv, cumm/conv/main_real_spconv.py:91-145; its iterator forms
+// the table's index per access, cumm/conv/sparse_iters.py:280-357.)
+//
+// Any order is a valid input of the convolution kernels; it decides only how many kernel offsets a tile
+// of 64 or 128 positions has in the OR of its masks, which is what a tile costs.  This one needs two
+// radix passes of nine bits, because its key has 18 bits:
+//   * one mask word: ascending number of offsets, then ascending value as a rank among the words with
+//     that many bits (combinatorial number system), exact up to five offsets (101 584 words of 27
+//     bits), the rank scaled into an equal share of what is left of the 18 bits above that.  The
+//     tiles' offsets add up to what the full 32-bit sort by count and value gives (45 114 against
+//     45 113 at 1 M voxels), which needs four passes.
+//   * several words: a Gray code of the twelve outer planes of the kernel (is there a neighbour with
+//     the lowest, second, second last, last index along z, y, x), then six bits of hash.  With
+//     hundreds of offsets hardly two masks are equal; what neighbours in the order share is the side
+//     on which their neighbours lie.  5 x 5 x 5 on 120 k voxels: 49 k (tile, offset) steps against 87 k in
+//     the order by count and hash.
+// Chain of kernels: clear - masks, keys and both histograms - two passes - position.  The passes are the
+// single-sweep kind (ticket, ranks by ballot, look-back, scatter; stable); they are bound by their
+// dependent round trips at 10^5 positions and by memory at 10^6.  The position kernel fetches only the
+// entries whose bit is set (one in twenty of a sparse cloud's) and writes -1 for the rest.
+// Measured (kernel times): the tables of a frame of 120 k voxels - submanifold and stride 2, 326 k output
+// sites - 125 us in ten launches; with masks by atomics, a sort each and a gather of every entry it
+// was 305 us in 27.
+#include <cstring>
+
+#include "launch.h"
+#include "lds_dma.h"
+
+namespace cummhip {
+
+namespace {
+
+constexpr int kDigit = 9, kDigitBins = 1 << kDigit;      // 512
+constexpr int kKeyBits = 2 * kDigit;
+constexpr int kPassThreads = 1024, kPassWaves = kPassThreads / 64;
+constexpr int kHistCopies = 8;                            // spread of the histogram atomics
+constexpr int kExact = 5;                                 // offsets up to which a one-word key is exact
+constexpr uint32_t kAggregate = 1u << 30, kInclusive = 2u << 30, kCount = (1u << 30) - 1u;
+constexpr int kSpins = 1 << 20;                           // (about a second)
+constexpr int kPosOffsets = 16;                            // offsets per workgroup of the position kernel
+
+struct Side {
+  const int32_t *indices;      // [kv, n]
+  int32_t n, chunks;
+  uint32_t *raw;               // [n, words] masks by row
+  uint32_t *keys;              // [n]
+  int32_t *tmp_rows;           // [n] after the first pass
+  uint16_t *tmp_high;          // [n]
+  uint32_t *hist;              // [2][kHistCopies][kDigitBins]
+  uint32_t *state;             // [2][chunks][kDigitBins] look-back words
+  uint32_t *tickets;           // [2]
+  uint32_t *sorted;            // [n, words]
+  int32_t *order;              // [n]
+  int32_t *by_pos, *by_pos_rev;   // [kv, n]; the second, with its offsets reversed, may be NULL
+  int32_t *hint_slot;          // or NULL
+};
+
+struct OrderParams {
+  Side side[2];
+  int32_t sides, kv, words, pass;
+  int32_t *give_ups;
+  uint32_t base[kExact + 2];   // first key of the words with c offsets; [kExact + 1]: of those with more
+  uint32_t share;              // keys per number of offsets above kExact
+  float per_word[33];          // share / number of words with c offsets, c > kExact
+  // planes[i]: the offsets of outer plane i (several words)
+  uint32_t planes[12][4];
+  uint32_t filter;
+};
+
+__global__ __launch_bounds__(256) void order_clear_kernel(const OrderParams p) {
+  const int i0 = blockIdx.x * 256 + threadIdx.x, step = gridDim.x * 256;
+  for (int s = 0; s < p.sides; ++s) {
+    const Side &d = p.side[s];
+    for (int i = i0; i < 2 * kHistCopies * kDigitBins; i += step) d.hist[i] = 0u;
+    for (int i = i0; i < 2 * d.chunks * kDigitBins; i += step) d.state[i] = 0u;
+    if (i0 < 2) d.tickets[i0] = 0u;
+    if (i0 < 8 && d.hint_slot != nullptr)   // names no array yet; the two counts start at "everything" / "nothing"
+      d.hint_slot[i0] = i0 == 4 ? (d.n / 128) * 128 : (i0 == 5 ? ((d.n + 63) / 64) * 64 : 0);
+  }
+}
+
+// rank of a word among those with as many bits, ascending value: sum of C(position of the i-th bit, i)
+__device__ __forceinline__ uint32_t word_key(const OrderParams &p, uint32_t m) {
+  const int c = __builtin_popcount(m);
+  if (c <= kExact) {
+    uint32_t rank = 0, rest = m;
+#pragma unroll
+    for (int i = 1; i <= kExact; ++i) {
+      if (rest == 0u) break;
+      const uint32_t b = (uint32_t)__builtin_ctz(rest);
+      rest &= rest - 1u;
+      uint32_t v = b;                                    // C(b, i)
+      if (i >= 2) v = v * (b - 1u) / 2u;
+      if (i >= 3) v = v * (b - 2u) / 3u;
+      if (i >= 4) v = v * (b - 3u) / 4u;
+      if (i >= 5) v = v * (b - 4u) / 5u;
+      rank += b >= (uint32_t)i ? v : 0u;
+    }
+    return p.base[c] + rank;
+  }
+  // more offsets: the rank in floating point (its leading digits are all that is kept)
+  float rank = 0.0f;
+  uint32_t rest = m;
+  int i = 1;
+  while (rest != 0u) {
+    const float b = (float)__builtin_ctz(rest);
+    rest &= rest - 1u;
+    float v = b >= (float)i ? 1.0f : 0.0f;
+    for (int t = 0; t < i; ++t) v *= (b - (float)t) / (float)(t + 1);
+    rank += v;
+    ++i;
+  }
+  const uint32_t at = (uint32_t)(rank * p.per_word[c]);
+  return p.base[kExact + 1] + (uint32_t)(c - kExact - 1) * p.share + (at < p.share ? at : p.share - 1u);
+}
+
+__device__ __forceinline__ uint32_t words_key(const OrderParams &p, const uint32_t *w) {
+  uint32_t planes = 0u, h = 0u;
+#pragma unroll
+  for (int i = 0; i < 12; ++i) {
+    const uint32_t any = (w[0] & p.planes[i][0]) | (w[1] & p.planes[i][1]) | (w[2] & p.planes[i][2]) | (w[3] & p.planes[i][3]);
+    planes |= any ? 1u << i : 0u;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) h = (h ^ w[i]) * 0x9E3779B1u;
+  // the place of `planes` in the Gray code
+  planes ^= planes >> 1;
+  planes ^= planes >> 2;
+  planes ^= planes >> 4;
+  planes ^= planes >> 8;
+  return (planes << (kKeyBits - 12)) | (h >> (32 - (kKeyBits - 12)));
+}
+
+// side and index inside it of a workgroup, when side 0 has `first` workgroups
+__device__ __forceinline__ int side_of(int first, int *block) {
+  const int s = *block >= first ? 1 : 0;
+  *block -= s ? first : 0;
+  return s;
+}
+
+// One position per lane: its mask out of the table (every row read coalesced, kv independent loads), its
+// key, and the digits of the key into the histograms of both passes.
+template <int WORDS>
+__global__ __launch_bounds__(256) void order_masks_kernel(const OrderParams p) {
+  __shared__ uint32_t hist[2][kDigitBins];
+  const int t = threadIdx.x, lane = t & 63;
+  int block = blockIdx.x;
+  const Side &d = p.side[side_of((p.side[0].n + 255) / 256, &block)];
+  for (int i = t; i < 2 * kDigitBins; i += 256) (&hist[0][0])[i] = 0u;
+  const int o = block * 256 + t;
+  const bool on = o < d.n;
+  uint32_t w[4] = {0u, 0u, 0u, 0u};
+  const int32_t *col = d.indices + (on ? o : 0);
+#pragma unroll
+  for (int q = 0; q < WORDS; ++q) {
+    const int hi = p.kv - 32 * q < 32 ? p.kv - 32 * q : 32;
+    for (int b0 = 0; b0 < hi; b0 += 8) {
+      int v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = col[(int64_t)(32 * q + (b0 + u < hi ? b0 + u : 0)) * d.n];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) w[q] |= b0 + u < hi && v[u] >= 0 ? 1u << (b0 + u) : 0u;
+    }
+  }
+  const uint32_t key = WORDS == 1 ? word_key(p, w[0]) : words_key(p, w);
+  if (on) {
+#pragma unroll
+    for (int q = 0; q < WORDS; ++q) d.raw[(int64_t)o * WORDS + q] = w[q];
+    d.keys[o] = key;
+  }
+  __syncthreads();
+  // most waves of a sparse cloud hold one key: one add for all lanes
+  const unsigned long long live = __ballot(on);
+  if (live != 0ull) {
+    const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)key);
+    if (__ballot(on && key == first) == live) {
+      if (lane < 2) atomicAdd(&hist[lane][(first >> (lane * kDigit)) & (kDigitBins - 1)], (uint32_t)__popcll(live));
+    } else if (on) {
+      atomicAdd(&hist[0][key & (kDigitBins - 1)], 1u);
+      atomicAdd(&hist[1][key >> kDigit], 1u);
+    }
+  }
+  __syncthreads();
+  for (int i = t; i < 2 * kDigitBins; i += 256) {
+    const uint32_t c = (&hist[0][0])[i];
+    if (c) atomicAdd(&d.hist[((i >> kDigit) * kHistCopies + (block & (kHistCopies - 1))) * kDigitBins + (i & (kDigitBins - 1))], c);
+  }
+}
+
+// One pass over one digit (0: the low one, rows in ascending order to tmp; 1: the high one, tmp to
+// order).  A workgroup takes the next chunk by ticket (its predecessors have then started), ranks
+// its keys per digit in position order, publishes its counts, adds up those of the chunks before it and
+// scatters.  Words carry flag and value: relaxed device-scope accesses do.
+template <int ITEMS>
+__global__ __launch_bounds__(kPassThreads) void order_pass_kernel(const OrderParams p) {
+  constexpr int kChunk = kPassThreads * ITEMS;
+  __shared__ uint32_t wave_hist[kPassWaves][kDigitBins];
+  __shared__ uint32_t bin_base[kDigitBins];
+  __shared__ uint32_t wave_sum[8];
+  __shared__ int chunk_of_block;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  int block = blockIdx.x;
+  const Side &d = p.side[side_of(p.side[0].chunks, &block)];
+  const bool low = p.pass == 0;
+  if (t == 0) chunk_of_block = (int)atomicAdd(&d.tickets[p.pass], 1u);
+  // keys per bin of the whole input (thread = bin), while the ticket is on its way
+  uint32_t total = 0;
+  if (t < kDigitBins) {
+#pragma unroll
+    for (int c = 0; c < kHistCopies; ++c) total += d.hist[(p.pass * kHistCopies + c) * kDigitBins + t];
+  }
+  for (int i = t; i < kPassWaves * kDigitBins; i += kPassThreads) (&wave_hist[0][0])[i] = 0u;
+  __syncthreads();
+  const int chunk = chunk_of_block;
+  if (chunk >= d.chunks) return;      // (never: one workgroup per chunk)
+  // wave w owns positions [base, base + 64 ITEMS), item u of lane l is position base + 64 u + l
+  const int64_t base = (int64_t)chunk * kChunk + (int64_t)wave * (64 * ITEMS);
+  uint32_t digit[ITEMS], high[ITEMS];
+  int32_t row[ITEMS];
+  uint32_t rank[ITEMS];
+#pragma unroll
+  for (int u = 0; u < ITEMS; ++u) {
+    const int64_t pos = base + u * 64 + lane;
+    const int64_t at = pos < d.n ? pos : d.n - 1;
+    if (low) {
+      const uint32_t key = d.keys[at];
+      digit[u] = key & (kDigitBins - 1);
+      high[u] = key >> kDigit;
+      row[u] = (int32_t)pos;
+    } else {
+      digit[u] = d.tmp_high[at];
+      row[u] = d.tmp_rows[at];
+    }
+  }
+  // first place of each bin: exclusive prefix over the bins
+  uint32_t incl = total;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t up = (uint32_t)__shfl_up((int)incl, off, 64);
+    if (lane >= off) incl += up;
+  }
+  if (t < kDigitBins && lane == 63) wave_sum[wave] = incl;
+#pragma unroll
+  for (int u = 0; u < ITEMS; ++u) {
+    const bool valid = base + u * 64 + lane < d.n;
+    unsigned long long peers = __ballot(valid);
+#pragma unroll
+    for (int b = 0; b < kDigit; ++b) {
+      const unsigned long long has = __ballot((digit[u] >> b) & 1u);
+      peers &= ((digit[u] >> b) & 1u) ? has : ~has;
+    }
+    const uint32_t before = (uint32_t)__popcll(peers & ((1ull << lane) - 1ull));
+    uint32_t prev = 0;
+    if (valid) prev = wave_hist[wave][digit[u]];
+    __builtin_amdgcn_wave_barrier();
+    if (valid && before == 0) wave_hist[wave][digit[u]] = prev + (uint32_t)__popcll(peers);
+    __builtin_amdgcn_wave_barrier();
+    rank[u] = prev + before;
+  }
+  __syncthreads();
+  if (t < kDigitBins) {
+    uint32_t first = incl - total;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) first += w < wave ? wave_sum[w] : 0u;
+    uint32_t count = 0;
+#pragma unroll
+    for (int w = 0; w < kPassWaves; ++w) {
+      const uint32_t c = wave_hist[w][t];
+      wave_hist[w][t] = count;
+      count += c;
+    }
+    uint32_t *state = d.state + (size_t)p.pass * d.chunks * kDigitBins;
+    __hip_atomic_store(&state[(size_t)chunk * kDigitBins + t], (chunk == 0 ? kInclusive : kAggregate) | count, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+    uint32_t before = 0;
+    if (chunk > 0) {
+      constexpr int kLook = 32;      // words per round trip
+      bool done = false, gave_up = false;
+      int j = chunk - 1, spins = 0;
+      while (!done && !gave_up) {
+        uint32_t sw[kLook];
+#pragma unroll
+        for (int i = 0; i < kLook; ++i)
+          sw[i] = j - i >= 0 ? __hip_atomic_load(&state[(size_t)(j - i) * kDigitBins + t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                             : kInclusive;
+        int taken = 0;
+#pragma unroll
+        for (int i = 0; i < kLook; ++i) {
+          if (!done && taken == i) {
+            const uint32_t flag = sw[i] >> 30;
+            if (flag != 0u) {
+              before += sw[i] & kCount;
+              ++taken;
+              done = flag == 2u;
+            }
+          }
+        }
+        j -= taken;
+        if (!done && taken == 0) {
+          if (++spins > kSpins) gave_up = true;
+          __builtin_amdgcn_s_sleep(1);
+        }
+      }
+      if (gave_up && p.give_ups != nullptr) atomicAdd(p.give_ups, 1);
+      __hip_atomic_store(&state[(size_t)chunk * kDigitBins + t], kInclusive | (before + count), __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    }
+    bin_base[t] = first + before;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < ITEMS; ++u) {
+    if (base + u * 64 + lane < d.n) {
+      const uint32_t dst = bin_base[digit[u]] + wave_hist[wave][digit[u]] + rank[u];
+      if (dst < (uint32_t)d.n) {      // (always, unless a look-back gave up)
+        if (low) {
+          d.tmp_rows[dst] = row[u];
+          d.tmp_high[dst] = (uint16_t)high[u];
+        } else {
+          d.order[dst] = row[u];
+        }
+      }
+    }
+  }
+}
+
+// 256 positions and kPosOffsets offsets per workgroup: masks, table(s) by position, and (offset slice 0)
+// the counts of the launch hints - as sort_finish_kernel, whose remarks on give-ups hold here too: the
+// identity order replaces one that cannot be trusted.
+constexpr int kLight = 3, kHeavy = 10;
+template <int WORDS>
+__global__ __launch_bounds__(256) void order_position_kernel(const OrderParams p) {
+  __shared__ uint32_t half_or[4];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  int block = blockIdx.x;
+  const Side &d = p.side[side_of((p.side[0].n + 255) / 256, &block)];
+  const int pos = block * 256 + t;
+  const bool on = pos < d.n;
+  const bool broken = p.give_ups != nullptr && __hip_atomic_load(p.give_ups, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+  int row = on ? (broken ? pos : d.order[pos]) : -1;
+  const int k0 = blockIdx.y * kPosOffsets;
+  const int word = k0 / 32;
+  const bool have = row >= 0 && row < d.n;
+  const uint32_t mine = have ? d.raw[(int64_t)row * WORDS + word] : 0u;
+  const uint32_t bits = mine >> (k0 & 31);
+  int v[kPosOffsets];
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t *>(d.indices), 0,
+                                                                      (int)((uint32_t)p.kv * (uint32_t)d.n * 4u), 0x00020000);
+#pragma unroll
+  for (int u = 0; u < kPosOffsets; ++u)      // (a clear bit is fetched outside the table: no memory is touched)
+    v[u] = __builtin_amdgcn_raw_buffer_load_b32(rs, (bits >> u) & 1u ? (uint32_t)((k0 + u) * d.n + row) * 4u : 0x80000000u, 0, 0);
+  if (on) {
+#pragma unroll
+    for (int u = 0; u < kPosOffsets; ++u) {
+      if (k0 + u >= p.kv) break;
+      const int e = (bits >> u) & 1u ? v[u] : -1;
+      d.by_pos[(int64_t)(k0 + u) * d.n + pos] = e;
+      if (d.by_pos_rev != nullptr) d.by_pos_rev[(int64_t)(p.kv - 1 - k0 - u) * d.n + pos] = e;
+    }
+    if ((k0 & 31) == 0) d.sorted[(int64_t)pos * WORDS + word] = mine;
+    if (broken && blockIdx.y == 0) d.order[pos] = pos;
+  }
+  if (WORDS > 1 || blockIdx.y != 0 || d.hint_slot == nullptr) return;
+  if (broken) {
+    if (block == 0 && t < 8) d.hint_slot[t] = 0;
+    return;
+  }
+  const uint32_t o = wave_or_dpp(mine);
+  if (lane == 0) half_or[wave] = o;
+  __syncthreads();
+  if (t < 2) {
+    const int run = block * 2 + t;
+    const int c0 = __builtin_popcount(half_or[2 * t]), c1 = __builtin_popcount(half_or[2 * t + 1]);
+    if (run < d.n / 128 && (c0 > kLight || c1 > kLight)) atomicMin(&d.hint_slot[4], run * 128);
+    if (c0 >= kHeavy || c1 >= kHeavy) atomicMin(&d.hint_slot[5], run * 128 + (c0 >= kHeavy ? 0 : 64));
+  }
+  if (block == 0 && t == 0) {
+    const uint64_t a = (uint64_t)d.sorted;
+    d.hint_slot[0] = (int32_t)(uint32_t)a;
+    d.hint_slot[1] = (int32_t)(uint32_t)(a >> 32);
+    d.hint_slot[2] = d.n;
+    d.hint_slot[3] = (int32_t)p.filter;
+    d.hint_slot[6] = 1;
+  }
+}
+
+size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
+// chunks of 4096 positions up to 2^18 (few chunks: a pass is as long as one chunk's chain), 8192 above
+int pass_items(int n) { return n <= (1 << 18) ? 4 : 8; }
+
+}  // namespace
+
+size_t order_pairs_workspace_bytes(int n, int words) {
+  const size_t nn = (size_t)(n > 0 ? n : 1);
+  const size_t chunks = (nn + 4095) / 4096;
+  return up256(4 * nn * words) + 2 * up256(4 * nn) + up256(2 * nn) + up256(4 * 2 * kHistCopies * kDigitBins) +
+         up256(4 * 2 * chunks * kDigitBins) + 256;
+}
+
+hipError_t launch_order_pairs(const OrderPairsSide *sides, int n_sides, int kv, const int32_t *ksize, void *workspace,
+                              int32_t *give_ups, hipStream_t s) {
+  OrderParams p;
+  std::memset(&p, 0, sizeof(p));
+  p.kv = kv; p.words = (kv + 31) / 32; p.give_ups = give_ups;
+  p.filter = kv < 32 ? (1u << kv) - 1u : 0xFFFFFFFFu;
+  char *at = reinterpret_cast<char *>(workspace);
+  auto take = [&](size_t bytes) { char *q = at; at += up256(bytes); return q; };
+  int most = 0;
+  for (int i = 0; i < n_sides; ++i)
+    if (sides[i].n > 0 && sides[i].n > most) most = sides[i].n;
+  const int items = pass_items(most), chunk = kPassThreads * items;
+  for (int i = 0; i < n_sides; ++i) {
+    if (sides[i].n <= 0) continue;
+    Side &d = p.side[p.sides++];
+    const size_t n = (size_t)sides[i].n;
+    d.indices = sides[i].indices; d.n = sides[i].n; d.chunks = (int)((n + chunk - 1) / chunk);
+    d.sorted = sides[i].sorted; d.order = sides[i].order; d.by_pos = sides[i].by_pos; d.by_pos_rev = sides[i].by_pos_rev;
+    d.hint_slot = p.words == 1 ? sides[i].hint_slot : nullptr;
+    char *const begin = at;
+    d.raw = reinterpret_cast<uint32_t *>(take(4 * n * p.words));
+    d.keys = reinterpret_cast<uint32_t *>(take(4 * n));
+    d.tmp_rows = reinterpret_cast<int32_t *>(take(4 * n));
+    d.tmp_high = reinterpret_cast<uint16_t *>(take(2 * n));
+    d.hist = reinterpret_cast<uint32_t *>(take(4 * 2 * kHistCopies * kDigitBins));
+    d.state = reinterpret_cast<uint32_t *>(take(4 * 2 * (size_t)d.chunks * kDigitBins));
+    d.tickets = reinterpret_cast<uint32_t *>(take(256));
+    at = begin + order_pairs_workspace_bytes(d.n, p.words);
+  }
+  if (p.sides == 0) return hipSuccess;
+  if (p.words == 1) {
+    // words of kv bits with c offsets: C(kv, c)
+    double choose = 1.0;
+    uint32_t next = 0;
+    for (int c = 0; c <= kv; ++c) {
+      if (c <= kExact) {
+        p.base[c] = next;
+        next += (uint32_t)choose;
+      }
+      if (c == (kExact < kv ? kExact : kv)) {
+        for (int e = c + 1; e <= kExact + 1; ++e) p.base[e] = next;
+        p.share = kv > kExact ? ((1u << kKeyBits) - next) / (uint32_t)(kv - kExact) : 1u;
+      }
+      if (c > kExact) p.per_word[c] = (float)((double)p.share / choose);
+      choose = choose * (kv - c) / (c + 1);
+    }
+  } else {
+    for (int k = 0; k < kv; ++k) {
+      const int i[3] = {k / (ksize[1] * ksize[2]), (k / ksize[2]) % ksize[1], k % ksize[2]};
+      for (int a = 0; a < 3; ++a) {
+        // the two lowest and the two highest planes of an axis (an axis of three has its outer ones only)
+        const int last = ksize[a] - 1, mid = last / 2;
+        const int plane = last == 0 || i[a] == mid ? -1 : (i[a] < mid ? (i[a] == 0 ? 0 : 1) : (i[a] == last ? 3 : 2));
+        if (plane >= 0) p.planes[a * 4 + plane][k / 32] |= 1u << (k % 32);
+      }
+    }
+  }
+  int blocks = 0, chunks = 0;
+  for (int i = 0; i < p.sides; ++i) {
+    blocks += (p.side[i].n + 255) / 256;
+    chunks += p.side[i].chunks;
+  }
+  const int clear = 2 * chunks * kDigitBins / 256;
+  hipLaunchKernelGGL(order_clear_kernel, dim3(clear > 1024 ? 1024 : clear), dim3(256), 0, s, p);
+  switch (p.words) {
+  case 1: hipLaunchKernelGGL(order_masks_kernel<1>, dim3(blocks), dim3(256), 0, s, p); break;
+  case 2: hipLaunchKernelGGL(order_masks_kernel<2>, dim3(blocks), dim3(256), 0, s, p); break;
+  case 3: hipLaunchKernelGGL(order_masks_kernel<3>, dim3(blocks), dim3(256), 0, s, p); break;
+  default: hipLaunchKernelGGL(order_masks_kernel<4>, dim3(blocks), dim3(256), 0, s, p); break;
+  }
+  for (p.pass = 0; p.pass < 2; ++p.pass) {
+    if (items == 4) hipLaunchKernelGGL(order_pass_kernel<4>, dim3(chunks), dim3(kPassThreads), 0, s, p);
+    else hipLaunchKernelGGL(order_pass_kernel<8>, dim3(chunks), dim3(kPassThreads), 0, s, p);
+  }
+  const dim3 grid(blocks, (kv + kPosOffsets - 1) / kPosOffsets);
+  switch (p.words) {
+  case 1: hipLaunchKernelGGL(order_position_kernel<1>, grid, dim3(256), 0, s, p); break;
+  case 2: hipLaunchKernelGGL(order_position_kernel<2>, grid, dim3(256), 0, s, p); break;
+  case 3: hipLaunchKernelGGL(order_position_kernel<3>, grid, dim3(256), 0, s, p); break;
+  default: hipLaunchKernelGGL(order_position_kernel<4>, grid, dim3(256), 0, s, p); break;
+  }
+  return hipGetLastError();
+}
+
+}  // namespace cummhip

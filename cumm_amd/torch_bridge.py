@@ -201,7 +201,6 @@ class SparseConvGeometry:
         self._tensors = {}
         lib, arr3 = _capi.lib(), ctypes.c_int32 * 3
         shape, ks, pad, dil = (arr3(*[int(v) for v in a]) for a in (spatial_shape, ksize, padding, dilation))
-        masks = words == 1       # (the builders make masks of one word)
         if self.subm:
             pairs._check_odd_ksize(ksize)
             self.n_out = n_out = n_in
@@ -209,8 +208,8 @@ class SparseConvGeometry:
             self._allocate()
             ws = _bytes(lib.cumm_hip_subm_pairs_workspace(n_in), dev)
             _capi.check(lib.cumm_hip_subm_pairs(
-                coords.data_ptr(), n_in, shape, ks, dil, self._ptr["indices_fwd"], self._ptr["indices_bwd"],
-                self._ptr["raw_fwd"] if masks else None, self._ptr["raw_bwd"] if masks else None, ws.data_ptr(), ws.numel(), s))
+                coords.data_ptr(), n_in, shape, ks, dil, self._ptr["indices_fwd"], self._ptr["indices_bwd"], None, None,
+                ws.data_ptr(), ws.numel(), s))
         else:
             st = arr3(*[int(v) for v in stride])
             geo = (shape, ks, st, pad, dil)
@@ -227,17 +226,21 @@ class SparseConvGeometry:
             self._allocate()
             _capi.check(lib.cumm_hip_conv_pairs_fill(
                 coords.data_ptr(), n_in, int(batch_size), *geo, n_out, self.out_coords.data_ptr(), self._ptr["indices_fwd"],
-                self._ptr["indices_bwd"], self._ptr["raw_fwd"] if masks else None, self._ptr["raw_bwd"] if masks else None,
-                ws.data_ptr(), ws.numel(), s))
-        for side, n in (("fwd", n_out), ("bwd", n_in)):
-            if side == "fwd" or not self.subm:
-                self._sort(side, n)
-            # the pair tables once more in the order of the sorted positions: what forward and
-            # backward-input read (a tile's entries for one offset are then consecutive in memory);
-            # backward-weight keeps the table by row
-            _capi.check(lib.cumm_hip_pairs_by_position(self._ptr["indices_" + side], self._ptr["order_" + side], kv, n,
-                                                       self._ptr["indices_%s_pos" % side], s))
-        if not masks:
+                self._ptr["indices_bwd"], None, None, ws.data_ptr(), ws.numel(), s))
+        # masks, an order of the positions by them, and the pair tables once more in that order: what
+        # forward and backward-input read (a tile's entries for one offset are then consecutive in
+        # memory); backward-weight keeps the table by row
+        p = self._ptr
+        sides = (_capi.OrderSide * 2)()
+        for d, side, n in ((sides[0], "fwd", n_out), (sides[1], "bwd", n_in)):
+            d.indices, d.n = p["indices_" + side], n
+            d.sorted_mask, d.argsort, d.by_position = p["mask_" + side], p["order_" + side], p["indices_%s_pos" % side]
+        count = 2
+        if self.subm:      # (one order serves both; the backward table is the forward one with its offsets reversed)
+            sides[0].by_position_reversed, count = p["indices_bwd_pos"], 1
+        ws = _bytes(lib.cumm_hip_order_pairs_workspace(sides, count, kv), dev)
+        _capi.check(lib.cumm_hip_order_pairs(sides, count, ks, ws.data_ptr(), ws.numel(), s))
+        if words > 1:
             self._make_lists()
 
     def _allocate(self) -> None:
@@ -245,11 +248,10 @@ class SparseConvGeometry:
         mask = [self.n_out] if words == 1 else [n_out, words]
         spec = [("indices_fwd", [kv, n_out], tv.int32), ("indices_bwd", [kv, n_in], tv.int32),
                 ("indices_fwd_pos", [kv, n_out], tv.int32), ("indices_bwd_pos", [kv, n_in], tv.int32),
-                ("mask_fwd", mask, tv.uint32), ("order_fwd", [n_out], tv.int32), ("raw_fwd", mask, tv.uint32)]
+                ("mask_fwd", mask, tv.uint32), ("order_fwd", [n_out], tv.int32)]
         mask = [n_in] if words == 1 else [n_in, words]
         if not self.subm:
             spec += [("mask_bwd", mask, tv.uint32), ("order_bwd", [n_in], tv.int32)]
-        spec.append(("raw_bwd", mask, tv.uint32))
         self._spec, at = {}, 0
         for name, dims, dtype in spec:
             self._spec[name] = (at, dims, dtype)
@@ -263,24 +265,6 @@ class SparseConvGeometry:
         if self.subm:      # the forward masks serve the backward-input pass, bit-reversed in the kernel
             for name in ("mask", "order"):
                 self._spec[name + "_bwd"], self._ptr[name + "_bwd"] = self._spec[name + "_fwd"], self._ptr[name + "_fwd"]
-
-    def _sort(self, side: str, n: int) -> None:
-        lib, p, s = _capi.lib(), self._ptr, self._stream
-        if self.words > 1:
-            # the builders give no masks for these volumes: made from the tables, sorted by offset count
-            # and word pattern
-            _capi.check(lib.cumm_hip_masks_from_pairs(p["indices_" + side], self.kv, n, p["raw_" + side], s))
-            ws = _bytes(lib.cumm_hip_sort_by_mask_words_workspace(n), self._device)
-            _capi.check(lib.cumm_hip_sort_by_mask_words(p["raw_" + side], n, self.words, p["mask_" + side], p["order_" + side],
-                                                        ws.data_ptr(), ws.numel(), s))
-            return
-        # (a mask has one bit per kernel offset: a filter of that width spares the sort the passes over
-        # the bits above it; the library's order by offset count where the masks leave room for the
-        # count: same rows, lighter tiles, and the few many-offset tiles in a short run at the end)
-        bits = (1 << self.kv) - 1 if self.kv < 32 else 0xFFFFFFFF
-        ws = _bytes(lib.cumm_hip_sort_by_mask_workspace(n), self._device)
-        _capi.check(lib.cumm_hip_sort_by_mask_ordered(p["raw_" + side], n, bits, 1 if self.kv <= 27 else 0, p["mask_" + side],
-                                                      p["order_" + side], ws.data_ptr(), ws.numel(), s))
 
     def _make_lists(self) -> None:
         """The per-offset pair lists of backward-weight; their counts come to the host."""

@@ -362,6 +362,28 @@ size_t cumm_hip_pair_lists_workspace(int kv, int n);
 int cumm_hip_pair_lists(const int32_t *indices, int kv, int n, int32_t *pair_in, int32_t *pair_out, int32_t *counts,
                         void *workspace, size_t workspace_bytes, void *stream);
 
+/* From finished pair tables to what the forward and backward-input kernels read, for one table or for the
+ * two of a strided layer: masks (bit r of word w set wherever indices[32 w + r][o] >= 0, ceil(kv / 32)
+ * words), an order of the positions by them, and the masks and the table in that order:
+ *   sorted_mask [n, words], argsort [n], by_position[k][pos] = indices[k][argsort[pos]] ([kv, n]),
+ *   by_position_reversed[kv - 1 - k] = by_position[k] (NULL = not wanted: the backward table of a
+ *   submanifold layer).
+ * Positions come in ascending number of kernel offsets (one word) or grouped by the sides on which
+ * their neighbours lie (several); equal masks lie together; the order repeats from run to run.  The
+ * launch hints of the sorted masks are left as cumm_hip_sort_by_mask_ordered leaves them.  Two radix
+ * passes for all tables together, where cumm_hip_sort_by_mask_ordered, whose order is exact, takes four
+ * for each.  workspace: cumm_hip_order_pairs_workspace bytes, 256-byte aligned. */
+typedef struct CummHipOrderSide {
+  const int32_t *indices;      /* [kv, n] */
+  int32_t n;
+  uint32_t *sorted_mask;
+  int32_t *argsort;
+  int32_t *by_position, *by_position_reversed;
+} CummHipOrderSide;
+size_t cumm_hip_order_pairs_workspace(const CummHipOrderSide *sides, int n_sides, int kv);
+int cumm_hip_order_pairs(const CummHipOrderSide *sides, int n_sides, const int32_t *ksize, void *workspace,
+                         size_t workspace_bytes, void *stream);
+
 /* Backward-weight of the per-offset convolution for all offsets at once:
  *   dw[:, r, :] = sum over i < counts[r] of dout[pair_out[r][i]]^T inp[pair_in[r][i]]
  * dw [K, lists, C], dout [rows_out, K], inp [rows_in, C] (f16 / bf16, fp32 sums in a fixed order, rounded

@@ -1,0 +1,97 @@
+"""cumm_hip_order_pairs (order_inst.hip): masks, order, tables by position and launch hints of finished pair
+tables, against the host builders - sizes around the chunks and tiles, one and two tables, one to
+four mask words, kernel volumes from 1 to 125."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import helpers as H
+from cumm_amd import _capi, pairs
+from cumm_amd import tensorview as tv
+
+pytestmark = pytest.mark.gpu
+
+
+def _table(rng, kv, n, density):
+    t = np.where(rng.random((kv, n)) < density, rng.integers(0, max(n, 1), size=(kv, n)), -1).astype(np.int32)
+    t[kv // 2, : n // 2] = np.arange(n // 2)
+    return t
+
+
+def _order(tables, ksize, reverse):
+    lib, kv = _capi.lib(), tables[0].shape[0]
+    words = (kv + 31) // 32
+    sides, keep, outs = (_capi.OrderSide * 2)(), [], []
+    for s, t in zip(sides, tables):
+        n = t.shape[1]
+        d = H.dev(t, "i32")
+        o = {"mask": tv.empty([n, words], tv.uint32, 0), "order": tv.empty([n], tv.int32, 0), "pos": tv.empty([kv, n], tv.int32, 0),
+             "rev": tv.empty([kv, n], tv.int32, 0)}
+        s.indices, s.n, s.sorted_mask, s.argsort = d.byte_pointer(), n, o["mask"].byte_pointer(), o["order"].byte_pointer()
+        s.by_position = o["pos"].byte_pointer()
+        s.by_position_reversed = o["rev"].byte_pointer() if reverse else None
+        keep.append(d)
+        outs.append(o)
+    need = int(lib.cumm_hip_order_pairs_workspace(sides, len(tables), kv))
+    ws = H.dev(np.full(need, 0xA5, np.uint8), "u8")
+    _capi.check(lib.cumm_hip_order_pairs(sides, len(tables), (ctypes.c_int32 * 3)(*ksize), ws.byte_pointer(), ws.nbytes, 0))
+    _capi.check(lib.cumm_hip_device_synchronize())
+    return [{k: H.host(v) for k, v in o.items()} for o in outs], outs
+
+
+@pytest.mark.parametrize("ksize", [(3, 3, 3), (1, 1, 1), (2, 2, 2), (4, 4, 2), (3, 3, 5), (5, 5, 5)])
+@pytest.mark.parametrize("n,n2", [(1, 0), (63, 64), (256, 257), (4096, 4097), (9000, 130), (270000, 1000)])
+def test_masks_order_and_tables(ksize, n, n2):
+    kv = int(np.prod(ksize))
+    if n > 100000 and kv > 40:
+        n = 40000      # (the same branches with a smaller table)
+    print("case order", ksize, n, n2, flush=True)
+    rng = np.random.default_rng(n + kv)
+    tables = [_table(rng, kv, n, 0.05 if kv > 8 else 0.4)] + ([_table(rng, kv, n2, 0.3)] if n2 else [])
+    got, dev = _order(tables, ksize, reverse=n2 == 0 or n == 256)
+    for t, g, d in zip(tables, got, dev):
+        m = pairs.masks_from_pairs(t)
+        order = g["order"]
+        assert np.array_equal(np.sort(order), np.arange(t.shape[1]))
+        np.testing.assert_array_equal(g["mask"], m[order])
+        np.testing.assert_array_equal(g["pos"], pairs.pairs_by_position(t, order))
+        if n2 == 0 or n == 256:
+            np.testing.assert_array_equal(g["rev"], g["pos"][::-1])
+        if m.shape[1] == 1:
+            s = g["mask"][:, 0]
+            count = np.array([bin(int(v)).count("1") for v in s])
+            assert np.all(np.diff(count) >= 0)
+            light = count[1:] <= 5
+            same = np.diff(count) == 0
+            assert np.all(np.diff(s.astype(np.int64))[light & same] >= 0)      # exact up to five offsets
+            # stable: equal words of up to five offsets in row order
+            eq = (np.diff(s.astype(np.int64)) == 0) & light
+            assert np.all(np.diff(order)[eq] > 0)
+            bits = (1 << kv) - 1 if kv < 32 else 0xFFFFFFFF
+            if t is tables[-1] or t.shape[1] != tables[-1].shape[1]:
+                hints = pairs.hints_device(d["mask"].view([t.shape[1]]), bits)
+                if hints != (-1, -1):      # (the two arrays' slots may coincide: then the second one's stand)
+                    assert hints == (pairs.light_prefix(s, bits, 3), pairs.heavy_from(s, bits))
+    again, _ = _order(tables, ksize, reverse=False)
+    for g, a in zip(got, again):
+        np.testing.assert_array_equal(g["order"], a["order"])
+
+
+def test_a_tile_has_as_few_offsets_as_in_the_exact_order():
+    """What the order is for: the offsets of all tiles of 64, on a cloud, against the 32-bit sort by count and
+    value (one word) and against the order by count and hash (5 x 5 x 5)."""
+    coords, grid = H.small_cloud(5, 6000)
+    for ksize in ((3, 3, 3), (5, 5, 5)):
+        host = pairs.subm_pairs(coords, grid, ksize)
+        (g,), _ = _order([host.indices_fwd], ksize, reverse=False)
+        m = pairs.masks_from_pairs(host.indices_fwd)
+        other = pairs.sort_by_mask(m[:, 0], (1 << 27) - 1, by_offset_count=True)[1] if m.shape[1] == 1 else pairs.sort_by_mask_words(m)[1]
+
+        def steps(order):
+            s = m[order]
+            pad = np.zeros(((len(s) + 63) // 64 * 64, s.shape[1]), np.uint32)
+            pad[: len(s)] = s
+            w = np.bitwise_or.reduce(pad.reshape(-1, 64, s.shape[1]), axis=1)
+            return sum(bin(int(v)).count("1") for v in w.ravel())
+        assert steps(g["order"]) <= steps(other) * 1.01 + 2
