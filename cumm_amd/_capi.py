@@ -131,6 +131,7 @@ SYMBOLS = {
     "cumm_hip_relu_backward": (C.c_int, [_VP, _VP, _VP, C.c_size_t, C.c_int, _VP]),
     "cumm_hip_column_sum_workspace": (C.c_size_t, [C.c_int64, C.c_int]),
     "cumm_hip_column_sum": (C.c_int, [_VP, _VP, C.c_int64, C.c_int, C.c_int, _VP, C.c_size_t, _VP]),
+    "cumm_hip_relu_backward_sums": (C.c_int, [_VP, _VP, _VP, _VP, C.c_int64, C.c_int, C.c_int, _VP, C.c_size_t, _VP]),
     "cumm_hip_gather_rows": (C.c_int, [_VP, _VP, _VP, C.c_int, C.c_int, C.c_size_t, _VP]),
     "cumm_hip_scatter_add_rows": (C.c_int, [_VP, _VP, _VP, C.c_int, C.c_int, C.c_int, C.c_int, _VP]),
 }

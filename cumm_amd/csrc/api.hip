@@ -1677,8 +1677,8 @@ size_t cumm_hip_column_sum_workspace(int64_t rows, int channels) {
   return sizeof(float) * (size_t)column_sum_blocks(rows, channels) * (size_t)channels;
 }
 
-int cumm_hip_column_sum(void *dst, const void *src, int64_t rows, int channels, int dtype, void *workspace,
-                        size_t workspace_bytes, void *stream) {
+static int column_sum_checked(void *dst, const void *src, const void *out, void *gated, int64_t rows, int channels, int dtype,
+                              void *workspace, size_t workspace_bytes, void *stream) {
   if (rows < 0 || channels < 0) return fail(CUMM_HIP_EINVAL, "bad arguments");
   if (!is_float16_like(dtype)) return fail(CUMM_HIP_EINVAL, "dtype must be f16 or bf16");
   if (channels % 8 || channels > 2048) return fail(CUMM_HIP_EINVAL, "channels must be a multiple of 8, at most 2048");
@@ -1689,10 +1689,23 @@ int cumm_hip_column_sum(void *dst, const void *src, int64_t rows, int channels, 
   if (reinterpret_cast<uintptr_t>(workspace) & 3u) return fail(CUMM_HIP_EINVAL, "workspace must be 4-byte aligned");
   ColumnSumParams p;
   std::memset(&p, 0, sizeof(p));
-  p.dst = dst; p.src = src; p.partial = reinterpret_cast<float *>(workspace); p.rows = rows; p.channels = channels;
+  p.dst = dst; p.src = src; p.out = out; p.gated = gated;
+  p.partial = reinterpret_cast<float *>(workspace); p.rows = rows; p.channels = channels;
   hipError_t e = launch_column_sum(p, dtype == CUMM_HIP_BF16, reinterpret_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "column_sum launch");
   return CUMM_HIP_OK;
+}
+
+int cumm_hip_column_sum(void *dst, const void *src, int64_t rows, int channels, int dtype, void *workspace,
+                        size_t workspace_bytes, void *stream) {
+  return column_sum_checked(dst, src, nullptr, nullptr, rows, channels, dtype, workspace, workspace_bytes, stream);
+}
+
+int cumm_hip_relu_backward_sums(void *gated, void *sums, const void *grad, const void *out, int64_t rows, int channels, int dtype,
+                                void *workspace, size_t workspace_bytes, void *stream) {
+  if (rows > 0 && channels > 0 && (!gated || !out || !aligned16(gated) || !aligned16(out)))
+    return fail(CUMM_HIP_EINVAL, "gated, grad and out must be 16-byte aligned and not empty");
+  return column_sum_checked(sums, grad, out, gated, rows, channels, dtype, workspace, workspace_bytes, stream);
 }
 
 int cumm_hip_copy_kernel(void *dst, const void *src, size_t bytes, void *stream) {

@@ -4,12 +4,18 @@
 //   finish_rows      out[r, c] = cvt(act(alpha * acc[r, c] + beta * bias[c])) from an fp32 image of
 //                    the result (the per-offset "native" convolution accumulates in fp32 and
 //                    rounds once, here)
-//   relu_backward    dst = grad where the forward output was positive, else 0
+//   relu_backward    dst = grad where the forward output was positive, else 0; with sums also the
+//                    column sums of dst, which then cost no pass of their own
 //   column_sum       dst[c] = cvt(sum over rows of src[r, c]) in fp32, in a fixed order (the
 //                    gradient of a bias): per-block partial sums, then a sum over blocks in
 //                    block order, so the result is the same from run to run
 //
-// All three move 16-byte pieces (8 two-byte elements), consecutive lanes on consecutive pieces.
+// All three move 16-byte pieces (8 two-byte elements), consecutive lanes on consecutive pieces.  The gate
+// and the sums are bound by HBM and run as many short workgroups in memory order: a resident grid
+// whose workgroups walk the tensor with a stride drifts apart and loses open pages (gate of 652 k rows of
+// 256 channels, 1.0 GB: 203 us with 4096 workgroups walking, 169 us with one per 256 pieces).  Operands
+// that are read once and exceed what the last-level cache keeps are loaded non-temporally (1 M rows
+// of 128: 130 -> 110 us; 161 us for the 1.0 GB); below kStreamBytes that gives nothing.
 #include "launch.h"
 
 namespace cummhip {
@@ -56,24 +62,37 @@ __global__ __launch_bounds__(256) void finish_rows_kernel(const FinishRowsParams
   }
 }
 
+constexpr int kBatch = 4;   // pieces per operand that a row lane of the sums has on their way
+
 template <class T>
-__global__ __launch_bounds__(256) void relu_backward_kernel(v4i *dst, const v4i *grad, const v4i *out, size_t vecs) {
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < vecs; i += (size_t)gridDim.x * 256) {
-    const v4i g = grad[i], o = out[i];
-    const uint16_t *gh = reinterpret_cast<const uint16_t *>(&g);
-    const uint16_t *oh = reinterpret_cast<const uint16_t *>(&o);
-    v4i r;
-    uint16_t *rh = reinterpret_cast<uint16_t *>(&r);
+__device__ __forceinline__ v4i gate8(const v4i &g, const v4i &o) {
+  const uint16_t *gh = reinterpret_cast<const uint16_t *>(&g);
+  const uint16_t *oh = reinterpret_cast<const uint16_t *>(&o);
+  v4i r;
+  uint16_t *rh = reinterpret_cast<uint16_t *>(&r);
 #pragma unroll
-    for (int x = 0; x < 8; ++x) rh[x] = Elem<T>::to_float(oh[x]) > 0.0f ? gh[x] : (uint16_t)0;
-    dst[i] = r;
-  }
+  for (int x = 0; x < 8; ++x) rh[x] = Elem<T>::to_float(oh[x]) > 0.0f ? gh[x] : (uint16_t)0;
+  return r;
 }
 
-// partial[b][c] = sum of src[r][c] over the rows of block b.  Thread t takes the 8-channel piece
-// t % V of the rows t / V, t / V + R, ... of its block (V pieces per row, R = 256 / V rows at a
-// time); the R row lanes of a piece are then summed through LDS in lane order.
-template <class T>
+constexpr size_t kStreamBytes = (size_t)64 << 20;
+
+template <bool NT>
+__device__ __forceinline__ v4i load_piece(const v4i *p) {
+  return NT ? __builtin_nontemporal_load(p) : *p;
+}
+
+template <class T, bool NT>
+__global__ __launch_bounds__(256) void relu_backward_kernel(v4i *dst, const v4i *grad, const v4i *out, size_t vecs) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < vecs) dst[i] = gate8<T>(load_piece<NT>(grad + i), load_piece<NT>(out + i));
+}
+
+// partial[b][c] = sum of src[r][c] over the rows of block b - with GATE of the gated rows, which are
+// written to gated on the way.  Thread t takes the 8-channel piece t % V of the rows t / V, t / V + R,
+// ... of its block (V pieces per row, R = 256 / V rows at a time); the R row lanes of a piece are then
+// summed through LDS in lane order.
+template <class T, bool GATE, bool NT>
 __global__ __launch_bounds__(256) void column_partial_kernel(const ColumnSumParams p) {
   __shared__ float lds[256][9];
   const int V = p.channels / 8;
@@ -85,11 +104,29 @@ __global__ __launch_bounds__(256) void column_partial_kernel(const ColumnSumPara
     const int64_t r0 = (int64_t)blockIdx.x * p.rows_per_block;
     int64_t r1 = r0 + p.rows_per_block;
     if (r1 > p.rows) r1 = p.rows;
-    for (int64_t r = r0 + lane_row; r < r1; r += R) {
-      float f[8];
-      unpack8<T>(*reinterpret_cast<const v4i *>(reinterpret_cast<const uint16_t *>(p.src) + r * p.channels + piece * 8), f);
+    const v4i *src = reinterpret_cast<const v4i *>(p.src) + piece;
+    const v4i *out = reinterpret_cast<const v4i *>(p.out) + piece;
+    v4i *gated = reinterpret_cast<v4i *>(p.gated) + piece;
+    for (int64_t r = r0 + lane_row; r < r1; r += kBatch * R) {
+      v4i g[kBatch], o[kBatch];
 #pragma unroll
-      for (int x = 0; x < 8; ++x) s[x] += f[x];
+      for (int u = 0; u < kBatch; ++u) {
+        const int64_t at = (r + u * R < r1 ? r + u * R : r) * V;
+        g[u] = load_piece<NT>(src + at);
+        if constexpr (GATE) o[u] = load_piece<NT>(out + at);
+      }
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        if (r + u * R >= r1) break;
+        if constexpr (GATE) {
+          g[u] = gate8<T>(g[u], o[u]);
+          gated[(r + u * R) * V] = g[u];
+        }
+        float f[8];
+        unpack8<T>(g[u], f);
+#pragma unroll
+        for (int x = 0; x < 8; ++x) s[x] += f[x];
+      }
     }
   }
 #pragma unroll
@@ -105,33 +142,42 @@ __global__ __launch_bounds__(256) void column_partial_kernel(const ColumnSumPara
   }
 }
 
-// dst[c] = cvt(sum over blocks) in a fixed shape: sixteen threads per channel, thread j adds the j-th
-// sixteenth of the blocks in block order (eight loads in flight at a time: one thread walking all
-// 1024 blocks took 54 us), then the sixteen sums are added in order
-template <class T>
-__global__ __launch_bounds__(256) void column_final_kernel(const ColumnSumParams p) {
-  __shared__ float part[16][17];
+// Sum over blocks in a fixed shape: 64 threads per channel, thread j adds the j-th 64th of the blocks in
+// block order (eight loads in flight at a time), then sixteen sums each are added in order, then
+// those four.  The blocks of slice blockIdx.y of gridDim.y; the last stage (one slice) converts.
+template <class T, bool LAST>
+__global__ __launch_bounds__(1024) void column_final_kernel(const ColumnSumParams p, const float *from, int blocks, float *to) {
+  __shared__ float part[64][17];
   const int cl = threadIdx.x & 15, j = threadIdx.x >> 4;
   const int c = blockIdx.x * 16 + cl;
-  const int share = (p.blocks + 15) >> 4;
-  const int b0 = j * share, b1 = b0 + share < p.blocks ? b0 + share : p.blocks;
+  const int slice = (blocks + gridDim.y - 1) / gridDim.y;
+  const int first = (int)blockIdx.y * slice, end = first + slice < blocks ? first + slice : blocks;
+  const int share = (end - first + 63) >> 6;
+  const int b0 = first + j * share, b1 = b0 + share < end ? b0 + share : end;
   float s = 0.0f;
   if (c < p.channels) {
     for (int b = b0; b < b1; b += 8) {
       float v[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = b + u < b1 ? p.partial[(int64_t)(b + u) * p.channels + c] : 0.0f;
+      for (int u = 0; u < 8; ++u) v[u] = b + u < b1 ? from[(int64_t)(b + u) * p.channels + c] : 0.0f;
 #pragma unroll
       for (int u = 0; u < 8; ++u) s += v[u];
     }
   }
   part[j][cl] = s;
   __syncthreads();
-  if (j == 0 && c < p.channels) {
-    float total = part[0][cl];
+  if (j < 4) {
+    s = part[j * 16][cl];
 #pragma unroll
-    for (int k = 1; k < 16; ++k) total += part[k][cl];
-    reinterpret_cast<uint16_t *>(p.dst)[c] = Elem<T>::from_float(total);
+    for (int k = 1; k < 16; ++k) s += part[j * 16 + k][cl];
+  }
+  __syncthreads();
+  if (j < 4) part[j][cl] = s;
+  __syncthreads();
+  if (j == 0 && c < p.channels) {
+    const float total = ((part[0][cl] + part[1][cl]) + part[2][cl]) + part[3][cl];
+    if constexpr (LAST) reinterpret_cast<uint16_t *>(p.dst)[c] = Elem<T>::from_float(total);
+    else to[(int64_t)blockIdx.y * p.channels + c] = total;
   }
 }
 
@@ -151,37 +197,73 @@ hipError_t launch_finish_rows(const FinishRowsParams &p, bool bf16, hipStream_t 
   return hipGetLastError();
 }
 
+template <class T>
+static void relu_backward(void *dst, const void *grad, const void *out, size_t vecs, hipStream_t s) {
+  const dim3 grid((unsigned)((vecs + 255) / 256));
+  v4i *d = reinterpret_cast<v4i *>(dst);
+  const v4i *g = reinterpret_cast<const v4i *>(grad), *o = reinterpret_cast<const v4i *>(out);
+  if (vecs * 16 > kStreamBytes) hipLaunchKernelGGL((relu_backward_kernel<T, true>), grid, dim3(256), 0, s, d, g, o, vecs);
+  else hipLaunchKernelGGL((relu_backward_kernel<T, false>), grid, dim3(256), 0, s, d, g, o, vecs);
+}
+
 hipError_t launch_relu_backward(void *dst, const void *grad, const void *out, size_t vecs, bool bf16, hipStream_t s) {
   if (vecs == 0) return hipSuccess;
-  if (bf16)
-    hipLaunchKernelGGL(relu_backward_kernel<BF16>, dim3(grid_for(vecs)), dim3(256), 0, s, reinterpret_cast<v4i *>(dst),
-                       reinterpret_cast<const v4i *>(grad), reinterpret_cast<const v4i *>(out), vecs);
-  else
-    hipLaunchKernelGGL(relu_backward_kernel<F16>, dim3(grid_for(vecs)), dim3(256), 0, s, reinterpret_cast<v4i *>(dst),
-                       reinterpret_cast<const v4i *>(grad), reinterpret_cast<const v4i *>(out), vecs);
+  if ((vecs + 255) / 256 > 0x7fffffffull) return hipErrorInvalidValue;
+  if (bf16) relu_backward<BF16>(dst, grad, out, vecs, s);
+  else relu_backward<F16>(dst, grad, out, vecs, s);
   return hipGetLastError();
 }
 
-int column_sum_blocks(int64_t rows, int channels) {
+// Rows per block: two batches per row lane (32 KB of each operand), more below kFewBlocks blocks' worth of
+// rows, where one stage of sums is to do (at most 1024 blocks).
+constexpr int kFewBlocks = 1024, kSlices = 64;
+static int64_t column_rows_per_block(int64_t rows, int channels) {
   const int V = channels / 8;
   const int R = V > 0 && V <= 256 ? 256 / V : 1;
-  // about 16 row steps per block, at most 1024 blocks
-  int64_t blocks = (rows + (int64_t)R * 16 - 1) / ((int64_t)R * 16);
-  if (blocks > 1024) blocks = 1024;
-  return (int)(blocks > 0 ? blocks : 1);
+  const int64_t small = (int64_t)R * 2 * kBatch;
+  const int64_t blocks = (rows + small - 1) / small;
+  if (blocks > 4 * kFewBlocks) return small;
+  int64_t few = blocks;
+  if (few > kFewBlocks) few = kFewBlocks;
+  return few > 0 ? (rows + few - 1) / few : 1;
+}
+static int column_blocks(int64_t rows, int channels) {
+  const int64_t per = column_rows_per_block(rows, channels);
+  return rows > 0 ? (int)((rows + per - 1) / per) : 1;
+}
+// rows of partial sums in the workspace: one per block, and one per slice of the first of two stages
+int column_sum_blocks(int64_t rows, int channels) {
+  const int blocks = column_blocks(rows, channels);
+  return blocks > kFewBlocks ? blocks + kSlices : blocks;
+}
+
+template <class T>
+static hipError_t column_sum(const ColumnSumParams &p, hipStream_t s) {
+  const bool stream = (size_t)p.rows * (size_t)p.channels * 2 > kStreamBytes;
+  if (p.gated != nullptr) {
+    if (stream) hipLaunchKernelGGL((column_partial_kernel<T, true, true>), dim3(p.blocks), dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((column_partial_kernel<T, true, false>), dim3(p.blocks), dim3(256), 0, s, p);
+  } else {
+    if (stream) hipLaunchKernelGGL((column_partial_kernel<T, false, true>), dim3(p.blocks), dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((column_partial_kernel<T, false, false>), dim3(p.blocks), dim3(256), 0, s, p);
+  }
+  const unsigned groups = (unsigned)((p.channels + 15) / 16);
+  const float *from = p.partial;
+  int blocks = p.blocks;
+  if (blocks > kFewBlocks) {
+    float *to = p.partial + (int64_t)blocks * p.channels;
+    hipLaunchKernelGGL((column_final_kernel<T, false>), dim3(groups, kSlices), dim3(1024), 0, s, p, from, blocks, to);
+    from = to;
+    blocks = kSlices;
+  }
+  hipLaunchKernelGGL((column_final_kernel<T, true>), dim3(groups), dim3(1024), 0, s, p, from, blocks, nullptr);
+  return hipGetLastError();
 }
 
 hipError_t launch_column_sum(ColumnSumParams p, bool bf16, hipStream_t s) {
-  p.blocks = column_sum_blocks(p.rows, p.channels);
-  p.rows_per_block = (p.rows + p.blocks - 1) / p.blocks;
-  if (bf16) {
-    hipLaunchKernelGGL(column_partial_kernel<BF16>, dim3(p.blocks), dim3(256), 0, s, p);
-    hipLaunchKernelGGL(column_final_kernel<BF16>, dim3((p.channels + 15) / 16), dim3(256), 0, s, p);
-  } else {
-    hipLaunchKernelGGL(column_partial_kernel<F16>, dim3(p.blocks), dim3(256), 0, s, p);
-    hipLaunchKernelGGL(column_final_kernel<F16>, dim3((p.channels + 15) / 16), dim3(256), 0, s, p);
-  }
-  return hipGetLastError();
+  p.blocks = column_blocks(p.rows, p.channels);
+  p.rows_per_block = column_rows_per_block(p.rows, p.channels);
+  return bf16 ? column_sum<BF16>(p, s) : column_sum<F16>(p, s);
 }
 
 }  // namespace cummhip

@@ -197,6 +197,8 @@ hipError_t launch_relu_backward(void *dst, const void *grad, const void *out, si
 struct ColumnSumParams {
   void *dst;            // [channels]
   const void *src;      // [rows, channels]
+  const void *out;      // [rows, channels] forward output whose positive elements let src through,
+  void *gated;          // and the gated rows; NULL both: plain sums
   float *partial;       // [blocks, channels] fp32
   int64_t rows, rows_per_block;
   int32_t channels, blocks;

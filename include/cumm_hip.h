@@ -447,6 +447,12 @@ int cumm_hip_relu_backward(void *dst, const void *grad, const void *out, size_t 
 size_t cumm_hip_column_sum_workspace(int64_t rows, int channels);
 int cumm_hip_column_sum(void *dst, const void *src, int64_t rows, int channels, int dtype, void *workspace,
                         size_t workspace_bytes, void *stream);
+/* Both at once, reading grad once: gated [rows, channels] = grad where out is positive, else 0, and sums
+ * [channels] = the column sums of gated (the input gradient's gate and the bias gradient of a layer with a
+ * fused ReLU); the same results as the two calls, workspace as cumm_hip_column_sum. */
+int cumm_hip_relu_backward_sums(void *gated, void *sums, const void *grad, const void *out, int64_t rows, int channels,
+                                int dtype, void *workspace, size_t workspace_bytes, void *stream);
+
 
 /* Plain device-to-device copy kernel of `bytes` bytes (16-byte aligned); used to
  * calibrate the HBM traffic counters against a transfer of known size. */

@@ -68,3 +68,27 @@ def test_column_sum(dtype, rows, channels):
     scale = np.abs(H.as_f32(src, dtype)).astype(np.float64).sum(axis=0) + 1e-6
     ulp16 = 2.0 ** (-10 if dtype == "f16" else -7)
     assert np.all(np.abs(got - exact) <= 1e-5 * scale + ulp16 * np.abs(exact))
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("rows,channels", [(1, 8), (4097, 2048), (33000, 64), (530000, 72), (0, 64)])
+def test_gate_and_sums_in_one_pass(dtype, rows, channels):
+    """cumm_hip_relu_backward_sums against the two calls it stands for: the same bits (one and two stages
+    of partial sums, tensors below and above the size that is loaded non-temporally)."""
+    rng = np.random.default_rng(rows + channels)
+    pool = rng.normal(0, 1, size=1 << 16).astype(np.float32)
+    grad = H.to_storage(np.resize(pool, rows * channels).reshape(rows, channels), dtype)
+    out = H.to_storage(np.maximum(np.resize(pool[7:], rows * channels).reshape(rows, channels), 0), dtype)
+    lib, tvt = _capi.lib(), H.TV_DTYPE[dtype]
+    d_g, d_o = H.dev(grad, dtype), H.dev(out, dtype)
+    gated, gated2 = tv.zeros([max(rows, 1), channels], tvt, 0), tv.zeros([max(rows, 1), channels], tvt, 0)
+    sums, sums2 = tv.zeros([channels], tvt, 0), tv.zeros([channels], tvt, 0)
+    need = int(lib.cumm_hip_column_sum_workspace(rows, channels))
+    ws = tv.empty([need], tv.uint8, 0)
+    _capi.check(lib.cumm_hip_relu_backward_sums(gated.byte_pointer(), sums.byte_pointer(), d_g.byte_pointer(), d_o.byte_pointer(),
+                                                rows, channels, tvt, ws.byte_pointer(), need, 0))
+    _capi.check(lib.cumm_hip_relu_backward(gated2.byte_pointer(), d_g.byte_pointer(), d_o.byte_pointer(), rows * channels, tvt, 0))
+    _capi.check(lib.cumm_hip_column_sum(sums2.byte_pointer(), gated2.byte_pointer(), rows, channels, tvt, ws.byte_pointer(), need, 0))
+    np.testing.assert_array_equal(H.host(gated), H.host(gated2))
+    np.testing.assert_array_equal(H.host(sums), H.host(sums2))
+    assert np.array_equal(H.host(gated)[:rows], np.where(H.as_f32(out, dtype) > 0, grad, np.zeros_like(grad)))
