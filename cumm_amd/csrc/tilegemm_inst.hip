@@ -29,40 +29,87 @@ static hipError_t launch_xy(bool xk, bool yk, const TileGemmParams &p, dim3 grid
   return hipGetLastError();
 }
 
-// Plain GEMM with both operands contiguous along the contraction, two-byte elements, shapes
-// the LDS-ring kernel takes without a remainder in k and with 16-byte output pieces.  Its result
-// does not depend on the tile (one fp32 sum over k in ascending order per element either way).
-// Measured on 4096^3 f16 (TFLOP/s): 256 x 256 x 32 per step with 2 x 4 waves of 128 x 64 and
-// three stages 1089, the same with 4 x 2 waves of 64 x 128 954, with four stages 1066, with 64
-// per step and two stages 1011; 128 x 128 x 64 with 2 x 2 waves and two stages 966; 256 x 128 x 32
-// with three stages 902; the register-staged kernel 583.
-template <class T, int WM, int WN, int RBW, int NBW, int KS, int NS>
+// Plain GEMM of two-byte elements in every layout, shapes with 16-byte pieces along each operand's and
+// the result's contiguous dimension: the LDS-ring kernels.  (One fp32 sum over k per element whatever
+// the tile - in eight parts, added in order, for the kernel that splits k over its waves.)
+template <class T, int WM, int WN, int RBW, int NBW, int KS, int NS, bool XT, bool YT>
 static hipError_t launch_dense_ring_as(const TileGemmParams &p, hipStream_t s) {
   constexpr int TM = WM * RBW * 16, TN = WN * NBW * 16;
-  if (!counted_waits_hold<densegemm_lds_kernel<T, WM, WN, RBW, NBW, KS, NS>>()) return hipErrorNotSupported;
+  if (!counted_waits_hold<densegemm_lds_kernel<T, WM, WN, RBW, NBW, KS, NS, XT, YT>>()) return hipErrorNotSupported;
   const int tiles_m = (p.m + TM - 1) / TM, tiles_n = (p.n + TN - 1) / TN;
-  hipLaunchKernelGGL((densegemm_lds_kernel<T, WM, WN, RBW, NBW, KS, NS>), dim3((unsigned)(tiles_m * tiles_n)),
+  hipLaunchKernelGGL((densegemm_lds_kernel<T, WM, WN, RBW, NBW, KS, NS, XT, YT>), dim3((unsigned)(tiles_m * tiles_n)),
                      dim3(WM * WN * 64), 0, s, p, tiles_m, tiles_n);
   return hipGetLastError();
 }
 
+// the large tile: fragments double-buffered in registers
+template <class T, bool XT, bool YT>
+static hipError_t launch_dense_pipe(const TileGemmParams &p, hipStream_t s) {
+  if (!counted_waits_hold<densegemm_pipe_kernel<T, 2, 4, 8, 4, 4, XT, YT>>()) return hipErrorNotSupported;
+  const int tiles_m = (p.m + 255) / 256, tiles_n = (p.n + 255) / 256;
+  hipLaunchKernelGGL((densegemm_pipe_kernel<T, 2, 4, 8, 4, 4, XT, YT>), dim3((unsigned)(tiles_m * tiles_n)), dim3(512), 0, s, p, tiles_m,
+                     tiles_n);
+  return hipGetLastError();
+}
+
+// Which tile: the least estimated time, from measurements of f16 products (us; n = tiles per CU, rounded up,
+// of 256 CUs; k in elements; the second figure for rows that are no whole number of 128-byte lines, whose
+// fetches touch a line more each):
+//   64 x 64 x 64, 2 x 2 waves, three stages     3.5 + n (0.21 + 0.0033 / 0.0045 k), 0.0035 k for n = 1
+//                                               (1024^3 7.1; 2000 x 776 x 1160 12.4; 2048^3 28; 3000^3 152)
+//   the same with k split over eight waves      3.8 + 0.0018 n k    (256 x 256 x 4096: 11.2 against 15.8;
+//                                                                    one workgroup per CU: only for n = 1)
+//   128 x 64 x 64, three stages                 5.0 + 0.0105 / 0.0135 k per two tiles of a CU, 0.0076 k for
+//                                               one alone (1536 x 1536 x 4096 38 against 40; 2048^3 25)
+//   128 x 128 x 64, two stages                  5.0 + 0.0172 k per two tiles of a CU, 0.0138 k for one
+//                                               (2504^3 50 against 73; 2048 x 4096^2 73 against 96)
+//   256 x 256 x 32, 2 x 4 waves, four stages    8.5 + 0.0255 n k    (4096^3 120; 3000^3 85 against 104)
+// The step-by-step cost of the small tiles is the chain of a step; from two workgroups per CU on it is the
+// 64 bytes per clock that a CU fetches: a 64 x 64 tile needs 512 bytes per MFMA of 16 x 16 x 32 (four clocks of
+// the CU's matrix cores), a 128 x 128 tile 256, a 256 x 256 tile 128.
+template <class T, bool XT, bool YT>
+static hipError_t launch_dense_ring_layout(const TileGemmParams &p, hipStream_t s) {
+  const auto per_cu = [&](int tm, int tn) {
+    return (double)(((int64_t)((p.m + tm - 1) / tm) * ((p.n + tn - 1) / tn) + 255) / 256);
+  };
+  const double k = p.k, n64 = per_cu(64, 64), n128 = per_cu(128, 64), n256 = per_cu(256, 256);
+  const bool lines = p.ldx % 64 == 0 && p.ldy % 64 == 0;
+  const double t64 = 3.5 + (n64 == 1 ? 0.0035 * k : n64 * (0.21 + (lines ? 0.0033 : 0.0045) * k));
+  const double tw = n64 > 1 ? 1e30 : 3.8 + 0.0018 * k + ((int64_t)((p.m + 63) / 64) * ((p.n + 63) / 64) > 32 ? 0.0025 * k : 0.0);
+  const double t128 = 5.0 + (n128 > 1 ? (lines ? 0.0105 : 0.0135) * (double)(((int)n128 + 1) / 2) : 0.0076) * k;
+  const double n128s = per_cu(128, 128);
+  const double t128s = 5.0 + (n128s > 1 ? 0.0172 * (double)(((int)n128s + 1) / 2) : 0.0138) * k;
+  const double t256 = 8.5 + 0.0255 * n256 * k;
+  if (t256 <= t128s && t256 <= t128 && t256 <= t64 && t256 <= tw) return launch_dense_pipe<T, XT, YT>(p, s);
+  if (t128s <= t128 && t128s <= t64 && t128s <= tw) return launch_dense_ring_as<T, 2, 2, 4, 4, 2, 2, XT, YT>(p, s);
+  if (t128 <= t64 && t128 <= tw) return launch_dense_ring_as<T, 2, 2, 4, 2, 2, 3, XT, YT>(p, s);
+  if (tw < t64) {
+    if (!counted_waits_hold<densegemm_wave_kernel<T, 8, 1, 2, XT, YT>>()) return hipErrorNotSupported;
+    const int tiles_m = (p.m + 63) / 64, tiles_n = (p.n + 63) / 64;
+    hipLaunchKernelGGL((densegemm_wave_kernel<T, 8, 1, 2, XT, YT>), dim3((unsigned)(tiles_m * tiles_n)), dim3(512), 0, s, p, tiles_m,
+                       tiles_n);
+    return hipGetLastError();
+  }
+  return launch_dense_ring_as<T, 2, 2, 2, 2, 2, 3, XT, YT>(p, s);
+}
+
 template <class T>
-static bool launch_dense_ring(const TileGemmParams &p, hipStream_t s, hipError_t *err) {
+static bool launch_dense_ring(bool xk, bool yk, const TileGemmParams &p, hipStream_t s, hipError_t *err) {
   if constexpr (Elem<T>::kBytes != 2) {
     return false;
   } else {
     const auto al16 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15u) == 0; };
+    const int64_t y_rows = yk ? p.m : p.k, y_cols = yk ? p.k : p.m, x_rows = xk ? p.n : p.k, x_cols = xk ? p.k : p.n;
     const bool ok = p.kv == 1 && p.split_k == 1 && !p.x_gather && !p.y_gather && !p.red_mask &&
-                    p.k >= 64 && p.k % 64 == 0 && p.n % 8 == 0 && p.ldx % 8 == 0 && p.ldy % 8 == 0 &&
-                    p.ldc % 8 == 0 && p.ldd % 8 == 0 && al16(p.X) && al16(p.Y) && al16(p.C) && al16(p.D) &&
-                    ((int64_t)(p.m - 1) * p.ldy + p.k) * 2 < ((int64_t)1 << 31) &&
-                    ((int64_t)(p.n - 1) * p.ldx + p.k) * 2 < ((int64_t)1 << 31);
+                    p.m > 0 && p.n > 0 && p.k > 0 && y_cols % 8 == 0 && x_cols % 8 == 0 && p.n % 8 == 0 &&
+                    p.ldx % 8 == 0 && p.ldy % 8 == 0 && p.ldc % 8 == 0 && p.ldd % 8 == 0 &&
+                    al16(p.X) && al16(p.Y) && al16(p.C) && al16(p.D) &&
+                    ((y_rows - 1) * p.ldy + y_cols) * 2 < ((int64_t)1 << 31) && ((x_rows - 1) * p.ldx + x_cols) * 2 < ((int64_t)1 << 31);
     if (!ok) return false;
-    const int64_t big_tiles = (int64_t)((p.m + 255) / 256) * ((p.n + 255) / 256);
-    const int64_t mid_tiles = (int64_t)((p.m + 127) / 128) * ((p.n + 127) / 128);
-    if (big_tiles >= 256) *err = launch_dense_ring_as<T, 2, 4, 8, 4, 1, 3>(p, s);       // a tile per CU at least
-    else if (mid_tiles >= 64) *err = launch_dense_ring_as<T, 2, 2, 4, 4, 2, 2>(p, s);
-    else return false;
+    if (xk && yk) *err = launch_dense_ring_layout<T, false, false>(p, s);
+    else if (yk) *err = launch_dense_ring_layout<T, true, false>(p, s);
+    else if (xk) *err = launch_dense_ring_layout<T, false, true>(p, s);
+    else *err = launch_dense_ring_layout<T, true, true>(p, s);
     return *err != hipErrorNotSupported;     // (the register-staged kernel takes over)
   }
 }
@@ -70,10 +117,8 @@ static bool launch_dense_ring(const TileGemmParams &p, hipStream_t s, hipError_t
 hipError_t CUMM_LAUNCH_NAME(int tm, int tn, bool xk, bool yk, const TileGemmParams &p, dim3 grid, hipStream_t s) {
   using T = CUMM_ELEM;
   if constexpr (!kWide) {
-    if (xk && yk) {
-      hipError_t err = hipSuccess;
-      if (launch_dense_ring<T>(p, s, &err)) return err;
-    }
+    hipError_t err = hipSuccess;
+    if (launch_dense_ring<T>(xk, yk, p, s, &err)) return err;
   }
   if (tm == 64 && tn == 64) return launch_xy<T, 2, 2>(xk, yk, p, grid, s);
   if (tm == 128 && tn == 128) return launch_xy<T, 4, 4>(xk, yk, p, grid, s);

@@ -1,0 +1,72 @@
+"""Dense matmul2 on the LDS-ring kernels in all layouts (densegemm_lds.h): tile edges and remainders in m, n
+and k, each kernel of the dispatch, alpha / beta with a separate source and with a bias, against torch's
+fp32 product of the same operands."""
+import numpy as np
+import pytest
+
+import helpers as H
+from cumm_amd import tensorview as tv
+from cumm_amd.gemm.main import GemmMainUnitTest
+from cumm_amd.tensorview.gemm import Activation, GemmParams, ShuffleStrideType
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+# one rounding to the type of values around sqrt(k), and fp32 sums of k products
+TOL = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}
+
+
+def _run(dtype, m, n, k, ta, tb, source, alpha=1.0, beta=0.0, relu=False):
+    from cumm_amd.torch_bridge import torch2tensor
+    tdt = {"f16": torch.float16, "bf16": torch.bfloat16}[dtype]
+    gen = torch.Generator(device="cuda").manual_seed(m * 131 + n * 17 + k)
+    rnd = lambda *s: torch.randn(*s, generator=gen, device="cuda").to(tdt)
+    a, b = rnd(*((k, m) if ta else (m, k))), rnd(*((n, k) if tb else (k, n)))
+    c = torch.full((m, n), float("nan"), dtype=tdt, device="cuda")
+    p = GemmParams()
+    p.algo_desp = H.find_gemm_desp(dtype, ShuffleStrideType.NoShuffle, 64, 64, ta, tb)
+    p.a, p.b, p.c = torch2tensor(a), torch2tensor(b), torch2tensor(c)
+    ref = alpha * ((a.float().t() if ta else a.float()) @ (b.float().t() if tb else b.float()))
+    if source != "none":
+        d = rnd(n) if source == "bias" else rnd(m, n)
+        p.d = torch2tensor(d)
+        ref = ref + beta * d.float()
+    p.alpha, p.beta = alpha, beta
+    if relu:
+        p.act_type, ref = Activation.ReLU, ref.clamp_min(0)
+    GemmMainUnitTest.matmul2(p)
+    torch.cuda.synchronize()
+    err = (c.float() - ref).abs()
+    bound = TOL[dtype] * ref.abs() + 3e-6 * k ** 0.5 * 4 + 1e-6 + TOL[dtype] * 1e-2
+    assert bool((err <= bound).all()), float((err - bound).max())
+
+
+@pytest.mark.parametrize("ta,tb", [(False, True), (False, False), (True, False), (True, True)])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_edges_of_tiles_and_steps(dtype, ta, tb):
+    torch.backends.cuda.matmul.allow_tf32 = False
+    for m in (8, 64, 72, 200):
+        for n in (8, 64, 136):
+            for k in (8, 24, 32, 64, 72, 328):
+                print("case dense", dtype, ta, tb, m, n, k, flush=True)
+                _run(dtype, m, n, k, ta, tb, "none")
+    # any number of rows of a row-major operand; any k where both operands have it as their row index
+    if not ta:
+        for m in (1, 63, 65, 191):
+            _run(dtype, m, 72, 104, ta, tb, "none")
+    if ta and not tb:
+        for k in (1, 7, 33, 1001):
+            _run(dtype, 72, 200, k, ta, tb, "none")
+
+
+@pytest.mark.parametrize("ta,tb", [(False, True), (False, False), (True, False), (True, True)])
+@pytest.mark.parametrize("m,n,k", [(136, 72, 2056),        # k over eight waves
+                                   (1000, 1064, 520),      # 64 x 64
+                                   (1992, 2040, 1032),     # 128 x 64
+                                   (2040, 2056, 1032),     # 128 x 128
+                                   (4088, 4088, 1048)])    # 256 x 256
+def test_each_kernel_with_its_epilogue(m, n, k, ta, tb):
+    torch.backends.cuda.matmul.allow_tf32 = False
+    print("case dense epilogue", m, n, k, ta, tb, flush=True)
+    _run("f16", m, n, k, ta, tb, "matrix", alpha=0.5, beta=2.0)
+    _run("bf16", m, n, k, ta, tb, "bias", alpha=1.0, beta=1.0, relu=True)
