@@ -1143,8 +1143,9 @@ static uint32_t pairs_slots(int n) {
   return slots;
 }
 
-// hash table slots (16 bytes each), then one presence word per slot pair
-size_t cumm_hip_subm_pairs_workspace(int n) { return (size_t)pairs_slots(n) * 16 + (size_t)pairs_slots(n) * 4; }
+// 20 bytes per slot, the size callers have had so far: hash table slots of 8 bytes, one presence word per
+// slot, a flag
+size_t cumm_hip_subm_pairs_workspace(int n) { return (size_t)pairs_slots(n) * 20; }
 
 int cumm_hip_subm_pairs(const int32_t *coords, int n, const int32_t *spatial_shape, const int32_t *ksize,
                         const int32_t *dilation, int32_t *indices_fwd, int32_t *indices_bwd,
@@ -1180,8 +1181,9 @@ int cumm_hip_subm_pairs(const int32_t *coords, int n, const int32_t *spatial_sha
   }
   p.ind_f = indices_fwd; p.ind_b = indices_bwd; p.mask_f = mask_fwd; p.mask_b = mask_bwd;
   p.table = workspace; p.slot_mask = pairs_slots(n) - 1u;
-  p.filter = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(workspace) + (size_t)pairs_slots(n) * 16);
+  p.filter = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(workspace) + (size_t)pairs_slots(n) * 8);
   p.filter_mask = pairs_slots(n) - 1u;
+  p.wide = p.filter + pairs_slots(n);
   p.kx = ksize[2];
   p.center_k = -1;
   for (int k = 0; k < (int)kv; ++k)
@@ -1318,7 +1320,13 @@ void conv_pairs_params(ConvPairsParams *p, const ConvPairsLayout &l, const int32
   std::memset(p, 0, sizeof(*p));
   p->coords = coords; p->n_in = n_in; p->batch = batch_size;
   p->kv = ksize[0] * ksize[1] * ksize[2];
-  for (int d = 0; d < 3; ++d) { p->out_shape[d] = out_shape[d]; p->stride[d] = stride[d]; p->pad[d] = padding[d]; }
+  p->kx = ksize[2];
+  for (int d = 0; d < 3; ++d) {
+    p->out_shape[d] = out_shape[d]; p->stride[d] = stride[d]; p->pad[d] = padding[d];
+    p->out_inv[d] = 1.0 / out_shape[d];
+    while ((1ull << p->div_shift[d]) < (unsigned long long)stride[d]) ++p->div_shift[d];
+    p->div_mul[d] = (uint32_t)(((1ull << (31 + p->div_shift[d])) + (unsigned)stride[d] - 1ull) / (unsigned)stride[d]);
+  }
   for (int k = 0; k < p->kv; ++k) {
     p->koff[k][0] = (k / (ksize[1] * ksize[2])) * dilation[0];
     p->koff[k][1] = ((k / ksize[2]) % ksize[1]) * dilation[1];

@@ -85,10 +85,11 @@ struct SubmPairsParams {
   int32_t off[kMaxKernelVolume][3];   // (k_zyx - center) * dilation per kernel offset
   int32_t *ind_f, *ind_b;  // [kv, n]; ind_b may be NULL
   uint32_t *mask_f, *mask_b;   // may be NULL (must be for kernel volumes above 32)
-  void *table;             // (slot_mask + 1) slots of 16 bytes
+  void *table;             // (slot_mask + 1) slots of 8 bytes
   uint32_t slot_mask;
   uint32_t *filter;        // (filter_mask + 1) presence words
   uint32_t filter_mask;
+  uint32_t *wide;          // one word: do any keys around these voxels need more than 32 bits?
   int32_t kx;              // offsets along x (kv = kz * ky * kx)
   int32_t center_k;        // the offset (0, 0, 0), whose pair is the voxel itself; -1 if there is none
 };
@@ -99,6 +100,9 @@ struct ConvPairsParams {
   const int32_t *coords;        // [n_in, 4] (batch, z, y, x)
   int32_t n_in, n_out, kv, batch;
   int32_t out_shape[3], stride[3], pad[3];
+  int32_t kx;                   // offsets along x (kv = kz * ky * kx)
+  uint32_t div_mul[3], div_shift[3];   // division by stride[d] as a multiplication
+  double out_inv[3];            // 1 / out_shape[d]
   int32_t koff[kMaxKernelVolume][3];   // k_zyx * dilation per kernel offset
   void *table;                  // (slot_mask + 1) slots of 16 bytes: {output site key, output row}
   uint32_t slot_mask;

@@ -9,8 +9,10 @@
 //
 // The table depends on the geometry only, never on the hash, so it is bit-exact against the host
 // builder whatever the hash.  Integer work, bound by HBM / L2 traffic:
-//   * open addressing with linear probing over 16-byte slots {64-bit key, row}: one load returns
-//     both, the table of 2N..4N slots (2-4 MB at 120 k voxels) stays in L2;
+//   * open addressing with linear probing over 8-byte slots {low word of the key, row}: one
+//     compare-and-swap inserts both, one load returns both, the table of 2N..4N slots (1-2 MB at
+//     120 k voxels) stays in L2.  Keys of more than 32 bits set a flag; only then does a match go on
+//     to the matching row's coordinates;
 //   * in front of the table sits a hashed presence bitmap, one 32-bit word per run of 32 sites
 //     along x (1 MB at 120 k voxels, L2-resident): most look-ups of a sparse cloud are misses,
 //     and the word turns them away - all x-neighbours of a row with one load - before they cost
@@ -18,6 +20,8 @@
 //   * the lookup kernel is one lane per (voxel, (kz, ky)): for a fixed offset consecutive lanes
 //     write consecutive table entries (coalesced).  Measured at 120 k voxels: one lane per voxel
 //     walking its 27 offsets 127 us, one lane per (voxel, offset) without the bitmap 66 us;
+//   * what remains is integer arithmetic: hashes and keys in 32 bits, a division by a stride as a
+//     multiplication, coordinates of output sites once per word of 32 of them.
 #include <hip/hip_runtime.h>
 
 #include <cstring>
@@ -35,6 +39,8 @@ struct __attribute__((aligned(16))) Slot {
   int32_t pad;
 };
 constexpr unsigned long long kEmptyKey = ~0ull;
+// slots of the submanifold table: low word of the key below the row; no row is all ones
+constexpr unsigned long long kEmptySlot = ~0ull;
 
 __device__ __forceinline__ unsigned long long mix64(unsigned long long k) {
   k ^= k >> 33;
@@ -45,11 +51,19 @@ __device__ __forceinline__ unsigned long long mix64(unsigned long long k) {
   return k;
 }
 
+__device__ __forceinline__ uint32_t mix32(uint32_t k) {
+  k *= 0x9E3779B1u;
+  k ^= k >> 15;
+  k *= 0x2C1B3C6Du;
+  return k ^ (k >> 13);
+}
+
 // one launch empties the table, the presence words and the masks
 __global__ __launch_bounds__(256) void pairs_clear_kernel(const SubmPairsParams p) {
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-  if (i <= p.slot_mask) reinterpret_cast<Slot *>(p.table)[i] = Slot{kEmptyKey, -1, 0};
+  if (i <= p.slot_mask) reinterpret_cast<unsigned long long *>(p.table)[i] = kEmptySlot;
   if (i <= p.filter_mask) p.filter[i] = 0u;
+  if (i == 0) *p.wide = 0u;
   if (i < (uint32_t)p.n) {
     // every voxel pairs with itself through the centre offset: that bit is set here, and the
     // look-up kernel neither probes the table nor touches the masks for it
@@ -61,11 +75,20 @@ __global__ __launch_bounds__(256) void pairs_clear_kernel(const SubmPairsParams 
 __device__ __forceinline__ unsigned long long coord_key(int b, int z, int y, int x, const SubmPairsParams &p) {
   return (((unsigned long long)b * p.shape[0] + z) * p.shape[1] + y) * p.shape[2] + x;
 }
+// line (b, z, y) of the grid, modulo 2^32; line * shape[2] + x is the low word of the key
+__device__ __forceinline__ uint32_t coord_line(int b, int z, int y, const SubmPairsParams &p) {
+  return ((uint32_t)b * (uint32_t)p.shape[0] + (uint32_t)z) * (uint32_t)p.shape[1] + (uint32_t)y;
+}
 // presence word of the 32 sites (b, z, y, 32*(x/32) ..): hashed, without a key, so a set bit
 // means "maybe" (two runs may share a word) and a clear bit means "certainly absent"
-__device__ __forceinline__ uint32_t presence_index(int b, int z, int y, int x, const SubmPairsParams &p) {
-  const unsigned long long run = (((unsigned long long)b * p.shape[0] + z) * p.shape[1] + y) * ((p.shape[2] + 31) >> 5) + (x >> 5);
-  return (uint32_t)mix64(run ^ 0x9e3779b97f4a7c15ull) & p.filter_mask;
+__device__ __forceinline__ uint32_t presence_index(uint32_t line, int run, const SubmPairsParams &p) {
+  return mix32(line * (uint32_t)((p.shape[2] + 31) >> 5) + (uint32_t)run) & p.filter_mask;
+}
+// is the row of a slot whose low word matches the site (b, z, y, x)?  Keys of 32 bits say all
+__device__ __forceinline__ bool same_site(const SubmPairsParams &p, uint32_t wide, uint32_t row, unsigned long long key) {
+  if (wide == 0u) return true;
+  const int4 c = reinterpret_cast<const int4 *>(p.coords)[row];
+  return coord_key(c.x, c.y, c.z, c.w, p) == key;
 }
 
 __global__ __launch_bounds__(256) void pairs_insert_kernel(const SubmPairsParams p) {
@@ -73,16 +96,20 @@ __global__ __launch_bounds__(256) void pairs_insert_kernel(const SubmPairsParams
   if (i >= p.n) return;
   const int4 c = reinterpret_cast<const int4 *>(p.coords)[i];
   const unsigned long long key = coord_key(c.x, c.y, c.z, c.w, p);
-  Slot *table = reinterpret_cast<Slot *>(p.table);
-  atomicOr(&p.filter[presence_index(c.x, c.y, c.z, c.w, p)], 1u << (c.w & 31));
-  uint32_t h = (uint32_t)mix64(key) & p.slot_mask;
+  unsigned long long *table = reinterpret_cast<unsigned long long *>(p.table);
+  atomicOr(&p.filter[presence_index(coord_line(c.x, c.y, c.z, p), c.w >> 5, p)], 1u << (c.w & 31));
+  const uint32_t low = (uint32_t)key;
+  // do this key and those of all sites around it (which lie in the same grid) fit 32 bits?
+  const unsigned long long last = coord_key(c.x, p.shape[0] - 1, p.shape[1] - 1, p.shape[2] - 1, p);
+  if (((key | last) >> 32) != 0ull) atomicOr(p.wide, 1u);
+  uint32_t h = mix32(low) & p.slot_mask;
+  const unsigned long long mine = ((unsigned long long)(uint32_t)i << 32) | low;
   // at most `slots` probes: the table has at least twice as many slots as voxels
   for (uint32_t probe = 0; probe <= p.slot_mask; ++probe) {
-    const unsigned long long prev = atomicCAS(&table[h].key, kEmptyKey, key);
-    if (prev == kEmptyKey || prev == key) {
-      table[h].row = i;   // (coordinates are unique: the caller's contract, as in spconv)
-      break;
-    }
+    const unsigned long long prev = atomicCAS(&table[h], kEmptySlot, mine);
+    if (prev == kEmptySlot) break;
+    // (coordinates are unique: the caller's contract, as in spconv; a repeated one is dropped)
+    if ((uint32_t)prev == low && same_site(p, 1u, (uint32_t)(prev >> 32), key)) break;
     h = (h + 1) & p.slot_mask;
   }
 }
@@ -92,14 +119,19 @@ __global__ __launch_bounds__(256) void pairs_insert_kernel(const SubmPairsParams
 // of the neighbour's run of 32 sites answers all of a row's x-neighbours with one 4-byte load from
 // a table that stays in L2, and only "maybe" goes on to the hash table.  grid.y = KZ*KY,
 // consecutive lanes = consecutive voxels: every table row is written coalesced.  The masks are
-// OR-ed with atomics, one per PAIR, into words that the clear kernel zeroed.
+// OR-ed with atomics, one per lane with a pair, into words that the clear kernel set.
 __global__ __launch_bounds__(256) void pairs_lookup_kernel(const SubmPairsParams p) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   const int zy = blockIdx.y;
   if (i >= p.n) return;
   const int4 c = reinterpret_cast<const int4 *>(p.coords)[i];
-  const Slot *table = reinterpret_cast<const Slot *>(p.table);
-  uint32_t have_index = ~0u, word = 0;
+  const unsigned long long *table = reinterpret_cast<const unsigned long long *>(p.table);
+  const uint32_t wide = *p.wide;
+  const int z = c.y + p.off[zy * p.kx][0], y = c.z + p.off[zy * p.kx][1];
+  const bool line_in = z >= 0 && z < p.shape[0] && y >= 0 && y < p.shape[1];
+  const uint32_t line = coord_line(c.x, z, y, p);
+  int have_run = -1;
+  uint32_t word = 0, bits_f = 0, bits_b = 0;
   for (int kx = 0; kx < p.kx; ++kx) {
     const int k = zy * p.kx + kx;
     if (k == p.center_k) {
@@ -107,33 +139,38 @@ __global__ __launch_bounds__(256) void pairs_lookup_kernel(const SubmPairsParams
       if (p.ind_b) p.ind_b[(int64_t)(p.kv - 1 - k) * p.n + i] = i;
       continue;
     }
-    const int z = c.y + p.off[k][0], y = c.z + p.off[k][1], x = c.w + p.off[k][2];
+    const int x = c.w + p.off[k][2];
     int row = -1;
-    if (z >= 0 && z < p.shape[0] && y >= 0 && y < p.shape[1] && x >= 0 && x < p.shape[2]) {
-      const uint32_t index = presence_index(c.x, z, y, x, p);
-      if (index != have_index) {
-        word = p.filter[index];
-        have_index = index;
+    if (line_in && x >= 0 && x < p.shape[2]) {
+      if ((x >> 5) != have_run) {
+        have_run = x >> 5;
+        word = p.filter[presence_index(line, have_run, p)];
       }
       if ((word >> (x & 31)) & 1u) {
-        const unsigned long long key = coord_key(c.x, z, y, x, p);
-        uint32_t h = (uint32_t)mix64(key) & p.slot_mask;
-        Slot s = table[h];
+        const uint32_t low = line * (uint32_t)p.shape[2] + (uint32_t)x;
+        const unsigned long long key = wide != 0u ? coord_key(c.x, z, y, x, p) : 0ull;
+        uint32_t h = mix32(low) & p.slot_mask;
         // a collision walks on until the key or an empty slot turns up (the table is never full)
-        for (uint32_t probe = 0; s.key != key && s.key != kEmptyKey && probe <= p.slot_mask; ++probe) {
+        for (uint32_t probe = 0; probe <= p.slot_mask; ++probe) {
+          const unsigned long long s = table[h];
+          if (s == kEmptySlot) break;
+          if ((uint32_t)s == low && same_site(p, wide, (uint32_t)(s >> 32), key)) {
+            row = (int)(uint32_t)(s >> 32);
+            break;
+          }
           h = (h + 1) & p.slot_mask;
-          s = table[h];
         }
-        if (s.key == key) row = s.row;
       }
     }
     p.ind_f[(int64_t)k * p.n + i] = row;
     if (p.ind_b) p.ind_b[(int64_t)(p.kv - 1 - k) * p.n + i] = row;
-    if (row >= 0) {
-      if (p.mask_f) atomicOr(&p.mask_f[i], 1u << k);
-      if (p.mask_b) atomicOr(&p.mask_b[i], 1u << (p.kv - 1 - k));
+    if (row >= 0 && k < 32) {      // (masks of one word only)
+      bits_f |= 1u << k;
+      bits_b |= 1u << ((p.kv - 1 - k) & 31);
     }
   }
+  if (p.mask_f && bits_f) atomicOr(&p.mask_f[i], bits_f);
+  if (p.mask_b && bits_b) atomicOr(&p.mask_b[i], bits_b);
 }
 
 // ---- regular (strided) sparse convolution: an output site is active iff an input falls into
@@ -275,7 +312,6 @@ __global__ __launch_bounds__(256) void conv_pairs_rows_kernel(const ConvPairsPar
   if (p.mask_f) p.mask_f[j] = 0u;
 }
 
-template <bool BITS>
 __global__ __launch_bounds__(256) void conv_pairs_fill_kernel(const ConvPairsParams p) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   const int k = blockIdx.y;
@@ -283,19 +319,14 @@ __global__ __launch_bounds__(256) void conv_pairs_fill_kernel(const ConvPairsPar
   unsigned long long key = 0;
   int row = -1;
   if (conv_out_site(p, reinterpret_cast<const int4 *>(p.coords)[i], k, &key)) {
-    if constexpr (BITS) {
-      const uint32_t word = p.bits[key >> 5], b = (uint32_t)key & 31u;
-      if ((word >> b) & 1u) row = (int)(p.prefix[key >> 5] + (uint32_t)__popc(word & ((1u << b) - 1u)));
-    } else {
-      const Slot *table = reinterpret_cast<const Slot *>(p.table);
-      uint32_t h = (uint32_t)mix64(key) & p.slot_mask;
-      Slot s = table[h];
-      for (uint32_t probe = 0; s.key != key && s.key != kEmptyKey && probe <= p.slot_mask; ++probe) {
-        h = (h + 1) & p.slot_mask;
-        s = table[h];
-      }
-      if (s.key == key) row = s.row;
+    const Slot *table = reinterpret_cast<const Slot *>(p.table);
+    uint32_t h = (uint32_t)mix64(key) & p.slot_mask;
+    Slot s = table[h];
+    for (uint32_t probe = 0; s.key != key && s.key != kEmptyKey && probe <= p.slot_mask; ++probe) {
+      h = (h + 1) & p.slot_mask;
+      s = table[h];
     }
+    if (s.key == key) row = s.row;
   }
   if (p.ind_b) p.ind_b[(int64_t)k * p.n_in + i] = row;
   if (row >= 0 && row < p.n_out) {
@@ -314,23 +345,90 @@ __global__ __launch_bounds__(256) void conv_bits_clear_kernel(const ConvPairsPar
     reinterpret_cast<v4i *>(p.bits)[q] = zero;
 }
 
+// num / stride where that is exact and inside the output grid; the quotient of a number below 2^31 is
+// (2 num * mul) >> (32 + shift) with mul = ceil(2^(31 + shift) / stride), 2^shift >= stride
+__device__ __forceinline__ bool conv_out_index(const ConvPairsParams &p, int d, int num, uint32_t *q) {
+  const uint32_t g = __umulhi((uint32_t)num << 1, p.div_mul[d]) >> p.div_shift[d];
+  *q = g;
+  return num >= 0 && g * (uint32_t)p.stride[d] == (uint32_t)num && g < (uint32_t)p.out_shape[d];
+}
+// key of the first site of the output line that input c reaches through offsets (kz, ky) = zy
+__device__ __forceinline__ bool conv_out_line(const ConvPairsParams &p, const int4 c, int zy, unsigned long long *first) {
+  const int k = zy * p.kx;
+  uint32_t z, y;
+  const bool in = conv_out_index(p, 0, c.y + p.pad[0] - p.koff[k][0], &z) & conv_out_index(p, 1, c.z + p.pad[1] - p.koff[k][1], &y);
+  *first = (((unsigned long long)(uint32_t)c.x * (uint32_t)p.out_shape[0] + z) * (uint32_t)p.out_shape[1] + y) * (uint32_t)p.out_shape[2];
+  return in && c.x >= 0 && c.x < p.batch;
+}
+
+// One lane per (input, (kz, ky)), grid.y = KZ * KY: the sites of a line that fall into one word go out in
+// one atomic.  (One lane per (input, offset) with divisions in 64 bits: 18.4 us at 120 k voxels, 32.7 at
+// 300 k; the arithmetic was what bound it.)
 __global__ __launch_bounds__(256) void conv_bits_sites_kernel(const ConvPairsParams p) {
   const int i = blockIdx.x * 256 + threadIdx.x;
-  const int k = blockIdx.y;
+  const int zy = blockIdx.y;
   if (i >= p.n_in) return;
-  unsigned long long key = 0;
-  if (!conv_out_site(p, reinterpret_cast<const int4 *>(p.coords)[i], k, &key)) return;
-  const uint32_t bit = 1u << ((uint32_t)key & 31u);
+  const int4 c = reinterpret_cast<const int4 *>(p.coords)[i];
+  unsigned long long first, at = ~0ull;
+  if (!conv_out_line(p, c, zy, &first)) return;
+  uint32_t bits = 0;
   // a third of the candidates repeat a site: look first (a set bit stays set)
-  if (!(__atomic_load_n(&p.bits[key >> 5], __ATOMIC_RELAXED) & bit)) atomicOr(&p.bits[key >> 5], bit);
+  for (int kx = 0; kx < p.kx; ++kx) {
+    uint32_t x;
+    if (!conv_out_index(p, 2, c.w + p.pad[2] - p.koff[zy * p.kx + kx][2], &x)) continue;
+    const unsigned long long key = first + x;
+    if ((key >> 5) != at) {
+      if (bits && (__atomic_load_n(&p.bits[at], __ATOMIC_RELAXED) & bits) != bits) atomicOr(&p.bits[at], bits);
+      at = key >> 5;
+      bits = 0u;
+    }
+    bits |= 1u << ((uint32_t)key & 31u);
+  }
+  if (bits && (__atomic_load_n(&p.bits[at], __ATOMIC_RELAXED) & bits) != bits) atomicOr(&p.bits[at], bits);
+}
+
+// the pairs of those lanes: backward table coalesced, forward entries where they belong
+__global__ __launch_bounds__(256) void conv_bits_fill_kernel(const ConvPairsParams p) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  const int zy = blockIdx.y;
+  if (i >= p.n_in) return;
+  const int4 c = reinterpret_cast<const int4 *>(p.coords)[i];
+  unsigned long long first, at = ~0ull;
+  const bool line_in = conv_out_line(p, c, zy, &first);
+  uint32_t word = 0, before = 0, mine = 0;
+  for (int kx = 0; kx < p.kx; ++kx) {
+    const int k = zy * p.kx + kx;
+    uint32_t x;
+    int row = -1;
+    if (conv_out_index(p, 2, c.w + p.pad[2] - p.koff[k][2], &x) && line_in) {
+      const unsigned long long key = first + x;
+      const uint32_t b = (uint32_t)key & 31u;
+      if ((key >> 5) != at) {
+        at = key >> 5;
+        word = p.bits[at];
+        before = p.prefix[at];
+      }
+      if ((word >> b) & 1u) row = (int)(before + (uint32_t)__popc(word & ((1u << b) - 1u)));
+    }
+    if (p.ind_b) p.ind_b[(int64_t)k * p.n_in + i] = row;
+    if (row >= 0 && row < p.n_out) {
+      p.ind_f[(int64_t)k * p.n_out + row] = i;
+      if (p.mask_f) atomicOr(&p.mask_f[row], 1u << (k & 31));
+      mine |= 1u << (k & 31);
+    }
+  }
+  if (p.mask_b && mine) atomicOr(&p.mask_b[i], mine);
 }
 
 // ---- prefix[w] = number of set bits in the words before w (exclusive scan of the words' bit counts),
-// prefix[n_words] = their total.  Three small kernels: bit counts per block of kScanBlock words, one
-// workgroup that turns the block counts into offsets (carrying its running sum from one batch of
-// 256 blocks to the next), and the scan inside every block again, now with its offset.
-constexpr int kScanPerThread = 16;
+// prefix[n_words] = their total.  Two small kernels: bit counts per block of kScanBlock words, and the
+// scan inside every block, with the counts of the blocks before it: up to kScanDirect blocks each
+// workgroup adds those up itself, above that (134 M sites) one workgroup turns them into offsets in
+// between, kScanBatch blocks at a time.
+constexpr int kScanPerThread = 4;                   // (one 16-byte load: n_words is a multiple of 4)
 constexpr int kScanBlock = 256 * kScanPerThread;   // words per workgroup
+constexpr unsigned long long kScanDirect = 4096;
+constexpr int kScanOffsets = 8, kScanBatch = 256 * kScanOffsets;
 
 // a workgroup-wide exclusive scan of one value per thread (256 threads); returns the total in *total
 __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t *lds_waves, uint32_t *total) {
@@ -355,54 +453,62 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t *l
   return before + incl - v;
 }
 
+__device__ __forceinline__ v4i scan_words(const uint32_t *bits, unsigned long long n_words, unsigned long long first) {
+  const v4i none = {0, 0, 0, 0};
+  const v4i w = first < n_words ? *reinterpret_cast<const v4i *>(bits + first) : none;
+  return v4i{__builtin_popcount(w.x), __builtin_popcount(w.y), __builtin_popcount(w.z), __builtin_popcount(w.w)};
+}
+
 __global__ __launch_bounds__(256) void bit_scan_block_sums_kernel(const uint32_t *__restrict__ bits, unsigned long long n_words,
                                                                   uint32_t *__restrict__ block_sums) {
   __shared__ uint32_t lds_waves[4];
-  const unsigned long long base = (unsigned long long)blockIdx.x * kScanBlock;
-  uint32_t c = 0;
-#pragma unroll
-  for (int u = 0; u < kScanPerThread; ++u) {
-    const unsigned long long w = base + (unsigned long long)u * 256 + threadIdx.x;
-    c += w < n_words ? (uint32_t)__popc(bits[w]) : 0u;
-  }
+  const v4i c = scan_words(bits, n_words, (unsigned long long)blockIdx.x * kScanBlock + threadIdx.x * 4u);
   uint32_t total;
-  (void)block_exclusive_scan(c, lds_waves, &total);
+  (void)block_exclusive_scan((uint32_t)(c.x + c.y + c.z + c.w), lds_waves, &total);
   if (threadIdx.x == 0) block_sums[blockIdx.x] = total;
 }
 
-__global__ __launch_bounds__(256) void bit_scan_block_offsets_kernel(uint32_t *__restrict__ block_sums, unsigned long long n_blocks,
-                                                                     uint32_t *__restrict__ total_out) {
+__global__ __launch_bounds__(256) void bit_scan_block_offsets_kernel(uint32_t *__restrict__ block_sums, unsigned long long n_blocks) {
   __shared__ uint32_t lds_waves[4];
   uint32_t carry = 0;
-  for (unsigned long long b0 = 0; b0 < n_blocks; b0 += 256) {
-    const unsigned long long b = b0 + threadIdx.x;
-    const uint32_t v = b < n_blocks ? block_sums[b] : 0u;
-    uint32_t total;
-    const uint32_t excl = block_exclusive_scan(v, lds_waves, &total);
-    if (b < n_blocks) block_sums[b] = carry + excl;
+  for (unsigned long long b0 = 0; b0 < n_blocks; b0 += kScanBatch) {
+    const unsigned long long b = b0 + threadIdx.x * kScanOffsets;
+    uint32_t v[kScanOffsets], mine = 0, total;
+#pragma unroll
+    for (int u = 0; u < kScanOffsets; ++u) {
+      v[u] = b + u < n_blocks ? block_sums[b + u] : 0u;
+      mine += v[u];
+    }
+    uint32_t run = carry + block_exclusive_scan(mine, lds_waves, &total);
+#pragma unroll
+    for (int u = 0; u < kScanOffsets; ++u) {
+      if (b + u < n_blocks) block_sums[b + u] = run;
+      run += v[u];
+    }
     carry += total;
   }
-  if (threadIdx.x == 0) *total_out = carry;
 }
 
+// DIRECT: block_sums are counts, else offsets
+template <bool DIRECT>
 __global__ __launch_bounds__(256) void bit_scan_write_kernel(const uint32_t *__restrict__ bits, unsigned long long n_words,
                                                              const uint32_t *__restrict__ block_sums, uint32_t *__restrict__ prefix) {
   __shared__ uint32_t lds_waves[4];
-  // thread t owns kScanPerThread consecutive words (so that its own scan is a running sum)
-  const unsigned long long first = (unsigned long long)blockIdx.x * kScanBlock + (unsigned long long)threadIdx.x * kScanPerThread;
-  uint32_t cnt[kScanPerThread], mine = 0;
-#pragma unroll
-  for (int u = 0; u < kScanPerThread; ++u) {
-    cnt[u] = first + u < n_words ? (uint32_t)__popc(bits[first + u]) : 0u;
-    mine += cnt[u];
+  // thread t owns four consecutive words (so that its own scan is a running sum)
+  const unsigned long long first = (unsigned long long)blockIdx.x * kScanBlock + threadIdx.x * 4u;
+  const v4i c = scan_words(bits, n_words, first);
+  uint32_t base, total;
+  if constexpr (DIRECT) {
+    uint32_t mine = 0;
+    for (uint32_t b = threadIdx.x; b < blockIdx.x; b += 256u) mine += block_sums[b];
+    (void)block_exclusive_scan(mine, lds_waves, &base);
+  } else {
+    base = block_sums[blockIdx.x];
   }
-  uint32_t total;
-  uint32_t run = block_sums[blockIdx.x] + block_exclusive_scan(mine, lds_waves, &total);
-#pragma unroll
-  for (int u = 0; u < kScanPerThread; ++u) {
-    if (first + u < n_words) prefix[first + u] = run;
-    run += cnt[u];
-  }
+  const uint32_t excl = block_exclusive_scan((uint32_t)(c.x + c.y + c.z + c.w), lds_waves, &total);
+  const int run = (int)(base + excl);
+  if (first < n_words) *reinterpret_cast<v4i *>(prefix + first) = v4i{run, run + c.x, run + c.x + c.y, run + c.x + c.y + c.z};
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) prefix[n_words] = base + total;
 }
 
 // ---- the pieces of a 64-bit key sort out of two stable 32-bit sorts (sort_inst.hip)
@@ -422,7 +528,19 @@ __global__ __launch_bounds__(256) void key_gather_kernel(const unsigned long lon
   if (i < n) out[i] = keys[perm1[perm2 ? perm2[i] : i]];
 }
 
-// table prefill, masks, and the coordinates of the active sites, word by word
+// n / d and n % d for n below 2^52, by a reciprocal of 53 bits (at most one off)
+__device__ __forceinline__ unsigned long long split_site(unsigned long long n, int d, double inv, int *rem) {
+  long long q = (long long)((double)n * inv);
+  long long r = (long long)n - q * d;
+  if (r < 0) { --q; r += d; }
+  if (r >= d) { ++q; r -= d; }
+  *rem = (int)r;
+  return (unsigned long long)q;
+}
+
+// table prefill, masks, and the coordinates of the active sites, word by word: those of a word's first
+// site, then along the grid from one set bit to the next (divisions per site in 64 bits were half of
+// 20.5 us at 447 k output sites)
 __global__ __launch_bounds__(256) void conv_bits_rows_kernel(const ConvPairsParams p) {
   const unsigned long long j = blockIdx.x * 256ull + threadIdx.x, step = gridDim.x * 256ull;
   {
@@ -438,16 +556,28 @@ __global__ __launch_bounds__(256) void conv_bits_rows_kernel(const ConvPairsPara
     for (unsigned long long o = j; o < (unsigned long long)p.n_out; o += step) p.mask_f[o] = 0u;
   for (unsigned long long w = j; w < p.n_words; w += step) {
     uint32_t word = p.bits[w];
+    if (word == 0u) continue;
     uint32_t row = p.prefix[w];
+    int4 c;
+    unsigned long long rest = split_site(w * 32ull, p.out_shape[2], p.out_inv[2], &c.w);
+    rest = split_site(rest, p.out_shape[1], p.out_inv[1], &c.z);
+    c.x = (int)split_site(rest, p.out_shape[0], p.out_inv[0], &c.y);
+    int at = 0;
     while (word != 0u) {
       const int b = __ffs((int)word) - 1;
       word &= word - 1u;
-      unsigned long long site = w * 32ull + (unsigned long long)b;
-      int4 c;
-      c.w = (int)(site % (unsigned long long)p.out_shape[2]); site /= (unsigned long long)p.out_shape[2];
-      c.z = (int)(site % (unsigned long long)p.out_shape[1]); site /= (unsigned long long)p.out_shape[1];
-      c.y = (int)(site % (unsigned long long)p.out_shape[0]); site /= (unsigned long long)p.out_shape[0];
-      c.x = (int)site;
+      c.w += b - at;
+      at = b;
+      while (c.w >= p.out_shape[2]) {
+        c.w -= p.out_shape[2];
+        if (++c.z == p.out_shape[1]) {
+          c.z = 0;
+          if (++c.y == p.out_shape[0]) {
+            c.y = 0;
+            ++c.x;
+          }
+        }
+      }
       if (row < (uint32_t)p.n_out) reinterpret_cast<int4 *>(p.out_coords)[row] = c;
       ++row;
     }
@@ -688,12 +818,12 @@ hipError_t launch_conv_pairs_fill(const ConvPairsParams &p, hipStream_t s) {
     if (wgs > 16384ull) wgs = 16384ull;
     hipLaunchKernelGGL(conv_bits_rows_kernel, dim3((unsigned)wgs), dim3(256), 0, s, p);
     if (p.n_in > 0)
-      hipLaunchKernelGGL(conv_pairs_fill_kernel<true>, dim3((p.n_in + 255) / 256, p.kv), dim3(256), 0, s, p);
+      hipLaunchKernelGGL(conv_bits_fill_kernel, dim3((p.n_in + 255) / 256, p.kv / p.kx), dim3(256), 0, s, p);
     return hipGetLastError();
   }
   hipLaunchKernelGGL(conv_pairs_rows_kernel, dim3((most + 255) / 256), dim3(256), 0, s, p);
   if (p.n_in > 0)
-    hipLaunchKernelGGL(conv_pairs_fill_kernel<false>, dim3((p.n_in + 255) / 256, p.kv), dim3(256), 0, s, p);
+    hipLaunchKernelGGL(conv_pairs_fill_kernel, dim3((p.n_in + 255) / 256, p.kv), dim3(256), 0, s, p);
   return hipGetLastError();
 }
 
@@ -709,15 +839,19 @@ hipError_t launch_conv_pairs_bits(const ConvPairsParams &p, void *temp, size_t t
   if (wgs == 0ull) wgs = 1ull;
   hipLaunchKernelGGL(conv_bits_clear_kernel, dim3((unsigned)wgs), dim3(256), 0, s, p);
   if (p.n_in > 0)
-    hipLaunchKernelGGL(conv_bits_sites_kernel, dim3((p.n_in + 255) / 256, p.kv), dim3(256), 0, s, p);
+    hipLaunchKernelGGL(conv_bits_sites_kernel, dim3((p.n_in + 255) / 256, p.kv / p.kx), dim3(256), 0, s, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const unsigned long long n_blocks = (p.n_words + kScanBlock - 1) / kScanBlock;
   if (n_blocks == 0ull || n_blocks > 0x7fffffffull || temp_bytes < conv_pairs_scan_temp_bytes((size_t)p.n_words)) return hipErrorInvalidValue;
   uint32_t *block_sums = reinterpret_cast<uint32_t *>(temp);
   hipLaunchKernelGGL(bit_scan_block_sums_kernel, dim3((unsigned)n_blocks), dim3(256), 0, s, p.bits, p.n_words, block_sums);
-  hipLaunchKernelGGL(bit_scan_block_offsets_kernel, dim3(1), dim3(256), 0, s, block_sums, n_blocks, p.prefix + p.n_words);
-  hipLaunchKernelGGL(bit_scan_write_kernel, dim3((unsigned)n_blocks), dim3(256), 0, s, p.bits, p.n_words, block_sums, p.prefix);
+  if (n_blocks <= kScanDirect) {
+    hipLaunchKernelGGL(bit_scan_write_kernel<true>, dim3((unsigned)n_blocks), dim3(256), 0, s, p.bits, p.n_words, block_sums, p.prefix);
+  } else {
+    hipLaunchKernelGGL(bit_scan_block_offsets_kernel, dim3(1), dim3(256), 0, s, block_sums, n_blocks);
+    hipLaunchKernelGGL(bit_scan_write_kernel<false>, dim3((unsigned)n_blocks), dim3(256), 0, s, p.bits, p.n_words, block_sums, p.prefix);
+  }
   return hipGetLastError();
 }
 

@@ -308,3 +308,41 @@ def test_sort_by_offset_count_against_the_host(n, kind):
         pairs.sort_by_mask_device(d_mask, 0xFFFFFFFF, by_offset_count=True)
     from cumm_amd.gemm.main import GemmMainUnitTest
     GemmMainUnitTest.device_synchronize()
+
+
+def _neighbourhoods(rng, centres, reach=3, each=40):
+    pts = (centres[:, None, :] + rng.integers(-reach, reach + 1, size=(centres.shape[0], each, 3))).reshape(-1, 3)
+    coords = np.unique(pts, axis=0)
+    return np.concatenate([np.zeros((coords.shape[0], 1), np.int64), coords], axis=1)
+
+
+def test_subm_pairs_keys_of_more_than_32_bits():
+    """Sites whose keys agree in the low 32 bits (512 x 4096 x 2048 sites are 2^32: batches 0 and 3 of that
+    grid; a grid of 4096 x 2048 x 2048 with z 1024 apart), beside neighbours of their own; and voxels next to
+    the 2^32-th site, whose neighbours' keys go on from zero in 32 bits."""
+    rng = np.random.default_rng(17)
+    centres = np.stack([rng.integers(8, 500, 60), rng.integers(8, 4000, 60), rng.integers(8, 2000, 60)], 1)
+    one = _neighbourhoods(rng, centres)
+    for shape, shift in (((512, 4096, 2048), (3, 0, 0, 0)), ((4096, 2048, 2048), (0, 1024, 0, 0))):
+        print("case wide keys", shape, flush=True)
+        first = one[(one[:, 1] < shape[0]) & (one[:, 2] < shape[1])]
+        second = first[rng.random(first.shape[0]) < 0.6] + np.array(shift)
+        coords = np.concatenate([first, second]).astype(np.int32)
+        _check_case(coords[rng.permutation(coords.shape[0])], shape)
+    edge = np.array([[0, 1023, 2047, 2047], [0, 1024, 0, 0], [0, 0, 0, 0], [0, 0, 0, 1], [0, 1024, 0, 1], [0, 1023, 2047, 2046]],
+                    np.int32)
+    _check_case(edge, (2048, 2048, 2048))
+
+
+@pytest.mark.parametrize("shape,batch", [((1, 1, 5000), 3), ((700, 9, 1), 2), ((9, 300, 2), 2), ((5, 33, 31), 4), ((64, 2048, 2048), 1)])
+@pytest.mark.parametrize("stride", [(1, 1, 1), (3, 5, 7)])
+def test_sparse_conv_pairs_line_lengths(shape, batch, stride):
+    """Output lines shorter than a word of the bitmap, strides that are no powers of two, and a grid whose
+    bitmap has more blocks than a workgroup of its scan adds up by itself."""
+    print("case sparse conv lines", shape, batch, stride, flush=True)
+    rng = np.random.default_rng(23)
+    n = 3000
+    coords = np.stack([rng.integers(0, m, n) for m in (batch,) + shape], 1).astype(np.int32)
+    coords = np.unique(coords, axis=0)
+    coords = coords[rng.permutation(coords.shape[0])]
+    _check_conv_case(coords, shape, stride=stride, batch_size=batch)
