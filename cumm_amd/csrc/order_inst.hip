@@ -19,10 +19,12 @@
 //     the order by count and hash.
 // Chain of kernels: clear - masks, keys and both histograms - two passes - position.  The passes are the
 // single-sweep kind (ticket, ranks by ballot, look-back, scatter; stable); they are bound by their
-// dependent round trips at 10^5 positions and by memory at 10^6.  The position kernel fetches only the
-// entries whose bit is set (one in twenty of a sparse cloud's) and writes -1 for the rest.
+// dependent round trips at 10^5 positions and by memory at 10^6; chunks of half the size on twice the
+// workgroups: 17.5 for 17.7 us at 300 k positions, 31.1 for 23.2 at 1.1 M.  The mask kernel reads the
+// tables at 4.2 TB/s.  The position kernel writes them again; what it fetches by row is little more
+// than a word pair per position (51.5 -> 39.1 us at 1.1 M positions against a fetch of mask and entries).
 // Measured (kernel times): the tables of a frame of 120 k voxels - submanifold and stride 2, 326 k output
-// sites - 125 us in ten launches; with masks by atomics, a sort each and a gather of every entry it
+// sites - 120 us in ten launches; with masks by atomics, a sort each and a gather of every entry it
 // was 305 us in 27.
 #include <cstring>
 
@@ -36,16 +38,16 @@ namespace {
 constexpr int kDigit = 9, kDigitBins = 1 << kDigit;      // 512
 constexpr int kKeyBits = 2 * kDigit;
 constexpr int kPassThreads = 1024, kPassWaves = kPassThreads / 64;
+constexpr int kMaskBatch = 16;                            // table rows whose loads are in flight together
 constexpr int kHistCopies = 8;                            // spread of the histogram atomics
 constexpr int kExact = 5;                                 // offsets up to which a one-word key is exact
 constexpr uint32_t kAggregate = 1u << 30, kInclusive = 2u << 30, kCount = (1u << 30) - 1u;
 constexpr int kSpins = 1 << 20;                           // (about a second)
-constexpr int kPosOffsets = 16;                            // offsets per workgroup of the position kernel
 
 struct Side {
   const int32_t *indices;      // [kv, n]
   int32_t n, chunks;
-  uint32_t *raw;               // [n, words] masks by row
+  uint32_t *raw;               // [n, words] masks by row; one word: [n, 2] mask and lead
   uint32_t *keys;              // [n]
   int32_t *tmp_rows;           // [n] after the first pass
   uint16_t *tmp_high;          // [n]
@@ -134,6 +136,10 @@ __device__ __forceinline__ uint32_t words_key(const OrderParams &p, const uint32
   return (planes << (kKeyBits - 12)) | (h >> (32 - (kKeyBits - 12)));
 }
 
+// What lies beside a one-word mask: is the row's entry for the middle offset the row itself (as
+// everywhere in a submanifold table), and the entry of its lowest other offset.
+constexpr uint32_t kSelf = 0x80000000u, kLeadEntry = 0x7FFFFFFFu;
+
 // side and index inside it of a workgroup, when side 0 has `first` workgroups
 __device__ __forceinline__ int side_of(int first, int *block) {
   const int s = *block >= first ? 1 : 0;
@@ -142,7 +148,7 @@ __device__ __forceinline__ int side_of(int first, int *block) {
 }
 
 // One position per lane: its mask out of the table (every row read coalesced, kv independent loads), its
-// key, and the digits of the key into the histograms of both passes.
+// key, the entry of its lowest offset, and the digits of the key into the histograms of both passes.
 template <int WORDS>
 __global__ __launch_bounds__(256) void order_masks_kernel(const OrderParams p) {
   __shared__ uint32_t hist[2][kDigitBins];
@@ -153,22 +159,38 @@ __global__ __launch_bounds__(256) void order_masks_kernel(const OrderParams p) {
   const int o = block * 256 + t;
   const bool on = o < d.n;
   uint32_t w[4] = {0u, 0u, 0u, 0u};
-  const int32_t *col = d.indices + (on ? o : 0);
+  uint32_t lead = 0u;
+  bool self = false;
+  // (kv * n entries are below 2^31 bytes: the row of the table is a scalar offset)
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t *>(d.indices), 0,
+                                                                      (int)((uint32_t)p.kv * (uint32_t)d.n * 4u), 0x00020000);
+  const uint32_t at = (uint32_t)(on ? o : 0) * 4u;
 #pragma unroll
   for (int q = 0; q < WORDS; ++q) {
     const int hi = p.kv - 32 * q < 32 ? p.kv - 32 * q : 32;
-    for (int b0 = 0; b0 < hi; b0 += 8) {
-      int v[8];
+    for (int b0 = ((hi - 1) / kMaskBatch) * kMaskBatch; b0 >= 0; b0 -= kMaskBatch) {      // (the lowest offset last)
+      int v[kMaskBatch];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = col[(int64_t)(32 * q + (b0 + u < hi ? b0 + u : 0)) * d.n];
+      for (int u = 0; u < kMaskBatch; ++u) v[u] = __builtin_amdgcn_raw_buffer_load_b32(rs, at, (32 * q + (b0 + u < hi ? b0 + u : 0)) * d.n * 4, 0);
 #pragma unroll
-      for (int u = 0; u < 8; ++u) w[q] |= b0 + u < hi && v[u] >= 0 ? 1u << (b0 + u) : 0u;
+      for (int u = kMaskBatch - 1; u >= 0; --u) {
+        const bool has = b0 + u < hi && v[u] >= 0;
+        w[q] |= has ? 1u << (b0 + u) : 0u;
+        if constexpr (WORDS == 1) {
+          if (b0 + u == p.kv / 2) self = v[u] == o;
+          else lead = has ? (uint32_t)v[u] : lead;
+        }
+      }
     }
   }
   const uint32_t key = WORDS == 1 ? word_key(p, w[0]) : words_key(p, w);
   if (on) {
+    if constexpr (WORDS == 1) {
+      reinterpret_cast<uint2 *>(d.raw)[o] = uint2{w[0], self ? lead | kSelf : lead};
+    } else {
 #pragma unroll
-    for (int q = 0; q < WORDS; ++q) d.raw[(int64_t)o * WORDS + q] = w[q];
+      for (int q = 0; q < WORDS; ++q) d.raw[(int64_t)o * WORDS + q] = w[q];
+    }
     d.keys[o] = key;
   }
   __syncthreads();
@@ -327,9 +349,13 @@ __global__ __launch_bounds__(kPassThreads) void order_pass_kernel(const OrderPar
   }
 }
 
-// 256 positions and kPosOffsets offsets per workgroup: masks, table(s) by position, and (offset slice 0)
-// the counts of the launch hints - as sort_finish_kernel, whose remarks on give-ups hold here too: the
-// identity order replaces one that cannot be trusted.
+// 256 positions and the offsets of one mask word per workgroup: masks, table(s) by position, and (one
+// word) the counts of the launch hints - as sort_finish_kernel, whose remarks on give-ups hold here too:
+// the identity order replaces one that cannot be trusted.  A fetch by row costs a sector for four
+// bytes: of one-word masks the lowest offset's entry comes with the mask, the middle one's is mostly
+// the row itself, and of the others those are fetched that some lane of the wave has (the positions are
+// sorted by their masks: few).  (Mask and entry carried through both passes instead: 14 us less here
+// at 1.1 M positions, 20 us more there.)
 constexpr int kLight = 3, kHeavy = 10;
 template <int WORDS>
 __global__ __launch_bounds__(256) void order_position_kernel(const OrderParams p) {
@@ -340,28 +366,49 @@ __global__ __launch_bounds__(256) void order_position_kernel(const OrderParams p
   const int pos = block * 256 + t;
   const bool on = pos < d.n;
   const bool broken = p.give_ups != nullptr && __hip_atomic_load(p.give_ups, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
-  int row = on ? (broken ? pos : d.order[pos]) : -1;
-  const int k0 = blockIdx.y * kPosOffsets;
-  const int word = k0 / 32;
-  const bool have = row >= 0 && row < d.n;
-  const uint32_t mine = have ? d.raw[(int64_t)row * WORDS + word] : 0u;
-  const uint32_t bits = mine >> (k0 & 31);
-  int v[kPosOffsets];
+  const int row = on ? (broken ? pos : d.order[pos]) : -1;
+  const int word = blockIdx.y, k0 = 32 * word;
+  uint32_t mine = 0u, lead = 0u;
+  if (row >= 0 && row < d.n) {
+    if constexpr (WORDS == 1) {
+      const uint2 both = reinterpret_cast<const uint2 *>(d.raw)[row];
+      mine = both.x;
+      lead = both.y;
+    } else {
+      mine = d.raw[(int64_t)row * WORDS + word];
+    }
+  }
+  const int middle = p.kv / 2;
+  const bool self = (lead & kSelf) != 0u;
+  const int lead_at = WORDS == 1 ? __ffs((int)(mine & ~(1u << middle))) - 1 : -1;
+  uint32_t fetch = mine;
+  if (lead_at >= 0) fetch &= ~(1u << lead_at);
+  if (self) fetch &= ~(1u << middle);
+  const uint32_t fetch_or = wave_or_dpp(fetch);
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t *>(d.indices), 0,
                                                                       (int)((uint32_t)p.kv * (uint32_t)d.n * 4u), 0x00020000);
+  int v[32];
 #pragma unroll
-  for (int u = 0; u < kPosOffsets; ++u)      // (a clear bit is fetched outside the table: no memory is touched)
-    v[u] = __builtin_amdgcn_raw_buffer_load_b32(rs, (bits >> u) & 1u ? (uint32_t)((k0 + u) * d.n + row) * 4u : 0x80000000u, 0, 0);
+  for (int u = 0; u < 32; ++u) {
+    v[u] = u == lead_at ? (int)(lead & kLeadEntry) : (self && u == middle ? row : -1);
+    if ((fetch_or >> u) & 1u) {      // (a clear bit is fetched outside the table: no memory is touched)
+      const int e = __builtin_amdgcn_raw_buffer_load_b32(
+          rs, (fetch >> u) & 1u ? (uint32_t)((k0 + u) * d.n + row) * 4u : 0x80000000u, 0, 0);
+      v[u] = (fetch >> u) & 1u ? e : v[u];
+    }
+  }
+  const int bytes = (int)((uint32_t)p.kv * (uint32_t)d.n * 4u);
+  const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(d.by_pos, 0, bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rev = __builtin_amdgcn_make_buffer_rsrc(d.by_pos_rev, 0, d.by_pos_rev ? bytes : 0, 0x00020000);
   if (on) {
 #pragma unroll
-    for (int u = 0; u < kPosOffsets; ++u) {
+    for (int u = 0; u < 32; ++u) {
       if (k0 + u >= p.kv) break;
-      const int e = (bits >> u) & 1u ? v[u] : -1;
-      d.by_pos[(int64_t)(k0 + u) * d.n + pos] = e;
-      if (d.by_pos_rev != nullptr) d.by_pos_rev[(int64_t)(p.kv - 1 - k0 - u) * d.n + pos] = e;
+      __builtin_amdgcn_raw_buffer_store_b32(v[u], to, (uint32_t)pos * 4u, (k0 + u) * d.n * 4, 0);
+      if (d.by_pos_rev != nullptr) __builtin_amdgcn_raw_buffer_store_b32(v[u], rev, (uint32_t)pos * 4u, (p.kv - 1 - k0 - u) * d.n * 4, 0);
     }
-    if ((k0 & 31) == 0) d.sorted[(int64_t)pos * WORDS + word] = mine;
-    if (broken && blockIdx.y == 0) d.order[pos] = pos;
+    d.sorted[(int64_t)pos * WORDS + word] = mine;
+    if (broken && word == 0) d.order[pos] = pos;
   }
   if (WORDS > 1 || blockIdx.y != 0 || d.hint_slot == nullptr) return;
   if (broken) {
@@ -396,7 +443,7 @@ int pass_items(int n) { return n <= (1 << 18) ? 4 : 8; }
 size_t order_pairs_workspace_bytes(int n, int words) {
   const size_t nn = (size_t)(n > 0 ? n : 1);
   const size_t chunks = (nn + 4095) / 4096;
-  return up256(4 * nn * words) + 2 * up256(4 * nn) + up256(2 * nn) + up256(4 * 2 * kHistCopies * kDigitBins) +
+  return up256(4 * nn * (words == 1 ? 2 : words)) + 2 * up256(4 * nn) + up256(2 * nn) + up256(4 * 2 * kHistCopies * kDigitBins) +
          up256(4 * 2 * chunks * kDigitBins) + 256;
 }
 
@@ -420,7 +467,7 @@ hipError_t launch_order_pairs(const OrderPairsSide *sides, int n_sides, int kv, 
     d.sorted = sides[i].sorted; d.order = sides[i].order; d.by_pos = sides[i].by_pos; d.by_pos_rev = sides[i].by_pos_rev;
     d.hint_slot = p.words == 1 ? sides[i].hint_slot : nullptr;
     char *const begin = at;
-    d.raw = reinterpret_cast<uint32_t *>(take(4 * n * p.words));
+    d.raw = reinterpret_cast<uint32_t *>(take(4 * n * (p.words == 1 ? 2 : p.words)));
     d.keys = reinterpret_cast<uint32_t *>(take(4 * n));
     d.tmp_rows = reinterpret_cast<int32_t *>(take(4 * n));
     d.tmp_high = reinterpret_cast<uint16_t *>(take(2 * n));
@@ -474,7 +521,7 @@ hipError_t launch_order_pairs(const OrderPairsSide *sides, int n_sides, int kv, 
     if (items == 4) hipLaunchKernelGGL(order_pass_kernel<4>, dim3(chunks), dim3(kPassThreads), 0, s, p);
     else hipLaunchKernelGGL(order_pass_kernel<8>, dim3(chunks), dim3(kPassThreads), 0, s, p);
   }
-  const dim3 grid(blocks, (kv + kPosOffsets - 1) / kPosOffsets);
+  const dim3 grid(blocks, p.words);
   switch (p.words) {
   case 1: hipLaunchKernelGGL(order_position_kernel<1>, grid, dim3(256), 0, s, p); break;
   case 2: hipLaunchKernelGGL(order_position_kernel<2>, grid, dim3(256), 0, s, p); break;

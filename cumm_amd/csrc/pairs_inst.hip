@@ -80,9 +80,12 @@ __device__ __forceinline__ uint32_t coord_line(int b, int z, int y, const SubmPa
   return ((uint32_t)b * (uint32_t)p.shape[0] + (uint32_t)z) * (uint32_t)p.shape[1] + (uint32_t)y;
 }
 // presence word of the 32 sites (b, z, y, 32*(x/32) ..): hashed, without a key, so a set bit
-// means "maybe" (two runs may share a word) and a clear bit means "certainly absent"
-__device__ __forceinline__ uint32_t presence_index(uint32_t line, int run, const SubmPairsParams &p) {
-  return mix32(line * (uint32_t)((p.shape[2] + 31) >> 5) + (uint32_t)run) & p.filter_mask;
+// means "maybe" (two runs may share a word) and a clear bit means "certainly absent".  The words of
+// 2 x 8 lines lie in one 64-byte block: the neighbours of a voxel are in a few of them
+__device__ __forceinline__ uint32_t presence_index(int b, int z, int y, int run, const SubmPairsParams &p) {
+  const uint32_t block = (((uint32_t)b * (uint32_t)((p.shape[0] + 1) >> 1) + (uint32_t)(z >> 1)) * (uint32_t)((p.shape[1] + 7) >> 3) +
+                          (uint32_t)(y >> 3)) * (uint32_t)((p.shape[2] + 31) >> 5) + (uint32_t)run;
+  return ((mix32(block) << 4) | (uint32_t)((z & 1) << 3) | (uint32_t)(y & 7)) & p.filter_mask;
 }
 // is the row of a slot whose low word matches the site (b, z, y, x)?  Keys of 32 bits say all
 __device__ __forceinline__ bool same_site(const SubmPairsParams &p, uint32_t wide, uint32_t row, unsigned long long key) {
@@ -97,7 +100,7 @@ __global__ __launch_bounds__(256) void pairs_insert_kernel(const SubmPairsParams
   const int4 c = reinterpret_cast<const int4 *>(p.coords)[i];
   const unsigned long long key = coord_key(c.x, c.y, c.z, c.w, p);
   unsigned long long *table = reinterpret_cast<unsigned long long *>(p.table);
-  atomicOr(&p.filter[presence_index(coord_line(c.x, c.y, c.z, p), c.w >> 5, p)], 1u << (c.w & 31));
+  atomicOr(&p.filter[presence_index(c.x, c.y, c.z, c.w >> 5, p)], 1u << (c.w & 31));
   const uint32_t low = (uint32_t)key;
   // do this key and those of all sites around it (which lie in the same grid) fit 32 bits?
   const unsigned long long last = coord_key(c.x, p.shape[0] - 1, p.shape[1] - 1, p.shape[2] - 1, p);
@@ -114,15 +117,31 @@ __global__ __launch_bounds__(256) void pairs_insert_kernel(const SubmPairsParams
   }
 }
 
+// Workgroups go to the eight XCDs in turn.  This hands each of them a contiguous run of the inputs, all
+// lines of offsets of a block of inputs one after the other, so that what neighbours share is fetched
+// into one L2: -> block of inputs (or one past the last), *zy = line of offsets.
+constexpr unsigned kXcds = 8;
+__host__ __device__ __forceinline__ unsigned xcd_grid(unsigned blocks, unsigned lines) {
+  return kXcds * ((blocks + kXcds - 1) / kXcds) * lines;
+}
+__device__ __forceinline__ int xcd_block(unsigned lines, int *zy) {
+  const unsigned per = gridDim.x / (kXcds * lines), j = blockIdx.x / kXcds;
+  *zy = (int)(j % lines);
+  return (int)((blockIdx.x % kXcds) * per + j / lines);
+}
+
 // One lane per (voxel, (kz, ky)): it walks the KX offsets along x.  19 of 20 look-ups of a sparse
 // cloud are misses, and a miss in the table costs two or more 64-byte sectors; the presence word
 // of the neighbour's run of 32 sites answers all of a row's x-neighbours with one 4-byte load from
-// a table that stays in L2, and only "maybe" goes on to the hash table.  grid.y = KZ*KY,
-// consecutive lanes = consecutive voxels: every table row is written coalesced.  The masks are
-// OR-ed with atomics, one per lane with a pair, into words that the clear kernel set.
+// a table that stays in L2, and only "maybe" goes on to the hash table.
+// Consecutive lanes = consecutive voxels: every table row is written coalesced.  The masks are
+// OR-ed with atomics, one per lane with a pair, into words that the clear kernel set.  With the
+// presence words of neighbouring lines in one block, the workgroups in runs per XCD and the loads of
+// three offsets in flight: 44 -> 33 us at 300 k voxels; at 120 k the 23 us stay, the chain coordinates
+// - presence - slot, cold in every L2.
 __global__ __launch_bounds__(256) void pairs_lookup_kernel(const SubmPairsParams p) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  const int zy = blockIdx.y;
+  int zy;
+  const int i = xcd_block((unsigned)(p.kv / p.kx), &zy) * 256 + threadIdx.x;
   if (i >= p.n) return;
   const int4 c = reinterpret_cast<const int4 *>(p.coords)[i];
   const unsigned long long *table = reinterpret_cast<const unsigned long long *>(p.table);
@@ -130,43 +149,53 @@ __global__ __launch_bounds__(256) void pairs_lookup_kernel(const SubmPairsParams
   const int z = c.y + p.off[zy * p.kx][0], y = c.z + p.off[zy * p.kx][1];
   const bool line_in = z >= 0 && z < p.shape[0] && y >= 0 && y < p.shape[1];
   const uint32_t line = coord_line(c.x, z, y, p);
-  int have_run = -1;
-  uint32_t word = 0, bits_f = 0, bits_b = 0;
-  for (int kx = 0; kx < p.kx; ++kx) {
-    const int k = zy * p.kx + kx;
-    if (k == p.center_k) {
-      p.ind_f[(int64_t)k * p.n + i] = i;
-      if (p.ind_b) p.ind_b[(int64_t)(p.kv - 1 - k) * p.n + i] = i;
-      continue;
+  uint32_t bits_f = 0, bits_b = 0;
+  constexpr int kBatch = 3;      // offsets whose loads are in flight together
+  for (int kx0 = 0; kx0 < p.kx; kx0 += kBatch) {
+    uint32_t word[kBatch], low[kBatch], h[kBatch];
+    unsigned long long slot[kBatch];
+    bool maybe[kBatch];
+    int x[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const int k = zy * p.kx + (kx0 + u < p.kx ? kx0 + u : kx0);
+      x[u] = c.w + p.off[k][2];
+      maybe[u] = kx0 + u < p.kx && k != p.center_k && line_in && x[u] >= 0 && x[u] < p.shape[2];
+      word[u] = 0u;
+      // (the words of one run are one load for most lanes)
+      if (maybe[u]) word[u] = u > 0 && maybe[u - 1] && (x[u] >> 5) == (x[u - 1] >> 5) ? 0u : p.filter[presence_index(c.x, z, y, x[u] >> 5, p)];
     }
-    const int x = c.w + p.off[k][2];
-    int row = -1;
-    if (line_in && x >= 0 && x < p.shape[2]) {
-      if ((x >> 5) != have_run) {
-        have_run = x >> 5;
-        word = p.filter[presence_index(line, have_run, p)];
-      }
-      if ((word >> (x & 31)) & 1u) {
-        const uint32_t low = line * (uint32_t)p.shape[2] + (uint32_t)x;
-        const unsigned long long key = wide != 0u ? coord_key(c.x, z, y, x, p) : 0ull;
-        uint32_t h = mix32(low) & p.slot_mask;
-        // a collision walks on until the key or an empty slot turns up (the table is never full)
-        for (uint32_t probe = 0; probe <= p.slot_mask; ++probe) {
-          const unsigned long long s = table[h];
-          if (s == kEmptySlot) break;
-          if ((uint32_t)s == low && same_site(p, wide, (uint32_t)(s >> 32), key)) {
-            row = (int)(uint32_t)(s >> 32);
-            break;
-          }
-          h = (h + 1) & p.slot_mask;
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      if (u > 0 && maybe[u] && maybe[u - 1] && (x[u] >> 5) == (x[u - 1] >> 5)) word[u] = word[u - 1];
+      low[u] = line * (uint32_t)p.shape[2] + (uint32_t)x[u];
+      h[u] = mix32(low[u]) & p.slot_mask;
+      slot[u] = kEmptySlot;
+    }
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+      if (maybe[u] && ((word[u] >> (x[u] & 31)) & 1u)) slot[u] = table[h[u]];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      if (kx0 + u >= p.kx) break;
+      const int k = zy * p.kx + kx0 + u;
+      int row = k == p.center_k ? i : -1;
+      // a collision walks on until the key or an empty slot turns up (the table is never full)
+      for (uint32_t probe = 0; slot[u] != kEmptySlot && probe <= p.slot_mask; ++probe) {
+        if ((uint32_t)slot[u] == low[u] &&
+            same_site(p, wide, (uint32_t)(slot[u] >> 32), wide != 0u ? coord_key(c.x, z, y, x[u], p) : 0ull)) {
+          row = (int)(uint32_t)(slot[u] >> 32);
+          break;
         }
+        h[u] = (h[u] + 1) & p.slot_mask;
+        slot[u] = table[h[u]];
       }
-    }
-    p.ind_f[(int64_t)k * p.n + i] = row;
-    if (p.ind_b) p.ind_b[(int64_t)(p.kv - 1 - k) * p.n + i] = row;
-    if (row >= 0 && k < 32) {      // (masks of one word only)
-      bits_f |= 1u << k;
-      bits_b |= 1u << ((p.kv - 1 - k) & 31);
+      p.ind_f[(int64_t)k * p.n + i] = row;
+      if (p.ind_b) p.ind_b[(int64_t)(p.kv - 1 - k) * p.n + i] = row;
+      if (row >= 0 && k < 32 && k != p.center_k) {      // (masks of one word only)
+        bits_f |= 1u << k;
+        bits_b |= 1u << ((p.kv - 1 - k) & 31);
+      }
     }
   }
   if (p.mask_f && bits_f) atomicOr(&p.mask_f[i], bits_f);
@@ -361,8 +390,9 @@ __device__ __forceinline__ bool conv_out_line(const ConvPairsParams &p, const in
   return in && c.x >= 0 && c.x < p.batch;
 }
 
-// One lane per (input, (kz, ky)), grid.y = KZ * KY: the sites of a line that fall into one word go out in
-// one atomic.  (One lane per (input, offset) with divisions in 64 bits: 18.4 us at 120 k voxels, 32.7 at
+// One lane per (input, (kz, ky)): the sites of a line that fall into one word go out in
+// one atomic.  grid.y = KZ * KY, so that the lanes that repeat a site mostly run after the one that sets it
+// (in the order of xcd_block they run beside it: 25.6 against 18.0 us).  (One lane per (input, offset) with divisions in 64 bits: 18.4 us at 120 k voxels, 32.7 at
 // 300 k; the arithmetic was what bound it.)
 __global__ __launch_bounds__(256) void conv_bits_sites_kernel(const ConvPairsParams p) {
   const int i = blockIdx.x * 256 + threadIdx.x;
@@ -389,8 +419,8 @@ __global__ __launch_bounds__(256) void conv_bits_sites_kernel(const ConvPairsPar
 
 // the pairs of those lanes: backward table coalesced, forward entries where they belong
 __global__ __launch_bounds__(256) void conv_bits_fill_kernel(const ConvPairsParams p) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  const int zy = blockIdx.y;
+  int zy;
+  const int i = xcd_block((unsigned)(p.kv / p.kx), &zy) * 256 + threadIdx.x;
   if (i >= p.n_in) return;
   const int4 c = reinterpret_cast<const int4 *>(p.coords)[i];
   unsigned long long first, at = ~0ull;
@@ -818,7 +848,7 @@ hipError_t launch_conv_pairs_fill(const ConvPairsParams &p, hipStream_t s) {
     if (wgs > 16384ull) wgs = 16384ull;
     hipLaunchKernelGGL(conv_bits_rows_kernel, dim3((unsigned)wgs), dim3(256), 0, s, p);
     if (p.n_in > 0)
-      hipLaunchKernelGGL(conv_bits_fill_kernel, dim3((p.n_in + 255) / 256, p.kv / p.kx), dim3(256), 0, s, p);
+      hipLaunchKernelGGL(conv_bits_fill_kernel, dim3(xcd_grid((unsigned)(p.n_in + 255) / 256u, (unsigned)(p.kv / p.kx))), dim3(256), 0, s, p);
     return hipGetLastError();
   }
   hipLaunchKernelGGL(conv_pairs_rows_kernel, dim3((most + 255) / 256), dim3(256), 0, s, p);
@@ -862,7 +892,7 @@ hipError_t launch_subm_pairs(const SubmPairsParams &p, hipStream_t s) {
   if ((uint32_t)p.n > most) most = (uint32_t)p.n;
   hipLaunchKernelGGL(pairs_clear_kernel, dim3((most + 255) / 256), dim3(256), 0, s, p);
   hipLaunchKernelGGL(pairs_insert_kernel, dim3((p.n + 255) / 256), dim3(256), 0, s, p);
-  hipLaunchKernelGGL(pairs_lookup_kernel, dim3((p.n + 255) / 256, p.kv / p.kx), dim3(256), 0, s, p);
+  hipLaunchKernelGGL(pairs_lookup_kernel, dim3(xcd_grid((unsigned)(p.n + 255) / 256u, (unsigned)(p.kv / p.kx))), dim3(256), 0, s, p);
   return hipGetLastError();
 }
 
