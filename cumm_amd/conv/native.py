@@ -8,7 +8,7 @@ of its kernels, cumm/conv/main_real_spconv.py:309-403:
 
     forward          out[pair_out[k]]  += inp[pair_in[k]]   @ W[:, k, :].T     (matmul2, ShuffleAC)
     backward-input   dinp[pair_in[k]]  += dout[pair_out[k]] @ W[:, k, :]       (matmul2, ShuffleAC)
-    backward-weight  dW[:, k, :]        = dout[pair_out[k]].T @ inp[pair_in[k]] (matmul2, ShuffleAB)
+    backward-weight  dW[:, k, :]        = dout[pair_out[k]].T @ inp[pair_in[k]] (all offsets in one call)
 
 Forward and backward-input accumulate all offsets in an fp32 image (the f16 / bf16 -> f32 kernels)
 and round once at the end (``cumm_hip_finish_rows``, with bias and activation): one rounding, as
@@ -163,7 +163,7 @@ def backward_input(dout: tv.Tensor, weight: tv.Tensor, dinp: tv.Tensor, lists, *
     plan_backward_input(dout, weight, dinp, lists, stream=stream, acc=acc)()
 
 
-class _WeightPlan:
+class WeightPlan:
     """Backward-weight of all kernel offsets in one call of the library (``cumm_hip_wgrad_pairs``),
     validated once: run on the tensors it was made for, or through ``rebind`` on others of the same
     shapes and types by address."""
@@ -211,16 +211,55 @@ class _WeightPlan:
         return self._pairs[3]
 
 
-def plan_backward_weight(dout: tv.Tensor, inp: tv.Tensor, dweight: tv.Tensor, lists, *, stream: int = 0) -> _WeightPlan:
+def plan_backward_weight(dout: tv.Tensor, inp: tv.Tensor, dweight: tv.Tensor, lists, *, stream: int = 0):
     """Backward-weight as a reusable plan: dweight[:, k, :] of every kernel offset (zeros for an
     offset without pairs)."""
     _check(inp, dweight, lists, dout.dim(0))
     if dout.dim(1) != dweight.dim(0) or dout.dtype != inp.dtype or dweight.dim(2) != inp.dim(1):
         raise RuntimeError("error")
-    for t in (dout, inp, dweight):
-        if t.device < 0 or not t.is_contiguous():
-            raise ValueError("operands must be contiguous device tensors")
-    return _WeightPlan(dout, inp, dweight, lists, stream)
+    if not _in_one_call(dout, inp, dweight, lists):
+        return WeightSteps(dout, inp, dweight, lists, stream)
+    return WeightPlan(dout, inp, dweight, lists, stream)
+
+
+def _in_one_call(dout, inp, dweight, lists) -> bool:
+    """What ``cumm_hip_wgrad_pairs`` takes: whole tensors at 16-byte addresses, up to 128 offsets."""
+    return (all(t.is_contiguous() and t.byte_pointer() % 16 == 0 for t in (dout, inp, dweight)) and
+            lists.pair_in.is_contiguous() and lists.pair_out.is_contiguous() and lists.pair_in.shape == lists.pair_out.shape and
+            dweight.dim(1) <= 128)
+
+
+class WeightSteps:
+    """Backward-weight as one gathered product per kernel offset: rows with a stride of their own, more
+    offsets than one call takes."""
+
+    _NO_PAIR = {}
+
+    def __init__(self, dout, inp, dweight, lists, stream):
+        self.steps = []
+        for k in range(dweight.dim(1)):
+            cnt = int(lists.counts[k])
+            p = GemmParams()
+            p.algo_desp = _find(inp.dtype, inp.dtype, ShuffleStrideType.ShuffleAB, 64, 64, True, False).copy()
+            p.a, p.b, p.c = dout, inp, dweight.select(1, k)
+            if cnt > 0:
+                p.a_inds = lists.pair_out.select(0, k).slice_first_axis(0, cnt)
+                p.b_inds = lists.pair_in.select(0, k).slice_first_axis(0, cnt)
+            else:      # one step of absent rows writes the zeros
+                dev = inp.device
+                if dev not in self._NO_PAIR:
+                    self._NO_PAIR[dev] = tv.from_numpy(np.full(32, -1, np.int32)).cuda()
+                p.a_inds = p.b_inds = self._NO_PAIR[dev]
+            p.stream = stream
+            self.steps.append(p)
+
+    def __call__(self) -> None:
+        for p in self.steps:
+            GemmMainUnitTest.matmul2(p)
+
+    @property
+    def launches(self) -> int:
+        return len(self.steps)
 
 
 def backward_weight(dout: tv.Tensor, inp: tv.Tensor, dweight: tv.Tensor, lists, *, split_k_slices: int = 1,
@@ -229,6 +268,7 @@ def backward_weight(dout: tv.Tensor, inp: tv.Tensor, dweight: tv.Tensor, lists, 
     ``split_k_slices`` is what a caller of the per-offset products would pass; the pairs are spread
     over the device in any case.  ``workspace`` is used when it is large enough."""
     plan = plan_backward_weight(dout, inp, dweight, lists, stream=stream)
-    if workspace is not None and not workspace.empty() and workspace.nbytes >= plan.workspace_bytes:
+    if (isinstance(plan, WeightPlan) and workspace is not None and not workspace.empty() and
+            workspace.nbytes >= plan.workspace_bytes and workspace.byte_pointer() % 16 == 0):
         plan._workspace = workspace
     plan()      # (a workspace of its own goes away with the plan: freeing device memory waits for it)

@@ -387,8 +387,7 @@ class _SparseConvFunction(torch.autograd.Function):
             key = ("wgrad_pairs", dtype, weight.shape)
             plan = g._launches.get(key)
             if plan is None:
-                plan = native.plan_backward_weight(torch2tensor(grad_out), torch2tensor(features), torch2tensor(grad_w),
-                                                   g.lists, stream=stream)
+                plan = native.WeightPlan(torch2tensor(grad_out), torch2tensor(features), torch2tensor(grad_w), g.lists, stream)
                 plan.release()      # (every call brings its own tensors)
                 g._launches[key] = plan
             ws = _bytes(plan.workspace_bytes, grad_out.device)

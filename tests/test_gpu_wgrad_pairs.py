@@ -87,3 +87,26 @@ def test_shuffle_ab_epilogue_on_either_side_of_the_dispatch(pairs, dtype, out):
     assert np.abs(got - ref).max() <= tol * max(np.abs(ref).max(), 1.0)
     cd = desp_to_c(p.algo_desp)
     assert (int(_capi.lib().cumm_hip_query_gemm_optional_workspace(ctypes.byref(cd), m, n, pairs)) > 0) == (pairs >= 256)
+
+
+@pytest.mark.parametrize("kv,wide", [(27, True), (130, False), (130, True)])
+def test_backward_weight_of_strided_rows_and_of_more_offsets_than_one_call_takes(kv, wide):
+    """Features and gradients that are columns of wider tensors, and more than 128 offsets: one product per
+    offset, with the results of whole tensors."""
+    from types import SimpleNamespace
+    from cumm_amd.conv import native
+    print("case backward_weight", kv, wide, flush=True)
+    rng = np.random.default_rng(kv)
+    rows, k_out, c_in, most = 600, 24, 40, 300
+    dout, inp = _data(rng, (rows, k_out + 8 * wide), "f16"), _data(rng, (rows, c_in + 16 * wide), "f16")
+    counts = rng.integers(0, most, size=kv).astype(np.int32)
+    counts[3] = 0
+    po, pi = (rng.integers(0, rows, size=(kv, most)).astype(np.int32) for _ in range(2))
+    view = lambda a, n: H.dev(a, "f16").slice_axis(1, 0, n) if wide else H.dev(a, "f16")
+    dw = H.dev(_data(rng, (k_out, kv, c_in), "f16"), "f16")
+    lists = SimpleNamespace(pair_in=H.dev(pi, "i32"), pair_out=H.dev(po, "i32"), counts=counts)
+    native.backward_weight(view(dout, k_out), view(inp, c_in), dw, lists)
+    got = H.as_f32(H.host(dw), "f16")
+    f_out, f_in = H.as_f32(dout, "f16")[:, :k_out], H.as_f32(inp, "f16")[:, :c_in]
+    ref = np.stack([f_out[po[r, :n]].T @ f_in[pi[r, :n]] for r, n in enumerate(counts)], axis=1)
+    assert np.abs(got - ref).max() <= TOL["f16"] * max(np.abs(ref).max(), 1.0)
