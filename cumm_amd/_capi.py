@@ -92,6 +92,7 @@ SYMBOLS = {
     "cumm_hip_memset": (C.c_int, [_VP, C.c_int, C.c_size_t, _VP]),
     "cumm_hip_stream_create": (C.c_int, [_PVP]),
     "cumm_hip_stream_destroy": (C.c_int, [_VP]),
+    "cumm_hip_stream_is_capturing": (C.c_int, [_VP]),
     "cumm_hip_stream_synchronize": (C.c_int, [_VP]),
     "cumm_hip_device_synchronize": (C.c_int, []),
     "cumm_hip_take_async_errors": (C.c_int, [C.POINTER(C.c_int32)]),

@@ -1084,6 +1084,12 @@ int cumm_hip_stream_destroy(void *stream) {
   HIP_TRY(hipStreamDestroy(reinterpret_cast<hipStream_t>(stream)));
   return CUMM_HIP_OK;
 }
+int cumm_hip_stream_is_capturing(void *stream) {
+  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(reinterpret_cast<hipStream_t>(stream), &s) == hipSuccess) return s != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return 1;
+}
 int cumm_hip_stream_synchronize(void *stream) {
   HIP_TRY(hipStreamSynchronize(reinterpret_cast<hipStream_t>(stream)));
   return report_async_errors();

@@ -83,6 +83,15 @@ def _check_device(*tens):
         raise RuntimeError("operands must be device tensors (call .cuda() first)")
 
 
+def _outside_graphs(fn, args):
+    """The entry point, without the workspace that belongs to the argument block while its stream is
+    recorded into a graph."""
+    bare = _capi.GemmArgs.from_buffer_copy(args)
+    bare.workspace, bare.workspace_bytes = None, 0
+    bare_ref, capturing = ctypes.byref(bare), _capi.lib().cumm_hip_stream_is_capturing
+    return lambda cdesc_ref, args_ref, stream: fn(cdesc_ref, bare_ref if capturing(stream) else args_ref, stream)
+
+
 class GemmMainUnitTest:
     """Static operator functions, as the reference's pybind class."""
 
@@ -246,6 +255,7 @@ class GemmMainUnitTest:
                 raise ValueError("operands must be contiguous along their last dimension")
 
         workspace = params.workspace
+        optional = recorded = 0
         workspace_size = desp.query_workspace_size(m, n, k, split_k_slices)
         if workspace_size > 0:
             if not workspace.empty():
@@ -255,10 +265,13 @@ class GemmMainUnitTest:
                 workspace = empty([workspace_size], uint8, 0)
         else:
             # one slice needs no workspace (the caller's, which other calls may share, stays unused); where
-            # the library can use one all the same it is kept with the validated arguments
+            # the library can use one all the same it is kept with the validated arguments.  Not for a
+            # call that is recorded into a graph: nothing may be allocated then, and the graph may outlive
+            # the parameter object.
             workspace = Tensor()
             optional = int(_capi.lib().cumm_hip_query_gemm_optional_workspace(ctypes.byref(desp_to_c(desp)), m, n, k))
-            if optional > 0:
+            recorded = optional > 0 and _capi.lib().cumm_hip_stream_is_capturing(params.stream)
+            if optional > 0 and not recorded:
                 workspace = empty([optional], uint8, 0)
 
         args = _capi.GemmArgs()
@@ -291,7 +304,9 @@ class GemmMainUnitTest:
         if name:
             params.timer.record(name, params.stream)
         _capi.check(status)
-        if not name:
+        if optional > 0:
+            fn = _outside_graphs(fn, args)
+        if not name and not recorded:
             # validated argument block for unchanged repeat calls; the workspace it may point to
             # is kept alive with it
             params.__dict__["_prepared"] = (

@@ -242,6 +242,9 @@ int cumm_hip_memcpy_d2d(void *dst, const void *src, size_t bytes, void *stream);
 int cumm_hip_memset(void *ptr, int value, size_t bytes, void *stream);
 int cumm_hip_stream_create(void **stream);             /* host out-param; default priority */
 int cumm_hip_stream_destroy(void *stream);
+/* 1 while work on the stream is recorded into a HIP graph (or may not be started because another stream
+ * is), else 0 */
+int cumm_hip_stream_is_capturing(void *stream);
 /* GemmMainUnitTest.stream_synchronize / device_synchronize (cumm/gemm/main.py:1028-1047).
  * Both also report what a kernel could only find out while running: a serial split-K slice whose
  * bounded wait at the semaphore (tv::Semaphore, include/tensorview/gemm/arch/semaphore.h:37-100,

@@ -110,3 +110,42 @@ def test_backward_weight_of_strided_rows_and_of_more_offsets_than_one_call_takes
     f_out, f_in = H.as_f32(dout, "f16")[:, :k_out], H.as_f32(inp, "f16")[:, :c_in]
     ref = np.stack([f_out[po[r, :n]].T @ f_in[pi[r, :n]] for r, n in enumerate(counts)], axis=1)
     assert np.abs(got - ref).max() <= TOL["f16"] * max(np.abs(ref).max(), 1.0)
+
+
+@pytest.mark.parametrize("first", ["recorded", "eager"])
+def test_shuffle_ab_recorded_into_a_graph(first):
+    """Nothing is allocated while a stream is recorded, and a graph keeps its results when the parameter
+    object it was recorded from is gone."""
+    import torch
+    print("case shuffle_ab graph", first, flush=True)
+    rng = np.random.default_rng(3)
+    rows, m, n, pairs = 2000, 64, 72, 1000
+    a, b = _data(rng, (rows, m), "f16"), _data(rng, (rows, n), "f16")
+    ai, bi = (rng.integers(0, rows, size=pairs).astype(np.int32) for _ in range(2))
+    c = tv.zeros([m, n], tv.float16, 0)
+    p = GemmParams()
+    p.algo_desp = H.find_gemm_desp("f16", ShuffleStrideType.ShuffleAB, 64, 64, True, False)
+    p.a, p.b, p.c, p.a_inds, p.b_inds = H.dev(a, "f16"), H.dev(b, "f16"), c, H.dev(ai, "i32"), H.dev(bi, "i32")
+    keep = (p.a, p.b, p.a_inds, p.b_inds)
+    if first == "eager":
+        GemmMainUnitTest.matmul2(p)
+    warm = GemmParams()      # (loads the kernel that the graph will hold)
+    warm.algo_desp = p.algo_desp
+    warm.a, warm.b, warm.c = p.a, p.b, c
+    warm.a_inds, warm.b_inds = p.a_inds.slice_first_axis(0, 100), p.b_inds.slice_first_axis(0, 100)
+    GemmMainUnitTest.matmul2(warm)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        p.stream = torch.cuda.current_stream().cuda_stream
+        GemmMainUnitTest.matmul2(p)
+    # (a workspace that the graph used would be in p's prepared arguments: it has none)
+    ref = H.as_f32(a, "f16")[ai].T @ H.as_f32(b, "f16")[bi]
+    del p
+    for _ in range(3):
+        c.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.abs(H.as_f32(H.host(c), "f16") - ref).max() <= TOL["f16"] * np.abs(ref).max()
+    del keep
