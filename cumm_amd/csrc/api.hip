@@ -1149,9 +1149,19 @@ static uint32_t pairs_slots(int n) {
   return slots;
 }
 
-// 20 bytes per slot, the size callers have had so far: hash table slots of 8 bytes, one presence word per
-// slot, a flag
-size_t cumm_hip_subm_pairs_workspace(int n) { return (size_t)pairs_slots(n) * 20; }
+// The submanifold workspace: hash table slots of 8 bytes, pairs_slots() presence words, a flag.  The table
+// is a third full at most: insertion and look-up last as long as the longest run of taken slots, which
+// grows steeply from there to a half (120 k voxels in 2^18 and 2^19 slots: insertion 21.8 and 14.0 us, look-up
+// 21.0 and 16.8 us; 300 k voxels in 2^20 and 2^21, where memory bounds both: 32.9 and 29.1, 34.4 and 31.4, but
+// clearing 4.7 and 7.9 us).  A workspace of 20 bytes per pairs_slots() is enough for any n, the table then
+// half full.
+static uint32_t subm_slots(int n) {
+  const uint32_t slots = pairs_slots(n);
+  return slots < (1u << 31) && slots < 3ull * (uint32_t)(n > 0 ? n : 0) ? 2u * slots : slots;
+}
+size_t cumm_hip_subm_pairs_workspace(int n) {
+  return (size_t)pairs_slots(n) * 20 + (subm_slots(n) > pairs_slots(n) ? 16 : 0);
+}
 
 int cumm_hip_subm_pairs(const int32_t *coords, int n, const int32_t *spatial_shape, const int32_t *ksize,
                         const int32_t *dilation, int32_t *indices_fwd, int32_t *indices_bwd,
@@ -1173,8 +1183,9 @@ int cumm_hip_subm_pairs(const int32_t *coords, int n, const int32_t *spatial_sha
     return fail(CUMM_HIP_EINVAL, "submanifold convolution needs odd kernel sizes");
   for (int d = 0; d < 3; ++d)
     if (spatial_shape[d] < 1 || dilation[d] < 1) return fail(CUMM_HIP_EINVAL, "spatial_shape and dilation must be positive");
-  if (!workspace || workspace_bytes < cumm_hip_subm_pairs_workspace(n))
+  if (!workspace || workspace_bytes < (size_t)pairs_slots(n) * 20)
     return fail(CUMM_HIP_ERUNTIME, "workspace at least %zu bytes.", cumm_hip_subm_pairs_workspace(n));
+  const uint32_t slots = workspace_bytes < cumm_hip_subm_pairs_workspace(n) ? pairs_slots(n) : subm_slots(n);
   SubmPairsParams p;
   std::memset(&p, 0, sizeof(p));
   p.coords = coords; p.n = n; p.kv = (int)kv;
@@ -1186,8 +1197,8 @@ int cumm_hip_subm_pairs(const int32_t *coords, int n, const int32_t *spatial_sha
     p.off[k][2] = (kx - ksize[2] / 2) * dilation[2];
   }
   p.ind_f = indices_fwd; p.ind_b = indices_bwd; p.mask_f = mask_fwd; p.mask_b = mask_bwd;
-  p.table = workspace; p.slot_mask = pairs_slots(n) - 1u;
-  p.filter = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(workspace) + (size_t)pairs_slots(n) * 8);
+  p.table = workspace; p.slot_mask = slots - 1u;
+  p.filter = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(workspace) + (size_t)slots * 8);
   p.filter_mask = pairs_slots(n) - 1u;
   p.wide = p.filter + pairs_slots(n);
   p.kx = ksize[2];

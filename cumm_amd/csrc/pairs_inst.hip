@@ -107,7 +107,9 @@ __global__ __launch_bounds__(256) void pairs_insert_kernel(const SubmPairsParams
   if (((key | last) >> 32) != 0ull) atomicOr(p.wide, 1u);
   uint32_t h = mix32(low) & p.slot_mask;
   const unsigned long long mine = ((unsigned long long)(uint32_t)i << 32) | low;
-  // at most `slots` probes: the table has at least twice as many slots as voxels
+  // at most `slots` probes: the table has at least twice as many slots as voxels.  (Skipping taken slots
+  // by loads of eight at a time: 13.6 for 14.0 us at 120 k voxels, 34.1 for 37.2 at 300 k with run-to-run
+  // differences as large; not worth its code.)
   for (uint32_t probe = 0; probe <= p.slot_mask; ++probe) {
     const unsigned long long prev = atomicCAS(&table[h], kEmptySlot, mine);
     if (prev == kEmptySlot) break;
@@ -137,8 +139,8 @@ __device__ __forceinline__ int xcd_block(unsigned lines, int *zy) {
 // Consecutive lanes = consecutive voxels: every table row is written coalesced.  The masks are
 // OR-ed with atomics, one per lane with a pair, into words that the clear kernel set.  With the
 // presence words of neighbouring lines in one block, the workgroups in runs per XCD and the loads of
-// three offsets in flight: 44 -> 33 us at 300 k voxels; at 120 k the 23 us stay, the chain coordinates
-// - presence - slot, cold in every L2.
+// three offsets in flight: 44 -> 33 us at 300 k voxels; at 120 k the chain coordinates - presence - slots,
+// cold in every L2, bounds it (21.0 us, 16.8 with a table a third full at most instead of half).
 __global__ __launch_bounds__(256) void pairs_lookup_kernel(const SubmPairsParams p) {
   int zy;
   const int i = xcd_block((unsigned)(p.kv / p.kx), &zy) * 256 + threadIdx.x;

@@ -41,6 +41,30 @@ def test_subm_pairs_dense_block_and_kernel_shapes():
     _check_case(coords, (8, 9, 10), ksize=(3, 3, 3), dilation=(2, 2, 2))
 
 
+@pytest.mark.parametrize("n", [341, 342, 512, 513, 682, 683, 100000])
+def test_subm_pairs_in_either_workspace(n):
+    """The table in the workspace that the library asks for, and half as large in 20 bytes per slot of
+    twice as many slots as voxels: on either side of the sizes where the two differ, collisions in both."""
+    print("case subm pairs workspace", n, flush=True)
+    import ctypes as C
+    lib, arr3 = _capi.lib(), C.c_int32 * 3
+    shape = (16, 128, 128)
+    cells = np.random.default_rng(n).choice(int(np.prod(shape)), size=n, replace=False)
+    coords = np.stack((np.zeros(n, np.int64),) + np.unravel_index(cells, shape), axis=1).astype(np.int32)
+    ref = pairs.subm_pairs(coords, shape)
+    slots = max(1024, 1 << (2 * n - 1).bit_length())
+    asked = int(lib.cumm_hip_subm_pairs_workspace(n))
+    assert (asked > 20 * slots) == (slots < 3 * n)
+    d = H.dev(coords, "i32")
+    for nbytes in (20 * slots, asked):
+        ws = tv.zeros([nbytes], tv.uint8, 0)
+        fwd, bwd = tv.zeros([27, n], tv.int32, 0), tv.zeros([27, n], tv.int32, 0)
+        _capi.check(lib.cumm_hip_subm_pairs(d.byte_pointer(), n, arr3(*shape), arr3(3, 3, 3), arr3(1, 1, 1), fwd.byte_pointer(),
+                                            bwd.byte_pointer(), None, None, ws.byte_pointer(), nbytes, 0))
+        np.testing.assert_array_equal(H.host(fwd), ref.indices_fwd)
+        np.testing.assert_array_equal(H.host(bwd), ref.indices_bwd)
+
+
 def test_subm_pairs_and_sort_full_size():
     """The benchmark's voxel set (120 k voxels in 41 x 1600 x 1408): tables, masks, sorted masks and
     argsort, bit-exact; then a split filter."""
