@@ -101,7 +101,15 @@ def _desp_like(dtype, op, parallel=False, dynamic=False):
     return _DESP_LIKE[key].copy()
 
 
-_PTRS = ("ptr_A", "ptr_B", "ptr_C", "ptr_D", "bias_pointer", "workspace")
+# the fields of the argument block that hold each tensor's address.  By the pass and never by comparing
+# addresses: tensors of a call may share their storage (a gradient that is the layer's own input).  D is the
+# result itself where no bias is added.
+_FIELDS = {
+    ConvOpType.Forward: {"input": ("ptr_A",), "weight": ("ptr_B",), "output": ("ptr_C", "ptr_D")},
+    ConvOpType.BackwardInput: {"output": ("ptr_A",), "weight": ("ptr_B",), "input": ("ptr_C", "ptr_D")},
+    ConvOpType.BackwardWeight: {"output": ("ptr_A",), "input": ("ptr_B",), "weight": ("ptr_C", "ptr_D"), "workspace": ("workspace",)},
+}
+_WITH_BIAS = dict(_FIELDS[ConvOpType.Forward], output=("ptr_C",), bias=("ptr_D", "bias_pointer"))
 
 
 class _Launch:
@@ -123,12 +131,9 @@ class _Launch:
         if prep is None:
             raise RuntimeError("the operator call left no validated argument block")
         args = _copy(prep[5])
-        fields = {}
+        fields = _WITH_BIAS if "bias" in roles else _FIELDS[ConvOpType(params.conv_algo_desp.op_type)]
         for role, t in roles.items():
-            ptr = t.data_ptr()
-            # (an empty tensor has no address to find in the block: nothing to patch)
-            fields[role] = tuple(f for f in _PTRS if ptr and t.numel() and getattr(args, f) == ptr)
-            if t.numel() and not fields[role]:
+            if t.numel() and any(getattr(args, f) != t.data_ptr() for f in fields[role]):
                 raise RuntimeError("the argument block does not point at the %s tensor" % role)
         return cls(prep[1], prep[4], args, fields, int(params.conv_algo_desp.tile_shape[0]))
 

@@ -205,3 +205,43 @@ def test_deterministic_switch_gives_the_same_weight_gradient_twice():
     assert torch.equal(first, second)
     scale = float(default.float().abs().max())
     assert float((first.float() - default.float()).abs().max()) < 1e-2 * scale
+
+
+@pytest.mark.parametrize("strided,shared", [(False, False), (False, True), (True, False)])
+def test_a_call_validated_on_one_geometry_runs_on_another(monkeypatch, strided, shared):
+    """Two clouds of different sizes in one power of two: the second one's forward and backward are the first
+    one's validated calls with other addresses and row numbers - also when the first call's gradient was
+    the layer's own input (``shared``)."""
+    from cumm_amd import torch_bridge as tb
+    print("case moved call", strided, shared, flush=True)
+    channels = 40 + 8 * (2 * strided + shared)       # a kind of call that no other test has made
+    stride = (2, 2, 2) if strided else None
+    torch.manual_seed(11)
+    weight = (torch.randn(channels, 27, channels) * 0.05).half()
+
+    def rel(a, b):
+        return float((a.float().cpu() - b).abs().max() / b.abs().max().clamp_min(1e-6))
+
+    sizes = []
+    for trip, n in enumerate((2300, 3100)):
+        coords, grid = H.small_cloud(40 + trip, n)
+        geo = tb.SparseConvGeometry(torch.as_tensor(coords, device="cuda"), grid, stride=stride)
+        host = pairs.sparse_conv_pairs(coords, grid) if strided else pairs.subm_pairs(coords, grid)
+        sizes.append((geo.n_in, geo.n_out))
+        feat = torch.randn(geo.n_in, channels).half()
+        f_d, w_d = feat.cuda().requires_grad_(True), weight.cuda().requires_grad_(True)
+        gout = torch.randn(geo.n_out, channels).half()
+        g_d = gout.cuda()
+        if shared and trip == 0:
+            g_d, gout = f_d.detach(), feat
+        if trip == 1:      # no prelude from here on
+            monkeypatch.setattr(tb.ConvMainUnitTest, "implicit_gemm2", None)
+        out = tb.sparse_conv(f_d, w_d, None, geo)
+        out.backward(g_d)
+        f_r, w_r = feat.float().requires_grad_(True), weight.float().requires_grad_(True)
+        ref = _reference(f_r, w_r, None, host.indices_fwd, relu=False)
+        (ref * gout.float()).sum().backward()
+        assert rel(out.detach(), ref.detach()) < 1e-2, trip
+        assert rel(f_d.grad, f_r.grad) < 1e-2, trip
+        assert rel(w_d.grad, w_r.grad) < 1e-2, trip
+    assert sizes[0] != sizes[1] and all(tb._size_class(a) == tb._size_class(b) for a, b in zip(*sizes))

@@ -1,0 +1,92 @@
+"""Host logic of the torch bridge that needs no GPU: the argument blocks of validated calls, whose addresses
+are never dereferenced here."""
+import pytest
+
+from cumm_amd import _capi
+from cumm_amd import tensorview as tv
+from cumm_amd.conv.main import ConvMainUnitTest
+from cumm_amd.tensorview.gemm import ConvOpType, ConvParams
+
+torch = pytest.importorskip("torch")
+
+
+class _Recorder:
+    """The library with some entry points replaced by what keeps their arguments."""
+
+    def __init__(self, *names):
+        self._real, self._names, self.calls = _capi.lib(), names, []
+
+    def __getattr__(self, name):
+        if name not in self._names:
+            return getattr(self._real, name)
+
+        def entry(*args):
+            self.calls.append((name,) + tuple(type(a._obj).from_buffer_copy(a._obj) if hasattr(a, "_obj") else a for a in args))
+            return 0
+        return entry
+
+
+@pytest.fixture
+def recorded(monkeypatch):
+    def use(*names):
+        r = _Recorder(*names)
+        monkeypatch.setattr(_capi, "_lib", r)
+        return r
+    return use
+
+
+class _At:
+    """What a call sees of a tensor: its address."""
+
+    def __init__(self, address):
+        self.address = address
+
+    def data_ptr(self):
+        return self.address
+
+    def numel(self):
+        return 1
+
+
+N, C, KV = 1000, 64, 27
+
+
+def _params(op, addresses, bias=None):
+    at = lambda role, shape: tv.from_blob(addresses[role], shape, tv.float16, 0)
+    blob = lambda shape, dtype: tv.from_blob(0x7E0000000000, shape, dtype, 0)
+    p = ConvParams(3, op)
+    p.conv_algo_desp = [d for d in ConvMainUnitTest.get_all_conv_algo_desp()
+                        if d.dtype_a == tv.float16 and d.dtype_c == tv.float16 and ConvOpType(d.op_type) == op][0].copy()
+    p.input, p.weight, p.output = at("input", [N, C]), at("weight", [C, KV, C]), at("output", [N, C])
+    p.indices, p.mask_argsort = blob([KV, N], tv.int32), blob([N], tv.int32)
+    p.mask = blob([N], tv.uint32)
+    if op == ConvOpType.BackwardWeight:
+        p.mask_width = 64
+    if bias is not None:
+        p.bias, p.beta = tv.from_blob(bias, [C], tv.float16, 0), 1.0
+    return p
+
+
+@pytest.mark.parametrize("op,with_bias", [(ConvOpType.Forward, False), (ConvOpType.Forward, True), (ConvOpType.BackwardInput, False),
+                                          (ConvOpType.BackwardWeight, False)])
+@pytest.mark.parametrize("shared", [(), ("input", "output"), ("input", "weight"), ("weight", "output"), ("input", "weight", "output")])
+def test_a_call_keeps_its_tensors_apart_whatever_the_first_one_shared(recorded, op, with_bias, shared):
+    """A block that was validated with tensors at one address, replayed with tensors at three."""
+    from cumm_amd import torch_bridge as tb
+    lib = recorded("cumm_hip_sparse_conv")
+    first = {"input": 0x7F0000000000, "weight": 0x7F1000000000, "output": 0x7F2000000000}
+    first.update({role: 0x7F3000000000 for role in shared})
+    p = _params(op, first, bias=0x7F4000000000 if with_bias else None)
+    ConvMainUnitTest.implicit_gemm2(p)
+    roles = {role: _At(a) for role, a in first.items()}
+    if with_bias:
+        roles["bias"] = _At(0x7F4000000000)
+    launch = tb._Launch.of(p, roles)
+    new = {role: 0x600000000000 + (i << 32) for i, role in enumerate(roles)}
+    launch(0, **{role: _At(a) for role, a in new.items()})
+    args = lib.calls[-1][2]
+    a, b, c = {ConvOpType.Forward: ("input", "weight", "output"), ConvOpType.BackwardInput: ("output", "weight", "input"),
+               ConvOpType.BackwardWeight: ("output", "input", "weight")}[op]
+    assert (args.ptr_A, args.ptr_B, args.ptr_C) == (new[a], new[b], new[c])
+    assert args.ptr_D == new["bias" if with_bias else c]
+    assert args.bias_pointer == (new["bias"] if with_bias else None)
