@@ -184,6 +184,7 @@ class SparseConvGeometry:
     All tables lie in one block from torch's caching allocator (a new cloud per iteration then
     allocates nothing from the driver); ``indices_fwd`` and the other tables are views of it."""
 
+    _TILES = (64, 128)      # positions per tile of the kernels that reduce masks
     _TABLES = ("indices_fwd", "indices_bwd", "mask_fwd", "order_fwd", "mask_bwd", "order_bwd", "indices_fwd_pos", "indices_bwd_pos")
 
     def __init__(self, coords: torch.Tensor, spatial_shape: Sequence[int], ksize=(3, 3, 3), stride=None,
@@ -202,7 +203,7 @@ class SparseConvGeometry:
         # launches - stays on the device: the sort leaves it in the library's table under the sorted
         # array's address and the launches look it up there; 0 = not given here)
         self.light_fwd = self.light_bwd = 0
-        self._reduced = {}
+        self._reduced, self._reduced_streams = {}, {}
         self._launches = {}      # calls of the layers on this geometry, see _Launch
         self._tensors = {}
         lib, arr3 = _capi.lib(), ctypes.c_int32 * 3
@@ -258,6 +259,8 @@ class SparseConvGeometry:
         mask = [n_in] if words == 1 else [n_in, words]
         if not self.subm:
             spec += [("mask_bwd", mask, tv.uint32), ("order_bwd", [n_in], tv.int32)]
+        if words == 1:     # (in the block and not where the first forward pass runs: see reduced_mask)
+            spec += [("reduced_%d" % w, [max((n_out + w - 1) // w, 1)], tv.int32) for w in SparseConvGeometry._TILES]
         self._spec, at = {}, 0
         for name, dims, dtype in spec:
             self._spec[name] = (at, dims, dtype)
@@ -298,22 +301,36 @@ class SparseConvGeometry:
         if stream != self._stream:
             current = torch.cuda.current_stream()
             self._block.record_stream(current)
-            for buf in self._reduced.values():
-                buf.record_stream(current)
             if self.lists is not None:
                 self._list_block.record_stream(current)
+        for width, own in self._reduced_streams.items():
+            if stream != own:
+                self._reduced[width].record_stream(torch.cuda.current_stream())
 
     def reduced_mask(self, width: int) -> torch.Tensor:
         """One word per run of ``width`` sorted output positions: the forward launch writes (all of) the
-        OR of the run's masks here (its ``mask_output``), and backward-weight reads it."""
+        OR of the run's masks here (its ``mask_output``), and backward-weight reads it.  The words of the
+        kernels' tile heights lie in the block of the tables: memory that the first forward pass took from
+        its own stream's pool could be in use there still when another stream writes it, and again while
+        another stream reads it."""
         buf = self._reduced.get(width)
         if buf is None:
-            tiles = (self.n_out + width - 1) // width
-            buf = self._reduced[width] = torch.empty(max(tiles, 1), dtype=torch.int32, device=self._device)
+            tiles, place = max((self.n_out + width - 1) // width, 1), self._spec.get("reduced_%d" % width)
+            if place is not None:
+                buf = self._block[place[0]:place[0] + 4 * tiles].view(torch.int32)
+            else:
+                buf = torch.empty(tiles, dtype=torch.int32, device=self._device)
+                self._reduced_streams[width] = current_stream()
+            self._reduced[width] = buf
         return buf
 
     def reduced_mask_buffer(self, width: int) -> tv.Tensor:
-        return torch2tensor(self.reduced_mask(width)).type_view(tv.uint32)
+        """``reduced_mask`` as a tv tensor; zeros until a forward pass with tiles of that height has run."""
+        fresh = width not in self._reduced
+        buf = self.reduced_mask(width)
+        if fresh:
+            buf.zero_()
+        return torch2tensor(buf).type_view(tv.uint32)
 
 
 def _same_device(*tensors) -> None:

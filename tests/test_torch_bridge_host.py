@@ -90,3 +90,53 @@ def test_a_call_keeps_its_tensors_apart_whatever_the_first_one_shared(recorded, 
     assert (args.ptr_A, args.ptr_B, args.ptr_C) == (new[a], new[b], new[c])
     assert args.ptr_D == new["bias" if with_bias else c]
     assert args.bias_pointer == (new["bias"] if with_bias else None)
+
+
+def _geometry(monkeypatch, tb, n=1000, stream=1):
+    """A submanifold geometry of ``n`` voxels as its constructor leaves it on ``stream``, in host memory; the
+    second result lists what is recorded for another stream, by the address of its memory."""
+    now, recorded = [stream], []
+    monkeypatch.setattr(tb, "current_stream", lambda: now[0])
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: now[0])
+    monkeypatch.setattr(torch.Tensor, "record_stream", lambda t, s: recorded.append((t.untyped_storage().data_ptr(), s)))
+    g = object.__new__(tb.SparseConvGeometry)
+    g._stream, g._device, g.subm, g.kv, g.words, g.n_in, g.n_out = stream, torch.device("cpu"), True, 27, 1, n, n
+    g.lists, g._reduced, g._reduced_streams, g._launches, g._tensors = None, {}, {}, {}, {}
+    g._allocate()
+    return g, recorded, now
+
+
+def test_reduced_masks_belong_to_the_streams_that_use_them(monkeypatch):
+    """Built on one stream, first used on a second, used again on the first: the words of the kernels' tile
+    heights lie in the block of the tables, others are recorded for every stream but their own."""
+    from cumm_amd import torch_bridge as tb
+    for n in (0, 1, 64, 65, 1000):
+        g, recorded, now = _geometry(monkeypatch, tb, n)
+        now[0] = 2
+        g.used_on(2)
+        words = {w: g.reduced_mask(w) for w in (64, 128, 32)}
+        block = g._block.untyped_storage().data_ptr()
+        assert recorded == [(block, 2)]
+        for w, t in words.items():
+            assert t.numel() == max((n + w - 1) // w, 1) and t.dtype == torch.int32
+            assert (t.untyped_storage().data_ptr() == block) == (w != 32)
+        spans = sorted((t.data_ptr(), t.data_ptr() + 4 * t.numel()) for w, t in words.items() if w != 32)
+        spans += [(g._ptr["order_fwd"], g._ptr["order_fwd"] + 4 * n)]
+        spans.sort()
+        assert all(a[1] <= b[0] for a, b in zip(spans, spans[1:])) and spans[-1][1] <= block + g._block.numel()
+        now[0] = 1
+        g.used_on(1)
+        assert recorded[1:] == [(words[32].untyped_storage().data_ptr(), 1)]
+        assert g.reduced_mask(64) is words[64]
+
+
+def test_a_reduced_mask_that_no_pass_has_written_is_zero(monkeypatch):
+    from cumm_amd import torch_bridge as tb
+    g, _, _ = _geometry(monkeypatch, tb)
+    g._block.fill_(0xA5)
+    for w in (64, 32):
+        g.reduced_mask_buffer(w)
+        assert not g.reduced_mask(w).any()
+    g.reduced_mask(64).fill_(7)
+    g.reduced_mask_buffer(64)
+    assert bool((g.reduced_mask(64) == 7).all())
