@@ -333,11 +333,6 @@ class SparseConvGeometry:
         return torch2tensor(buf).type_view(tv.uint32)
 
 
-def _same_device(*tensors) -> None:
-    if any(t.device != tensors[0].device for t in tensors):
-        raise ValueError("all tensors must be on the same device")
-
-
 class _SparseConvFunction(torch.autograd.Function):
 
     @staticmethod
@@ -432,9 +427,11 @@ class _SparseConvFunction(torch.autograd.Function):
 
 def _kind(g: SparseConvGeometry, key, n_pos: int, *tensors):
     """The key of a call in _KINDS; the tensors of a first call are checked here for what the operator's
-    prelude checks and a moved call does not (types and shapes are in the key)."""
-    _same_device(*tensors)
-    return key + (g.kv, g.subm, _size_class(n_pos), tensors[0].device.index)
+    prelude checks and a moved call does not: one device, that of the tables (types and shapes are in the
+    key)."""
+    if any(t.device != g._device for t in tensors):
+        raise ValueError("all tensors must be on the same device")
+    return key + (g.kv, g.subm, _size_class(n_pos), g._device.index)
 
 
 def _forward_launch(g: SparseConvGeometry, key, roles, relu, stream) -> _Launch:

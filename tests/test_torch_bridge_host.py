@@ -140,3 +140,14 @@ def test_a_reduced_mask_that_no_pass_has_written_is_zero(monkeypatch):
     g.reduced_mask(64).fill_(7)
     g.reduced_mask_buffer(64)
     assert bool((g.reduced_mask(64) == 7).all())
+
+
+def test_a_moved_call_refuses_tensors_on_another_device_than_the_tables(monkeypatch):
+    """The tensors agree among themselves, the geometry lies elsewhere; and one tensor alone elsewhere."""
+    from cumm_amd import torch_bridge as tb
+    g, _, _ = _geometry(monkeypatch, tb)
+    here, there = torch.empty(1), torch.empty(1, device="meta")
+    assert tb._kind(g, ("fwd",), 1000, here, here)[0] == "fwd"
+    for tensors in ((there, there, there), (here, there, here), (there, here, here)):
+        with pytest.raises(ValueError, match="same device"):
+            tb._kind(g, ("fwd",), 1000, *tensors)
