@@ -174,6 +174,22 @@ def _bytes(n: int, device) -> torch.Tensor:
     return torch.empty(max(int(n), 256), dtype=torch.uint8, device=device)
 
 
+class _HandedOut:
+    """What a tv tensor over the block of a geometry keeps alive: its memory goes back to torch's allocator as
+    tv's own storage goes back to the driver, when the device has finished with it.  (The operators run
+    such a tensor on streams that torch's allocator does not hear of.)"""
+
+    def __init__(self, block: torch.Tensor):
+        self.block = block
+
+    def __del__(self):
+        try:
+            if not torch.cuda.is_current_stream_capturing():
+                torch.cuda.synchronize(self.block.device)
+        except Exception:
+            pass
+
+
 class SparseConvGeometry:
     """Pair tables, masks and sorts of one convolution geometry, built on the GPU once and shared by
     every layer (and every pass) that uses it.  Kernel volumes up to 32 have one mask word per
@@ -284,7 +300,9 @@ class SparseConvGeometry:
         ws = _bytes(need, self._device)
         _capi.check(lib.cumm_hip_pair_lists(self._ptr["indices_fwd"], kv, n, lists[0].data_ptr(), lists[1].data_ptr(),
                                             counts.data_ptr(), ws.data_ptr(), ws.numel(), self._stream))
-        self.lists = pairs.DevicePairLists(torch2tensor(lists[0]), torch2tensor(lists[1]), counts.cpu().numpy())
+        handed = _HandedOut(lists)
+        pair_in, pair_out = (tv.from_blob(t.data_ptr(), [kv, n], tv.int32, self._device.index, keepalive=handed) for t in lists)
+        self.lists = pairs.DevicePairLists(pair_in, pair_out, counts.cpu().numpy())
         self._list_block = lists
 
     def __getattr__(self, name: str):
@@ -293,7 +311,8 @@ class SparseConvGeometry:
         t = self._tensors.get(name)
         if t is None:
             _, dims, dtype = self._spec[name]
-            t = self._tensors[name] = tv.from_blob(self._ptr[name], dims, dtype, self._device.index, keepalive=self._block)
+            t = self._tensors[name] = tv.from_blob(self._ptr[name], dims, dtype, self._device.index,
+                                                    keepalive=_HandedOut(self._block))
         return t
 
     def used_on(self, stream: int) -> None:

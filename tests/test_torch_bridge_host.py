@@ -151,3 +151,32 @@ def test_a_moved_call_refuses_tensors_on_another_device_than_the_tables(monkeypa
     for tensors in ((there, there, there), (here, there, here), (there, here, here)):
         with pytest.raises(ValueError, match="same device"):
             tb._kind(g, ("fwd",), 1000, *tensors)
+
+
+def test_tables_that_were_handed_out_go_back_when_the_device_has_finished(monkeypatch):
+    """A tv tensor of a table that outlives its geometry: the block is alive until the wait is over, and no
+    wait is made for a geometry whose tables nobody took, nor while the stream is recorded."""
+    from cumm_amd import torch_bridge as tb
+    import gc
+    import weakref
+    waits, capturing = [], [False]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    for taken in (True, False):
+        g, _, _ = _geometry(monkeypatch, tb)
+        block = weakref.ref(g._block)
+        monkeypatch.setattr(torch.cuda, "synchronize", lambda d: waits.append(block() is not None))
+        table = g.indices_fwd_pos if taken else None
+        if taken:
+            assert table.byte_pointer() == g._ptr["indices_fwd_pos"] and g.indices_fwd_pos is table
+        del g
+        gc.collect()
+        assert waits == [] and (block() is not None) == taken
+        del table
+        gc.collect()
+        assert waits == ([True] if taken else []) and block() is None
+        del waits[:]
+    g, _, _ = _geometry(monkeypatch, tb)
+    capturing[0] = g.order_fwd is not None
+    del g
+    gc.collect()
+    assert waits == []
