@@ -253,18 +253,42 @@ class SparseConvGeometry:
         # masks, an order of the positions by them, and the pair tables once more in that order: what
         # forward and backward-input read (a tile's entries for one offset are then consecutive in
         # memory); backward-weight keeps the table by row
-        p = self._ptr
+        if 4 * kv * max(n_in, n_out) < 1 << 31:
+            self._order(ks)
+        else:
+            self._order_one_by_one()
+        if words > 1:
+            self._make_lists()
+
+    def _order(self, ks) -> None:
+        lib, p = _capi.lib(), self._ptr
         sides = (_capi.OrderSide * 2)()
-        for d, side, n in ((sides[0], "fwd", n_out), (sides[1], "bwd", n_in)):
+        for d, side, n in ((sides[0], "fwd", self.n_out), (sides[1], "bwd", self.n_in)):
             d.indices, d.n = p["indices_" + side], n
             d.sorted_mask, d.argsort, d.by_position = p["mask_" + side], p["order_" + side], p["indices_%s_pos" % side]
         count = 2
         if self.subm:      # (one order serves both; the backward table is the forward one with its offsets reversed)
             sides[0].by_position_reversed, count = p["indices_bwd_pos"], 1
-        ws = _bytes(lib.cumm_hip_order_pairs_workspace(sides, count, kv), dev)
-        _capi.check(lib.cumm_hip_order_pairs(sides, count, ks, ws.data_ptr(), ws.numel(), s))
-        if words > 1:
-            self._make_lists()
+        ws = _bytes(lib.cumm_hip_order_pairs_workspace(sides, count, self.kv), self._device)
+        _capi.check(lib.cumm_hip_order_pairs(sides, count, ks, ws.data_ptr(), ws.numel(), self._stream))
+
+    def _order_one_by_one(self) -> None:
+        """``_order`` for tables of 2^31 bytes and more, which cumm_hip_order_pairs and the launches refuse:
+        whoever builds one wants the tables (the per-offset convolution walks lists of them)."""
+        lib, p, s, kv, words = _capi.lib(), self._ptr, self._stream, self.kv, self.words
+        for side, n in (("fwd", self.n_out), ("bwd", self.n_in)):
+            if side == "fwd" or not self.subm:
+                raw = torch.empty((n, words), dtype=torch.int32, device=self._device)
+                _capi.check(lib.cumm_hip_masks_from_pairs(p["indices_" + side], kv, n, raw.data_ptr(), s))
+                need = lib.cumm_hip_sort_by_mask_workspace(n) if words == 1 else lib.cumm_hip_sort_by_mask_words_workspace(n)
+                ws = _bytes(need, self._device)
+                to = (p["mask_" + side], p["order_" + side], ws.data_ptr(), ws.numel(), s)
+                if words == 1:
+                    bits = (1 << kv) - 1 if kv < 32 else 0xFFFFFFFF
+                    _capi.check(lib.cumm_hip_sort_by_mask_ordered(raw.data_ptr(), n, bits, int(kv <= 27), *to))
+                else:
+                    _capi.check(lib.cumm_hip_sort_by_mask_words(raw.data_ptr(), n, words, *to))
+            _capi.check(lib.cumm_hip_pairs_by_position(p["indices_" + side], p["order_" + side], kv, n, p["indices_%s_pos" % side], s))
 
     def _allocate(self) -> None:
         n_out, n_in, kv, words = self.n_out, self.n_in, self.kv, self.words

@@ -245,3 +245,39 @@ def test_a_call_validated_on_one_geometry_runs_on_another(monkeypatch, strided, 
         assert rel(f_d.grad, f_r.grad) < 1e-2, trip
         assert rel(w_d.grad, w_r.grad) < 1e-2, trip
     assert sizes[0] != sizes[1] and all(tb._size_class(a) == tb._size_class(b) for a, b in zip(*sizes))
+
+
+@pytest.mark.parametrize("strided", [False, True])
+def test_a_geometry_whose_tables_exceed_31_bits_of_bytes(strided):
+    """More voxels than the launches take (a table of 2^31 bytes): the geometry has its tables, masks and order,
+    a forward pass is refused.  A full box of voxels, so that every entry is known."""
+    from cumm_amd import torch_bridge as tb
+    print("case large tables", strided, flush=True)
+    kv, shape = (27, (20, 1000, 1000)) if not strided else (25, (22, 1000, 1000))
+    n = shape[0] * shape[1] * shape[2]
+    assert 4 * kv * n >= 1 << 31
+    row = torch.arange(n, dtype=torch.int32, device="cuda")
+    zyx = [row // (shape[1] * shape[2]), row // shape[2] % shape[1], row % shape[2]]
+    coords = torch.stack([torch.zeros_like(row)] + zyx, 1)
+    ksize = (3, 3, 3) if not strided else (1, 5, 5)
+    geo = tb.SparseConvGeometry(coords, shape, ksize, (1, 1, 1) if strided else None, tuple(k // 2 for k in ksize))
+    del coords
+    assert (geo.n_in, geo.n_out) == (n, n)
+    t = lambda name: tb.tensor2torch(getattr(geo, name), clone=False, cast_uint_to_int=True)
+    fwd, mask, order, pos, bwd, bwd_pos, bwd_order = (t(x) for x in ("indices_fwd", "mask_fwd", "order_fwd", "indices_fwd_pos",
+                                                                     "indices_bwd", "indices_bwd_pos", "order_bwd"))
+    bits = torch.zeros_like(row)
+    for k in range(kv):
+        at = (k // (ksize[1] * ksize[2]), k // ksize[2] % ksize[1], k % ksize[2])
+        d = [a - s // 2 for a, s in zip(at, ksize)]
+        inside = torch.ones(n, dtype=torch.bool, device="cuda")
+        for c, e, s in zip(zyx, d, shape):
+            inside &= (c + e >= 0) & (c + e < s)
+        want = torch.where(inside, row + (d[0] * shape[1] + d[1]) * shape[2] + d[2], torch.full_like(row, -1))
+        assert torch.equal(fwd[k], want) and torch.equal(bwd[kv - 1 - k], want), k
+        assert torch.equal(pos[k], want[order.long()]) and torch.equal(bwd_pos[k], bwd[k][bwd_order.long()]), k
+        bits |= torch.where(inside, 1 << k, 0).to(torch.int32)
+    assert torch.equal(mask, bits[order.long()]) and torch.equal(torch.sort(order).values, row)
+    with pytest.raises(RuntimeError):
+        tb.sparse_conv(torch.zeros(n, 8, dtype=torch.float16, device="cuda"), torch.zeros(8, kv, 8, dtype=torch.float16, device="cuda"),
+                       None, geo)
