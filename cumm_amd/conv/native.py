@@ -20,7 +20,7 @@ import numpy as np
 
 from .. import _capi
 from .. import tensorview as tv
-from ..gemm.main import GemmMainUnitTest
+from ..gemm.main import GemmMainUnitTest, _check_device, _check_dtype
 from ..tensorview.gemm import Activation, GemmParams, ShuffleStrideType
 
 
@@ -174,7 +174,8 @@ class WeightPlan:
         lib = _capi.lib()
         kv, k_out, c_in = dweight.dim(1), dweight.dim(0), dweight.dim(2)
         self._fn = lib.cumm_hip_wgrad_pairs
-        self._counts = np.ascontiguousarray(lists.counts, np.int32)
+        # (a count beyond its list ends with the list, as a slice of it does)
+        self._counts = np.ascontiguousarray(np.clip(lists.counts, 0, lists.pair_in.dim(1)), np.int32)
         counts = self._counts.ctypes.data
         self._pairs = (lists.pair_out.byte_pointer(), lists.pair_in.byte_pointer(), counts, kv, lists.pair_in.dim(1))
         self._sizes = (dout.dim(0), inp.dim(0), k_out, c_in, dweight.dtype)
@@ -215,8 +216,11 @@ def plan_backward_weight(dout: tv.Tensor, inp: tv.Tensor, dweight: tv.Tensor, li
     """Backward-weight as a reusable plan: dweight[:, k, :] of every kernel offset (zeros for an
     offset without pairs)."""
     _check(inp, dweight, lists, dout.dim(0))
-    if dout.dim(1) != dweight.dim(0) or dout.dtype != inp.dtype or dweight.dim(2) != inp.dim(1):
+    if dout.ndim != 2 or dout.dim(1) != dweight.dim(0) or dout.dtype != inp.dtype or dweight.dim(2) != inp.dim(1):
         raise RuntimeError("error")
+    _check_device(dout, inp, dweight, lists.pair_in, lists.pair_out)
+    _check_dtype(lists.pair_in, tv.int32, "pair_in")
+    _check_dtype(lists.pair_out, tv.int32, "pair_out")
     if not _in_one_call(dout, inp, dweight, lists):
         return WeightSteps(dout, inp, dweight, lists, stream)
     return WeightPlan(dout, inp, dweight, lists, stream)

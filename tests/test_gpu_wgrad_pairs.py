@@ -12,6 +12,7 @@ from cumm_amd.gemm.main import GemmMainUnitTest, desp_to_c
 from cumm_amd.tensorview.gemm import GemmParams, ShuffleStrideType
 import helpers as H
 
+torch = pytest.importorskip("torch")      # (before the library: one HIP runtime in the process)
 pytestmark = pytest.mark.gpu
 
 # the result is rounded once from fp32 sums: half a unit in the last place of the largest element, and
@@ -116,7 +117,6 @@ def test_backward_weight_of_strided_rows_and_of_more_offsets_than_one_call_takes
 def test_shuffle_ab_recorded_into_a_graph(first):
     """Nothing is allocated while a stream is recorded, and a graph keeps its results when the parameter
     object it was recorded from is gone."""
-    import torch
     print("case shuffle_ab graph", first, flush=True)
     rng = np.random.default_rng(3)
     rows, m, n, pairs = 2000, 64, 72, 1000
