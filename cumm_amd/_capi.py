@@ -69,6 +69,7 @@ class OrderSide(C.Structure):
 _VP, _PVP = C.c_void_p, C.POINTER(C.c_void_p)
 SYMBOLS = {
     "cumm_hip_gemm": (C.c_int, [C.POINTER(GemmDesc), C.POINTER(GemmArgs), _VP]),
+    "cumm_hip_gemm_in_workspace": (C.c_int, [C.POINTER(GemmDesc), C.POINTER(GemmArgs), _VP]),
     "cumm_hip_sparse_conv": (C.c_int, [C.POINTER(ConvDesc), C.POINTER(SparseConvArgs), _VP]),
     "cumm_hip_sparse_conv_static_ws": (C.c_int, [C.POINTER(ConvDesc), C.POINTER(SparseConvArgs), _VP]),
     "cumm_hip_query_gemm_workspace": (C.c_int64, [C.POINTER(GemmDesc), C.c_int, C.c_int, C.c_int, C.c_int]),

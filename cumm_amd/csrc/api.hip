@@ -581,7 +581,7 @@ int cumm_hip_list_conv_algos(CummHipConvDesc *out, int cap) {
 }
 
 // ---------------------------------------------------------------------------------------------
-int cumm_hip_gemm(const CummHipGemmDesc *desc, const CummHipGemmArgs *a, void *stream_) {
+static int gemm_impl(const CummHipGemmDesc *desc, const CummHipGemmArgs *a, void *stream_, bool in_workspace) {
   if (!desc || !a) return fail(CUMM_HIP_EINVAL, "null descriptor or arguments");
   const CummHipGemmDesc &d = *desc;
   const int fam = gemm_family(d);
@@ -680,7 +680,7 @@ int cumm_hip_gemm(const CummHipGemmDesc *desc, const CummHipGemmArgs *a, void *s
     p.y_gather = a->indiceA; p.x_gather = a->indiceBorC;
     p.rows_y = a->rows_A; p.rows_x = a->rows_B;
     uint32_t a_bytes = 0, b_bytes = 0;
-    if (a->split_k_slices == 1 && a->workspace && a->rows_A > 0 && a->rows_B > 0 && wgrad_pairs_serves(d, m, n, a->k) &&
+    if (in_workspace && a->split_k_slices == 1 && a->workspace && a->rows_A > 0 && a->rows_B > 0 && wgrad_pairs_serves(d, m, n, a->k) &&
         extent32(a->rows_A, lda, m, 2, &a_bytes) && extent32(a->rows_B, ldb, n, 2, &b_bytes) && (int64_t)a->k * 4 < (int64_t)1 << 31) {
       WgradPairsParams w;
       std::memset(&w, 0, sizeof(w));
@@ -718,6 +718,12 @@ int cumm_hip_gemm(const CummHipGemmDesc *desc, const CummHipGemmArgs *a, void *s
   hipError_t e = launch_tilegemm(dt, wide, tm, tn, xk, yk, p, grid, stream);
   if (e != hipSuccess) return hip_fail(e, "GEMM launch");
   return CUMM_HIP_OK;
+}
+
+int cumm_hip_gemm(const CummHipGemmDesc *desc, const CummHipGemmArgs *a, void *stream) { return gemm_impl(desc, a, stream, false); }
+
+int cumm_hip_gemm_in_workspace(const CummHipGemmDesc *desc, const CummHipGemmArgs *a, void *stream) {
+  return gemm_impl(desc, a, stream, true);
 }
 
 // ---------------------------------------------------------------------------------------------

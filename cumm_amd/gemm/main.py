@@ -83,13 +83,12 @@ def _check_device(*tens):
         raise RuntimeError("operands must be device tensors (call .cuda() first)")
 
 
-def _outside_graphs(fn, args):
-    """The entry point, without the workspace that belongs to the argument block while its stream is
-    recorded into a graph."""
-    bare = _capi.GemmArgs.from_buffer_copy(args)
-    bare.workspace, bare.workspace_bytes = None, 0
-    bare_ref, capturing = ctypes.byref(bare), _capi.lib().cumm_hip_stream_is_capturing
-    return lambda cdesc_ref, args_ref, stream: fn(cdesc_ref, bare_ref if capturing(stream) else args_ref, stream)
+def _in_workspace(cdesc_ref, args_ref, stream):
+    """The entry point that uses the workspace of the argument block; while the stream is recorded into a
+    graph, which may outlive the block, the one that does not."""
+    lib = _capi.lib()
+    fn = lib.cumm_hip_gemm if lib.cumm_hip_stream_is_capturing(stream) else lib.cumm_hip_gemm_in_workspace
+    return fn(cdesc_ref, args_ref, stream)
 
 
 class GemmMainUnitTest:
@@ -299,13 +298,11 @@ class GemmMainUnitTest:
         name = repr(desp) if params.timer.enable else ""
         if name:
             params.timer.record(name, params.stream)
-        fn = _capi.lib().cumm_hip_gemm
+        fn = _in_workspace if optional > 0 else _capi.lib().cumm_hip_gemm
         status = fn(ctypes.byref(cdesc), ctypes.byref(args), params.stream)
         if name:
             params.timer.record(name, params.stream)
         _capi.check(status)
-        if optional > 0:
-            fn = _outside_graphs(fn, args)
         if not name and not recorded:
             # validated argument block for unchanged repeat calls; the workspace it may point to
             # is kept alive with it

@@ -163,6 +163,10 @@ typedef struct CummHipSparseConvArgs {
 /* Replaces GemmMainUnitTest.matmul2 below its prelude
  * (cumm/gemm/main.py:1176-1335: dispatch on the descriptor and launch). */
 int cumm_hip_gemm(const CummHipGemmDesc *desc, const CummHipGemmArgs *args, void *stream);
+/* The same call, which may also use args->workspace (16-byte aligned) with split_k_slices == 1, where
+ * cumm_hip_gemm leaves it alone: see cumm_hip_query_gemm_optional_workspace.  Calls that may overlap
+ * in time, on several streams or from several threads, each need a workspace of their own then. */
+int cumm_hip_gemm_in_workspace(const CummHipGemmDesc *desc, const CummHipGemmArgs *args, void *stream);
 
 /* Replaces ConvMainUnitTest.implicit_gemm2 below its prelude for mask_sparse
  * descriptors (cumm/conv/main.py:483-745). */
@@ -191,8 +195,8 @@ int64_t cumm_hip_query_gemm_workspace(const CummHipGemmDesc *desc, int m, int n,
 int64_t cumm_hip_query_conv_workspace(const CummHipConvDesc *desc, int m, int n, int k, int split_k_slices,
                                       int kernel_volume);
 
-/* Bytes of workspace with which a launch with split_k_slices == 1, which needs none, is faster: a
- * product with few outputs and a long contraction (ShuffleAB of two-byte elements) is then cut
+/* Bytes of workspace with which cumm_hip_gemm_in_workspace runs a product with split_k_slices == 1
+ * faster: one with few outputs and a long contraction (ShuffleAB of two-byte elements) is then cut
  * along the contraction, its partial sums kept in fp32 and rounded once.  0 = none is of use, -1
  * for bad arguments.  (No counterpart in the reference, which splits only into slices that the
  * caller asks for.) */

@@ -149,3 +149,62 @@ def test_shuffle_ab_recorded_into_a_graph(first):
         torch.cuda.synchronize()
         assert np.abs(H.as_f32(H.host(c), "f16") - ref).max() <= TOL["f16"] * np.abs(ref).max()
     del keep
+
+
+def _shuffle_ab(rng, rows, m, n, pairs):
+    a, b = _data(rng, (rows, m), "f16"), _data(rng, (rows, n), "f16")
+    ai, bi = (rng.integers(0, rows, size=pairs).astype(np.int32) for _ in range(2))
+    p = GemmParams()
+    p.algo_desp = H.find_gemm_desp("f16", ShuffleStrideType.ShuffleAB, 64, 64, True, False)
+    p.a, p.b, p.a_inds, p.b_inds = H.dev(a, "f16"), H.dev(b, "f16"), H.dev(ai, "i32"), H.dev(bi, "i32")
+    p.c = tv.zeros([m, n], tv.float16, 0)
+    return p, H.as_f32(a, "f16")[ai].T @ H.as_f32(b, "f16")[bi]
+
+
+@pytest.mark.parametrize("entry,used", [("cumm_hip_gemm", False), ("cumm_hip_gemm_in_workspace", True)])
+def test_one_slice_uses_a_workspace_only_where_the_caller_says_so(entry, used):
+    """A workspace passed along with split_k_slices == 1, as a caller of several streams may share it."""
+    print("case shuffle_ab workspace", entry, flush=True)
+    m, n, pairs = 64, 136, 5000
+    p, ref = _shuffle_ab(np.random.default_rng(4), 3000, m, n, pairs)
+    lib, cd = _capi.lib(), desp_to_c(p.algo_desp)
+    ws = H.dev(np.full(int(lib.cumm_hip_query_gemm_optional_workspace(ctypes.byref(cd), m, n, pairs)), 0xA5, np.uint8), "u8")
+    args = _capi.GemmArgs()
+    args.m, args.n, args.k, args.alpha, args.split_k_slices = m, n, pairs, 1.0, 1
+    args.ptr_A, args.ptr_B, args.ptr_C = p.a.byte_pointer(), p.b.byte_pointer(), p.c.byte_pointer()
+    args.stride_A, args.stride_B, args.stride_C = m, n, n
+    args.indiceA, args.indiceBorC = p.a_inds.byte_pointer(), p.b_inds.byte_pointer()
+    args.workspace, args.workspace_bytes = ws.byte_pointer(), ws.nbytes
+    args.rows_A, args.rows_B, args.rows_C = 3000, 3000, m
+    _capi.check(getattr(lib, entry)(ctypes.byref(cd), ctypes.byref(args), 0))
+    assert np.abs(H.as_f32(H.host(p.c), "f16") - ref).max() <= TOL["f16"] * np.abs(ref).max()
+    assert bool((H.host(ws) != 0xA5).any()) == used
+
+
+def test_a_validated_call_recorded_into_a_graph_leaves_its_workspace_alone():
+    """The call is validated on the stream that is recorded afterwards, the parameter object stays as it is."""
+    print("case shuffle_ab graph validated", flush=True)
+    p, ref = _shuffle_ab(np.random.default_rng(5), 2000, 64, 72, 1000)
+    few, _ = _shuffle_ab(np.random.default_rng(6), 2000, 64, 72, 100)      # (loads the kernel that the graph will hold)
+    GemmMainUnitTest.matmul2(few)
+    side = torch.cuda.Stream()
+    p.stream = side.cuda_stream
+    GemmMainUnitTest.matmul2(p)
+    kept = p.__dict__["_prepared"]
+    workspace = kept[6]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        GemmMainUnitTest.matmul2(p)
+    assert p.__dict__["_prepared"] is kept and workspace.nbytes > 0
+    for _ in range(3):
+        workspace.fill_int_(0x5A)
+        p.c.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.abs(H.as_f32(H.host(p.c), "f16") - ref).max() <= TOL["f16"] * np.abs(ref).max()
+        assert bool((H.host(workspace) == 0x5A).all())
+        GemmMainUnitTest.matmul2(p)      # the eager call still uses it
+        torch.cuda.synchronize()
+        assert bool((H.host(workspace) != 0x5A).any())
