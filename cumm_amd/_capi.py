@@ -83,6 +83,7 @@ SYMBOLS = {
     "cumm_hip_last_error": (C.c_char_p, []),
     "cumm_hip_last_wgrad_path": (C.c_int, []),
     "cumm_hip_device_count": (C.c_int, [C.POINTER(C.c_int)]),
+    "cumm_hip_get_device": (C.c_int, [C.POINTER(C.c_int)]),
     "cumm_hip_malloc": (C.c_int, [_PVP, C.c_size_t]),
     "cumm_hip_free": (C.c_int, [_VP]),
     "cumm_hip_host_malloc": (C.c_int, [_PVP, C.c_size_t]),

@@ -723,7 +723,7 @@ static int gemm_impl(const CummHipGemmDesc *desc, const CummHipGemmArgs *a, void
 int cumm_hip_gemm(const CummHipGemmDesc *desc, const CummHipGemmArgs *a, void *stream) { return gemm_impl(desc, a, stream, false); }
 
 int cumm_hip_gemm_in_workspace(const CummHipGemmDesc *desc, const CummHipGemmArgs *a, void *stream) {
-  return gemm_impl(desc, a, stream, true);
+  return gemm_impl(desc, a, stream, !cumm_hip_stream_is_capturing(stream));
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1033,6 +1033,11 @@ int cumm_hip_device_count(int *count) {
   if (!count) return fail(CUMM_HIP_EINVAL, "null out-param");
   hipError_t e = hipGetDeviceCount(count);
   if (e != hipSuccess) { *count = 0; return hip_fail(e, "hipGetDeviceCount"); }
+  return CUMM_HIP_OK;
+}
+int cumm_hip_get_device(int *device) {
+  if (!device) return fail(CUMM_HIP_EINVAL, "null out-param");
+  HIP_TRY(hipGetDevice(device));
   return CUMM_HIP_OK;
 }
 int cumm_hip_malloc(void **ptr, size_t bytes) {

@@ -165,7 +165,8 @@ typedef struct CummHipSparseConvArgs {
 int cumm_hip_gemm(const CummHipGemmDesc *desc, const CummHipGemmArgs *args, void *stream);
 /* The same call, which may also use args->workspace (16-byte aligned) with split_k_slices == 1, where
  * cumm_hip_gemm leaves it alone: see cumm_hip_query_gemm_optional_workspace.  Calls that may overlap
- * in time, on several streams or from several threads, each need a workspace of their own then. */
+ * in time, on several streams or from several threads, each need a workspace of their own then.  While
+ * the stream is recorded into a graph, which may outlive the workspace, it is cumm_hip_gemm. */
 int cumm_hip_gemm_in_workspace(const CummHipGemmDesc *desc, const CummHipGemmArgs *args, void *stream);
 
 /* Replaces ConvMainUnitTest.implicit_gemm2 below its prelude for mask_sparse
@@ -236,6 +237,7 @@ int cumm_hip_last_wgrad_path(void);
 /* ---- device backend of tv::Tensor / tv::Context (include/tensorview/tensor.h:181-330
  * allocation, :1395 zero_, :1525-1766 copy_/cpu()/cuda(); include/tensorview/contexts/core.h:429-500) */
 int cumm_hip_device_count(int *count);                 /* host out-param */
+int cumm_hip_get_device(int *device);                  /* the calling thread's current device */
 int cumm_hip_malloc(void **ptr, size_t bytes);         /* host out-param */
 int cumm_hip_free(void *ptr);
 int cumm_hip_host_malloc(void **ptr, size_t bytes);    /* pinned host memory */

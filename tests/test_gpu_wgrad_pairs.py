@@ -208,3 +208,33 @@ def test_a_validated_call_recorded_into_a_graph_leaves_its_workspace_alone():
         GemmMainUnitTest.matmul2(p)      # the eager call still uses it
         torch.cuda.synchronize()
         assert bool((H.host(workspace) != 0x5A).any())
+
+
+def test_new_parameter_objects_allocate_no_workspace_of_their_own(monkeypatch):
+    """A loop over offsets with an object per call, and one object that is given new index lists."""
+    print("case shuffle_ab new objects", flush=True)
+    p, ref = _shuffle_ab(np.random.default_rng(7), 3000, 64, 72, 4000)
+    real, calls = _capi.lib(), []
+
+    class Counting:
+        def __getattr__(self, name):
+            if name in ("cumm_hip_malloc", "cumm_hip_free"):
+                calls.append(name)
+            return getattr(real, name)
+
+    def again():
+        q = GemmParams()
+        q.algo_desp = p.algo_desp
+        q.a, q.b, q.c, q.a_inds, q.b_inds = p.a, p.b, p.c, p.a_inds, p.b_inds
+        GemmMainUnitTest.matmul2(q)
+    full = p.a_inds, p.b_inds
+    GemmMainUnitTest.matmul2(p)
+    again()
+    monkeypatch.setattr(_capi, "_lib", Counting())
+    for pairs in (4000, 300, 4000):
+        again()
+        p.a_inds, p.b_inds = (t.slice_first_axis(0, pairs) for t in full)
+        GemmMainUnitTest.matmul2(p)
+    monkeypatch.setattr(_capi, "_lib", real)
+    assert calls == []
+    assert np.abs(H.as_f32(H.host(p.c), "f16") - ref).max() <= TOL["f16"] * np.abs(ref).max()
