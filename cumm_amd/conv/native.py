@@ -14,13 +14,15 @@ Forward and backward-input accumulate all offsets in an fp32 image (the f16 / bf
 and round once at the end (``cumm_hip_finish_rows``, with bias and activation): one rounding, as
 the mask-based kernels make, instead of one per offset.
 """
+import ctypes
+import threading
 from typing import Optional
 
 import numpy as np
 
 from .. import _capi
 from .. import tensorview as tv
-from ..gemm.main import GemmMainUnitTest, _check_device, _check_dtype
+from ..gemm.main import GemmMainUnitTest, _check_device, _check_dtype, _Slots, desp_to_c
 from ..tensorview.gemm import Activation, GemmParams, ShuffleStrideType
 
 
@@ -170,7 +172,7 @@ class WeightPlan:
 
     def __init__(self, dout, inp, dweight, lists, stream):
         self._tensors, self._lists, self._stream = (dout, inp, dweight), lists, stream
-        self._workspace = None
+        self._slots = None
         lib = _capi.lib()
         kv, k_out, c_in = dweight.dim(1), dweight.dim(0), dweight.dim(2)
         self._fn = lib.cumm_hip_wgrad_pairs
@@ -194,9 +196,10 @@ class WeightPlan:
         """Run on other tensors of the same shapes (device addresses), on ``stream``.  Without a
         workspace (``workspace_bytes`` bytes) the plan's own is used: one run at a time then."""
         if workspace_ptr is None:
-            if self._workspace is None:
-                self._workspace = tv.empty([max(self.workspace_bytes, 16)], tv.uint8, 0)
-            workspace_ptr = self._workspace.byte_pointer()
+            slots = self._slots
+            if slots is None or slots.stream != stream:
+                slots = self._slots = _Slots(_Slots._device(), stream, max(self.workspace_bytes, 16), id(self))
+            workspace_ptr = slots.tensor.byte_pointer()
         status = self._fn(dweight_ptr, dout_ptr, inp_ptr, *self._pairs, *self._sizes, workspace_ptr, self.workspace_bytes, stream)
         if status:
             _capi.check(status)
@@ -235,14 +238,18 @@ def _in_one_call(dout, inp, dweight, lists) -> bool:
 
 class WeightSteps:
     """Backward-weight as one gathered product per kernel offset: rows with a stride of their own, more
-    offsets than one call takes."""
+    offsets than one call takes.  The first run validates each product; runs after it, and ``rebind`` on
+    other tensors of the same shapes, go straight to the C entry points.  The products run one after the
+    other on one stream and share a workspace."""
 
     _NO_PAIR = {}
 
     def __init__(self, dout, inp, dweight, lists, stream):
-        self.steps = []
+        self.steps, self._tensors, self._stream = [], (dout, inp, dweight), stream
+        self._blocks, self._slots, self._lock = None, None, threading.Lock()
+        self._workspace_bytes = 0
         for k in range(dweight.dim(1)):
-            cnt = int(lists.counts[k])
+            cnt = min(int(lists.counts[k]), lists.pair_in.dim(1))
             p = GemmParams()
             p.algo_desp = _find(inp.dtype, inp.dtype, ShuffleStrideType.ShuffleAB, 64, 64, True, False).copy()
             p.a, p.b, p.c = dout, inp, dweight.select(1, k)
@@ -255,15 +262,77 @@ class WeightSteps:
                     self._NO_PAIR[dev] = tv.from_numpy(np.full(32, -1, np.int32)).cuda()
                 p.a_inds = p.b_inds = self._NO_PAIR[dev]
             p.stream = stream
+            self._workspace_bytes = max(self._workspace_bytes, self._optional(p))
             self.steps.append(p)
 
-    def __call__(self) -> None:
+    @staticmethod
+    def _optional(p) -> int:
+        return int(_capi.lib().cumm_hip_query_gemm_optional_workspace(
+            ctypes.byref(desp_to_c(p.algo_desp)), p.a.dim(1), p.b.dim(1), p.a_inds.dim(0)))
+
+    def split(self, slices: int, workspace: Optional[tv.Tensor]) -> None:
+        """Cut the products that are not spread over the device in any case into ``slices`` where they have
+        pairs enough."""
         for p in self.steps:
-            GemmMainUnitTest.matmul2(p)
+            if self._optional(p) <= 0 and p.a_inds.dim(0) >= 4096 * slices:
+                p.split_k_slices = slices
+            if workspace is not None:
+                p.workspace = workspace
+
+    def _share(self, stream: int) -> None:
+        if self._workspace_bytes > 0 and (self._slots is None or self._slots.stream != stream):
+            self._slots = _Slots(_Slots._device(), stream, self._workspace_bytes, None)
+
+    def __call__(self) -> None:
+        if self._tensors is None:
+            raise RuntimeError("the plan has released its tensors: use rebind")
+        with self._lock:      # (a product's two launches and the next one's use the same workspace)
+            if self._blocks is not None:
+                self._run(*(t.byte_pointer() for t in self._tensors), self._stream)
+                return
+            self._share(self._stream)
+            for p in self.steps:
+                p.__dict__["_slots"] = self._slots
+                GemmMainUnitTest.matmul2(p)
+            blocks = []
+            base = self._tensors[2].byte_pointer()
+            for p in self.steps:
+                prep = p.__dict__.get("_prepared")
+                if prep is None:      # (recorded into a graph: validated again by the next run)
+                    return
+                args = prep[5]
+                blocks.append((prep[1], prep[2], prep[3], args, args.ptr_C - base, bool(args.workspace) and args.split_k_slices == 1,
+                               prep[4], prep[6]))
+            self._blocks = blocks
+
+    def _run(self, dout_ptr: int, inp_ptr: int, dweight_ptr: int, stream: int) -> None:
+        self._share(stream)
+        for fn, cdesc_ref, args_ref, args, delta, shares, _, _ in self._blocks:
+            args.ptr_A, args.ptr_B = dout_ptr, inp_ptr
+            args.ptr_C = args.ptr_D = dweight_ptr + delta
+            if shares:
+                args.workspace, args.workspace_bytes = self._slots.tensor.byte_pointer(), self._slots.tensor.nbytes
+            status = fn(cdesc_ref, args_ref, stream)
+            if status:
+                _capi.check(status)
+
+    def rebind(self, dout_ptr: int, inp_ptr: int, dweight_ptr: int, stream: int) -> None:
+        """Run on other tensors of the same shapes and strides (device addresses), on ``stream``."""
+        with self._lock:
+            if self._blocks is None:
+                raise RuntimeError("the plan has not run yet")
+            self._run(dout_ptr, inp_ptr, dweight_ptr, stream)
+
+    def release(self) -> None:
+        """Forget the tensors of the first run (a caller that goes on through ``rebind`` with its own): the
+        argument blocks hold addresses only, the pair lists belong to their owner."""
+        if self._blocks is None:
+            raise RuntimeError("the plan has not run yet")
+        self._launches, self.steps, self._tensors = self.launches, [], None
 
     @property
     def launches(self) -> int:
-        return len(self.steps)
+        return len(self.steps) if self._tensors is not None else self._launches
 
 
 def backward_weight(dout: tv.Tensor, inp: tv.Tensor, dweight: tv.Tensor, lists, *, split_k_slices: int = 1,
@@ -272,7 +341,11 @@ def backward_weight(dout: tv.Tensor, inp: tv.Tensor, dweight: tv.Tensor, lists, 
     ``split_k_slices`` is what a caller of the per-offset products would pass; the pairs are spread
     over the device in any case.  ``workspace`` is used when it is large enough."""
     plan = plan_backward_weight(dout, inp, dweight, lists, stream=stream)
-    if (isinstance(plan, WeightPlan) and workspace is not None and not workspace.empty() and
-            workspace.nbytes >= plan.workspace_bytes and workspace.byte_pointer() % 16 == 0):
-        plan._workspace = workspace
-    plan()      # (a workspace of its own goes away with the plan: freeing device memory waits for it)
+    if isinstance(plan, WeightSteps):
+        plan.split(split_k_slices, workspace)
+        plan()
+    elif (workspace is not None and not workspace.empty() and workspace.nbytes >= plan.workspace_bytes and
+          workspace.byte_pointer() % 16 == 0):
+        plan.rebind(dout.byte_pointer(), inp.byte_pointer(), dweight.byte_pointer(), stream, workspace.byte_pointer())
+    else:
+        plan()

@@ -7,7 +7,7 @@ m/n/k extraction, workspace rules; the launch itself goes through the C ABI
 """
 import bisect
 import ctypes
-from typing import Dict, List, Tuple
+from typing import Dict, List, Optional, Tuple
 
 from .. import _capi
 from ..tensorview import Tensor, empty, int32, uint8
@@ -94,10 +94,11 @@ class _Slots:
     object at a time has a buffer: threads that launch on one stream have one each.  (A stream has to be
     finished when it is destroyed, so the handle may come again.)"""
 
-    _MOST = 8          # buffers that wait for an owner, of 8 MB at most
+    _MOST = 8          # buffers that wait for an owner,
+    _LARGEST = 1 << 23   # each of so many bytes at most (one product needs no more)
     _spare = {}        # (device, stream, number) -> tensor; single dict operations only, which threads may mix
 
-    def __init__(self, device: int, stream: int, nbytes: int, owner: int):
+    def __init__(self, device: int, stream: int, nbytes: int, owner: Optional[int]):
         self.device, self.stream, self.owner, self.tensor = device, stream, owner, None
         for i in range(self._MOST):
             t = self._spare.pop((self.device, stream, i), None)
@@ -105,7 +106,7 @@ class _Slots:
                 self.tensor = t
                 break
         if self.tensor is None:
-            self.tensor = empty([max(1 << (nbytes - 1).bit_length(), 1 << 16)], uint8, 0)
+            self.tensor = empty([nbytes if nbytes > self._LARGEST else max(1 << (nbytes - 1).bit_length(), 1 << 16)], uint8, 0)
 
     @staticmethod
     def _device() -> int:
@@ -116,15 +117,15 @@ class _Slots:
     @classmethod
     def of(cls, params, nbytes: int) -> Tensor:
         kept, device = params.__dict__.get("_slots"), cls._device()
-        # (not for a copy of the object that took it: copies may run beside it)
-        if (kept is None or kept.owner != id(params) or kept.stream != params.stream or kept.device != device or
+        # (not for a copy of the object that took it: copies may run beside it; None: shared on purpose)
+        if (kept is None or kept.owner not in (None, id(params)) or kept.stream != params.stream or kept.device != device or
                 kept.tensor.nbytes < nbytes):
             kept = params.__dict__["_slots"] = cls(device, params.stream, nbytes, id(params))
         return kept.tensor
 
     def __del__(self):
         t, self.tensor = getattr(self, "tensor", None), None
-        if t is None:
+        if t is None or t.nbytes > self._LARGEST:
             return
         try:
             for i in range(self._MOST):

@@ -238,3 +238,32 @@ def test_new_parameter_objects_allocate_no_workspace_of_their_own(monkeypatch):
     monkeypatch.setattr(_capi, "_lib", real)
     assert calls == []
     assert np.abs(H.as_f32(H.host(p.c), "f16") - ref).max() <= TOL["f16"] * np.abs(ref).max()
+
+
+def test_a_plan_of_single_products_on_other_tensors_and_another_stream():
+    """Columns of wider tensors: the plan's second run, on tensors of its own and a second stream."""
+    from types import SimpleNamespace
+    from cumm_amd.conv import native
+    print("case weight steps rebind", flush=True)
+    rng = np.random.default_rng(8)
+    kv, rows, k_out, c_in, most = 5, 900, 24, 40, 3000
+    counts = np.array([3000, 0, 17, 257, 1500], np.int32)
+    po, pi = (rng.integers(0, rows, size=(kv, most)).astype(np.int32) for _ in range(2))
+    lists = SimpleNamespace(pair_in=H.dev(pi, "i32"), pair_out=H.dev(po, "i32"), counts=counts)
+    sets = []
+    for _ in range(2):
+        dout, inp = _data(rng, (rows, k_out + 8), "f16"), _data(rng, (rows, c_in + 16), "f16")
+        f_out, f_in = H.as_f32(dout, "f16")[:, :k_out], H.as_f32(inp, "f16")[:, :c_in]
+        ref = np.stack([f_out[po[r, :n]].T @ f_in[pi[r, :n]] for r, n in enumerate(counts)], axis=1)
+        sets.append((H.dev(dout, "f16").slice_axis(1, 0, k_out), H.dev(inp, "f16").slice_axis(1, 0, c_in),
+                     H.dev(_data(rng, (k_out, kv, c_in), "f16"), "f16"), ref))
+    plan = native.plan_backward_weight(*sets[0][:3], lists)
+    assert isinstance(plan, native.WeightSteps)
+    side = torch.cuda.Stream()
+    plan()
+    plan()
+    torch.cuda.synchronize()
+    plan.rebind(*(t.byte_pointer() for t in sets[1][:3]), side.cuda_stream)
+    torch.cuda.synchronize()
+    for _, _, dw, ref in sets:
+        assert np.abs(H.as_f32(H.host(dw), "f16") - ref).max() <= TOL["f16"] * np.abs(ref).max()

@@ -63,3 +63,82 @@ def test_host_tensors_other_devices_and_other_list_types_are_refused(calls):
 def test_a_count_ends_with_its_list(calls, counts):
     _run(_operands(len(counts), counts))
     assert calls[0][0].tolist() == [min(max(c, 0), MOST) for c in counts] and calls[0][1] == MOST
+
+
+@pytest.fixture
+def products(monkeypatch):
+    """The argument blocks that reach cumm_hip_gemm and cumm_hip_gemm_in_workspace, in order; host memory
+    stands for the workspaces."""
+    from cumm_amd.gemm import main
+    real, made = _capi.lib(), []
+
+    class Library:
+        def __getattr__(self, name):
+            if name not in ("cumm_hip_gemm", "cumm_hip_gemm_in_workspace", "cumm_hip_stream_is_capturing"):
+                return getattr(real, name)
+            if name == "cumm_hip_stream_is_capturing":
+                return lambda stream: 0
+
+            def entry(desc, args, stream):
+                made.append((name, _capi.GemmArgs.from_buffer_copy(args._obj), stream))
+                return 0
+            return entry
+    monkeypatch.setattr(_capi, "_lib", Library())
+    monkeypatch.setattr(main, "empty", lambda shape, dtype, device: tv.Tensor(shape, dtype))
+    monkeypatch.setattr(main._Slots, "_device", staticmethod(lambda: 0))
+    monkeypatch.setattr(main._Slots, "_spare", {})
+    monkeypatch.setattr(native.WeightSteps, "_NO_PAIR", {0: tv.from_blob(0x7D0000000000, [32], tv.int32, 0)})
+    return made
+
+
+def _wide_operands(kv, counts, k_out=K, c_in=C):
+    """Gradients and features that are columns of wider tensors: one product per offset."""
+    blob = lambda at, shape, dtype: tv.from_blob(at, shape, dtype, 0)
+    lists = SimpleNamespace(pair_in=blob(0x7F0000000000, [kv, 50000], tv.int32), pair_out=blob(0x7F1000000000, [kv, 50000], tv.int32),
+                            counts=np.asarray(counts))
+    return (blob(0x7F2000000000, [ROWS, k_out + 8], tv.float16).slice_axis(1, 0, k_out),
+            blob(0x7F3000000000, [ROWS, c_in + 8], tv.float16).slice_axis(1, 0, c_in), blob(0x7F4000000000, [k_out, kv, c_in], tv.float16),
+            lists)
+
+
+def test_a_plan_of_single_products_runs_again_on_other_tensors(products):
+    counts = [5000, 0, 12, 300, 40000]
+    plan = native.plan_backward_weight(*_wide_operands(5, counts), stream=3)
+    assert isinstance(plan, native.WeightSteps) and plan.launches == 5
+    for early in (lambda: plan.rebind(1 << 20, 2 << 20, 3 << 20, 0), plan.release):
+        with pytest.raises(RuntimeError, match="not run yet"):
+            early()
+    plan()
+    first = products[:]
+    assert [a.k for _, a, _ in first] == [5000, 32, 12, 300, 40000] and {s for _, _, s in first} == {3}
+    # products with pairs enough share one workspace, the others have none
+    spread = [name == "cumm_hip_gemm_in_workspace" for name, _, _ in first]
+    assert spread == [True, False, False, True, True]
+    assert len({a.workspace for (_, a, _), w in zip(first, spread) if w}) == 1
+    assert all(a.workspace is None for (_, a, _), w in zip(first, spread) if not w)
+    plan.release()
+    assert plan.launches == 5
+    with pytest.raises(RuntimeError, match="released"):
+        plan()
+    del products[:]
+    base = 0x600000000000
+    plan.rebind(base, base + (1 << 30), base + (2 << 30), 9)
+    for (name, a, stream), (was_name, was, _) in zip(products, first):
+        assert name == was_name and stream == 9 and (a.m, a.n, a.k) == (was.m, was.n, was.k)
+        assert (a.ptr_A, a.ptr_B) == (base, base + (1 << 30))
+        assert a.ptr_C == a.ptr_D == base + (2 << 30) + (was.ptr_C - 0x7F4000000000)
+        assert (a.indiceA, a.indiceBorC) == (was.indiceA, was.indiceBorC)
+    other = {a.workspace for (_, a, _), w in zip(products, spread) if w}
+    assert len(other) == 1 and other != {a.workspace for (_, a, _), w in zip(first, spread) if w}      # (another stream)
+
+
+def test_slices_are_what_the_caller_asks_for_where_no_workspace_spreads_the_pairs(products):
+    """Outputs of more tiles than the spread kernel takes; with few pairs and one slice as it was."""
+    workspace = tv.from_blob(0x7E0000000000, [1 << 20], tv.uint8, 0)
+    operands = _wide_operands(3, [40000, 100, 16384], k_out=1088, c_in=1024)
+    native.backward_weight(*operands, split_k_slices=4, workspace=workspace)
+    assert [(a.split_k_slices, name) for name, a, _ in products] == [(4, "cumm_hip_gemm"), (1, "cumm_hip_gemm"), (4, "cumm_hip_gemm")]
+    assert all(a.workspace == (0x7E0000000000 if a.split_k_slices > 1 else None) for _, a, _ in products)
+    del products[:]
+    native.backward_weight(*_wide_operands(2, [40000, 100]), split_k_slices=4)
+    assert [(a.split_k_slices, name) for name, a, _ in products] == [(1, "cumm_hip_gemm_in_workspace"), (1, "cumm_hip_gemm")]
