@@ -406,13 +406,16 @@ hipError_t run_wgrad_pairs(WgradPairsParams *w, WgradPairsFinalizeParams *f, con
 }
 
 // ShuffleAB products of two-byte operands with one slice whose pairs are many against their output
-// take the pair-list kernel: from kWgradPairsMin pairs on (its two launches take 8.0 us for 256 pairs of
-// 64 x 64 channels, the tiled kernel's one 9.4 us; for 192 pairs that one takes 7.6 us) and while the
-// output is not itself enough tiles to fill the device.
-constexpr int kWgradPairsMin = 256;
+// take the pair-list kernel, while the output is not itself enough tiles to fill the device: from
+// kWgradPairsMin pairs on (its two launches take 8.0 us for 256 pairs of 64 x 64 channels, the tiled kernel's
+// one 9.4 us; for 192 pairs that one takes 7.6 us), above kWgradPairsFewBlocks channel blocks, whose slots
+// are more to write and add up, from kWgradPairsMinLarge (1024 x 1024 channels: 256 pairs 12.2 us, tiled
+// 10.1; 400 pairs 12.8 and 14.6).
+constexpr int kWgradPairsMin = 256, kWgradPairsFewBlocks = 32, kWgradPairsMinLarge = 384;
 bool wgrad_pairs_serves(const CummHipGemmDesc &d, int m, int n, int k) {
-  return d.shuffle_type == CUMM_HIP_SHUFFLE_AB && is_float16_like(d.dtype_a) && k >= kWgradPairsMin && m % 8 == 0 && n % 8 == 0 &&
-         (int64_t)((m + 63) / 64) * ((n + 63) / 64) <= 256;
+  const int64_t blocks = (int64_t)((m + 63) / 64) * ((n + 63) / 64);
+  return d.shuffle_type == CUMM_HIP_SHUFFLE_AB && is_float16_like(d.dtype_a) && m % 8 == 0 && n % 8 == 0 && blocks <= 256 &&
+         k >= (blocks > kWgradPairsFewBlocks ? kWgradPairsMinLarge : kWgradPairsMin);
 }
 
 }  // namespace

@@ -82,11 +82,16 @@ __global__ __launch_bounds__(256) void wgrad_pairs_kernel(const WgradPairsParams
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, q = lane >> 4;
 
-  // the channel blocks of one share run on one XCD (numbers w, w + 8, ...), one after the other: the
-  // second block finds the rows' other halves in that XCD's L2
+  // The channel blocks of one share run on one XCD (numbers w, w + 8, ...), one after the other: the
+  // second block finds the rows' other halves in that XCD's L2.  Fewer than eight shares (more than 32
+  // blocks) would leave XCDs idle: each then takes an eighth of all blocks of all shares in that order
+  // (150 k pairs, 1024 x 1024 channels, one share: 5185 -> 736 us, 512 x 512: 258 -> 143 us; from eight
+  // shares on the first map is the faster one, 128 x 128 channels 20.0 and 20.8 us).
   const int combos = p.kblocks * p.cblocks;
   const int xcd = blockIdx.x & 7, nth = blockIdx.x >> 3;
-  const int b = (nth / combos) * 8 + xcd, combo = nth % combos;
+  const int unit = p.wgs >= 8 ? nth : xcd * (int)(gridDim.x >> 3) + nth;
+  const int combo = unit % combos;
+  const int b = p.wgs >= 8 ? (unit / combos) * 8 + xcd : unit / combos;
   if (b >= p.wgs) return;
   const int kb = combo / p.cblocks, cb = combo % p.cblocks;
 

@@ -23,7 +23,8 @@ hipError_t CUMM_CAT(launch_wgrad_pairs_, CUMM_NAME)(const WgradPairsParams &p, c
                                                     int most_slots, hipStream_t s) {
   using T = CUMM_ELEM;
   if (!counted_waits_hold<wgrad_pairs_kernel<T>>()) return hipErrorNotSupported;
-  const unsigned grid = (unsigned)((p.wgs + 7) / 8 * 8) * (unsigned)(p.kblocks * p.cblocks);
+  const unsigned combos = (unsigned)(p.kblocks * p.cblocks), wgs = (unsigned)p.wgs;
+  const unsigned grid = wgs >= 8u ? (wgs + 7u) / 8u * 8u * combos : (wgs * combos + 7u) / 8u * 8u;     // (as the kernel maps them)
   if (grid) {
     hipLaunchKernelGGL(wgrad_pairs_kernel<T>, dim3(grid), dim3(256), 0, s, p);
     const hipError_t e = hipGetLastError();

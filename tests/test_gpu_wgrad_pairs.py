@@ -267,3 +267,15 @@ def test_a_plan_of_single_products_on_other_tensors_and_another_stream():
     torch.cuda.synchronize()
     for _, _, dw, ref in sets:
         assert np.abs(H.as_f32(H.host(dw), "f16") - ref).max() <= TOL["f16"] * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("k_out,c_in,pairs", [(576, 256, 400), (576, 520, 3000), (1024, 1024, 384), (1000, 1016, 5000), (2048, 136, 700)])
+def test_more_channel_blocks_than_a_share_fits_one_xcd(k_out, c_in, pairs):
+    """36 to 256 blocks of 64 x 64 channels: fewer than eight shares of the pairs, one for the largest."""
+    print("case wgrad_pairs blocks", k_out, c_in, pairs, flush=True)
+    p, ref = _shuffle_ab(np.random.default_rng(pairs), 2500, k_out, c_in, pairs)
+    GemmMainUnitTest.matmul2(p)
+    cd = desp_to_c(p.algo_desp)
+    assert int(_capi.lib().cumm_hip_query_gemm_optional_workspace(ctypes.byref(cd), k_out, c_in, pairs)) > 0
+    assert int(_capi.lib().cumm_hip_query_gemm_optional_workspace(ctypes.byref(cd), k_out, c_in, 383)) == 0
+    assert np.abs(H.as_f32(H.host(p.c), "f16") - ref).max() <= TOL["f16"] * np.abs(ref).max()
