@@ -1536,7 +1536,8 @@ static bool wgrad_pairs_args(const int32_t *counts, int lists, int K, int C) {
   if (!counts || lists < 1 || lists > kWgradPairsMaxLists || K <= 0 || C <= 0 || K % 8 || C % 8) return false;
   int64_t steps = 0;
   for (int r = 0; r < lists; ++r) {
-    if (counts[r] < 0) return false;
+    // (a list is read through a descriptor of its bytes, beyond whose first 2^31 absent entries are fetched)
+    if (counts[r] < 0 || counts[r] >= 1 << 29) return false;
     steps += ((int64_t)counts[r] + 31) / 32;
   }
   return steps < (int64_t)1 << 30 && (int64_t)((K + 63) / 64) * ((C + 63) / 64) < 4096;

@@ -142,3 +142,16 @@ def test_slices_are_what_the_caller_asks_for_where_no_workspace_spreads_the_pair
     del products[:]
     native.backward_weight(*_wide_operands(2, [40000, 100]), split_k_slices=4)
     assert [(a.split_k_slices, name) for name, a, _ in products] == [(1, "cumm_hip_gemm_in_workspace"), (1, "cumm_hip_gemm")]
+
+
+def test_lists_of_2_to_the_29_pairs_and_more_are_refused():
+    """Their bytes do not fit the 31 bits of an offset inside a list."""
+    lib = _capi.lib()
+    for counts, taken in (([(1 << 29) - 1], True), ([1 << 29], False), ([5, 1 << 30, 7], False), ([2147483647], False), ([-1], False)):
+        c = np.array(counts, np.int32)
+        need = lib.cumm_hip_wgrad_pairs_workspace(c.ctypes.data, len(counts), 64, 64)
+        assert (need > 0) == taken and (taken or need == -1), counts
+        if not taken:
+            at = 1 << 20      # (never read: the counts are refused first)
+            assert lib.cumm_hip_wgrad_pairs(at, at, at, at, at, c.ctypes.data, len(counts), 1 << 31, 10, 10, 64, 64, tv.float16, at,
+                                            1 << 40, None) == _capi.EINVAL
