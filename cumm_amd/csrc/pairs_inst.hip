@@ -121,12 +121,18 @@ __global__ __launch_bounds__(256) void pairs_insert_kernel(const SubmPairsParams
 
 // Workgroups go to the eight XCDs in turn.  This hands each of them a contiguous run of the inputs, all
 // lines of offsets of a block of inputs one after the other, so that what neighbours share is fetched
-// into one L2: -> block of inputs (or one past the last), *zy = line of offsets.
+// into one L2: -> block of inputs (or one past the last), *zy = line of offsets.  A launch has fewer than 2^32
+// threads along x: from there on the lines go along y, one after the other.
 constexpr unsigned kXcds = 8;
-__host__ __device__ __forceinline__ unsigned xcd_grid(unsigned blocks, unsigned lines) {
-  return kXcds * ((blocks + kXcds - 1) / kXcds) * lines;
+inline dim3 xcd_grid(unsigned blocks, unsigned lines) {
+  const unsigned long long all = (unsigned long long)kXcds * ((blocks + kXcds - 1) / kXcds) * lines;
+  return all < (1ull << 32) / 256 ? dim3((unsigned)all) : dim3(blocks, lines);
 }
 __device__ __forceinline__ int xcd_block(unsigned lines, int *zy) {
+  if (gridDim.y > 1) {
+    *zy = (int)blockIdx.y;
+    return (int)blockIdx.x;
+  }
   const unsigned per = gridDim.x / (kXcds * lines), j = blockIdx.x / kXcds;
   *zy = (int)(j % lines);
   return (int)((blockIdx.x % kXcds) * per + j / lines);
@@ -850,7 +856,7 @@ hipError_t launch_conv_pairs_fill(const ConvPairsParams &p, hipStream_t s) {
     if (wgs > 16384ull) wgs = 16384ull;
     hipLaunchKernelGGL(conv_bits_rows_kernel, dim3((unsigned)wgs), dim3(256), 0, s, p);
     if (p.n_in > 0)
-      hipLaunchKernelGGL(conv_bits_fill_kernel, dim3(xcd_grid((unsigned)(p.n_in + 255) / 256u, (unsigned)(p.kv / p.kx))), dim3(256), 0, s, p);
+      hipLaunchKernelGGL(conv_bits_fill_kernel, xcd_grid((unsigned)(p.n_in + 255) / 256u, (unsigned)(p.kv / p.kx)), dim3(256), 0, s, p);
     return hipGetLastError();
   }
   hipLaunchKernelGGL(conv_pairs_rows_kernel, dim3((most + 255) / 256), dim3(256), 0, s, p);
@@ -894,7 +900,7 @@ hipError_t launch_subm_pairs(const SubmPairsParams &p, hipStream_t s) {
   if ((uint32_t)p.n > most) most = (uint32_t)p.n;
   hipLaunchKernelGGL(pairs_clear_kernel, dim3((most + 255) / 256), dim3(256), 0, s, p);
   hipLaunchKernelGGL(pairs_insert_kernel, dim3((p.n + 255) / 256), dim3(256), 0, s, p);
-  hipLaunchKernelGGL(pairs_lookup_kernel, dim3(xcd_grid((unsigned)(p.n + 255) / 256u, (unsigned)(p.kv / p.kx))), dim3(256), 0, s, p);
+  hipLaunchKernelGGL(pairs_lookup_kernel, xcd_grid((unsigned)(p.n + 255) / 256u, (unsigned)(p.kv / p.kx)), dim3(256), 0, s, p);
   return hipGetLastError();
 }
 

@@ -6,6 +6,7 @@ import helpers as H
 from cumm_amd import _capi, pairs, synth
 from cumm_amd import tensorview as tv
 
+torch = pytest.importorskip("torch")      # (before the library: one HIP runtime in the process)
 pytestmark = pytest.mark.gpu
 
 
@@ -370,3 +371,42 @@ def test_sparse_conv_pairs_line_lengths(shape, batch, stride):
     coords = np.unique(coords, axis=0)
     coords = coords[rng.permutation(coords.shape[0])]
     _check_conv_case(coords, shape, stride=stride, batch_size=batch)
+
+
+@pytest.mark.parametrize("strided", [False, True])
+def test_more_lookups_than_threads_of_one_launch_axis(strided):
+    """36 M voxels and 121 lines of offsets, 2^32 lanes and more: a full box of voxels, so that every entry is
+    known."""
+    import ctypes as C
+    print("case 2^32 look-ups", strided, flush=True)
+    lib, arr3 = _capi.lib(), C.c_int32 * 3
+    shape, ksize = (36, 1000, 1000), (11, 11, 1)
+    n, kv = shape[0] * shape[1] * shape[2], 121
+    assert n * kv >= 1 << 32
+    row = torch.arange(n, dtype=torch.int32, device="cuda")
+    zyx = [row // (shape[1] * shape[2]), row // shape[2] % shape[1], row % shape[2]]
+    coords = torch.stack([torch.zeros_like(row)] + zyx, 1)
+    tables = [torch.full((kv, n), -7, dtype=torch.int32, device="cuda") for _ in range(2 if strided else 1)]
+    if strided:
+        geo = [arr3(*v) for v in (shape, ksize, (1, 1, 1), (5, 5, 0), (1, 1, 1))]
+        ws = torch.empty(int(lib.cumm_hip_conv_pairs_workspace(n, 1, *geo)), dtype=torch.uint8, device="cuda")
+        out_shape, found = arr3(), C.c_int32(0)
+        _capi.check(lib.cumm_hip_conv_pairs_sites(coords.data_ptr(), n, 1, *geo, out_shape, C.byref(found), ws.data_ptr(), ws.numel(), 0))
+        assert found.value == n and tuple(out_shape) == shape
+        sites = torch.empty_like(coords)
+        _capi.check(lib.cumm_hip_conv_pairs_fill(coords.data_ptr(), n, 1, *geo, n, sites.data_ptr(), tables[0].data_ptr(),
+                                                 tables[1].data_ptr(), None, None, ws.data_ptr(), ws.numel(), 0))
+        _capi.check(lib.cumm_hip_device_synchronize())
+        assert torch.equal(sites, coords)
+    else:
+        ws = torch.empty(int(lib.cumm_hip_subm_pairs_workspace(n)), dtype=torch.uint8, device="cuda")
+        _capi.check(lib.cumm_hip_subm_pairs(coords.data_ptr(), n, arr3(*shape), arr3(*ksize), arr3(1, 1, 1), tables[0].data_ptr(), None,
+                                            None, None, ws.data_ptr(), ws.numel(), 0))
+        _capi.check(lib.cumm_hip_device_synchronize())
+    for k in range(kv):
+        dz, dy = k // 11 - 5, k % 11 - 5
+        for sign, table in zip((1, -1), tables):      # the backward table looks the other way
+            z, y = zyx[0] + sign * dz, zyx[1] + sign * dy
+            inside = (z >= 0) & (z < shape[0]) & (y >= 0) & (y < shape[1])
+            want = torch.where(inside, row + sign * (dz * shape[1] + dy) * shape[2], torch.full_like(row, -1))
+            assert torch.equal(table[k], want), (k, sign)
