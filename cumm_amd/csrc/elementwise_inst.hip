@@ -197,21 +197,26 @@ hipError_t launch_finish_rows(const FinishRowsParams &p, bool bf16, hipStream_t 
   return hipGetLastError();
 }
 
+constexpr size_t kGatePieces = (size_t)1 << 31;      // of one launch, which has fewer than 2^32 threads
+
 template <class T>
-static void relu_backward(void *dst, const void *grad, const void *out, size_t vecs, hipStream_t s) {
-  const dim3 grid((unsigned)((vecs + 255) / 256));
+static hipError_t relu_backward(void *dst, const void *grad, const void *out, size_t vecs, hipStream_t s) {
   v4i *d = reinterpret_cast<v4i *>(dst);
   const v4i *g = reinterpret_cast<const v4i *>(grad), *o = reinterpret_cast<const v4i *>(out);
-  if (vecs * 16 > kStreamBytes) hipLaunchKernelGGL((relu_backward_kernel<T, true>), grid, dim3(256), 0, s, d, g, o, vecs);
-  else hipLaunchKernelGGL((relu_backward_kernel<T, false>), grid, dim3(256), 0, s, d, g, o, vecs);
+  const bool stream = vecs * 16 > kStreamBytes;
+  for (size_t at = 0; at < vecs; at += kGatePieces) {
+    const size_t n = vecs - at < kGatePieces ? vecs - at : kGatePieces;
+    const dim3 grid((unsigned)((n + 255) / 256));
+    if (stream) hipLaunchKernelGGL((relu_backward_kernel<T, true>), grid, dim3(256), 0, s, d + at, g + at, o + at, n);
+    else hipLaunchKernelGGL((relu_backward_kernel<T, false>), grid, dim3(256), 0, s, d + at, g + at, o + at, n);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 hipError_t launch_relu_backward(void *dst, const void *grad, const void *out, size_t vecs, bool bf16, hipStream_t s) {
-  if (vecs == 0) return hipSuccess;
-  if ((vecs + 255) / 256 > 0x7fffffffull) return hipErrorInvalidValue;
-  if (bf16) relu_backward<BF16>(dst, grad, out, vecs, s);
-  else relu_backward<F16>(dst, grad, out, vecs, s);
-  return hipGetLastError();
+  return bf16 ? relu_backward<BF16>(dst, grad, out, vecs, s) : relu_backward<F16>(dst, grad, out, vecs, s);
 }
 
 // Rows per block: two batches per row lane (32 KB of each operand), more below kFewBlocks blocks' worth of

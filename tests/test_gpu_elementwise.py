@@ -9,6 +9,7 @@ from cumm_amd import _capi
 from cumm_amd import tensorview as tv
 from oracle import numerics as onm
 
+torch = pytest.importorskip("torch")      # (before the library: one HIP runtime in the process)
 pytestmark = pytest.mark.gpu
 
 
@@ -92,3 +93,21 @@ def test_gate_and_sums_in_one_pass(dtype, rows, channels):
     np.testing.assert_array_equal(H.host(gated), H.host(gated2))
     np.testing.assert_array_equal(H.host(sums), H.host(sums2))
     assert np.array_equal(H.host(gated)[:rows], np.where(H.as_f32(out, dtype) > 0, grad, np.zeros_like(grad)))
+
+
+def test_relu_backward_of_more_pieces_than_a_launch_has_threads():
+    """2^32 pieces of eight elements and a few more (64 GiB), in place; the elements that pass lie at both ends
+    of every launch."""
+    vecs = (1 << 32) + 5
+    n = 8 * vecs
+    print("case relu_backward", n, flush=True)
+    x = torch.full((n,), -1.0, dtype=torch.float16, device="cuda")
+    on = sorted({0, 7, 8 * 255, 8 * (1 << 31) - 1, 8 * (1 << 31), 8 * (1 << 31) + 9, 8 * (1 << 32) - 1, 8 * (1 << 32), n - 1})
+    at = torch.tensor(on, device="cuda")
+    x[at] = 2.0
+    _capi.check(_capi.lib().cumm_hip_relu_backward(x.data_ptr(), x.data_ptr(), x.data_ptr(), n, tv.float16,
+                                                   torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert bool((x[at] == 2.0).all())
+    passed = sum(int(torch.count_nonzero(x[i:i + (1 << 31)])) for i in range(0, n, 1 << 31))
+    assert passed == len(on)
