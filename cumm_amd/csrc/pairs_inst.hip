@@ -104,7 +104,9 @@ __global__ __launch_bounds__(256) void pairs_insert_kernel(const SubmPairsParams
   const uint32_t low = (uint32_t)key;
   // do this key and those of all sites around it (which lie in the same grid) fit 32 bits?
   const unsigned long long last = coord_key(c.x, p.shape[0] - 1, p.shape[1] - 1, p.shape[2] - 1, p);
-  if (((key | last) >> 32) != 0ull) atomicOr(p.wide, 1u);
+  // (a store, always of the same value: atomic updates of one word complete one at a time.  300 k voxels in
+  // a grid of 2^34 sites, all kernels: 105 -> 74 us; 146 us with an atomic load first)
+  if (((key | last) >> 32) != 0ull) *p.wide = 1u;
   uint32_t h = mix32(low) & p.slot_mask;
   const unsigned long long mine = ((unsigned long long)(uint32_t)i << 32) | low;
   // at most `slots` probes: the table has at least twice as many slots as voxels.  (Skipping taken slots
