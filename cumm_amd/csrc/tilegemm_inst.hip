@@ -52,34 +52,60 @@ static hipError_t launch_dense_pipe(const TileGemmParams &p, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Which tile: the least estimated time, from measurements of f16 products (us; n = tiles per CU, rounded up,
-// of 256 CUs; k in elements; the second figure for rows that are no whole number of 128-byte lines, whose
-// fetches touch a line more each):
-//   64 x 64 x 64, 2 x 2 waves, three stages     3.5 + n (0.21 + 0.0033 / 0.0045 k), 0.0035 k for n = 1
-//                                               (1024^3 7.1; 2000 x 776 x 1160 12.4; 2048^3 28; 3000^3 152)
-//   the same with k split over eight waves      3.8 + 0.0018 n k    (256 x 256 x 4096: 11.2 against 15.8;
-//                                                                    one workgroup per CU: only for n = 1)
-//   128 x 64 x 64, three stages                 5.0 + 0.0105 / 0.0135 k per two tiles of a CU, 0.0076 k for
-//                                               one alone (1536 x 1536 x 4096 38 against 40; 2048^3 25)
-//   128 x 128 x 64, two stages                  5.0 + 0.0172 k per two tiles of a CU, 0.0138 k for one
-//                                               (2504^3 50 against 73; 2048 x 4096^2 73 against 96)
-//   256 x 256 x 32, 2 x 4 waves, four stages    8.5 + 0.0255 n k    (4096^3 120; 3000^3 85 against 104)
+// Which tile: the least estimated time, from measurements of f16 products on the 256 CUs that the figures are
+// for (us; n = tiles per CU, rounded up; k in elements; the larger of two lines where there are two: the
+// first is what a tile takes beside its steps, most of it its stores, the second the fetches of long
+// contractions, with a second figure for rows that are no whole number of 128-byte lines, whose fetches
+// touch a line more each):
+//   64 x 64 x 64, 2 x 2 waves, three stages   n = 1: 3.6 + 0.0039 k;  else
+//                                             2.6 + n (0.95 + 0.0026 k), from n = 8 on 1.05;
+//                                             2.6 + n (0.21 + 0.0033 / 0.0045 k)
+//                                             (1024^3 8.1; 2048^3 28; 3000^3 152; 3000^2 x 128 13.7)
+//   the same with k split over eight waves    n = 1 only: up to 32 tiles 3.8 + 0.0018 k (256 x 256 x 4096: 11.2
+//                                             against 15.8); more tiles of whole lines 4.3 + 0.0018 k while
+//                                             the tiles' rows fit the L2s (tiles * k up to 160 k: 512 x 320 x
+//                                             4096 11.8 - 15 against 18.7 - 20; 1024 x 512 x 1024 6.4 against
+//                                             7.7), beyond that 3.6 + 0.0038 k with an operand contiguous
+//                                             along its rows (1024^2 x 4096: nn 18.8 against 21.0, nt 21.6
+//                                             against 20.8).  Not for broken lines: 1344 x 440 x 2080
+//                                             nn 14.4 against 12.4
+//   128 x 64 x 64, three stages               n = 1: 5.8;  5.0 + 0.006 k;  else p = n / 2 rounded up:
+//                                             2.0 + p (4.4 + 0.008 k), from p = 3 on 0.0095;  5.0 + 0.0105 / 0.0135 p k
+//                                             (1536 x 1536 x 4096 38 against 40; 2048^3 25; 2048^2 x 256 8.7)
+//   128 x 128 x 64, two stages                n = 1: 9.0 + 0.0095 k;  5.0 + 0.0138 k;  else p = n / 2 rounded up:
+//                                             2.5 + p (8.0 + 0.0125 k);  5.0 + 0.0172 p k
+//                                             (2504^3 50 against 73; 2048 x 4096^2 73 against 96)
+//   256 x 256 x 32, 2 x 4 waves, four stages  2.0 + n (14.8 + 0.0235 k), up to k = 384 with result rows that are
+//                                             no whole lines, which it stores past the caches, 20.0;
+//                                             8.5 + 0.0255 n k
+//                                             (4096^3 120; 3000^3 85 against 104; 4096^2 x 256 21.5 against 27;
+//                                             tn 5768 x 2456 x 192 28 against 23)
 // The step-by-step cost of the small tiles is the chain of a step; from two workgroups per CU on it is the
 // 64 bytes per clock that a CU fetches: a 64 x 64 tile needs 512 bytes per MFMA of 16 x 16 x 32 (four clocks of
 // the CU's matrix cores), a 128 x 128 tile 256, a 256 x 256 tile 128.
+constexpr int kFigureCus = 256;
+inline int tiles_per_cu(const TileGemmParams &p, int tm, int tn) {
+  return (int)(((int64_t)((p.m + tm - 1) / tm) * ((p.n + tn - 1) / tn) + kFigureCus - 1) / kFigureCus);
+}
+
 template <class T, bool XT, bool YT>
 static hipError_t launch_dense_ring_layout(const TileGemmParams &p, hipStream_t s) {
-  const auto per_cu = [&](int tm, int tn) {
-    return (double)(((int64_t)((p.m + tm - 1) / tm) * ((p.n + tn - 1) / tn) + 255) / 256);
-  };
-  const double k = p.k, n64 = per_cu(64, 64), n128 = per_cu(128, 64), n256 = per_cu(256, 256);
+  const auto most = [](double a, double b) { return a > b ? a : b; };
+  const double k = p.k;
   const bool lines = p.ldx % 64 == 0 && p.ldy % 64 == 0;
-  const double t64 = 3.5 + (n64 == 1 ? 0.0035 * k : n64 * (0.21 + (lines ? 0.0033 : 0.0045) * k));
-  const double tw = n64 > 1 ? 1e30 : 3.8 + 0.0018 * k + ((int64_t)((p.m + 63) / 64) * ((p.n + 63) / 64) > 32 ? 0.0025 * k : 0.0);
-  const double t128 = 5.0 + (n128 > 1 ? (lines ? 0.0105 : 0.0135) * (double)(((int)n128 + 1) / 2) : 0.0076) * k;
-  const double n128s = per_cu(128, 128);
-  const double t128s = 5.0 + (n128s > 1 ? 0.0172 * (double)(((int)n128s + 1) / 2) : 0.0138) * k;
-  const double t256 = 8.5 + 0.0255 * n256 * k;
+  const int n64 = tiles_per_cu(p, 64, 64), n128 = tiles_per_cu(p, 128, 64), n128s = tiles_per_cu(p, 128, 128), n256 = tiles_per_cu(p, 256, 256);
+  const double tiles = (double)((p.m + 63) / 64) * ((p.n + 63) / 64);
+  const double t64 = n64 == 1 ? 3.6 + 0.0039 * k : 2.6 + n64 * most((n64 >= 8 ? 1.05 : 0.95) + 0.0026 * k, 0.21 + (lines ? 0.0033 : 0.0045) * k);
+  double tw = 1e30;
+  if (tiles <= 32) tw = 3.8 + 0.0018 * k;
+  else if (n64 == 1 && lines && tiles * k <= 160.0 * 1024) tw = 4.3 + 0.0018 * k;
+  else if (n64 == 1 && lines && (XT || YT)) tw = 3.6 + 0.0038 * k;
+  const double p128 = (n128 + 1) / 2, p128s = (n128s + 1) / 2;
+  const double t128 = n128 == 1 ? most(5.8, 5.0 + 0.006 * k)
+                                : most(2.0 + p128 * (4.4 + (p128 >= 3 ? 0.0095 : 0.008) * k), 5.0 + (lines ? 0.0105 : 0.0135) * p128 * k);
+  const double t128s = n128s == 1 ? most(9.0 + 0.0095 * k, 5.0 + 0.0138 * k)
+                                  : most(2.5 + p128s * (8.0 + 0.0125 * k), 5.0 + 0.0172 * p128s * k);
+  const double t256 = most(2.0 + n256 * ((p.ldc % 64 == 0 || k > 384 ? 14.8 : 20.0) + 0.0235 * k), 8.5 + 0.0255 * n256 * k);
   if (t256 <= t128s && t256 <= t128 && t256 <= t64 && t256 <= tw) return launch_dense_pipe<T, XT, YT>(p, s);
   if (t128s <= t128 && t128s <= t64 && t128s <= tw) return launch_dense_ring_as<T, 2, 2, 4, 4, 2, 2, XT, YT>(p, s);
   if (t128 <= t64 && t128 <= tw) return launch_dense_ring_as<T, 2, 2, 4, 2, 2, 3, XT, YT>(p, s);
@@ -91,6 +117,15 @@ static hipError_t launch_dense_ring_layout(const TileGemmParams &p, hipStream_t 
     return hipGetLastError();
   }
   return launch_dense_ring_as<T, 2, 2, 2, 2, 2, 3, XT, YT>(p, s);
+}
+
+// Contractions of a step or two have nothing to stream: half a step always, and up to a step and a half with
+// several tiles per CU, where what counts is how many workgroups start and store at once, the
+// register-staged kernel in 64 x 64 tiles is the faster one (536 x 928 x 16 3.7 us and 4.2; 3000^2 x 8 to 64: 8.6 - 11.5 us against 13.0 and more; 1352 x 3720 x 72 8.7 and 9.9; 4096^2 x 64 16.1 -
+// 19.2 and 17.7; with k = 128 13.8 and 13.6 at 3000^2).
+inline bool dense_ring_streams(const TileGemmParams &p) {
+  const int n = tiles_per_cu(p, 64, 64);
+  return p.k > (n >= 4 ? 96 : 32);
 }
 
 template <class T>
@@ -106,6 +141,10 @@ static bool launch_dense_ring(bool xk, bool yk, const TileGemmParams &p, hipStre
                     al16(p.X) && al16(p.Y) && al16(p.C) && al16(p.D) &&
                     ((y_rows - 1) * p.ldy + y_cols) * 2 < ((int64_t)1 << 31) && ((x_rows - 1) * p.ldx + x_cols) * 2 < ((int64_t)1 << 31);
     if (!ok) return false;
+    if (!dense_ring_streams(p)) {
+      *err = launch_xy<T, 2, 2>(xk, yk, p, dim3((p.m + 63) / 64, (p.n + 63) / 64, 1), s);
+      return true;
+    }
     if (xk && yk) *err = launch_dense_ring_layout<T, false, false>(p, s);
     else if (yk) *err = launch_dense_ring_layout<T, true, false>(p, s);
     else if (xk) *err = launch_dense_ring_layout<T, false, true>(p, s);

@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 TOL = {"f16": 2.0 ** -11, "bf16": 2.0 ** -8}
 
 
-def _run(dtype, m, n, k, ta, tb, source, alpha=1.0, beta=0.0, relu=False):
+def _run(dtype, m, n, k, ta, tb, source, alpha=1.0, beta=0.0, relu=False, tile=64):
     from cumm_amd.torch_bridge import torch2tensor
     tdt = {"f16": torch.float16, "bf16": torch.bfloat16}[dtype]
     gen = torch.Generator(device="cuda").manual_seed(m * 131 + n * 17 + k)
@@ -24,7 +24,7 @@ def _run(dtype, m, n, k, ta, tb, source, alpha=1.0, beta=0.0, relu=False):
     a, b = rnd(*((k, m) if ta else (m, k))), rnd(*((n, k) if tb else (k, n)))
     c = torch.full((m, n), float("nan"), dtype=tdt, device="cuda")
     p = GemmParams()
-    p.algo_desp = H.find_gemm_desp(dtype, ShuffleStrideType.NoShuffle, 64, 64, ta, tb)
+    p.algo_desp = H.find_gemm_desp(dtype, ShuffleStrideType.NoShuffle, tile, tile, ta, tb)
     p.a, p.b, p.c = torch2tensor(a), torch2tensor(b), torch2tensor(c)
     ref = alpha * ((a.float().t() if ta else a.float()) @ (b.float().t() if tb else b.float()))
     if source != "none":
@@ -70,3 +70,16 @@ def test_each_kernel_with_its_epilogue(m, n, k, ta, tb):
     print("case dense epilogue", m, n, k, ta, tb, flush=True)
     _run("f16", m, n, k, ta, tb, "matrix", alpha=0.5, beta=2.0)
     _run("bf16", m, n, k, ta, tb, "bias", alpha=1.0, beta=1.0, relu=True)
+
+
+@pytest.mark.parametrize("ta,tb", [(False, True), (False, False), (True, False), (True, True)])
+@pytest.mark.parametrize("tile", [64, 128])
+def test_short_contractions_on_either_side_of_the_streaming_kernels(tile, ta, tb):
+    """k from half a step to a step and a half, with fewer and with more than three tiles per CU, whatever tile
+    the descriptor has: the register-staged kernel below the line, the streaming ones above it."""
+    torch.backends.cuda.matmul.allow_tf32 = False
+    for m, n in ((200, 136), (1992, 2056)):
+        for k in (8, 32, 40, 64, 96, 104):
+            print("case dense short", tile, m, n, k, ta, tb, flush=True)
+            _run("f16", m, n, k, ta, tb, "matrix", alpha=0.5, beta=2.0, tile=tile)
+            _run("bf16", m, n, k, ta, tb, "bias", alpha=1.0, beta=1.0, relu=True, tile=tile)
