@@ -281,3 +281,56 @@ def test_a_geometry_whose_tables_exceed_31_bits_of_bytes(strided):
     with pytest.raises(RuntimeError):
         tb.sparse_conv(torch.zeros(n, 8, dtype=torch.float16, device="cuda"), torch.zeros(8, kv, 8, dtype=torch.float16, device="cuda"),
                        None, geo)
+
+
+def test_a_geometry_shared_by_streams_and_threads():
+    """Built on the default stream, used by two threads on streams of their own, each with its tensors, and on
+    the default stream again; the threads' first passes make the validated calls at the same time."""
+    import threading
+
+    from cumm_amd import torch_bridge as tb
+    print("case shared geometry", flush=True)
+    coords, grid = H.small_cloud(51, 3000)
+    geo = tb.SparseConvGeometry(torch.as_tensor(coords, device="cuda"), grid, stride=(2, 2, 2))
+    host = pairs.sparse_conv_pairs(coords, grid)
+    c_in, k_out = 72, 88      # a kind of call that no other test has made
+    gen = torch.Generator().manual_seed(4)
+    jobs = []
+    for _ in range(2):
+        feat, weight = torch.randn(geo.n_in, c_in, generator=gen).half(), (torch.randn(k_out, 27, c_in, generator=gen) * 0.05).half()
+        gout = torch.randn(geo.n_out, k_out, generator=gen).half()
+        f_r, w_r = feat.float().requires_grad_(True), weight.float().requires_grad_(True)
+        ref = _reference(f_r, w_r, None, host.indices_fwd, relu=False)
+        (ref * gout.float()).sum().backward()
+        jobs.append((feat.cuda(), weight.cuda(), gout.cuda(), (ref.detach(), f_r.grad, w_r.grad)))
+    torch.cuda.synchronize()
+    results, errors = [[], []], []
+
+    def work(i, passes):
+        try:
+            feat, weight, gout, _ = jobs[i]
+            for _ in range(passes):
+                f_d, w_d = feat.clone().requires_grad_(True), weight.clone().requires_grad_(True)
+                out = tb.sparse_conv(f_d, w_d, None, geo)
+                out.backward(gout)
+                results[i].append((out.detach(), f_d.grad, w_d.grad))
+        except Exception as e:      # (a thread's exception is the test's)
+            errors.append(e)
+
+    def on_a_stream(i):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            work(i, 6)
+        stream.synchronize()
+    threads = [threading.Thread(target=on_a_stream, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    work(0, 1)
+    torch.cuda.synchronize()
+    assert errors == [] and [len(r) for r in results] == [7, 6]
+    for got, (_, _, _, want) in zip(results, jobs):
+        for passed in got:
+            for a, b in zip(passed, want):
+                assert float((a.float().cpu() - b).abs().max() / b.abs().max()) < 1e-2
