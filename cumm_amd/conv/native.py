@@ -1,10 +1,9 @@
 """Per-offset ("native") sparse convolution: one gather-GEMM-scatter per kernel offset.
 
 ``SparseConvAlgo.Native`` of the reference (include/tensorview/gemm/core/constants.h:34-38): what
-its callers fall back to when the mask-based kernels do not apply, and the only path for kernel
-volumes above 32, which 32-bit masks cannot describe (the reference's ``dynamic_mask`` loader,
-cumm/gemm/blockmma/mma.py:78-269, is not built here).  The pattern is the reference's own check
-of its kernels, cumm/conv/main_real_spconv.py:309-403:
+its callers fall back to when the mask-based kernels do not apply; kernel volumes above 32 take the
+``dynamic_mask`` descriptors forward and backward-input, and this path for their weight gradient.  The
+pattern is the reference's own check of its kernels, cumm/conv/main_real_spconv.py:309-403:
 
     forward          out[pair_out[k]]  += inp[pair_in[k]]   @ W[:, k, :].T     (matmul2, ShuffleAC)
     backward-input   dinp[pair_in[k]]  += dout[pair_out[k]] @ W[:, k, :]       (matmul2, ShuffleAC)

@@ -14,8 +14,10 @@
 // and the sums are bound by HBM and run as many short workgroups in memory order: a resident grid
 // whose workgroups walk the tensor with a stride drifts apart and loses open pages (gate of 652 k rows of
 // 256 channels, 1.0 GB: 203 us with 4096 workgroups walking, 169 us with one per 256 pieces).  Operands
-// that are read once and exceed what the last-level cache keeps are loaded non-temporally (1 M rows
-// of 128: 130 -> 110 us; 161 us for the 1.0 GB); below kStreamBytes that gives nothing.
+// of more than kStreamBytes are loaded non-temporally (1 M rows of 128: 130 -> 110 us; 161 us for the
+// 1.0 GB; 64 MB with the gradient fresh from its producer 36 -> 33 us, all of it in memory 59 -> 37;
+// only where the last-level cache holds all three tensors, from a call just before, up to 90 MB each,
+// it costs: 300 k rows of 128 again and again 34 -> 37 us).
 #include "launch.h"
 
 namespace cummhip {

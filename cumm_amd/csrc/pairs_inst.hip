@@ -402,8 +402,8 @@ __device__ __forceinline__ bool conv_out_line(const ConvPairsParams &p, const in
 
 // One lane per (input, (kz, ky)): the sites of a line that fall into one word go out in
 // one atomic.  grid.y = KZ * KY, so that the lanes that repeat a site mostly run after the one that sets it
-// (in the order of xcd_block they run beside it: 25.6 against 18.0 us).  (One lane per (input, offset) with divisions in 64 bits: 18.4 us at 120 k voxels, 32.7 at
-// 300 k; the arithmetic was what bound it.)
+// (in the order of xcd_block they run beside it: 25.6 against 18.0 us).  (One lane per (input, offset) with
+// divisions in 64 bits: 18.4 us at 120 k voxels, 32.7 at 300 k; the arithmetic was what bound it.)
 __global__ __launch_bounds__(256) void conv_bits_sites_kernel(const ConvPairsParams p) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   const int zy = blockIdx.y;

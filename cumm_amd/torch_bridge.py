@@ -200,7 +200,6 @@ class SparseConvGeometry:
     All tables lie in one block from torch's caching allocator (a new cloud per iteration then
     allocates nothing from the driver); ``indices_fwd`` and the other tables are views of it."""
 
-    _TILES = (64, 128)      # positions per tile of the kernels that reduce masks
     _TABLES = ("indices_fwd", "indices_bwd", "mask_fwd", "order_fwd", "mask_bwd", "order_bwd", "indices_fwd_pos", "indices_bwd_pos")
 
     def __init__(self, coords: torch.Tensor, spatial_shape: Sequence[int], ksize=(3, 3, 3), stride=None,
@@ -219,7 +218,7 @@ class SparseConvGeometry:
         # launches - stays on the device: the sort leaves it in the library's table under the sorted
         # array's address and the launches look it up there; 0 = not given here)
         self.light_fwd = self.light_bwd = 0
-        self._reduced, self._reduced_streams = {}, {}
+        self._reduced, self._reduced_streams, self._written = {}, {}, set()
         self._launches = {}      # calls of the layers on this geometry, see _Launch
         self._tensors = {}
         lib, arr3 = _capi.lib(), ctypes.c_int32 * 3
@@ -299,8 +298,6 @@ class SparseConvGeometry:
         mask = [n_in] if words == 1 else [n_in, words]
         if not self.subm:
             spec += [("mask_bwd", mask, tv.uint32), ("order_bwd", [n_in], tv.int32)]
-        if words == 1:     # (in the block and not where the first forward pass runs: see reduced_mask)
-            spec += [("reduced_%d" % w, [max((n_out + w - 1) // w, 1)], tv.int32) for w in SparseConvGeometry._TILES]
         self._spec, at = {}, 0
         for name, dims, dtype in spec:
             self._spec[name] = (at, dims, dtype)
@@ -308,9 +305,14 @@ class SparseConvGeometry:
             for d in dims:
                 size *= d
             at += (size + 255) // 256 * 256
+        # the words of tiles of 64 and of 128 positions, rounded up to 256 bytes (see reduced_address)
+        reduced_64, reduced_128 = at, at + (n_out // 64 + 64) // 64 * 256
+        if words == 1:
+            at = reduced_128 + (n_out // 128 + 64) // 64 * 256
         self._block = _bytes(at, self._device)
         base = self._block.data_ptr()
         self._ptr = {name: base + v[0] for name, v in self._spec.items()}
+        self._reduced_at = {64: base + reduced_64, 128: base + reduced_128} if words == 1 else {}
         if self.subm:      # the forward masks serve the backward-input pass, bit-reversed in the kernel
             for name in ("mask", "order"):
                 self._spec[name + "_bwd"], self._ptr[name + "_bwd"] = self._spec[name + "_fwd"], self._ptr[name + "_fwd"]
@@ -350,30 +352,30 @@ class SparseConvGeometry:
             if stream != own:
                 self._reduced[width].record_stream(torch.cuda.current_stream())
 
-    def reduced_mask(self, width: int) -> torch.Tensor:
+    def reduced_address(self, width: int) -> int:
         """One word per run of ``width`` sorted output positions: the forward launch writes (all of) the
         OR of the run's masks here (its ``mask_output``), and backward-weight reads it.  The words of the
         kernels' tile heights lie in the block of the tables: memory that the first forward pass took from
         its own stream's pool could be in use there still when another stream writes it, and again while
         another stream reads it."""
+        self._written.add(width)
+        if width in self._reduced_at:
+            return self._reduced_at[width]
         buf = self._reduced.get(width)
         if buf is None:
-            tiles, place = max((self.n_out + width - 1) // width, 1), self._spec.get("reduced_%d" % width)
-            if place is not None:
-                buf = self._block[place[0]:place[0] + 4 * tiles].view(torch.int32)
-            else:
-                buf = torch.empty(tiles, dtype=torch.int32, device=self._device)
-                self._reduced_streams[width] = current_stream()
-            self._reduced[width] = buf
-        return buf
+            buf = torch.empty(max((self.n_out + width - 1) // width, 1), dtype=torch.int32, device=self._device)
+            self._reduced[width], self._reduced_streams[width] = buf, current_stream()
+        return buf.data_ptr()
 
     def reduced_mask_buffer(self, width: int) -> tv.Tensor:
-        """``reduced_mask`` as a tv tensor; zeros until a forward pass with tiles of that height has run."""
-        fresh = width not in self._reduced
-        buf = self.reduced_mask(width)
+        """Those words as a tv tensor; zeros until a forward pass with tiles of that height has run."""
+        fresh = width not in self._written
+        at, count = self.reduced_address(width), max((self.n_out + width - 1) // width, 1)
+        owner = self._reduced.get(width, self._block)
         if fresh:
-            buf.zero_()
-        return torch2tensor(buf).type_view(tv.uint32)
+            first = at - owner.data_ptr()
+            (owner[first:first + 4 * count] if owner is self._block else owner).zero_()
+        return tv.from_blob(at, [count], tv.uint32, self._device.index, keepalive=owner)
 
 
 class _SparseConvFunction(torch.autograd.Function):
@@ -483,7 +485,7 @@ def _forward_launch(g: SparseConvGeometry, key, roles, relu, stream) -> _Launch:
     known = _KINDS.get(kind)
     if known is not None and features.numel() and out.numel():
         launch = known.on(g.n_out, g.n_in, g.n_out, g._ptr["indices_fwd_pos"], g._ptr["mask_fwd"], g._ptr["order_fwd"],
-                          g.reduced_mask(known.tile_m).data_ptr() if g.words == 1 else None)
+                          g.reduced_address(known.tile_m) if g.words == 1 else None)
         g._launches[key] = launch
         return launch
     p = ConvParams(3, ConvOpType.Forward)
@@ -547,7 +549,7 @@ def _backward_weight_launch(g: SparseConvGeometry, key, features, weight, grad_w
     kind = _kind(g, key, n_pos, grad_out, features, grad_w)
     known = _KINDS.get(kind)
     if known is not None and features.numel() and grad_out.numel():
-        return known.on(n_pos, g.n_in, g.n_out, g._ptr["indices_fwd"], g.reduced_mask(tile_m).data_ptr(), g._ptr["order_fwd"],
+        return known.on(n_pos, g.n_in, g.n_out, g._ptr["indices_fwd"], g.reduced_address(tile_m), g._ptr["order_fwd"],
                         None), need
     p = ConvParams(3, ConvOpType.BackwardWeight)
     p.conv_algo_desp = desp

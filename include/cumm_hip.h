@@ -377,8 +377,9 @@ int cumm_hip_pair_lists(const int32_t *indices, int kv, int n, int32_t *pair_in,
  *   sorted_mask [n, words], argsort [n], by_position[k][pos] = indices[k][argsort[pos]] ([kv, n]),
  *   by_position_reversed[kv - 1 - k] = by_position[k] (NULL = not wanted: the backward table of a
  *   submanifold layer).
- * Positions come in ascending number of kernel offsets (one word) or grouped by the sides on which
- * their neighbours lie (several); equal masks lie together; the order repeats from run to run.  The
+ * Positions come in ascending number of kernel offsets (one word; equal masks lie together up to five
+ * offsets, above that masks of like rank mix) or grouped by the sides on which their neighbours lie
+ * (several); the order repeats from run to run.  The
  * launch hints of the sorted masks are left as cumm_hip_sort_by_mask_ordered leaves them.  Two radix
  * passes for all tables together, where cumm_hip_sort_by_mask_ordered, whose order is exact, takes four
  * for each.  workspace: cumm_hip_order_pairs_workspace bytes, 256-byte aligned. */

@@ -101,7 +101,7 @@ def _geometry(monkeypatch, tb, n=1000, stream=1):
     monkeypatch.setattr(torch.Tensor, "record_stream", lambda t, s: recorded.append((t.untyped_storage().data_ptr(), s)))
     g = object.__new__(tb.SparseConvGeometry)
     g._stream, g._device, g.subm, g.kv, g.words, g.n_in, g.n_out = stream, torch.device("cpu"), True, 27, 1, n, n
-    g.lists, g._reduced, g._reduced_streams, g._launches, g._tensors = None, {}, {}, {}, {}
+    g.lists, g._reduced, g._reduced_streams, g._written, g._launches, g._tensors = None, {}, {}, set(), {}, {}
     g._allocate()
     return g, recorded, now
 
@@ -114,32 +114,35 @@ def test_reduced_masks_belong_to_the_streams_that_use_them(monkeypatch):
         g, recorded, now = _geometry(monkeypatch, tb, n)
         now[0] = 2
         g.used_on(2)
-        words = {w: g.reduced_mask(w) for w in (64, 128, 32)}
+        at = {w: (g.reduced_address(w), 4 * max((n + w - 1) // w, 1)) for w in (64, 128, 32)}
         block = g._block.untyped_storage().data_ptr()
         assert recorded == [(block, 2)]
-        for w, t in words.items():
-            assert t.numel() == max((n + w - 1) // w, 1) and t.dtype == torch.int32
-            assert (t.untyped_storage().data_ptr() == block) == (w != 32)
-        spans = sorted((t.data_ptr(), t.data_ptr() + 4 * t.numel()) for w, t in words.items() if w != 32)
-        spans += [(g._ptr["order_fwd"], g._ptr["order_fwd"] + 4 * n)]
-        spans.sort()
-        assert all(a[1] <= b[0] for a, b in zip(spans, spans[1:])) and spans[-1][1] <= block + g._block.numel()
+        spans = sorted([(a, a + size) for w, (a, size) in at.items() if w != 32] + [(g._ptr["order_fwd"], g._ptr["order_fwd"] + 4 * n)])
+        assert block <= spans[0][0] and spans[-1][1] <= block + g._block.numel()
+        assert all(x[1] <= y[0] for x, y in zip(spans, spans[1:]))
+        assert not block <= at[32][0] < block + g._block.numel()
         now[0] = 1
         g.used_on(1)
-        assert recorded[1:] == [(words[32].untyped_storage().data_ptr(), 1)]
-        assert g.reduced_mask(64) is words[64]
+        assert recorded[1:] == [(at[32][0], 1)]
+        assert all(g.reduced_address(w) == a for w, (a, _) in at.items())
 
 
 def test_a_reduced_mask_that_no_pass_has_written_is_zero(monkeypatch):
+    import ctypes
     from cumm_amd import torch_bridge as tb
     g, _, _ = _geometry(monkeypatch, tb)
     g._block.fill_(0xA5)
+
+    def words(w):
+        t = g.reduced_mask_buffer(w)
+        assert t.dtype == tv.uint32 and t.shape == [(1000 + w - 1) // w] and t.byte_pointer() == g.reduced_address(w)
+        return (ctypes.c_uint32 * t.size).from_address(t.byte_pointer())
     for w in (64, 32):
-        g.reduced_mask_buffer(w)
-        assert not g.reduced_mask(w).any()
-    g.reduced_mask(64).fill_(7)
-    g.reduced_mask_buffer(64)
-    assert bool((g.reduced_mask(64) == 7).all())
+        assert not any(words(w))
+    g.reduced_address(128)      # (what a forward pass asks for, and fills)
+    for w in (64, 32, 128):
+        ctypes.memset(g.reduced_address(w), 7, 4)
+        assert words(w)[0] == 0x07070707
 
 
 def test_a_moved_call_refuses_tensors_on_another_device_than_the_tables(monkeypatch):
