@@ -201,6 +201,7 @@ class SparseConvGeometry:
     allocates nothing from the driver); ``indices_fwd`` and the other tables are views of it."""
 
     _TABLES = ("indices_fwd", "indices_bwd", "mask_fwd", "order_fwd", "mask_bwd", "order_bwd", "indices_fwd_pos", "indices_bwd_pos")
+    _lists = _list_block = None      # (several mask words only)
 
     def __init__(self, coords: torch.Tensor, spatial_shape: Sequence[int], ksize=(3, 3, 3), stride=None,
                  padding=(1, 1, 1), dilation=(1, 1, 1), batch_size: int = 1):
@@ -213,7 +214,6 @@ class SparseConvGeometry:
         self.n_in = n_in = int(coords.shape[0])
         self.kv = kv = int(ksize[0]) * int(ksize[1]) * int(ksize[2])
         self.words = words = (kv + 31) // 32
-        self.lists = None
         # (how far the light end of each sorted order reaches - the hint of the forward and backward-input
         # launches - stays on the device: the sort leaves it in the library's table under the sorted
         # array's address and the launches look it up there; 0 = not given here)
@@ -326,12 +326,19 @@ class SparseConvGeometry:
         ws = _bytes(need, self._device)
         _capi.check(lib.cumm_hip_pair_lists(self._ptr["indices_fwd"], kv, n, lists[0].data_ptr(), lists[1].data_ptr(),
                                             counts.data_ptr(), ws.data_ptr(), ws.numel(), self._stream))
-        handed = _HandedOut(lists)
-        pair_in, pair_out = (tv.from_blob(t.data_ptr(), [kv, n], tv.int32, self._device.index, keepalive=handed) for t in lists)
-        self.lists = pairs.DevicePairLists(pair_in, pair_out, counts.cpu().numpy())
         self._list_block = lists
+        self._lists = self._lists_over(lists, counts.cpu().numpy())
+
+    def _lists_over(self, keepalive, counts) -> pairs.DevicePairLists:
+        pair_in, pair_out = (tv.from_blob(t.data_ptr(), [self.kv, self.n_out], tv.int32, self._device.index, keepalive=keepalive)
+                             for t in self._list_block)
+        return pairs.DevicePairLists(pair_in, pair_out, counts)
 
     def __getattr__(self, name: str):
+        if name == "lists":      # (the passes take their own, whose streams are recorded)
+            own = self._lists
+            self.lists = None if own is None else self._lists_over(_HandedOut(self._list_block), own.counts)
+            return self.lists
         if name not in SparseConvGeometry._TABLES or "_spec" not in self.__dict__:
             raise AttributeError(name)
         t = self._tensors.get(name)
@@ -346,7 +353,7 @@ class SparseConvGeometry:
         if stream != self._stream:
             current = torch.cuda.current_stream()
             self._block.record_stream(current)
-            if self.lists is not None:
+            if self._lists is not None:
                 self._list_block.record_stream(current)
         for width, own in self._reduced_streams.items():
             if stream != own:
@@ -449,7 +456,7 @@ class _SparseConvFunction(torch.autograd.Function):
             key = ("wgrad_pairs", dtype, weight.shape)
             plan = g._launches.get(key)
             if plan is None:
-                plan = native.WeightPlan(torch2tensor(grad_out), torch2tensor(features), torch2tensor(grad_w), g.lists, stream)
+                plan = native.WeightPlan(torch2tensor(grad_out), torch2tensor(features), torch2tensor(grad_w), g._lists, stream)
                 plan.release()      # (every call brings its own tensors)
                 g._launches[key] = plan
             ws = _bytes(plan.workspace_bytes, grad_out.device)

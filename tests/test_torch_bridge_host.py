@@ -183,3 +183,36 @@ def test_tables_that_were_handed_out_go_back_when_the_device_has_finished(monkey
     del g
     gc.collect()
     assert waits == []
+
+
+def test_pair_lists_wait_only_where_they_were_handed_out(monkeypatch):
+    """The lists of a geometry with several mask words: the passes' own go back without a wait (their streams
+    are recorded), those that somebody took keep the memory until the device has finished."""
+    from cumm_amd import torch_bridge as tb
+    import gc
+    import weakref
+    waits = []
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    for taken in (True, False):
+        g, recorded, now = _geometry(monkeypatch, tb)
+        del g.lists
+        g._list_block = torch.zeros((2, 27, 1000), dtype=torch.int32)
+        g._lists = g._lists_over(g._list_block, torch.zeros(27, dtype=torch.int32).numpy())
+        block = weakref.ref(g._list_block)
+        monkeypatch.setattr(torch.cuda, "synchronize", lambda d: waits.append(block() is not None))
+        now[0] = 2
+        g.used_on(2)
+        assert [s for _, s in recorded] == [2, 2] and recorded[1][0] == g._list_block.data_ptr()
+        lists = g.lists if taken else None
+        if taken:
+            assert g.lists is lists and [t.byte_pointer() for t in lists[:2]] == [t.data_ptr() for t in g._list_block]
+        del g
+        gc.collect()
+        assert waits == [] and (block() is not None) == taken
+        del lists
+        gc.collect()
+        assert waits == ([True] if taken else []) and block() is None
+        del waits[:]
+    g, _, _ = _geometry(monkeypatch, tb)
+    del g.lists
+    assert g.lists is None
