@@ -167,11 +167,15 @@ def backward_input(dout: tv.Tensor, weight: tv.Tensor, dinp: tv.Tensor, lists, *
 class WeightPlan:
     """Backward-weight of all kernel offsets in one call of the library (``cumm_hip_wgrad_pairs``),
     validated once: run on the tensors it was made for, or through ``rebind`` on others of the same
-    shapes and types by address."""
+    shapes and types by address.
+
+    A run that is recorded into a graph does without a workspace of the plan's own - nothing may be
+    allocated then, and the graph may outlive the plan, whose workspace other calls get afterwards -
+    and makes one product per offset instead."""
 
     def __init__(self, dout, inp, dweight, lists, stream):
         self._tensors, self._lists, self._stream = (dout, inp, dweight), lists, stream
-        self._slots = None
+        self._slots, self._forms = None, _forms(dout, inp, dweight)
         lib = _capi.lib()
         kv, k_out, c_in = dweight.dim(1), dweight.dim(0), dweight.dim(2)
         self._fn = lib.cumm_hip_wgrad_pairs
@@ -195,6 +199,9 @@ class WeightPlan:
         """Run on other tensors of the same shapes (device addresses), on ``stream``.  Without a
         workspace (``workspace_bytes`` bytes) the plan's own is used: one run at a time then."""
         if workspace_ptr is None:
+            if _capi.lib().cumm_hip_stream_is_capturing(stream):
+                WeightSteps(*_views(self._forms, dout_ptr, inp_ptr, dweight_ptr), self._lists, stream)()
+                return
             slots = self._slots
             if slots is None or slots.stream != stream:
                 slots = self._slots = _Slots(_Slots._device(), stream, max(self.workspace_bytes, 16), id(self))
@@ -214,6 +221,15 @@ class WeightPlan:
         return self._pairs[3]
 
 
+def _forms(*tensors):
+    """What a tensor is beside its address."""
+    return [(list(t.shape), list(t.stride), t.dtype, t.device) for t in tensors]
+
+
+def _views(forms, *addresses):
+    return [tv.from_blob_strided(at, *form) for at, form in zip(addresses, forms)]
+
+
 def plan_backward_weight(dout: tv.Tensor, inp: tv.Tensor, dweight: tv.Tensor, lists, *, stream: int = 0):
     """Backward-weight as a reusable plan: dweight[:, k, :] of every kernel offset (zeros for an
     offset without pairs)."""
@@ -225,6 +241,8 @@ def plan_backward_weight(dout: tv.Tensor, inp: tv.Tensor, dweight: tv.Tensor, li
     _check_dtype(lists.pair_out, tv.int32, "pair_out")
     if not _in_one_call(dout, inp, dweight, lists):
         return WeightSteps(dout, inp, dweight, lists, stream)
+    if (np.asarray(lists.counts) <= 0).any() and not _capi.lib().cumm_hip_stream_is_capturing(stream):
+        WeightSteps.no_pair(inp.device)      # (for runs that are recorded)
     return WeightPlan(dout, inp, dweight, lists, stream)
 
 
@@ -237,14 +255,22 @@ def _in_one_call(dout, inp, dweight, lists) -> bool:
 
 class WeightSteps:
     """Backward-weight as one gathered product per kernel offset: rows with a stride of their own, more
-    offsets than one call takes.  The first run validates each product; runs after it, and ``rebind`` on
-    other tensors of the same shapes, go straight to the C entry points.  The products run one after the
-    other on one stream and share a workspace."""
+    offsets than one call takes, runs that are recorded into a graph.  The first run validates each
+    product; runs after it, and ``rebind`` on other tensors of the same shapes, go straight to the C entry
+    points.  The products run one after the other on one stream and share a workspace."""
 
     _NO_PAIR = {}
 
+    @classmethod
+    def no_pair(cls, dev: int) -> tv.Tensor:
+        """The pairs of an offset without any: absent rows, whose product is zero."""
+        if dev not in cls._NO_PAIR:
+            cls._NO_PAIR[dev] = tv.from_numpy(np.full(32, -1, np.int32)).cuda()
+        return cls._NO_PAIR[dev]
+
     def __init__(self, dout, inp, dweight, lists, stream):
-        self.steps, self._tensors, self._stream = [], (dout, inp, dweight), stream
+        self.steps, self._tensors, self._lists, self._stream = [], (dout, inp, dweight), lists, stream
+        self._forms, self._launches, self._ran = _forms(dout, inp, dweight), dweight.dim(1), False
         self._blocks, self._slots, self._lock = None, None, threading.Lock()
         self._workspace_bytes = 0
         for k in range(dweight.dim(1)):
@@ -256,10 +282,7 @@ class WeightSteps:
                 p.a_inds = lists.pair_out.select(0, k).slice_first_axis(0, cnt)
                 p.b_inds = lists.pair_in.select(0, k).slice_first_axis(0, cnt)
             else:      # one step of absent rows writes the zeros
-                dev = inp.device
-                if dev not in self._NO_PAIR:
-                    self._NO_PAIR[dev] = tv.from_numpy(np.full(32, -1, np.int32)).cuda()
-                p.a_inds = p.b_inds = self._NO_PAIR[dev]
+                p.a_inds = p.b_inds = self.no_pair(inp.device)
             p.stream = stream
             self._workspace_bytes = max(self._workspace_bytes, self._optional(p))
             self.steps.append(p)
@@ -279,7 +302,9 @@ class WeightSteps:
                 p.workspace = workspace
 
     def _share(self, stream: int) -> None:
-        if self._workspace_bytes > 0 and (self._slots is None or self._slots.stream != stream):
+        # (the products of a recorded run use none)
+        if (self._workspace_bytes > 0 and (self._slots is None or self._slots.stream != stream) and
+                not _capi.lib().cumm_hip_stream_is_capturing(stream)):
             self._slots = _Slots(_Slots._device(), stream, self._workspace_bytes, None)
 
     def __call__(self) -> None:
@@ -293,6 +318,7 @@ class WeightSteps:
             for p in self.steps:
                 p.__dict__["_slots"] = self._slots
                 GemmMainUnitTest.matmul2(p)
+            self._ran = True
             blocks = []
             base = self._tensors[2].byte_pointer()
             for p in self.steps:
@@ -318,20 +344,25 @@ class WeightSteps:
     def rebind(self, dout_ptr: int, inp_ptr: int, dweight_ptr: int, stream: int) -> None:
         """Run on other tensors of the same shapes and strides (device addresses), on ``stream``."""
         with self._lock:
-            if self._blocks is None:
+            if not self._ran:
                 raise RuntimeError("the plan has not run yet")
-            self._run(dout_ptr, inp_ptr, dweight_ptr, stream)
+            if self._blocks is None:      # (recorded so far, which validates nothing for good)
+                again = WeightSteps(*_views(self._forms, dout_ptr, inp_ptr, dweight_ptr), self._lists, stream)
+                again()
+                self._blocks, self._slots = again._blocks, again._slots
+            else:
+                self._run(dout_ptr, inp_ptr, dweight_ptr, stream)
 
     def release(self) -> None:
         """Forget the tensors of the first run (a caller that goes on through ``rebind`` with its own): the
         argument blocks hold addresses only, the pair lists belong to their owner."""
-        if self._blocks is None:
+        if not self._ran:
             raise RuntimeError("the plan has not run yet")
-        self._launches, self.steps, self._tensors = self.launches, [], None
+        self.steps, self._tensors = [], None
 
     @property
     def launches(self) -> int:
-        return len(self.steps) if self._tensors is not None else self._launches
+        return self._launches
 
 
 def backward_weight(dout: tv.Tensor, inp: tv.Tensor, dweight: tv.Tensor, lists, *, split_k_slices: int = 1,

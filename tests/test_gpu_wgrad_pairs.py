@@ -151,6 +151,42 @@ def test_shuffle_ab_recorded_into_a_graph(first):
     del keep
 
 
+@pytest.mark.parametrize("first", ["recorded", "eager"])
+def test_all_offsets_recorded_into_a_graph(first):
+    """A graph that outlives the plan it was recorded from, whose own workspace others use afterwards."""
+    from types import SimpleNamespace
+    from cumm_amd.conv import native
+    print("case all offsets graph", first, flush=True)
+    rng = np.random.default_rng(8)
+    rows, k_out, c_in, most, counts = 600, 64, 72, 300, np.array([300, 0, 257], np.int32)
+    dout, inp = _data(rng, (rows, k_out), "f16"), _data(rng, (rows, c_in), "f16")
+    po, pi = (rng.integers(0, rows, size=(3, most)).astype(np.int32) for _ in range(2))
+    lists = SimpleNamespace(pair_in=H.dev(pi, "i32"), pair_out=H.dev(po, "i32"), counts=counts)
+    operands = (H.dev(dout, "f16"), H.dev(inp, "f16"), tv.zeros([k_out, 3, c_in], tv.float16, 0))
+    ref = np.stack([H.as_f32(dout, "f16")[po[r, :n]].T @ H.as_f32(inp, "f16")[pi[r, :n]] for r, n in enumerate(counts)], axis=1)
+    few, _ = _shuffle_ab(np.random.default_rng(6), 2000, 64, 72, 100)      # (loads the kernel that the graph will hold)
+    GemmMainUnitTest.matmul2(few)
+    side = torch.cuda.Stream()
+    plan = native.plan_backward_weight(*operands, lists, stream=side.cuda_stream)
+    if first == "eager":
+        plan()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        plan()
+    del plan
+    for _ in range(3):
+        other, want = _shuffle_ab(rng, 2000, 64, 72, 1000)
+        operands[2].zero_()
+        torch.cuda.synchronize()
+        other.stream = side.cuda_stream
+        graph.replay()
+        GemmMainUnitTest.matmul2(other)
+        torch.cuda.synchronize()
+        for got, r in ((operands[2], ref), (other.c, want)):
+            assert np.abs(H.as_f32(H.host(got), "f16") - r).max() <= TOL["f16"] * np.abs(r).max()
+
+
 def _shuffle_ab(rng, rows, m, n, pairs):
     a, b = _data(rng, (rows, m), "f16"), _data(rng, (rows, n), "f16")
     ai, bi = (rng.integers(0, rows, size=pairs).astype(np.int32) for _ in range(2))

@@ -27,6 +27,7 @@ def calls(monkeypatch):
                 return 0
             return entry
     monkeypatch.setattr(_capi, "_lib", Library())
+    monkeypatch.setattr(native.WeightSteps, "_NO_PAIR", {0: tv.from_blob(0x7D0000000000, [32], tv.int32, 0)})
     return made
 
 
@@ -142,6 +143,82 @@ def test_slices_are_what_the_caller_asks_for_where_no_workspace_spreads_the_pair
     del products[:]
     native.backward_weight(*_wide_operands(2, [40000, 100]), split_k_slices=4)
     assert [(a.split_k_slices, name) for name, a, _ in products] == [(1, "cumm_hip_gemm_in_workspace"), (1, "cumm_hip_gemm")]
+
+
+@pytest.fixture
+def recording(products, monkeypatch):
+    """``products``, and whether the streams are recorded: nothing may be allocated then."""
+    from cumm_amd.gemm import main
+    recorded, plain = [1], _capi.lib()
+
+    class Library:
+        def __getattr__(self, name):
+            if name == "cumm_hip_stream_is_capturing":
+                return lambda stream: recorded[0]
+            if name == "cumm_hip_wgrad_pairs":
+                return lambda *args: products.append((name, args[-3], args[-1])) or 0
+            return getattr(plain, name)
+
+    def empty(shape, dtype, device):
+        assert not recorded[0]
+        return tv.Tensor(shape, dtype)
+    monkeypatch.setattr(_capi, "_lib", Library())
+    monkeypatch.setattr(main, "empty", empty)
+    return recorded
+
+
+def test_a_recorded_run_has_no_workspace_but_the_callers(products, recording):
+    """The graph may outlive the plan, whose workspace others get then."""
+    counts = [5, 0, 96]
+    operands = _operands(3, counts)
+    dout, inp, dweight, lists = operands
+    workspace = tv.from_blob(0x7E0000000000, [1 << 28], tv.uint8, 0)
+
+    def single_products(at, stream):
+        assert [(name, a.k) for name, a, _ in products] == [("cumm_hip_gemm", k) for k in (5, 32, 96)]
+        for r, (_, a, s) in enumerate(products):
+            assert (a.ptr_A, a.ptr_B, a.ptr_C, a.workspace, s) == (at[0], at[1], at[2] + r * C * 2, None, stream)
+        assert products[2][1].indiceA == lists.pair_out.byte_pointer() + 2 * MOST * 4
+        del products[:]
+    here = [t.byte_pointer() for t in (dout, inp, dweight)]
+    native.backward_weight(*operands, stream=4)
+    single_products(here, 4)
+    native.backward_weight(*operands, stream=4, workspace=workspace)
+    assert products == [("cumm_hip_wgrad_pairs", 0x7E0000000000, 4)]
+    del products[:]
+    plan = native.plan_backward_weight(*operands, stream=4)
+    for recorded in (0, 1, 0):
+        recording[0] = recorded
+        for run, at, stream in ((plan, here, 4), (lambda: plan.rebind(1 << 40, 2 << 40, 3 << 40, 5), [i << 40 for i in (1, 2, 3)], 5)):
+            run()
+            if recorded:
+                single_products(at, stream)
+            else:
+                assert [(name, s) for name, _, s in products] == [("cumm_hip_wgrad_pairs", stream)]
+                del products[:]
+
+
+def test_a_plan_of_single_products_that_was_recorded_first(products, recording):
+    counts = [5000, 0, 300]
+    plan = native.plan_backward_weight(*_wide_operands(3, counts), stream=3)
+    plan()
+    assert [(name, a.workspace) for name, a, _ in products] == [("cumm_hip_gemm", None)] * 3
+    first = products[:]
+    plan.release()
+    assert plan.launches == 3
+    base = 0x600000000000
+    for recorded in (1, 0, 0):
+        recording[0] = recorded
+        del products[:]
+        plan.rebind(base, base + (1 << 30), base + (2 << 30), 9)
+        want = ["cumm_hip_gemm_in_workspace" if k > 32 and not recorded else "cumm_hip_gemm" for k in (5000, 32, 300)]
+        assert [name for name, _, _ in products] == want
+        for (name, a, stream), (_, was, _) in zip(products, first):
+            assert (a.ptr_A, a.ptr_B, stream, a.k) == (base, base + (1 << 30), 9, was.k) and bool(a.workspace) == ("in_work" in name)
+            assert a.ptr_C == base + (2 << 30) + (was.ptr_C - 0x7F4000000000) and a.stride_A == was.stride_A == K + 8
+    # on a stream of its own, recorded: nothing is allocated for it, and the entry point uses no workspace
+    recording[0] = 1
+    plan.rebind(base, base + (1 << 30), base + (2 << 30), 10)
 
 
 def test_lists_of_2_to_the_29_pairs_and_more_are_refused():
