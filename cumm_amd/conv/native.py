@@ -179,13 +179,12 @@ class WeightPlan:
         lib = _capi.lib()
         kv, k_out, c_in = dweight.dim(1), dweight.dim(0), dweight.dim(2)
         self._fn = lib.cumm_hip_wgrad_pairs
-        # (a count beyond its list ends with the list, as a slice of it does)
-        self._counts = np.ascontiguousarray(np.clip(lists.counts, 0, lists.pair_in.dim(1)), np.int32)
+        self._counts = _counts(lists)
         counts = self._counts.ctypes.data
         self._pairs = (lists.pair_out.byte_pointer(), lists.pair_in.byte_pointer(), counts, kv, lists.pair_in.dim(1))
         self._sizes = (dout.dim(0), inp.dim(0), k_out, c_in, dweight.dtype)
         #: bytes of workspace that a run needs
-        self.workspace_bytes = int(lib.cumm_hip_wgrad_pairs_workspace(counts, kv, k_out, c_in))
+        self.workspace_bytes = _wgrad_workspace(self._counts, dweight)
         if self.workspace_bytes < 0:
             raise RuntimeError("at most 128 kernel offsets, channel counts multiples of 8")
 
@@ -247,10 +246,20 @@ def plan_backward_weight(dout: tv.Tensor, inp: tv.Tensor, dweight: tv.Tensor, li
 
 
 def _in_one_call(dout, inp, dweight, lists) -> bool:
-    """What ``cumm_hip_wgrad_pairs`` takes: whole tensors at 16-byte addresses, up to 128 offsets."""
+    """What ``cumm_hip_wgrad_pairs`` takes: whole tensors at 16-byte addresses, up to 128 offsets - and lists
+    and channels below its limits (-1 for those above), which single products do not have."""
     return (all(t.is_contiguous() and t.byte_pointer() % 16 == 0 for t in (dout, inp, dweight)) and
             lists.pair_in.is_contiguous() and lists.pair_out.is_contiguous() and lists.pair_in.shape == lists.pair_out.shape and
-            dweight.dim(1) <= 128)
+            dweight.dim(1) <= 128 and _wgrad_workspace(_counts(lists), dweight) >= 0)
+
+
+def _counts(lists) -> np.ndarray:
+    """(A count beyond its list ends with the list, as a slice of it does.)"""
+    return np.ascontiguousarray(np.clip(lists.counts, 0, lists.pair_in.dim(1)), np.int32)
+
+
+def _wgrad_workspace(counts: np.ndarray, dweight) -> int:
+    return int(_capi.lib().cumm_hip_wgrad_pairs_workspace(counts.ctypes.data, dweight.dim(1), dweight.dim(0), dweight.dim(2)))
 
 
 class WeightSteps:

@@ -232,3 +232,17 @@ def test_lists_of_2_to_the_29_pairs_and_more_are_refused():
             at = 1 << 20      # (never read: the counts are refused first)
             assert lib.cumm_hip_wgrad_pairs(at, at, at, at, at, c.ctypes.data, len(counts), 1 << 31, 10, 10, 64, 64, tv.float16, at,
                                             1 << 40, None) == _capi.EINVAL
+
+
+def test_what_one_call_does_not_take_goes_out_as_single_products(products):
+    """4096 blocks of 64 x 64 channels and more; the plan takes a block less in one call."""
+    for k_out, c_in, single in ((4096, 4096, True), (4096, 4032, False)):
+        blob = lambda at, shape, dtype: tv.from_blob(at << 32, shape, dtype, 0)
+        lists = SimpleNamespace(pair_in=blob(0x7F00, [2, 100], tv.int32), pair_out=blob(0x7F01, [2, 100], tv.int32),
+                                counts=np.array([100, 7]))
+        operands = (blob(0x7F02, [ROWS, k_out], tv.float16), blob(0x7F03, [ROWS, c_in], tv.float16),
+                    blob(0x7F04, [k_out, 2, c_in], tv.float16), lists)
+        assert isinstance(native.plan_backward_weight(*operands), native.WeightSteps) == single
+        if single:
+            native.backward_weight(*operands)
+            assert [(name, a.k) for name, a, _ in products] == [("cumm_hip_gemm", 100), ("cumm_hip_gemm", 7)]
