@@ -121,8 +121,9 @@ static hipError_t launch_dense_ring_layout(const TileGemmParams &p, hipStream_t 
 
 // Contractions of a step or two have nothing to stream: half a step always, and up to a step and a half with
 // several tiles per CU, where what counts is how many workgroups start and store at once, the
-// register-staged kernel in 64 x 64 tiles is the faster one (536 x 928 x 16 3.7 us and 4.2; 3000^2 x 8 to 64: 8.6 - 11.5 us against 13.0 and more; 1352 x 3720 x 72 8.7 and 9.9; 4096^2 x 64 16.1 -
-// 19.2 and 17.7; with k = 128 13.8 and 13.6 at 3000^2).
+// register-staged kernel in 64 x 64 tiles is the faster one (536 x 928 x 16 3.7 us and 4.2; 3000^2 x 8 to 64:
+// 8.6 - 11.5 us against 13.0 and more; 1352 x 3720 x 72 8.7 and 9.9; 4096^2 x 64 16.1 - 19.2 and 17.7; with
+// k = 128 13.8 and 13.6 at 3000^2).
 inline bool dense_ring_streams(const TileGemmParams &p) {
   const int n = tiles_per_cu(p, 64, 64);
   return p.k > (n >= 4 ? 96 : 32);

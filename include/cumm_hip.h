@@ -398,8 +398,8 @@ int cumm_hip_order_pairs(const CummHipOrderSide *sides, int n_sides, const int32
  *   dw[:, r, :] = sum over i < counts[r] of dout[pair_out[r][i]]^T inp[pair_in[r][i]]
  * dw [K, lists, C], dout [rows_out, K], inp [rows_in, C] (f16 / bf16, fp32 sums in a fixed order, rounded
  * once); pair_out / pair_in [lists, list_stride] on the device, counts [lists] on the HOST; at most 128
- * lists of fewer than 2^29 pairs; an offset without pairs gets zeros; row numbers outside the tensors contribute nothing.  What
- * a caller of the reference does with one ShuffleAB matmul2 per offset
+ * lists of fewer than 2^29 pairs; an offset without pairs gets zeros; row numbers outside the tensors
+ * contribute nothing.  What a caller of the reference does with one ShuffleAB matmul2 per offset
  * (cumm/conv/main_real_spconv.py:375-403).  workspace: cumm_hip_wgrad_pairs_workspace bytes (-1 for
  * arguments that are not taken), 16-byte aligned. */
 int64_t cumm_hip_wgrad_pairs_workspace(const int32_t *counts, int lists, int K, int C);
