@@ -2,7 +2,7 @@
 
 TEST INFRASTRUCTURE ONLY.  Nothing in the shipped package imports this
 directory; it is used by tests/, by ``__graft_entry__.smoke()`` and by the
-``cpu_baseline`` leg of ``bench.py`` as the checker / the timed CPU baseline.
+``cpu_baseline`` leg of ``bench.py`` as the expected result / the timed CPU baseline.
 
 Every function restates, in numpy (plus a few lines of C for the float
 operations whose rounding must be fixed), what the reference computes; the
