@@ -5,7 +5,8 @@
 // on the global side).
 //
 // What differs from tilegemm.h, and why:
-//   * the wave tile (RBW x NBW blocks of 16 x 16) and the step depth are template parameters;
+//   * the wave tile (RBW x NBW blocks of 16 x 16), the step depth and the number of wave groups that share
+//     a tile's steps are template parameters;
 //     per k-step of 32 a wave reads (RBW + NBW) KB of fragments for RBW*NBW MFMAs, so larger wave
 //     tiles need fewer LDS bytes per MFMA (the chip lowers its clock under MFMA load, what
 //     counts is work per MFMA, not only cycles);
@@ -87,9 +88,10 @@ struct DenseOperand {
     }
   }
 
-  // fragments of the SLAB_BLOCKS blocks of slab `slab`, step slice ks
+  // fragments of the SLAB_BLOCKS blocks of slab `slab`, step slice ks (counted from slice `first`, which a
+  // transposed operand gets with the base address)
   template <int N>
-  __device__ __forceinline__ void offsets(int lane, int slab, int (&rd)[N]) const {
+  __device__ __forceinline__ void offsets(int lane, int slab, int (&rd)[N], int first = 0) const {
     const int l16 = lane & 15, q = lane >> 4;
     if constexpr (TR) {
       static_assert(N == SLAB_BLOCKS, "a read offset per block");
@@ -100,10 +102,10 @@ struct DenseOperand {
         rd[b] = e * (ROWS * 2) + (((col >> 3) ^ swap_tr(e)) * 16) + (col & 7) * 2;
       }
     } else {
-      static_assert(N == KS, "a read offset per step slice");
+      static_assert(N <= KS, "a read offset per step slice");
 #pragma unroll
       for (int s = 0; s < N; ++s)
-        rd[s] = (slab * (SLAB_BLOCKS * 16) * LPR + l16 * LPR + ((s * 4 + q) ^ swap_kc(l16))) * 16;
+        rd[s] = (slab * (SLAB_BLOCKS * 16) * LPR + l16 * LPR + (((first + s) * 4 + q) ^ swap_kc(l16))) * 16;
     }
   }
   template <int N>
@@ -189,14 +191,21 @@ __device__ __forceinline__ void dense_epilogue(const TileGemmParams &p, const ty
   }
 }
 
-template <class T, int WM, int WN, int RBW, int NBW, int KS, int NS, bool XT, bool YT>
-__global__ __launch_bounds__(WM *WN * 64) void densegemm_lds_kernel(const TileGemmParams p, int tiles_m, int tiles_n) {
+// The waves of a workgroup are WM x WN wave tiles, times WK groups that share them: group g takes the slices
+// g KS / WK .. of a step's KS slices of 32 k, and the groups' sums are added up in LDS at the end.  Eight
+// waves per workgroup throughout: with four, one per SIMD where a CU has a single workgroup, a step is the
+// chain barrier - fragment reads - products of one wave (more stages do not shorten it: 2000 x 776 x 1160
+// bf16 14.5 us with three, 15.5 with six); a second wave per SIMD reads while the first multiplies.  Over
+// 290 random products of 64 .. 4096 the time is 0.92 of that with four waves: 1024^3 nt 8.8 -> 7.5 us,
+// 2000 x 776 x 1160 nn 14.5 -> 11.9, 2048^3 tn 28.4 -> 23.6, 1344 x 3328 x 880 tn 22.1 -> 18.0.
+template <class T, int WM, int WN, int WK, int RBW, int NBW, int KS, int NS, bool XT, bool YT>
+__global__ __launch_bounds__(WM *WN *WK * 64) void densegemm_lds_kernel(const TileGemmParams p, int tiles_m, int tiles_n) {
   using E = Elem<T>;
   using AccV = typename E::AccV;
   constexpr int TM = WM * RBW * 16;
   constexpr int TN = WN * NBW * 16;
-  using OpY = DenseOperand<TM, KS, WM * WN, YT, RBW, false>;
-  using OpX = DenseOperand<TN, KS, WM * WN, XT, NBW, !XT>;
+  using OpY = DenseOperand<TM, KS, WM * WN * WK, YT, RBW, false>;
+  using OpX = DenseOperand<TN, KS, WM * WN * WK, XT, NBW, !XT>;
   constexpr int STAGE = (OpY::VECS + OpX::VECS) * 16;
   constexpr int L = NS - 1;                // steps the loads run ahead
   constexpr int WAIT_STEP = (L - 1) * (OpY::IP + OpX::IP);   // loads issued after those of step s when it starts
@@ -209,7 +218,8 @@ __global__ __launch_bounds__(WM *WN * 64) void densegemm_lds_kernel(const TileGe
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / WN, wn = wave % WN;
+  const int wk = wave / (WM * WN), wm = wave / WN % WM, wn = wave % WN;
+  constexpr int KW = KS / WK;
   int tile_m, tile_n;
   dense_tile(tiles_m, tiles_n, &tile_m, &tile_n);
   const int m0 = tile_m * TM, n0 = tile_n * TN;
@@ -221,9 +231,9 @@ __global__ __launch_bounds__(WM *WN * 64) void densegemm_lds_kernel(const TileGe
   const uint32_t y_bytes = (uint32_t)(((int64_t)((YT ? p.k : p.m) - 1) * p.ldy + (YT ? p.m : p.k)) * 2);
   const uint32_t x_bytes = (uint32_t)(((int64_t)((XT ? p.k : p.n) - 1) * p.ldx + (XT ? p.n : p.k)) * 2);
   const int steps = (p.k + BK - 1) / BK;
-  int y_rd[YT ? RBW : KS], x_rd[XT ? NBW : KS];
-  y.offsets(lane, wm, y_rd);
-  x.offsets(lane, wn, x_rd);
+  int y_rd[YT ? RBW : KW], x_rd[XT ? NBW : KW];
+  y.offsets(lane, wm, y_rd, wk * KW);
+  x.offsets(lane, wn, x_rd, wk * KW);
 
   AccV acc[RBW][NBW];
 #pragma unroll
@@ -249,20 +259,20 @@ __global__ __launch_bounds__(WM *WN * 64) void densegemm_lds_kernel(const TileGe
     wait_vmcnt<WAIT_STEP>();
     lds_barrier();
     const char *st = ring + cs * STAGE;
-    v4i yf[RBW][KS], xf[NBW][KS];
+    v4i yf[RBW][KW], xf[NBW][KW];
 #pragma unroll
     for (int nb = 0; nb < NBW; ++nb)
 #pragma unroll
-      for (int k = 0; k < KS; ++k) xf[nb][k] = OpX::fragment(st + OpY::VECS * 16, x_rd, k, nb);
+      for (int k = 0; k < KW; ++k) xf[nb][k] = OpX::fragment(st + OpY::VECS * 16 + (XT ? wk * KW * 32 * TN * 2 : 0), x_rd, k, nb);
 #pragma unroll
     for (int rb = 0; rb < RBW; ++rb)
 #pragma unroll
-      for (int k = 0; k < KS; ++k) yf[rb][k] = OpY::fragment(st, y_rd, k, rb);
+      for (int k = 0; k < KW; ++k) yf[rb][k] = OpY::fragment(st + (YT ? wk * KW * 32 * TM * 2 : 0), y_rd, k, rb);
     issue(s + L, ls);
     cs = cs + 1 == NS ? 0 : cs + 1;
     ls = ls + 1 == NS ? 0 : ls + 1;
 #pragma unroll
-    for (int k = 0; k < KS; ++k)
+    for (int k = 0; k < KW; ++k)
 #pragma unroll
       for (int rb = 0; rb < RBW; ++rb)
 #pragma unroll
@@ -270,7 +280,33 @@ __global__ __launch_bounds__(WM *WN * 64) void densegemm_lds_kernel(const TileGe
   }
   wait_vmcnt<0>();
 
-  dense_epilogue<E, RBW, NBW, XT, false>(p, acc, m0 + wm * (RBW * 16), n0 + wn * (NBW * 16), lane);
+  if constexpr (WK == 1) {
+    dense_epilogue<E, RBW, NBW, XT, false>(p, acc, m0 + wm * (RBW * 16), n0 + wn * (NBW * 16), lane);
+  } else {
+    // each group finishes its share of the row blocks: it adds up all groups' sums of them, in group order
+    constexpr int RO = RBW / WK;
+    static_assert(RBW % WK == 0 && NS * STAGE >= WM * WN * WK * RBW * NBW * 1024, "the ring holds every group's sums");
+    AccV own[RO][NBW];
+    __builtin_amdgcn_s_waitcnt(0xC07F);     // lgkmcnt(0): this wave has read its last stage,
+    lds_barrier();                          // and so has every other
+    v4f *park = reinterpret_cast<v4f *>(ring);   // [group][wave of the group][rb][nb][lane]
+    const int wg = wave % (WM * WN);
+#pragma unroll
+    for (int rb = 0; rb < RBW; ++rb)
+#pragma unroll
+      for (int nb = 0; nb < NBW; ++nb) park[(((wk * (WM * WN) + wg) * RBW + rb) * NBW + nb) * 64 + lane] = acc[rb][nb];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RO; ++r)
+#pragma unroll
+      for (int nb = 0; nb < NBW; ++nb) {
+        AccV t = park[((wg * RBW + wk * RO + r) * NBW + nb) * 64 + lane];
+#pragma unroll
+        for (int g = 1; g < WK; ++g) t += park[(((g * (WM * WN) + wg) * RBW + wk * RO + r) * NBW + nb) * 64 + lane];
+        own[r][nb] = t;
+      }
+    dense_epilogue<E, RO, NBW, XT, false>(p, own, m0 + wm * (RBW * 16) + wk * RO * 16, n0 + wn * (NBW * 16), lane);
+  }
 }
 
 // The large tile, pipelined through registers: while the MFMAs of step s run on one set of fragments, the

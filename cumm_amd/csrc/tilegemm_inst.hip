@@ -1,4 +1,6 @@
 // Instantiations of the LDS-tiled GEMM for one element type (selected with -DCUMM_ELEM=...).
+#include <algorithm>
+
 #include "launch.h"
 #include "densegemm_lds.h"
 
@@ -31,14 +33,15 @@ static hipError_t launch_xy(bool xk, bool yk, const TileGemmParams &p, dim3 grid
 
 // Plain GEMM of two-byte elements in every layout, shapes with 16-byte pieces along each operand's and
 // the result's contiguous dimension: the LDS-ring kernels.  (One fp32 sum over k per element whatever
-// the tile - in eight parts, added in order, for the kernel that splits k over its waves.)
-template <class T, int WM, int WN, int RBW, int NBW, int KS, int NS, bool XT, bool YT>
+// the tile - in two parts where two groups of waves share it, in eight, added in order, for the kernel that
+// splits k over its waves.)
+template <class T, int WM, int WN, int WK, int RBW, int NBW, int KS, int NS, bool XT, bool YT>
 static hipError_t launch_dense_ring_as(const TileGemmParams &p, hipStream_t s) {
   constexpr int TM = WM * RBW * 16, TN = WN * NBW * 16;
-  if (!counted_waits_hold<densegemm_lds_kernel<T, WM, WN, RBW, NBW, KS, NS, XT, YT>>()) return hipErrorNotSupported;
+  if (!counted_waits_hold<densegemm_lds_kernel<T, WM, WN, WK, RBW, NBW, KS, NS, XT, YT>>()) return hipErrorNotSupported;
   const int tiles_m = (p.m + TM - 1) / TM, tiles_n = (p.n + TN - 1) / TN;
-  hipLaunchKernelGGL((densegemm_lds_kernel<T, WM, WN, RBW, NBW, KS, NS, XT, YT>), dim3((unsigned)(tiles_m * tiles_n)),
-                     dim3(WM * WN * 64), 0, s, p, tiles_m, tiles_n);
+  hipLaunchKernelGGL((densegemm_lds_kernel<T, WM, WN, WK, RBW, NBW, KS, NS, XT, YT>), dim3((unsigned)(tiles_m * tiles_n)),
+                     dim3(WM * WN * WK * 64), 0, s, p, tiles_m, tiles_n);
   return hipGetLastError();
 }
 
@@ -52,34 +55,32 @@ static hipError_t launch_dense_pipe(const TileGemmParams &p, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Which tile: the least estimated time, from measurements of f16 products on the 256 CUs that the figures are
-// for (us; n = tiles per CU, rounded up; k in elements; the larger of two lines where there are two: the
-// first is what a tile takes beside its steps, most of it its stores, the second the fetches of long
-// contractions, with a second figure for rows that are no whole number of 128-byte lines, whose fetches
-// touch a line more each):
-//   64 x 64 x 64, 2 x 2 waves, three stages   n = 1: 3.6 + 0.0039 k;  else
-//                                             2.6 + n (0.95 + 0.0026 k), from n = 8 on 1.05;
-//                                             2.6 + n (0.21 + 0.0033 / 0.0045 k)
-//                                             (1024^3 8.1; 2048^3 28; 3000^3 152; 3000^2 x 128 13.7)
-//   the same with k split over eight waves    n = 1 only: up to 32 tiles 3.8 + 0.0018 k (256 x 256 x 4096: 11.2
-//                                             against 15.8); more tiles of whole lines 4.3 + 0.0018 k while
-//                                             the tiles' rows fit the L2s (tiles * k up to 160 k: 512 x 320 x
-//                                             4096 11.8 - 15 against 18.7 - 20; 1024 x 512 x 1024 6.4 against
-//                                             7.7), beyond that 3.6 + 0.0038 k with an operand contiguous
-//                                             along its rows (1024^2 x 4096: nn 18.8 against 21.0, nt 21.6
-//                                             against 20.8).  Not for broken lines: 1344 x 440 x 2080
-//                                             nn 14.4 against 12.4
-//   128 x 64 x 64, three stages               n = 1: 5.8;  5.0 + 0.006 k;  else p = n / 2 rounded up:
-//                                             2.0 + p (4.4 + 0.008 k), from p = 3 on 0.0095;  5.0 + 0.0105 / 0.0135 p k
-//                                             (1536 x 1536 x 4096 38 against 40; 2048^3 25; 2048^2 x 256 8.7)
-//   128 x 128 x 64, two stages                n = 1: 9.0 + 0.0095 k;  5.0 + 0.0138 k;  else p = n / 2 rounded up:
-//                                             2.5 + p (8.0 + 0.0125 k);  5.0 + 0.0172 p k
-//                                             (2504^3 50 against 73; 2048 x 4096^2 73 against 96)
-//   256 x 256 x 32, 2 x 4 waves, four stages  2.0 + n (14.8 + 0.0235 k), up to k = 384 with result rows that are
-//                                             no whole lines, which it stores past the caches, 20.0;
-//                                             8.5 + 0.0255 n k
-//                                             (4096^3 120; 3000^3 85 against 104; 4096^2 x 256 21.5 against 27;
-//                                             tn 5768 x 2456 x 192 28 against 23)
+// Which tile: the least estimated time, fitted to 290 random products of 64 .. 4096 in bf16 on the 256 CUs
+// that the figures are for (us; n = tiles per CU, rounded up; k in elements; where there are two figures,
+// the second is for rows that are no whole number of 128-byte lines, whose fetches touch a line more each).
+// What it picks is 1.3 % slower than the fastest of the seven on average.
+//   64 x 64 x 64, 2 x 2 x 2 waves, three stages   up to 32 tiles 3.7 + 0.0036 k;  n = 1: 3.7 + 0.0040 /
+//                                              0.0046 k;  n = 2: 4.9 + 0.0063 / 0.0076 k;  else 2.4 + n (1.12 + 0.0031 /
+//                                              0.0040 k)              (3000 x 1000 x 504 11.3)
+//   64 x 64 x 128, four stages                 n = 1 only: up to 32 tiles 4.1 + 0.0026 / 0.0030 k, else 4.2 + 0.0030 /
+//                                              0.0038 k               (1024^3 7.5 against 8.0; 424 x 656 x 2992
+//                                              15.6 against 18.7; two tiles per CU 1.3 times as long)
+//   64 x 64, k split over eight waves          up to 32 tiles 4.2 + 0.0020 k, with broken lines and tiles * k above
+//                                              40 k 0.0032 k (128 x 192 x 3008 9.7 against 12.2; 96 x 80 x 3344,
+//                                              broken, 10.2 against 12.8; 920 x 96 x 3816, broken, 24.9 against 17.1)
+//   64 x 128 x 64, 2 x 4 waves, three stages   n = 1: 4.4 + 0.0053 / 0.0060 k;  n = 2: 5.8 + 0.0085 / 0.0104 k;  else
+//                                              3.5 + n (1.6 + 0.0039 / 0.0057 k)
+//                                              (2000 x 776 x 1160 11.9 against 13.8; 1504^3 18.5 against 19.7)
+//   128 x 128 x 64, 2 x 4 waves, four stages   n = 1 only: 7.0 + 0.0072 / 0.0080 k, at least 9.4
+//                                              (2048^3 23.5 against 27; 3488 x 600 x 1072 15.1 against 15.8)
+//   the same, two stages (two workgroups       n = 2: 8.2 + 0.0122 k;  else n (3.9 + 0.0077 k) / 4.0 + n (3.4 + 0.0088 k)
+//   per CU)                                    (1344 x 3328 x 880 18.0 against 21.1; 3224 x 1392 x 2968 45.7 against
+//                                              54.9)
+//   256 x 256 x 32, 2 x 4 waves, four stages   2.0 + n (14.8 + 0.0235 k), up to k = 384 with result rows that are
+//                                              no whole lines, which it stores past the caches, 20.0;
+//                                              8.5 + 0.0255 n k
+//                                              (4096^3 120; 3000^3 85 against 104; 4096^2 x 256 21.5 against 27;
+//                                              tn 5768 x 2456 x 192 28 against 23)
 // The step-by-step cost of the small tiles is the chain of a step; from two workgroups per CU on it is the
 // 64 bytes per clock that a CU fetches: a 64 x 64 tile needs 512 bytes per MFMA of 16 x 16 x 32 (four clocks of
 // the CU's matrix cores), a 128 x 128 tile 256, a 256 x 256 tile 128.
@@ -93,30 +94,37 @@ static hipError_t launch_dense_ring_layout(const TileGemmParams &p, hipStream_t 
   const auto most = [](double a, double b) { return a > b ? a : b; };
   const double k = p.k;
   const bool lines = p.ldx % 64 == 0 && p.ldy % 64 == 0;
-  const int n64 = tiles_per_cu(p, 64, 64), n128 = tiles_per_cu(p, 128, 64), n128s = tiles_per_cu(p, 128, 128), n256 = tiles_per_cu(p, 256, 256);
+  const auto of = [&](double whole, double broken) { return lines ? whole : broken; };
+  const int n64 = tiles_per_cu(p, 64, 64), n128 = tiles_per_cu(p, 64, 128), n128s = tiles_per_cu(p, 128, 128), n256 = tiles_per_cu(p, 256, 256);
   const double tiles = (double)((p.m + 63) / 64) * ((p.n + 63) / 64);
-  const double t64 = n64 == 1 ? 3.6 + 0.0039 * k : 2.6 + n64 * most((n64 >= 8 ? 1.05 : 0.95) + 0.0026 * k, 0.21 + (lines ? 0.0033 : 0.0045) * k);
-  double tw = 1e30;
-  if (tiles <= 32) tw = 3.8 + 0.0018 * k;
-  else if (n64 == 1 && lines && tiles * k <= 160.0 * 1024) tw = 4.3 + 0.0018 * k;
-  else if (n64 == 1 && lines && (XT || YT)) tw = 3.6 + 0.0038 * k;
-  const double p128 = (n128 + 1) / 2, p128s = (n128s + 1) / 2;
-  const double t128 = n128 == 1 ? most(5.8, 5.0 + 0.006 * k)
-                                : most(2.0 + p128 * (4.4 + (p128 >= 3 ? 0.0095 : 0.008) * k), 5.0 + (lines ? 0.0105 : 0.0135) * p128 * k);
-  const double t128s = n128s == 1 ? most(9.0 + 0.0095 * k, 5.0 + 0.0138 * k)
-                                  : most(2.5 + p128s * (8.0 + 0.0125 * k), 5.0 + 0.0172 * p128s * k);
+  const bool few = tiles <= 32;
+  const double t64 = few        ? 3.7 + 0.0036 * k
+                     : n64 == 1 ? 3.7 + of(0.0040, 0.0046) * k
+                     : n64 == 2 ? 4.9 + of(0.0063, 0.0076) * k
+                                : 2.4 + n64 * (1.12 + of(0.0031, 0.0040) * k);
+  const double t64k = few ? 4.1 + of(0.0026, 0.0030) * k : (n64 == 1 ? 4.2 + of(0.0030, 0.0038) * k : 1e30);
+  const double tw = few ? 4.2 + (lines || tiles * k <= 40000 ? 0.0020 : 0.0032) * k : 1e30;
+  const double t128 = n128 == 1   ? 4.4 + of(0.0053, 0.0060) * k
+                      : n128 == 2 ? 5.8 + of(0.0085, 0.0104) * k
+                                  : 3.5 + n128 * (1.6 + of(0.0039, 0.0057) * k);
+  const double t128s = n128s == 1   ? most(9.4, 7.0 + of(0.0072, 0.0080) * k)
+                       : n128s == 2 ? 8.2 + 0.0122 * k
+                                    : of(n128s * (3.9 + 0.0077 * k), 4.0 + n128s * (3.4 + 0.0088 * k));
   const double t256 = most(2.0 + n256 * ((p.ldc % 64 == 0 || k > 384 ? 14.8 : 20.0) + 0.0235 * k), 8.5 + 0.0255 * n256 * k);
-  if (t256 <= t128s && t256 <= t128 && t256 <= t64 && t256 <= tw) return launch_dense_pipe<T, XT, YT>(p, s);
-  if (t128s <= t128 && t128s <= t64 && t128s <= tw) return launch_dense_ring_as<T, 2, 2, 4, 4, 2, 2, XT, YT>(p, s);
-  if (t128 <= t64 && t128 <= tw) return launch_dense_ring_as<T, 2, 2, 4, 2, 2, 3, XT, YT>(p, s);
-  if (tw < t64) {
+  const double least = std::min({t64, t64k, tw, t128, t128s, t256});
+  if (least == t256) return launch_dense_pipe<T, XT, YT>(p, s);
+  if (least == t128s)
+    return n128s == 1 ? launch_dense_ring_as<T, 2, 4, 1, 4, 2, 2, 4, XT, YT>(p, s) : launch_dense_ring_as<T, 2, 4, 1, 4, 2, 2, 2, XT, YT>(p, s);
+  if (least == t128) return launch_dense_ring_as<T, 2, 4, 1, 2, 2, 2, 3, XT, YT>(p, s);
+  if (least == t64k) return launch_dense_ring_as<T, 2, 2, 2, 2, 2, 4, 4, XT, YT>(p, s);
+  if (least == tw) {
     if (!counted_waits_hold<densegemm_wave_kernel<T, 8, 1, 2, XT, YT>>()) return hipErrorNotSupported;
     const int tiles_m = (p.m + 63) / 64, tiles_n = (p.n + 63) / 64;
     hipLaunchKernelGGL((densegemm_wave_kernel<T, 8, 1, 2, XT, YT>), dim3((unsigned)(tiles_m * tiles_n)), dim3(512), 0, s, p, tiles_m,
                        tiles_n);
     return hipGetLastError();
   }
-  return launch_dense_ring_as<T, 2, 2, 2, 2, 2, 3, XT, YT>(p, s);
+  return launch_dense_ring_as<T, 2, 2, 2, 2, 2, 2, 3, XT, YT>(p, s);
 }
 
 // Contractions of a step or two have nothing to stream: half a step always, and up to a step and a half with

@@ -83,3 +83,20 @@ def test_short_contractions_on_either_side_of_the_streaming_kernels(tile, ta, tb
             print("case dense short", tile, m, n, k, ta, tb, flush=True)
             _run("f16", m, n, k, ta, tb, "matrix", alpha=0.5, beta=2.0, tile=tile)
             _run("bf16", m, n, k, ta, tb, "bias", alpha=1.0, beta=1.0, relu=True, tile=tile)
+
+
+@pytest.mark.parametrize("ta,tb", [(False, True), (False, False), (True, False), (True, True)])
+@pytest.mark.parametrize("m,n,k", [(72, 136, 72),          # few tiles, one step and a remainder, two wave groups
+                                   (72, 136, 1032),        # k over eight waves / 128 of k per step by the lines
+                                   (1000, 1000, 136),      # 64 x 64, a tile per CU
+                                   (1000, 1000, 904),      # 64 x 64, 128 of k per step, remainder of a group's slice
+                                   (1992, 776, 1160),      # 64 x 128
+                                   (2040, 1992, 1992),     # 128 x 128, a tile per CU
+                                   (1992, 3336, 872)])     # 128 x 128, two tiles per CU
+def test_kernels_of_eight_waves(m, n, k, ta, tb):
+    """Every tile of the eight-wave kernels at ragged m, n and k: row and column remainders, a last step whose k
+    ends inside one wave group's slice."""
+    torch.backends.cuda.matmul.allow_tf32 = False
+    print("case dense eight waves", m, n, k, ta, tb, flush=True)
+    _run("f16", m, n, k, ta, tb, "matrix", alpha=0.5, beta=2.0)
+    _run("bf16", m, n, k, ta, tb, "none")
