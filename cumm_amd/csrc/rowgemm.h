@@ -80,6 +80,8 @@ struct RowGemmParams {
   // non-zero (descriptors with num_stage 3): a contraction of more than 128 bytes is walked in
   // 64-byte chunks through three stages where the tile has such a kernel (128 x 128)
   int32_t small_stages;
+  // two groups of waves per tile: bit k of word k / 32 set = offset k belongs to the first group
+  uint32_t first_group[4];
 };
 
 // An offset no buffer contains: every operand is smaller than 2 GiB (checked on the host), and

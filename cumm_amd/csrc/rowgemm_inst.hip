@@ -55,11 +55,62 @@ constexpr int lds_stages(int TM, int TN, int KS) {
 template <class T, int TM, int TN>
 constexpr bool has_mask_words_kernel() { return Elem<T>::kBytes == 2 && !kWide && TM == TN; }
 
+// The offsets of the first of two groups.  Fixed by their numbers, so that a row's sum is the same in whatever
+// order the positions lie; halved on the sets that tiles have: all offsets of a dense neighbourhood, and in
+// the backward-input pass of a strided layer, per axis, the even or the odd indices.  The parity of the sum of
+// the halved indices does that for square and cubic kernels (strided 128 -> 128 backward-input 10.1 us, by the
+// parity of the number 12.2); other volumes go by the parity of the number.
+static void first_group_offsets(int kv, uint32_t (&words)[4]) {
+  int side = 2, dims = 0;
+  for (; side * side <= kv && dims == 0; ++side)
+    for (int d = 2, v = side * side; d <= 3 && v <= kv; ++d, v *= side)
+      if (v == kv) dims = d;
+  --side;      // (the loop leaves one past)
+  for (uint32_t &w : words) w = 0;
+  for (int k = 0; k < kv && k < 128; ++k) {
+    int sum = k;
+    if (dims > 0) {
+      sum = 0;
+      for (int d = 0, rest = k; d < dims; ++d, rest /= side) sum += (rest % side) >> 1;
+    }
+    if ((sum & 1) == 0) words[k / 32] |= 1u << (k % 32);
+  }
+}
+
+// Launches of few workgroups, 64 x 64 tiles: two groups of waves per tile, each for half of the kernel
+// offsets.  Such a launch is as long as its heaviest tile, and that is a chain of steps of about 0.5 us each
+// (0.33 with one mask word), whatever the number of ring stages or of waves in one group: a wave's own
+// instructions, one after the other.  A step of both groups takes 0.7 us for two offsets.  Two stages per
+// group (64 KB): two workgroups per CU.  Where the device is full the plain kernel has more tiles in flight
+// and is the faster one; the line, in workgroups, from f16 forward passes on one cloud (us, plain / groups):
+//   one step per offset       384    64 channels, 173 workgroups 12.8 / 10.7, 347 12.9 / 11.1, 500 10.9 / 11.2, 691
+//                                    11.1 / 11.6 (mixed tile shapes on the left)
+//   rows of 64 bytes          1024   16 channels, 125 workgroups 10.1 / 8.6, 691 10.3 / 9.4, 1375 10.4 / 11.2;  32 -> 96
+//                                    channels, 1000 workgroups 10.3 / 9.7, 1382 10.5 / 11.9
+//   several steps per offset  1024   128 -> 128 channels, 500 workgroups 21.7 / 18.2, 1000 22.3 / 19.6, 2750 23.8 / 34.5
+//   several mask words        1024   5 x 5 x 5, 64 channels, 125 workgroups 62.6 / 44.3, 469 62.1 / 45.3, 938 62.2 / 53.8,
+//                                    1875 66.1 / 69.9
+template <class T, int TM, int TN, int KS, bool WT, int MW>
+static bool launch_two_groups(const RowGemmParams &p, dim3 grid, hipStream_t s, hipError_t *err) {
+  if constexpr (TM == 64 && TN == 64 && KS <= 2 && !kWide && (!WT || Elem<T>::kBytes == 2)) {
+    const unsigned most = MW > 1 || p.chunk_shift > 0 || KS == 1 ? 1024u : 384u;
+    if (p.mask == nullptr || (uint64_t)grid.x * grid.y > most) return false;
+    if (!counted_waits_hold<rowgemm_lds_kernel<T, 2, 2, 2, 2, KS, 2, WT, false, MW, 2>>()) return false;
+    RowGemmParams q = p;
+    first_group_offsets(p.kv, q.first_group);
+    hipLaunchKernelGGL((rowgemm_lds_kernel<T, 2, 2, 2, 2, KS, 2, WT, false, MW, 2>), grid, dim3(512), 0, s, q);
+    *err = hipGetLastError();
+    return true;
+  }
+  return false;
+}
+
 template <class T, int NW, int RB, int TN, int KS, bool WT>
 static hipError_t launch_one(const RowGemmParams &p, hipStream_t s) {
   constexpr int TM = NW * RB * 16;
   dim3 grid((p.n_pos + TM - 1) / TM, (p.k_out + TN - 1) / TN, 1);
   if (grid.x == 0 || grid.y == 0) return hipSuccess;
+  hipError_t err = hipSuccess;
   constexpr int chunk_e = 4 * KS * Elem<T>::kPerVec;
   if (p.mask_words > 1) {
     // kernel volumes above 32 (the reference's dynamic-mask kernels): the LDS-streaming kernel
@@ -73,6 +124,7 @@ static hipError_t launch_one(const RowGemmParams &p, hipStream_t s) {
         RowGemmParams q = p;
         const int nch = (p.c_in + chunk_m - 1) / chunk_m;
         while ((1 << q.chunk_shift) < nch) ++q.chunk_shift;
+        if (q.chunk_shift <= 3 && launch_two_groups<T, TM, TN, KSM, WT, 4>(q, grid, s, &err)) return err;
         if (q.chunk_shift <= 3 && counted_waits_hold<rowgemm_lds_kernel<T, 2, 2, TM / 32, TN / 32, KSM, NSM, WT, false, 4>>()) {
           hipLaunchKernelGGL((rowgemm_lds_kernel<T, 2, 2, TM / 32, TN / 32, KSM, NSM, WT, false, 4>), grid, dim3(256), 0, s, q);
           return hipGetLastError();
@@ -114,9 +166,10 @@ static hipError_t launch_one(const RowGemmParams &p, hipStream_t s) {
       int shift = 0;
       while ((1 << shift) < nch) ++shift;
       if (shift <= 3 && (WT ? p.w_stride_n == 1 : p.w_stride_c == 1)) {
+        RowGemmParams q = p;
+        q.chunk_shift = shift;
+        if (launch_two_groups<T, TM, TN, 2, WT, 1>(q, grid, s, &err)) return err;
         if (counted_waits_hold<rowgemm_lds_kernel<T, 2, 2, TM / 32, TN / 32, 2, NS2, WT, kWide>>()) {
-          RowGemmParams q = p;
-          q.chunk_shift = shift;
           hipLaunchKernelGGL((rowgemm_lds_kernel<T, 2, 2, TM / 32, TN / 32, 2, NS2, WT, kWide>), grid, dim3(256), 0, s, q);
           return hipGetLastError();
         }
@@ -127,6 +180,7 @@ static hipError_t launch_one(const RowGemmParams &p, hipStream_t s) {
   if constexpr (NS > 0 && (!WT || Elem<T>::kBytes == 2)) {
     // the LDS-streaming kernel: 2 x 2 waves, each TM/2 rows by TN/2 channels
     if (p.c_in <= chunk_e && (WT ? p.w_stride_n == 1 : p.w_stride_c == 1)) {
+      if (launch_two_groups<T, TM, TN, KS, WT, 1>(p, grid, s, &err)) return err;
       if constexpr (TM == 64 && TN == 64 && Elem<T>::kBytes == 2 && KS <= 2 && !kWide) {
         if (p.hint_slot != nullptr && grid.y == 1 && p.chunk_shift == 0 && p.mask != nullptr &&
             counted_waits_hold<rowgemm_lds_mixed_kernel<T, KS, WT>>()) {

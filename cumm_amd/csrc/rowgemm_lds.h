@@ -61,6 +61,7 @@ struct LdsRing {
   v4i *rows[4];
   v4i *weights[4];
   int (*idx[4])[64];
+  v4i *park;      // WK groups: where they leave sums for each other (a stage of every group)
 };
 
 // One tile: rows [tile * TM, tile * TM + TM) of the sorted positions, column block col.
@@ -73,7 +74,11 @@ struct LdsRing {
 // cumm/gemm/blockmma/mma.py:78-269): p.mask_words = ceil(kv / 32) words per position, word w of
 // position pos at mask[pos * mask_words + w] holding offsets 32 w .. 32 w + 31; mask_out likewise
 // per tile; the filter applies to every word.
-template <class T, int WM, int WN, int RBW, int NBW, int KS, int NS, bool WT, bool WIDE, bool HALVES, int MW = 1, bool HALF32 = false>
+// WK: groups of WM x WN waves that share the tile.  With two, the first takes the kernel offsets of
+// p.first_group and the second the others (whatever the tile's list: a row's sum does not depend on its
+// neighbours), each with a ring of its own, and at the end they add up their sums in LDS, each of them for
+// half of the row blocks.
+template <class T, int WM, int WN, int RBW, int NBW, int KS, int NS, bool WT, bool WIDE, bool HALVES, int MW = 1, bool HALF32 = false, int WK = 1>
 __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const int tile, const int col, const LdsRing &lds) {
   static_assert(MW == 1 || MW == 4, "one mask word, or up to four");
   static_assert(MW == 1 || (!HALVES && !HALF32), "the tile shapes of a mixed launch take one mask word");
@@ -110,7 +115,9 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave_of_all = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = WK == 1 ? 0 : wave_of_all / NW;
+  const int wave = WK == 1 ? wave_of_all : wave_of_all % NW;
   const int wm = wave / WN, wn = wave % WN;
   const int m = lane & 15;
   const int q = lane >> 4;
@@ -338,6 +345,19 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
     n_offsets = 0;
 #pragma unroll
     for (int w = 0; w < MW; ++w) n_offsets += __builtin_popcount(kwords[w]);
+  }
+  if constexpr (WK == 2) {      // this group's offsets; the barriers of both are the longer list's
+    int first = __builtin_popcount(kmask & p.first_group[0]);
+    kmask &= group == 0 ? p.first_group[0] : ~p.first_group[0];
+    if constexpr (MW > 1) {
+      first = 0;
+#pragma unroll
+      for (int w = 0; w < MW; ++w) {
+        first += __builtin_popcount(kwords[w] & p.first_group[w]);
+        kwords[w] &= group == 0 ? p.first_group[w] : ~p.first_group[w];
+      }
+    }
+    n_offsets = first > n_offsets - first ? first : n_offsets - first;
   }
   const int n_steps = n_offsets << p.chunk_shift;
 
@@ -632,6 +652,27 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
   for (int rb = 0; rb < RBW; ++rb)
 #pragma unroll
     for (int i = 0; i < SRC_N; ++i) keep_after_wait(src_pre[rb][i]);
+  if constexpr (WK > 1) {
+    static_assert(WK == 2 && RBW % 2 == 0 && !HALVES && !HALF32, "two groups, half of the row blocks each");
+    constexpr int RO = RBW / 2;
+    __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): this wave has read its last stage,
+    lds_barrier();                        // and so has every other
+    AccV *park = reinterpret_cast<AccV *>(lds.park);      // [group][wave][block]
+#pragma unroll
+    for (int r = 0; r < RO; ++r)
+#pragma unroll
+      for (int nb = 0; nb < NBW; ++nb) park[((wave_of_all * RO + r) * NBW + nb) * 64 + lane] = group == 0 ? acc[RO + r][nb] : acc[r][nb];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RO; ++r)
+#pragma unroll
+      for (int nb = 0; nb < NBW; ++nb) {
+        const AccV other = park[((((1 - group) * NW + wave) * RO + r) * NBW + nb) * 64 + lane];
+        if (group == 0) acc[r][nb] = acc[r][nb] + other;
+        else acc[RO + r][nb] = other + acc[RO + r][nb];
+      }
+  }
+  auto mine = [&](int rb) __attribute__((always_inline)) -> bool { return WK == 1 || rb / (RBW / WK) == group; };
   // (a 64-row tile without any offset is left alone when exit_on_empty is set: so is that half)
   if (HALVES && half_skipped) return;
   // ---- epilogue: lane (q, m) holds, for each of its rows, channels ch0 .. ch0 + 4*NBW - 1.
@@ -643,7 +684,7 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
 #pragma unroll
     for (int rb = 0; rb < RBW; ++rb) {
       const int o = out_row[rb];
-      const bool row_ok = o >= 0 && o < p.rows_c;
+      const bool row_ok = o >= 0 && o < p.rows_c && mine(rb);
 #pragma unroll
       for (int nb = 0; nb < NBW; ++nb) {
         const int ch = ch0 + nb * 4;
@@ -661,6 +702,7 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
       constexpr int NG = CPLW / 8;   // 16-byte groups
 #pragma unroll
       for (int rb = 0; rb < RBW; ++rb) {
+        if (!mine(rb)) continue;
         const int o = out_row[rb];
         const bool row_ok = o >= 0 && o < p.rows_c;
 #pragma unroll
@@ -690,6 +732,7 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
       typedef int vNi __attribute__((ext_vector_type(ND)));
 #pragma unroll
       for (int rb = 0; rb < RBW; ++rb) {
+        if (!mine(rb)) continue;
         const int o = out_row[rb];
         const bool ok = o >= 0 && o < p.rows_c && ch0 < p.k_out;
         const uint32_t coff = ok ? (uint32_t)((int64_t)o * p.ldc + ch0) : kOob;
@@ -737,26 +780,31 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
   }
 }
 
-template <class T, int WM, int WN, int RBW, int NBW, int KS, int NS, bool WT = false, bool WIDE = false, int MW = 1>
-__global__ __launch_bounds__(WM *WN * 64) void rowgemm_lds_kernel(const RowGemmParams p) {
+template <class T, int WM, int WN, int RBW, int NBW, int KS, int NS, bool WT = false, bool WIDE = false, int MW = 1, int WK = 1>
+__global__ __launch_bounds__(WM *WN *WK * 64) void rowgemm_lds_kernel(const RowGemmParams p) {
   constexpr int NW = WM * WN;
   constexpr int LPR = 4 * KS;
   constexpr int A_V = WM * RBW * 16 * LPR;
   constexpr int STAGE_V = (WM * RBW * 16 + WN * NBW * 16) * LPR;
-  __shared__ v4i st0[STAGE_V];
-  __shared__ v4i st1[STAGE_V];
-  __shared__ v4i st2[NS > 2 ? STAGE_V : 1];
-  __shared__ v4i st3[NS > 3 ? STAGE_V : 1];
+  __shared__ v4i st0[WK * STAGE_V];
+  __shared__ v4i st1[WK * STAGE_V];
+  __shared__ v4i st2[NS > 2 ? WK * STAGE_V : 1];
+  __shared__ v4i st3[NS > 3 ? WK * STAGE_V : 1];
   // pair-table entries also travel global -> LDS directly: every vector load of the step loop is
   // then counted by hand, none returns into a register the compiler would guard with waits of
   // its own.  Slot [d][wave][l] is written by lane l of the wave (lanes >= RPW write zeros).
   // (one array per slot, like the stages)
-  __shared__ int ix0[NW][64];
-  __shared__ int ix1[NW][64];
-  __shared__ int ix2[NS > 2 ? NW : 1][64];
-  __shared__ int ix3[NS > 3 ? NW : 1][64];
-  const LdsRing lds = {{st0, st1, st2, st3}, {st0 + A_V, st1 + A_V, NS > 2 ? st2 + A_V : st2, NS > 3 ? st3 + A_V : st3},
-                       {ix0, ix1, ix2, ix3}};
+  __shared__ int ix0[WK * NW][64];
+  __shared__ int ix1[WK * NW][64];
+  __shared__ int ix2[NS > 2 ? WK * NW : 1][64];
+  __shared__ int ix3[NS > 3 ? WK * NW : 1][64];
+  static_assert(WK == 1 || STAGE_V >= NW * (RBW / 2 * NBW) * 64, "a stage of every group holds the sums they exchange");
+  const int group = WK == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) / NW;
+  const int gs = group * STAGE_V, gi = group * NW;
+  const LdsRing lds = {{st0 + gs, st1 + gs, NS > 2 ? st2 + gs : st2, NS > 3 ? st3 + gs : st3},
+                       {st0 + gs + A_V, st1 + gs + A_V, NS > 2 ? st2 + gs + A_V : st2, NS > 3 ? st3 + gs + A_V : st3},
+                       {ix0 + gi, ix1 + gi, NS > 2 ? ix2 + gi : ix2, NS > 3 ? ix3 + gi : ix3},
+                       st0};
 
   // Workgroups are dispatched in the order of their linear number, round-robin over the 8 XCDs.
   // With several column blocks per row tile, the workgroups of one row tile are given numbers 8
@@ -778,7 +826,7 @@ __global__ __launch_bounds__(WM *WN * 64) void rowgemm_lds_kernel(const RowGemmP
     }
   }
   const int tile = (int)gridDim.x - 1 - tile_rank;  // heaviest tiles first (masks sorted ascending)
-  rowgemm_lds_tile<T, WM, WN, RBW, NBW, KS, NS, WT, WIDE, false, MW>(p, tile, col, lds);
+  rowgemm_lds_tile<T, WM, WN, RBW, NBW, KS, NS, WT, WIDE, false, MW, false, WK>(p, tile, col, lds);
 }
 
 // Tiles of two shapes in one launch, for one column block of 64 channels (grid.x = number of
@@ -834,14 +882,14 @@ __global__ __launch_bounds__(256) void rowgemm_lds_mixed_kernel(const RowGemmPar
   if (rank < halves) {
     if constexpr (KS == 2) {
       constexpr int R32 = 32 * 4 * KS;      // 16-byte vectors of 32 rows
-      const LdsRing lds = {{st0, st1, st2, nullptr}, {st0 + R32, st1 + R32, st2 + R32, nullptr}, {ix0, ix1, ix2, nullptr}};
+      const LdsRing lds = {{st0, st1, st2, nullptr}, {st0 + R32, st1 + R32, st2 + R32, nullptr}, {ix0, ix1, ix2, nullptr}, nullptr};
       rowgemm_lds_tile<T, 2, 2, 1, 2, KS, 3, WT, false, false, 1, true>(p, 2 * tiles - 1 - rank, 0, lds);
     }
   } else if (rank - halves < singles) {
-    const LdsRing lds = {{st0, st1, st2, nullptr}, {st0 + R64, st1 + R64, st2 + R64, nullptr}, {ix0, ix1, ix2, nullptr}};
+    const LdsRing lds = {{st0, st1, st2, nullptr}, {st0 + R64, st1 + R64, st2 + R64, nullptr}, {ix0, ix1, ix2, nullptr}, nullptr};
     rowgemm_lds_tile<T, 2, 2, 2, 2, KS, 3, WT, false, false>(p, tiles - heavy - 1 - (rank - halves), 0, lds);
   } else if (rank - halves - singles < pairs) {
-    const LdsRing lds = {{st0, st1, nullptr, nullptr}, {st2, st2 + R64, nullptr, nullptr}, {ix0, ix1, nullptr, nullptr}};
+    const LdsRing lds = {{st0, st1, nullptr, nullptr}, {st2, st2 + R64, nullptr, nullptr}, {ix0, ix1, nullptr, nullptr}, nullptr};
     rowgemm_lds_tile<T, 2, 2, 4, 2, KS, 2, WT, false, true>(p, pairs - 1 - (rank - halves - singles), 0, lds);
   }
 }
