@@ -394,6 +394,7 @@ class _SparseConvFunction(torch.autograd.Function):
             raise ValueError("features must be [%d, C]: one row per input site of the geometry" % geometry.n_in)
         if weight.dim() != 3 or weight.shape[1] != geometry.kv or weight.shape[2] != features.shape[1]:
             raise ValueError("weight must be [K, %d, %d]" % (geometry.kv, features.shape[1]))
+        _check_device(geometry, features, weight, bias)      # (a remembered call takes addresses)
         out = torch.empty((geometry.n_out, weight.shape[0]), dtype=features.dtype, device=features.device)
         roles = {"input": features, "weight": weight, "output": out}
         if bias is not None:
@@ -413,6 +414,7 @@ class _SparseConvFunction(torch.autograd.Function):
     def backward(ctx, grad_out):
         features, weight, out = ctx.saved_tensors
         g: SparseConvGeometry = ctx.geometry
+        _check_device(g, features, weight, out, grad_out)      # (saved-tensor hooks may have moved them)
         grad_out = grad_out.contiguous()
         dtype = _TORCH_TO_TV[features.dtype]
         stream = current_stream()
@@ -477,12 +479,16 @@ class _SparseConvFunction(torch.autograd.Function):
         return grad_in, grad_w, grad_b, None, None
 
 
+def _check_device(g: SparseConvGeometry, *tensors) -> None:
+    if any(t is not None and t.device != g._device for t in tensors):
+        raise ValueError("all tensors must be on the same device")
+
+
 def _kind(g: SparseConvGeometry, key, n_pos: int, *tensors):
     """The key of a call in _KINDS; the tensors of a first call are checked here for what the operator's
     prelude checks and a moved call does not: one device, that of the tables (types and shapes are in the
     key)."""
-    if any(t.device != g._device for t in tensors):
-        raise ValueError("all tensors must be on the same device")
+    _check_device(g, *tensors)
     return key + (g.kv, g.subm, _size_class(n_pos), g._device.index)
 
 

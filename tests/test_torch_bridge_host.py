@@ -216,3 +216,41 @@ def test_pair_lists_wait_only_where_they_were_handed_out(monkeypatch):
     g, _, _ = _geometry(monkeypatch, tb)
     del g.lists
     assert g.lists is None
+
+
+def test_a_remembered_call_refuses_tensors_on_another_device(monkeypatch):
+    """A call that the geometry remembers takes addresses: the device of every tensor is looked at before each
+    of them, in both passes - the first use on a geometry was checked, later ones were not."""
+    from cumm_amd import torch_bridge as tb
+    g, _, _ = _geometry(monkeypatch, tb)
+    calls = []
+
+    class Launch:
+        tile_m = 64
+
+        def __call__(self, stream, *a, **tensors):
+            calls.append(tensors)
+
+    class Known(dict):
+        def get(self, key, default=None):
+            return (Launch(), 256) if key[0] == "wgrad" else Launch()
+    g._launches = Known()
+    monkeypatch.setattr(tb._capi, "lib", lambda: None)
+    x, w, b, y = torch.zeros(1000, 8).half(), torch.zeros(16, 27, 8).half(), torch.zeros(16).half(), torch.zeros(1000, 16).half()
+    away = lambda t: t.to("meta")
+    assert tb._SparseConvFunction.apply(x, w, b, g, False).shape == (1000, 16) and len(calls) == 1
+    for tensors in ((away(x), w, b), (x, away(w), b), (x, w, away(b))):
+        with pytest.raises(ValueError, match="same device"):
+            tb._SparseConvFunction.apply(*tensors, g, False)
+    assert len(calls) == 1
+    ctx = type("Ctx", (), dict(geometry=g, relu=False, has_bias=False, tile_m=64, needs_input_grad=(True, True, False)))()
+
+    def backward(x, w, y):
+        ctx.saved_tensors = (x, w, None)
+        return tb._SparseConvFunction.backward(ctx, y)
+    backward(x, w, y)
+    assert len(calls) == 3
+    for tensors in ((away(x), w, y), (x, away(w), y), (x, w, away(y))):
+        with pytest.raises(ValueError, match="same device"):
+            backward(*tensors)
+    assert len(calls) == 3
