@@ -5,6 +5,7 @@
 This replaces the reference's NVRTC / pccm JIT builds
 (cumm/nvrtc/__init__.py:179-283, cumm/gemm/main_real.py:59-70).
 """
+import importlib.util
 import os
 import subprocess
 import sys
@@ -14,6 +15,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(CSRC, "obj")
 LIB = os.path.join(HERE, "libcummhip.so")
+TORCH_LIB = os.path.join(HERE, "_torch_native.so")
+TORCH_SRC = os.path.join(CSRC, "torch_native.cpp")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-gpu-rdc",
@@ -87,6 +90,29 @@ def build(force=False, verbose=False, jobs=None):
             print(" ".join(cmd), flush=True)
         subprocess.check_call(cmd)
     return LIB
+
+
+def build_torch_native(force=False, verbose=False):
+    """Compile the native half of torch_bridge.py (host code against torch's headers) if stale or ``force``."""
+    stamp = max(os.path.getmtime(f) for f in (TORCH_SRC, os.path.join(HERE, "..", "include", "cumm_hip.h")))
+    if not force and os.path.exists(TORCH_LIB) and os.path.getmtime(TORCH_LIB) >= stamp:
+        return TORCH_LIB
+    import sysconfig
+    import torch
+    root = os.path.dirname(torch.__file__)
+    include = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+               os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"), sysconfig.get_paths()["include"]]
+    cmd = (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            "-DTORCH_EXTENSION_NAME=_torch_native", "-DTORCH_API_INCLUDE_EXTENSION_H"] +
+           [a for d in include for a in ("-isystem", d)] + [TORCH_SRC, "-o", TORCH_LIB + ".tmp", "-L" + os.path.join(root, "lib")] +
+           ["-l" + n for n in ("torch", "torch_cpu", "torch_hip", "torch_python", "c10", "c10_hip")])
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("g++ failed for %s:\n%s" % (TORCH_SRC, res.stdout))
+    os.replace(TORCH_LIB + ".tmp", TORCH_LIB)
+    return TORCH_LIB
 
 
 # ---- check of the generated code around the hand-written vector-memory instructions
@@ -211,3 +237,5 @@ if __name__ == "__main__":
         sys.exit(1 if hits else 0)
     build(force="--force" in sys.argv, verbose=True)
     print(LIB)
+    if importlib.util.find_spec("torch") is not None:      # (only torch_bridge.py needs it)
+        print(build_torch_native(force="--force" in sys.argv, verbose=True))

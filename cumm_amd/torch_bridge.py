@@ -9,6 +9,7 @@ and the bias gradient of the backward pass.  Imported on demand: nothing else in
 needs torch.
 """
 import ctypes
+import os
 from typing import Optional, Sequence, Tuple
 
 import torch
@@ -166,6 +167,45 @@ def _copy(args: _capi.SparseConvArgs) -> _capi.SparseConvArgs:
 _KINDS = {}
 
 
+# the keys of the calls that native code knows too, by the number it knows them by
+_NATIVE_KEYS = []
+_NATIVE_SYMBOLS = ("sparse_conv", "last_error", "relu_backward", "relu_backward_sums", "column_sum", "column_sum_workspace",
+                   "query_conv_workspace", "query_wgrad_ordered_workspace", "wgrad_pairs", "wgrad_pairs_workspace", "subm_pairs",
+                   "subm_pairs_workspace", "conv_pairs_workspace", "conv_pairs_sites", "conv_pairs_fill", "order_pairs",
+                   "order_pairs_workspace")
+_native_module = None
+
+
+def _native():
+    """The native half of this module (csrc/torch_native.cpp); built first if it is not there."""
+    global _native_module
+    if _native_module is None:
+        from . import build
+        if not os.path.exists(build.TORCH_LIB):
+            build.build_torch_native()
+        from . import _torch_native as native
+        native.bind({"cumm_hip_" + n: ctypes.cast(getattr(_capi.lib(), "cumm_hip_" + n), ctypes.c_void_p).value
+                     for n in _NATIVE_SYMBOLS})
+        native.set_backward(_backward)
+        _native_module = native
+    return _native_module
+
+
+def _remember(g: "SparseConvGeometry", key, kind, launch: "_Launch", op: ConvOpType, features, weight, bias=None) -> None:
+    """A validated call of a kind, for the geometries to come - here and in native code."""
+    _KINDS[kind] = launch
+    if g._native is None:
+        return
+    relu, tile_m, deterministic = key[5] if key[0] == "fwd" else False, 0, False
+    if key[0] == "wgrad":
+        tile_m, deterministic = key[3], key[4]
+    n_pos = g.n_in if op == ConvOpType.BackwardInput else g.n_out
+    if _native().remember(op.value, features.dtype, weight.dtype, None if bias is None else bias.dtype, int(weight.shape[0]),
+                          int(weight.shape[2]), g.kv, g.subm, _size_class(n_pos), g._device.index, bool(relu), tile_m, deterministic,
+                          bytes(launch.cdesc), bytes(launch.args), launch.tile_m, len(_NATIVE_KEYS)):
+        _NATIVE_KEYS.append(key)
+
+
 def _size_class(n: int) -> int:
     return max(n - 1, 0).bit_length()      # (the tuner's bucket of the position count)
 
@@ -202,78 +242,54 @@ class SparseConvGeometry:
 
     _TABLES = ("indices_fwd", "indices_bwd", "mask_fwd", "order_fwd", "mask_bwd", "order_bwd", "indices_fwd_pos", "indices_bwd_pos")
     _lists = _list_block = None      # (several mask words only)
+    _native = None                   # the geometry as native code has it
 
     def __init__(self, coords: torch.Tensor, spatial_shape: Sequence[int], ksize=(3, 3, 3), stride=None,
                  padding=(1, 1, 1), dilation=(1, 1, 1), batch_size: int = 1):
         if coords.dtype != torch.int32 or not coords.is_cuda or coords.dim() != 2 or coords.shape[1] != 4:
             raise ValueError("coords must be a cuda int32 tensor [N, 4] of (batch, z, y, x)")
-        coords = coords.contiguous()
-        self._stream = s = current_stream()
-        self._device = dev = coords.device
         self.subm = stride is None
-        self.n_in = n_in = int(coords.shape[0])
-        self.kv = kv = int(ksize[0]) * int(ksize[1]) * int(ksize[2])
+        if self.subm:
+            pairs._check_odd_ksize(ksize)
+        three = lambda a: tuple(int(v) for v in a)
+        ksize = three(ksize)
+        self.kv = kv = ksize[0] * ksize[1] * ksize[2]
         self.words = words = (kv + 31) // 32
+        self._stream, self._device, self.n_in = current_stream(), coords.device, int(coords.shape[0])
         # (how far the light end of each sorted order reaches - the hint of the forward and backward-input
         # launches - stays on the device: the sort leaves it in the library's table under the sorted
         # array's address and the launches look it up there; 0 = not given here)
         self.light_fwd = self.light_bwd = 0
         self._reduced, self._reduced_streams, self._written = {}, {}, set()
-        self._launches = {}      # calls of the layers on this geometry, see _Launch
+        self._own_launches = {}      # calls of the layers on this geometry, see _Launch
         self._tensors = {}
-        lib, arr3 = _capi.lib(), ctypes.c_int32 * 3
-        shape, ks, pad, dil = (arr3(*[int(v) for v in a]) for a in (spatial_shape, ksize, padding, dilation))
-        if self.subm:
-            pairs._check_odd_ksize(ksize)
-            self.n_out = n_out = n_in
-            self.out_coords, self.out_shape = coords, tuple(int(v) for v in spatial_shape)
-            self._allocate()
-            ws = _bytes(lib.cumm_hip_subm_pairs_workspace(n_in), dev)
-            _capi.check(lib.cumm_hip_subm_pairs(
-                coords.data_ptr(), n_in, shape, ks, dil, self._ptr["indices_fwd"], self._ptr["indices_bwd"], None, None,
-                ws.data_ptr(), ws.numel(), s))
-        else:
-            st = arr3(*[int(v) for v in stride])
-            geo = (shape, ks, st, pad, dil)
-            need = int(lib.cumm_hip_conv_pairs_workspace(n_in, int(batch_size), *geo))
-            if need == 0:
-                raise ValueError("bad geometry (kernel volume 1..128, non-empty output grid) or too many voxels")
-            ws = _bytes(need, dev)
-            out_shape, found = arr3(), ctypes.c_int32(0)
-            _capi.check(lib.cumm_hip_conv_pairs_sites(coords.data_ptr(), n_in, int(batch_size), *geo, out_shape,
-                                                      ctypes.byref(found), ws.data_ptr(), ws.numel(), s))
-            self.n_out = n_out = int(found.value)
-            self.out_shape = tuple(int(v) for v in out_shape)
-            self.out_coords = torch.empty((n_out, 4), dtype=torch.int32, device=dev)
-            self._allocate()
-            _capi.check(lib.cumm_hip_conv_pairs_fill(
-                coords.data_ptr(), n_in, int(batch_size), *geo, n_out, self.out_coords.data_ptr(), self._ptr["indices_fwd"],
-                self._ptr["indices_bwd"], None, None, ws.data_ptr(), ws.numel(), s))
+        self._native, self.out_coords, self.out_shape, ordered = _native().build(
+            coords.contiguous(), three(spatial_shape), ksize, None if self.subm else three(stride), three(padding), three(dilation),
+            int(batch_size))
+        self.n_out, self._block = self._native.n_out, self._native.block
         # masks, an order of the positions by them, and the pair tables once more in that order: what
         # forward and backward-input read (a tile's entries for one offset are then consecutive in
         # memory); backward-weight keeps the table by row
-        if 4 * kv * max(n_in, n_out) < 1 << 31:
-            self._order(ks)
-        else:
+        if not ordered:
             self._order_one_by_one()
         if words > 1:
             self._make_lists()
 
-    def _order(self, ks) -> None:
-        lib, p = _capi.lib(), self._ptr
-        sides = (_capi.OrderSide * 2)()
-        for d, side, n in ((sides[0], "fwd", self.n_out), (sides[1], "bwd", self.n_in)):
-            d.indices, d.n = p["indices_" + side], n
-            d.sorted_mask, d.argsort, d.by_position = p["mask_" + side], p["order_" + side], p["indices_%s_pos" % side]
-        count = 2
-        if self.subm:      # (one order serves both; the backward table is the forward one with its offsets reversed)
-            sides[0].by_position_reversed, count = p["indices_bwd_pos"], 1
-        ws = _bytes(lib.cumm_hip_order_pairs_workspace(sides, count, self.kv), self._device)
-        _capi.check(lib.cumm_hip_order_pairs(sides, count, ks, ws.data_ptr(), ws.numel(), self._stream))
+    @property
+    def _launches(self):
+        """The calls of the layers on this geometry; those made by native code without a _Launch here."""
+        if self._native is not None:
+            for i in self._native.used:
+                self._own_launches.setdefault(_NATIVE_KEYS[i], None)
+        return self._own_launches
+
+    @_launches.setter
+    def _launches(self, calls):
+        self._own_launches = calls
 
     def _order_one_by_one(self) -> None:
-        """``_order`` for tables of 2^31 bytes and more, which cumm_hip_order_pairs and the launches refuse:
-        whoever builds one wants the tables (the per-offset convolution walks lists of them)."""
+        """For tables of 2^31 bytes and more, which cumm_hip_order_pairs and the launches refuse: whoever builds
+        one wants the tables (the per-offset convolution walks lists of them)."""
         lib, p, s, kv, words = _capi.lib(), self._ptr, self._stream, self.kv, self.words
         for side, n in (("fwd", self.n_out), ("bwd", self.n_in)):
             if side == "fwd" or not self.subm:
@@ -290,6 +306,11 @@ class SparseConvGeometry:
             _capi.check(lib.cumm_hip_pairs_by_position(p["indices_" + side], p["order_" + side], kv, n, p["indices_%s_pos" % side], s))
 
     def _allocate(self) -> None:
+        self._block = _bytes(self._lay_out(0), self._device)
+        self._lay_out(self._block.data_ptr())
+
+    def _lay_out(self, base: int) -> int:
+        """Where the tables lie in the block (torch_native.cpp has the same); its size."""
         n_out, n_in, kv, words = self.n_out, self.n_in, self.kv, self.words
         mask = [self.n_out] if words == 1 else [n_out, words]
         spec = [("indices_fwd", [kv, n_out], tv.int32), ("indices_bwd", [kv, n_in], tv.int32),
@@ -309,13 +330,12 @@ class SparseConvGeometry:
         reduced_64, reduced_128 = at, at + (n_out // 64 + 64) // 64 * 256
         if words == 1:
             at = reduced_128 + (n_out // 128 + 64) // 64 * 256
-        self._block = _bytes(at, self._device)
-        base = self._block.data_ptr()
         self._ptr = {name: base + v[0] for name, v in self._spec.items()}
         self._reduced_at = {64: base + reduced_64, 128: base + reduced_128} if words == 1 else {}
         if self.subm:      # the forward masks serve the backward-input pass, bit-reversed in the kernel
             for name in ("mask", "order"):
                 self._spec[name + "_bwd"], self._ptr[name + "_bwd"] = self._spec[name + "_fwd"], self._ptr[name + "_fwd"]
+        return at
 
     def _make_lists(self) -> None:
         """The per-offset pair lists of backward-weight; their counts come to the host."""
@@ -327,7 +347,9 @@ class SparseConvGeometry:
         _capi.check(lib.cumm_hip_pair_lists(self._ptr["indices_fwd"], kv, n, lists[0].data_ptr(), lists[1].data_ptr(),
                                             counts.data_ptr(), ws.data_ptr(), ws.numel(), self._stream))
         self._list_block = lists
-        self._lists = self._lists_over(lists, counts.cpu().numpy())
+        counts = counts.cpu().numpy()
+        self._lists = self._lists_over(lists, counts)
+        self._native.set_lists(lists, counts.clip(0, n).tolist())
 
     def _lists_over(self, keepalive, counts) -> pairs.DevicePairLists:
         pair_in, pair_out = (tv.from_blob(t.data_ptr(), [self.kv, self.n_out], tv.int32, self._device.index, keepalive=keepalive)
@@ -339,7 +361,10 @@ class SparseConvGeometry:
             own = self._lists
             self.lists = None if own is None else self._lists_over(_HandedOut(self._list_block), own.counts)
             return self.lists
-        if name not in SparseConvGeometry._TABLES or "_spec" not in self.__dict__:
+        if name in ("_spec", "_ptr", "_reduced_at") and self._native is not None:
+            self._lay_out(self._block.data_ptr())      # (where somebody asks)
+            return self.__dict__[name]
+        if name not in SparseConvGeometry._TABLES or self.__dict__.get("_block") is None:
             raise AttributeError(name)
         t = self._tensors.get(name)
         if t is None:
@@ -376,7 +401,7 @@ class SparseConvGeometry:
 
     def reduced_mask_buffer(self, width: int) -> tv.Tensor:
         """Those words as a tv tensor; zeros until a forward pass with tiles of that height has run."""
-        fresh = width not in self._written
+        fresh = width not in self._written and not (self._native is not None and self._native.written(width))
         at, count = self.reduced_address(width), max((self.n_out + width - 1) // width, 1)
         owner = self._reduced.get(width, self._block)
         if fresh:
@@ -402,7 +427,7 @@ class _SparseConvFunction(torch.autograd.Function):
         stream = current_stream()
         geometry.used_on(stream)
         key = ("fwd", features.dtype, weight.dtype, weight.shape, None if bias is None else (bias.dtype, bias.shape), relu)
-        launch = geometry._launches.get(key)
+        launch = geometry._own_launches.get(key)
         if launch is None:
             launch = _forward_launch(geometry, key, roles, relu, stream)
         launch(stream, **roles)
@@ -413,70 +438,74 @@ class _SparseConvFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_out):
         features, weight, out = ctx.saved_tensors
-        g: SparseConvGeometry = ctx.geometry
-        _check_device(g, features, weight, out, grad_out)      # (saved-tensor hooks may have moved them)
-        grad_out = grad_out.contiguous()
-        dtype = _TORCH_TO_TV[features.dtype]
-        stream = current_stream()
-        g.used_on(stream)
-        lib = _capi.lib()
-        grad_in = grad_w = grad_b = None
-        # the gradient passes where the fused ReLU let the output through; its column sums are the
-        # bias gradient (one pass over the gradient for both)
-        rows, k_out = int(grad_out.shape[0]), int(grad_out.shape[1])
-        if ctx.has_bias and ctx.needs_input_grad[2]:
-            grad_b = torch.empty(k_out, dtype=grad_out.dtype, device=grad_out.device)
-            need = int(lib.cumm_hip_column_sum_workspace(rows, k_out))
-            ws = _bytes(need, grad_out.device)
-            if ctx.relu:
-                gated = torch.empty_like(grad_out)
-                _capi.check(lib.cumm_hip_relu_backward_sums(gated.data_ptr(), grad_b.data_ptr(), grad_out.data_ptr(), out.data_ptr(),
-                                                            rows, k_out, dtype, ws.data_ptr(), ws.numel(), stream))
-                grad_out = gated
-            else:
-                _capi.check(lib.cumm_hip_column_sum(grad_b.data_ptr(), grad_out.data_ptr(), rows, k_out, dtype,
-                                                    ws.data_ptr(), ws.numel(), stream))
-        elif ctx.relu:
+        return _backward(ctx.geometry, features, weight, out, grad_out, ctx.needs_input_grad, ctx.relu, ctx.has_bias, ctx.tile_m) + (None, None)
+
+
+def _backward(g: SparseConvGeometry, features, weight, out, grad_out, needed, relu: bool, has_bias: bool, tile_m: int):
+    """The gradients of features, weight and bias (None where not ``needed``)."""
+    _check_device(g, features, weight, out, grad_out)      # (saved-tensor hooks may have moved them)
+    grad_out = grad_out.contiguous()
+    dtype = _TORCH_TO_TV[features.dtype]
+    stream = current_stream()
+    g.used_on(stream)
+    lib = _capi.lib()
+    grad_in = grad_w = grad_b = None
+    # the gradient passes where the fused ReLU let the output through; its column sums are the
+    # bias gradient (one pass over the gradient for both)
+    rows, k_out = int(grad_out.shape[0]), int(grad_out.shape[1])
+    if has_bias and needed[2]:
+        grad_b = torch.empty(k_out, dtype=grad_out.dtype, device=grad_out.device)
+        need = int(lib.cumm_hip_column_sum_workspace(rows, k_out))
+        ws = _bytes(need, grad_out.device)
+        if relu:
             gated = torch.empty_like(grad_out)
-            _capi.check(lib.cumm_hip_relu_backward(gated.data_ptr(), grad_out.data_ptr(), out.data_ptr(),
-                                                   grad_out.numel(), dtype, stream))
+            _capi.check(lib.cumm_hip_relu_backward_sums(gated.data_ptr(), grad_b.data_ptr(), grad_out.data_ptr(), out.data_ptr(),
+                                                        rows, k_out, dtype, ws.data_ptr(), ws.numel(), stream))
             grad_out = gated
-        if ctx.needs_input_grad[0]:
-            # inputs that feed no output site sit in tiles the kernel skips (mask 0): zero them
-            grad_in = torch.empty_like(features) if g.subm else torch.zeros_like(features)
-            roles = {"input": grad_in, "weight": weight, "output": grad_out}
-            key = ("dgrad", dtype, weight.shape)
-            launch = g._launches.get(key)
-            if launch is None:
-                launch = _backward_input_launch(g, key, roles, dtype, stream)
-            launch(stream, **roles)
-        if ctx.needs_input_grad[1] and g.words > 1:
-            # no mask kernel for this pass: the products of all kernel offsets over their pair lists, in
-            # one call (an offset without pairs writes zeros)
-            from .conv import native
-            grad_w = torch.empty_like(weight)
-            key = ("wgrad_pairs", dtype, weight.shape)
-            plan = g._launches.get(key)
-            if plan is None:
-                plan = native.WeightPlan(torch2tensor(grad_out), torch2tensor(features), torch2tensor(grad_w), g._lists, stream)
-                plan.release()      # (every call brings its own tensors)
-                g._launches[key] = plan
-            ws = _bytes(plan.workspace_bytes, grad_out.device)
-            plan.rebind(grad_out.data_ptr(), features.data_ptr(), grad_w.data_ptr(), stream, ws.data_ptr())
-        elif ctx.needs_input_grad[1]:
-            grad_w = torch.empty_like(weight)
-            # torch's switch for reproducible results selects the fixed-order sum of the partial blocks
-            deterministic = bool(torch.are_deterministic_algorithms_enabled())
-            key = ("wgrad", dtype, weight.shape, ctx.tile_m, deterministic)
-            hit = g._launches.get(key)
-            if hit is None:
-                hit = g._launches[key] = _backward_weight_launch(g, key, features, weight, grad_w, grad_out, dtype, stream)
-            launch, need = hit
-            # the workspace comes from torch's caching allocator (the prelude's own would be a
-            # device allocation per call)
-            ws = _bytes(need, grad_out.device)
-            launch(stream, need, input=features, weight=grad_w, output=grad_out, workspace=ws)
-        return grad_in, grad_w, grad_b, None, None
+        else:
+            _capi.check(lib.cumm_hip_column_sum(grad_b.data_ptr(), grad_out.data_ptr(), rows, k_out, dtype,
+                                                ws.data_ptr(), ws.numel(), stream))
+    elif relu:
+        gated = torch.empty_like(grad_out)
+        _capi.check(lib.cumm_hip_relu_backward(gated.data_ptr(), grad_out.data_ptr(), out.data_ptr(),
+                                               grad_out.numel(), dtype, stream))
+        grad_out = gated
+    if needed[0]:
+        # inputs that feed no output site sit in tiles the kernel skips (mask 0): zero them
+        grad_in = torch.empty_like(features) if g.subm else torch.zeros_like(features)
+        roles = {"input": grad_in, "weight": weight, "output": grad_out}
+        key = ("dgrad", dtype, weight.shape)
+        launch = g._own_launches.get(key)
+        if launch is None:
+            launch = _backward_input_launch(g, key, roles, dtype, stream)
+        launch(stream, **roles)
+    if needed[1] and g.words > 1:
+        # no mask kernel for this pass: the products of all kernel offsets over their pair lists, in
+        # one call (an offset without pairs writes zeros)
+        from .conv import native
+        grad_w = torch.empty_like(weight)
+        key = ("wgrad_pairs", dtype, weight.shape)
+        plan = g._own_launches.get(key)
+        if plan is None:
+            plan = native.WeightPlan(torch2tensor(grad_out), torch2tensor(features), torch2tensor(grad_w), g._lists, stream)
+            plan.release()      # (every call brings its own tensors)
+            g._own_launches[key] = plan
+        ws = _bytes(plan.workspace_bytes, grad_out.device)
+        plan.rebind(grad_out.data_ptr(), features.data_ptr(), grad_w.data_ptr(), stream, ws.data_ptr())
+    elif needed[1]:
+        grad_w = torch.empty_like(weight)
+        # torch's switch for reproducible results selects the fixed-order sum of the partial blocks
+        deterministic = bool(torch.are_deterministic_algorithms_enabled())
+        key = ("wgrad", dtype, weight.shape, tile_m, deterministic)
+        hit = g._own_launches.get(key)
+        if hit is None:
+            hit = g._own_launches[key] = _backward_weight_launch(g, key, features, weight, grad_w, grad_out, dtype, stream)
+        launch, need = hit
+        # the workspace comes from torch's caching allocator (the prelude's own would be a
+        # device allocation per call)
+        ws = _bytes(need, grad_out.device)
+        launch(stream, need, input=features, weight=grad_w, output=grad_out, workspace=ws)
+    return grad_in, grad_w, grad_b
 
 
 def _check_device(g: SparseConvGeometry, *tensors) -> None:
@@ -499,7 +528,8 @@ def _forward_launch(g: SparseConvGeometry, key, roles, relu, stream) -> _Launch:
     if known is not None and features.numel() and out.numel():
         launch = known.on(g.n_out, g.n_in, g.n_out, g._ptr["indices_fwd_pos"], g._ptr["mask_fwd"], g._ptr["order_fwd"],
                           g.reduced_address(known.tile_m) if g.words == 1 else None)
-        g._launches[key] = launch
+        g._own_launches[key] = launch
+        _remember(g, key, kind, known, ConvOpType.Forward, features, weight, bias)
         return launch
     p = ConvParams(3, ConvOpType.Forward)
     dtype = _TORCH_TO_TV[features.dtype]
@@ -520,8 +550,8 @@ def _forward_launch(g: SparseConvGeometry, key, roles, relu, stream) -> _Launch:
     if g.words == 1:
         p.mask_output = g.reduced_mask_buffer(int(p.conv_algo_desp.tile_shape[0]))
     ConvMainUnitTest.implicit_gemm2(p)
-    launch = g._launches[key] = _Launch.of(p, roles)
-    _KINDS[kind] = launch
+    launch = g._own_launches[key] = _Launch.of(p, roles)
+    _remember(g, key, kind, launch, ConvOpType.Forward, features, weight, bias)
     return launch
 
 
@@ -531,7 +561,8 @@ def _backward_input_launch(g: SparseConvGeometry, key, roles, dtype, stream) -> 
     known = _KINDS.get(kind)
     if known is not None and grad_in.numel() and grad_out.numel():
         launch = known.on(g.n_in, g.n_in, g.n_out, g._ptr["indices_bwd_pos"], g._ptr["mask_bwd"], g._ptr["order_bwd"], None)
-        g._launches[key] = launch
+        g._own_launches[key] = launch
+        _remember(g, key, kind, known, ConvOpType.BackwardInput, grad_in, weight)
         return launch
     p = ConvParams(3, ConvOpType.BackwardInput)
     p.conv_algo_desp = _desp_like(dtype, ConvOpType.BackwardInput, dynamic=g.words > 1)
@@ -544,8 +575,8 @@ def _backward_input_launch(g: SparseConvGeometry, key, roles, dtype, stream) -> 
     p.stream = stream
     _TUNER.tune_conv(p)
     ConvMainUnitTest.implicit_gemm2(p)
-    launch = g._launches[key] = _Launch.of(p, roles)
-    _KINDS[kind] = launch
+    launch = g._own_launches[key] = _Launch.of(p, roles)
+    _remember(g, key, kind, launch, ConvOpType.BackwardInput, grad_in, weight)
     return launch
 
 
@@ -574,7 +605,8 @@ def _backward_weight_launch(g: SparseConvGeometry, key, features, weight, grad_w
     p.workspace = torch2tensor(ws)
     p.stream = stream
     ConvMainUnitTest.implicit_gemm2(p)
-    launch = _KINDS[kind] = _Launch.of(p, {"input": features, "weight": grad_w, "output": grad_out, "workspace": ws})
+    launch = _Launch.of(p, {"input": features, "weight": grad_w, "output": grad_out, "workspace": ws})
+    _remember(g, key, kind, launch, ConvOpType.BackwardWeight, features, grad_w)
     return launch, need
 
 
@@ -582,6 +614,11 @@ def sparse_conv(features: torch.Tensor, weight: torch.Tensor, bias: Optional[tor
                 geometry: SparseConvGeometry, relu: bool = False) -> torch.Tensor:
     """features [N_in, C], weight [K, kv, C] (f16 / bf16, cuda) -> [N_out, K]; differentiable in
     features, weight and bias."""
+    native = geometry._native
+    if native is not None and not torch._C._are_functorch_transforms_active() and not torch.compiler.is_compiling():
+        out = _native_module.forward(features, weight, bias, geometry, native, bool(relu))
+        if out is not None:
+            return out
     return _SparseConvFunction.apply(features, weight, bias, geometry, relu)
 
 

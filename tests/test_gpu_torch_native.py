@@ -1,0 +1,120 @@
+"""The torch bridge's native calls against its Python function: the same bits, the same refusals, and the parts of
+autograd that a node of one's own has to keep (saved-tensor hooks, version checks, graphs kept and freed,
+gradients nobody asked for, streams)."""
+import pytest
+
+import helpers as H
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+def _setup(ksize=3, strided=False, c=48, k=40, dtype=torch.float16, n=1500, seed=3):
+    from cumm_amd import torch_bridge as tb
+    coords, grid = H.small_cloud(seed, n)
+    geo = tb.SparseConvGeometry(torch.as_tensor(coords, device="cuda"), grid, (ksize,) * 3, (2, 2, 2) if strided else None,
+                                (ksize // 2,) * 3)
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    rnd = lambda *s: (torch.randn(*s, generator=gen, device="cuda") * 0.2).to(dtype)
+    return tb, geo, rnd(geo.n_in, c), rnd(k, ksize ** 3, c), rnd(k), rnd(geo.n_out, k)
+
+
+def _grads(call, x, w, b, g, which=(True, True, True)):
+    leaves = [t.detach().clone().requires_grad_(r) if t is not None else None for t, r in zip((x, w, b), which)]
+    out = call(*leaves)
+    asked = [t for t in leaves if t is not None and t.requires_grad]
+    return (out.detach(),) + torch.autograd.grad(out, asked, g)
+
+
+@pytest.mark.parametrize("ksize,strided,dtype", [(3, False, torch.float16), (3, True, torch.bfloat16), (5, False, torch.bfloat16)])
+@pytest.mark.parametrize("relu", [False, True])
+@pytest.mark.parametrize("with_bias", [False, True])
+def test_same_bits_as_the_python_function(ksize, strided, dtype, relu, with_bias):
+    print("case native", ksize, strided, dtype, relu, with_bias, flush=True)
+    tb, geo, x, w, b, g = _setup(ksize, strided, dtype=dtype)
+    assert geo._native.tables() == {**geo._ptr, **{"reduced_%d" % w: a for w, a in geo._reduced_at.items()}}
+    b = b if with_bias else None
+    python = lambda *t: tb._SparseConvFunction.apply(*t, geo, relu)
+    native = lambda *t: tb._native().forward(*t, geo, geo._native, relu)
+    torch.use_deterministic_algorithms(True, warn_only=True)
+    try:
+        want = _grads(python, x, w, b, g)
+        got = _grads(native, x, w, b, g)
+        assert len(got) == len(want) and all(torch.equal(a, c) for a, c in zip(got, want))
+        # strided operands and gradients; gradients of some only
+        wide = torch.empty(w.shape[0], w.shape[1], 2 * w.shape[2], dtype=w.dtype, device="cuda")[:, :, ::2].copy_(w)
+        got = _grads(native, torch.stack([x, x], 1)[:, 0], wide, b, torch.stack([g, g], 2)[:, :, 1])
+        assert all(torch.equal(a, c) for a, c in zip(got, want))
+        for which in ((True, False, False), (False, True, False), (False, False, True)):
+            if which[2] and not with_bias:
+                continue
+            got = _grads(native, x, w, b, g, which)
+            assert torch.equal(got[1], want[1 + which.index(True)])
+    finally:
+        torch.use_deterministic_algorithms(False)
+    with torch.no_grad():
+        assert not tb.sparse_conv(x.requires_grad_(True), w, b, geo, relu).requires_grad
+
+
+def test_what_autograd_keeps():
+    tb, geo, x, w, b, g = _setup()
+    conv = lambda *t: tb.sparse_conv(*t, geo, True)
+    want = _grads(conv, x, w, b, g)
+    x, w, b = (t.detach().clone().requires_grad_(True) for t in (x, w, b))
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t.data_ptr()) or t.cpu(), lambda t: t.cuda()):
+        out = conv(x, w, b)
+    assert out.grad_fn.name() == "_SparseConvFunctionBackward" and len(packed) == 3
+    got = torch.autograd.grad(out, (x, w, b), g, retain_graph=True)
+    assert all(torch.equal(a, c) for a, c in zip(got[::2], want[1::2]))
+    again = torch.autograd.grad(out, (x, w, b), g)
+    assert torch.equal(again[0], got[0])
+    with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.grad(out, (x, w, b), g)
+    for changed in (lambda o: o.add_(1), lambda o: w.data_ptr() and w.detach().add_(1)):
+        out = conv(x, w, b)
+        with torch.no_grad():
+            changed(out)
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            torch.autograd.grad(out, (x, w, b), g)
+    # a gradient that nobody computed is zero
+    out = conv(x, w, b)
+    zero = torch.autograd.grad(out, (x, w, b), torch.zeros_like(out))
+    assert all(not t.any() for t in zero)
+
+
+def test_what_is_left_to_python():
+    import torch.autograd.forward_ad as fwad
+    tb, geo, x, w, b, g = _setup()
+    tb.sparse_conv(x, w, b, geo)
+    native = lambda *t: tb._native().forward(*t, geo, geo._native, False)
+    assert native(x, w, b) is not None
+    assert native(x[:-1], w, b) is None and native(x, w[:, :26], b) is None and native(x, w, b[:-1]) is None
+    assert native(x.cpu(), w, b) is None and native(x.float(), w, b) is None and native(x, w.bfloat16(), b) is None
+    assert native(x[:, :0], w[:, :, :0], b) is None
+    with fwad.dual_level():
+        dual = fwad.make_dual(x, torch.ones_like(x))
+        assert native(dual, w, b) is None
+        with pytest.raises(Exception):
+            tb.sparse_conv(dual, w, b, geo)
+    with pytest.raises(Exception):
+        torch.func.vmap(lambda t: tb.sparse_conv(t, w, b, geo))(torch.stack([x, x]))
+    with pytest.raises(ValueError):
+        tb.sparse_conv(x[:-1], w, b, geo)
+    with pytest.raises(ValueError):
+        tb.sparse_conv(x, w.cpu(), b, geo)
+
+
+def test_on_another_stream_and_after_the_geometry():
+    tb, geo, x, w, b, g = _setup()
+    conv = lambda *t: tb.sparse_conv(*t, geo, True)
+    want = _grads(conv, x, w, b, g)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    x, w, b = (t.detach().clone().requires_grad_(True) for t in (x, w, b))
+    with torch.cuda.stream(stream):
+        out = conv(x, w, b)
+        del geo
+        got = torch.autograd.grad(out, (x, w, b), g)
+    stream.synchronize()
+    assert torch.equal(out.detach(), want[0]) and torch.equal(got[0], want[1]) and torch.equal(got[2], want[3])
