@@ -122,7 +122,7 @@ hipError_t launch_conv_pairs_sort(const ConvPairsParams &p, unsigned long long m
                                   int32_t *give_ups, hipStream_t s);
 hipError_t launch_conv_pairs_fill(const ConvPairsParams &p, hipStream_t s);
 size_t conv_pairs_scan_temp_bytes(size_t n_words);
-hipError_t launch_conv_pairs_bits(const ConvPairsParams &p, void *temp, size_t temp_bytes, hipStream_t s);
+hipError_t launch_conv_pairs_bits(const ConvPairsParams &p, void *temp, size_t temp_bytes, uint32_t *host_total, hipStream_t s);
 // What input preparation knows about a sorted mask array and a later forward / backward-input
 // launch on the same array can use without being told: a table of kLightHintSlots slots of eight
 // words in device memory, one table per GPU, indexed by a hash of the array's address.  Slot =

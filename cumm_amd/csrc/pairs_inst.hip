@@ -532,7 +532,8 @@ __global__ __launch_bounds__(256) void bit_scan_block_offsets_kernel(uint32_t *_
 // DIRECT: block_sums are counts, else offsets
 template <bool DIRECT>
 __global__ __launch_bounds__(256) void bit_scan_write_kernel(const uint32_t *__restrict__ bits, unsigned long long n_words,
-                                                             const uint32_t *__restrict__ block_sums, uint32_t *__restrict__ prefix) {
+                                                             const uint32_t *__restrict__ block_sums, uint32_t *__restrict__ prefix,
+                                                             uint32_t *host_total) {
   __shared__ uint32_t lds_waves[4];
   // thread t owns four consecutive words (so that its own scan is a running sum)
   const unsigned long long first = (unsigned long long)blockIdx.x * kScanBlock + threadIdx.x * 4u;
@@ -546,6 +547,9 @@ __global__ __launch_bounds__(256) void bit_scan_write_kernel(const uint32_t *__r
     base = block_sums[blockIdx.x];
   }
   const uint32_t excl = block_exclusive_scan((uint32_t)(c.x + c.y + c.z + c.w), lds_waves, &total);
+  // (the host waits for the total: it goes out before anything else is written)
+  if (host_total != nullptr && blockIdx.x == gridDim.x - 1 && threadIdx.x == 0)
+    __hip_atomic_store(host_total, base + total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   const int run = (int)(base + excl);
   if (first < n_words) *reinterpret_cast<v4i *>(prefix + first) = v4i{run, run + c.x, run + c.x + c.y, run + c.x + c.y + c.z};
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) prefix[n_words] = base + total;
@@ -872,8 +876,8 @@ size_t conv_pairs_scan_temp_bytes(size_t n_words) {
   return 4 * ((n_words + kScanBlock - 1) / kScanBlock + 1);
 }
 
-// bitmap of the active output sites and its prefix sums
-hipError_t launch_conv_pairs_bits(const ConvPairsParams &p, void *temp, size_t temp_bytes, hipStream_t s) {
+// bitmap of the active output sites, its prefix sums and, in host memory, their total
+hipError_t launch_conv_pairs_bits(const ConvPairsParams &p, void *temp, size_t temp_bytes, uint32_t *host_total, hipStream_t s) {
   unsigned long long wgs = (p.n_words / 4 + 255ull) / 256ull;
   if (wgs > 16384ull) wgs = 16384ull;
   if (wgs == 0ull) wgs = 1ull;
@@ -887,10 +891,12 @@ hipError_t launch_conv_pairs_bits(const ConvPairsParams &p, void *temp, size_t t
   uint32_t *block_sums = reinterpret_cast<uint32_t *>(temp);
   hipLaunchKernelGGL(bit_scan_block_sums_kernel, dim3((unsigned)n_blocks), dim3(256), 0, s, p.bits, p.n_words, block_sums);
   if (n_blocks <= kScanDirect) {
-    hipLaunchKernelGGL(bit_scan_write_kernel<true>, dim3((unsigned)n_blocks), dim3(256), 0, s, p.bits, p.n_words, block_sums, p.prefix);
+    hipLaunchKernelGGL(bit_scan_write_kernel<true>, dim3((unsigned)n_blocks), dim3(256), 0, s, p.bits, p.n_words, block_sums, p.prefix,
+                       host_total);
   } else {
     hipLaunchKernelGGL(bit_scan_block_offsets_kernel, dim3(1), dim3(256), 0, s, block_sums, n_blocks);
-    hipLaunchKernelGGL(bit_scan_write_kernel<false>, dim3((unsigned)n_blocks), dim3(256), 0, s, p.bits, p.n_words, block_sums, p.prefix);
+    hipLaunchKernelGGL(bit_scan_write_kernel<false>, dim3((unsigned)n_blocks), dim3(256), 0, s, p.bits, p.n_words, block_sums, p.prefix,
+                       host_total);
   }
   return hipGetLastError();
 }
