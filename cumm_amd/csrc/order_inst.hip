@@ -19,14 +19,18 @@
 //     end, from which the convolution kernels start: a launch ends with its longest tile otherwise.
 //     5 x 5 x 5 on 120 k voxels: 47 k (tile, offset) steps against 87 k in the order by count and hash, 46 k
 //     without the weight, but forward 74.8 -> 66.1 us, backward-input 74.8 -> 65.8.
-// Chain of kernels: clear - masks, keys and both histograms - two passes - position.  The passes are the
-// single-sweep kind (ticket, ranks by ballot, look-back, scatter; stable); they are bound by their
-// dependent round trips at 10^5 positions and by memory at 10^6; chunks of half the size on twice the
-// workgroups: 17.5 for 17.7 us at 300 k positions, 31.1 for 23.2 at 1.1 M.  The mask kernel reads the
-// tables at 4.2 TB/s.  The position kernel writes them again; what it fetches by row is little more
-// than a word pair per position (51.5 -> 39.1 us at 1.1 M positions against a fetch of mask and entries).
+// Chain of kernels: masks, keys and the digits' counts per block of 512 positions - sums of the counts over
+// the blocks - two passes - position.  The first pass knows every chunk's place from the sums, the second
+// looks back (ticket, flagged words); both rank by ballot and are stable.  (Instead of a kernel that clears,
+// counts by device-wide atomics and look-backs in both passes: a pass over 447 k positions of two tables 21.2 ->
+// 15.9 us, over 120 k 13.2 -> 9.6, the sums 5 - 7 us for 3 - 4 of clearing.  Each pass adding up the counts by itself
+// took the 6 us back; look-back words alone are not what a pass waits for.)  Chunks of half the size on
+// twice the workgroups: 17.5 for 17.7 us at 300 k positions, 31.1 for 23.2 at 1.1 M.  The mask kernel reads the
+// tables at 4.4 TB/s (1024 positions per workgroup 35.7 for 27.2 us at 1.1 M).  The position kernel writes them
+// again; what it fetches by row is little more than a word pair per position (51.5 -> 39.1 us at 1.1 M positions
+// against a fetch of mask and entries).
 // Measured (kernel times): the tables of a frame of 120 k voxels - submanifold and stride 2, 326 k output
-// sites - 120 us in ten launches; with masks by atomics, a sort each and a gather of every entry it
+// sites - 105 us in ten launches; with masks by atomics, a sort each and a gather of every entry it
 // was 305 us in 27.
 #include <cstring>
 
@@ -41,7 +45,8 @@ constexpr int kDigit = 9, kDigitBins = 1 << kDigit;      // 512
 constexpr int kKeyBits = 2 * kDigit;
 constexpr int kPassThreads = 1024, kPassWaves = kPassThreads / 64;
 constexpr int kMaskBatch = 16;                            // table rows whose loads are in flight together
-constexpr int kHistCopies = 8;                            // spread of the histogram atomics
+constexpr int kBlock = 512;                               // positions per workgroup of the masks kernel
+constexpr int kScanRows = 48;                             // blocks per thread and trip of the scan
 constexpr int kExact = 5;                                 // offsets up to which a one-word key is exact
 constexpr uint32_t kAggregate = 1u << 30, kInclusive = 2u << 30, kCount = (1u << 30) - 1u;
 constexpr int kSpins = 1 << 20;                           // (about a second)
@@ -53,9 +58,11 @@ struct Side {
   uint32_t *keys;              // [n]
   int32_t *tmp_rows;           // [n] after the first pass
   uint16_t *tmp_high;          // [n]
-  uint32_t *hist;              // [2][kHistCopies][kDigitBins]
-  uint32_t *state;             // [2][chunks][kDigitBins] look-back words
-  uint32_t *tickets;           // [2]
+  uint32_t *counts[2];         // per pass [rows + 1][kDigitBins]: keys per digit and block of positions, then
+                               // the same of the blocks before it, and at the end of all
+  int32_t rows;                // blocks
+  uint32_t *state;             // [chunks][kDigitBins] look-back words of the second pass
+  uint32_t *ticket;
   uint32_t *sorted;            // [n, words]
   int32_t *order;              // [n]
   int32_t *by_pos, *by_pos_rev;   // [kv, n]; the second, with its offsets reversed, may be NULL
@@ -65,6 +72,7 @@ struct Side {
 struct OrderParams {
   Side side[2];
   int32_t sides, kv, words, pass;
+  int32_t rows_per_chunk;
   int32_t *give_ups;
   uint32_t base[kExact + 2];   // first key of the words with c offsets; [kExact + 1]: of those with more
   uint32_t share;              // keys per number of offsets above kExact
@@ -73,18 +81,6 @@ struct OrderParams {
   uint32_t planes[12][4];
   uint32_t filter;
 };
-
-__global__ __launch_bounds__(256) void order_clear_kernel(const OrderParams p) {
-  const int i0 = blockIdx.x * 256 + threadIdx.x, step = gridDim.x * 256;
-  for (int s = 0; s < p.sides; ++s) {
-    const Side &d = p.side[s];
-    for (int i = i0; i < 2 * kHistCopies * kDigitBins; i += step) d.hist[i] = 0u;
-    for (int i = i0; i < 2 * d.chunks * kDigitBins; i += step) d.state[i] = 0u;
-    if (i0 < 2) d.tickets[i0] = 0u;
-    if (i0 < 8 && d.hint_slot != nullptr)   // names no array yet; the two counts start at "everything" / "nothing"
-      d.hint_slot[i0] = i0 == 4 ? (d.n / 128) * 128 : (i0 == 5 ? ((d.n + 63) / 64) * 64 : 0);
-  }
-}
 
 // rank of a word among those with as many bits, ascending value: sum of C(position of the i-th bit, i)
 __device__ __forceinline__ uint32_t word_key(const OrderParams &p, uint32_t m) {
@@ -152,22 +148,32 @@ __device__ __forceinline__ int side_of(int first, int *block) {
 }
 
 // One position per lane: its mask out of the table (every row read coalesced, kv independent loads), its
-// key, the entry of its lowest offset, and the digits of the key into the histograms of both passes.
+// key, the entry of its lowest offset, and how many of the block's keys have which digit, for both
+// passes.  A block's counts are a row of its own, so that nothing has to be zero before.  (Eight positions
+// per lane, one after the other: fewer rows, but 55 us for 27 at 1.1 M positions.)
 template <int WORDS>
-__global__ __launch_bounds__(256) void order_masks_kernel(const OrderParams p) {
+__global__ __launch_bounds__(kBlock) void order_masks_kernel(const OrderParams p) {
   __shared__ uint32_t hist[2][kDigitBins];
   const int t = threadIdx.x, lane = t & 63;
   int block = blockIdx.x;
-  const Side &d = p.side[side_of((p.side[0].n + 255) / 256, &block)];
-  for (int i = t; i < 2 * kDigitBins; i += 256) (&hist[0][0])[i] = 0u;
-  const int o = block * 256 + t;
+  const Side &d = p.side[side_of(p.side[0].rows, &block)];
+  static_assert(kBlock == kDigitBins, "a thread per digit");
+  hist[0][t] = hist[1][t] = 0u;
+  if (block % p.rows_per_chunk == 0) d.state[(size_t)(block / p.rows_per_chunk) * kDigitBins + t] = 0u;
+  if (block == 0) {
+    if (t == 0) *d.ticket = 0u;
+    if (t < 8 && d.hint_slot != nullptr)   // names no array yet; the two counts start at "everything" / "nothing"
+      d.hint_slot[t] = t == 4 ? (d.n / 128) * 128 : (t == 5 ? ((d.n + 63) / 64) * 64 : 0);
+  }
+  __syncthreads();
+  // (kv * n entries are below 2^31 bytes: the row of the table is a scalar offset)
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t *>(d.indices), 0,
+                                                                      (int)((uint32_t)p.kv * (uint32_t)d.n * 4u), 0x00020000);
+  const int o = block * kBlock + t;
   const bool on = o < d.n;
   uint32_t w[4] = {0u, 0u, 0u, 0u};
   uint32_t lead = 0u;
   bool self = false;
-  // (kv * n entries are below 2^31 bytes: the row of the table is a scalar offset)
-  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t *>(d.indices), 0,
-                                                                      (int)((uint32_t)p.kv * (uint32_t)d.n * 4u), 0x00020000);
   const uint32_t at = (uint32_t)(on ? o : 0) * 4u;
 #pragma unroll
   for (int q = 0; q < WORDS; ++q) {
@@ -197,7 +203,6 @@ __global__ __launch_bounds__(256) void order_masks_kernel(const OrderParams p) {
     }
     d.keys[o] = key;
   }
-  __syncthreads();
   // most waves of a sparse cloud hold one key: one add for all lanes
   const unsigned long long live = __ballot(on);
   if (live != 0ull) {
@@ -210,16 +215,58 @@ __global__ __launch_bounds__(256) void order_masks_kernel(const OrderParams p) {
     }
   }
   __syncthreads();
-  for (int i = t; i < 2 * kDigitBins; i += 256) {
-    const uint32_t c = (&hist[0][0])[i];
-    if (c) atomicAdd(&d.hist[((i >> kDigit) * kHistCopies + (block & (kHistCopies - 1))) * kDigitBins + (i & (kDigitBins - 1))], c);
+  d.counts[0][(size_t)block * kDigitBins + t] = hist[0][t];
+  d.counts[1][(size_t)block * kDigitBins + t] = hist[1][t];
+}
+
+// Counts -> sums over the blocks before, and the totals behind the last.  A workgroup takes 16 digits of one
+// pass and table in 64 runs of blocks, 48 blocks of each at a time (one trip up to 1.5 M positions).  (Rows past a
+// run's end are fetched outside the matrix: as conditional loads each waited for the one before, 18 us for 5.)
+__global__ __launch_bounds__(1024) void order_scan_kernel(const OrderParams p) {
+  __shared__ uint32_t run_sum[64][16];
+  const int digit = threadIdx.x & 15, run = threadIdx.x >> 4;
+  const Side &d = p.side[blockIdx.y >> 1];
+  const __amdgpu_buffer_rsrc_t rs =
+      __builtin_amdgcn_make_buffer_rsrc(d.counts[blockIdx.y & 1], 0, (int)((uint32_t)(d.rows + 1) * (kDigitBins * 4u)), 0x00020000);
+  const uint32_t col = (uint32_t)(blockIdx.x * 16 + digit) * 4u;
+  const int per = (d.rows + 63) / 64, r0 = run * per, r1 = r0 + per < d.rows ? r0 + per : d.rows;
+  const auto at = [&](int r) -> uint32_t { return r < r1 ? (uint32_t)r * (kDigitBins * 4u) + col : 0x80000000u; };
+  uint32_t v[kScanRows], sum = 0;
+  for (int t0 = 0; t0 < per; t0 += kScanRows) {
+#pragma unroll
+    for (int u = 0; u < kScanRows; ++u) v[u] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, t0 + u < per ? at(r0 + t0 + u) : 0x80000000u, 0, 0);
+#pragma unroll
+    for (int u = 0; u < kScanRows; ++u) sum += v[u];
   }
+  run_sum[run][digit] = sum;
+  __syncthreads();
+  uint32_t before = 0, all = 0;
+#pragma unroll 16
+  for (int i = 0; i < 64; ++i) {
+    const uint32_t x = run_sum[i][digit];
+    before += i < run ? x : 0u;
+    all += x;
+  }
+  for (int t0 = 0; t0 < per; t0 += kScanRows) {
+    if (per > kScanRows) {
+#pragma unroll
+      for (int u = 0; u < kScanRows; ++u) v[u] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, t0 + u < per ? at(r0 + t0 + u) : 0x80000000u, 0, 0);
+    }
+#pragma unroll
+    for (int u = 0; u < kScanRows; ++u) {
+      __builtin_amdgcn_raw_buffer_store_b32((int)before, rs, t0 + u < per ? at(r0 + t0 + u) : 0x80000000u, 0, 0);
+      before += v[u];
+    }
+  }
+  if (run == 0) __builtin_amdgcn_raw_buffer_store_b32((int)all, rs, (uint32_t)d.rows * (kDigitBins * 4u) + col, 0, 0);
 }
 
 // One pass over one digit (0: the low one, rows in ascending order to tmp; 1: the high one, tmp to
-// order).  A workgroup takes the next chunk by ticket (its predecessors have then started), ranks
-// its keys per digit in position order, publishes its counts, adds up those of the chunks before it and
-// scatters.  Words carry flag and value: relaxed device-scope accesses do.
+// order).  A workgroup ranks the keys of a chunk per digit in position order and scatters them.  Where a
+// chunk's keys of a digit begin: in the first pass the blocks' counts say it; in the second, whose chunks are
+// made by the first, a workgroup takes the next chunk by ticket (its predecessors have then started),
+// publishes its counts and adds up those of the chunks before it.  Words carry flag and value: relaxed
+// device-scope accesses do.
 template <int ITEMS>
 __global__ __launch_bounds__(kPassThreads) void order_pass_kernel(const OrderParams p) {
   constexpr int kChunk = kPassThreads * ITEMS;
@@ -231,16 +278,18 @@ __global__ __launch_bounds__(kPassThreads) void order_pass_kernel(const OrderPar
   int block = blockIdx.x;
   const Side &d = p.side[side_of(p.side[0].chunks, &block)];
   const bool low = p.pass == 0;
-  if (t == 0) chunk_of_block = (int)atomicAdd(&d.tickets[p.pass], 1u);
-  // keys per bin of the whole input (thread = bin), while the ticket is on its way
-  uint32_t total = 0;
-  if (t < kDigitBins) {
-#pragma unroll
-    for (int c = 0; c < kHistCopies; ++c) total += d.hist[(p.pass * kHistCopies + c) * kDigitBins + t];
-  }
+  int chunk = block;
+  if (!low && t == 0) chunk_of_block = (int)atomicAdd(d.ticket, 1u);
   for (int i = t; i < kPassWaves * kDigitBins; i += kPassThreads) (&wave_hist[0][0])[i] = 0u;
+  // keys per bin of the whole input and (first pass) of the chunks before this one
+  uint32_t total = 0, earlier = 0;
+  if (t < kDigitBins) {
+    const uint32_t *c = d.counts[p.pass] + t;
+    total = c[(size_t)d.rows * kDigitBins];
+    earlier = c[(size_t)(block * p.rows_per_chunk) * kDigitBins];
+  }
   __syncthreads();
-  const int chunk = chunk_of_block;
+  if (!low) chunk = chunk_of_block;
   if (chunk >= d.chunks) return;      // (never: one workgroup per chunk)
   // wave w owns positions [base, base + 64 ITEMS), item u of lane l is position base + 64 u + l
   const int64_t base = (int64_t)chunk * kChunk + (int64_t)wave * (64 * ITEMS);
@@ -298,11 +347,12 @@ __global__ __launch_bounds__(kPassThreads) void order_pass_kernel(const OrderPar
       wave_hist[w][t] = count;
       count += c;
     }
-    uint32_t *state = d.state + (size_t)p.pass * d.chunks * kDigitBins;
-    __hip_atomic_store(&state[(size_t)chunk * kDigitBins + t], (chunk == 0 ? kInclusive : kAggregate) | count, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-    uint32_t before = 0;
-    if (chunk > 0) {
+    uint32_t before = low ? earlier : 0u;
+    uint32_t *state = d.state;
+    if (!low)
+      __hip_atomic_store(&state[(size_t)chunk * kDigitBins + t], (chunk == 0 ? kInclusive : kAggregate) | count, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    if (!low && chunk > 0) {
       constexpr int kLook = 32;      // words per round trip
       bool done = false, gave_up = false;
       int j = chunk - 1, spins = 0;
@@ -441,14 +491,15 @@ __global__ __launch_bounds__(256) void order_position_kernel(const OrderParams p
 size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
 // chunks of 4096 positions up to 2^18 (few chunks: a pass is as long as one chunk's chain), 8192 above
 int pass_items(int n) { return n <= (1 << 18) ? 4 : 8; }
+int mask_rows(int n) { return (int)(((int64_t)n + kBlock - 1) / kBlock); }
 
 }  // namespace
 
 size_t order_pairs_workspace_bytes(int n, int words) {
   const size_t nn = (size_t)(n > 0 ? n : 1);
   const size_t chunks = (nn + 4095) / 4096;
-  return up256(4 * nn * (words == 1 ? 2 : words)) + 2 * up256(4 * nn) + up256(2 * nn) + up256(4 * 2 * kHistCopies * kDigitBins) +
-         up256(4 * 2 * chunks * kDigitBins) + 256;
+  return up256(4 * nn * (words == 1 ? 2 : words)) + 2 * up256(4 * nn) + up256(2 * nn) + 2 * up256(4 * ((size_t)mask_rows((int)nn) + 1) * kDigitBins) +
+         up256(4 * chunks * kDigitBins) + 256;
 }
 
 hipError_t launch_order_pairs(const OrderPairsSide *sides, int n_sides, int kv, const int32_t *ksize, void *workspace,
@@ -463,6 +514,7 @@ hipError_t launch_order_pairs(const OrderPairsSide *sides, int n_sides, int kv, 
   for (int i = 0; i < n_sides; ++i)
     if (sides[i].n > 0 && sides[i].n > most) most = sides[i].n;
   const int items = pass_items(most), chunk = kPassThreads * items;
+  p.rows_per_chunk = chunk / kBlock;
   for (int i = 0; i < n_sides; ++i) {
     if (sides[i].n <= 0) continue;
     Side &d = p.side[p.sides++];
@@ -475,9 +527,10 @@ hipError_t launch_order_pairs(const OrderPairsSide *sides, int n_sides, int kv, 
     d.keys = reinterpret_cast<uint32_t *>(take(4 * n));
     d.tmp_rows = reinterpret_cast<int32_t *>(take(4 * n));
     d.tmp_high = reinterpret_cast<uint16_t *>(take(2 * n));
-    d.hist = reinterpret_cast<uint32_t *>(take(4 * 2 * kHistCopies * kDigitBins));
-    d.state = reinterpret_cast<uint32_t *>(take(4 * 2 * (size_t)d.chunks * kDigitBins));
-    d.tickets = reinterpret_cast<uint32_t *>(take(256));
+    d.rows = mask_rows(d.n);
+    for (uint32_t *&c : d.counts) c = reinterpret_cast<uint32_t *>(take(4 * ((size_t)d.rows + 1) * kDigitBins));
+    d.state = reinterpret_cast<uint32_t *>(take(4 * (size_t)d.chunks * kDigitBins));
+    d.ticket = reinterpret_cast<uint32_t *>(take(256));
     at = begin + order_pairs_workspace_bytes(d.n, p.words);
   }
   if (p.sides == 0) return hipSuccess;
@@ -513,14 +566,15 @@ hipError_t launch_order_pairs(const OrderPairsSide *sides, int n_sides, int kv, 
     blocks += (p.side[i].n + 255) / 256;
     chunks += p.side[i].chunks;
   }
-  const int clear = 2 * chunks * kDigitBins / 256;
-  hipLaunchKernelGGL(order_clear_kernel, dim3(clear > 1024 ? 1024 : clear), dim3(256), 0, s, p);
+  int rows = 0;
+  for (int i = 0; i < p.sides; ++i) rows += p.side[i].rows;
   switch (p.words) {
-  case 1: hipLaunchKernelGGL(order_masks_kernel<1>, dim3(blocks), dim3(256), 0, s, p); break;
-  case 2: hipLaunchKernelGGL(order_masks_kernel<2>, dim3(blocks), dim3(256), 0, s, p); break;
-  case 3: hipLaunchKernelGGL(order_masks_kernel<3>, dim3(blocks), dim3(256), 0, s, p); break;
-  default: hipLaunchKernelGGL(order_masks_kernel<4>, dim3(blocks), dim3(256), 0, s, p); break;
+  case 1: hipLaunchKernelGGL(order_masks_kernel<1>, dim3(rows), dim3(kBlock), 0, s, p); break;
+  case 2: hipLaunchKernelGGL(order_masks_kernel<2>, dim3(rows), dim3(kBlock), 0, s, p); break;
+  case 3: hipLaunchKernelGGL(order_masks_kernel<3>, dim3(rows), dim3(kBlock), 0, s, p); break;
+  default: hipLaunchKernelGGL(order_masks_kernel<4>, dim3(rows), dim3(kBlock), 0, s, p); break;
   }
+  hipLaunchKernelGGL(order_scan_kernel, dim3(kDigitBins / 16, 2 * p.sides), dim3(1024), 0, s, p);
   for (p.pass = 0; p.pass < 2; ++p.pass) {
     if (items == 4) hipLaunchKernelGGL(order_pass_kernel<4>, dim3(chunks), dim3(kPassThreads), 0, s, p);
     else hipLaunchKernelGGL(order_pass_kernel<8>, dim3(chunks), dim3(kPassThreads), 0, s, p);

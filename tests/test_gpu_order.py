@@ -95,3 +95,20 @@ def test_a_tile_has_as_few_offsets_as_in_the_exact_order():
             w = np.bitwise_or.reduce(pad.reshape(-1, 64, s.shape[1]), axis=1)
             return sum(bin(int(v)).count("1") for v in w.ravel())
         assert steps(g["order"]) <= steps(other) * 1.01 + 2
+
+
+@pytest.mark.parametrize("n,n2", [(511, 513), (512 * 64, 512 * 64 + 1), (512 * 64 * 48 - 1, 40), (512 * 64 * 48 + 513, 600000)])
+def test_counts_of_many_blocks(n, n2):
+    """The digits' counts per block of 512 positions, summed in runs of blocks: a block, a run, and more blocks
+    than one trip takes; exact and stable up to five offsets."""
+    print("case order blocks", n, n2, flush=True)
+    rng = np.random.default_rng(n)
+    tables = [np.where(rng.random((8, m)) < 0.3, np.int32(3), np.int32(-1)) for m in (n, n2)]
+    got, _ = _order(tables, (2, 2, 2), reverse=False)
+    for t, g in zip(tables, got):
+        m = pairs.masks_from_pairs(t)[:, 0].astype(np.int64)
+        count = np.array([bin(v).count("1") for v in range(256)])[m]
+        light = count <= 5
+        want = np.lexsort((m, count))
+        assert np.array_equal(g["order"][: int(light.sum())], want[: int(light.sum())])
+        assert np.array_equal(np.sort(g["order"]), np.arange(len(m))) and np.array_equal(g["mask"][:, 0], m[g["order"]])
