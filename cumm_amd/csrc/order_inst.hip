@@ -22,15 +22,15 @@
 // Chain of kernels: masks, keys and the digits' counts per block of 512 positions - sums of the counts over
 // the blocks - two passes - position.  The first pass knows every chunk's place from the sums, the second
 // looks back (ticket, flagged words); both rank by ballot and are stable.  (Instead of a kernel that clears,
-// counts by device-wide atomics and look-backs in both passes: a pass over 447 k positions of two tables 21.2 ->
-// 15.9 us, over 120 k 13.2 -> 9.6, the sums 5 - 7 us for 3 - 4 of clearing.  Each pass adding up the counts by itself
-// took the 6 us back; look-back words alone are not what a pass waits for.)  Chunks of half the size on
-// twice the workgroups: 17.5 for 17.7 us at 300 k positions, 31.1 for 23.2 at 1.1 M.  The mask kernel reads the
-// tables at 4.4 TB/s (1024 positions per workgroup 35.7 for 27.2 us at 1.1 M).  The position kernel writes them
-// again; what it fetches by row is little more than a word pair per position (51.5 -> 39.1 us at 1.1 M positions
-// against a fetch of mask and entries).
+// counts by device-wide atomics and look-backs in both passes.  The first pass can then be cut as finely as
+// the device is wide: 1024 positions per workgroup, over 447 k positions of two tables 21.2 -> 7.1 us, over
+// 120 k 13.2 -> 4.8; the second 21.2 -> 15.2, 13.2 -> 11.4; the sums 5 - 7 us for 3 - 4 of clearing.  Each pass
+// adding up the counts by itself instead took 6 us back.)  The mask kernel reads the tables at 4.4 TB/s (1024
+// positions per workgroup 35.7 for 27.2 us at 1.1 M).  The position kernel writes them again; what it fetches by
+// row is little more than a word pair per position (51.5 -> 39.1 us at 1.1 M positions against a fetch of mask
+// and entries).
 // Measured (kernel times): the tables of a frame of 120 k voxels - submanifold and stride 2, 326 k output
-// sites - 105 us in ten launches; with masks by atomics, a sort each and a gather of every entry it
+// sites - 95 us in ten launches; with masks by atomics, a sort each and a gather of every entry it
 // was 305 us in 27.
 #include <cstring>
 
@@ -71,7 +71,7 @@ struct Side {
 
 struct OrderParams {
   Side side[2];
-  int32_t sides, kv, words, pass;
+  int32_t sides, kv, words;
   int32_t rows_per_chunk;
   int32_t *give_ups;
   uint32_t base[kExact + 2];   // first key of the words with c offsets; [kExact + 1]: of those with more
@@ -261,13 +261,13 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const OrderParams p) {
   if (run == 0) __builtin_amdgcn_raw_buffer_store_b32((int)all, rs, (uint32_t)d.rows * (kDigitBins * 4u) + col, 0, 0);
 }
 
-// One pass over one digit (0: the low one, rows in ascending order to tmp; 1: the high one, tmp to
+// One pass over one digit (LOW: the low one, rows in ascending order to tmp; else the high one, tmp to
 // order).  A workgroup ranks the keys of a chunk per digit in position order and scatters them.  Where a
 // chunk's keys of a digit begin: in the first pass the blocks' counts say it; in the second, whose chunks are
 // made by the first, a workgroup takes the next chunk by ticket (its predecessors have then started),
 // publishes its counts and adds up those of the chunks before it.  Words carry flag and value: relaxed
 // device-scope accesses do.
-template <int ITEMS>
+template <int ITEMS, bool LOW>
 __global__ __launch_bounds__(kPassThreads) void order_pass_kernel(const OrderParams p) {
   constexpr int kChunk = kPassThreads * ITEMS;
   __shared__ uint32_t wave_hist[kPassWaves][kDigitBins];
@@ -276,21 +276,21 @@ __global__ __launch_bounds__(kPassThreads) void order_pass_kernel(const OrderPar
   __shared__ int chunk_of_block;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   int block = blockIdx.x;
-  const Side &d = p.side[side_of(p.side[0].chunks, &block)];
-  const bool low = p.pass == 0;
+  const auto chunks_of = [](const Side &side) { return LOW ? (side.n + kChunk - 1) / kChunk : side.chunks; };
+  const Side &d = p.side[side_of(chunks_of(p.side[0]), &block)];
   int chunk = block;
-  if (!low && t == 0) chunk_of_block = (int)atomicAdd(d.ticket, 1u);
+  if (!LOW && t == 0) chunk_of_block = (int)atomicAdd(d.ticket, 1u);
   for (int i = t; i < kPassWaves * kDigitBins; i += kPassThreads) (&wave_hist[0][0])[i] = 0u;
   // keys per bin of the whole input and (first pass) of the chunks before this one
   uint32_t total = 0, earlier = 0;
   if (t < kDigitBins) {
-    const uint32_t *c = d.counts[p.pass] + t;
+    const uint32_t *c = d.counts[LOW ? 0 : 1] + t;
     total = c[(size_t)d.rows * kDigitBins];
-    earlier = c[(size_t)(block * p.rows_per_chunk) * kDigitBins];
+    if constexpr (LOW) earlier = c[(size_t)(block * (kChunk / kBlock)) * kDigitBins];
   }
   __syncthreads();
-  if (!low) chunk = chunk_of_block;
-  if (chunk >= d.chunks) return;      // (never: one workgroup per chunk)
+  if constexpr (!LOW) chunk = chunk_of_block;
+  if (chunk >= chunks_of(d)) return;      // (never: one workgroup per chunk)
   // wave w owns positions [base, base + 64 ITEMS), item u of lane l is position base + 64 u + l
   const int64_t base = (int64_t)chunk * kChunk + (int64_t)wave * (64 * ITEMS);
   uint32_t digit[ITEMS], high[ITEMS];
@@ -300,7 +300,7 @@ __global__ __launch_bounds__(kPassThreads) void order_pass_kernel(const OrderPar
   for (int u = 0; u < ITEMS; ++u) {
     const int64_t pos = base + u * 64 + lane;
     const int64_t at = pos < d.n ? pos : d.n - 1;
-    if (low) {
+    if constexpr (LOW) {
       const uint32_t key = d.keys[at];
       digit[u] = key & (kDigitBins - 1);
       high[u] = key >> kDigit;
@@ -347,12 +347,12 @@ __global__ __launch_bounds__(kPassThreads) void order_pass_kernel(const OrderPar
       wave_hist[w][t] = count;
       count += c;
     }
-    uint32_t before = low ? earlier : 0u;
+    uint32_t before = LOW ? earlier : 0u;
     uint32_t *state = d.state;
-    if (!low)
+    if (!LOW)
       __hip_atomic_store(&state[(size_t)chunk * kDigitBins + t], (chunk == 0 ? kInclusive : kAggregate) | count, __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_AGENT);
-    if (!low && chunk > 0) {
+    if (!LOW && chunk > 0) {
       constexpr int kLook = 32;      // words per round trip
       bool done = false, gave_up = false;
       int j = chunk - 1, spins = 0;
@@ -392,7 +392,7 @@ __global__ __launch_bounds__(kPassThreads) void order_pass_kernel(const OrderPar
     if (base + u * 64 + lane < d.n) {
       const uint32_t dst = bin_base[digit[u]] + wave_hist[wave][digit[u]] + rank[u];
       if (dst < (uint32_t)d.n) {      // (always, unless a look-back gave up)
-        if (low) {
+        if constexpr (LOW) {
           d.tmp_rows[dst] = row[u];
           d.tmp_high[dst] = (uint16_t)high[u];
         } else {
@@ -489,7 +489,8 @@ __global__ __launch_bounds__(256) void order_position_kernel(const OrderParams p
 }
 
 size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
-// chunks of 4096 positions up to 2^18 (few chunks: a pass is as long as one chunk's chain), 8192 above
+// chunks of the second pass: 4096 positions up to 2^18 (few chunks: it is as long as one chunk's chain), 8192
+// above (120 k positions: 11.4 us, with 1024 12.7, 8192 14.2; 1.1 M: 19.5 us, with 4096 22.8, 1024 43.1)
 int pass_items(int n) { return n <= (1 << 18) ? 4 : 8; }
 int mask_rows(int n) { return (int)(((int64_t)n + kBlock - 1) / kBlock); }
 
@@ -575,10 +576,11 @@ hipError_t launch_order_pairs(const OrderPairsSide *sides, int n_sides, int kv, 
   default: hipLaunchKernelGGL(order_masks_kernel<4>, dim3(rows), dim3(kBlock), 0, s, p); break;
   }
   hipLaunchKernelGGL(order_scan_kernel, dim3(kDigitBins / 16, 2 * p.sides), dim3(1024), 0, s, p);
-  for (p.pass = 0; p.pass < 2; ++p.pass) {
-    if (items == 4) hipLaunchKernelGGL(order_pass_kernel<4>, dim3(chunks), dim3(kPassThreads), 0, s, p);
-    else hipLaunchKernelGGL(order_pass_kernel<8>, dim3(chunks), dim3(kPassThreads), 0, s, p);
-  }
+  int chunks_low = 0;
+  for (int i = 0; i < p.sides; ++i) chunks_low += (p.side[i].n + kPassThreads - 1) / kPassThreads;
+  hipLaunchKernelGGL((order_pass_kernel<1, true>), dim3(chunks_low), dim3(kPassThreads), 0, s, p);
+  if (items == 4) hipLaunchKernelGGL((order_pass_kernel<4, false>), dim3(chunks), dim3(kPassThreads), 0, s, p);
+  else hipLaunchKernelGGL((order_pass_kernel<8, false>), dim3(chunks), dim3(kPassThreads), 0, s, p);
   const dim3 grid(blocks, p.words);
   switch (p.words) {
   case 1: hipLaunchKernelGGL(order_position_kernel<1>, grid, dim3(256), 0, s, p); break;
