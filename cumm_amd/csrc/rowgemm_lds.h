@@ -268,14 +268,14 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
       return m;
     }
   };
-  // bit k of a row's words (k wave-uniform; k < 0 comes with a descriptor without records)
-  auto has_bit = [&](const Words m, int k) __attribute__((always_inline)) -> uint32_t {
-    if constexpr (MW == 1) {
-      return (m >> (k & 31)) & 1u;
-    } else {
-      const uint32_t v = k < 32 ? m[0] : (k < 64 ? m[1] : (k < 96 ? m[2] : m[3]));
-      return (v >> (k & 31)) & 1u;
-    }
+  // The word of a row's mask that holds offset k (k wave-uniform; k < 0 comes with a descriptor without
+  // records).  Offsets come in ascending order: with several words it is picked when the number of the word
+  // changes, not per offset and row (three selects each).  A step is a wave's own instructions, one after the
+  // other: 5 x 5 x 5 of 120 k rows, 64 channels, forward 66 -> 58 us, of 8 k rows 44 -> 36, with the list of
+  // offsets in one register instead of two.
+  auto word_of = [&](const Words m, int word) __attribute__((always_inline)) -> uint32_t {
+    if constexpr (MW == 1) return m;
+    else return word == 0 ? m[0] : (word == 1 ? m[1] : (word == 2 ? m[2] : m[3]));
   };
   // memory row of a sorted position (the position itself without an argsort), -1 past the end
   auto row_of = [&](int pos, int raw) __attribute__((always_inline)) -> int { return pos < p.n_pos ? (has_rows ? raw : pos) : -1; };
@@ -368,18 +368,18 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
   // lane j of klist holds the j-th kernel offset of the tile (-1 past the end): lane b pushes
   // b+1 to the lane of its rank among the set bits, lanes without a bit push into lane 63, which
   // nobody reads; a lane nobody pushed to reads 0.
-  // With several mask words the list takes two registers (up to 128 offsets) and every lane works
-  // out its own entry: the tile's words are wave-uniform, so lane j picks the word that holds the
+  // With several mask words a lane holds two numbers (up to 128 offsets) and works out its own
+  // entries: the tile's words are wave-uniform, so lane j picks the word that holds the
   // offset of rank j and finds the position of that set bit by halving.
-  constexpr int KL = MW == 1 ? 1 : 2;
-  int klist[KL];
+  int klist;
   if constexpr (MW == 1) {
     const bool bit = lane < 32 && ((kmask >> lane) & 1u);
     const int rank = __builtin_popcount(kmask & ((1u << (lane & 31)) - 1u));
-    klist[0] = __builtin_amdgcn_ds_permute(bit ? rank * 4 : 63 * 4, bit ? lane + 1 : 0) - 1;
+    klist = __builtin_amdgcn_ds_permute(bit ? rank * 4 : 63 * 4, bit ? lane + 1 : 0) - 1;
   } else {
+    klist = 0;
 #pragma unroll
-    for (int h = 0; h < KL; ++h) {
+    for (int h = 0; h < 2; ++h) {
       int r = h * 64 + lane;          // rank wanted
       uint32_t m = 0;
       int base = 0;
@@ -402,25 +402,27 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
         r -= up ? c : 0;
         m = up ? m >> width : m;
       }
-      klist[h] = found ? base + pos : -1;
+      klist |= ((found ? base + pos : -1) & 0xffff) << (16 * h);
     }
   }
   // kernel offset of step j (-1 past the end of the tile's list)
   auto k_of_step = [&](int j) __attribute__((always_inline)) -> int {
     const int i = j >> p.chunk_shift;
-    if constexpr (MW == 1) {
-      return __builtin_amdgcn_readlane(klist[0], i & 63);
-    } else {
-      const int lo = __builtin_amdgcn_readlane(klist[0], i & 63);
-      const int hi = __builtin_amdgcn_readlane(klist[KL - 1], i & 63);
-      return i < 64 ? lo : (i < 128 ? hi : -1);
-    }
+    const int both = __builtin_amdgcn_readlane(klist, i & 63);
+    if constexpr (MW == 1) return both;
+    else return i < 128 ? (int)(int16_t)(both >> ((i & 64) >> 2)) : -1;
   };
 
+  int key_word = 0;
+  uint32_t key_now = word_of(key_bits, 0);
   auto issue_idx = [&](int j, int *slot) __attribute__((always_inline)) {
     const int k = k_of_step(j);
+    if (MW > 1 && (k >> 5) != key_word) {
+      key_word = k >> 5;
+      key_now = word_of(key_bits, key_word);
+    }
     const v4i rs = rsrc_words(p.gather, k >= 0 ? g_bytes : 0u);
-    dma_b32(rs, lds_addr(slot), has_bit(key_bits, k) ? key_off : kOob, (uint32_t)k * g_k_bytes);
+    dma_b32(rs, lds_addr(slot), (key_now >> (k & 31)) & 1u ? key_off : kOob, (uint32_t)k * g_k_bytes);
   };
   // The entries of the first offsets are requested now; the address work below (row chunks, weight
   // rows, fragment slots) overlaps their round trip.
@@ -558,8 +560,17 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
     for (int t = 0; t < IPA; ++t) dst[t] = has_gather ? slot[t * RPI + lrow] : a_key[t];
   };
   constexpr int CHUNK_E = LPR * PV;      // contraction elements of a stage row
+  int a_word = 0;
+  uint32_t a_now[IPA];
+#pragma unroll
+  for (int t = 0; t < IPA; ++t) a_now[t] = word_of(a_bits[t], 0);
   auto issue_operands = [&](int j, const int (&src)[IPA], v4i *st, v4i *stw) __attribute__((always_inline)) {
     const int k = k_of_step(j);
+    if (MW > 1 && (k >> 5) != a_word) {
+      a_word = k >> 5;
+#pragma unroll
+      for (int t = 0; t < IPA; ++t) a_now[t] = word_of(a_bits[t], a_word);
+    }
     const int cc = j & ((1 << p.chunk_shift) - 1);          // chunk of the contraction
     const int cc_e = cc * CHUNK_E;                           // its first element
     const uint32_t cc_b = (uint32_t)cc * (LPR * 16u);        // ... as bytes inside a row
@@ -570,7 +581,7 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
       // a_col is out of range already for a row without a key or a chunk past the contraction;
       // adding a row offset below 2 GiB keeps it out of range
       const uint32_t v = (uint32_t)src[t];
-      const uint32_t voff = v < (uint32_t)p.rows_a && has_bit(a_bits[t], k) && cc_e + a_cpos[t] < p.c_in
+      const uint32_t voff = (v < (uint32_t)p.rows_a) & (((a_now[t] >> (k & 31)) & 1u) != 0u) & (cc_e + a_cpos[t] < p.c_in)
                                 ? v * a_row_bytes + a_col[t] + cc_b
                                 : kOob;
       dma_b128(rs_a, lds_addr(st + (wave * IPA + t) * 64), voff, 0u);
