@@ -413,31 +413,38 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
     else return i < 128 ? (int)(int16_t)(both >> ((i & 64) >> 2)) : -1;
   };
 
+  // all ones where the word `lacking` (a mask word inverted) has bit k % 32, else zero: one instruction
+  auto gate = [](uint32_t lacking, int k) __attribute__((always_inline)) -> uint32_t { return (uint32_t)__builtin_amdgcn_sbfe((int)lacking, k, 1); };
+  int k_ahead[DI];         // the offsets whose entries are on their way, one per slot
   int key_word = 0;
-  uint32_t key_now = word_of(key_bits, 0);
-  auto issue_idx = [&](int j, int *slot) __attribute__((always_inline)) {
+  uint32_t key_lacks = ~word_of(key_bits, 0);
+  auto issue_idx = [&](int j, int *slot, int &k_slot) __attribute__((always_inline)) {
     const int k = k_of_step(j);
+    k_slot = k;
     if (MW > 1 && (k >> 5) != key_word) {
       key_word = k >> 5;
-      key_now = word_of(key_bits, key_word);
+      key_lacks = ~word_of(key_bits, key_word);
     }
     const v4i rs = rsrc_words(p.gather, k >= 0 ? g_bytes : 0u);
-    dma_b32(rs, lds_addr(slot), (key_now >> (k & 31)) & 1u ? key_off : kOob, (uint32_t)k * g_k_bytes);
+    dma_b32(rs, lds_addr(slot), key_off | (gate(key_lacks, k) & kOob), (uint32_t)k * g_k_bytes);
   };
   // The entries of the first offsets are requested now; the address work below (row chunks, weight
   // rows, fragment slots) overlaps their round trip.
   if (n_steps > 0) {
     auto first = [&](auto jc) -> bool {
-      issue_idx(decltype(jc)::value, idx_slot(jc));
+      issue_idx(decltype(jc)::value, idx_slot(jc), k_ahead[decltype(jc)::value]);
       return false;
     };
     run_steps(first, std::make_integer_sequence<int, DI>{});
   }
 
-  int a_key[IPA];          // without a pair table the gathered row is the key itself
+  constexpr int CHUNK_E = LPR * PV;      // contraction elements of a stage row
+  const int last_cc = (p.c_in - 1) / CHUNK_E;      // last chunk of the contraction, and its first element
+  const int last_e = last_cc * CHUNK_E;
+  int a_key[IPA];          // without a pair table the gathered row is the key itself (with one, 0)
   uint32_t a_col[IPA];     // byte offset of the fetched chunk inside the gathered row, or kOob
   Words a_bits[IPA];       // mask words of the row
-  int a_cpos[IPA];         // first contraction element of the fetched chunk (in the first chunk of the row)
+  uint32_t a_last[IPA];    // rows to fetch from in the last chunk: none where the lane is past the contraction
 #pragma unroll
   for (int t = 0; t < IPA; ++t) {
     const int r = (wave * IPA + t) * RPI + lrow;
@@ -447,11 +454,12 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
     const int key = pos < p.n_pos ? (p.gather_by_pos ? pos : row) : -1;
     a_key[t] = key >= 0 && key < p.n_idx ? key : -1;
     const int c = lchunk ^ swz(r);
-    a_cpos[t] = c * PV;
+    a_last[t] = last_e + c * PV < p.c_in ? (uint32_t)p.rows_a : 0u;
     a_col[t] = a_key[t] >= 0 ? (uint32_t)c * 16u : kOob;
+    a_key[t] = has_gather ? 0 : a_key[t];
   }
   uint32_t w_voff[IPW];
-  int w_cpos[IPW];         // contraction element (WT: contraction row) the lane fetches, first chunk
+  uint32_t w_last[IPW];    // ... and in the last chunk of the contraction
   // WT: chunk XOR of contraction row e.  A transposing read has, per 16 lanes, four rows e .. e+3
   // and four chunks 4*NBW/8 apart (see wt_rd below), 8 bytes of each.  Rows of 128 bytes (TN = 64)
   // alternate between the halves of the 256 bytes the banks span, so rows e and e+2 must use
@@ -468,14 +476,14 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
       const int i = rho & 15, nb = (rho >> 4) % NBW, wq = rho / (16 * NBW);
       const int n = n0 + wq * (16 * NBW) + (i >> 2) * (4 * NBW) + nb * 4 + (i & 3);
       const int c = lchunk ^ swz(rho);
-      w_cpos[t] = c * PV;
       w_voff[t] = n < p.k_out ? (uint32_t)((int64_t)n * p.w_stride_n * E::kBytes) + (uint32_t)c * 16u : kOob;
+      w_last[t] = last_e + c * PV < p.c_in ? w_voff[t] : kOob;
     } else {
       const int e = (wave * IPW + t) * RPIW + lane / LPRW;   // contraction row
       const int c = (lane % LPRW) ^ swz_w(e);                 // chunk of the row this lane fetches
       const int n = n0 + c * PV;
-      w_cpos[t] = e;
       w_voff[t] = n < p.k_out ? (uint32_t)(((int64_t)e * p.w_stride_c + n) * E::kBytes) : kOob;
+      w_last[t] = last_e + e < p.c_in ? w_voff[t] : kOob;
     }
   }
 
@@ -554,43 +562,46 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
   const uint32_t a_row_bytes = (uint32_t)p.lda * E::kBytes;
   const uint32_t w_k_bytes = (uint32_t)p.w_stride_k * E::kBytes;
 
-  // entries of this lane's rows out of the wave's slot (its own loads: no barrier needed)
+  // Entries of this lane's rows out of the wave's slot (its own loads: no barrier needed).  Without a pair
+  // table the slot holds zeros, the values loaded without records, and the key comes in by the same OR: as a
+  // choice it was two branches per step.
   auto read_idx = [&](const int *slot, int (&dst)[IPA]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int t = 0; t < IPA; ++t) dst[t] = has_gather ? slot[t * RPI + lrow] : a_key[t];
+    for (int t = 0; t < IPA; ++t) dst[t] = slot[t * RPI + lrow];
   };
-  constexpr int CHUNK_E = LPR * PV;      // contraction elements of a stage row
   int a_word = 0;
-  uint32_t a_now[IPA];
+  uint32_t a_lacks[IPA];
 #pragma unroll
-  for (int t = 0; t < IPA; ++t) a_now[t] = word_of(a_bits[t], 0);
-  auto issue_operands = [&](int j, const int (&src)[IPA], v4i *st, v4i *stw) __attribute__((always_inline)) {
-    const int k = k_of_step(j);
+  for (int t = 0; t < IPA; ++t) a_lacks[t] = ~word_of(a_bits[t], 0);
+  // Operands of step j, kernel offset k.  The conditions of a row load are folded into few instructions: a
+  // row without the offset's bit becomes row 2^32 - 1, and the rows a lane may fetch from are none in the
+  // last chunk if the lane is past the contraction there.
+  auto issue_operands = [&](int j, int k, const int (&src)[IPA], v4i *st, v4i *stw) __attribute__((always_inline)) {
     if (MW > 1 && (k >> 5) != a_word) {
       a_word = k >> 5;
 #pragma unroll
-      for (int t = 0; t < IPA; ++t) a_now[t] = word_of(a_bits[t], a_word);
+      for (int t = 0; t < IPA; ++t) a_lacks[t] = ~word_of(a_bits[t], a_word);
     }
     const int cc = j & ((1 << p.chunk_shift) - 1);          // chunk of the contraction
     const int cc_e = cc * CHUNK_E;                           // its first element
     const uint32_t cc_b = (uint32_t)cc * (LPR * 16u);        // ... as bytes inside a row
-    const v4i rs_a = rsrc_words(p.A, k >= 0 ? p.a_bytes : 0u);
-    const v4i rs_w = rsrc_words(p.W, k >= 0 ? p.w_bytes : 0u);
+    const bool last = cc == last_cc;
+    const bool some = (k | (last_cc - cc)) >= 0;             // past the list or the contraction: no records
+    const v4i rs_a = rsrc_words(p.A, some ? p.a_bytes : 0u);
+    const v4i rs_w = rsrc_words(p.W, some ? p.w_bytes : 0u);
 #pragma unroll
     for (int t = 0; t < IPA; ++t) {
       // a_col is out of range already for a row without a key or a chunk past the contraction;
       // adding a row offset below 2 GiB keeps it out of range
-      const uint32_t v = (uint32_t)src[t];
-      const uint32_t voff = (v < (uint32_t)p.rows_a) & (((a_now[t] >> (k & 31)) & 1u) != 0u) & (cc_e + a_cpos[t] < p.c_in)
-                                ? v * a_row_bytes + a_col[t] + cc_b
-                                : kOob;
+      const uint32_t v = (uint32_t)src[t] | (uint32_t)a_key[t] | gate(a_lacks[t], k);
+      const uint32_t voff = v < (last ? a_last[t] : (uint32_t)p.rows_a) ? v * a_row_bytes + a_col[t] + cc_b : kOob;
       dma_b128(rs_a, lds_addr(st + (wave * IPA + t) * 64), voff, 0u);
     }
     // k = -1 comes with zero records; a transposed weight tile steps CHUNK_E contraction rows
     const uint32_t soff = (uint32_t)k * w_k_bytes + (WT ? (uint32_t)cc_e * (uint32_t)p.w_stride_c * E::kBytes : cc_b);
 #pragma unroll
     for (int t = 0; t < IPW; ++t)
-      dma_b128(rs_w, lds_addr(stw + (wave * IPW + t) * 64), cc_e + w_cpos[t] < p.c_in ? w_voff[t] : kOob, soff);
+      dma_b128(rs_w, lds_addr(stw + (wave * IPW + t) * 64), last ? w_last[t] : w_voff[t], soff);
   };
 
   if (n_steps > 0) {
@@ -602,8 +613,8 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
       wait_vmcnt<DI - 1 + j * (PER_STEP - 1)>();   // entries of offset j have landed
       int v[IPA];
       read_idx(idx_slot(std::integral_constant<int, j % DI>{}), v);
-      issue_operands(j, v, stage(std::integral_constant<int, j % NS>{}), stage_w(std::integral_constant<int, j % NS>{}));
-      issue_idx(j + DI, idx_slot(std::integral_constant<int, j % DI>{}));
+      issue_operands(j, k_ahead[j % DI], v, stage(std::integral_constant<int, j % NS>{}), stage_w(std::integral_constant<int, j % NS>{}));
+      issue_idx(j + DI, idx_slot(std::integral_constant<int, j % DI>{}), k_ahead[j % DI]);
       return false;
     };
     run_steps(fill, std::make_integer_sequence<int, L>{});
@@ -643,8 +654,8 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
       for (int rb = 0; rb < RBW; ++rb)
 #pragma unroll
         for (int s = 0; s < KS; ++s) af[rb][s] = st[a_rd[s] + rb * 16 * LPR];
-      issue_operands(done + L, v, stage(std::integral_constant<int, sl>{}), stage_w(std::integral_constant<int, sl>{}));
-      issue_idx(done + L + DI, idx_slot(std::integral_constant<int, si>{}));
+      issue_operands(done + L, k_ahead[si], v, stage(std::integral_constant<int, sl>{}), stage_w(std::integral_constant<int, sl>{}));
+      issue_idx(done + L + DI, idx_slot(std::integral_constant<int, si>{}), k_ahead[si]);
 #pragma unroll
       for (int rb = 0; rb < RBW; ++rb)
 #pragma unroll
