@@ -47,6 +47,7 @@ constexpr int kPassThreads = 1024, kPassWaves = kPassThreads / 64;
 constexpr int kMaskBatch = 16;                            // table rows whose loads are in flight together
 constexpr int kBlock = 512;                               // positions per workgroup of the masks kernel
 constexpr int kScanRows = 48;                             // blocks per thread and trip of the scan
+constexpr uint32_t kNowhere = 0xF0000000u;                // past any matrix of counts (up to 2^31 + 2048 bytes: 2^20 rows and the sums)
 constexpr int kExact = 5;                                 // offsets up to which a one-word key is exact
 constexpr uint32_t kAggregate = 1u << 30, kInclusive = 2u << 30, kCount = (1u << 30) - 1u;
 constexpr int kSpins = 1 << 20;                           // (about a second)
@@ -230,11 +231,11 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const OrderParams p) {
       __builtin_amdgcn_make_buffer_rsrc(d.counts[blockIdx.y & 1], 0, (int)((uint32_t)(d.rows + 1) * (kDigitBins * 4u)), 0x00020000);
   const uint32_t col = (uint32_t)(blockIdx.x * 16 + digit) * 4u;
   const int per = (d.rows + 63) / 64, r0 = run * per, r1 = r0 + per < d.rows ? r0 + per : d.rows;
-  const auto at = [&](int r) -> uint32_t { return r < r1 ? (uint32_t)r * (kDigitBins * 4u) + col : 0x80000000u; };
+  const auto at = [&](int r) -> uint32_t { return r < r1 ? (uint32_t)r * (kDigitBins * 4u) + col : kNowhere; };
   uint32_t v[kScanRows], sum = 0;
   for (int t0 = 0; t0 < per; t0 += kScanRows) {
 #pragma unroll
-    for (int u = 0; u < kScanRows; ++u) v[u] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, t0 + u < per ? at(r0 + t0 + u) : 0x80000000u, 0, 0);
+    for (int u = 0; u < kScanRows; ++u) v[u] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, t0 + u < per ? at(r0 + t0 + u) : kNowhere, 0, 0);
 #pragma unroll
     for (int u = 0; u < kScanRows; ++u) sum += v[u];
   }
@@ -250,11 +251,11 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const OrderParams p) {
   for (int t0 = 0; t0 < per; t0 += kScanRows) {
     if (per > kScanRows) {
 #pragma unroll
-      for (int u = 0; u < kScanRows; ++u) v[u] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, t0 + u < per ? at(r0 + t0 + u) : 0x80000000u, 0, 0);
+      for (int u = 0; u < kScanRows; ++u) v[u] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, t0 + u < per ? at(r0 + t0 + u) : kNowhere, 0, 0);
     }
 #pragma unroll
     for (int u = 0; u < kScanRows; ++u) {
-      __builtin_amdgcn_raw_buffer_store_b32((int)before, rs, t0 + u < per ? at(r0 + t0 + u) : 0x80000000u, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b32((int)before, rs, t0 + u < per ? at(r0 + t0 + u) : kNowhere, 0, 0);
       before += v[u];
     }
   }

@@ -6,6 +6,8 @@ import ctypes
 import numpy as np
 import pytest
 
+torch = pytest.importorskip("torch")      # (before the library: one HIP runtime in the process)
+
 import helpers as H
 from cumm_amd import _capi, pairs
 from cumm_amd import tensorview as tv
@@ -112,3 +114,26 @@ def test_counts_of_many_blocks(n, n2):
         want = np.lexsort((m, count))
         assert np.array_equal(g["order"][: int(light.sum())], want[: int(light.sum())])
         assert np.array_equal(np.sort(g["order"]), np.arange(len(m))) and np.array_equal(g["mask"][:, 0], m[g["order"]])
+
+
+def test_most_positions():
+    """A table of one offset just under 2^31 bytes: 2^20 blocks of counts, whose sums begin 2^31 bytes into the
+    matrix."""
+    print("case order most positions", flush=True)
+    lib, n = _capi.lib(), (1 << 29) - 1
+    index = torch.arange(n, dtype=torch.int32, device="cuda")
+    on = (index * 40503 & 0x300) == 0
+    table = torch.where(on, index, torch.tensor(-1, dtype=torch.int32, device="cuda"))
+    mask, order, by_position = (torch.empty(n, dtype=torch.int32, device="cuda") for _ in range(3))
+    sides = (_capi.OrderSide * 2)()
+    sides[0].indices, sides[0].n, sides[0].sorted_mask = table.data_ptr(), n, mask.data_ptr()
+    sides[0].argsort, sides[0].by_position, sides[0].by_position_reversed = order.data_ptr(), by_position.data_ptr(), None
+    ws = torch.empty(int(lib.cumm_hip_order_pairs_workspace(sides, 1, 1)), dtype=torch.uint8, device="cuda")
+    _capi.check(lib.cumm_hip_order_pairs(sides, 1, (ctypes.c_int32 * 3)(1, 1, 1), ws.data_ptr(), ws.numel(), 0))
+    _capi.check(lib.cumm_hip_device_synchronize())
+    without = n - int(on.sum())
+    assert bool((mask[:without] == 0).all()) and bool((mask[without:] == 1).all())
+    for begin, end, want in ((0, without, False), (without, n, True)):      # stable: ascending, each of its kind
+        rows = order[begin:end]
+        assert bool((rows[1:] > rows[:-1]).all()) and int(rows[0]) >= 0 and int(rows[-1]) < n
+        assert bool((by_position[begin:end] == (rows if want else -1)).all())
