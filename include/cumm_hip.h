@@ -337,7 +337,7 @@ int cumm_hip_query_light_hint(const uint32_t *sorted_mask, int n, uint32_t mask_
  * (batch, z, y, x) order; output o gathers the input at o*stride - padding + k_zyx*dilation.
  *
  * cumm_hip_conv_pairs_sites finds the active sites: writes out_shape[3] and *n_out (host) and
- *   SYNCHRONISES the stream once to do so (the caller sizes its tables by n_out).
+ *   WAITS once, until what it has launched is done, to do so (the caller sizes its tables by n_out).
  * cumm_hip_conv_pairs_fill, with the same coords, geometry and workspace (untouched in between)
  *   and that n_out: out_coords [n_out, 4], indices_fwd [kv, n_out] (both 16-byte aligned), mask_fwd [n_out];
  *   indices_bwd [kv, n_in] / mask_bwd [n_in] may be NULL (indices_bwd[k][i] = the output row that

@@ -373,6 +373,37 @@ def test_sparse_conv_pairs_line_lengths(shape, batch, stride):
     _check_conv_case(coords, shape, stride=stride, batch_size=batch)
 
 
+@pytest.mark.parametrize("shape", [(5, 33, 31), (41, 800, 704), (64, 2048, 2048)])
+def test_sites_are_there_when_their_number_is(shape):
+    """What cumm_hip_conv_pairs_sites leaves in its workspace is used on another stream as soon as it returns: one
+    workgroup of the scan, a few hundred, and more than one adds up by itself."""
+    import ctypes as C
+    print("case sites on another stream", shape, flush=True)
+    lib, arr3 = _capi.lib(), C.c_int32 * 3
+    size = shape[0] * shape[1] * shape[2]
+    site = torch.unique(torch.randint(0, size, (min(size // 2, 200000),), device="cuda", generator=torch.Generator("cuda").manual_seed(5)))
+    zyx = [site // (shape[1] * shape[2]), site // shape[2] % shape[1], site % shape[2]]
+    coords = torch.stack([torch.zeros_like(site)] + zyx, 1).to(torch.int32)
+    n = coords.shape[0]
+    geo = [arr3(*v) for v in (shape, (1, 1, 1), (1, 1, 1), (0, 0, 0), (1, 1, 1))]
+    ws = torch.empty(int(lib.cumm_hip_conv_pairs_workspace(n, 1, *geo)), dtype=torch.uint8, device="cuda")
+    sites = torch.empty_like(coords)
+    table = torch.empty((1, n), dtype=torch.int32, device="cuda")
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for repeat in range(3):
+        ws.fill_(0xA5)
+        sites.fill_(-7)
+        torch.cuda.synchronize()
+        out_shape, found = arr3(), C.c_int32(0)
+        _capi.check(lib.cumm_hip_conv_pairs_sites(coords.data_ptr(), n, 1, *geo, out_shape, C.byref(found), ws.data_ptr(), ws.numel(),
+                                                  streams[0].cuda_stream))
+        assert found.value == n
+        _capi.check(lib.cumm_hip_conv_pairs_fill(coords.data_ptr(), n, 1, *geo, n, sites.data_ptr(), table.data_ptr(), None, None, None,
+                                                 ws.data_ptr(), ws.numel(), streams[1].cuda_stream))
+        torch.cuda.synchronize()
+        assert torch.equal(sites, coords) and torch.equal(table[0], torch.arange(n, dtype=torch.int32, device="cuda"))
+
+
 @pytest.mark.parametrize("strided", [False, True])
 def test_more_lookups_than_threads_of_one_launch_axis(strided):
     """36 M voxels and 121 lines of offsets, 2^32 lanes and more: a full box of voxels, so that every entry is
