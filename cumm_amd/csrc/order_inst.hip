@@ -24,13 +24,13 @@
 // looks back (ticket, flagged words); both rank by ballot and are stable.  (Instead of a kernel that clears,
 // counts by device-wide atomics and look-backs in both passes.  The first pass can then be cut as finely as
 // the device is wide: 1024 positions per workgroup, over 447 k positions of two tables 21.2 -> 7.1 us, over
-// 120 k 13.2 -> 4.8; the second 21.2 -> 15.2, 13.2 -> 11.4; the sums 5 - 7 us for 3 - 4 of clearing.  Each pass
+// 120 k 13.2 -> 4.8; the second 21.2 -> 15.2, 13.2 -> 11.4; the sums 5 us for 3 - 4 of clearing.  Each pass
 // adding up the counts by itself instead took 6 us back.)  The mask kernel reads the tables at 4.4 TB/s (1024
 // positions per workgroup 35.7 for 27.2 us at 1.1 M).  The position kernel writes them again; what it fetches by
 // row is little more than a word pair per position (51.5 -> 39.1 us at 1.1 M positions against a fetch of mask
 // and entries).
 // Measured (kernel times): the tables of a frame of 120 k voxels - submanifold and stride 2, 326 k output
-// sites - 95 us in ten launches; with masks by atomics, a sort each and a gather of every entry it
+// sites - 98 us in ten launches; with masks by atomics, a sort each and a gather of every entry it
 // was 305 us in 27.
 #include <cstring>
 
@@ -46,7 +46,7 @@ constexpr int kKeyBits = 2 * kDigit;
 constexpr int kPassThreads = 1024, kPassWaves = kPassThreads / 64;
 constexpr int kMaskBatch = 16;                            // table rows whose loads are in flight together
 constexpr int kBlock = 512;                               // positions per workgroup of the masks kernel
-constexpr int kScanRows = 48;                             // blocks per thread and trip of the scan
+constexpr int kLowBlocks = kPassThreads / kBlock;         // blocks per chunk of the first pass
 constexpr uint32_t kNowhere = 0xF0000000u;                // past any matrix of counts (up to 2^31 + 2048 bytes: 2^20 rows and the sums)
 constexpr int kExact = 5;                                 // offsets up to which a one-word key is exact
 constexpr uint32_t kAggregate = 1u << 30, kInclusive = 2u << 30, kCount = (1u << 30) - 1u;
@@ -220,24 +220,33 @@ __global__ __launch_bounds__(kBlock) void order_masks_kernel(const OrderParams p
   d.counts[1][(size_t)block * kDigitBins + t] = hist[1][t];
 }
 
-// Counts -> sums over the blocks before, and the totals behind the last.  A workgroup takes 16 digits of one
-// pass and table in 64 runs of blocks, 48 blocks of each at a time (one trip up to 1.5 M positions).  (Rows past a
-// run's end are fetched outside the matrix: as conditional loads each waited for the one before, 18 us for 5.)
+// blocks per run of the scan: whole chunks of the first pass
+__host__ __device__ constexpr int scan_run(int rows) { return (rows + 64 * kLowBlocks - 1) / (64 * kLowBlocks) * kLowBlocks; }
+
+// Counts -> totals behind the last block and, for the first pass, the sums over the blocks before every chunk
+// (the second pass wants the totals alone).  A workgroup takes 16 digits of one pass and table in 64 runs of
+// blocks, ROWS blocks of each at a time.  (Rows past a run's end are fetched outside the matrix: as conditional
+// loads each waited for the one before, 18 us for 5.  They cost their issue all the same: ROWS is the least of
+// three that takes a run in one trip, 48 where none does, and of the sums only those that are read are written:
+// with 48 and all of them 120 k positions 7.0 us for 4.7, 447 k of two tables 8.6 for 5.3, 1.4 M 12.7 for 8.6.)
+template <int ROWS>
 __global__ __launch_bounds__(1024) void order_scan_kernel(const OrderParams p) {
   __shared__ uint32_t run_sum[64][16];
+  static_assert(ROWS % kLowBlocks == 0, "a chunk of the first pass begins at the same row of every trip");
   const int digit = threadIdx.x & 15, run = threadIdx.x >> 4;
+  const bool low = (blockIdx.y & 1) == 0;
   const Side &d = p.side[blockIdx.y >> 1];
   const __amdgpu_buffer_rsrc_t rs =
-      __builtin_amdgcn_make_buffer_rsrc(d.counts[blockIdx.y & 1], 0, (int)((uint32_t)(d.rows + 1) * (kDigitBins * 4u)), 0x00020000);
+      __builtin_amdgcn_make_buffer_rsrc(low ? d.counts[0] : d.counts[1], 0, (int)((uint32_t)(d.rows + 1) * (kDigitBins * 4u)), 0x00020000);
   const uint32_t col = (uint32_t)(blockIdx.x * 16 + digit) * 4u;
-  const int per = (d.rows + 63) / 64, r0 = run * per, r1 = r0 + per < d.rows ? r0 + per : d.rows;
-  const auto at = [&](int r) -> uint32_t { return r < r1 ? (uint32_t)r * (kDigitBins * 4u) + col : kNowhere; };
-  uint32_t v[kScanRows], sum = 0;
-  for (int t0 = 0; t0 < per; t0 += kScanRows) {
+  const int per = scan_run(d.rows), r0 = run * per, r1 = r0 + per < d.rows ? r0 + per : d.rows;
+  const auto at = [&](int t) -> uint32_t { return t < per && r0 + t < r1 ? (uint32_t)(r0 + t) * (kDigitBins * 4u) + col : kNowhere; };
+  uint32_t v[ROWS], sum = 0;
+  for (int t0 = 0; t0 < per; t0 += ROWS) {
 #pragma unroll
-    for (int u = 0; u < kScanRows; ++u) v[u] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, t0 + u < per ? at(r0 + t0 + u) : kNowhere, 0, 0);
+    for (int u = 0; u < ROWS; ++u) v[u] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, at(t0 + u), 0, 0);
 #pragma unroll
-    for (int u = 0; u < kScanRows; ++u) sum += v[u];
+    for (int u = 0; u < ROWS; ++u) sum += v[u];
   }
   run_sum[run][digit] = sum;
   __syncthreads();
@@ -248,18 +257,19 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const OrderParams p) {
     before += i < run ? x : 0u;
     all += x;
   }
-  for (int t0 = 0; t0 < per; t0 += kScanRows) {
-    if (per > kScanRows) {
+  if (run == 0) __builtin_amdgcn_raw_buffer_store_b32((int)all, rs, (uint32_t)d.rows * (kDigitBins * 4u) + col, 0, 0);
+  if (!low) return;
+  for (int t0 = 0; t0 < per; t0 += ROWS) {
+    if (per > ROWS) {
 #pragma unroll
-      for (int u = 0; u < kScanRows; ++u) v[u] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, t0 + u < per ? at(r0 + t0 + u) : kNowhere, 0, 0);
+      for (int u = 0; u < ROWS; ++u) v[u] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, at(t0 + u), 0, 0);
     }
 #pragma unroll
-    for (int u = 0; u < kScanRows; ++u) {
-      __builtin_amdgcn_raw_buffer_store_b32((int)before, rs, t0 + u < per ? at(r0 + t0 + u) : kNowhere, 0, 0);
+    for (int u = 0; u < ROWS; ++u) {
+      if (u % kLowBlocks == 0) __builtin_amdgcn_raw_buffer_store_b32((int)before, rs, at(t0 + u), 0, 0);
       before += v[u];
     }
   }
-  if (run == 0) __builtin_amdgcn_raw_buffer_store_b32((int)all, rs, (uint32_t)d.rows * (kDigitBins * 4u) + col, 0, 0);
 }
 
 // One pass over one digit (LOW: the low one, rows in ascending order to tmp; else the high one, tmp to
@@ -287,7 +297,7 @@ __global__ __launch_bounds__(kPassThreads) void order_pass_kernel(const OrderPar
   if (t < kDigitBins) {
     const uint32_t *c = d.counts[LOW ? 0 : 1] + t;
     total = c[(size_t)d.rows * kDigitBins];
-    if constexpr (LOW) earlier = c[(size_t)(block * (kChunk / kBlock)) * kDigitBins];
+    if constexpr (LOW) earlier = c[(size_t)(block * kLowBlocks) * kDigitBins];
   }
   __syncthreads();
   if constexpr (!LOW) chunk = chunk_of_block;
@@ -576,7 +586,12 @@ hipError_t launch_order_pairs(const OrderPairsSide *sides, int n_sides, int kv, 
   case 3: hipLaunchKernelGGL(order_masks_kernel<3>, dim3(rows), dim3(kBlock), 0, s, p); break;
   default: hipLaunchKernelGGL(order_masks_kernel<4>, dim3(rows), dim3(kBlock), 0, s, p); break;
   }
-  hipLaunchKernelGGL(order_scan_kernel, dim3(kDigitBins / 16, 2 * p.sides), dim3(1024), 0, s, p);
+  int run = 0;
+  for (int i = 0; i < p.sides; ++i) run = scan_run(p.side[i].rows) > run ? scan_run(p.side[i].rows) : run;
+  const dim3 scan_grid(kDigitBins / 16, 2 * p.sides);
+  if (run <= 8) hipLaunchKernelGGL(order_scan_kernel<8>, scan_grid, dim3(1024), 0, s, p);
+  else if (run <= 24) hipLaunchKernelGGL(order_scan_kernel<24>, scan_grid, dim3(1024), 0, s, p);
+  else hipLaunchKernelGGL(order_scan_kernel<48>, scan_grid, dim3(1024), 0, s, p);
   int chunks_low = 0;
   for (int i = 0; i < p.sides; ++i) chunks_low += (p.side[i].n + kPassThreads - 1) / kPassThreads;
   hipLaunchKernelGGL((order_pass_kernel<1, true>), dim3(chunks_low), dim3(kPassThreads), 0, s, p);

@@ -99,10 +99,12 @@ def test_a_tile_has_as_few_offsets_as_in_the_exact_order():
         assert steps(g["order"]) <= steps(other) * 1.01 + 2
 
 
-@pytest.mark.parametrize("n,n2", [(511, 513), (512 * 64, 512 * 64 + 1), (512 * 64 * 48 - 1, 40), (512 * 64 * 48 + 513, 600000)])
+@pytest.mark.parametrize("n,n2", [(511, 513), (512 * 64, 512 * 64 + 1), (1, 512 * 128 + 1), (512 * 64 * 8, 70),
+                                  (512 * 64 * 8 + 1, 3), (512 * 64 * 24, 1030), (512 * 64 * 24 + 1, 512 * 64 * 8),
+                                  (512 * 64 * 48 - 1, 40), (512 * 64 * 48 + 513, 600000)])
 def test_counts_of_many_blocks(n, n2):
-    """The digits' counts per block of 512 positions, summed in runs of blocks: a block, a run, and more blocks
-    than one trip takes; exact and stable up to five offsets."""
+    """The digits' counts per block of 512 positions, summed in runs of blocks: a block, a run, the runs of one
+    trip of 8, 24 and 48 blocks, and more; exact and stable up to five offsets."""
     print("case order blocks", n, n2, flush=True)
     rng = np.random.default_rng(n)
     tables = [np.where(rng.random((8, m)) < 0.3, np.int32(3), np.int32(-1)) for m in (n, n2)]
