@@ -1463,7 +1463,7 @@ int cumm_hip_conv_pairs_sites(const int32_t *coords, int n_in, int batch_size, c
   conv_pairs_params(&p, l, coords, n_in, batch_size, out_shape, ksize, stride, padding, dilation, workspace);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   char *temp = reinterpret_cast<char *>(workspace) + l.off_temp;
-  // Either way the caller sizes its tables by the number of sites: the one synchronisation of the path.
+  // Either way the caller sizes its tables by the number of sites: the one wait of the path.
   if (l.bitmap) {
     HostWord word;
     if (int rc = word.take()) return rc;

@@ -323,7 +323,7 @@ def sparse_conv_pairs_device(coords, spatial_shape: Sequence[int], ksize=(3, 3, 
                              stream: int = 0, out=None) -> DeviceConvPairTable:
     """GPU counterpart of :func:`sparse_conv_pairs`: ``coords`` is a device ``tv.Tensor`` [N, 4]
     int32 of unique (batch, z, y, x); the tables stay on the device.  Two library calls with one
-    stream synchronisation between them (the number of active output sites sizes the tables), as
+    wait between them (the number of active output sites sizes the tables), as
     with spconv's generate_conv_inds_mask_stage1 / stage2.  Batch indices are 0 .. batch_size-1.
     ``out``: the table of an earlier call; its tensors are written again when the number of output
     sites is the same (with ``workspace`` the call then allocates nothing)."""
