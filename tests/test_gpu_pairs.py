@@ -404,6 +404,40 @@ def test_sites_are_there_when_their_number_is(shape):
         assert torch.equal(sites, coords) and torch.equal(table[0], torch.arange(n, dtype=torch.int32, device="cuda"))
 
 
+def test_sites_of_a_large_grid_at_the_rate_of_their_memory():
+    """2^31 sites: the bitmap is cleared, written once, read twice and its sums are written, 2^30 bytes; the call takes
+    what a clear of twice that takes and a launch's overhead, not a turn per workgroup of the scan at one address
+    (927 us against 271; a clear of 2^31 bytes takes 410 at 5.2 TB/s)."""
+    import ctypes as C
+    import time
+    print("case sites of a large grid", flush=True)
+    lib, arr3 = _capi.lib(), C.c_int32 * 3
+    geo = [arr3(*v) for v in ((512, 2048, 2048), (1, 1, 1), (1, 1, 1), (0, 0, 0), (1, 1, 1))]
+    n = 1000
+    coords = torch.zeros(n, 4, dtype=torch.int32, device="cuda")
+    coords[:, 2] = torch.arange(n, device="cuda")
+    ws = torch.empty(int(lib.cumm_hip_conv_pairs_workspace(n, 1, *geo)), dtype=torch.uint8, device="cuda")
+    out_shape, found = arr3(), C.c_int32(0)
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def least(call):
+        times = []
+        for _ in range(20):
+            torch.cuda.synchronize()
+            start = time.perf_counter()
+            call()
+            torch.cuda.synchronize()
+            times.append(time.perf_counter() - start)
+        return min(times)
+
+    def sites():
+        _capi.check(lib.cumm_hip_conv_pairs_sites(coords.data_ptr(), n, 1, *geo, out_shape, C.byref(found), ws.data_ptr(), ws.numel(), stream))
+    took = least(sites)
+    assert found.value == n
+    cleared = least(torch.empty(1 << 31, dtype=torch.uint8, device="cuda").zero_)
+    assert took < cleared + 100e-6, (took, cleared)
+
+
 @pytest.mark.parametrize("strided", [False, True])
 def test_more_lookups_than_threads_of_one_launch_axis(strided):
     """36 M voxels and 121 lines of offsets, 2^32 lanes and more: a full box of voxels, so that every entry is
