@@ -6,10 +6,10 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
-#include <thread>
 #include <string>
 #include <vector>
 
+#include "host_word.h"
 #include "launch.h"
 
 using namespace cummhip;
@@ -263,62 +263,6 @@ int async_status_ptr(int32_t **out) {
   *out = g_status_ptr[dev];
   return CUMM_HIP_OK;
 }
-
-// A word of pinned host memory that a kernel writes and the calling thread waits for: no copy behind the
-// kernel, and the thread looks at the word itself instead of waiting for the stream (a frame's strided
-// geometry on 2 k voxels 101 -> 76 us, copy and wake-up were a quarter of it).  Words go round in a pool, one per
-// call in progress at most; one whose kernel may still write stays out of it.
-constexpr uint32_t kNotYet = 0xFFFFFFFFu;
-std::mutex g_words_lock;
-std::vector<uint32_t *> g_words;
-
-struct HostWord {
-  uint32_t *at = nullptr;
-  bool settled = false;
-  int take() {
-    {
-      std::lock_guard<std::mutex> guard(g_words_lock);
-      if (!g_words.empty()) {
-        at = g_words.back();
-        g_words.pop_back();
-      }
-    }
-    if (at == nullptr) {
-      void *host = nullptr;
-      HIP_TRY(hipHostMalloc(&host, 64, hipHostMallocPortable));
-      at = reinterpret_cast<uint32_t *>(host);
-    }
-    __atomic_store_n(at, kNotYet, __ATOMIC_RELEASE);
-    return CUMM_HIP_OK;
-  }
-  // until the word is there; the stream is looked at now and then, for errors and for a launch that has ended
-  hipError_t wait(hipStream_t s, uint32_t *value) {
-    for (unsigned spin = 1;; ++spin) {
-      uint32_t v = __atomic_load_n(at, __ATOMIC_ACQUIRE);
-      if (v == kNotYet && spin % 512 == 0) {
-        const hipError_t e = hipStreamQuery(s);
-        if (e != hipSuccess && e != hipErrorNotReady) return e;
-        (void)hipGetLastError();      // ("not ready" is no error of this call)
-        if (e == hipErrorNotReady) {
-          if (spin >= 1u << 16) std::this_thread::yield();
-          continue;
-        }
-        v = __atomic_load_n(at, __ATOMIC_ACQUIRE);
-      } else if (v == kNotYet) {
-        __builtin_ia32_pause();
-        continue;
-      }
-      settled = true;
-      *value = v;
-      return hipSuccess;
-    }
-  }
-  ~HostWord() {
-    if (!settled) return;
-    std::lock_guard<std::mutex> guard(g_words_lock);
-    g_words.push_back(at);
-  }
-};
 
 // After a synchronisation: anything to report on this device?
 int take_async_errors(int32_t *timeouts, int32_t *sort_give_ups = nullptr) {
@@ -1466,7 +1410,7 @@ int cumm_hip_conv_pairs_sites(const int32_t *coords, int n_in, int batch_size, c
   // Either way the caller sizes its tables by the number of sites: the one wait of the path.
   if (l.bitmap) {
     HostWord word;
-    if (int rc = word.take()) return rc;
+    HIP_TRY(word.take());
     hipError_t e = launch_conv_pairs_bits(p, temp, l.total - l.off_temp, word.at, s);
     if (e != hipSuccess) return hip_fail(e, "output site launch");
     uint32_t total = 0;
