@@ -16,6 +16,7 @@
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/dynamo/compiled_autograd.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/extension.h>
 
@@ -270,6 +271,21 @@ bool plain(const Tensor &t, const Geometry &g) {
          !t.key_set().has(c10::DispatchKey::Python) && !t._fw_grad(0).defined();
 }
 
+struct SparseConvBackward;
+
+// Nodes that torch's compiled autograd has met, by the number that its graph has of them: a graph is used again
+// for other nodes, so that it takes the number - a tensor, one of its inputs - and not the node.
+struct Met {
+  std::mutex mutex;
+  std::unordered_map<int64_t, std::weak_ptr<torch::autograd::Node>> nodes;
+  int64_t next = 0;
+};
+Met &met() {
+  static Met *all = new Met();      // (nodes may outlive the statics)
+  return *all;
+}
+torch::autograd::variable_list run_met(const torch::autograd::variable_list &grads, const std::vector<c10::IValue> &args);
+
 struct SparseConvBackward : public torch::autograd::Node {
   GeometryPtr g;
   py::object owner;      // the bridge's geometry (for the Python path)
@@ -278,6 +294,7 @@ struct SparseConvBackward : public torch::autograd::Node {
   at::TensorOptions options;
   bool relu = false, has_bias = false;
   int tile_m = 0;
+  mutable Tensor number;      // in met()
 
   std::string name() const override { return "_SparseConvFunctionBackward"; }
   void release_variables() override {
@@ -286,6 +303,10 @@ struct SparseConvBackward : public torch::autograd::Node {
     out.reset_data();
   }
   ~SparseConvBackward() override {
+    if (number.defined()) {
+      std::lock_guard<std::mutex> lock(met().mutex);
+      met().nodes.erase(*number.data_ptr<int64_t>());
+    }
     if (!Py_IsInitialized()) {
       owner.release();
     } else {
@@ -297,11 +318,56 @@ struct SparseConvBackward : public torch::autograd::Node {
   torch::autograd::variable_list apply(torch::autograd::variable_list &&grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
     const Tensor x = features.unpack(), w = weight.unpack(), y = relu ? out.unpack(getptr()) : Tensor();
-    at::AutoGradMode no_grad(false);
-    Tensor gy = grads[0].defined() ? grads[0].contiguous() : at::zeros(sizes, options);
     const bool need[3] = {task_should_compute_output(0), task_should_compute_output(1), has_bias && task_should_compute_output(2)};
+    return gradients(x, w, y, grads[0], need);
+  }
+
+  torch::autograd::variable_list gradients(const Tensor &x, const Tensor &w, const Tensor &y, const Tensor &grad, const bool (&need)[3]) {
+    at::AutoGradMode no_grad(false);
+    Tensor gy = grad.defined() ? grad.contiguous() : at::zeros(sizes, options);
     torch::autograd::variable_list result(3);
     if (!native(x, w, y, gy, need, result)) python(x, w, y, gy, need, result);
+    return result;
+  }
+
+  // ---- compiled autograd: what of the node is an input of its graph, and the call that the graph makes (opaque to
+  // it: it takes addresses)
+  void compiled_args(torch::dynamo::autograd::CompiledNodeArgs &args) const override {
+    if (!number.defined()) {
+      std::lock_guard<std::mutex> lock(met().mutex);
+      number = at::full({1}, met().next, at::kLong);
+      met().nodes[met().next++] = const_cast<SparseConvBackward *>(this)->weak_from_this();
+    }
+    args.collect(features, false);
+    args.collect(weight, false);
+    args.collect(relu);
+    if (relu) args.collect(out, true);
+    args.collect(has_bias);
+    args.collect(number);
+  }
+
+  torch::autograd::variable_list apply_with_saved(const torch::autograd::variable_list &grads,
+                                                  torch::dynamo::autograd::SwapSavedVariables &saved) override {
+    namespace ca = torch::dynamo::autograd;
+    saved.before(features);
+    saved.before(weight);
+    if (relu) saved.before(out);
+    saved.before(number);
+    std::vector<c10::IValue> args = {number, task_should_compute_output(0), task_should_compute_output(1),
+                                     has_bias && task_should_compute_output(2), features.unpack(), weight.unpack()};
+    if (relu) args.emplace_back(out.unpack(getptr()));
+    std::vector<at::TypePtr> types;
+    for (const c10::IValue &a : args) types.push_back(a.isTensor() ? at::TypePtr(at::TensorType::get()) : a.type());
+    const auto &compiler = ca::getPyCompilerInterface();
+    const std::string call = compiler->bind_function(saved.get_py_compiler(), "sparse_conv_backward", run_met, types,
+                                                     /*is_custom_function=*/true, /*is_traceable=*/false);
+    auto result = compiler->call_function(
+        saved.get_py_compiler(), "apply_functional", call, grads, args,
+        ca::IValuePacker<std::vector<std::optional<torch::autograd::InputMetadata>>>::pack(ca::get_input_metadata(next_edges())));
+    saved.after(features);
+    saved.after(weight);
+    if (relu) saved.after(out);
+    saved.after(number);
     return result;
   }
 
@@ -393,6 +459,19 @@ struct SparseConvBackward : public torch::autograd::Node {
     }
   }
 };
+
+torch::autograd::variable_list run_met(const torch::autograd::variable_list &grads, const std::vector<c10::IValue> &args) {
+  std::shared_ptr<torch::autograd::Node> node;
+  {
+    std::lock_guard<std::mutex> lock(met().mutex);
+    const auto it = met().nodes.find(args[0].toTensor().item<int64_t>());
+    if (it != met().nodes.end()) node = it->second.lock();
+  }
+  TORCH_CHECK(node != nullptr, "a compiled backward pass of a sparse convolution that is no longer there");
+  const bool need[3] = {args[1].toBool(), args[2].toBool(), args[3].toBool()};
+  return static_cast<SparseConvBackward &>(*node).gradients(args[4].toTensor(), args[5].toTensor(), args.size() > 6 ? args[6].toTensor() : Tensor(),
+                                                            grads[0], need);
+}
 
 // the forward pass, or an undefined tensor where the call is the bridge's own
 Tensor run_forward(const Tensor &features, const Tensor &weight, const std::optional<Tensor> &bias, const py::object &owner, Geometry &g,

@@ -118,3 +118,27 @@ def test_on_another_stream_and_after_the_geometry():
         got = torch.autograd.grad(out, (x, w, b), g)
     stream.synchronize()
     assert torch.equal(out.detach(), want[0]) and torch.equal(got[0], want[1]) and torch.equal(got[2], want[3])
+
+
+def test_compiled_autograd():
+    """A backward pass under torch's compiled autograd (its graph run as it is): the gradients of the ordinary one, also
+    where the graph of one layer serves the next - another geometry of the same sizes."""
+    from torch._dynamo import compiled_autograd
+    for ksize, strided, relu, with_bias in ((3, False, True, True), (3, True, False, False), (5, False, True, False)):
+        for seed in (3, 4):
+            print("case compiled autograd", ksize, strided, relu, with_bias, seed, flush=True)
+            tb, geo, x, w, b, g = _setup(ksize, strided, seed=seed)
+            conv = lambda *t: tb.sparse_conv(*t, geo, relu)
+            leaves = lambda: [t.detach().clone().requires_grad_(True) for t in ((x, w, b) if with_bias else (x, w))]
+            of = lambda ts: tuple(ts) + (() if with_bias else (None,))
+            torch.use_deterministic_algorithms(True, warn_only=True)
+            try:
+                one, two = leaves(), leaves()
+                conv(*of(one)).backward(g)
+                out = conv(*of(two))
+                assert out.grad_fn.name() == "_SparseConvFunctionBackward"
+                with compiled_autograd._enable(lambda graph: torch.compile(graph, backend="eager")):
+                    out.backward(g)
+                assert all(torch.equal(p.grad, q.grad) for p, q in zip(one, two))
+            finally:
+                torch.use_deterministic_algorithms(False)
