@@ -298,6 +298,7 @@ struct SparseConvBackward : public torch::autograd::Node {
 
   std::string name() const override { return "_SparseConvFunctionBackward"; }
   void release_variables() override {
+    std::lock_guard<std::mutex> lock(mutex_);      // (another thread may be in apply)
     features.reset_data();
     weight.reset_data();
     out.reset_data();

@@ -83,6 +83,38 @@ def test_what_autograd_keeps():
     assert all(not t.any() for t in zero)
 
 
+def test_a_node_used_by_two_threads_while_one_frees_it():
+    """A backward pass that frees the graph, beside calls of the node from another thread: each call has the right
+    gradients or the error of a freed graph."""
+    import threading
+    tb, geo, x, w, b, g = _setup()
+    want = _grads(lambda *t: tb.sparse_conv(*t, geo, True), x, w, b, g)
+    leaves = [t.detach().clone().requires_grad_(True) for t in (x, w, b)]
+    torch.cuda.synchronize()
+    for trip in range(20):
+        out = tb.sparse_conv(*leaves, geo, True)
+        start, calls, wrong = threading.Barrier(2), [0, 0], []
+
+        def call(freeing):
+            start.wait()
+            for _ in range(1 if freeing else 8):
+                try:
+                    got = torch.autograd.grad(out, leaves, g) if freeing else out.grad_fn(g)
+                    torch.cuda.synchronize()
+                    calls[freeing] += 1
+                    if not (torch.equal(got[0], want[1]) and torch.equal(got[2], want[3])):
+                        wrong.append((trip, freeing))
+                except RuntimeError as e:
+                    if freeing or "second time" not in str(e):
+                        wrong.append((trip, freeing, str(e)))
+        threads = [threading.Thread(target=call, args=(f,)) for f in (True, False)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not wrong and calls[1] == 1
+
+
 def test_what_is_left_to_python():
     import torch.autograd.forward_ad as fwad
     tb, geo, x, w, b, g = _setup()
