@@ -10,6 +10,7 @@ needs torch.
 """
 import ctypes
 import os
+import warnings
 from typing import Optional, Sequence, Tuple
 
 import torch
@@ -177,18 +178,24 @@ _native_module = None
 
 
 def _native():
-    """The native half of this module (csrc/torch_native.cpp); built first if it is not there."""
+    """The native half of this module (csrc/torch_native.cpp), built first if it is not there; None where that cannot
+    be done - no host compiler, no headers of torch: the functions here make all calls then."""
     global _native_module
     if _native_module is None:
         from . import build
-        if not os.path.exists(build.TORCH_LIB):
-            build.build_torch_native()
-        from . import _torch_native as native
-        native.bind({"cumm_hip_" + n: ctypes.cast(getattr(_capi.lib(), "cumm_hip_" + n), ctypes.c_void_p).value
-                     for n in _NATIVE_SYMBOLS})
-        native.set_backward(_backward)
-        _native_module = native
-    return _native_module
+        try:
+            if not os.path.exists(build.TORCH_LIB):
+                build.build_torch_native()
+            from . import _torch_native as native
+        except (ImportError, OSError, RuntimeError) as e:
+            warnings.warn("the native half of the torch bridge is not there, Python makes its calls: %s" % e, RuntimeWarning)
+            _native_module = False
+        else:
+            native.bind({"cumm_hip_" + n: ctypes.cast(getattr(_capi.lib(), "cumm_hip_" + n), ctypes.c_void_p).value
+                         for n in _NATIVE_SYMBOLS})
+            native.set_backward(_backward)
+            _native_module = native
+    return _native_module or None
 
 
 def _remember(g: "SparseConvGeometry", key, kind, launch: "_Launch", op: ConvOpType, features, weight, bias=None) -> None:
@@ -263,10 +270,14 @@ class SparseConvGeometry:
         self._reduced, self._reduced_streams, self._written = {}, {}, set()
         self._own_launches = {}      # calls of the layers on this geometry, see _Launch
         self._tensors = {}
-        self._native, self.out_coords, self.out_shape, ordered = _native().build(
-            coords.contiguous(), three(spatial_shape), ksize, None if self.subm else three(stride), three(padding), three(dilation),
-            int(batch_size))
-        self.n_out, self._block = self._native.n_out, self._native.block
+        geo = (coords.contiguous(), three(spatial_shape), ksize, None if self.subm else three(stride), three(padding), three(dilation),
+               int(batch_size))
+        native = _native()
+        if native is not None:
+            self._native, self.out_coords, self.out_shape, ordered = native.build(*geo)
+            self.n_out, self._block = self._native.n_out, self._native.block
+        else:
+            ordered = self._build(*geo)
         # masks, an order of the positions by them, and the pair tables once more in that order: what
         # forward and backward-input read (a tile's entries for one offset are then consecutive in
         # memory); backward-weight keeps the table by row
@@ -274,6 +285,45 @@ class SparseConvGeometry:
             self._order_one_by_one()
         if words > 1:
             self._make_lists()
+
+    def _build(self, coords, spatial_shape, ksize, stride, padding, dilation, batch_size) -> bool:
+        """Tables, order and tables by position, where native code does not make them; False: large tables, to be
+        ordered by _order_one_by_one."""
+        lib, arr3, s, dev, n_in = _capi.lib(), ctypes.c_int32 * 3, self._stream, self._device, self.n_in
+        shape, ks, pad, dil = (arr3(*a) for a in (spatial_shape, ksize, padding, dilation))
+        if self.subm:
+            self.n_out, self.out_coords, self.out_shape = n_in, coords, spatial_shape
+            self._allocate()
+            ws = _bytes(lib.cumm_hip_subm_pairs_workspace(n_in), dev)
+            _capi.check(lib.cumm_hip_subm_pairs(coords.data_ptr(), n_in, shape, ks, dil, self._ptr["indices_fwd"], self._ptr["indices_bwd"],
+                                                None, None, ws.data_ptr(), ws.numel(), s))
+        else:
+            geo = (shape, ks, arr3(*stride), pad, dil)
+            need = int(lib.cumm_hip_conv_pairs_workspace(n_in, batch_size, *geo))
+            if need == 0:
+                raise ValueError("bad geometry (kernel volume 1..128, non-empty output grid) or too many voxels")
+            ws = _bytes(need, dev)
+            out_shape, found = arr3(), ctypes.c_int32(0)
+            _capi.check(lib.cumm_hip_conv_pairs_sites(coords.data_ptr(), n_in, batch_size, *geo, out_shape, ctypes.byref(found),
+                                                      ws.data_ptr(), ws.numel(), s))
+            self.n_out, self.out_shape = int(found.value), tuple(out_shape)
+            self.out_coords = torch.empty((self.n_out, 4), dtype=torch.int32, device=dev)
+            self._allocate()
+            _capi.check(lib.cumm_hip_conv_pairs_fill(coords.data_ptr(), n_in, batch_size, *geo, self.n_out, self.out_coords.data_ptr(),
+                                                     self._ptr["indices_fwd"], self._ptr["indices_bwd"], None, None, ws.data_ptr(),
+                                                     ws.numel(), s))
+        if 4 * self.kv * max(n_in, self.n_out) >= 1 << 31:
+            return False
+        sides, p = (_capi.OrderSide * 2)(), self._ptr
+        for d, side, n in ((sides[0], "fwd", self.n_out), (sides[1], "bwd", n_in)):
+            d.indices, d.n = p["indices_" + side], n
+            d.sorted_mask, d.argsort, d.by_position = p["mask_" + side], p["order_" + side], p["indices_%s_pos" % side]
+        count = 2
+        if self.subm:      # (one order serves both; the backward table is the forward one with its offsets reversed)
+            sides[0].by_position_reversed, count = p["indices_bwd_pos"], 1
+        ws = _bytes(lib.cumm_hip_order_pairs_workspace(sides, count, self.kv), dev)
+        _capi.check(lib.cumm_hip_order_pairs(sides, count, ks, ws.data_ptr(), ws.numel(), s))
+        return True
 
     @property
     def _launches(self):
@@ -349,7 +399,8 @@ class SparseConvGeometry:
         self._list_block = lists
         counts = counts.cpu().numpy()
         self._lists = self._lists_over(lists, counts)
-        self._native.set_lists(lists, counts.clip(0, n).tolist())
+        if self._native is not None:
+            self._native.set_lists(lists, counts.clip(0, n).tolist())
 
     def _lists_over(self, keepalive, counts) -> pairs.DevicePairLists:
         pair_in, pair_out = (tv.from_blob(t.data_ptr(), [self.kv, self.n_out], tv.int32, self._device.index, keepalive=keepalive)

@@ -174,3 +174,22 @@ def test_compiled_autograd():
                 assert all(torch.equal(p.grad, q.grad) for p, q in zip(one, two))
             finally:
                 torch.use_deterministic_algorithms(False)
+
+
+@pytest.mark.parametrize("ksize,strided", [(3, False), (3, True), (5, False)])
+def test_without_the_native_half(monkeypatch, ksize, strided):
+    """On a machine without a host compiler the bridge's own functions make every call: the same tables and bits."""
+    print("case without native", ksize, strided, flush=True)
+    tb, geo, x, w, b, g = _setup(ksize, strided)
+    torch.use_deterministic_algorithms(True, warn_only=True)
+    try:
+        want = _grads(lambda *t: tb.sparse_conv(*t, geo, True), x, w, b, g)
+        monkeypatch.setattr(tb, "_native_module", False)
+        _, own, *_ = _setup(ksize, strided)
+        assert own._native is None and own.out_shape == geo.out_shape and torch.equal(own.out_coords, geo.out_coords)
+        for name in tb.SparseConvGeometry._TABLES:
+            assert (H.host(getattr(own, name)) == H.host(getattr(geo, name))).all(), name
+        got = _grads(lambda *t: tb.sparse_conv(*t, own, True), x, w, b, g)
+        assert all(torch.equal(a, c) for a, c in zip(got, want))
+    finally:
+        torch.use_deterministic_algorithms(False)

@@ -254,3 +254,17 @@ def test_a_remembered_call_refuses_tensors_on_another_device(monkeypatch):
         with pytest.raises(ValueError, match="same device"):
             backward(*tensors)
     assert len(calls) == 3
+
+
+@pytest.mark.parametrize("error", [RuntimeError("g++ failed"), FileNotFoundError("g++")])
+def test_a_machine_without_a_host_compiler_is_told_and_served(monkeypatch, tmp_path, error):
+    from cumm_amd import build, torch_bridge as tb
+
+    def fail(*a, **k):
+        raise error
+    monkeypatch.setattr(build, "TORCH_LIB", str(tmp_path / "_torch_native.so"))
+    monkeypatch.setattr(build, "build_torch_native", fail)
+    monkeypatch.setattr(tb, "_native_module", None)
+    with pytest.warns(RuntimeWarning, match="g\\+\\+"):
+        assert tb._native() is None
+    assert tb._native() is None      # (and does not try again)
