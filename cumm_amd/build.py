@@ -5,6 +5,7 @@
 This replaces the reference's NVRTC / pccm JIT builds
 (cumm/nvrtc/__init__.py:179-283, cumm/gemm/main_real.py:59-70).
 """
+import hashlib
 import importlib.util
 import os
 import subprocess
@@ -92,18 +93,32 @@ def build(force=False, verbose=False, jobs=None):
     return LIB
 
 
+def _torch_native_stamp():
+    """What the native half was built from: its source, the interface it shares with the library and torch."""
+    import torch
+    h = hashlib.sha256()
+    for f in (TORCH_SRC, os.path.join(HERE, "..", "include", "cumm_hip.h")):
+        with open(f, "rb") as stream:
+            h.update(stream.read())
+    h.update(("%s %s" % (torch.__version__, sys.implementation.cache_tag)).encode())
+    return h.hexdigest()[:32]
+
+
 def build_torch_native(force=False, verbose=False):
-    """Compile the native half of torch_bridge.py (host code against torch's headers) if stale or ``force``."""
-    stamp = max(os.path.getmtime(f) for f in (TORCH_SRC, os.path.join(HERE, "..", "include", "cumm_hip.h")))
-    if not force and os.path.exists(TORCH_LIB) and os.path.getmtime(TORCH_LIB) >= stamp:
-        return TORCH_LIB
+    """Compile the native half of torch_bridge.py (host code against torch's headers) if ``force`` or if what is there
+    was built from something else: it has the layouts of the interface compiled in."""
+    stamp = _torch_native_stamp()
+    if not force and os.path.exists(TORCH_LIB):
+        with open(TORCH_LIB, "rb") as stream:
+            if ("cumm_torch_native:" + stamp).encode() in stream.read():
+                return TORCH_LIB
     import sysconfig
     import torch
     root = os.path.dirname(torch.__file__)
     include = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
                os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"), sysconfig.get_paths()["include"]]
     cmd = (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-            "-DTORCH_EXTENSION_NAME=_torch_native", "-DTORCH_API_INCLUDE_EXTENSION_H"] +
+            "-DTORCH_EXTENSION_NAME=_torch_native", "-DCUMM_STAMP=\"%s\"" % stamp, "-DTORCH_API_INCLUDE_EXTENSION_H"] +
            [a for d in include for a in ("-isystem", d)] + [TORCH_SRC, "-o", TORCH_LIB + ".tmp", "-L" + os.path.join(root, "lib")] +
            ["-l" + n for n in ("torch", "torch_cpu", "torch_hip", "torch_python", "c10", "c10_hip")])
     if verbose:

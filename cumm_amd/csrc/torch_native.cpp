@@ -542,6 +542,7 @@ py::object forward(const Tensor &features, const Tensor &weight, const std::opti
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.attr("stamp") = "cumm_torch_native:" CUMM_STAMP;      // (build.py looks for it in the file)
   py::class_<Geometry, GeometryPtr>(m, "Geometry")
       .def_readonly("block", &Geometry::block)
       .def_readonly("n_in", &Geometry::n_in)

@@ -9,7 +9,6 @@ and the bias gradient of the backward pass.  Imported on demand: nothing else in
 needs torch.
 """
 import ctypes
-import os
 import warnings
 from typing import Optional, Sequence, Tuple
 
@@ -178,14 +177,13 @@ _native_module = None
 
 
 def _native():
-    """The native half of this module (csrc/torch_native.cpp), built first if it is not there; None where that cannot
-    be done - no host compiler, no headers of torch: the functions here make all calls then."""
+    """The native half of this module (csrc/torch_native.cpp), built first if it is not there or not of these sources
+    and this torch; None where that cannot be done - no host compiler, no headers of torch: the functions here make all calls then."""
     global _native_module
     if _native_module is None:
         from . import build
         try:
-            if not os.path.exists(build.TORCH_LIB):
-                build.build_torch_native()
+            build.build_torch_native()
             from . import _torch_native as native
         except (ImportError, OSError, RuntimeError) as e:
             warnings.warn("the native half of the torch bridge is not there, Python makes its calls: %s" % e, RuntimeWarning)

@@ -1,5 +1,8 @@
 """Host logic of the torch bridge that needs no GPU: the argument blocks of validated calls, whose addresses
 are never dereferenced here."""
+import os
+import subprocess
+
 import pytest
 
 from cumm_amd import _capi
@@ -268,3 +271,28 @@ def test_a_machine_without_a_host_compiler_is_told_and_served(monkeypatch, tmp_p
     with pytest.warns(RuntimeWarning, match="g\\+\\+"):
         assert tb._native() is None
     assert tb._native() is None      # (and does not try again)
+
+
+def test_a_native_half_of_other_sources_is_built_again(monkeypatch, tmp_path):
+    """By what it was built from, not by its age: a file that came with an archive is as old as anything."""
+    from cumm_amd import build
+    source, lib = tmp_path / "torch_native.cpp", tmp_path / "_torch_native.so"
+    source.write_text("one")
+    monkeypatch.setattr(build, "TORCH_SRC", str(source))
+    monkeypatch.setattr(build, "TORCH_LIB", str(lib))
+    built = []
+
+    def compiler(cmd, **k):
+        built.append(cmd)
+        with open(cmd[cmd.index("-o") + 1], "w") as f:
+            f.write("..cumm_torch_native:" + [a for a in cmd if a.startswith("-DCUMM_STAMP=")][0].split('"')[1] + "..")
+        return subprocess.CompletedProcess(cmd, 0, "")
+    monkeypatch.setattr(build.subprocess, "run", compiler)
+    for text, count in (("one", 1), ("one", 1), ("two", 2), ("two", 2)):
+        source.write_text(text)
+        os.utime(source, (0, 0))
+        assert build.build_torch_native() == str(lib)
+        assert len(built) == count, text
+    monkeypatch.setattr(torch, "__version__", "another")
+    build.build_torch_native()
+    assert len(built) == 3
