@@ -10,6 +10,7 @@ import importlib.util
 import os
 import subprocess
 import sys
+import threading
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -112,6 +113,8 @@ def build_torch_native(force=False, verbose=False):
         with open(TORCH_LIB, "rb") as stream:
             if ("cumm_torch_native:" + stamp).encode() in stream.read():
                 return TORCH_LIB
+    # (a name of its own: several processes may find it missing at once)
+    out = "%s.%d.%d.tmp" % (TORCH_LIB, os.getpid(), threading.get_ident())
     import sysconfig
     import torch
     root = os.path.dirname(torch.__file__)
@@ -119,14 +122,18 @@ def build_torch_native(force=False, verbose=False):
                os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"), sysconfig.get_paths()["include"]]
     cmd = (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
             "-DTORCH_EXTENSION_NAME=_torch_native", "-DCUMM_STAMP=\"%s\"" % stamp, "-DTORCH_API_INCLUDE_EXTENSION_H"] +
-           [a for d in include for a in ("-isystem", d)] + [TORCH_SRC, "-o", TORCH_LIB + ".tmp", "-L" + os.path.join(root, "lib")] +
+           [a for d in include for a in ("-isystem", d)] + [TORCH_SRC, "-o", out, "-L" + os.path.join(root, "lib")] +
            ["-l" + n for n in ("torch", "torch_cpu", "torch_hip", "torch_python", "c10", "c10_hip")])
     if verbose:
         print(" ".join(cmd), flush=True)
-    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
-    if res.returncode != 0:
-        raise RuntimeError("g++ failed for %s:\n%s" % (TORCH_SRC, res.stdout))
-    os.replace(TORCH_LIB + ".tmp", TORCH_LIB)
+    try:
+        res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+        if res.returncode != 0:
+            raise RuntimeError("g++ failed for %s:\n%s" % (TORCH_SRC, res.stdout))
+        os.replace(out, TORCH_LIB)
+    finally:
+        if os.path.exists(out):
+            os.remove(out)
     return TORCH_LIB
 
 

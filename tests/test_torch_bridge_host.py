@@ -2,6 +2,7 @@
 are never dereferenced here."""
 import os
 import subprocess
+import threading
 
 import pytest
 
@@ -296,3 +297,35 @@ def test_a_native_half_of_other_sources_is_built_again(monkeypatch, tmp_path):
     monkeypatch.setattr(torch, "__version__", "another")
     build.build_torch_native()
     assert len(built) == 3
+
+
+def test_builds_of_the_native_half_at_once_do_not_share_a_file(monkeypatch, tmp_path):
+    """A build that ends while another one writes puts its own whole file in place; one that fails leaves nothing."""
+    from cumm_amd import build
+    monkeypatch.setattr(build, "TORCH_LIB", str(tmp_path / "_torch_native.so"))
+    inside = []
+
+    def compiler(cmd, **k):
+        out = cmd[cmd.index("-o") + 1]
+        with open(out, "w") as f:
+            f.write("half")
+        if not inside:
+            inside.append(out)
+            other = threading.Thread(target=build.build_torch_native, kwargs=dict(force=True))
+            other.start()
+            other.join()
+            assert open(build.TORCH_LIB).read() == "whole"
+        with open(out, "w") as f:
+            f.write("whole")
+        return subprocess.CompletedProcess(cmd, 0, "")
+    monkeypatch.setattr(build.subprocess, "run", compiler)
+    build.build_torch_native(force=True)
+    assert open(build.TORCH_LIB).read() == "whole" and os.listdir(tmp_path) == ["_torch_native.so"]
+
+    def failing(cmd, **k):
+        compiler(cmd)
+        return subprocess.CompletedProcess(cmd, 1, "no")
+    monkeypatch.setattr(build.subprocess, "run", failing)
+    with pytest.raises(RuntimeError, match="no"):
+        build.build_torch_native(force=True)
+    assert os.listdir(tmp_path) == ["_torch_native.so"]
