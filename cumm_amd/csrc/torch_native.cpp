@@ -106,7 +106,7 @@ int size_class(int64_t n) {      // (the tuner's bucket of the position count)
 struct Kind {
   CummHipConvDesc desc;
   CummHipSparseConvArgs args;
-  int index, tile_m;
+  int tile_m;
 };
 // pass, types of features / weight / bias (-1: none), K, C, kernel volume, submanifold, size class, device, ReLU,
 // tile height and determinism (backward-weight)
@@ -128,12 +128,11 @@ const Kind *find_kind(const Key &key) {
 }
 
 bool remember(int op, at::ScalarType x, at::ScalarType w, std::optional<at::ScalarType> bias, int64_t k_out, int64_t c_in, int kv, bool subm, int cls, int device,
-              bool relu, int tile_m, bool deterministic, const std::string &desc, const std::string &args, int launch_tile_m, int index) {
+              bool relu, int tile_m, bool deterministic, const std::string &desc, const std::string &args, int launch_tile_m) {
   Kind kind;
   if (desc.size() != sizeof(kind.desc) || args.size() != sizeof(kind.args)) throw py::value_error("argument blocks of another layout");
   std::memcpy(&kind.desc, desc.data(), desc.size());
   std::memcpy(&kind.args, args.data(), args.size());
-  kind.index = index;
   kind.tile_m = launch_tile_m;
   std::lock_guard<std::mutex> lock(kinds_mutex);
   return kinds.emplace(Key(op, (int)x, (int)w, bias.has_value() ? (int)*bias : -1, k_out, c_in, kv, subm, cls, device, relu, tile_m, deterministic), kind).second;
@@ -152,8 +151,7 @@ struct Geometry {
   int32_t *indices_fwd, *indices_bwd, *indices_fwd_pos, *indices_bwd_pos, *order_fwd, *order_bwd;
   uint32_t *mask_fwd, *mask_bwd, *reduced_64, *reduced_128;
   std::atomic<bool> written_64{false}, written_128{false};
-  std::mutex used_mutex;
-  std::vector<int> used;
+  std::atomic<bool> made[3] = {};      // passes made here: forward, backward-input, backward-weight
 
   void allocate() {
     const int64_t pos_words = words;
@@ -177,12 +175,6 @@ struct Geometry {
     if ((void *)s.stream() == stream) return;
     block.record_stream(s.unwrap());
     if (lists.defined()) lists.record_stream(s.unwrap());
-  }
-  void note(int index) {
-    std::lock_guard<std::mutex> lock(used_mutex);
-    for (int i : used)
-      if (i == index) return;
-    used.push_back(index);
   }
 };
 using GeometryPtr = std::shared_ptr<Geometry>;
@@ -420,7 +412,7 @@ struct SparseConvBackward : public torch::autograd::Node {
       a.ptr_A = gy.data_ptr(); a.ptr_B = w.data_ptr();
       a.ptr_C = result[0].data_ptr(); a.ptr_D = a.ptr_C;
       check(api.sparse_conv(&dgrad->desc, &a, s));
-      g->note(dgrad->index);
+      g->made[1] = true;
     }
     if (need[1] && wgrad) {
       result[1] = at::empty_like(w);
@@ -433,7 +425,7 @@ struct SparseConvBackward : public torch::autograd::Node {
       a.ptr_C = result[1].data_ptr(); a.ptr_D = a.ptr_C;
       a.workspace = ws.data_ptr(); a.workspace_bytes = (size_t)size;
       check(api.sparse_conv(&wgrad->desc, &a, s));
-      g->note(wgrad->index);
+      g->made[2] = true;
     } else if (need[1]) {
       // the products of all kernel offsets over their pair lists (an offset without pairs writes zeros)
       result[1] = at::empty_like(w);
@@ -441,6 +433,7 @@ struct SparseConvBackward : public torch::autograd::Node {
       const int32_t *pair_in = g->lists.data_ptr<int32_t>(), *pair_out = pair_in + (int64_t)g->kv * g->n_out;
       check(api.wgrad_pairs(result[1].data_ptr(), gy.data_ptr(), x.data_ptr(), pair_out, pair_in, g->counts.data(), g->kv, g->n_out,
                             (int)g->n_out, (int)g->n_in, (int)k_out, (int)c_in, dtype, ws.data_ptr(), (size_t)list_bytes, s));
+      g->made[2] = true;
     }
     return true;
   }
@@ -505,7 +498,7 @@ Tensor run_forward(const Tensor &features, const Tensor &weight, const std::opti
       a.ptr_D = a.bias_pointer = b.data_ptr();
     }
     check(api.sparse_conv(&kind->desc, &a, stream.stream()));
-    g.note(kind->index);
+    g.made[0] = true;
     if (g.words == 1) (kind->tile_m == 64 ? g.written_64 : g.written_128) = true;
   }
   if (differentiable) {
@@ -547,11 +540,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
       .def_readonly("block", &Geometry::block)
       .def_readonly("n_in", &Geometry::n_in)
       .def_readonly("n_out", &Geometry::n_out)
-      .def_property_readonly("used",
-                             [](Geometry &g) {
-                               std::lock_guard<std::mutex> lock(g.used_mutex);
-                               return g.used;
-                             })
+      .def("made", [](const Geometry &g, int pass) { return g.made[pass].load(); })
       .def("written", [](const Geometry &g, int width) { return width == 64 ? g.written_64.load() : (width == 128 && g.written_128.load()); })
       .def("set_lists",
            [](Geometry &g, const Tensor &lists, std::vector<int32_t> counts) {

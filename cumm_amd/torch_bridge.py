@@ -167,8 +167,6 @@ def _copy(args: _capi.SparseConvArgs) -> _capi.SparseConvArgs:
 _KINDS = {}
 
 
-# the keys of the calls that native code knows too, by the number it knows them by
-_NATIVE_KEYS = []
 _NATIVE_SYMBOLS = ("sparse_conv", "last_error", "relu_backward", "relu_backward_sums", "column_sum", "column_sum_workspace",
                    "query_conv_workspace", "query_wgrad_ordered_workspace", "wgrad_pairs", "wgrad_pairs_workspace", "subm_pairs",
                    "subm_pairs_workspace", "conv_pairs_workspace", "conv_pairs_sites", "conv_pairs_fill", "order_pairs",
@@ -205,10 +203,9 @@ def _remember(g: "SparseConvGeometry", key, kind, launch: "_Launch", op: ConvOpT
     if key[0] == "wgrad":
         tile_m, deterministic = key[3], key[4]
     n_pos = g.n_in if op == ConvOpType.BackwardInput else g.n_out
-    if _native().remember(op.value, features.dtype, weight.dtype, None if bias is None else bias.dtype, int(weight.shape[0]),
-                          int(weight.shape[2]), g.kv, g.subm, _size_class(n_pos), g._device.index, bool(relu), tile_m, deterministic,
-                          bytes(launch.cdesc), bytes(launch.args), launch.tile_m, len(_NATIVE_KEYS)):
-        _NATIVE_KEYS.append(key)
+    _native().remember(op.value, features.dtype, weight.dtype, None if bias is None else bias.dtype, int(weight.shape[0]),
+                       int(weight.shape[2]), g.kv, g.subm, _size_class(n_pos), g._device.index, bool(relu), tile_m, deterministic,
+                       bytes(launch.cdesc), bytes(launch.args), launch.tile_m)
 
 
 def _size_class(n: int) -> int:
@@ -325,11 +322,13 @@ class SparseConvGeometry:
 
     @property
     def _launches(self):
-        """The calls of the layers on this geometry; those made by native code without a _Launch here."""
+        """The calls of the layers on this geometry; of a pass that native code made alone, its name."""
+        calls = dict(self._own_launches)
         if self._native is not None:
-            for i in self._native.used:
-                self._own_launches.setdefault(_NATIVE_KEYS[i], None)
-        return self._own_launches
+            names = ("fwd", "dgrad", "wgrad" if self.words == 1 else "wgrad_pairs")
+            own = {key[0] for key in calls}
+            calls.update({(name,): None for i, name in enumerate(names) if self._native.made(i) and name not in own})
+        return calls
 
     @_launches.setter
     def _launches(self, calls):

@@ -193,3 +193,28 @@ def test_without_the_native_half(monkeypatch, ksize, strided):
         assert all(torch.equal(a, c) for a, c in zip(got, want))
     finally:
         torch.use_deterministic_algorithms(False)
+
+
+def test_two_first_calls_at_once(monkeypatch):
+    """Two threads' first calls of a kind - a forward pass and, while it is being remembered, a backward one: each
+    pass of a later geometry is what it is."""
+    import threading
+    tb, geo, x, w, b, g = _setup(c=56, k=88)
+    native, met = tb._native(), []
+    remember = native.remember
+
+    def both(*args):
+        if not met:
+            met.append(args)
+            needed = (True, False, False)
+            other = threading.Thread(target=tb._backward, args=(geo, x, w, None, g, needed, False, False, 64))
+            other.start()
+            other.join()
+            met.append(None)
+        return remember(*args)
+    monkeypatch.setattr(native, "remember", both)
+    tb._SparseConvFunction.apply(x, w, b, geo, False)
+    assert len(met) == 2
+    _, later, x, w, b, g = _setup(c=56, k=88)
+    assert native.forward(x, w, b, later, later._native, False) is not None
+    assert [key[0] for key in later._launches] == ["fwd"]
