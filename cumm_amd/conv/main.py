@@ -231,7 +231,7 @@ class ConvMainUnitTest:
         args.kernel_volume = kernel_volume
         args.mode, args.groups = 1, 1      # ConvMode.CrossCorrelation, ungrouped: all the reference's mask kernels do
         args.d_is_bias = int(not bias.empty())
-        args.deterministic = int(ordered)
+        args.deterministic = int(ordered or (bool(getattr(params, "deterministic", False)) and op_type != ConvOpType.BackwardWeight))
         args.bias_pointer = _ptr(bias)
         args.scale_pointer = _ptr(scale)
         args.rows_in, args.rows_out = inp.dim(0), output.dim(0)

@@ -82,6 +82,8 @@ struct RowGemmParams {
   int32_t small_stages;
   // two groups of waves per tile: bit k of word k / 32 set = offset k belongs to the first group
   uint32_t first_group[4];
+  // non-zero: every row's sum in the one order that all tiles share
+  int32_t one_order;
 };
 
 // An offset no buffer contains: every operand is smaller than 2 GiB (checked on the host), and

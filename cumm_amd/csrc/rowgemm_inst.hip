@@ -94,7 +94,7 @@ template <class T, int TM, int TN, int KS, bool WT, int MW>
 static bool launch_two_groups(const RowGemmParams &p, dim3 grid, hipStream_t s, hipError_t *err) {
   if constexpr (TM == 64 && TN == 64 && KS <= 2 && !kWide && (!WT || Elem<T>::kBytes == 2)) {
     const unsigned most = MW > 1 || p.chunk_shift > 0 || KS == 1 ? 1024u : 384u;
-    if (p.mask == nullptr || (uint64_t)grid.x * grid.y > most) return false;
+    if (p.mask == nullptr || p.one_order || (uint64_t)grid.x * grid.y > most) return false;
     if (!counted_waits_hold<rowgemm_lds_kernel<T, 2, 2, 2, 2, KS, 2, WT, false, MW, 2>>()) return false;
     RowGemmParams q = p;
     first_group_offsets(p.kv, q.first_group);

@@ -109,7 +109,7 @@ struct Kind {
   int tile_m;
 };
 // pass, types of features / weight / bias (-1: none), K, C, kernel volume, submanifold, size class, device, ReLU,
-// tile height and determinism (backward-weight)
+// tile height (backward-weight) and determinism
 using Key = std::tuple<int, int, int, int, int64_t, int64_t, int, bool, int, int, bool, int, bool>;
 struct KeyHash {
   size_t operator()(const Key &k) const {
@@ -374,7 +374,7 @@ struct SparseConvBackward : public torch::autograd::Node {
     const Kind *dgrad = nullptr, *wgrad = nullptr;
     int64_t list_bytes = 0;
     const int64_t k_out = w.size(0), c_in = w.size(2);
-    if (need[0] && !(dgrad = find_kind(key_of(*g, CUMM_HIP_OP_BACKWARD_INPUT, x, w, -1, g->n_in, false, 0, false)))) return false;
+    if (need[0] && !(dgrad = find_kind(key_of(*g, CUMM_HIP_OP_BACKWARD_INPUT, x, w, -1, g->n_in, false, 0, deterministic)))) return false;
     if (need[1] && g->words == 1 &&
         (!reduced_at(*g, tile_m) ||
          !(wgrad = find_kind(key_of(*g, CUMM_HIP_OP_BACKWARD_WEIGHT, x, w, -1, g->n_out, false, tile_m, deterministic)))))
@@ -476,7 +476,7 @@ Tensor run_forward(const Tensor &features, const Tensor &weight, const std::opti
       c10::impl::TorchDispatchModeTLS::any_modes_set() || torch::jit::tracer::isTracing())
     return Tensor();
   const Kind *kind = find_kind(key_of(g, CUMM_HIP_OP_FORWARD, features, weight, bias.has_value() ? (int)bias->scalar_type() : -1, g.n_out,
-                                      relu, 0, false));
+                                      relu, 0, at::globalContext().deterministicAlgorithms()));
   if (kind == nullptr || (g.words == 1 && reduced_at(g, kind->tile_m) == nullptr)) return Tensor();
   const bool differentiable =
       at::GradMode::is_enabled() && (features.requires_grad() || weight.requires_grad() || (bias.has_value() && bias->requires_grad()));

@@ -464,7 +464,8 @@ class ConvParams(_Versioned):
         self.stream = 0
         # not in the reference's struct: backward-weight with a split_k_parallel descriptor adds its
         # partial sums in a fixed order (the same bits from run to run), as the reference's serial
-        # split-K does, at the speed of the balanced kernels
+        # split-K does, at the speed of the balanced kernels; forward and backward-input add up a row in
+        # one order whatever the tile and the number of rows
         self.deterministic = False
         # not in the reference's struct either: a hint for forward / backward-input, the number of
         # leading positions of the sorted order in tiles of one or two kernel offsets

@@ -199,9 +199,7 @@ def _remember(g: "SparseConvGeometry", key, kind, launch: "_Launch", op: ConvOpT
     _KINDS[kind] = launch
     if g._native is None:
         return
-    relu, tile_m, deterministic = key[5] if key[0] == "fwd" else False, 0, False
-    if key[0] == "wgrad":
-        tile_m, deterministic = key[3], key[4]
+    relu, tile_m, deterministic = key[5] if key[0] == "fwd" else False, key[3] if key[0] == "wgrad" else 0, key[-1]
     n_pos = g.n_in if op == ConvOpType.BackwardInput else g.n_out
     _native().remember(op.value, features.dtype, weight.dtype, None if bias is None else bias.dtype, int(weight.shape[0]),
                        int(weight.shape[2]), g.kv, g.subm, _size_class(n_pos), g._device.index, bool(relu), tile_m, deterministic,
@@ -474,7 +472,7 @@ class _SparseConvFunction(torch.autograd.Function):
             roles["bias"] = bias = bias.contiguous()
         stream = current_stream()
         geometry.used_on(stream)
-        key = ("fwd", features.dtype, weight.dtype, weight.shape, None if bias is None else (bias.dtype, bias.shape), relu)
+        key = ("fwd", features.dtype, weight.dtype, weight.shape, None if bias is None else (bias.dtype, bias.shape), relu, _deterministic())
         launch = geometry._own_launches.get(key)
         if launch is None:
             launch = _forward_launch(geometry, key, roles, relu, stream)
@@ -522,7 +520,7 @@ def _backward(g: SparseConvGeometry, features, weight, out, grad_out, needed, re
         # inputs that feed no output site sit in tiles the kernel skips (mask 0): zero them
         grad_in = torch.empty_like(features) if g.subm else torch.zeros_like(features)
         roles = {"input": grad_in, "weight": weight, "output": grad_out}
-        key = ("dgrad", dtype, weight.shape)
+        key = ("dgrad", dtype, weight.shape, _deterministic())
         launch = g._own_launches.get(key)
         if launch is None:
             launch = _backward_input_launch(g, key, roles, dtype, stream)
@@ -542,9 +540,7 @@ def _backward(g: SparseConvGeometry, features, weight, out, grad_out, needed, re
         plan.rebind(grad_out.data_ptr(), features.data_ptr(), grad_w.data_ptr(), stream, ws.data_ptr())
     elif needed[1]:
         grad_w = torch.empty_like(weight)
-        # torch's switch for reproducible results selects the fixed-order sum of the partial blocks
-        deterministic = bool(torch.are_deterministic_algorithms_enabled())
-        key = ("wgrad", dtype, weight.shape, tile_m, deterministic)
+        key = ("wgrad", dtype, weight.shape, tile_m, _deterministic())
         hit = g._own_launches.get(key)
         if hit is None:
             hit = g._own_launches[key] = _backward_weight_launch(g, key, features, weight, grad_w, grad_out, dtype, stream)
@@ -554,6 +550,12 @@ def _backward(g: SparseConvGeometry, features, weight, out, grad_out, needed, re
         ws = _bytes(need, grad_out.device)
         launch(stream, need, input=features, weight=grad_w, output=grad_out, workspace=ws)
     return grad_in, grad_w, grad_b
+
+
+def _deterministic() -> bool:
+    """torch's switch for reproducible results: rows added up in one order whatever tile the tuner has picked, weight
+    gradients by the fixed-order sum of the partial blocks."""
+    return bool(torch.are_deterministic_algorithms_enabled())
 
 
 def _check_device(g: SparseConvGeometry, *tensors) -> None:
@@ -591,6 +593,7 @@ def _forward_launch(g: SparseConvGeometry, key, roles, relu, stream) -> _Launch:
         p.bias, p.beta = torch2tensor(bias), 1.0
     if relu:
         p.act_type = Activation.ReLU
+    p.deterministic = key[-1]
     p.stream = stream
     _TUNER.tune_conv(p)
     # the tile masks the forward launch computes anyway are what backward-weight needs
@@ -620,6 +623,7 @@ def _backward_input_launch(g: SparseConvGeometry, key, roles, dtype, stream) -> 
     p.mask_int_count = g.words
     p.reverse_mask = g.subm
     p.light_prefix = g.light_bwd
+    p.deterministic = key[-1]
     p.stream = stream
     _TUNER.tune_conv(p)
     ConvMainUnitTest.implicit_gemm2(p)

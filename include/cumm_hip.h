@@ -124,7 +124,10 @@ typedef struct CummHipSparseConvArgs {
   int32_t deterministic;            /* backward-weight with a split_k_parallel descriptor: non-zero = partial sums
                                        added in a fixed order (same bits from run to run on one device), as the
                                        reference's serial split-K is (cumm/conv/kernel.py:1004-1014, 1068-1083);
-                                       workspace: cumm_hip_query_wgrad_ordered_workspace.  Ignored elsewhere. */
+                                       workspace: cumm_hip_query_wgrad_ordered_workspace.  Forward and backward-input:
+                                       non-zero = a row's bits depend neither on the tile of the descriptor nor on how
+                                       many rows the launch has (64 x 64 tiles add up a row in two parts where a launch
+                                       has few of them, every other tile in one: a rounding apart).  Ignored elsewhere. */
   const void *bias_pointer;         /* int8 inference: f32 [K] */
   const void *scale_pointer;        /* int8 inference: f32 [K] */
   int32_t rows_in, rows_out;        /* row counts of the input / output feature tensors */

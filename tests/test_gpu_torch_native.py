@@ -218,3 +218,23 @@ def test_two_first_calls_at_once(monkeypatch):
     _, later, x, w, b, g = _setup(c=56, k=88)
     assert native.forward(x, w, b, later, later._native, False) is not None
     assert [key[0] for key in later._launches] == ["fwd"]
+
+
+def test_one_order_where_reproducible_results_are_asked_for():
+    """A scene's features alone and in a batch of 60 of it - few tiles, many tiles - under torch's switch: the same bits,
+    natively and from Python; of the input gradient too."""
+    tb, _, x, w, b, g = _setup(c=64, k=64)
+    coords, grid = H.small_cloud(3, 1500)
+    scene = torch.as_tensor(coords, device="cuda")
+    batch = scene.repeat(60, 1)
+    batch[:, 0] = torch.arange(60, device="cuda", dtype=torch.int32).repeat_interleave(len(scene))
+    alone, many = (tb.SparseConvGeometry(c, grid, batch_size=n) for c, n in ((scene, 1), (batch.contiguous(), 60)))
+    torch.use_deterministic_algorithms(True, warn_only=True)
+    try:
+        for trip in range(2):      # (a first call, and one in native code)
+            one = _grads(lambda *t: tb.sparse_conv(*t, alone, False), x, w, b, g)
+            all_ = _grads(lambda *t: tb.sparse_conv(*t, many, False), x.repeat(60, 1), w, b, g.repeat(60, 1))
+            for got, want in zip(all_[:2], one[:2]):
+                assert all(torch.equal(part, want) for part in got.view(60, len(scene), -1)), trip
+    finally:
+        torch.use_deterministic_algorithms(False)

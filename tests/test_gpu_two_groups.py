@@ -26,12 +26,12 @@ def _words(table):
     return m if words > 1 else m[:, 0].contiguous()
 
 
-def _run(op, dtype, table, x, w, order):
+def _run(op, dtype, table, x, w, order, tile=64, deterministic=False):
     from cumm_amd.torch_bridge import torch2tensor as t
     kv, n = table.shape
     mask = _words(table)
     p = ConvParams(3, op)
-    p.conv_algo_desp = H.find_conv_desp(dtype, op, 64, 64, dynamic_mask=kv > 32)
+    p.conv_algo_desp = H.find_conv_desp(dtype, op, tile, tile, dynamic_mask=kv > 32)
     out = torch.full((n, w.shape[0] if op == ConvOpType.Forward else w.shape[2]), 7.0, dtype=x.dtype, device="cuda")
     if op == ConvOpType.Forward:
         p.input, p.output = t(x), t(out)
@@ -43,6 +43,7 @@ def _run(op, dtype, table, x, w, order):
                                   [1] if kv <= 32 else [mask.shape[1], 1], tv.uint32, 0, keepalive=sorted_mask)
     p.mask_argsort = t(order)
     p.mask_int_count = (kv + 31) // 32
+    p.deterministic = deterministic
     ConvMainUnitTest.implicit_gemm2(p)
     torch.cuda.synchronize()
     return out
@@ -97,3 +98,26 @@ def test_against_the_sum_over_the_table(op, dtype, kv, c, k, n, which):
     again = _run(op, dtype, table, x, w, other)
     present = (table >= 0).any(0)
     assert torch.equal(got[present], again[present])
+
+
+@pytest.mark.parametrize("op", [ConvOpType.Forward, ConvOpType.BackwardInput])
+@pytest.mark.parametrize("dtype,kv,c,k", [("f16", 27, 64, 64), ("bf16", 27, 128, 136), ("f16", 27, 24, 32), ("bf16", 125, 64, 64)])
+def test_one_order_on_request(op, dtype, kv, c, k):
+    """With ``deterministic`` a row has the same bits in every tile, and in a launch of 700 rows or of 70 000."""
+    print("case one order", op, dtype, kv, c, k, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(kv + c)
+    tdt = {"f16": torch.float16, "bf16": torch.bfloat16}[dtype]
+    rows, n, copies = 705, 700, 100
+    table = torch.randint(0, rows, (kv, n), generator=gen, device="cuda", dtype=torch.int32)
+    table = torch.where(torch.rand(kv, n, generator=gen, device="cuda") < 0.3, table, -1).contiguous()
+    x = torch.randn(rows, c if op == ConvOpType.Forward else k, generator=gen, device="cuda").to(tdt)
+    w = (torch.randn(k, kv, c, generator=gen, device="cuda") * 0.05).to(tdt)
+    order = torch.argsort(_words(table) if kv <= 32 else _words(table)[:, 0], stable=True).to(torch.int32)
+    alone = [_run(op, dtype, table, x, w, order, tile, True) for tile in (64, 128)]
+    many = table.repeat(1, copies)
+    order = torch.argsort(_words(many) if kv <= 32 else _words(many)[:, 0], stable=True).to(torch.int32)
+    batch = [_run(op, dtype, many, x, w, order, tile, True).view(copies, n, -1) for tile in (64, 128)]
+    present = (table >= 0).any(0)
+    assert torch.equal(alone[0][present], alone[1][present])
+    for b in batch:
+        assert all(torch.equal(b[i][present], alone[0][present]) for i in range(copies))
