@@ -26,12 +26,12 @@ def _words(table):
     return m if words > 1 else m[:, 0].contiguous()
 
 
-def _run(op, dtype, table, x, w, order, tile=64, deterministic=False):
+def _run(op, dtype, table, x, w, order):
     from cumm_amd.torch_bridge import torch2tensor as t
     kv, n = table.shape
     mask = _words(table)
     p = ConvParams(3, op)
-    p.conv_algo_desp = H.find_conv_desp(dtype, op, tile, tile, dynamic_mask=kv > 32)
+    p.conv_algo_desp = H.find_conv_desp(dtype, op, 64, 64, dynamic_mask=kv > 32)
     out = torch.full((n, w.shape[0] if op == ConvOpType.Forward else w.shape[2]), 7.0, dtype=x.dtype, device="cuda")
     if op == ConvOpType.Forward:
         p.input, p.output = t(x), t(out)
@@ -43,7 +43,6 @@ def _run(op, dtype, table, x, w, order, tile=64, deterministic=False):
                                   [1] if kv <= 32 else [mask.shape[1], 1], tv.uint32, 0, keepalive=sorted_mask)
     p.mask_argsort = t(order)
     p.mask_int_count = (kv + 31) // 32
-    p.deterministic = deterministic
     ConvMainUnitTest.implicit_gemm2(p)
     torch.cuda.synchronize()
     return out
@@ -54,6 +53,7 @@ def _run(op, dtype, table, x, w, order, tile=64, deterministic=False):
     ("f16", 27, 64, 64, 1, "all"), ("f16", 27, 64, 64, 63, "centre"), ("bf16", 27, 16, 24, 65, "all"),
     ("f16", 27, 64, 64, 64 * 384, "all"), ("f16", 27, 64, 64, 64 * 384 + 1, "all"),
     ("bf16", 27, 32, 64, 64 * 1024, "all"), ("bf16", 27, 32, 64, 64 * 1024 + 1, "all"),
+    ("f16", 27, 136, 128, 64 * 512 + 1, "all"),
     ("f16", 27, 136, 128, 64 * 512, "all"), ("f16", 27, 128, 72, 4000, "even"),
     ("f16", 32, 64, 64, 500, "all"), ("bf16", 9, 48, 64, 700, "all"), ("f16", 1, 64, 64, 200, "all"),
     ("f16", 125, 64, 64, 1000, "all"), ("bf16", 125, 24, 64, 64, "centre"), ("f16", 75, 72, 64, 300, "all"),
@@ -102,7 +102,7 @@ def test_against_the_sum_over_the_table(op, dtype, kv, c, k, n, which):
 
 @pytest.mark.parametrize("op", [ConvOpType.Forward, ConvOpType.BackwardInput])
 @pytest.mark.parametrize("dtype,kv,c,k", [("f16", 27, 64, 64), ("bf16", 27, 128, 136), ("f16", 27, 24, 32), ("bf16", 125, 64, 64)])
-def test_one_order_on_request(op, dtype, kv, c, k):
+def test_one_order_on_request(monkeypatch, op, dtype, kv, c, k):
     """With ``deterministic`` a row has the same bits in every tile, and in a launch of 700 rows or of 70 000."""
     print("case one order", op, dtype, kv, c, k, flush=True)
     gen = torch.Generator(device="cuda").manual_seed(kv + c)
@@ -112,11 +112,16 @@ def test_one_order_on_request(op, dtype, kv, c, k):
     table = torch.where(torch.rand(kv, n, generator=gen, device="cuda") < 0.3, table, -1).contiguous()
     x = torch.randn(rows, c if op == ConvOpType.Forward else k, generator=gen, device="cuda").to(tdt)
     w = (torch.randn(k, kv, c, generator=gen, device="cuda") * 0.05).to(tdt)
-    order = torch.argsort(_words(table) if kv <= 32 else _words(table)[:, 0], stable=True).to(torch.int32)
-    alone = [_run(op, dtype, table, x, w, order, tile, True) for tile in (64, 128)]
-    many = table.repeat(1, copies)
-    order = torch.argsort(_words(many) if kv <= 32 else _words(many)[:, 0], stable=True).to(torch.int32)
-    batch = [_run(op, dtype, many, x, w, order, tile, True).view(copies, n, -1) for tile in (64, 128)]
+    find, call = H.find_conv_desp, ConvMainUnitTest.implicit_gemm2
+
+    def run(table, tile):
+        order = torch.argsort(_words(table) if kv <= 32 else _words(table)[:, 0], stable=True).to(torch.int32)
+        with monkeypatch.context() as m:
+            m.setattr(H, "find_conv_desp", lambda *a, **k: find(*a[:2], tile, tile, **k))
+            m.setattr(ConvMainUnitTest, "implicit_gemm2", staticmethod(lambda p: setattr(p, "deterministic", True) or call(p)))
+            return _run(op, dtype, table, x, w, order)
+    alone = [run(table, tile) for tile in (64, 128)]
+    batch = [run(table.repeat(1, copies), tile).view(copies, n, -1) for tile in (64, 128)]
     present = (table >= 0).any(0)
     assert torch.equal(alone[0][present], alone[1][present])
     for b in batch:
