@@ -56,6 +56,60 @@ def test_same_bits_as_the_python_function(ksize, strided, dtype, relu, with_bias
         assert not tb.sparse_conv(x.requires_grad_(True), w, b, geo, relu).requires_grad
 
 
+@pytest.fixture
+def no_python():
+    """A native backward pass that falls back to Python fails."""
+    from cumm_amd import torch_bridge as tb
+
+    def fell_back(*a):
+        raise AssertionError("the backward pass went to Python")
+    tb._native().set_backward(fell_back)
+    yield
+    tb._native().set_backward(tb._backward)
+
+
+@pytest.mark.parametrize("ksize,strided,dtype", [(3, False, torch.float16), (3, True, torch.bfloat16), (5, False, torch.bfloat16)])
+@pytest.mark.parametrize("relu", [False, True])
+@pytest.mark.parametrize("with_bias", [False, True])
+@pytest.mark.parametrize("deterministic", [False, True])
+def test_a_known_backward_pass_stays_native(no_python, ksize, strided, dtype, relu, with_bias, deterministic):
+    print("case stays native", ksize, strided, dtype, relu, with_bias, deterministic, flush=True)
+    tb, geo, x, w, b, g = _setup(ksize, strided, dtype=dtype)
+    b = b if with_bias else None
+    torch.use_deterministic_algorithms(deterministic, warn_only=True)
+    try:
+        want = _grads(lambda *t: tb._SparseConvFunction.apply(*t, geo, relu), x, w, b, g)
+        _, later, *_ = _setup(ksize, strided, dtype=dtype)      # (another geometry of the kind: only what was remembered serves it)
+        got = _grads(lambda *t: tb._native().forward(*t, later, later._native, relu), x, w, b, g)
+        # (the weight gradient's atomics: sums in any order, and one rounding to the type)
+        for i, (a, c) in enumerate(zip(got, want)):
+            if i == 2 and not deterministic:
+                assert (a.float() - c.float()).norm() <= 2.0 ** -8 * c.float().norm()
+            else:
+                assert torch.equal(a, c)
+    finally:
+        torch.use_deterministic_algorithms(False)
+
+
+def test_a_gradient_that_nobody_has(no_python):
+    """The node is given no gradient at all: zeros."""
+    class Nothing(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, t):
+            ctx.set_materialize_grads(False)
+            return t * 1
+
+        @staticmethod
+        def backward(ctx, grad):
+            return None
+    tb, geo, x, w, b, g = _setup()
+    _grads(lambda *t: tb._SparseConvFunction.apply(*t, geo, True), x, w, b, g)
+    leaves = [t.detach().clone().requires_grad_(True) for t in (x, w, b)]
+    out = tb.sparse_conv(*leaves, geo, True)
+    for got, leaf in zip(torch.autograd.grad(Nothing.apply(out), leaves, g), leaves):
+        assert got.shape == leaf.shape and got.dtype == leaf.dtype and not got.any()
+
+
 def test_what_autograd_keeps():
     tb, geo, x, w, b, g = _setup()
     conv = lambda *t: tb.sparse_conv(*t, geo, True)
