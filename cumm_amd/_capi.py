@@ -126,6 +126,8 @@ SYMBOLS = {
     "cumm_hip_pair_lists": (C.c_int, [_VP, C.c_int, C.c_int, _VP, _VP, _VP, _VP, C.c_size_t, _VP]),
     "cumm_hip_order_pairs_workspace": (C.c_size_t, [C.POINTER(OrderSide), C.c_int, C.c_int]),
     "cumm_hip_order_pairs": (C.c_int, [C.POINTER(OrderSide), C.c_int, C.POINTER(C.c_int32), _VP, C.c_size_t, _VP]),
+    "cumm_hip_order_pairs_coarse_workspace": (C.c_size_t, [C.POINTER(OrderSide), C.c_int, C.c_int]),
+    "cumm_hip_order_pairs_coarse": (C.c_int, [C.POINTER(OrderSide), C.c_int, C.POINTER(C.c_int32), _VP, C.c_size_t, _VP]),
     "cumm_hip_wgrad_pairs_workspace": (C.c_int64, [_VP, C.c_int, C.c_int, C.c_int]),
     "cumm_hip_wgrad_pairs": (C.c_int, [_VP, _VP, _VP, _VP, _VP, _VP, C.c_int, C.c_int64, C.c_int, C.c_int, C.c_int, C.c_int,
                                        C.c_int, _VP, C.c_size_t, _VP]),

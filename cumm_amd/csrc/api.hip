@@ -1493,15 +1493,21 @@ int cumm_hip_pair_lists(const int32_t *indices, int kv, int n, int32_t *pair_in,
 }
 
 // ---- masks, order and tables by position
-size_t cumm_hip_order_pairs_workspace(const CummHipOrderSide *sides, int n_sides, int kv) {
+static size_t order_workspace(const CummHipOrderSide *sides, int n_sides, int kv, bool coarse) {
   if (!sides || n_sides < 1 || n_sides > 2 || kv < 1 || kv > kMaxKernelVolume) return 0;
   size_t bytes = 0;
-  for (int i = 0; i < n_sides; ++i) bytes += order_pairs_workspace_bytes(sides[i].n, (kv + 31) / 32);
+  for (int i = 0; i < n_sides; ++i) bytes += order_pairs_workspace_bytes(sides[i].n, (kv + 31) / 32, coarse);
   return bytes;
 }
+size_t cumm_hip_order_pairs_workspace(const CummHipOrderSide *sides, int n_sides, int kv) {
+  return order_workspace(sides, n_sides, kv, false);
+}
+size_t cumm_hip_order_pairs_coarse_workspace(const CummHipOrderSide *sides, int n_sides, int kv) {
+  return order_workspace(sides, n_sides, kv, true);
+}
 
-int cumm_hip_order_pairs(const CummHipOrderSide *sides, int n_sides, const int32_t *ksize, void *workspace,
-                         size_t workspace_bytes, void *stream) {
+static int order_pairs(const CummHipOrderSide *sides, int n_sides, const int32_t *ksize, void *workspace, size_t workspace_bytes,
+                       bool coarse, void *stream) {
   if (!sides || !ksize || n_sides < 1 || n_sides > 2) return fail(CUMM_HIP_EINVAL, "one or two tables");
   const int64_t kv = (int64_t)ksize[0] * ksize[1] * ksize[2];
   if (ksize[0] < 1 || ksize[1] < 1 || ksize[2] < 1 || kv > kMaxKernelVolume)
@@ -1525,14 +1531,22 @@ int cumm_hip_order_pairs(const CummHipOrderSide *sides, int n_sides, const int32
   if (!any) return CUMM_HIP_OK;
   // (the two tables' hints may hash to one slot: the second one's then stand)
   if (n_sides == 2 && s[0].hint_slot == s[1].hint_slot) s[0].hint_slot = nullptr;
-  const size_t need = cumm_hip_order_pairs_workspace(sides, n_sides, (int)kv);
+  const size_t need = order_workspace(sides, n_sides, (int)kv, coarse);
   if (!workspace || workspace_bytes < need) return fail(CUMM_HIP_ERUNTIME, "workspace at least %zu bytes.", need);
   if (reinterpret_cast<uintptr_t>(workspace) & 255u) return fail(CUMM_HIP_EINVAL, "workspace must be 256-byte aligned");
   int32_t *status = nullptr;
   if (int rc = async_status_ptr(&status)) return rc;
-  const hipError_t e = launch_order_pairs(s, n_sides, (int)kv, ksize, workspace, status + 1, reinterpret_cast<hipStream_t>(stream));
+  const hipError_t e = launch_order_pairs(s, n_sides, (int)kv, ksize, workspace, status + 1, coarse, reinterpret_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "pair order launch");
   return CUMM_HIP_OK;
+}
+int cumm_hip_order_pairs(const CummHipOrderSide *sides, int n_sides, const int32_t *ksize, void *workspace,
+                         size_t workspace_bytes, void *stream) {
+  return order_pairs(sides, n_sides, ksize, workspace, workspace_bytes, false, stream);
+}
+int cumm_hip_order_pairs_coarse(const CummHipOrderSide *sides, int n_sides, const int32_t *ksize, void *workspace,
+                                size_t workspace_bytes, void *stream) {
+  return order_pairs(sides, n_sides, ksize, workspace, workspace_bytes, true, stream);
 }
 
 // ---- weight gradients of the per-offset convolution, all offsets in one launch

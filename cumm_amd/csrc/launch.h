@@ -153,9 +153,9 @@ struct OrderPairsSide {
   int32_t *by_pos, *by_pos_rev;   // [kv, n]; by_pos_rev[kv - 1 - k] = by_pos[k], or NULL
   int32_t *hint_slot;
 };
-size_t order_pairs_workspace_bytes(int n, int words);      // per table
+size_t order_pairs_workspace_bytes(int n, int words, bool coarse);      // per table
 hipError_t launch_order_pairs(const OrderPairsSide *sides, int n_sides, int kv, const int32_t *ksize, void *workspace,
-                              int32_t *give_ups, hipStream_t s);
+                              int32_t *give_ups, bool coarse, hipStream_t s);
 
 // per-offset lists of (input row, output row) out of a pair table [kv, n] (pairs_inst.hip)
 struct PairListsParams {

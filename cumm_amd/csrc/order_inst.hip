@@ -19,6 +19,15 @@
 //     end, from which the convolution kernels start: a launch ends with its longest tile otherwise.
 //     5 x 5 x 5 on 120 k voxels: 47 k (tile, offset) steps against 87 k in the order by count and hash, 46 k
 //     without the weight, but forward 74.8 -> 66.1 us, backward-input 74.8 -> 65.8.
+// Where the caller does not ask for more (coarse), one word and up to 2^20 positions have a key of 11 bits and
+// one pass: exact up to two offsets, the bins above that dealt out by number of offsets, without the middle
+// offset in a submanifold layer's table, which has it everywhere.  The chain is then masks, sums, pass, position:
+// of a frame's tables (120 k and 447 k positions) the second pass was 12 + 16 us of 98, frame of 120 k voxels
+// 239 -> 214.6 us, of 300 k forward and backward 616 -> 580.  (Tile, offset) steps against the key of 18 bits:
+// 1.000 - 1.005 up to 324 k positions, 1.016 at 792 k of a stride-2 table, whose layer (128 -> 256 channels, forward
+// and backward) is none the slower, 851 -> 847 us: rows of one bin stay in their order, neighbours near
+// each other.  At 1 M positions of a submanifold layer it is 1.05 (at 300 k 1.001), and its passes take 791 us for
+// 767: those have two radix passes above 2^19 positions.
 // Chain of kernels: masks, keys and the digits' counts per block of 512 positions - sums of the counts over
 // the blocks - two passes - position.  The first pass knows every chunk's place from the sums, the second
 // looks back (ticket, flagged words); both rank by ballot and are stable.  (Instead of a kernel that clears,
@@ -30,8 +39,9 @@
 // row is little more than a word pair per position (51.5 -> 39.1 us at 1.1 M positions against a fetch of mask
 // and entries).
 // Measured (kernel times): the tables of a frame of 120 k voxels - submanifold and stride 2, 326 k output
-// sites - 98 us in ten launches; with masks by atomics, a sort each and a gather of every entry it
-// was 305 us in 27.
+// sites - 98 us in ten launches, in eight with one pass 71; with masks by atomics, a sort each and a
+// gather of every entry it was 305 us in 27.
+#include <algorithm>
 #include <cstring>
 
 #include "launch.h"
@@ -52,16 +62,25 @@ constexpr int kExact = 5;                                 // offsets up to which
 constexpr uint32_t kAggregate = 1u << 30, kInclusive = 2u << 30, kCount = (1u << 30) - 1u;
 constexpr int kSpins = 1 << 20;                           // (about a second)
 
+// the order of one pass
+constexpr int kOnceDigit = 11, kOnceBins = 1 << kOnceDigit;      // 2048
+constexpr int kOnceExact = 2;                             // offsets up to which its key is exact
+constexpr int kOnceChunk = 1024;                          // positions per workgroup of the pass
+constexpr int kOnceMost = 1 << 20;                        // positions up to which it is taken,
+constexpr int kOnceMostReversed = 1 << 19;                // ... of a submanifold layer's table
+
 struct Side {
   const int32_t *indices;      // [kv, n]
   int32_t n, chunks;
   uint32_t *raw;               // [n, words] masks by row; one word: [n, 2] mask and lead
-  uint32_t *keys;              // [n]
+  uint32_t *keys;              // [n]; one pass: [n] of 16 bits
   int32_t *tmp_rows;           // [n] after the first pass
   uint16_t *tmp_high;          // [n]
   uint32_t *counts[2];         // per pass [rows + 1][kDigitBins]: keys per digit and block of positions, then
                                // the same of the blocks before it, and at the end of all
   int32_t rows;                // blocks
+  uint16_t *once_counts;       // one pass: [rows][kOnceBins] keys per bin and block of positions
+  uint32_t *once_before;       // [chunks + 1][kOnceBins] keys of the chunks before; at the end of all
   uint32_t *state;             // [chunks][kDigitBins] look-back words of the second pass
   uint32_t *ticket;
   uint32_t *sorted;            // [n, words]
@@ -78,31 +97,36 @@ struct OrderParams {
   uint32_t base[kExact + 2];   // first key of the words with c offsets; [kExact + 1]: of those with more
   uint32_t share;              // keys per number of offsets above kExact
   float per_word[33];          // share / number of words with c offsets, c > kExact
+  // one pass: is the middle offset left out of the key (a submanifold layer's masks all have it), the first
+  // key of the words with c (other) offsets, and for c > kOnceExact how many keys they have in all and per word
+  int32_t once_drop;
+  uint32_t once_base[34];
+  float once_per_word[33];
   // planes[i]: the offsets of outer plane i (several words)
   uint32_t planes[12][4];
   uint32_t filter;
 };
 
-// rank of a word among those with as many bits, ascending value: sum of C(position of the i-th bit, i)
-__device__ __forceinline__ uint32_t word_key(const OrderParams &p, uint32_t m) {
-  const int c = __builtin_popcount(m);
-  if (c <= kExact) {
-    uint32_t rank = 0, rest = m;
+// rank of a word among those with as many bits, ascending value: sum of C(position of the i-th bit, i).  Up to
+// kExact bits
+__device__ __forceinline__ uint32_t word_rank(uint32_t rest) {
+  uint32_t rank = 0;
 #pragma unroll
-    for (int i = 1; i <= kExact; ++i) {
-      if (rest == 0u) break;
-      const uint32_t b = (uint32_t)__builtin_ctz(rest);
-      rest &= rest - 1u;
-      uint32_t v = b;                                    // C(b, i)
-      if (i >= 2) v = v * (b - 1u) / 2u;
-      if (i >= 3) v = v * (b - 2u) / 3u;
-      if (i >= 4) v = v * (b - 3u) / 4u;
-      if (i >= 5) v = v * (b - 4u) / 5u;
-      rank += b >= (uint32_t)i ? v : 0u;
-    }
-    return p.base[c] + rank;
+  for (int i = 1; i <= kExact; ++i) {
+    if (rest == 0u) break;
+    const uint32_t b = (uint32_t)__builtin_ctz(rest);
+    rest &= rest - 1u;
+    uint32_t v = b;                                    // C(b, i)
+    if (i >= 2) v = v * (b - 1u) / 2u;
+    if (i >= 3) v = v * (b - 2u) / 3u;
+    if (i >= 4) v = v * (b - 3u) / 4u;
+    if (i >= 5) v = v * (b - 4u) / 5u;
+    rank += b >= (uint32_t)i ? v : 0u;
   }
-  // more offsets: the rank in floating point (its leading digits are all that is kept)
+  return rank;
+}
+// any number of bits: in floating point (its leading digits are all that is kept)
+__device__ __forceinline__ float word_rank_f32(uint32_t m) {
   float rank = 0.0f;
   uint32_t rest = m;
   int i = 1;
@@ -114,8 +138,25 @@ __device__ __forceinline__ uint32_t word_key(const OrderParams &p, uint32_t m) {
     rank += v;
     ++i;
   }
-  const uint32_t at = (uint32_t)(rank * p.per_word[c]);
+  return rank;
+}
+
+__device__ __forceinline__ uint32_t word_key(const OrderParams &p, uint32_t m) {
+  const int c = __builtin_popcount(m);
+  if (c <= kExact) return p.base[c] + word_rank(m);
+  const uint32_t at = (uint32_t)(word_rank_f32(m) * p.per_word[c]);
   return p.base[kExact + 1] + (uint32_t)(c - kExact - 1) * p.share + (at < p.share ? at : p.share - 1u);
+}
+
+// the key of the one pass
+__device__ __forceinline__ uint32_t once_key(const OrderParams &p, uint32_t m) {
+  const int middle = p.kv / 2;
+  if (p.once_drop) m = (m & ((1u << middle) - 1u)) | ((m >> middle >> 1) << middle);
+  const int c = __builtin_popcount(m);
+  if (c <= kOnceExact) return p.once_base[c] + word_rank(m);
+  const float rank = c <= kExact ? (float)word_rank(m) : word_rank_f32(m);
+  const uint32_t at = p.once_base[c] + (uint32_t)(rank * p.once_per_word[c]), last = p.once_base[c + 1] - 1u;
+  return at < last ? at : last;
 }
 
 __device__ __forceinline__ uint32_t words_key(const OrderParams &p, const uint32_t *w) {
@@ -152,17 +193,19 @@ __device__ __forceinline__ int side_of(int first, int *block) {
 // key, the entry of its lowest offset, and how many of the block's keys have which digit, for both
 // passes.  A block's counts are a row of its own, so that nothing has to be zero before.  (Eight positions
 // per lane, one after the other: fewer rows, but 55 us for 27 at 1.1 M positions.)
-template <int WORDS>
+template <int WORDS, bool ONCE = false>
 __global__ __launch_bounds__(kBlock) void order_masks_kernel(const OrderParams p) {
-  __shared__ uint32_t hist[2][kDigitBins];
+  constexpr int kCounts = ONCE ? kOnceBins : 2 * kDigitBins;
+  __shared__ uint32_t hist[kCounts];
   const int t = threadIdx.x, lane = t & 63;
   int block = blockIdx.x;
   const Side &d = p.side[side_of(p.side[0].rows, &block)];
-  static_assert(kBlock == kDigitBins, "a thread per digit");
-  hist[0][t] = hist[1][t] = 0u;
-  if (block % p.rows_per_chunk == 0) d.state[(size_t)(block / p.rows_per_chunk) * kDigitBins + t] = 0u;
+  static_assert(kBlock == kDigitBins && kOnceBins == 4 * kBlock, "a thread per digit, or per four");
+#pragma unroll
+  for (int i = 0; i < kCounts / kBlock; ++i) hist[i * kBlock + t] = 0u;
+  if (!ONCE && block % p.rows_per_chunk == 0) d.state[(size_t)(block / p.rows_per_chunk) * kDigitBins + t] = 0u;
   if (block == 0) {
-    if (t == 0) *d.ticket = 0u;
+    if (!ONCE && t == 0) *d.ticket = 0u;
     if (t < 8 && d.hint_slot != nullptr)   // names no array yet; the two counts start at "everything" / "nothing"
       d.hint_slot[t] = t == 4 ? (d.n / 128) * 128 : (t == 5 ? ((d.n + 63) / 64) * 64 : 0);
   }
@@ -194,7 +237,7 @@ __global__ __launch_bounds__(kBlock) void order_masks_kernel(const OrderParams p
       }
     }
   }
-  const uint32_t key = WORDS == 1 ? word_key(p, w[0]) : words_key(p, w);
+  const uint32_t key = ONCE ? once_key(p, w[0]) : (WORDS == 1 ? word_key(p, w[0]) : words_key(p, w));
   if (on) {
     if constexpr (WORDS == 1) {
       reinterpret_cast<uint2 *>(d.raw)[o] = uint2{w[0], self ? lead | kSelf : lead};
@@ -202,22 +245,36 @@ __global__ __launch_bounds__(kBlock) void order_masks_kernel(const OrderParams p
 #pragma unroll
       for (int q = 0; q < WORDS; ++q) d.raw[(int64_t)o * WORDS + q] = w[q];
     }
-    d.keys[o] = key;
+    if constexpr (ONCE) reinterpret_cast<uint16_t *>(d.keys)[o] = (uint16_t)key;
+    else d.keys[o] = key;
   }
   // most waves of a sparse cloud hold one key: one add for all lanes
   const unsigned long long live = __ballot(on);
   if (live != 0ull) {
     const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)key);
     if (__ballot(on && key == first) == live) {
-      if (lane < 2) atomicAdd(&hist[lane][(first >> (lane * kDigit)) & (kDigitBins - 1)], (uint32_t)__popcll(live));
+      if constexpr (ONCE) {
+        if (lane == 0) atomicAdd(&hist[first], (uint32_t)__popcll(live));
+      } else if (lane < 2) {
+        atomicAdd(&hist[lane * kDigitBins + ((first >> (lane * kDigit)) & (kDigitBins - 1))], (uint32_t)__popcll(live));
+      }
     } else if (on) {
-      atomicAdd(&hist[0][key & (kDigitBins - 1)], 1u);
-      atomicAdd(&hist[1][key >> kDigit], 1u);
+      if constexpr (ONCE) {
+        atomicAdd(&hist[key], 1u);
+      } else {
+        atomicAdd(&hist[key & (kDigitBins - 1)], 1u);
+        atomicAdd(&hist[kDigitBins + (key >> kDigit)], 1u);
+      }
     }
   }
   __syncthreads();
-  d.counts[0][(size_t)block * kDigitBins + t] = hist[0][t];
-  d.counts[1][(size_t)block * kDigitBins + t] = hist[1][t];
+  if constexpr (ONCE) {
+    const v4i c = reinterpret_cast<const v4i *>(hist)[t];
+    reinterpret_cast<uint2 *>(d.once_counts + (size_t)block * kOnceBins)[t] = uint2{(uint32_t)(c.x | c.y << 16), (uint32_t)(c.z | c.w << 16)};
+  } else {
+    d.counts[0][(size_t)block * kDigitBins + t] = hist[t];
+    d.counts[1][(size_t)block * kDigitBins + t] = hist[kDigitBins + t];
+  }
 }
 
 // blocks per run of the scan: whole chunks of the first pass
@@ -270,6 +327,100 @@ __global__ __launch_bounds__(1024) void order_scan_kernel(const OrderParams p) {
       before += v[u];
     }
   }
+}
+
+// The same for the one pass: 32 bins of a table per workgroup, two per thread (16-bit counts of blocks), the
+// sums before every chunk and the totals as 32 bits.  ROWS takes a run in one trip.
+template <int ROWS>
+__global__ __launch_bounds__(1024) void order_once_scan_kernel(const OrderParams p) {
+  __shared__ uint2 run_sum[64][16];
+  static_assert(ROWS % kLowBlocks == 0 && kLowBlocks * kBlock == kOnceChunk, "two blocks of a run are a chunk");
+  const int pair = threadIdx.x & 15, run = threadIdx.x >> 4;
+  const Side &d = p.side[blockIdx.y];
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(d.once_counts, 0, (int)((uint32_t)d.rows * (kOnceBins * 2u)), 0x00020000);
+  const uint32_t col = (uint32_t)(blockIdx.x * 16 + pair);
+  const int per = scan_run(d.rows), r0 = run * per, r1 = r0 + per < d.rows ? r0 + per : d.rows;
+  uint32_t v[ROWS];
+  uint2 sum = {0u, 0u}, before = {0u, 0u}, all = {0u, 0u};
+#pragma unroll
+  for (int u = 0; u < ROWS; ++u)      // (past the run's end: outside the matrix)
+    v[u] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, u < per && r0 + u < r1 ? (uint32_t)(r0 + u) * (kOnceBins * 2u) + col * 4u : kNowhere, 0, 0);
+#pragma unroll
+  for (int u = 0; u < ROWS; ++u) {
+    sum.x += v[u] & 0xFFFFu;
+    sum.y += v[u] >> 16;
+  }
+  run_sum[run][pair] = sum;
+  __syncthreads();
+#pragma unroll 16
+  for (int i = 0; i < 64; ++i) {
+    const uint2 x = run_sum[i][pair];
+    before.x += i < run ? x.x : 0u;
+    before.y += i < run ? x.y : 0u;
+    all.x += x.x;
+    all.y += x.y;
+  }
+  uint2 *to = reinterpret_cast<uint2 *>(d.once_before) + col;
+  if (run == 0) to[(size_t)d.chunks * (kOnceBins / 2)] = all;
+#pragma unroll
+  for (int u = 0; u < ROWS; ++u) {
+    if (u % kLowBlocks == 0 && u < per && r0 + u < r1) to[(size_t)((r0 + u) / kLowBlocks) * (kOnceBins / 2)] = before;
+    before.x += v[u] & 0xFFFFu;
+    before.y += v[u] >> 16;
+  }
+}
+
+// The one pass: a position per lane, its place = keys below its own + equal ones in the chunks before + in the
+// waves before + in the lanes before.  A wave's lanes of one key are found by ballot; their number, one byte,
+// goes to the key's 16 bytes, one for each wave, of which a lane adds up those before its own in four
+// instructions (a histogram of words per wave, added up bin by bin, would be 128 KB and 32 reads per thread).
+__global__ __launch_bounds__(kOnceChunk) void order_once_pass_kernel(const OrderParams p) {
+  constexpr int kWaves = kOnceChunk / 64;
+  static_assert(kWaves == 16 && kOnceBins == 2 * kOnceChunk, "sixteen bytes per bin, two bins per thread");
+  __shared__ v4i wave_counts[kOnceBins];
+  __shared__ uint32_t first[kOnceBins];
+  __shared__ uint32_t wave_sum[kWaves];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  int chunk = blockIdx.x;
+  const Side &d = p.side[side_of(p.side[0].chunks, &chunk)];
+  const int pos = chunk * kOnceChunk + t;
+  const bool on = pos < d.n;
+  const uint32_t key = reinterpret_cast<const uint16_t *>(d.keys)[on ? pos : d.n - 1];
+  const uint2 total = reinterpret_cast<const uint2 *>(d.once_before + (size_t)d.chunks * kOnceBins)[t];
+  wave_counts[t] = wave_counts[t + kOnceChunk] = v4i{0, 0, 0, 0};
+  const uint32_t before_chunk = d.once_before[(size_t)chunk * kOnceBins + key];
+  // first place of each bin: exclusive prefix over the totals
+  uint32_t incl = total.x + total.y;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t up = (uint32_t)__shfl_up((int)incl, off, 64);
+    if (lane >= off) incl += up;
+  }
+  if (lane == 63) wave_sum[wave] = incl;
+  unsigned long long peers = __ballot(on);
+#pragma unroll
+  for (int b = 0; b < kOnceDigit; ++b) {
+    const unsigned long long has = __ballot((key >> b) & 1u);
+    peers &= ((key >> b) & 1u) ? has : ~has;
+  }
+  const uint32_t rank = (uint32_t)__popcll(peers & ((1ull << lane) - 1ull));
+  __syncthreads();
+  if (on && rank == 0u) reinterpret_cast<uint8_t *>(&wave_counts[key])[wave] = (uint8_t)__popcll(peers);
+  uint32_t base = incl - total.x - total.y;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) base += w < wave ? wave_sum[w] : 0u;
+  reinterpret_cast<uint2 *>(first)[t] = uint2{base, base + total.x};
+  __syncthreads();
+  if (!on) return;
+  uint32_t dst = first[key] + before_chunk + rank;
+  const v4i c = wave_counts[key];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int bytes = wave - 4 * i;      // waves of these four before this one
+    const uint32_t those = bytes >= 4 ? ~0u : (bytes > 0 ? (1u << (8 * bytes)) - 1u : 0u);
+    dst = __builtin_amdgcn_sad_u8((uint32_t)c[i] & those, 0u, dst);
+  }
+  d.order[dst] = pos;
 }
 
 // One pass over one digit (LOW: the low one, rows in ascending order to tmp; else the high one, tmp to
@@ -507,15 +658,59 @@ int mask_rows(int n) { return (int)(((int64_t)n + kBlock - 1) / kBlock); }
 
 }  // namespace
 
-size_t order_pairs_workspace_bytes(int n, int words) {
+size_t order_pairs_workspace_bytes(int n, int words, bool coarse) {
   const size_t nn = (size_t)(n > 0 ? n : 1);
+  if (coarse && words == 1 && n <= kOnceMost) {
+    const size_t rows = (size_t)mask_rows((int)nn), chunks = (nn + kOnceChunk - 1) / kOnceChunk;
+    const size_t once = up256(8 * nn) + up256(2 * nn) + up256(2 * rows * kOnceBins) + up256(4 * (chunks + 1) * kOnceBins);
+    return std::max(once, order_pairs_workspace_bytes(n, words, false));      // (the other table may be larger)
+  }
   const size_t chunks = (nn + 4095) / 4096;
   return up256(4 * nn * (words == 1 ? 2 : words)) + 2 * up256(4 * nn) + up256(2 * nn) + 2 * up256(4 * ((size_t)mask_rows((int)nn) + 1) * kDigitBins) +
          up256(4 * chunks * kDigitBins) + 256;
 }
 
+// Keys of the one pass: exact up to kOnceExact offsets, and what is left of the bins dealt out to the larger
+// numbers of offsets, 0.6 of the rest to each (a cloud's masks thin out at about that rate, and at least one).
+static void once_keys(OrderParams &p) {
+  const int bits = p.kv - p.once_drop;
+  double choose = 1.0;
+  uint32_t next = 0;
+  for (int c = 0; c <= bits; ++c) {
+    p.once_base[c] = next;
+    uint32_t keys = (uint32_t)choose;
+    if (c > kOnceExact) {
+      const uint32_t left = (uint32_t)kOnceBins - next, others = (uint32_t)(bits - c);
+      keys = c == bits ? 1u : (uint32_t)std::min({choose, 0.6 * left, (double)(left - others)});
+      if (keys == 0u) keys = 1u;
+      p.once_per_word[c] = (float)((double)keys / choose);
+    }
+    next += keys;
+    choose = choose * (bits - c) / (c + 1);
+  }
+  p.once_base[bits + 1] = next;
+}
+
+static hipError_t launch_order_once(OrderParams &p, hipStream_t s) {
+  int rows = 0, chunks = 0, blocks = 0, run = 0;
+  for (int i = 0; i < p.sides; ++i) {
+    rows += p.side[i].rows;
+    chunks += p.side[i].chunks;
+    blocks += (p.side[i].n + 255) / 256;
+    run = std::max(run, scan_run(p.side[i].rows));
+  }
+  hipLaunchKernelGGL((order_masks_kernel<1, true>), dim3(rows), dim3(kBlock), 0, s, p);
+  const dim3 scan_grid(kOnceBins / 32, p.sides);
+  static_assert(kOnceMost / kBlock <= 64 * 32, "a run fits the largest trip");
+  if (run <= 8) hipLaunchKernelGGL(order_once_scan_kernel<8>, scan_grid, dim3(1024), 0, s, p);
+  else hipLaunchKernelGGL(order_once_scan_kernel<32>, scan_grid, dim3(1024), 0, s, p);
+  hipLaunchKernelGGL(order_once_pass_kernel, dim3(chunks), dim3(kOnceChunk), 0, s, p);
+  hipLaunchKernelGGL(order_position_kernel<1>, dim3(blocks), dim3(256), 0, s, p);
+  return hipGetLastError();
+}
+
 hipError_t launch_order_pairs(const OrderPairsSide *sides, int n_sides, int kv, const int32_t *ksize, void *workspace,
-                              int32_t *give_ups, hipStream_t s) {
+                              int32_t *give_ups, bool coarse, hipStream_t s) {
   OrderParams p;
   std::memset(&p, 0, sizeof(p));
   p.kv = kv; p.words = (kv + 31) / 32; p.give_ups = give_ups;
@@ -525,7 +720,9 @@ hipError_t launch_order_pairs(const OrderPairsSide *sides, int n_sides, int kv, 
   int most = 0;
   for (int i = 0; i < n_sides; ++i)
     if (sides[i].n > 0 && sides[i].n > most) most = sides[i].n;
-  const int items = pass_items(most), chunk = kPassThreads * items;
+  bool once = coarse && p.words == 1;
+  for (int i = 0; i < n_sides; ++i) once = once && sides[i].n <= (sides[i].by_pos_rev != nullptr ? kOnceMostReversed : kOnceMost);
+  const int items = pass_items(most), chunk = once ? kOnceChunk : kPassThreads * items;
   p.rows_per_chunk = chunk / kBlock;
   for (int i = 0; i < n_sides; ++i) {
     if (sides[i].n <= 0) continue;
@@ -536,16 +733,30 @@ hipError_t launch_order_pairs(const OrderPairsSide *sides, int n_sides, int kv, 
     d.hint_slot = p.words == 1 ? sides[i].hint_slot : nullptr;
     char *const begin = at;
     d.raw = reinterpret_cast<uint32_t *>(take(4 * n * (p.words == 1 ? 2 : p.words)));
+    d.rows = mask_rows(d.n);
+    if (once) {
+      d.keys = reinterpret_cast<uint32_t *>(take(2 * n));
+      d.once_counts = reinterpret_cast<uint16_t *>(take(2 * (size_t)d.rows * kOnceBins));
+      d.once_before = reinterpret_cast<uint32_t *>(take(4 * ((size_t)d.chunks + 1) * kOnceBins));
+      if (d.by_pos_rev != nullptr) p.once_drop = 1;      // (the table of a submanifold layer)
+      at = begin + order_pairs_workspace_bytes(d.n, p.words, coarse);
+      continue;
+    }
     d.keys = reinterpret_cast<uint32_t *>(take(4 * n));
     d.tmp_rows = reinterpret_cast<int32_t *>(take(4 * n));
     d.tmp_high = reinterpret_cast<uint16_t *>(take(2 * n));
-    d.rows = mask_rows(d.n);
     for (uint32_t *&c : d.counts) c = reinterpret_cast<uint32_t *>(take(4 * ((size_t)d.rows + 1) * kDigitBins));
     d.state = reinterpret_cast<uint32_t *>(take(4 * (size_t)d.chunks * kDigitBins));
     d.ticket = reinterpret_cast<uint32_t *>(take(256));
-    at = begin + order_pairs_workspace_bytes(d.n, p.words);
+    at = begin + order_pairs_workspace_bytes(d.n, p.words, coarse);
   }
   if (p.sides == 0) return hipSuccess;
+  if (once) {
+    p.give_ups = nullptr;      // (nothing looks back)
+    p.once_drop = p.sides == 1 ? p.once_drop : 0;
+    once_keys(p);
+    return launch_order_once(p, s);
+  }
   if (p.words == 1) {
     // words of kv bits with c offsets: C(kv, c)
     double choose = 1.0;

@@ -51,8 +51,8 @@ struct Api {
   CUMM_API(conv_pairs_workspace);
   CUMM_API(conv_pairs_sites);
   CUMM_API(conv_pairs_fill);
-  CUMM_API(order_pairs);
-  CUMM_API(order_pairs_workspace);
+  CUMM_API(order_pairs_coarse);
+  CUMM_API(order_pairs_coarse_workspace);
 #undef CUMM_API
 } api;
 
@@ -73,8 +73,8 @@ void bind(const py::dict &addresses) {
   CUMM_API(conv_pairs_workspace);
   CUMM_API(conv_pairs_sites);
   CUMM_API(conv_pairs_fill);
-  CUMM_API(order_pairs);
-  CUMM_API(order_pairs_workspace);
+  CUMM_API(order_pairs_coarse);
+  CUMM_API(order_pairs_coarse_workspace);
 #undef CUMM_API
 }
 
@@ -231,8 +231,8 @@ py::tuple build(const Tensor &coords, const Three &shape, const Three &ksize, co
         sides[0].by_position_reversed = g->indices_bwd_pos;
         count = 1;
       }
-      const Tensor ws = bytes((int64_t)api.order_pairs_workspace(sides, count, g->kv), g->device);
-      check(api.order_pairs(sides, count, ksize.data(), ws.data_ptr(), (size_t)ws.numel(), s));
+      const Tensor ws = bytes((int64_t)api.order_pairs_coarse_workspace(sides, count, g->kv), g->device);
+      check(api.order_pairs_coarse(sides, count, ksize.data(), ws.data_ptr(), (size_t)ws.numel(), s));
     }
   }
   return py::make_tuple(g, out_coords, py::make_tuple(out_shape[0], out_shape[1], out_shape[2]), ordered);

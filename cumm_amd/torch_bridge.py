@@ -169,8 +169,8 @@ _KINDS = {}
 
 _NATIVE_SYMBOLS = ("sparse_conv", "last_error", "relu_backward", "relu_backward_sums", "column_sum", "column_sum_workspace",
                    "query_conv_workspace", "query_wgrad_ordered_workspace", "wgrad_pairs", "wgrad_pairs_workspace", "subm_pairs",
-                   "subm_pairs_workspace", "conv_pairs_workspace", "conv_pairs_sites", "conv_pairs_fill", "order_pairs",
-                   "order_pairs_workspace")
+                   "subm_pairs_workspace", "conv_pairs_workspace", "conv_pairs_sites", "conv_pairs_fill", "order_pairs_coarse",
+                   "order_pairs_coarse_workspace")
 _native_module = None
 
 
@@ -314,8 +314,8 @@ class SparseConvGeometry:
         count = 2
         if self.subm:      # (one order serves both; the backward table is the forward one with its offsets reversed)
             sides[0].by_position_reversed, count = p["indices_bwd_pos"], 1
-        ws = _bytes(lib.cumm_hip_order_pairs_workspace(sides, count, self.kv), dev)
-        _capi.check(lib.cumm_hip_order_pairs(sides, count, ks, ws.data_ptr(), ws.numel(), s))
+        ws = _bytes(lib.cumm_hip_order_pairs_coarse_workspace(sides, count, self.kv), dev)
+        _capi.check(lib.cumm_hip_order_pairs_coarse(sides, count, ks, ws.data_ptr(), ws.numel(), s))
         return True
 
     @property

@@ -396,6 +396,13 @@ typedef struct CummHipOrderSide {
 size_t cumm_hip_order_pairs_workspace(const CummHipOrderSide *sides, int n_sides, int kv);
 int cumm_hip_order_pairs(const CummHipOrderSide *sides, int n_sides, const int32_t *ksize, void *workspace,
                          size_t workspace_bytes, void *stream);
+/* The same, where an order that repeats and groups like masks is enough: of tables of one mask word and
+ * up to 2^20 positions (2^19 with by_position_reversed) it is exact up to two offsets only (with
+ * by_position_reversed, alone: two beside the middle one, which does not count), which takes one radix pass
+ * instead of two; everything else as above. */
+size_t cumm_hip_order_pairs_coarse_workspace(const CummHipOrderSide *sides, int n_sides, int kv);
+int cumm_hip_order_pairs_coarse(const CummHipOrderSide *sides, int n_sides, const int32_t *ksize, void *workspace,
+                                size_t workspace_bytes, void *stream);
 
 /* Backward-weight of the per-offset convolution for all offsets at once:
  *   dw[:, r, :] = sum over i < counts[r] of dout[pair_out[r][i]]^T inp[pair_in[r][i]]

@@ -21,7 +21,7 @@ def _table(rng, kv, n, density):
     return t
 
 
-def _order(tables, ksize, reverse):
+def _order(tables, ksize, reverse, entry="cumm_hip_order_pairs"):
     lib, kv = _capi.lib(), tables[0].shape[0]
     words = (kv + 31) // 32
     sides, keep, outs = (_capi.OrderSide * 2)(), [], []
@@ -35,9 +35,9 @@ def _order(tables, ksize, reverse):
         s.by_position_reversed = o["rev"].byte_pointer() if reverse else None
         keep.append(d)
         outs.append(o)
-    need = int(lib.cumm_hip_order_pairs_workspace(sides, len(tables), kv))
+    need = int(getattr(lib, entry + "_workspace")(sides, len(tables), kv))
     ws = H.dev(np.full(need, 0xA5, np.uint8), "u8")
-    _capi.check(lib.cumm_hip_order_pairs(sides, len(tables), (ctypes.c_int32 * 3)(*ksize), ws.byte_pointer(), ws.nbytes, 0))
+    _capi.check(getattr(lib, entry)(sides, len(tables), (ctypes.c_int32 * 3)(*ksize), ws.byte_pointer(), ws.nbytes, 0))
     _capi.check(lib.cumm_hip_device_synchronize())
     return [{k: H.host(v) for k, v in o.items()} for o in outs], outs
 
@@ -139,3 +139,39 @@ def test_most_positions():
         rows = order[begin:end]
         assert bool((rows[1:] > rows[:-1]).all()) and int(rows[0]) >= 0 and int(rows[-1]) < n
         assert bool((by_position[begin:end] == (rows if want else -1)).all())
+
+
+@pytest.mark.parametrize("ksize,n,n2", [((3, 3, 3), 1, 0), ((3, 3, 3), 1023, 0), ((3, 3, 3), 1025, 64), ((4, 4, 2), 5000, 0), ((1, 1, 1), 700, 0),
+                                        ((1, 1, 2), 1024, 2049), ((3, 3, 3), 512 * 128 + 1, 0), ((3, 3, 3), 512 * 128 * 4 + 513, 1000),
+                                        ((2, 2, 2), 1 << 20, 3), ((2, 2, 2), 3, (1 << 20) + 1), ((2, 2, 2), 1 << 19, 0), ((5, 5, 5), 3000, 0)])
+def test_one_pass(ksize, n, n2):
+    """cumm_hip_order_pairs_coarse: a permutation that repeats, ascending by number of offsets (without the middle
+    one where a reversed table is asked for), stable and exact up to two of them; tables and hints as always.
+    Chunks of 1024 positions, runs of 8 and 32 blocks, the last table that takes one pass and the first of two."""
+    print("case one pass", ksize, n, n2, flush=True)
+    rng, kv, reverse = np.random.default_rng(n + n2), int(np.prod(ksize)), n2 == 0
+    tables = [_table(rng, kv, m, 0.08 if kv > 8 else 0.3) for m in (n, n2) if m]
+    got, dev = _order(tables, ksize, reverse, "cumm_hip_order_pairs_coarse")
+    again, _ = _order(tables, ksize, reverse, "cumm_hip_order_pairs_coarse")
+    for t, g, a, d in zip(tables, got, again, dev):
+        m = pairs.masks_from_pairs(t)
+        order = g["order"]
+        assert np.array_equal(np.sort(order), np.arange(t.shape[1])) and np.array_equal(order, a["order"])
+        np.testing.assert_array_equal(g["mask"], m[order])
+        np.testing.assert_array_equal(g["pos"], pairs.pairs_by_position(t, order))
+        if reverse:
+            np.testing.assert_array_equal(g["rev"], g["pos"][::-1])
+        if m.shape[1] > 1:
+            continue
+        word = m[:, 0].astype(np.int64)
+        if reverse:
+            low = (1 << (kv // 2)) - 1
+            word = (word & low) | (word >> (kv // 2 + 1) << (kv // 2))
+        count = sum((word >> b) & 1 for b in range(kv))
+        assert np.all(np.diff(count[order]) >= 0)
+        exact = int((count <= 2).sum())
+        np.testing.assert_array_equal(order[:exact], np.lexsort((word, count))[:exact])
+        bits, s = (1 << kv) - 1 if kv < 32 else 0xFFFFFFFF, g["mask"][:, 0]
+        hints = pairs.hints_device(d["mask"].view([t.shape[1]]), bits)
+        if hints != (-1, -1) and (t is tables[-1] or t.shape[1] != tables[-1].shape[1]):
+            assert hints[0] == pairs.light_prefix(s, bits, 3)
