@@ -60,6 +60,10 @@ class SparseConvArgs(C.Structure):
                 ("ungated_rows", C.c_int32), ("indices_by_position", C.c_int32), ("mask_int_count", C.c_int32)]
 
 
+class SparseConvMore(C.Structure):
+    _fields_ = [("write_empty", C.c_int32)]
+
+
 class OrderSide(C.Structure):
     _fields_ = [("indices", C.c_void_p), ("n", C.c_int32), ("sorted_mask", C.c_void_p), ("argsort", C.c_void_p),
                 ("by_position", C.c_void_p), ("by_position_reversed", C.c_void_p)]
@@ -71,6 +75,7 @@ SYMBOLS = {
     "cumm_hip_gemm": (C.c_int, [C.POINTER(GemmDesc), C.POINTER(GemmArgs), _VP]),
     "cumm_hip_gemm_in_workspace": (C.c_int, [C.POINTER(GemmDesc), C.POINTER(GemmArgs), _VP]),
     "cumm_hip_sparse_conv": (C.c_int, [C.POINTER(ConvDesc), C.POINTER(SparseConvArgs), _VP]),
+    "cumm_hip_sparse_conv_more": (C.c_int, [C.POINTER(ConvDesc), C.POINTER(SparseConvArgs), C.POINTER(SparseConvMore), _VP]),
     "cumm_hip_sparse_conv_static_ws": (C.c_int, [C.POINTER(ConvDesc), C.POINTER(SparseConvArgs), _VP]),
     "cumm_hip_query_gemm_workspace": (C.c_int64, [C.POINTER(GemmDesc), C.c_int, C.c_int, C.c_int, C.c_int]),
     "cumm_hip_query_gemm_optional_workspace": (C.c_int64, [C.POINTER(GemmDesc), C.c_int, C.c_int, C.c_int]),

@@ -322,7 +322,7 @@ int report_async_errors() {
   return CUMM_HIP_OK;
 }
 
-int sparse_conv_impl(const CummHipConvDesc *desc, const CummHipSparseConvArgs *a, void *stream_, void *workspace,
+int sparse_conv_impl(const CummHipConvDesc *desc, const CummHipSparseConvArgs *a, const CummHipSparseConvMore *more, void *stream_, void *workspace,
                      size_t workspace_bytes, size_t workspace_cap);
 
 // workspace of the fixed-order backward-weight: live-tile counts (128 bytes), the table of the
@@ -733,14 +733,20 @@ int cumm_hip_gemm_in_workspace(const CummHipGemmDesc *desc, const CummHipGemmArg
 // ---------------------------------------------------------------------------------------------
 int cumm_hip_sparse_conv(const CummHipConvDesc *desc, const CummHipSparseConvArgs *a, void *stream_) {
   if (!desc || !a) return fail(CUMM_HIP_EINVAL, "null descriptor or arguments");
-  return sparse_conv_impl(desc, a, stream_, a->workspace, a->workspace_bytes, 0);
+  return sparse_conv_impl(desc, a, nullptr, stream_, a->workspace, a->workspace_bytes, 0);
+}
+
+int cumm_hip_sparse_conv_more(const CummHipConvDesc *desc, const CummHipSparseConvArgs *a, const CummHipSparseConvMore *more,
+                              void *stream_) {
+  if (!desc || !a) return fail(CUMM_HIP_EINVAL, "null descriptor or arguments");
+  return sparse_conv_impl(desc, a, more, stream_, a->workspace, a->workspace_bytes, 0);
 }
 
 int cumm_hip_sparse_conv_static_ws(const CummHipConvDesc *desc, const CummHipSparseConvArgs *a, void *stream_) {
   if (!desc || !a) return fail(CUMM_HIP_EINVAL, "null descriptor or arguments");
   void *ws = nullptr;
   if (int rc = static_scratch(&ws)) return rc;
-  return sparse_conv_impl(desc, a, stream_, ws, CUMM_HIP_STATIC_WORKSPACE_BYTES, CUMM_HIP_STATIC_WORKSPACE_BYTES);
+  return sparse_conv_impl(desc, a, nullptr, stream_, ws, CUMM_HIP_STATIC_WORKSPACE_BYTES, CUMM_HIP_STATIC_WORKSPACE_BYTES);
 }
 
 }  // extern "C"
@@ -748,7 +754,7 @@ int cumm_hip_sparse_conv_static_ws(const CummHipConvDesc *desc, const CummHipSpa
 namespace {
 // workspace_cap != 0: the workspace is the library's own array of that size, and a problem that
 // needs more is an argument error (the caller cannot make it larger)
-int sparse_conv_impl(const CummHipConvDesc *desc, const CummHipSparseConvArgs *a, void *stream_, void *workspace,
+int sparse_conv_impl(const CummHipConvDesc *desc, const CummHipSparseConvArgs *a, const CummHipSparseConvMore *more, void *stream_, void *workspace,
                      size_t workspace_bytes, size_t workspace_cap) {
   const CummHipConvDesc &c = *desc;
   const CummHipGemmDesc &d = c.gemm;
@@ -805,7 +811,7 @@ int sparse_conv_impl(const CummHipConvDesc *desc, const CummHipSparseConvArgs *a
       p.rows_a = a->rows_out; p.rows_c = a->rows_in;
       p.w_stride_n = 1; p.w_stride_k = a->C; p.w_stride_c = (int64_t)kv * a->C;
       p.reverse_mask = a->reverse_mask;
-      p.exit_on_empty = 1;
+      p.exit_on_empty = more == nullptr || more->write_empty == 0;
     }
     p.ldd = a->d_is_bias ? 0 : p.ldc;
     p.alpha = a->alpha; p.beta = a->beta; p.act_alpha = a->act_alpha; p.act_beta = a->act_beta;

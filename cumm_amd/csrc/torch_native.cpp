@@ -37,6 +37,7 @@ namespace {
 struct Api {
 #define CUMM_API(name) decltype(&::cumm_hip_##name) name = nullptr
   CUMM_API(sparse_conv);
+  CUMM_API(sparse_conv_more);
   CUMM_API(last_error);
   CUMM_API(relu_backward);
   CUMM_API(relu_backward_sums);
@@ -59,6 +60,7 @@ struct Api {
 void bind(const py::dict &addresses) {
 #define CUMM_API(name) api.name = reinterpret_cast<decltype(api.name)>(addresses["cumm_hip_" #name].cast<uintptr_t>())
   CUMM_API(sparse_conv);
+  CUMM_API(sparse_conv_more);
   CUMM_API(last_error);
   CUMM_API(relu_backward);
   CUMM_API(relu_backward_sums);
@@ -406,12 +408,14 @@ struct SparseConvBackward : public torch::autograd::Node {
       gy = gated;
     }
     if (need[0]) {
-      // inputs that feed no output site sit in tiles the kernel skips (mask 0): zero them
-      result[0] = g->subm ? at::empty_like(x) : at::zeros_like(x);
+      // inputs that feed no output site lie in tiles of mask 0: the kernel writes their zeros
+      result[0] = at::empty_like(x);
+      CummHipSparseConvMore more = {};
+      more.write_empty = 1;
       CummHipSparseConvArgs a = moved(*dgrad, *g, g->n_in, g->indices_bwd_pos, g->mask_bwd, g->order_bwd, nullptr);
       a.ptr_A = gy.data_ptr(); a.ptr_B = w.data_ptr();
       a.ptr_C = result[0].data_ptr(); a.ptr_D = a.ptr_C;
-      check(api.sparse_conv(&dgrad->desc, &a, s));
+      check(api.sparse_conv_more(&dgrad->desc, &a, &more, s));
       g->made[1] = true;
     }
     if (need[1] && wgrad) {

@@ -163,6 +163,12 @@ typedef struct CummHipSparseConvArgs {
                                        Any other value than that is an error. */
 } CummHipSparseConvArgs;
 
+/* What a training program wants of the same launches beyond the reference's argument block; all zero = nothing. */
+typedef struct CummHipSparseConvMore {
+  int32_t write_empty;              /* backward-input.  Non-zero: rows of tiles without any kernel offset are written like
+                                       all others (zeros, with beta == 0), not left alone: the caller fills nothing */
+} CummHipSparseConvMore;
+
 /* Replaces GemmMainUnitTest.matmul2 below its prelude
  * (cumm/gemm/main.py:1176-1335: dispatch on the descriptor and launch). */
 int cumm_hip_gemm(const CummHipGemmDesc *desc, const CummHipGemmArgs *args, void *stream);
@@ -176,6 +182,9 @@ int cumm_hip_gemm_in_workspace(const CummHipGemmDesc *desc, const CummHipGemmArg
  * descriptors (cumm/conv/main.py:483-745). */
 int cumm_hip_sparse_conv(const CummHipConvDesc *desc, const CummHipSparseConvArgs *args,
                          void *stream);
+/* The same with more (NULL = the call above). */
+int cumm_hip_sparse_conv_more(const CummHipConvDesc *desc, const CummHipSparseConvArgs *args, const CummHipSparseConvMore *more,
+                              void *stream);
 
 /* cumm_hip_sparse_conv for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc) and so cannot provide the
