@@ -3,12 +3,17 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace cummhip {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 
 constexpr int kWave = 64;
 
@@ -34,6 +39,10 @@ template <> struct Elem<F16> {
   static __device__ __forceinline__ uint16_t from_float(float x) {
     return __builtin_bit_cast(uint16_t, (_Float16)x);  // v_cvt_f16_f32: round to nearest even
   }
+  // two of them, the first in the low half (v_cvt_pk_f16_f32: the same bits)
+  static __device__ __forceinline__ uint32_t from_floats(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{a, b}, v2h));
+  }
 };
 template <> struct Elem<BF16> {
   using Acc = float;
@@ -49,12 +58,15 @@ template <> struct Elem<BF16> {
     return __builtin_bit_cast(float, (uint32_t)bits << 16);
   }
   // round to nearest even on bit 16, NaN -> 0x7FFF
-  // (bfloat16_t(float), include/tensorview/gemm/dtypes/bfloat16.h:86-111 of the reference)
+  // (bfloat16_t(float), include/tensorview/gemm/dtypes/bfloat16.h:86-111 of the reference): the hardware's
+  // conversion, which gives these bits for everything but NaN, denormals among it (all 2^32 compared)
   static __device__ __forceinline__ uint16_t from_float(float x) {
-    uint32_t u = __builtin_bit_cast(uint32_t, x);
-    if (x != x) return 0x7FFF;
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
+    const uint16_t h = (uint16_t)from_floats(x, x);
+    return x != x ? (uint16_t)0x7FFF : h;
+  }
+  // two of them, the first in the low half; NaN becomes some NaN
+  static __device__ __forceinline__ uint32_t from_floats(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{a, b}, v2bf));
   }
 };
 template <> struct Elem<S8> {
@@ -67,6 +79,25 @@ template <> struct Elem<S8> {
     return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0);
   }
 };
+
+// Eight results rounded and packed, as from_float rounds each: half an instruction per element, and for bf16
+// another half that looks for NaN.  NUMBERS: there is none among them.
+template <class T, bool NUMBERS>
+__device__ __forceinline__ v4i round8(const float (&t)[8]) {
+  v4i v;
+#pragma unroll
+  for (int x = 0; x < 4; ++x) v[x] = (int)Elem<T>::from_floats(t[2 * x], t[2 * x + 1]);
+  if constexpr (std::is_same_v<T, BF16> && !NUMBERS) {
+    bool nan = false;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) nan |= __builtin_isunordered(t[2 * x], t[2 * x + 1]);
+    if (__builtin_expect(nan, 0)) {
+#pragma unroll
+      for (int x = 0; x < 4; ++x) v[x] = (int)((uint32_t)Elem<T>::from_float(t[2 * x]) | (uint32_t)Elem<T>::from_float(t[2 * x + 1]) << 16);
+    }
+  }
+  return v;
+}
 
 // activations: UnaryActivation, cumm/gemm/gemmmath/__init__.py:181-214 of the reference
 __device__ __forceinline__ float apply_act(float x, int act, float act_alpha) {

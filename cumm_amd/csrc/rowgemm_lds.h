@@ -538,11 +538,13 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
   };
   typedef int src_vec __attribute__((ext_vector_type(SRC_W)));
   src_vec src_pre[RBW][SRC_N] = {};
+  const bool shared_src = E::kBytes == 2 && p.ldd == 0;      // one row for all (a bias): fetched and converted once
   if (p.read_source && !WIDE) {   // (four-byte outputs read their source in the epilogue)
     const v4i rsw_d = rsrc_words(p.D, p.d_bytes);
 #pragma unroll
     for (int rb = 0; rb < RBW; ++rb) {
-      const int o = out_row[rb];
+      // (every load is issued, whatever it is for: behind a branch its register could be copied before it lands)
+      const int o = shared_src ? (rb == 0 ? 0 : -1) : out_row[rb];
       const bool row_ok = o >= 0 && o < p.rows_c;
 #pragma unroll
       for (int i = 0; i < SRC_N; ++i) {
@@ -715,13 +717,28 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
     }
     return;
   }
-  // MODE: 0 = alpha*acc, 1 = alpha*acc + beta*src, 2 = scale*acc + bias, 3 = ... + beta*src
+  // MODE: 0 = alpha*acc, 1 = alpha*acc + beta*src, 2 = scale*acc + bias, 3 = ... + beta*src, 4 = as 1 with one
+  // row of src for all.
+  // An element of a ReLU layer with a bias takes 2.5 vector instructions - fma, max, half a conversion - for 9
+  // when each was rounded by integer arithmetic and converted the bias again: these were 640 of the 1150
+  // instructions of a wave of a 128 x 128 tile with one or two offsets.  bf16 passes forward and backward: 128
+  // channels at 1 M voxels 766.6 -> 762.9 us, stride 2, 128 -> 256 at 300 k 825.7 -> 822.2.
   auto store_rows = [&](auto act_c, auto mode_c) {
     constexpr int ACT = decltype(act_c)::value;
     constexpr int MODE = decltype(mode_c)::value;
     constexpr bool SRC = (MODE & 1) != 0;
     if constexpr (E::kBytes == 2) {
       constexpr int NG = CPLW / 8;   // 16-byte groups
+      float shared[MODE == 4 ? CPLW : 1];
+      if constexpr (MODE == 4) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+          const v4i row = __builtin_bit_cast(v4i, src_pre[0][g]);
+          const uint16_t *sh = reinterpret_cast<const uint16_t *>(&row);
+#pragma unroll
+          for (int x = 0; x < 8; ++x) shared[g * 8 + x] = p.beta * E::to_float(sh[x]);
+        }
+      }
 #pragma unroll
       for (int rb = 0; rb < RBW; ++rb) {
         if (!mine(rb)) continue;
@@ -735,15 +752,15 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
           v4i src = {0, 0, 0, 0};
           if constexpr (SRC) src = __builtin_bit_cast(v4i, src_pre[rb][g]);
           const uint16_t *sh = reinterpret_cast<const uint16_t *>(&src);
-          v4i outv;
-          uint16_t *oh = reinterpret_cast<uint16_t *>(&outv);
+          float t[8];
 #pragma unroll
           for (int x = 0; x < 8; ++x) {
             const float a = acc[rb][g * 2 + (x >> 2)][x & 3];
-            float t = SRC ? __builtin_fmaf(p.alpha, a, p.beta * E::to_float(sh[x])) : p.alpha * a;
-            t = apply_act(t, ACT, p.act_alpha);
-            oh[x] = E::from_float(t);
+            if constexpr (MODE == 4) t[x] = __builtin_fmaf(p.alpha, a, shared[g * 8 + x]);
+            else t[x] = SRC ? __builtin_fmaf(p.alpha, a, p.beta * E::to_float(sh[x])) : p.alpha * a;
+            t[x] = apply_act(t[x], ACT, p.act_alpha);
           }
+          const v4i outv = round8<T, ACT == 1>(t);      // (a ReLU lets no NaN through)
           store_out_b128(outv, rs_c, coff, p.stream_stores != 0);
         }
       }
@@ -786,10 +803,11 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
     }
   };
   auto with_mode = [&](auto act_c) {
-    const int mode = (p.read_source ? 1 : 0) | (E::kBytes == 1 && p.int8_epilogue ? 2 : 0);
+    const int mode = p.read_source && shared_src ? 4 : (p.read_source ? 1 : 0) | (E::kBytes == 1 && p.int8_epilogue ? 2 : 0);
     switch (mode) {
     case 0: store_rows(act_c, std::integral_constant<int, 0>{}); break;
     case 1: store_rows(act_c, std::integral_constant<int, 1>{}); break;
+    case 4: if constexpr (E::kBytes == 2) store_rows(act_c, std::integral_constant<int, 4>{}); break;
     case 2: if constexpr (E::kBytes == 1) store_rows(act_c, std::integral_constant<int, 2>{}); break;
     default: if constexpr (E::kBytes == 1) store_rows(act_c, std::integral_constant<int, 3>{}); break;
     }

@@ -172,15 +172,14 @@ __global__ __launch_bounds__(256) void rowgemm_wave_kernel(const RowGemmParams p
           const int ch = ch0 + g * 8;
           const bool ok = row_ok && ch < p.k_out;
           const uint16_t *sh = reinterpret_cast<const uint16_t *>(&src[u][g]);
-          v4i outv;
-          uint16_t *oh = reinterpret_cast<uint16_t *>(&outv);
+          float t[8];
 #pragma unroll
           for (int x = 0; x < 8; ++x) {
             const float a = acc[g * 2 + (x >> 2)][x & 3];
-            float t = p.read_source ? __builtin_fmaf(p.alpha, a, p.beta * E::to_float(sh[x])) : p.alpha * a;
-            t = apply_act(t, p.act, p.act_alpha);
-            oh[x] = E::from_float(t);
+            t[x] = p.read_source ? __builtin_fmaf(p.alpha, a, p.beta * E::to_float(sh[x])) : p.alpha * a;
+            t[x] = apply_act(t[x], p.act, p.act_alpha);
           }
+          const v4i outv = round8<T, false>(t);
           __builtin_amdgcn_raw_buffer_store_b128(outv, rs_c, ok ? (uint32_t)((int64_t)o * p.ldc + ch) * 2u : kOob, 0, 0);
         }
       }

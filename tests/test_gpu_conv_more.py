@@ -7,8 +7,9 @@ import pytest
 
 import helpers as H
 from cumm_amd import _capi, pairs, synth
+from cumm_amd import tensorview as tv
 from cumm_amd.conv.main import ConvMainUnitTest
-from cumm_amd.tensorview.gemm import ConvOpType, ConvParams
+from cumm_amd.tensorview.gemm import Activation, ConvOpType, ConvParams
 
 pytestmark = pytest.mark.gpu
 
@@ -55,3 +56,49 @@ def test_write_empty(channels, tile, hint):
     assert (got[np.asarray(pt.mask_bwd) == 0] == 0.0).all()
     live = np.asarray(pt.mask_bwd) != 0
     np.testing.assert_array_equal(got[live], base[live])
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("tile", [(64, 64), (128, 128)])
+@pytest.mark.parametrize("act", [Activation.None_, Activation.ReLU])
+@pytest.mark.parametrize("with_bias", [False, True])
+def test_special_values_through_the_epilogue(dtype, tile, act, with_bias):
+    """Results that are NaN, infinite, overflow in the rounding or are a negative zero: the identity as weight of the
+    one kernel offset, so that a result is a feature times alpha plus the bias, rounded once."""
+    print("case special values", dtype, tile, act, with_bias, flush=True)
+    rng, n, c = np.random.default_rng(3), 300, 128 if tile[1] == 128 else 64
+    x = rng.normal(0, 1, size=(n, c)).astype(np.float32)
+    for i, v in enumerate((np.nan, np.inf, -np.inf, 0.0, -0.0, 65000.0, -65000.0, 3.3e38, -3.3e38)):
+        x[i * 7 % n, i::9] = v if dtype == "bf16" or abs(v) < 65504 or not np.isfinite(v) else 1.0
+    feat, bias = H.to_storage(x, dtype), H.to_storage(rng.normal(0, 1, size=c).astype(np.float32), dtype)
+    p = ConvParams(3, ConvOpType.Forward)
+    p.conv_algo_desp = H.find_conv_desp(dtype, ConvOpType.Forward, *tile)
+    w = np.zeros((c, 1, c), np.float32)
+    p.input, p.output = H.dev(feat, dtype), tv.zeros([n, c], H.TV_DTYPE[dtype], 0)
+    w[np.arange(c), 0, np.arange(c)] = 1.0
+    clean = np.nan_to_num(H.as_f32(feat, dtype), nan=0.0, posinf=0.0, neginf=0.0)
+    p.weight = H.dev(H.to_storage(w, dtype), dtype)
+    rows = np.arange(n, dtype=np.int32)
+    p.indices, p.mask, p.mask_argsort = H.dev(rows[None], "i32"), H.dev(np.ones(n, np.uint32), "u32"), H.dev(rows, "i32")
+    p.alpha, p.act_type = -1.5, act
+    if with_bias:
+        p.bias, p.beta = H.dev(bias, dtype), 1.0
+    ConvMainUnitTest.implicit_gemm2(p)
+    # (0 * inf and 0 * NaN of the other columns make all of such a row NaN before the epilogue)
+    whole = np.isfinite(H.as_f32(feat, dtype)).all(axis=1, keepdims=True)
+    acc = np.where(whole, clean, np.float32(np.nan))
+    with np.errstate(over="ignore", invalid="ignore"):
+        want = (acc.astype(np.float64) * -1.5 + (H.as_f32(bias, dtype) if with_bias else 0)).astype(np.float32)      # (the fused form)
+        if act == Activation.ReLU:
+            want = np.where(want > 0, want, np.float32(0))
+        want = H.to_storage(want, dtype)
+    got = H.host(p.output)
+    a, b = got.view(np.uint16), want.view(np.uint16)
+    nan = np.isnan(H.as_f32(want, dtype))
+    np.testing.assert_array_equal(np.isnan(H.as_f32(got, dtype)), nan)
+    assert nan.any() == (act == Activation.None_)
+    if dtype == "bf16":
+        assert (a[nan] == 0x7FFF).all()
+    np.testing.assert_array_equal(a[~nan] & 0x7FFF, b[~nan] & 0x7FFF)
+    keep = ~nan & ((a & 0x7FFF) != 0) if act == Activation.None_ else ~nan      # (the sign of a zero sum is the matrix unit's)
+    np.testing.assert_array_equal(a[keep], b[keep])
