@@ -60,8 +60,13 @@ class SparseConvArgs(C.Structure):
                 ("ungated_rows", C.c_int32), ("indices_by_position", C.c_int32), ("mask_int_count", C.c_int32)]
 
 
+class GateSums(C.Structure):
+    _fields_ = [("gated", C.c_void_p), ("sums", C.c_void_p), ("grad", C.c_void_p), ("out", C.c_void_p), ("rows", C.c_int64),
+                ("channels", C.c_int32), ("workspace", C.c_void_p), ("workspace_bytes", C.c_size_t)]
+
+
 class SparseConvMore(C.Structure):
-    _fields_ = [("write_empty", C.c_int32)]
+    _fields_ = [("write_empty", C.c_int32), ("sums", C.c_void_p)]
 
 
 class OrderSide(C.Structure):
@@ -136,6 +141,8 @@ SYMBOLS = {
     "cumm_hip_wgrad_pairs_workspace": (C.c_int64, [_VP, C.c_int, C.c_int, C.c_int]),
     "cumm_hip_wgrad_pairs": (C.c_int, [_VP, _VP, _VP, _VP, _VP, _VP, C.c_int, C.c_int64, C.c_int, C.c_int, C.c_int, C.c_int,
                                        C.c_int, _VP, C.c_size_t, _VP]),
+    "cumm_hip_wgrad_pairs_sums": (C.c_int, [_VP, _VP, _VP, _VP, _VP, _VP, C.c_int, C.c_int64, C.c_int, C.c_int, C.c_int, C.c_int,
+                                       C.c_int, _VP, _VP, C.c_size_t, _VP]),
     "cumm_hip_finish_rows": (C.c_int, [_VP, C.c_int, _VP, _VP, C.c_int64, C.c_int, C.c_float, C.c_float, C.c_int,
                                        C.c_float, _VP]),
     "cumm_hip_relu_backward": (C.c_int, [_VP, _VP, _VP, C.c_size_t, C.c_int, _VP]),

@@ -325,6 +325,24 @@ int report_async_errors() {
 int sparse_conv_impl(const CummHipConvDesc *desc, const CummHipSparseConvArgs *a, const CummHipSparseConvMore *more, void *stream_, void *workspace,
                      size_t workspace_bytes, size_t workspace_cap);
 
+// checked arguments of the gate and the sums of a gradient
+int gate_sums_params(const CummHipGateSums &g, int dtype, ColumnSumParams *p) {
+  if (g.rows < 0 || g.channels < 0) return fail(CUMM_HIP_EINVAL, "bad arguments");
+  if (!is_float16_like(dtype)) return fail(CUMM_HIP_EINVAL, "dtype must be f16 or bf16");
+  if (g.channels % 8 || g.channels > 2048) return fail(CUMM_HIP_EINVAL, "channels must be a multiple of 8, at most 2048");
+  std::memset(p, 0, sizeof(*p));
+  if (g.channels == 0) return CUMM_HIP_OK;
+  if (!g.sums || (!g.grad && g.rows > 0) || !aligned16(g.grad)) return fail(CUMM_HIP_EINVAL, "dst and src (16-byte aligned) must not be empty");
+  if ((g.gated != nullptr) != (g.out != nullptr) || !aligned16(g.gated) || !aligned16(g.out))
+    return fail(CUMM_HIP_EINVAL, "gated, grad and out must be 16-byte aligned and not empty");
+  const size_t need = sizeof(float) * (size_t)column_sum_blocks(g.rows, g.channels) * (size_t)g.channels;
+  if (!g.workspace || g.workspace_bytes < need) return fail(CUMM_HIP_ERUNTIME, "workspace at least %zu bytes.", need);
+  if (reinterpret_cast<uintptr_t>(g.workspace) & 3u) return fail(CUMM_HIP_EINVAL, "workspace must be 4-byte aligned");
+  p->dst = g.sums; p->src = g.grad; p->out = g.out; p->gated = g.gated;
+  p->partial = reinterpret_cast<float *>(g.workspace); p->rows = g.rows; p->channels = g.channels;
+  return CUMM_HIP_OK;
+}
+
 // workspace of the fixed-order backward-weight: live-tile counts (128 bytes), the table of the
 // workgroups per (offset, channel block), the live-tile lists, then the slots of partial sums
 struct OrderedLayout {
@@ -395,15 +413,15 @@ WgradPairsPlan wgrad_pairs_plan(const int32_t *counts, int lists, int K, int C, 
 }
 
 hipError_t run_wgrad_pairs(WgradPairsParams *w, WgradPairsFinalizeParams *f, const WgradPairsPlan &l, int lists, int K, int C, int dt,
-                           bool wide, void *workspace, hipStream_t stream) {
+                           bool wide, void *workspace, const ColumnSumParams *sums, hipStream_t stream) {
   w->slots = reinterpret_cast<float *>(workspace);
   w->K = f->K = K; w->C = f->C = C; w->lists = f->lists = lists;
   w->kblocks = f->kblocks = l.kblocks; w->cblocks = f->cblocks = l.cblocks;
   w->wgs = l.wgs; w->per_wg = f->per_wg = l.per_wg;
   f->slots = w->slots;
   std::memcpy(f->step0, w->step0, sizeof(int32_t) * (lists + 1));
-  return dt == CUMM_HIP_F16 ? launch_wgrad_pairs_f16(*w, *f, wide, l.most_slots, stream)
-                            : launch_wgrad_pairs_bf16(*w, *f, wide, l.most_slots, stream);
+  return dt == CUMM_HIP_F16 ? launch_wgrad_pairs_f16(*w, *f, wide, l.most_slots, sums, stream)
+                            : launch_wgrad_pairs_bf16(*w, *f, wide, l.most_slots, sums, stream);
 }
 
 // ShuffleAB products of two-byte operands with one slice whose pairs are many against their output
@@ -698,7 +716,7 @@ static int gemm_impl(const CummHipGemmDesc *desc, const CummHipGemmArgs *a, void
         f.dw = a->ptr_C; f.src = ptr_D; f.ldw = a->stride_C; f.lds = ldd;
         f.alpha = a->alpha; f.beta = a->beta; f.act_alpha = a->act_alpha; f.act = a->act_type;
         w.count[0] = count;
-        const hipError_t e = run_wgrad_pairs(&w, &f, l, 1, m, n, dt, wide, a->workspace, stream);
+        const hipError_t e = run_wgrad_pairs(&w, &f, l, 1, m, n, dt, wide, a->workspace, nullptr, stream);
         if (e == hipSuccess) return CUMM_HIP_OK;
         if (e != hipErrorNotSupported) return hip_fail(e, "pair-list weight gradient launch");
       }
@@ -786,7 +804,16 @@ int sparse_conv_impl(const CummHipConvDesc *desc, const CummHipSparseConvArgs *a
   if (a->C % pv || a->K % pv) return fail(CUMM_HIP_ERUNTIME, "C and K must be multiples of %d for this element type", pv);
   if (!d.split_k_serial && !d.split_k_parallel && a->split_k_slices > 1)
     return fail(CUMM_HIP_ERUNTIME, "algo don't support splitk but you provide split_k_slices > 1.");
-  if (a->N == 0) return CUMM_HIP_OK;
+  ColumnSumParams sums_params;
+  const ColumnSumParams *sums = nullptr;
+  if (more != nullptr && more->sums != nullptr) {
+    if (c.op_type != CUMM_HIP_OP_BACKWARD_WEIGHT || fam == 1) return fail(CUMM_HIP_EINVAL, "only backward-weight makes the gate and sums of a gradient");
+    if (more->sums->channels != a->K || more->sums->rows != a->rows_out || (more->sums->gated ? more->sums->gated : more->sums->grad) != a->ptr_A)
+      return fail(CUMM_HIP_EINVAL, "gate and sums are those of the gradient of this call");
+    if (int rc = gate_sums_params(*more->sums, dt, &sums_params)) return rc;
+    sums = &sums_params;
+  }
+  if (a->N == 0 && sums == nullptr) return CUMM_HIP_OK;
   const void *ptr_D = a->ptr_D ? a->ptr_D : a->ptr_C;
 
   if (fam == 1) {
@@ -857,6 +884,10 @@ int sparse_conv_impl(const CummHipConvDesc *desc, const CummHipSparseConvArgs *a
 
   // backward weight: dW[K, kv, C]; A = dOut [N, K], B = input [*, C]
   const int tm = d.tile_shape[0], tn = d.tile_shape[1], tk = d.tile_shape[2];
+  if (a->N == 0) {
+    HIP_TRY(launch_column_sum(*sums, dt == CUMM_HIP_BF16, stream));
+    return CUMM_HIP_OK;
+  }
   if (a->mask_width <= 0 || a->mask_width % tk) return fail(CUMM_HIP_ERUNTIME, "mask_width must be a positive multiple of tile k");
   if (fam == 3 && a->deterministic && !(a->split_k_slices > 1 && a->mask_width <= kWgradMaxPos))
     return fail(CUMM_HIP_EINVAL, "the fixed-order backward-weight needs split_k_slices > 1 and mask_width <= %d", kWgradMaxPos);
@@ -920,8 +951,8 @@ int sparse_conv_impl(const CummHipConvDesc *desc, const CummHipSparseConvArgs *a
     f.cblocks = lay.cblocks; f.per_r = lay.combos;
     f.mask_filter = a->mask_filter; f.alpha = a->alpha; f.beta = a->beta;
     f.slots_bytes = (uint32_t)((wgs + lay.keys - 1) * (int64_t)lay.block_bytes);
-    hipError_t e = dt == CUMM_HIP_F16 ? launch_wgrad_ordered_f16(w, pre, f, lay.wide, (int)wgs, stream)
-                                      : launch_wgrad_ordered_bf16(w, pre, f, lay.wide, (int)wgs, stream);
+    hipError_t e = dt == CUMM_HIP_F16 ? launch_wgrad_ordered_f16(w, pre, f, lay.wide, (int)wgs, sums, stream)
+                                      : launch_wgrad_ordered_bf16(w, pre, f, lay.wide, (int)wgs, sums, stream);
     if (e == hipErrorNotSupported)
       return fail(CUMM_HIP_ERUNTIME, "the fixed-order backward-weight kernel of this build uses scratch memory, which its "
                   "hand-counted waits do not allow; use a split_k_serial descriptor");
@@ -985,14 +1016,14 @@ int sparse_conv_impl(const CummHipConvDesc *desc, const CummHipSparseConvArgs *a
     } else {
       HIP_TRY(zero_device(workspace, need, stream));
     }
-    hipError_t e = dt == CUMM_HIP_F16 ? launch_wgrad_atomic_f16(w, pre, f, stream) : launch_wgrad_atomic_bf16(w, pre, f, stream);
+    hipError_t e = dt == CUMM_HIP_F16 ? launch_wgrad_atomic_f16(w, pre, f, sums, stream) : launch_wgrad_atomic_bf16(w, pre, f, sums, stream);
     if (e == hipErrorNotSupported && w.live_list != nullptr) {
       // the unit-walking kernel failed its load-time check (see counted_waits_hold): the scanning
       // kernel on one image, zeroed here
       w.live_cnt = nullptr; w.live_list = nullptr;
       w.images = f.images = 1;
       HIP_TRY(zero_device(workspace, need, stream));
-      e = dt == CUMM_HIP_F16 ? launch_wgrad_atomic_f16(w, pre, f, stream) : launch_wgrad_atomic_bf16(w, pre, f, stream);
+      e = dt == CUMM_HIP_F16 ? launch_wgrad_atomic_f16(w, pre, f, sums, stream) : launch_wgrad_atomic_bf16(w, pre, f, sums, stream);
     }
     if (e != hipSuccess) return hip_fail(e, "sparse conv wgrad launch");
     g_wgrad_path = w.live_list != nullptr ? CUMM_HIP_WGRAD_LISTS : CUMM_HIP_WGRAD_SCAN;
@@ -1030,6 +1061,7 @@ int sparse_conv_impl(const CummHipConvDesc *desc, const CummHipSparseConvArgs *a
     p.sem = reinterpret_cast<int32_t *>(workspace);
     if (int rc = async_status_ptr(&p.timeouts)) return rc;
   }
+  if (sums != nullptr) HIP_TRY(launch_column_sum(*sums, dt == CUMM_HIP_BF16, stream));
   hipError_t e = launch_tilegemm(dt, false, tm, tn, false, false, p, grid, stream);
   if (e != hipSuccess) return hip_fail(e, "sparse conv wgrad launch");
   g_wgrad_path = CUMM_HIP_WGRAD_TILED;
@@ -1573,6 +1605,13 @@ int64_t cumm_hip_wgrad_pairs_workspace(const int32_t *counts, int lists, int K, 
 int cumm_hip_wgrad_pairs(void *dw, const void *dout, const void *inp, const int32_t *pair_out, const int32_t *pair_in,
                          const int32_t *counts, int lists, int64_t list_stride, int rows_out, int rows_in, int K, int C,
                          int dtype, void *workspace, size_t workspace_bytes, void *stream) {
+  return cumm_hip_wgrad_pairs_sums(dw, dout, inp, pair_out, pair_in, counts, lists, list_stride, rows_out, rows_in, K, C, dtype, nullptr,
+                                   workspace, workspace_bytes, stream);
+}
+
+int cumm_hip_wgrad_pairs_sums(void *dw, const void *dout, const void *inp, const int32_t *pair_out, const int32_t *pair_in,
+                              const int32_t *counts, int lists, int64_t list_stride, int rows_out, int rows_in, int K, int C,
+                              int dtype, const CummHipGateSums *gate_sums, void *workspace, size_t workspace_bytes, void *stream) {
   if (!is_float16_like(dtype)) return fail(CUMM_HIP_EINVAL, "dtype must be f16 or bf16");
   if (!wgrad_pairs_args(counts, lists, K, C) || rows_out < 0 || rows_in < 0)
     return fail(CUMM_HIP_EINVAL, "1 to %d pair lists with counts on the host, channels multiples of 8", kWgradPairsMaxLists);
@@ -1594,11 +1633,18 @@ int cumm_hip_wgrad_pairs(void *dw, const void *dout, const void *inp, const int3
     if (!workspace || workspace_bytes < l.bytes) return fail(CUMM_HIP_ERUNTIME, "workspace at least %zu bytes.", l.bytes);
     if (!aligned16(workspace)) return fail(CUMM_HIP_EINVAL, "workspace must be 16-byte aligned");
   }
+  ColumnSumParams sums;
+  if (gate_sums != nullptr) {
+    if (gate_sums->channels != K || gate_sums->rows != rows_out || (gate_sums->gated ? gate_sums->gated : gate_sums->grad) != dout)
+      return fail(CUMM_HIP_EINVAL, "gate and sums are those of the gradient of this call");
+    if (int rc = gate_sums_params(*gate_sums, dtype, &sums)) return rc;
+  }
   w.dout = dout; w.inp = inp; w.pair_out = pair_out; w.pair_in = pair_in;
   w.ldy = K; w.ldx = C; w.list_stride = list_stride; w.rows_y = rows_out; w.rows_x = rows_in;
   std::memcpy(w.count, counts, sizeof(int32_t) * lists);
   f.dw = dw; f.src = dw; f.ldw = f.lds = (int64_t)lists * C; f.ldr = C; f.alpha = 1.0f;
-  const hipError_t e = run_wgrad_pairs(&w, &f, l, lists, K, C, dtype, false, workspace, reinterpret_cast<hipStream_t>(stream));
+  const hipError_t e = run_wgrad_pairs(&w, &f, l, lists, K, C, dtype, false, workspace, gate_sums ? &sums : nullptr,
+                                       reinterpret_cast<hipStream_t>(stream));
   if (e == hipErrorNotSupported)
     return fail(CUMM_HIP_ERUNTIME, "the pair-list kernel of this build uses scratch memory, which its hand-counted waits do not allow");
   if (e != hipSuccess) return hip_fail(e, "pair-list weight gradient launch");
@@ -1741,20 +1787,10 @@ size_t cumm_hip_column_sum_workspace(int64_t rows, int channels) {
   return sizeof(float) * (size_t)column_sum_blocks(rows, channels) * (size_t)channels;
 }
 
-static int column_sum_checked(void *dst, const void *src, const void *out, void *gated, int64_t rows, int channels, int dtype,
-                              void *workspace, size_t workspace_bytes, void *stream) {
-  if (rows < 0 || channels < 0) return fail(CUMM_HIP_EINVAL, "bad arguments");
-  if (!is_float16_like(dtype)) return fail(CUMM_HIP_EINVAL, "dtype must be f16 or bf16");
-  if (channels % 8 || channels > 2048) return fail(CUMM_HIP_EINVAL, "channels must be a multiple of 8, at most 2048");
-  if (channels == 0) return CUMM_HIP_OK;
-  if (!dst || (!src && rows > 0) || !aligned16(src)) return fail(CUMM_HIP_EINVAL, "dst and src (16-byte aligned) must not be empty");
-  const size_t need = sizeof(float) * (size_t)column_sum_blocks(rows, channels) * (size_t)channels;
-  if (!workspace || workspace_bytes < need) return fail(CUMM_HIP_ERUNTIME, "workspace at least %zu bytes.", need);
-  if (reinterpret_cast<uintptr_t>(workspace) & 3u) return fail(CUMM_HIP_EINVAL, "workspace must be 4-byte aligned");
+static int column_sum_checked(const CummHipGateSums &g, int dtype, void *stream) {
   ColumnSumParams p;
-  std::memset(&p, 0, sizeof(p));
-  p.dst = dst; p.src = src; p.out = out; p.gated = gated;
-  p.partial = reinterpret_cast<float *>(workspace); p.rows = rows; p.channels = channels;
+  if (int rc = gate_sums_params(g, dtype, &p)) return rc;
+  if (g.channels == 0) return CUMM_HIP_OK;
   hipError_t e = launch_column_sum(p, dtype == CUMM_HIP_BF16, reinterpret_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "column_sum launch");
   return CUMM_HIP_OK;
@@ -1762,14 +1798,15 @@ static int column_sum_checked(void *dst, const void *src, const void *out, void 
 
 int cumm_hip_column_sum(void *dst, const void *src, int64_t rows, int channels, int dtype, void *workspace,
                         size_t workspace_bytes, void *stream) {
-  return column_sum_checked(dst, src, nullptr, nullptr, rows, channels, dtype, workspace, workspace_bytes, stream);
+  return column_sum_checked({nullptr, dst, src, nullptr, rows, channels, workspace, workspace_bytes}, dtype, stream);
 }
 
 int cumm_hip_relu_backward_sums(void *gated, void *sums, const void *grad, const void *out, int64_t rows, int channels, int dtype,
                                 void *workspace, size_t workspace_bytes, void *stream) {
   if (rows > 0 && channels > 0 && (!gated || !out || !aligned16(gated) || !aligned16(out)))
     return fail(CUMM_HIP_EINVAL, "gated, grad and out must be 16-byte aligned and not empty");
-  return column_sum_checked(sums, grad, out, gated, rows, channels, dtype, workspace, workspace_bytes, stream);
+  const bool gate = rows > 0;      // (no rows, nothing to gate: the tensors may have no memory)
+  return column_sum_checked({gate ? gated : nullptr, sums, grad, gate ? out : nullptr, rows, channels, workspace, workspace_bytes}, dtype, stream);
 }
 
 int cumm_hip_copy_kernel(void *dst, const void *src, size_t bytes, void *stream) {

@@ -93,17 +93,23 @@ __global__ __launch_bounds__(256) void relu_backward_kernel(v4i *dst, const v4i 
 // partial[b][c] = sum of src[r][c] over the rows of block b - with GATE of the gated rows, which are
 // written to gated on the way.  Thread t takes the 8-channel piece t % V of the rows t / V, t / V + R,
 // ... of its block (V pieces per row, R = 256 / V rows at a time); the R row lanes of a piece are then
-// summed through LDS in lane order.
+// summed through LDS in lane order.  The first pre_blocks workgroups prepare a weight gradient instead
+// (wgrad_prepare: lists and zeros that depend on nothing here; in a launch of its own it is 4 us).
 template <class T, bool GATE, bool NT>
-__global__ __launch_bounds__(256) void column_partial_kernel(const ColumnSumParams p) {
+__global__ __launch_bounds__(256) void column_partial_kernel(const ColumnSumParams p, const WgradPrepareParams pre, int pre_blocks) {
   __shared__ float lds[256][9];
+  if ((int)blockIdx.x < pre_blocks) {
+    wgrad_prepare(pre, blockIdx.x, pre_blocks);
+    return;
+  }
+  const int64_t block = blockIdx.x - pre_blocks;
   const int V = p.channels / 8;
   const int R = 256 / V;
   const int t = threadIdx.x;
   const int piece = t % V, lane_row = t / V;
   float s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   if (lane_row < R) {
-    const int64_t r0 = (int64_t)blockIdx.x * p.rows_per_block;
+    const int64_t r0 = block * p.rows_per_block;
     int64_t r1 = r0 + p.rows_per_block;
     if (r1 > p.rows) r1 = p.rows;
     const v4i *src = reinterpret_cast<const v4i *>(p.src) + piece;
@@ -138,48 +144,23 @@ __global__ __launch_bounds__(256) void column_partial_kernel(const ColumnSumPara
     for (int j = 1; j < R; ++j)
 #pragma unroll
       for (int x = 0; x < 8; ++x) s[x] += lds[j * V + piece][x];
-    float *dst = p.partial + (int64_t)blockIdx.x * p.channels + piece * 8;
+    float *dst = p.partial + block * p.channels + piece * 8;
 #pragma unroll
     for (int x = 0; x < 8; ++x) dst[x] = s[x];
   }
 }
 
-// Sum over blocks in a fixed shape: 64 threads per channel, thread j adds the j-th 64th of the blocks in
-// block order (eight loads in flight at a time), then sixteen sums each are added in order, then
-// those four.  The blocks of slice blockIdx.y of gridDim.y; the last stage (one slice) converts.
+// The blocks of slice blockIdx.y of gridDim.y; the last stage (one slice) converts.
 template <class T, bool LAST>
-__global__ __launch_bounds__(1024) void column_final_kernel(const ColumnSumParams p, const float *from, int blocks, float *to) {
-  __shared__ float part[64][17];
-  const int cl = threadIdx.x & 15, j = threadIdx.x >> 4;
-  const int c = blockIdx.x * 16 + cl;
-  const int slice = (blocks + gridDim.y - 1) / gridDim.y;
-  const int first = (int)blockIdx.y * slice, end = first + slice < blocks ? first + slice : blocks;
-  const int share = (end - first + 63) >> 6;
-  const int b0 = first + j * share, b1 = b0 + share < end ? b0 + share : end;
-  float s = 0.0f;
-  if (c < p.channels) {
-    for (int b = b0; b < b1; b += 8) {
-      float v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = b + u < b1 ? from[(int64_t)(b + u) * p.channels + c] : 0.0f;
-#pragma unroll
-      for (int u = 0; u < 8; ++u) s += v[u];
-    }
-  }
-  part[j][cl] = s;
-  __syncthreads();
-  if (j < 4) {
-    s = part[j * 16][cl];
-#pragma unroll
-    for (int k = 1; k < 16; ++k) s += part[j * 16 + k][cl];
-  }
-  __syncthreads();
-  if (j < 4) part[j][cl] = s;
-  __syncthreads();
-  if (j == 0 && c < p.channels) {
-    const float total = ((part[0][cl] + part[1][cl]) + part[2][cl]) + part[3][cl];
-    if constexpr (LAST) reinterpret_cast<uint16_t *>(p.dst)[c] = Elem<T>::from_float(total);
-    else to[(int64_t)blockIdx.y * p.channels + c] = total;
+__global__ __launch_bounds__(256) void column_final_kernel(const ColumnFinalParams p, float *to) {
+  if constexpr (LAST) {
+    column_final<T>(p, blockIdx.x);
+  } else {
+    const int slice = (p.blocks + gridDim.y - 1) / gridDim.y;
+    const int first = (int)blockIdx.y * slice, end = first + slice < p.blocks ? first + slice : p.blocks;
+    const float total = column_final_sum(p.from, p.channels, first, end, blockIdx.x);
+    const int c = blockIdx.x * 16 + threadIdx.x;
+    if (threadIdx.x < 16 && c < p.channels) to[(int64_t)blockIdx.y * p.channels + c] = total;
   }
 }
 
@@ -245,32 +226,44 @@ int column_sum_blocks(int64_t rows, int channels) {
 }
 
 template <class T>
-static hipError_t column_sum(const ColumnSumParams &p, hipStream_t s) {
+static void column_partial(const ColumnSumParams &p, const WgradPrepareParams &pre, int pre_blocks, hipStream_t s) {
   const bool stream = (size_t)p.rows * (size_t)p.channels * 2 > kStreamBytes;
+  const dim3 grid((unsigned)(p.blocks + pre_blocks));
   if (p.gated != nullptr) {
-    if (stream) hipLaunchKernelGGL((column_partial_kernel<T, true, true>), dim3(p.blocks), dim3(256), 0, s, p);
-    else hipLaunchKernelGGL((column_partial_kernel<T, true, false>), dim3(p.blocks), dim3(256), 0, s, p);
+    if (stream) hipLaunchKernelGGL((column_partial_kernel<T, true, true>), grid, dim3(256), 0, s, p, pre, pre_blocks);
+    else hipLaunchKernelGGL((column_partial_kernel<T, true, false>), grid, dim3(256), 0, s, p, pre, pre_blocks);
   } else {
-    if (stream) hipLaunchKernelGGL((column_partial_kernel<T, false, true>), dim3(p.blocks), dim3(256), 0, s, p);
-    else hipLaunchKernelGGL((column_partial_kernel<T, false, false>), dim3(p.blocks), dim3(256), 0, s, p);
+    if (stream) hipLaunchKernelGGL((column_partial_kernel<T, false, true>), grid, dim3(256), 0, s, p, pre, pre_blocks);
+    else hipLaunchKernelGGL((column_partial_kernel<T, false, false>), grid, dim3(256), 0, s, p, pre, pre_blocks);
   }
-  const unsigned groups = (unsigned)((p.channels + 15) / 16);
-  const float *from = p.partial;
-  int blocks = p.blocks;
-  if (blocks > kFewBlocks) {
-    float *to = p.partial + (int64_t)blocks * p.channels;
-    hipLaunchKernelGGL((column_final_kernel<T, false>), dim3(groups, kSlices), dim3(1024), 0, s, p, from, blocks, to);
-    from = to;
-    blocks = kSlices;
-  }
-  hipLaunchKernelGGL((column_final_kernel<T, true>), dim3(groups), dim3(1024), 0, s, p, from, blocks, nullptr);
-  return hipGetLastError();
 }
 
-hipError_t launch_column_sum(ColumnSumParams p, bool bf16, hipStream_t s) {
+hipError_t launch_column_partial(ColumnSumParams p, const WgradPrepareParams *pre, int pre_blocks, bool bf16, hipStream_t s,
+                                 ColumnFinalParams *last) {
   p.blocks = column_blocks(p.rows, p.channels);
   p.rows_per_block = column_rows_per_block(p.rows, p.channels);
-  return bf16 ? column_sum<BF16>(p, s) : column_sum<F16>(p, s);
+  const WgradPrepareParams none = {};
+  if (bf16) column_partial<BF16>(p, pre ? *pre : none, pre ? pre_blocks : 0, s);
+  else column_partial<F16>(p, pre ? *pre : none, pre ? pre_blocks : 0, s);
+  hipError_t e = hipGetLastError();
+  *last = ColumnFinalParams{p.partial, p.dst, p.blocks, p.channels, (p.channels + 15) / 16};
+  if (e == hipSuccess && p.blocks > kFewBlocks) {
+    float *to = p.partial + (int64_t)p.blocks * p.channels;
+    hipLaunchKernelGGL((column_final_kernel<F16, false>), dim3((unsigned)last->groups, kSlices), dim3(256), 0, s, *last, to);
+    e = hipGetLastError();
+    last->from = to;
+    last->blocks = kSlices;
+  }
+  return e;
+}
+
+hipError_t launch_column_sum(const ColumnSumParams &p, bool bf16, hipStream_t s) {
+  ColumnFinalParams last;
+  const hipError_t e = launch_column_partial(p, nullptr, 0, bf16, s, &last);
+  if (e != hipSuccess) return e;
+  if (bf16) hipLaunchKernelGGL((column_final_kernel<BF16, true>), dim3((unsigned)last.groups), dim3(256), 0, s, last, nullptr);
+  else hipLaunchKernelGGL((column_final_kernel<F16, true>), dim3((unsigned)last.groups), dim3(256), 0, s, last, nullptr);
+  return hipGetLastError();
 }
 
 }  // namespace cummhip

@@ -52,18 +52,25 @@ hipError_t launch_tilegemm_wide_bf16(int tm, int tn, bool xk, bool yk, const Til
 hipError_t launch_tilegemm_wide_s8(int tm, int tn, bool xk, bool yk, const TileGemmParams &p, dim3 grid,
                                    hipStream_t s);
 
-// balanced backward-weight with fp32 atomics: main kernel then finalize (f16 / bf16 only)
-hipError_t launch_wgrad_atomic_f16(const WgradParams &p, const WgradPrepareParams &pre, const WgradFinalizeParams &f, hipStream_t s);
-hipError_t launch_wgrad_atomic_bf16(const WgradParams &p, const WgradPrepareParams &pre, const WgradFinalizeParams &f, hipStream_t s);
+struct ColumnSumParams;      // below
+
+// balanced backward-weight with fp32 atomics: main kernel then finalize (f16 / bf16 only).  sums (may be NULL): bias
+// sums, and the gate that makes p.dout, in the launches before and after the products
+hipError_t launch_wgrad_atomic_f16(const WgradParams &p, const WgradPrepareParams &pre, const WgradFinalizeParams &f, const ColumnSumParams *sums,
+                                    hipStream_t s);
+hipError_t launch_wgrad_atomic_bf16(const WgradParams &p, const WgradPrepareParams &pre, const WgradFinalizeParams &f, const ColumnSumParams *sums,
+                                    hipStream_t s);
 int wgrad_ordered_resident_f16(bool wide);
 int wgrad_ordered_resident_bf16(bool wide);
-hipError_t launch_wgrad_ordered_f16(const WgradParams &p, const WgradPrepareParams &pre, const WgradOrderedParams &f, bool wide, int wgs, hipStream_t s);
-hipError_t launch_wgrad_ordered_bf16(const WgradParams &p, const WgradPrepareParams &pre, const WgradOrderedParams &f, bool wide, int wgs, hipStream_t s);
+hipError_t launch_wgrad_ordered_f16(const WgradParams &p, const WgradPrepareParams &pre, const WgradOrderedParams &f, bool wide, int wgs,
+                                     const ColumnSumParams *sums, hipStream_t s);
+hipError_t launch_wgrad_ordered_bf16(const WgradParams &p, const WgradPrepareParams &pre, const WgradOrderedParams &f, bool wide, int wgs,
+                                     const ColumnSumParams *sums, hipStream_t s);
 
 // weight gradients over explicit pair lists (f16 / bf16 operands; wide: f32 result); most_slots = slots
 // of the list with most of them
-hipError_t launch_wgrad_pairs_f16(const WgradPairsParams &p, const WgradPairsFinalizeParams &f, bool wide, int most_slots, hipStream_t s);
-hipError_t launch_wgrad_pairs_bf16(const WgradPairsParams &p, const WgradPairsFinalizeParams &f, bool wide, int most_slots, hipStream_t s);
+hipError_t launch_wgrad_pairs_f16(const WgradPairsParams &p, const WgradPairsFinalizeParams &f, bool wide, int most_slots, const ColumnSumParams *sums, hipStream_t s);
+hipError_t launch_wgrad_pairs_bf16(const WgradPairsParams &p, const WgradPairsFinalizeParams &f, bool wide, int most_slots, const ColumnSumParams *sums, hipStream_t s);
 
 // tile shapes the tables above hold
 inline bool rowgemm_has_tile(int tm, int tn) {
@@ -208,6 +215,10 @@ struct ColumnSumParams {
   int32_t channels, blocks;
 };
 int column_sum_blocks(int64_t rows, int channels);
-hipError_t launch_column_sum(ColumnSumParams p, bool bf16, hipStream_t s);
+// (blocks and rows_per_block are filled in here)
+hipError_t launch_column_sum(const ColumnSumParams &p, bool bf16, hipStream_t s);
+// All but the last step, which *last describes; pre_blocks more workgroups prepare a weight gradient (pre may be NULL)
+hipError_t launch_column_partial(ColumnSumParams p, const WgradPrepareParams *pre, int pre_blocks, bool bf16, hipStream_t s,
+                                 ColumnFinalParams *last);
 
 }  // namespace cummhip

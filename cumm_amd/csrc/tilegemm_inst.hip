@@ -174,8 +174,16 @@ hipError_t CUMM_LAUNCH_NAME(int tm, int tn, bool xk, bool yk, const TileGemmPara
 }
 
 #if !defined(CUMM_NO_WGRAD_ATOMIC) && !CUMM_WIDE
+// The lists and zeros of a weight gradient: in the launch of the bias sums, if there is one (*last: their last step)
+template <class T>
+static hipError_t prepare(const WgradPrepareParams &pre, int blocks, const ColumnSumParams *sums, ColumnFinalParams *last, hipStream_t s) {
+  if (sums != nullptr) return launch_column_partial(*sums, &pre, blocks, std::is_same_v<T, BF16>, s, last);
+  hipLaunchKernelGGL(wgrad_prepare_kernel, dim3((unsigned)blocks), dim3(256), 0, s, pre);
+  return hipGetLastError();
+}
+
 hipError_t CUMM_CAT(launch_wgrad_atomic_, CUMM_NAME)(const WgradParams &p, const WgradPrepareParams &pre,
-                                                     const WgradFinalizeParams &f, hipStream_t s) {
+                                                     const WgradFinalizeParams &f, const ColumnSumParams *sums, hipStream_t s) {
   using T = CUMM_ELEM;
   const int groups = (p.num_red + p.tiles_per_wg - 1) / p.tiles_per_wg;
   // both channel counts above 64: units of 128 x 128 channels (one gather of the full rows)
@@ -184,6 +192,7 @@ hipError_t CUMM_CAT(launch_wgrad_atomic_, CUMM_NAME)(const WgradParams &p, const
   const int kblocks = (p.K + cpu_ - 1) / cpu_, cblocks = (p.C + cpu_ - 1) / cpu_;
   if (groups == 0 || p.kv == 0) return hipSuccess;
   hipError_t e;
+  ColumnFinalParams last = {};
   const bool units_ok = wide ? counted_waits_hold<wgrad_units_kernel<T, 2, 2, 1>>() : counted_waits_hold<wgrad_units_kernel<T, 1, 1, 2>>();
   if (p.live_list != nullptr && !units_ok) return hipErrorNotSupported;
   if (p.live_list != nullptr) {
@@ -202,8 +211,7 @@ hipError_t CUMM_CAT(launch_wgrad_atomic_, CUMM_NAME)(const WgradParams &p, const
       if (e != hipSuccess) return e;
       resident = cus * per_cu > 0 ? cus * per_cu : 1;
     }
-    hipLaunchKernelGGL(wgrad_prepare_kernel, dim3(p.kv + 256), dim3(256), 0, s, pre);
-    e = hipGetLastError();
+    e = prepare<T>(pre, p.kv + kWgradZeroBlocks, sums, &last, s);
     if (e != hipSuccess) return e;
     // With several 64 x 64 channel blocks a unit either takes one of them (more units: small
     // inputs) or walks them all on one set of pair lists (the centre offset alone then gives
@@ -216,12 +224,13 @@ hipError_t CUMM_CAT(launch_wgrad_atomic_, CUMM_NAME)(const WgradParams &p, const
     if (wide) hipLaunchKernelGGL((wgrad_units_kernel<T, 2, 2, 1>), units_grid, dim3(256), 0, s, q);
     else hipLaunchKernelGGL((wgrad_units_kernel<T, 1, 1, 2>), units_grid, dim3(256), 0, s, q);
   } else {
+    if (sums != nullptr && (e = launch_column_partial(*sums, nullptr, 0, std::is_same_v<T, BF16>, s, &last)) != hipSuccess) return e;
     dim3 grid(groups, p.kv * kblocks * cblocks, 1);
     hipLaunchKernelGGL((wgrad_atomic_kernel<T>), grid, dim3(256), 0, s, p);
   }
   e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((wgrad_finalize_kernel<T>), dim3((unsigned)((f.total / 4 + 255) / 256)), dim3(256), 0, s, f);
+  hipLaunchKernelGGL((wgrad_finalize_kernel<T>), dim3((unsigned)((f.total / 4 + 255) / 256) + last.groups), dim3(256), 0, s, f, last);
   return hipGetLastError();
 }
 
@@ -246,19 +255,20 @@ int CUMM_CAT(wgrad_ordered_resident_, CUMM_NAME)(bool wide) {
 }
 
 hipError_t CUMM_CAT(launch_wgrad_ordered_, CUMM_NAME)(const WgradParams &p, const WgradPrepareParams &pre,
-                                                      const WgradOrderedParams &f, bool wide, int wgs, hipStream_t s) {
+                                                      const WgradOrderedParams &f, bool wide, int wgs, const ColumnSumParams *sums,
+                                                      hipStream_t s) {
   using T = CUMM_ELEM;
   if (p.num_red == 0 || p.kv == 0 || wgs < 1) return hipSuccess;
   if (!(wide ? counted_waits_hold<wgrad_units_kernel<T, 2, 2, 1, true>>() : counted_waits_hold<wgrad_units_kernel<T, 1, 1, 2, true>>()))
     return hipErrorNotSupported;
-  hipLaunchKernelGGL(wgrad_prepare_kernel, dim3(p.kv), dim3(256), 0, s, pre);   // lists only: no image to zero
-  hipError_t e = hipGetLastError();
+  ColumnFinalParams last = {};
+  hipError_t e = prepare<T>(pre, p.kv, sums, &last, s);   // lists only: no image to zero
   if (e != hipSuccess) return e;
   if (wide) hipLaunchKernelGGL((wgrad_units_kernel<T, 2, 2, 1, true>), dim3(wgs), dim3(256), 0, s, p);
   else hipLaunchKernelGGL((wgrad_units_kernel<T, 1, 1, 2, true>), dim3(wgs), dim3(256), 0, s, p);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((wgrad_finalize_ordered_kernel<T>), dim3((unsigned)((f.total / 4 + 31) / 32)), dim3(256), 0, s, f);
+  hipLaunchKernelGGL((wgrad_finalize_ordered_kernel<T>), dim3((unsigned)((f.total / 4 + 31) / 32) + last.groups), dim3(256), 0, s, f, last);
   return hipGetLastError();
 }
 #endif

@@ -45,7 +45,7 @@ struct Api {
   CUMM_API(column_sum_workspace);
   CUMM_API(query_conv_workspace);
   CUMM_API(query_wgrad_ordered_workspace);
-  CUMM_API(wgrad_pairs);
+  CUMM_API(wgrad_pairs_sums);
   CUMM_API(wgrad_pairs_workspace);
   CUMM_API(subm_pairs);
   CUMM_API(subm_pairs_workspace);
@@ -68,7 +68,7 @@ void bind(const py::dict &addresses) {
   CUMM_API(column_sum_workspace);
   CUMM_API(query_conv_workspace);
   CUMM_API(query_wgrad_ordered_workspace);
-  CUMM_API(wgrad_pairs);
+  CUMM_API(wgrad_pairs_sums);
   CUMM_API(wgrad_pairs_workspace);
   CUMM_API(subm_pairs);
   CUMM_API(subm_pairs_workspace);
@@ -366,7 +366,7 @@ struct SparseConvBackward : public torch::autograd::Node {
     return result;
   }
 
-  bool native(const Tensor &x, const Tensor &w, const Tensor &y, Tensor gy, const bool (&need)[3], torch::autograd::variable_list &result) {
+  bool native(const Tensor &x, const Tensor &w, const Tensor &y, const Tensor &gy, const bool (&need)[3], torch::autograd::variable_list &result) {
     const int dtype = tv_type(x.scalar_type());
     const auto expected = [&](const Tensor &t) { return plain(t, *g) && t.is_contiguous() && t.scalar_type() == x.scalar_type(); };
     if (dtype < 0 || c10::impl::TorchDispatchModeTLS::any_modes_set() || !expected(x) || !expected(w) || !expected(gy) ||
@@ -389,35 +389,30 @@ struct SparseConvBackward : public torch::autograd::Node {
     const auto stream = current_stream();
     const auto s = stream.stream();
     g->used_on(stream);
-    // the gradient passes where the fused ReLU let the output through; its column sums are the bias gradient
+    // the gradient passes where the fused ReLU let the output through; its column sums are the bias gradient.
+    // With a weight gradient behind them its launches make both.
     const int64_t rows = gy.size(0);
+    Tensor sums_ws;
+    CummHipGateSums sums = {};
     if (need[2]) {
       result[2] = at::empty({k_out}, gy.options());
-      const Tensor ws = bytes((int64_t)api.column_sum_workspace(rows, (int)k_out), g->device);
-      if (relu) {
-        const Tensor gated = at::empty_like(gy);
-        check(api.relu_backward_sums(gated.data_ptr(), result[2].data_ptr(), gy.data_ptr(), y.data_ptr(), rows, (int)k_out, dtype,
-                                     ws.data_ptr(), (size_t)ws.numel(), s));
-        gy = gated;
-      } else {
-        check(api.column_sum(result[2].data_ptr(), gy.data_ptr(), rows, (int)k_out, dtype, ws.data_ptr(), (size_t)ws.numel(), s));
-      }
-    } else if (relu) {
-      const Tensor gated = at::empty_like(gy);
-      check(api.relu_backward(gated.data_ptr(), gy.data_ptr(), y.data_ptr(), (size_t)gy.numel(), dtype, s));
-      gy = gated;
+      sums_ws = bytes((int64_t)api.column_sum_workspace(rows, (int)k_out), g->device);
+      sums.sums = result[2].data_ptr(); sums.grad = gy.data_ptr();
+      sums.rows = rows; sums.channels = (int32_t)k_out;
+      sums.workspace = sums_ws.data_ptr(); sums.workspace_bytes = (size_t)sums_ws.numel();
     }
-    if (need[0]) {
-      // inputs that feed no output site lie in tiles of mask 0: the kernel writes their zeros
-      result[0] = at::empty_like(x);
-      CummHipSparseConvMore more = {};
-      more.write_empty = 1;
-      CummHipSparseConvArgs a = moved(*dgrad, *g, g->n_in, g->indices_bwd_pos, g->mask_bwd, g->order_bwd, nullptr);
-      a.ptr_A = gy.data_ptr(); a.ptr_B = w.data_ptr();
-      a.ptr_C = result[0].data_ptr(); a.ptr_D = a.ptr_C;
-      check(api.sparse_conv_more(&dgrad->desc, &a, &more, s));
-      g->made[1] = true;
+    Tensor gated = gy;
+    if (relu) {
+      gated = at::empty_like(gy);
+      sums.gated = gated.data_ptr(); sums.out = y.data_ptr();
     }
+    if (!need[1]) {
+      if (need[2] && relu)
+        check(api.relu_backward_sums(sums.gated, sums.sums, sums.grad, sums.out, rows, (int)k_out, dtype, sums.workspace, sums.workspace_bytes, s));
+      else if (need[2])
+        check(api.column_sum(sums.sums, sums.grad, rows, (int)k_out, dtype, sums.workspace, sums.workspace_bytes, s));
+    }
+    if (!need[2] && relu) check(api.relu_backward(gated.data_ptr(), gy.data_ptr(), y.data_ptr(), (size_t)gy.numel(), dtype, s));
     if (need[1] && wgrad) {
       result[1] = at::empty_like(w);
       int64_t size = api.query_conv_workspace(&wgrad->desc, (int)k_out, (int)(g->kv * c_in), (int)rows, wgrad->args.split_k_slices, g->kv);
@@ -425,19 +420,33 @@ struct SparseConvBackward : public torch::autograd::Node {
       size = std::max(size, (int64_t)256);
       const Tensor ws = bytes(size, g->device);
       CummHipSparseConvArgs a = moved(*wgrad, *g, rows, g->indices_fwd, reduced_at(*g, tile_m), g->order_fwd, nullptr);
-      a.ptr_A = gy.data_ptr(); a.ptr_B = x.data_ptr();
+      a.ptr_A = gated.data_ptr(); a.ptr_B = x.data_ptr();
       a.ptr_C = result[1].data_ptr(); a.ptr_D = a.ptr_C;
       a.workspace = ws.data_ptr(); a.workspace_bytes = (size_t)size;
-      check(api.sparse_conv(&wgrad->desc, &a, s));
+      CummHipSparseConvMore more = {};
+      more.sums = need[2] ? &sums : nullptr;
+      check(api.sparse_conv_more(&wgrad->desc, &a, &more, s));
       g->made[2] = true;
     } else if (need[1]) {
       // the products of all kernel offsets over their pair lists (an offset without pairs writes zeros)
       result[1] = at::empty_like(w);
       const Tensor ws = bytes(list_bytes, g->device);
       const int32_t *pair_in = g->lists.data_ptr<int32_t>(), *pair_out = pair_in + (int64_t)g->kv * g->n_out;
-      check(api.wgrad_pairs(result[1].data_ptr(), gy.data_ptr(), x.data_ptr(), pair_out, pair_in, g->counts.data(), g->kv, g->n_out,
-                            (int)g->n_out, (int)g->n_in, (int)k_out, (int)c_in, dtype, ws.data_ptr(), (size_t)list_bytes, s));
+      check(api.wgrad_pairs_sums(result[1].data_ptr(), gated.data_ptr(), x.data_ptr(), pair_out, pair_in, g->counts.data(), g->kv, g->n_out,
+                                 (int)g->n_out, (int)g->n_in, (int)k_out, (int)c_in, dtype, need[2] ? &sums : nullptr, ws.data_ptr(),
+                                 (size_t)list_bytes, s));
       g->made[2] = true;
+    }
+    if (need[0]) {
+      // inputs that feed no output site lie in tiles of mask 0: the kernel writes their zeros
+      result[0] = at::empty_like(x);
+      CummHipSparseConvMore more = {};
+      more.write_empty = 1;
+      CummHipSparseConvArgs a = moved(*dgrad, *g, g->n_in, g->indices_bwd_pos, g->mask_bwd, g->order_bwd, nullptr);
+      a.ptr_A = gated.data_ptr(); a.ptr_B = w.data_ptr();
+      a.ptr_C = result[0].data_ptr(); a.ptr_D = a.ptr_C;
+      check(api.sparse_conv_more(&dgrad->desc, &a, &more, s));
+      g->made[1] = true;
     }
     return true;
   }

@@ -26,6 +26,7 @@
 //     unit of one (offset, channel block) and stores it into a slot of its own; the last kernel adds
 //     the slots of an element in workgroup order.  Same bits from run to run on one device.
 #pragma once
+#include "column_sum.h"
 #include "common.h"
 #include "lds_dma.h"
 
@@ -236,17 +237,18 @@ struct WgradPrepareParams {
   int32_t *live_list;         // [kv * num_red]
 };
 
-// workgroup r < kv compacts the tiles of offset r; the others zero the fp32 image
-static __global__ __launch_bounds__(256) void wgrad_prepare_kernel(const WgradPrepareParams p) {
+// workgroup r < kv of 256 threads compacts the tiles of offset r; the others zero the fp32 image
+constexpr int kWgradZeroBlocks = 256;
+__device__ __forceinline__ void wgrad_prepare(const WgradPrepareParams &p, int block, int blocks) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if ((int)blockIdx.x >= p.kv) {
-    const int64_t nz = (int64_t)(gridDim.x - p.kv) * 256;   // scratch_floats is a multiple of 4
+  if (block >= p.kv) {
+    const int64_t nz = (int64_t)(blocks - p.kv) * 256;   // scratch_floats is a multiple of 4
     v4f *z = reinterpret_cast<v4f *>(p.scratch);
-    for (int64_t i = (int64_t)(blockIdx.x - p.kv) * 256 + tid; i < p.scratch_floats / 4; i += nz) z[i] = v4f{0, 0, 0, 0};
+    for (int64_t i = (int64_t)(block - p.kv) * 256 + tid; i < p.scratch_floats / 4; i += nz) z[i] = v4f{0, 0, 0, 0};
     return;
   }
   __shared__ int wave_cnt[2][4];
-  const int r = blockIdx.x;
+  const int r = block;
   const bool on = (p.mask_filter >> r) & 1u;
   int base = 0;
   constexpr int U = 8;   // mask words a thread has in flight
@@ -282,6 +284,7 @@ static __global__ __launch_bounds__(256) void wgrad_prepare_kernel(const WgradPr
   }
   if (tid == 0) p.live_cnt[r] = base;
 }
+static __global__ __launch_bounds__(256) void wgrad_prepare_kernel(const WgradPrepareParams p) { wgrad_prepare(p, blockIdx.x, gridDim.x); }
 
 // a / b for 0 <= a < 2^22, 0 < b < 2^22, without the long integer-division sequence
 __device__ __forceinline__ int fast_div(int a, int b) {
@@ -670,11 +673,17 @@ struct WgradFinalizeParams {
 };
 
 // dW = cvt(alpha * sum of the scratch images + beta * src) for the offsets enabled in mask_filter
-// Four consecutive elements per thread (C is a multiple of 8, so they share their offset).
+// Four consecutive elements per thread (C is a multiple of 8, so they share their offset).  The first workgroups
+// finish the bias sums of the same backward pass, if there are any: a launch of its own is 4.7 us.
 template <class T>
-__global__ __launch_bounds__(256) void wgrad_finalize_kernel(const WgradFinalizeParams p) {
+__global__ __launch_bounds__(256) void wgrad_finalize_kernel(const WgradFinalizeParams p, const ColumnFinalParams sums) {
   using E = Elem<T>;
-  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if ((int)blockIdx.x < sums.groups) {
+    column_final<T>(sums, blockIdx.x);
+    return;
+  }
+  const int64_t block = blockIdx.x - sums.groups;
+  const int64_t i = (block * 256 + threadIdx.x) * 4;
   if (i >= p.total) return;
   const int r = (int)((i / p.C) % p.kv);
   if (!((p.mask_filter >> r) & 1u)) return;
@@ -723,10 +732,15 @@ struct WgradOrderedParams {
 };
 
 template <class T>
-__global__ __launch_bounds__(256) void wgrad_finalize_ordered_kernel(const WgradOrderedParams p) {
+__global__ __launch_bounds__(256) void wgrad_finalize_ordered_kernel(const WgradOrderedParams p, const ColumnFinalParams sums) {
   using E = Elem<T>;
+  if ((int)blockIdx.x < sums.groups) {
+    column_final<T>(sums, blockIdx.x);
+    return;
+  }
+  const int64_t block = blockIdx.x - sums.groups;
   const int g = threadIdx.x & 7;
-  const int64_t i = ((int64_t)blockIdx.x * 32 + (threadIdx.x >> 3)) * 4;
+  const int64_t i = (block * 32 + (threadIdx.x >> 3)) * 4;
   const bool in_range = i < p.total;
   const int64_t ii = in_range ? i : 0;
   const int nn = (int)(ii % p.C);

@@ -26,6 +26,7 @@
 // (6.36 ms); the 125 lists of a 5 x 5 x 5 kernel over 120 k voxels (386 k pairs) 19.2 us + finalize
 // (16.1 ms).
 #pragma once
+#include "column_sum.h"
 #include "common.h"
 #include "lds_dma.h"
 
@@ -253,17 +254,21 @@ __global__ __launch_bounds__(256) void wgrad_pairs_kernel(const WgradPairsParams
 
 // Four consecutive channels of list blockIdx.y per group of G lanes; lane g adds the g-th share of the
 // slots first to last, then the G sums are combined pairwise: the order depends on the number of
-// slots only.  Latency-bound (loads in batches of eight).
+// slots only.  Latency-bound (loads in batches of eight).  With bias sums to finish their workgroups come first.
 template <class T, int G, bool WIDE>
-__global__ __launch_bounds__(256) void wgrad_pairs_finalize_kernel(const WgradPairsFinalizeParams p) {
+__global__ __launch_bounds__(256) void wgrad_pairs_finalize_kernel(const WgradPairsFinalizeParams p, const ColumnFinalParams sums) {
   using E = Elem<T>;
+  const int r = (int)blockIdx.y - (sums.groups > 0 ? 1 : 0);
+  if (r < 0) {
+    for (int group = blockIdx.x; group < sums.groups; group += gridDim.x) column_final<T>(sums, group);
+    return;
+  }
   const uint32_t g = threadIdx.x % G;
   const uint32_t group = blockIdx.x * (256 / G) + threadIdx.x / G;
   const uint32_t c4 = (uint32_t)p.C / 4u;
   const bool on = group < (uint32_t)p.K * c4;
   const uint32_t gg = on ? group : 0u;
   const int nn = (int)(gg % c4) * 4, mm = (int)(gg / c4);
-  const int r = blockIdx.y;
   const int combos = p.kblocks * p.cblocks;
   const int s0 = p.step0[r], s1 = p.step0[r + 1];
   const int b0 = s0 / p.per_wg;

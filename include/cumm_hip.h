@@ -163,10 +163,25 @@ typedef struct CummHipSparseConvArgs {
                                        Any other value than that is an error. */
 } CummHipSparseConvArgs;
 
+/* The bias gradient of a layer, and the gate of its fused ReLU in front of both: gated = grad where out > 0, else 0, and
+ * sums[c] = the sum of column c of gated.  gated and out NULL: sums of grad itself.  As cumm_hip_relu_backward_sums /
+ * cumm_hip_column_sum, whose rules for the operands and the workspace hold. */
+typedef struct CummHipGateSums {
+  void *gated;                      /* [rows, channels] */
+  void *sums;                       /* [channels] */
+  const void *grad, *out;           /* [rows, channels] */
+  int64_t rows;
+  int32_t channels;
+  void *workspace;                  /* cumm_hip_column_sum_workspace bytes, not shared with the call's own */
+  size_t workspace_bytes;
+} CummHipGateSums;
+
 /* What a training program wants of the same launches beyond the reference's argument block; all zero = nothing. */
 typedef struct CummHipSparseConvMore {
   int32_t write_empty;              /* backward-input.  Non-zero: rows of tiles without any kernel offset are written like
                                        all others (zeros, with beta == 0), not left alone: the caller fills nothing */
+  const CummHipGateSums *sums;      /* backward-weight, NULL = none.  Gate and bias gradient made by the launches of this call,
+                                       which reads the gated rows: ptr_A == gated (or grad) */
 } CummHipSparseConvMore;
 
 /* Replaces GemmMainUnitTest.matmul2 below its prelude
@@ -425,6 +440,10 @@ int64_t cumm_hip_wgrad_pairs_workspace(const int32_t *counts, int lists, int K, 
 int cumm_hip_wgrad_pairs(void *dw, const void *dout, const void *inp, const int32_t *pair_out, const int32_t *pair_in,
                          const int32_t *counts, int lists, int64_t list_stride, int rows_out, int rows_in, int K, int C,
                          int dtype, void *workspace, size_t workspace_bytes, void *stream);
+/* The same, with the gate and the bias gradient of the layer in its launches (sums NULL = the call above). */
+int cumm_hip_wgrad_pairs_sums(void *dw, const void *dout, const void *inp, const int32_t *pair_out, const int32_t *pair_in,
+                              const int32_t *counts, int lists, int64_t list_stride, int rows_out, int rows_in, int K, int C,
+                              int dtype, const CummHipGateSums *sums, void *workspace, size_t workspace_bytes, void *stream);
 
 /* Masks of a pair table, any kernel volume up to 128: mask [n, words], words = ceil(kv / 32), bit b of
  * word w of output o set wherever indices[32 w + b][o] >= 0 (the layout a dynamic_mask descriptor takes;

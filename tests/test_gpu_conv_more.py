@@ -102,3 +102,69 @@ def test_special_values_through_the_epilogue(dtype, tile, act, with_bias):
     np.testing.assert_array_equal(a[~nan] & 0x7FFF, b[~nan] & 0x7FFF)
     keep = ~nan & ((a & 0x7FFF) != 0) if act == Activation.None_ else ~nan      # (the sign of a zero sum is the matrix unit's)
     np.testing.assert_array_equal(a[keep], b[keep])
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("n,cin,k_out,slices,ordered", [
+    (1, 8, 8, 32, False),            # one row
+    (3000, 64, 64, 32, False),       # lists, a copy of the image per eighth of the units
+    (3000, 64, 64, 32, True),        # lists, slots in a fixed order
+    (2500, 136, 72, 32, False),      # units of 128 x 128 channels; a group of bias sums that is half empty
+    (2500, 136, 72, 32, True),
+    (3000, 64, 64, 1, False),        # the tiled kernel
+    (66000, 8, 1000, 32, False),     # sums in two stages
+])
+@pytest.mark.parametrize("relu", [False, True])
+def test_gate_and_sums_of_a_weight_gradient(dtype, n, cin, k_out, slices, ordered, relu):
+    """Gate and bias gradient in the launches of the weight gradient against numpy.  Small whole numbers: every sum is
+    exact in fp32 whatever its order, and is rounded once."""
+    print("case gate and sums", dtype, n, cin, k_out, slices, ordered, relu, flush=True)
+    rng = np.random.default_rng(n + cin)
+    grad, out, x = (rng.integers(-1, 2, size=(n, c)).astype(np.float32) for c in (k_out, k_out, cin))
+    kv = 2
+    indices = np.stack([rng.permutation(n), np.where(rng.random(n) < 0.5, rng.permutation(n), -1)]).astype(np.int32)
+    mask = (1 + 2 * (indices[1] >= 0)).astype(np.uint32)
+    ms, order = pairs.sort_by_mask(mask)
+    width = 64
+    red = np.bitwise_or.reduceat(ms, np.arange(0, n, width)).astype(np.uint32)
+    gated = np.where(out > 0, grad, np.float32(0)) if relu else grad
+    dw = np.stack([gated.T @ x[indices[0]], gated[indices[1] >= 0].T @ x[indices[1][indices[1] >= 0]]], axis=1)
+
+    p = ConvParams(3, ConvOpType.BackwardWeight)
+    p.conv_algo_desp = H.find_conv_desp(dtype, ConvOpType.BackwardWeight, 64, 64, split_k_parallel=True)
+    d_grad, d_out = H.dev(H.to_storage(grad, dtype), dtype), H.dev(H.to_storage(out, dtype), dtype)
+    d_gated = H.dev(H.to_storage(np.full_like(grad, 9.0), dtype), dtype) if relu else d_grad
+    p.input, p.output = H.dev(H.to_storage(x, dtype), dtype), d_gated
+    p.weight = tv.zeros([k_out, kv, cin], H.TV_DTYPE[dtype], 0)
+    p.indices, p.mask, p.mask_argsort = H.dev(indices, "i32"), H.dev(red, "u32"), H.dev(order, "i32")
+    p.mask_width, p.split_k_slices, p.deterministic = width, slices, ordered
+    ConvMainUnitTest.implicit_gemm2(p)      # (of whatever d_gated holds)
+    sums = tv.zeros([k_out], H.TV_DTYPE[dtype], 0)
+    need = int(_capi.lib().cumm_hip_column_sum_workspace(n, k_out))
+    ws = tv.zeros([need], tv.uint8, 0)
+    gs = _capi.GateSums(gated=d_gated.byte_pointer() if relu else None, sums=sums.byte_pointer(), grad=d_grad.byte_pointer(),
+                        out=d_out.byte_pointer() if relu else None, rows=n, channels=k_out, workspace=ws.byte_pointer(),
+                        workspace_bytes=need)
+    _again(p, sums=ctypes.addressof(gs))
+    np.testing.assert_array_equal(H.as_f32(H.host(d_gated), dtype), gated)
+    np.testing.assert_array_equal(H.host(sums).view(np.uint16), H.to_storage(gated.sum(axis=0), dtype).view(np.uint16))
+    np.testing.assert_array_equal(H.as_f32(H.host(p.weight), dtype), H.as_f32(H.to_storage(dw, dtype), dtype))
+
+
+def test_gate_and_sums_are_of_the_gradient_of_the_call():
+    """Sums of another tensor than the one that the call reads are refused, as is a pass without a weight gradient."""
+    lib, ws = _capi.lib(), tv.zeros([1 << 16], tv.uint8, 0)
+    t = [tv.zeros([64, 64], tv.float16, 0) for _ in range(3)]
+    gs = _capi.GateSums(gated=None, sums=ws.byte_pointer(), grad=t[2].byte_pointer(), rows=64, channels=64,
+                        workspace=ws.byte_pointer() + 4096, workspace_bytes=1 << 15)
+    for op, parallel in ((ConvOpType.BackwardWeight, True), (ConvOpType.Forward, False)):
+        p = ConvParams(3, op)
+        p.conv_algo_desp = H.find_conv_desp("f16", op, 64, 64, split_k_parallel=parallel)
+        p.input, p.output, p.weight = t[0], t[1], tv.zeros([64, 1, 64], tv.float16, 0)
+        p.indices, p.mask, p.mask_argsort = (H.dev(np.arange(64, dtype=np.int32)[None], "i32"), H.dev(np.ones(64, np.uint32), "u32"),
+                                             H.dev(np.arange(64, dtype=np.int32), "i32"))
+        if parallel:
+            p.mask, p.mask_width, p.split_k_slices = H.dev(np.ones(1, np.uint32), "u32"), 64, 4
+        ConvMainUnitTest.implicit_gemm2(p)
+        with pytest.raises(ValueError):
+            _again(p, sums=ctypes.addressof(gs))
