@@ -66,7 +66,7 @@ class GateSums(C.Structure):
 
 
 class SparseConvMore(C.Structure):
-    _fields_ = [("write_empty", C.c_int32), ("sums", C.c_void_p)]
+    _fields_ = [("write_empty", C.c_int32), ("sums", C.c_void_p), ("by_position", C.c_void_p)]
 
 
 class OrderSide(C.Structure):

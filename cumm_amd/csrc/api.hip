@@ -931,6 +931,7 @@ int sparse_conv_impl(const CummHipConvDesc *desc, const CummHipSparseConvArgs *a
     std::memset(&w, 0, sizeof(w));
     w.dout = a->ptr_A; w.inp = a->ptr_B; w.scratch = reinterpret_cast<float *>(base + lay.slots_at);
     w.argsort = a->mask_argsort_ptr; w.indices = a->indice_ptr; w.red_mask = a->mask_ptr;
+    w.by_position = more != nullptr ? more->by_position : nullptr;
     w.num_red = lay.num_red; w.mask_width = a->mask_width; w.mask_filter = a->mask_filter;
     w.n_pos = a->N; w.n_idx = a->N; w.rows_x = a->rows_in; w.rows_y = a->rows_out;
     w.K = a->K; w.C = a->C; w.kv = kv; w.tiles_per_wg = qt;
@@ -972,6 +973,7 @@ int sparse_conv_impl(const CummHipConvDesc *desc, const CummHipSparseConvArgs *a
     std::memset(&w, 0, sizeof(w));
     w.dout = a->ptr_A; w.inp = a->ptr_B; w.scratch = reinterpret_cast<float *>(workspace);
     w.argsort = a->mask_argsort_ptr; w.indices = a->indice_ptr; w.red_mask = a->mask_ptr;
+    w.by_position = more != nullptr ? more->by_position : nullptr;
     w.num_red = (a->N + a->mask_width - 1) / a->mask_width; w.mask_width = a->mask_width;
     w.mask_filter = a->mask_filter;
     w.n_pos = a->N; w.n_idx = a->N; w.rows_x = a->rows_in; w.rows_y = a->rows_out;

@@ -182,6 +182,23 @@ static hipError_t prepare(const WgradPrepareParams &pre, int blocks, const Colum
   return hipGetLastError();
 }
 
+// The unit-walking kernel, for 128 x 128 channels or 64 x 64
+template <class T, bool DET>
+static bool units_ok(bool wide, bool by_position) {
+  if (by_position) return wide ? counted_waits_hold<wgrad_units_kernel<T, 2, 2, 1, DET, true>>() : counted_waits_hold<wgrad_units_kernel<T, 1, 1, 2, DET, true>>();
+  return wide ? counted_waits_hold<wgrad_units_kernel<T, 2, 2, 1, DET>>() : counted_waits_hold<wgrad_units_kernel<T, 1, 1, 2, DET>>();
+}
+template <class T, bool DET>
+static void launch_units(bool wide, const WgradParams &p, dim3 grid, hipStream_t s) {
+  if (p.by_position != nullptr) {
+    if (wide) hipLaunchKernelGGL((wgrad_units_kernel<T, 2, 2, 1, DET, true>), grid, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((wgrad_units_kernel<T, 1, 1, 2, DET, true>), grid, dim3(256), 0, s, p);
+  } else {
+    if (wide) hipLaunchKernelGGL((wgrad_units_kernel<T, 2, 2, 1, DET>), grid, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((wgrad_units_kernel<T, 1, 1, 2, DET>), grid, dim3(256), 0, s, p);
+  }
+}
+
 hipError_t CUMM_CAT(launch_wgrad_atomic_, CUMM_NAME)(const WgradParams &p, const WgradPrepareParams &pre,
                                                      const WgradFinalizeParams &f, const ColumnSumParams *sums, hipStream_t s) {
   using T = CUMM_ELEM;
@@ -193,8 +210,7 @@ hipError_t CUMM_CAT(launch_wgrad_atomic_, CUMM_NAME)(const WgradParams &p, const
   if (groups == 0 || p.kv == 0) return hipSuccess;
   hipError_t e;
   ColumnFinalParams last = {};
-  const bool units_ok = wide ? counted_waits_hold<wgrad_units_kernel<T, 2, 2, 1>>() : counted_waits_hold<wgrad_units_kernel<T, 1, 1, 2>>();
-  if (p.live_list != nullptr && !units_ok) return hipErrorNotSupported;
+  if (p.live_list != nullptr && !units_ok<T, false>(wide, p.by_position != nullptr)) return hipErrorNotSupported;
   if (p.live_list != nullptr) {
     // lists + zeroed image, then a resident grid that walks the units
     static int resident_of[2][16] = {};
@@ -221,8 +237,7 @@ hipError_t CUMM_CAT(launch_wgrad_atomic_, CUMM_NAME)(const WgradParams &p, const
     // never more workgroups than units can exist
     const long long max_units = ((long long)groups * p.kv + p.kv) * (q.merge_blocks ? 1 : kblocks * cblocks);
     const dim3 units_grid((unsigned)(max_units < resident ? max_units : resident));
-    if (wide) hipLaunchKernelGGL((wgrad_units_kernel<T, 2, 2, 1>), units_grid, dim3(256), 0, s, q);
-    else hipLaunchKernelGGL((wgrad_units_kernel<T, 1, 1, 2>), units_grid, dim3(256), 0, s, q);
+    launch_units<T, false>(wide, q, units_grid, s);
   } else {
     if (sums != nullptr && (e = launch_column_partial(*sums, nullptr, 0, std::is_same_v<T, BF16>, s, &last)) != hipSuccess) return e;
     dim3 grid(groups, p.kv * kblocks * cblocks, 1);
@@ -259,13 +274,11 @@ hipError_t CUMM_CAT(launch_wgrad_ordered_, CUMM_NAME)(const WgradParams &p, cons
                                                       hipStream_t s) {
   using T = CUMM_ELEM;
   if (p.num_red == 0 || p.kv == 0 || wgs < 1) return hipSuccess;
-  if (!(wide ? counted_waits_hold<wgrad_units_kernel<T, 2, 2, 1, true>>() : counted_waits_hold<wgrad_units_kernel<T, 1, 1, 2, true>>()))
-    return hipErrorNotSupported;
+  if (!units_ok<T, true>(wide, p.by_position != nullptr)) return hipErrorNotSupported;
   ColumnFinalParams last = {};
   hipError_t e = prepare<T>(pre, p.kv, sums, &last, s);   // lists only: no image to zero
   if (e != hipSuccess) return e;
-  if (wide) hipLaunchKernelGGL((wgrad_units_kernel<T, 2, 2, 1, true>), dim3(wgs), dim3(256), 0, s, p);
-  else hipLaunchKernelGGL((wgrad_units_kernel<T, 1, 1, 2, true>), dim3(wgs), dim3(256), 0, s, p);
+  launch_units<T, true>(wide, p, dim3(wgs), s);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((wgrad_finalize_ordered_kernel<T>), dim3((unsigned)((f.total / 4 + 31) / 32) + last.groups), dim3(256), 0, s, f, last);

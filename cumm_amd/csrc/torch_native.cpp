@@ -425,6 +425,7 @@ struct SparseConvBackward : public torch::autograd::Node {
       a.workspace = ws.data_ptr(); a.workspace_bytes = (size_t)size;
       CummHipSparseConvMore more = {};
       more.sums = need[2] ? &sums : nullptr;
+      more.by_position = g->indices_fwd_pos;
       check(api.sparse_conv_more(&wgrad->desc, &a, &more, s));
       g->made[2] = true;
     } else if (need[1]) {

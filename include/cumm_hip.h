@@ -182,6 +182,9 @@ typedef struct CummHipSparseConvMore {
                                        all others (zeros, with beta == 0), not left alone: the caller fills nothing */
   const CummHipGateSums *sums;      /* backward-weight, NULL = none.  Gate and bias gradient made by the launches of this call,
                                        which reads the gated rows: ptr_A == gated (or grad) */
+  const int32_t *by_position;       /* backward-weight, NULL = none.  The table of indice_ptr by position as well
+                                       (cumm_hip_order_pairs, cumm_hip_pairs_by_position): [kernel_volume, N], column = sorted
+                                       position.  Kernels that can read it instead do */
 } CummHipSparseConvMore;
 
 /* Replaces GemmMainUnitTest.matmul2 below its prelude

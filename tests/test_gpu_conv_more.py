@@ -116,7 +116,8 @@ def test_special_values_through_the_epilogue(dtype, tile, act, with_bias):
 ])
 @pytest.mark.parametrize("relu", [False, True])
 def test_gate_and_sums_of_a_weight_gradient(dtype, n, cin, k_out, slices, ordered, relu):
-    """Gate and bias gradient in the launches of the weight gradient against numpy.  Small whole numbers: every sum is
+    """Gate and bias gradient in the launches of the weight gradient, with the table by row and by position, against
+    numpy.  Small whole numbers: every sum is
     exact in fp32 whatever its order, and is rounded once."""
     print("case gate and sums", dtype, n, cin, k_out, slices, ordered, relu, flush=True)
     rng = np.random.default_rng(n + cin)
@@ -145,10 +146,14 @@ def test_gate_and_sums_of_a_weight_gradient(dtype, n, cin, k_out, slices, ordere
     gs = _capi.GateSums(gated=d_gated.byte_pointer() if relu else None, sums=sums.byte_pointer(), grad=d_grad.byte_pointer(),
                         out=d_out.byte_pointer() if relu else None, rows=n, channels=k_out, workspace=ws.byte_pointer(),
                         workspace_bytes=need)
-    _again(p, sums=ctypes.addressof(gs))
-    np.testing.assert_array_equal(H.as_f32(H.host(d_gated), dtype), gated)
-    np.testing.assert_array_equal(H.host(sums).view(np.uint16), H.to_storage(gated.sum(axis=0), dtype).view(np.uint16))
-    np.testing.assert_array_equal(H.as_f32(H.host(p.weight), dtype), H.as_f32(H.to_storage(dw, dtype), dtype))
+    by_position = H.dev(np.ascontiguousarray(indices[:, order]), "i32")
+    for more in ({}, {"by_position": by_position.byte_pointer()}):
+        _again(p, sums=ctypes.addressof(gs), **more)
+        np.testing.assert_array_equal(H.as_f32(H.host(d_gated), dtype), gated)
+        np.testing.assert_array_equal(H.host(sums).view(np.uint16), H.to_storage(gated.sum(axis=0), dtype).view(np.uint16))
+        np.testing.assert_array_equal(H.as_f32(H.host(p.weight), dtype), H.as_f32(H.to_storage(dw, dtype), dtype))
+        for t in (sums, p.weight) + ((d_gated,) if relu else ()):
+            _capi.check(_capi.lib().cumm_hip_memset(t.byte_pointer(), 0x55, t.size * t.itemsize, None))
 
 
 def test_gate_and_sums_are_of_the_gradient_of_the_call():
