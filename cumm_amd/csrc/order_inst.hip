@@ -93,6 +93,7 @@ struct OrderParams {
   Side side[2];
   int32_t sides, kv, words;
   int32_t rows_per_chunk;
+  int32_t sparse;              // tables by position: only runs of 128 positions with a pair
   int32_t *give_ups;
   uint32_t base[kExact + 2];   // first key of the words with c offsets; [kExact + 1]: of those with more
   uint32_t share;              // keys per number of offsets above kExact
@@ -572,6 +573,10 @@ __global__ __launch_bounds__(kPassThreads) void order_pass_kernel(const OrderPar
 // the row itself, and of the others those are fetched that some lane of the wave has (the positions are
 // sorted by their masks: few).  (Mask and entry carried through both passes instead: 14 us less here
 // at 1.1 M positions, 20 us more there.)
+// sparse: of the 27 entries of a position one or two are pairs, and the kernels look at a table only where a tile of
+// 64 or 128 positions has the offset; the rest of it - 86 MB for 798 k positions - is not written: 38.4 -> 25.0 us at
+// 1.1 M positions, 17.4 -> 12.2 at 447 k, and the layers after it find more in the caches (stride 2, 32 -> 64 channels
+// forward 57 -> 50 us).
 constexpr int kLight = 3, kHeavy = 10;
 template <int WORDS>
 __global__ __launch_bounds__(256) void order_position_kernel(const OrderParams p) {
@@ -613,6 +618,10 @@ __global__ __launch_bounds__(256) void order_position_kernel(const OrderParams p
       v[u] = (fetch >> u) & 1u ? e : v[u];
     }
   }
+  const uint32_t o = wave_or_dpp(mine);
+  if (lane == 0) half_or[wave] = o;
+  __syncthreads();
+  const uint32_t write = p.sparse ? (uint32_t)__builtin_amdgcn_readfirstlane((int)(half_or[wave & ~1] | half_or[wave | 1])) : ~0u;
   const int bytes = (int)((uint32_t)p.kv * (uint32_t)d.n * 4u);
   const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(d.by_pos, 0, bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t rev = __builtin_amdgcn_make_buffer_rsrc(d.by_pos_rev, 0, d.by_pos_rev ? bytes : 0, 0x00020000);
@@ -620,6 +629,7 @@ __global__ __launch_bounds__(256) void order_position_kernel(const OrderParams p
 #pragma unroll
     for (int u = 0; u < 32; ++u) {
       if (k0 + u >= p.kv) break;
+      if (!((write >> u) & 1u)) continue;
       __builtin_amdgcn_raw_buffer_store_b32(v[u], to, (uint32_t)pos * 4u, (k0 + u) * d.n * 4, 0);
       if (d.by_pos_rev != nullptr) __builtin_amdgcn_raw_buffer_store_b32(v[u], rev, (uint32_t)pos * 4u, (p.kv - 1 - k0 - u) * d.n * 4, 0);
     }
@@ -631,9 +641,6 @@ __global__ __launch_bounds__(256) void order_position_kernel(const OrderParams p
     if (block == 0 && t < 8) d.hint_slot[t] = 0;
     return;
   }
-  const uint32_t o = wave_or_dpp(mine);
-  if (lane == 0) half_or[wave] = o;
-  __syncthreads();
   if (t < 2) {
     const int run = block * 2 + t;
     const int c0 = __builtin_popcount(half_or[2 * t]), c1 = __builtin_popcount(half_or[2 * t + 1]);
@@ -713,7 +720,7 @@ hipError_t launch_order_pairs(const OrderPairsSide *sides, int n_sides, int kv, 
                               int32_t *give_ups, bool coarse, hipStream_t s) {
   OrderParams p;
   std::memset(&p, 0, sizeof(p));
-  p.kv = kv; p.words = (kv + 31) / 32; p.give_ups = give_ups;
+  p.kv = kv; p.words = (kv + 31) / 32; p.give_ups = give_ups; p.sparse = coarse;
   p.filter = kv < 32 ? (1u << kv) - 1u : 0xFFFFFFFFu;
   char *at = reinterpret_cast<char *>(workspace);
   auto take = [&](size_t bytes) { char *q = at; at += up256(bytes); return q; };

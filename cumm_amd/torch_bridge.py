@@ -242,6 +242,7 @@ class SparseConvGeometry:
 
     _TABLES = ("indices_fwd", "indices_bwd", "mask_fwd", "order_fwd", "mask_bwd", "order_bwd", "indices_fwd_pos", "indices_bwd_pos")
     _lists = _list_block = None      # (several mask words only)
+    _partial = frozenset()           # tables by position that are written only where the launches read them
     _native = None                   # the geometry as native code has it
 
     def __init__(self, coords: torch.Tensor, spatial_shape: Sequence[int], ksize=(3, 3, 3), stride=None,
@@ -274,7 +275,9 @@ class SparseConvGeometry:
         # masks, an order of the positions by them, and the pair tables once more in that order: what
         # forward and backward-input read (a tile's entries for one offset are then consecutive in
         # memory); backward-weight keeps the table by row
-        if not ordered:
+        if ordered:
+            self._partial = frozenset(("indices_fwd_pos", "indices_bwd_pos"))
+        else:
             self._order_one_by_one()
         if words > 1:
             self._make_lists()
@@ -412,6 +415,24 @@ class SparseConvGeometry:
             return self.__dict__[name]
         if name not in SparseConvGeometry._TABLES or self.__dict__.get("_block") is None:
             raise AttributeError(name)
+        if name in self._partial:
+            self._complete(name)
+        return self._view(name)
+
+    def _complete(self, name: str) -> None:
+        """Whoever looks at a table by position gets all of it: the entries of runs without a pair are written too (the
+        others once more, as they are)."""
+        side, stream = name[8:11], current_stream()
+        n = self.n_out if side == "fwd" else self.n_in
+        if n:
+            self.used_on(stream)
+            _capi.check(_capi.lib().cumm_hip_pairs_by_position(self._ptr["indices_" + side], self._ptr["order_" + side], self.kv, n,
+                                                               self._ptr[name], stream))
+        if not torch.cuda.is_current_stream_capturing():
+            torch.cuda.current_stream().synchronize()      # (it may be read on any stream)
+            self._partial = self._partial - {name}
+
+    def _view(self, name: str) -> tv.Tensor:
         t = self._tensors.get(name)
         if t is None:
             _, dims, dtype = self._spec[name]
@@ -585,7 +606,7 @@ def _forward_launch(g: SparseConvGeometry, key, roles, relu, stream) -> _Launch:
     dtype = _TORCH_TO_TV[features.dtype]
     p.conv_algo_desp = _desp_like(dtype, ConvOpType.Forward, dynamic=g.words > 1)
     p.input, p.weight, p.output = torch2tensor(features), torch2tensor(weight), torch2tensor(out)
-    p.indices, p.mask, p.mask_argsort = g.indices_fwd_pos, g.mask_fwd, g.order_fwd
+    p.indices, p.mask, p.mask_argsort = g._view("indices_fwd_pos"), g.mask_fwd, g.order_fwd
     p.indices_by_position = True
     p.mask_int_count = g.words
     p.light_prefix = g.light_fwd
@@ -618,7 +639,7 @@ def _backward_input_launch(g: SparseConvGeometry, key, roles, dtype, stream) -> 
     p = ConvParams(3, ConvOpType.BackwardInput)
     p.conv_algo_desp = _desp_like(dtype, ConvOpType.BackwardInput, dynamic=g.words > 1)
     p.input, p.weight, p.output = torch2tensor(grad_in), torch2tensor(weight), torch2tensor(grad_out)
-    p.indices, p.mask, p.mask_argsort = g.indices_bwd_pos, g.mask_bwd, g.order_bwd
+    p.indices, p.mask, p.mask_argsort = g._view("indices_bwd_pos"), g.mask_bwd, g.order_bwd
     p.indices_by_position = True
     p.mask_int_count = g.words
     p.reverse_mask = g.subm

@@ -184,7 +184,8 @@ typedef struct CummHipSparseConvMore {
                                        which reads the gated rows: ptr_A == gated (or grad) */
   const int32_t *by_position;       /* backward-weight, NULL = none.  The table of indice_ptr by position as well
                                        (cumm_hip_order_pairs, cumm_hip_pairs_by_position): [kernel_volume, N], column = sorted
-                                       position.  Kernels that can read it instead do */
+                                       position; one of cumm_hip_order_pairs_coarse with a mask_width of 64 or 128.  Kernels
+                                       that can read it instead do */
 } CummHipSparseConvMore;
 
 /* Replaces GemmMainUnitTest.matmul2 below its prelude
@@ -426,7 +427,9 @@ int cumm_hip_order_pairs(const CummHipOrderSide *sides, int n_sides, const int32
 /* The same, where an order that repeats and groups like masks is enough: of tables of one mask word and
  * up to 2^20 positions (2^19 with by_position_reversed) it is exact up to two offsets only (with
  * by_position_reversed, alone: two beside the middle one, which does not count), which takes one radix pass
- * instead of two; everything else as above. */
+ * instead of two.  The tables by position are written where a tile looks at them: the entries of an offset
+ * in a run of 128 positions (from a multiple of 128) none of which has it are left alone.
+ * Everything else as above. */
 size_t cumm_hip_order_pairs_coarse_workspace(const CummHipOrderSide *sides, int n_sides, int kv);
 int cumm_hip_order_pairs_coarse(const CummHipOrderSide *sides, int n_sides, const int32_t *ksize, void *workspace,
                                 size_t workspace_bytes, void *stream);

@@ -21,6 +21,9 @@ def _table(rng, kv, n, density):
     return t
 
 
+UNWRITTEN = -7
+
+
 def _order(tables, ksize, reverse, entry="cumm_hip_order_pairs"):
     lib, kv = _capi.lib(), tables[0].shape[0]
     words = (kv + 31) // 32
@@ -28,8 +31,8 @@ def _order(tables, ksize, reverse, entry="cumm_hip_order_pairs"):
     for s, t in zip(sides, tables):
         n = t.shape[1]
         d = H.dev(t, "i32")
-        o = {"mask": tv.empty([n, words], tv.uint32, 0), "order": tv.empty([n], tv.int32, 0), "pos": tv.empty([kv, n], tv.int32, 0),
-             "rev": tv.empty([kv, n], tv.int32, 0)}
+        o = {"mask": tv.empty([n, words], tv.uint32, 0), "order": tv.empty([n], tv.int32, 0), "pos": H.dev(np.full((kv, n), UNWRITTEN, np.int32), "i32"),
+             "rev": H.dev(np.full((kv, n), UNWRITTEN, np.int32), "i32")}
         s.indices, s.n, s.sorted_mask, s.argsort = d.byte_pointer(), n, o["mask"].byte_pointer(), o["order"].byte_pointer()
         s.by_position = o["pos"].byte_pointer()
         s.by_position_reversed = o["rev"].byte_pointer() if reverse else None
@@ -158,7 +161,11 @@ def test_one_pass(ksize, n, n2):
         order = g["order"]
         assert np.array_equal(np.sort(order), np.arange(t.shape[1])) and np.array_equal(order, a["order"])
         np.testing.assert_array_equal(g["mask"], m[order])
-        np.testing.assert_array_equal(g["pos"], pairs.pairs_by_position(t, order))
+        want = pairs.pairs_by_position(t, order)
+        # (written where a run of 128 positions has the offset; elsewhere what was there)
+        runs = np.logical_or.reduceat(want >= 0, np.arange(0, t.shape[1], 128), axis=1)
+        written = np.repeat(runs, 128, axis=1)[:, :t.shape[1]]
+        np.testing.assert_array_equal(g["pos"], np.where(written, want, UNWRITTEN))
         if reverse:
             np.testing.assert_array_equal(g["rev"], g["pos"][::-1])
         if m.shape[1] > 1:

@@ -334,3 +334,21 @@ def test_a_geometry_shared_by_streams_and_threads():
         for passed in got:
             for a, b in zip(passed, want):
                 assert float((a.float().cpu() - b).abs().max() / b.abs().max()) < 1e-2
+
+
+@pytest.mark.parametrize("ksize,strided", [((3, 3, 3), False), ((3, 3, 3), True), ((5, 5, 5), False)])
+def test_tables_by_position_are_whole_for_who_looks(ksize, strided):
+    """The launches need entries only where a tile has the offset; the attribute is the whole table, and a layer that
+    ran before gives the same bits after."""
+    import torch
+    from cumm_amd import pairs, torch_bridge as tb
+    print("case whole tables", ksize, strided, flush=True)
+    coords, grid = H.small_cloud(3, 3000, grid=(16, 60, 60))
+    geo = tb.SparseConvGeometry(torch.as_tensor(coords, device="cuda"), grid, ksize, (2, 2, 2) if strided else None, tuple(k // 2 for k in ksize))
+    x = torch.randn(coords.shape[0], 64, device="cuda", dtype=torch.float16)
+    w = torch.randn(64, geo.kv, 64, device="cuda", dtype=torch.float16) * 0.1
+    before = tb.sparse_conv(x, w, None, geo)
+    for side in ("fwd", "bwd"):
+        table, order = H.host(getattr(geo, "indices_" + side)), H.host(getattr(geo, "order_" + side))
+        np.testing.assert_array_equal(H.host(getattr(geo, "indices_%s_pos" % side)), pairs.pairs_by_position(table, order))
+    assert torch.equal(before, tb.sparse_conv(x, w, None, geo))
