@@ -62,11 +62,11 @@ class SparseConvArgs(C.Structure):
 
 class GateSums(C.Structure):
     _fields_ = [("gated", C.c_void_p), ("sums", C.c_void_p), ("grad", C.c_void_p), ("out", C.c_void_p), ("rows", C.c_int64),
-                ("channels", C.c_int32), ("workspace", C.c_void_p), ("workspace_bytes", C.c_size_t)]
+                ("channels", C.c_int32), ("workspace", C.c_void_p), ("workspace_bytes", C.c_size_t), ("gate", C.c_void_p), ("order", C.c_void_p)]
 
 
 class SparseConvMore(C.Structure):
-    _fields_ = [("write_empty", C.c_int32), ("sums", C.c_void_p), ("by_position", C.c_void_p)]
+    _fields_ = [("write_empty", C.c_int32), ("sums", C.c_void_p), ("by_position", C.c_void_p), ("gate", C.c_void_p)]
 
 
 class OrderSide(C.Structure):
@@ -148,6 +148,7 @@ SYMBOLS = {
     "cumm_hip_relu_backward": (C.c_int, [_VP, _VP, _VP, C.c_size_t, C.c_int, _VP]),
     "cumm_hip_column_sum_workspace": (C.c_size_t, [C.c_int64, C.c_int]),
     "cumm_hip_column_sum": (C.c_int, [_VP, _VP, C.c_int64, C.c_int, C.c_int, _VP, C.c_size_t, _VP]),
+    "cumm_hip_gate_sums": (C.c_int, [C.POINTER(GateSums), C.c_int, _VP]),
     "cumm_hip_relu_backward_sums": (C.c_int, [_VP, _VP, _VP, _VP, C.c_int64, C.c_int, C.c_int, _VP, C.c_size_t, _VP]),
     "cumm_hip_gather_rows": (C.c_int, [_VP, _VP, _VP, C.c_int, C.c_int, C.c_size_t, _VP]),
     "cumm_hip_scatter_add_rows": (C.c_int, [_VP, _VP, _VP, C.c_int, C.c_int, C.c_int, C.c_int, _VP]),

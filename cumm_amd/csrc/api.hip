@@ -333,12 +333,14 @@ int gate_sums_params(const CummHipGateSums &g, int dtype, ColumnSumParams *p) {
   std::memset(p, 0, sizeof(*p));
   if (g.channels == 0) return CUMM_HIP_OK;
   if (!g.sums || (!g.grad && g.rows > 0) || !aligned16(g.grad)) return fail(CUMM_HIP_EINVAL, "dst and src (16-byte aligned) must not be empty");
-  if ((g.gated != nullptr) != (g.out != nullptr) || !aligned16(g.gated) || !aligned16(g.out))
-    return fail(CUMM_HIP_EINVAL, "gated, grad and out must be 16-byte aligned and not empty");
+  if ((g.gated != nullptr) != (g.out != nullptr || g.gate != nullptr) || (g.out && g.gate) || !aligned16(g.gated) || !aligned16(g.out))
+    return fail(CUMM_HIP_EINVAL, "gated, grad and out (or gate) must be 16-byte aligned and not empty");
+  if (g.gate && !g.order) return fail(CUMM_HIP_EINVAL, "a gate lies in the order of the positions, which must not be empty");
   const size_t need = sizeof(float) * (size_t)column_sum_blocks(g.rows, g.channels) * (size_t)g.channels;
   if (!g.workspace || g.workspace_bytes < need) return fail(CUMM_HIP_ERUNTIME, "workspace at least %zu bytes.", need);
   if (reinterpret_cast<uintptr_t>(g.workspace) & 3u) return fail(CUMM_HIP_EINVAL, "workspace must be 4-byte aligned");
   p->dst = g.sums; p->src = g.grad; p->out = g.out; p->gated = g.gated;
+  p->gate = reinterpret_cast<const uint8_t *>(g.gate); p->order = g.order;
   p->partial = reinterpret_cast<float *>(g.workspace); p->rows = g.rows; p->channels = g.channels;
   return CUMM_HIP_OK;
 }
@@ -813,6 +815,9 @@ int sparse_conv_impl(const CummHipConvDesc *desc, const CummHipSparseConvArgs *a
     if (int rc = gate_sums_params(*more->sums, dt, &sums_params)) return rc;
     sums = &sums_params;
   }
+  if (more != nullptr && more->gate != nullptr &&
+      (c.op_type != CUMM_HIP_OP_FORWARD || fam != 1 || !is_float16_like(dt) || wide || a->act_type != CUMM_HIP_ACT_RELU))
+    return fail(CUMM_HIP_EINVAL, "only a forward pass with ReLU and a two-byte output leaves a gate");
   if (a->N == 0 && sums == nullptr) return CUMM_HIP_OK;
   const void *ptr_D = a->ptr_D ? a->ptr_D : a->ptr_C;
 
@@ -874,6 +879,12 @@ int sparse_conv_impl(const CummHipConvDesc *desc, const CummHipSparseConvArgs *a
         (int64_t)kv * a->N * 4 >= (int64_t)1 << 31)
       return fail(CUMM_HIP_ERUNTIME, "your data exceed int32 range.");
     p.gather_bytes = (uint32_t)((int64_t)kv * a->N * 4);
+    if (more != nullptr && more->gate != nullptr) {
+      const int64_t bytes = (int64_t)((a->K + 63) / 64) * a->N * 8;
+      if (bytes >= (int64_t)1 << 31) return fail(CUMM_HIP_ERUNTIME, "your data exceed int32 range.");
+      p.gate = reinterpret_cast<uint8_t *>(more->gate);
+      p.gate_bytes = (uint32_t)bytes;
+    }
     p.stream_stores = p.c_bytes <= kStreamStoreMaxBytes;
     p.small_stages = d.num_stage >= 3;
     p.one_order = a->deterministic;
@@ -1798,9 +1809,14 @@ static int column_sum_checked(const CummHipGateSums &g, int dtype, void *stream)
   return CUMM_HIP_OK;
 }
 
+int cumm_hip_gate_sums(const CummHipGateSums *g, int dtype, void *stream) {
+  if (!g) return fail(CUMM_HIP_EINVAL, "null arguments");
+  return column_sum_checked(*g, dtype, stream);
+}
+
 int cumm_hip_column_sum(void *dst, const void *src, int64_t rows, int channels, int dtype, void *workspace,
                         size_t workspace_bytes, void *stream) {
-  return column_sum_checked({nullptr, dst, src, nullptr, rows, channels, workspace, workspace_bytes}, dtype, stream);
+  return column_sum_checked({nullptr, dst, src, nullptr, rows, channels, workspace, workspace_bytes, nullptr, nullptr}, dtype, stream);
 }
 
 int cumm_hip_relu_backward_sums(void *gated, void *sums, const void *grad, const void *out, int64_t rows, int channels, int dtype,
@@ -1808,7 +1824,8 @@ int cumm_hip_relu_backward_sums(void *gated, void *sums, const void *grad, const
   if (rows > 0 && channels > 0 && (!gated || !out || !aligned16(gated) || !aligned16(out)))
     return fail(CUMM_HIP_EINVAL, "gated, grad and out must be 16-byte aligned and not empty");
   const bool gate = rows > 0;      // (no rows, nothing to gate: the tensors may have no memory)
-  return column_sum_checked({gate ? gated : nullptr, sums, grad, gate ? out : nullptr, rows, channels, workspace, workspace_bytes}, dtype, stream);
+  return column_sum_checked({gate ? gated : nullptr, sums, grad, gate ? out : nullptr, rows, channels, workspace, workspace_bytes, nullptr, nullptr},
+                            dtype, stream);
 }
 
 int cumm_hip_copy_kernel(void *dst, const void *src, size_t bytes, void *stream) {

@@ -99,6 +99,21 @@ __device__ __forceinline__ v4i round8(const float (&t)[8]) {
   return v;
 }
 
+// One bit per result of a ReLU, +0 or positive: which of eight packed two-byte results are not zero.  (The minimum
+// is an asm statement because the compiler, which knows where the halves come from, makes a test for classes of
+// floating-point numbers out of it: 300 instructions for 9.)
+__device__ __forceinline__ uint32_t positive8(const v4i &v) {
+  uint32_t bits = 0;
+#pragma unroll
+  for (int x = 0; x < 4; ++x) {
+    const int two = v[x];
+    uint32_t one;
+    asm("v_pk_min_u16 %0, %1, %2" : "=v"(one) : "v"(two), "s"(0x00010001u));
+    bits |= one << (2 * x);
+  }
+  return (bits | bits >> 15) & 0xFFu;      // (low halves in bits 0, 2, 4, 6, high ones in 16, 18, ...)
+}
+
 // activations: UnaryActivation, cumm/gemm/gemmmath/__init__.py:181-214 of the reference
 __device__ __forceinline__ float apply_act(float x, int act, float act_alpha) {
   switch (act) {

@@ -204,12 +204,16 @@ struct FinishRowsParams {
   int32_t act;
 };
 hipError_t launch_finish_rows(const FinishRowsParams &p, bool bf16, hipStream_t s);
+// RowGemmParams::gate out of the output rows (two-byte elements, not negative) of n positions
+hipError_t launch_gate_bits(uint8_t *gate, const void *out, const int32_t *order, int n, int channels, hipStream_t s);
 hipError_t launch_relu_backward(void *dst, const void *grad, const void *out, size_t vecs, bool bf16, hipStream_t s);
 struct ColumnSumParams {
   void *dst;            // [channels]
   const void *src;      // [rows, channels]
-  const void *out;      // [rows, channels] forward output whose positive elements let src through,
-  void *gated;          // and the gated rows; NULL both: plain sums
+  const void *out;      // [rows, channels] forward output whose positive elements let src through, or
+  const uint8_t *gate;  // a bit for each of them by position (RowGemmParams::gate) and
+  const int32_t *order; // [rows] the row of a position;
+  void *gated;          // and the gated rows; NULL all: plain sums
   float *partial;       // [blocks, channels] fp32
   int64_t rows, rows_per_block;
   int32_t channels, blocks;

@@ -75,6 +75,10 @@ struct RowGemmParams {
   // rows are gated by their pair-table entry alone, cumm/conv/sparse_iters.py:629-631), instead of
   // only in the offsets whose bit its own mask word has
   int32_t ungated_rows;
+  // a ReLU layer that will be differentiated, or NULL: a bit for every positive result, by position:
+  // gate[((c / 64) * n_pos + pos) * 8 + c % 64 / 8], bit c % 8
+  uint8_t *gate;
+  uint32_t gate_bytes;
   // non-zero: the output rows are stored with the non-temporal hint (see kStreamStore)
   int32_t stream_stores;
   // non-zero (descriptors with num_stage 3): a contraction of more than 128 bytes is walked in
@@ -115,6 +119,47 @@ __device__ __forceinline__ void store_out_b64(V v, __amdgpu_buffer_rsrc_t rs, ui
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00020000);
+}
+
+// The gate's bits of channels [ch, ch + 8 NG) of a position, from their packed results (channels past the end are
+// zeros).  By position, so that a tile writes whole cache lines (scattered like the output rows, 16 bytes of each, they
+// took 12 us more at 1 M rows of 128 channels).  That launch takes 218 us with the bits, 212 without.
+// The four lanes of a position (16 apart) put their bytes together, for one store of 4 or 8 bytes.
+template <int NG>
+__device__ __forceinline__ void store_gate(const v4i (&outs)[NG], const RowGemmParams &p, bool ok, int pos, int ch) {
+  static_assert(NG == 1 || NG == 2, "a byte, or two");
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc(p.gate, p.gate_bytes);
+  uint32_t v = positive8(outs[0]);
+  if constexpr (NG == 2) v |= positive8(outs[NG - 1]) << 8;
+  // (rows of 16 lanes: {0, 0, 2, 2} and {1, 1, 3, 3}, then {01, 01} and {23, 23})
+  const auto s16 = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  const uint32_t pair = s16[0] | s16[1] << (8 * NG);
+  const auto s32 = __builtin_amdgcn_permlane32_swap(pair, pair, false, false);
+  // (of the first of the four lanes: its channels are the lowest, and below k_out if any are)
+  const uint32_t at = ok && ch < p.k_out && (threadIdx.x & 48) == 0 ? ((uint32_t)(ch >> 6) * (uint32_t)p.n_pos + (uint32_t)pos) * 8u + (uint32_t)((ch & 63) >> 3) : kOob;
+  if constexpr (NG == 2) {
+    typedef int v2i __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b64(v2i{(int)s32[0], (int)s32[1]}, rs, at, 0, 0);
+  } else {
+    __builtin_amdgcn_raw_buffer_store_b32((int)(s32[0] | s32[1] << 16), rs, at, 0, 0);
+  }
+}
+
+// The same for the four row blocks of a wave with 16 channels per lane, positions pos0 + 16 rb + lane % 16: the 4 x 4
+// pieces of two bytes change places among the lanes of a position, and one store takes 64 positions.
+template <int N>
+__device__ __forceinline__ void store_gate4(const uint32_t (&bits)[N], const RowGemmParams &p, const bool (&ok)[N], int pos0, int ch) {
+  constexpr int B1 = 1 % N, B2 = 2 % N, B3 = 3 % N;      // (named with fewer blocks too, where it is not called)
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc(p.gate, p.gate_bytes);
+  const uint32_t lane = threadIdx.x & 63u, block = lane >> 4;      // the row block that this lane stores
+  const auto s32 = __builtin_amdgcn_permlane32_swap(bits[0] | bits[B1] << 16, bits[B2] | bits[B3] << 16, false, false);
+  const auto lo = __builtin_amdgcn_permlane16_swap(s32[0], s32[0], false, false), hi = __builtin_amdgcn_permlane16_swap(s32[1], s32[1], false, false);
+  const uint32_t half = (block & 1u) ? 0x07060302u : 0x05040100u;
+  // (rows and channels past the end lie past the end of the plane's positions or in bytes that nobody reads)
+  const bool mine = block == 0 ? ok[0] : (block == 1 ? ok[B1] : (block == 2 ? ok[B2] : ok[B3]));
+  const uint32_t at = mine ? ((uint32_t)(ch >> 6) * (uint32_t)p.n_pos + (uint32_t)(pos0 + (int)lane)) * 8u : kOob;
+  typedef int v2i __attribute__((ext_vector_type(2)));
+  __builtin_amdgcn_raw_buffer_store_b64(v2i{(int)__builtin_amdgcn_perm(lo[1], lo[0], half), (int)__builtin_amdgcn_perm(hi[1], hi[0], half)}, rs, at, 0, 0);
 }
 
 // Four-byte outputs (s32 for s8 operands, f32 for f16 / bf16 operands; "s8,s8,s32,s32,s32" in

@@ -106,6 +106,9 @@ static bool launch_two_groups(const RowGemmParams &p, dim3 grid, hipStream_t s, 
 }
 
 template <class T, int NW, int RB, int TN, int KS, bool WT>
+static hipError_t launch_fallback(const RowGemmParams &p, dim3 grid, hipStream_t s);
+
+template <class T, int NW, int RB, int TN, int KS, bool WT>
 static hipError_t launch_one(const RowGemmParams &p, hipStream_t s) {
   constexpr int TM = NW * RB * 16;
   dim3 grid((p.n_pos + TM - 1) / TM, (p.k_out + TN - 1) / TN, 1);
@@ -195,6 +198,15 @@ static hipError_t launch_one(const RowGemmParams &p, hipStream_t s) {
       }
     }
   }
+  err = launch_fallback<T, NW, RB, TN, KS, WT>(p, grid, s);
+  if (err != hipSuccess || p.gate == nullptr) return err;
+  return launch_gate_bits(p.gate, p.C, p.out_rows, p.n_pos, p.k_out, s);      // (these kernels leave none)
+}
+
+// kernels whose waits the compiler counts
+template <class T, int NW, int RB, int TN, int KS, bool WT>
+static hipError_t launch_fallback(const RowGemmParams &p, dim3 grid, hipStream_t s) {
+  constexpr int chunk_e = 4 * KS * Elem<T>::kPerVec;
   if (p.c_in <= chunk_e) {
     constexpr int BW = step_width(TN, KS);
     constexpr int DA = rows_ahead(RB, KS, BW);

@@ -729,6 +729,9 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
     constexpr bool SRC = (MODE & 1) != 0;
     if constexpr (E::kBytes == 2) {
       constexpr int NG = CPLW / 8;   // 16-byte groups
+      constexpr bool GATE4 = ACT == 1 && NG == 2 && RBW == 4 && WK == 1;
+      uint32_t gate_bits[RBW];
+      bool gate_ok[RBW];
       float shared[MODE == 4 ? CPLW : 1];
       if constexpr (MODE == 4) {
 #pragma unroll
@@ -744,6 +747,7 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
         if (!mine(rb)) continue;
         const int o = out_row[rb];
         const bool row_ok = o >= 0 && o < p.rows_c;
+        v4i outs[NG];
 #pragma unroll
         for (int g = 0; g < NG; ++g) {
           const int ch = ch0 + g * 8;
@@ -762,7 +766,19 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
           }
           const v4i outv = round8<T, ACT == 1>(t);      // (a ReLU lets no NaN through)
           store_out_b128(outv, rs_c, coff, p.stream_stores != 0);
+          outs[g] = outv;
         }
+        if constexpr (ACT == 1) {
+          if constexpr (GATE4) {
+            gate_ok[rb] = row_ok;
+            gate_bits[rb] = p.gate != nullptr ? positive8(outs[0]) | positive8(outs[NG - 1]) << 8 : 0u;
+          } else if (p.gate != nullptr) {
+            store_gate(outs, p, row_ok, pos_base + (wm * RBW + rb) * 16 + m, ch0);
+          }
+        }
+      }
+      if constexpr (GATE4) {
+        if (p.gate != nullptr && n0 + wn * 64 < p.k_out) store_gate4(gate_bits, p, gate_ok, pos_base + wm * 64, n0 + wn * 64);
       }
     } else {
       // one-byte outputs: the lane's 4*NBW consecutive channels are 8 or 16 bytes of the row.

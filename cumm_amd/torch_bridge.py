@@ -167,7 +167,7 @@ def _copy(args: _capi.SparseConvArgs) -> _capi.SparseConvArgs:
 _KINDS = {}
 
 
-_NATIVE_SYMBOLS = ("sparse_conv", "sparse_conv_more", "last_error", "relu_backward", "relu_backward_sums", "column_sum", "column_sum_workspace",
+_NATIVE_SYMBOLS = ("sparse_conv_more", "last_error", "relu_backward", "gate_sums", "column_sum_workspace",
                    "query_conv_workspace", "query_wgrad_ordered_workspace", "wgrad_pairs_sums", "wgrad_pairs_workspace", "subm_pairs",
                    "subm_pairs_workspace", "conv_pairs_workspace", "conv_pairs_sites", "conv_pairs_fill", "order_pairs_coarse",
                    "order_pairs_coarse_workspace")

@@ -164,8 +164,8 @@ typedef struct CummHipSparseConvArgs {
 } CummHipSparseConvArgs;
 
 /* The bias gradient of a layer, and the gate of its fused ReLU in front of both: gated = grad where out > 0, else 0, and
- * sums[c] = the sum of column c of gated.  gated and out NULL: sums of grad itself.  As cumm_hip_relu_backward_sums /
- * cumm_hip_column_sum, whose rules for the operands and the workspace hold. */
+ * sums[c] = the sum of column c of gated.  gated, out and gate NULL: sums of grad itself.  As
+ * cumm_hip_relu_backward_sums / cumm_hip_column_sum, whose rules for the operands and the workspace hold. */
 typedef struct CummHipGateSums {
   void *gated;                      /* [rows, channels] */
   void *sums;                       /* [channels] */
@@ -174,6 +174,8 @@ typedef struct CummHipGateSums {
   int32_t channels;
   void *workspace;                  /* cumm_hip_column_sum_workspace bytes, not shared with the call's own */
   size_t workspace_bytes;
+  const void *gate;                 /* instead of out: what the forward call left (CummHipSparseConvMore::gate), */
+  const int32_t *order;             /* and its mask_argsort_ptr: [rows], every row once */
 } CummHipGateSums;
 
 /* What a training program wants of the same launches beyond the reference's argument block; all zero = nothing. */
@@ -186,6 +188,9 @@ typedef struct CummHipSparseConvMore {
                                        (cumm_hip_order_pairs, cumm_hip_pairs_by_position): [kernel_volume, N], column = sorted
                                        position; one of cumm_hip_order_pairs_coarse with a mask_width of 64 or 128.  Kernels
                                        that can read it instead do */
+  void *gate;                       /* forward with ReLU, f16 / bf16 output, NULL = none: a bit for every positive result, by
+                                       position: ceil(K / 64) * N * 8 bytes, channel c of position pos is bit c % 8 of byte
+                                       ((c / 64) * N + pos) * 8 + c % 64 / 8 */
 } CummHipSparseConvMore;
 
 /* Replaces GemmMainUnitTest.matmul2 below its prelude
@@ -504,6 +509,7 @@ int cumm_hip_column_sum(void *dst, const void *src, int64_t rows, int channels, 
 /* Both at once, reading grad once: gated [rows, channels] = grad where out is positive, else 0, and sums
  * [channels] = the column sums of gated (the input gradient's gate and the bias gradient of a layer with a
  * fused ReLU); the same results as the two calls, workspace as cumm_hip_column_sum. */
+int cumm_hip_gate_sums(const CummHipGateSums *g, int dtype, void *stream);
 int cumm_hip_relu_backward_sums(void *gated, void *sums, const void *grad, const void *out, int64_t rows, int channels,
                                 int dtype, void *workspace, size_t workspace_bytes, void *stream);
 

@@ -173,3 +173,58 @@ def test_gate_and_sums_are_of_the_gradient_of_the_call():
         ConvMainUnitTest.implicit_gemm2(p)
         with pytest.raises(ValueError):
             _again(p, sums=ctypes.addressof(gs))
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("ksize,cin,k_out,tile,n,hint", [
+    (3, 64, 64, (64, 64), 40000, 0), (3, 64, 64, (64, 64), 40000, -1),     # tile shapes mixed, and one
+    (3, 16, 24, (64, 64), 700, 0), (3, 64, 8, (64, 64), 700, 0),            # two groups of waves; one byte a position
+    (3, 64, 72, (128, 64), 700, 0), (3, 64, 136, (64, 128), 700, 0),        # a last group of one byte
+    (3, 64, 256, (128, 128), 700, 0), (3, 136, 128, (128, 128), 700, 0),
+    (5, 32, 40, (64, 64), 700, 0), (5, 32, 128, (128, 128), 700, 0),        # several mask words
+    (3, 520, 64, (64, 64), 700, 0),                                         # kernels that leave the gate to another one
+])
+def test_gate_of_a_forward_pass(dtype, ksize, cin, k_out, tile, n, hint):
+    """The bits that a ReLU layer leaves are those of its output; a gradient gated by them is what the output gives, its
+    sums (of whole numbers, exact in any order) too."""
+    print("case gate", dtype, ksize, cin, k_out, tile, n, hint, flush=True)
+    rng, lib = np.random.default_rng(k_out), _capi.lib()
+    coords, grid = H.small_cloud(5, n, grid=(20, 90, 90), clusters=12, sigma=6.0)
+    n, kv = coords.shape[0], ksize ** 3
+    table = pairs.subm_pairs_device(H.dev(coords, "i32"), grid, (ksize,) * 3)
+    p = ConvParams(3, ConvOpType.Forward)
+    if kv > 32:
+        p.conv_algo_desp = H.find_conv_desp(dtype, ConvOpType.Forward, *tile, dynamic_mask=True)
+        p.mask, p.mask_argsort = pairs.sort_by_mask_words_device(pairs.masks_from_pairs_device(table.indices_fwd))
+        p.mask_int_count = (kv + 31) // 32
+    else:
+        p.conv_algo_desp = H.find_conv_desp(dtype, ConvOpType.Forward, *tile)
+        p.mask, p.mask_argsort = pairs.sort_by_mask_device(table.mask_fwd, (1 << kv) - 1, by_offset_count=True)
+    p.input = H.dev(H.to_storage(rng.normal(0, 1, size=(n, cin)).astype(np.float32), dtype), dtype)
+    p.weight = H.dev(H.to_storage(rng.normal(0, 0.05, size=(k_out, kv, cin)).astype(np.float32), dtype), dtype)
+    p.output, p.bias, p.beta = tv.zeros([n, k_out], H.TV_DTYPE[dtype], 0), H.dev(H.to_storage(rng.normal(0, 0.3, size=k_out).astype(np.float32), dtype), dtype), 1.0
+    p.act_type, p.indices, p.light_prefix = Activation.ReLU, table.indices_fwd, hint
+    ConvMainUnitTest.implicit_gemm2(p)
+    before, groups = H.host(p.output).copy(), (k_out + 63) // 64
+    d_gate = tv.from_numpy(np.full((groups, n, 8), 0xA5, np.uint8)).cuda()
+    _again(p, gate=d_gate.byte_pointer())
+    out, order = H.host(p.output), H.host(p.mask_argsort)
+    np.testing.assert_array_equal(out.view(np.uint16), before.view(np.uint16))
+    want = np.packbits(H.as_f32(out, dtype)[order] > 0, axis=1, bitorder="little")      # [n, k_out / 8]
+    got = H.host(d_gate).transpose(1, 0, 2).reshape(n, groups * 8)[:, :k_out // 8]
+    np.testing.assert_array_equal(got, want)
+
+    need = int(lib.cumm_hip_column_sum_workspace(n, k_out))
+    grad = rng.integers(-2, 3, size=(n, k_out)).astype(np.float32)
+    d_grad, ws = H.dev(H.to_storage(grad, dtype), dtype), tv.zeros([need], tv.uint8, 0)
+    both = []
+    for source in ({"out": p.output.byte_pointer()}, {"gate": d_gate.byte_pointer(), "order": p.mask_argsort.byte_pointer()}):
+        gated, sums = tv.zeros([n, k_out], H.TV_DTYPE[dtype], 0), tv.zeros([k_out], H.TV_DTYPE[dtype], 0)
+        gs = _capi.GateSums(gated=gated.byte_pointer(), sums=sums.byte_pointer(), grad=d_grad.byte_pointer(), rows=n, channels=k_out,
+                            workspace=ws.byte_pointer(), workspace_bytes=need, **source)
+        _capi.check(lib.cumm_hip_gate_sums(ctypes.byref(gs), int(H.TV_DTYPE[dtype]), None))
+        _capi.check(lib.cumm_hip_device_synchronize())
+        both.append((H.host(gated).view(np.uint16), H.host(sums).view(np.uint16)))
+    np.testing.assert_array_equal(both[0][0], both[1][0])
+    np.testing.assert_array_equal(both[0][1], both[1][1])
+    np.testing.assert_array_equal(both[0][0] != 0, (H.as_f32(out, dtype) > 0) & (grad != 0))
