@@ -86,6 +86,7 @@ struct RowGemmParams {
   int32_t small_stages;
   // two groups of waves per tile: bit k of word k / 32 set = offset k belongs to the first group
   uint32_t first_group[4];
+  uint32_t even_group[4];      // with four: those of the first and third (first_group: of the first two)
   // non-zero: every row's sum in the one order that all tiles share
   int32_t one_order;
 };

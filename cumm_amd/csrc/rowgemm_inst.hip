@@ -55,18 +55,20 @@ constexpr int lds_stages(int TM, int TN, int KS) {
 template <class T, int TM, int TN>
 constexpr bool has_mask_words_kernel() { return Elem<T>::kBytes == 2 && !kWide && TM == TN; }
 
-// The offsets of the first of two groups.  Fixed by their numbers, so that a row's sum is the same in whatever
+// The offsets of the first of two groups (of the first two of four; and those of the first and third, by the
+// parity of the sum of the indices: 7, 7, 7 and 6 of 27 offsets, 32 and three times 31 of 125).  Fixed by their numbers, so that a row's sum is the same in whatever
 // order the positions lie; halved on the sets that tiles have: all offsets of a dense neighbourhood, and in
 // the backward-input pass of a strided layer, per axis, the even or the odd indices.  The parity of the sum of
 // the halved indices does that for square and cubic kernels (strided 128 -> 128 backward-input 10.1 us, by the
 // parity of the number 12.2); other volumes go by the parity of the number.
-static void first_group_offsets(int kv, uint32_t (&words)[4]) {
+static void first_group_offsets(int kv, uint32_t (&words)[4], uint32_t (&even)[4]) {
   int side = 2, dims = 0;
   for (; side * side <= kv && dims == 0; ++side)
     for (int d = 2, v = side * side; d <= 3 && v <= kv; ++d, v *= side)
       if (v == kv) dims = d;
   --side;      // (the loop leaves one past)
   for (uint32_t &w : words) w = 0;
+  for (uint32_t &w : even) w = 0;
   for (int k = 0; k < kv && k < 128; ++k) {
     int sum = k;
     if (dims > 0) {
@@ -74,6 +76,12 @@ static void first_group_offsets(int kv, uint32_t (&words)[4]) {
       for (int d = 0, rest = k; d < dims; ++d, rest /= side) sum += (rest % side) >> 1;
     }
     if ((sum & 1) == 0) words[k / 32] |= 1u << (k % 32);
+    int bits = k >> 1;
+    if (dims > 0) {
+      bits = 0;
+      for (int d = 0, rest = k; d < dims; ++d, rest /= side) bits += rest % side;
+    }
+    if ((bits & 1) == 0) even[k / 32] |= 1u << (k % 32);
   }
 }
 
@@ -90,6 +98,12 @@ static void first_group_offsets(int kv, uint32_t (&words)[4]) {
 //   several steps per offset  1024   128 -> 128 channels, 500 workgroups 21.7 / 18.2, 1000 22.3 / 19.6, 2750 23.8 / 34.5
 //   several mask words        1024   5 x 5 x 5, 64 channels, 125 workgroups 62.6 / 44.3, 469 62.1 / 45.3, 938 62.2 / 53.8,
 //                                    1875 66.1 / 69.9
+// Four groups where the device is emptier still: a quarter of the offsets each, one workgroup per CU (136 KB), all
+// sixteen waves of it on four SIMDs, so that a step takes longer; chains of many steps gain.  f16 forward, us, by
+// workgroups, two / four groups; rows of 64 bytes and one step per offset (16 channels) gain nothing:
+//   64 channels       32 9.8 / 9.5, 125 10.0 / 9.7, 250 10.2 / 10.0, 375 10.7 / 10.3
+//   128 -> 128        64 15.8 / 14.3, 250 16.3 / 14.8, 376 16.7 / 15.0, 500 17.0 / 16.9, 750 17.5 / 22.1
+//   5 x 5 x 5         32 33.8 / 29.7, 250 34.0 / 30.7, 500 37.4 / 32.9, 938 46.4 / 56.1; 32 channels: 32 25.5 / 21.8, 375 26.9 / 22.6
 template <class T, int TM, int TN, int KS, bool WT, int MW>
 static bool launch_two_groups(const RowGemmParams &p, dim3 grid, hipStream_t s, hipError_t *err) {
   if constexpr (TM == 64 && TN == 64 && KS <= 2 && !kWide && (!WT || Elem<T>::kBytes == 2)) {
@@ -97,7 +111,13 @@ static bool launch_two_groups(const RowGemmParams &p, dim3 grid, hipStream_t s, 
     if (p.mask == nullptr || p.one_order || (uint64_t)grid.x * grid.y > most) return false;
     if (!counted_waits_hold<rowgemm_lds_kernel<T, 2, 2, 2, 2, KS, 2, WT, false, MW, 2>>()) return false;
     RowGemmParams q = p;
-    first_group_offsets(p.kv, q.first_group);
+    first_group_offsets(p.kv, q.first_group, q.even_group);
+    const unsigned four = MW > 1 ? 512u : (KS == 2 ? 384u : 0u);
+    if ((uint64_t)grid.x * grid.y <= four && counted_waits_hold<rowgemm_lds_kernel<T, 2, 2, 2, 2, KS, 2, WT, false, MW, 4>>()) {
+      hipLaunchKernelGGL((rowgemm_lds_kernel<T, 2, 2, 2, 2, KS, 2, WT, false, MW, 4>), grid, dim3(1024), 0, s, q);
+      *err = hipGetLastError();
+      return true;
+    }
     hipLaunchKernelGGL((rowgemm_lds_kernel<T, 2, 2, 2, 2, KS, 2, WT, false, MW, 2>), grid, dim3(512), 0, s, q);
     *err = hipGetLastError();
     return true;

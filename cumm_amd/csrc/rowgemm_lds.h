@@ -62,6 +62,7 @@ struct LdsRing {
   v4i *weights[4];
   int (*idx[4])[64];
   v4i *park;      // WK groups: where they leave sums for each other (a stage of every group)
+  v4i *park1 = nullptr;      // (four groups)
 };
 
 // One tile: rows [tile * TM, tile * TM + TM) of the sorted positions, column block col.
@@ -77,7 +78,7 @@ struct LdsRing {
 // WK: groups of WM x WN waves that share the tile.  With two, the first takes the kernel offsets of
 // p.first_group and the second the others (whatever the tile's list: a row's sum does not depend on its
 // neighbours), each with a ring of its own, and at the end they add up their sums in LDS, each of them for
-// half of the row blocks.
+// half of the row blocks.  Four: by p.even_group too; the first two finish a row block each.
 template <class T, int WM, int WN, int RBW, int NBW, int KS, int NS, bool WT, bool WIDE, bool HALVES, int MW = 1, bool HALF32 = false, int WK = 1>
 __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const int tile, const int col, const LdsRing &lds) {
   static_assert(MW == 1 || MW == 4, "one mask word, or up to four");
@@ -345,6 +346,26 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
     n_offsets = 0;
 #pragma unroll
     for (int w = 0; w < MW; ++w) n_offsets += __builtin_popcount(kwords[w]);
+  }
+  if constexpr (WK == 4) {      // this group's offsets; the barriers of all are the longest list's
+    int most = 0;
+    uint32_t own[MW];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      int count = 0;
+#pragma unroll
+      for (int w = 0; w < MW; ++w) {
+        const uint32_t theirs = (MW == 1 ? kmask : kwords[w]) & (g < 2 ? p.first_group[w] : ~p.first_group[w]) &
+                                (g % 2 == 0 ? p.even_group[w] : ~p.even_group[w]);
+        if (g == group) own[w] = theirs;
+        count += __builtin_popcount(theirs);
+      }
+      most = count > most ? count : most;
+    }
+    kmask = own[0];
+#pragma unroll
+    for (int w = 0; w < MW; ++w) kwords[w] = own[w];
+    n_offsets = most;
   }
   if constexpr (WK == 2) {      // this group's offsets; the barriers of both are the longer list's
     int first = __builtin_popcount(kmask & p.first_group[0]);
@@ -676,7 +697,32 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
   for (int rb = 0; rb < RBW; ++rb)
 #pragma unroll
     for (int i = 0; i < SRC_N; ++i) keep_after_wait(src_pre[rb][i]);
-  if constexpr (WK > 1) {
+  if constexpr (WK == 4) {
+    static_assert(WK != 4 || (RBW == 2 && !HALVES && !HALF32), "the first two of four groups finish a row block each");
+    __builtin_amdgcn_s_waitcnt(0xC07F);   // (as below)
+    lds_barrier();
+    AccV *park[2] = {reinterpret_cast<AccV *>(lds.park), reinterpret_cast<AccV *>(lds.park1)};      // [group][wave][block]
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+      if (group != r) {
+#pragma unroll
+        for (int nb = 0; nb < NBW; ++nb) park[r][(wave_of_all * NBW + nb) * 64 + lane] = acc[r][nb];
+      }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+      if (group == r) {
+#pragma unroll
+        for (int nb = 0; nb < NBW; ++nb) {
+          AccV sum = r == 0 ? acc[r][nb] : park[r][(wave * NBW + nb) * 64 + lane];
+#pragma unroll
+          for (int g = 1; g < 4; ++g) sum = sum + (g == r ? acc[r][nb] : park[r][((g * NW + wave) * NBW + nb) * 64 + lane]);
+          acc[r][nb] = sum;
+        }
+      }
+    if (group > 1) return;
+  }
+  if constexpr (WK == 2) {
     static_assert(WK == 2 && RBW % 2 == 0 && !HALVES && !HALF32, "two groups, half of the row blocks each");
     constexpr int RO = RBW / 2;
     __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): this wave has read its last stage,
@@ -696,7 +742,7 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
         else acc[RO + r][nb] = other + acc[RO + r][nb];
       }
   }
-  auto mine = [&](int rb) __attribute__((always_inline)) -> bool { return WK == 1 || rb / (RBW / WK) == group; };
+  auto mine = [&](int rb) __attribute__((always_inline)) -> bool { return WK == 1 || (WK == 4 ? rb == group : rb / (RBW / (WK == 2 ? 2 : 1)) == group); };
   // (a 64-row tile without any offset is left alone when exit_on_empty is set: so is that half)
   if (HALVES && half_skipped) return;
   // ---- epilogue: lane (q, m) holds, for each of its rows, channels ch0 .. ch0 + 4*NBW - 1.
@@ -854,13 +900,13 @@ __global__ __launch_bounds__(WM *WN *WK * 64) void rowgemm_lds_kernel(const RowG
   __shared__ int ix1[WK * NW][64];
   __shared__ int ix2[NS > 2 ? WK * NW : 1][64];
   __shared__ int ix3[NS > 3 ? WK * NW : 1][64];
-  static_assert(WK == 1 || STAGE_V >= NW * (RBW / 2 * NBW) * 64, "a stage of every group holds the sums they exchange");
+  static_assert(WK == 1 || STAGE_V >= NW * (RBW / 2 * NBW) * 64, "a stage of every group holds the sums they exchange (of four: of a row block)");
   const int group = WK == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) / NW;
   const int gs = group * STAGE_V, gi = group * NW;
   const LdsRing lds = {{st0 + gs, st1 + gs, NS > 2 ? st2 + gs : st2, NS > 3 ? st3 + gs : st3},
                        {st0 + gs + A_V, st1 + gs + A_V, NS > 2 ? st2 + gs + A_V : st2, NS > 3 ? st3 + gs + A_V : st3},
                        {ix0 + gi, ix1 + gi, NS > 2 ? ix2 + gi : ix2, NS > 3 ? ix3 + gi : ix3},
-                       st0};
+                       st0, st1};
 
   // Workgroups are dispatched in the order of their linear number, round-robin over the 8 XCDs.
   // With several column blocks per row tile, the workgroups of one row tile are given numbers 8

@@ -126,3 +126,11 @@ def test_one_order_on_request(monkeypatch, op, dtype, kv, c, k):
     assert torch.equal(alone[0][present], alone[1][present])
     for b in batch:
         assert all(torch.equal(b[i][present], alone[0][present]) for i in range(copies))
+
+
+@pytest.mark.parametrize("op", [ConvOpType.Forward, ConvOpType.BackwardInput])
+@pytest.mark.parametrize("dtype,kv,c,k,n,which", [
+    ("f16", 27, 136, 64, 64 * 384, "all"), ("f16", 27, 136, 64, 64 * 384 + 1, "all"), ("bf16", 32, 40, 72, 64 * 192, "all"),
+    ("f16", 125, 32, 64, 64 * 512, "all"), ("bf16", 125, 64, 64, 64 * 512 + 1, "even"), ("bf16", 36, 16, 8, 1, "all")])
+def test_sides_of_the_line_of_four_groups(op, dtype, kv, c, k, n, which):
+    test_against_the_sum_over_the_table(op, dtype, kv, c, k, n, which)
