@@ -245,7 +245,8 @@ hipError_t CUMM_CAT(launch_wgrad_atomic_, CUMM_NAME)(const WgradParams &p, const
   }
   e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((wgrad_finalize_kernel<T>), dim3((unsigned)((f.total / 4 + 255) / 256) + last.groups), dim3(256), 0, s, f, last);
+  if (last.groups > 0) hipLaunchKernelGGL((wgrad_finalize_kernel<T, true>), dim3((unsigned)((f.total / 4 + 255) / 256) + last.groups), dim3(256), 0, s, f, last);
+  else hipLaunchKernelGGL((wgrad_finalize_kernel<T, false>), dim3((unsigned)((f.total / 4 + 255) / 256) + last.groups), dim3(256), 0, s, f, last);
   return hipGetLastError();
 }
 
@@ -281,7 +282,8 @@ hipError_t CUMM_CAT(launch_wgrad_ordered_, CUMM_NAME)(const WgradParams &p, cons
   launch_units<T, true>(wide, p, dim3(wgs), s);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((wgrad_finalize_ordered_kernel<T>), dim3((unsigned)((f.total / 4 + 31) / 32) + last.groups), dim3(256), 0, s, f, last);
+  if (last.groups > 0) hipLaunchKernelGGL((wgrad_finalize_ordered_kernel<T, true>), dim3((unsigned)((f.total / 4 + 31) / 32) + last.groups), dim3(256), 0, s, f, last);
+  else hipLaunchKernelGGL((wgrad_finalize_ordered_kernel<T, false>), dim3((unsigned)((f.total / 4 + 31) / 32) + last.groups), dim3(256), 0, s, f, last);
   return hipGetLastError();
 }
 #endif

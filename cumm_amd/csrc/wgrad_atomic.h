@@ -686,14 +686,17 @@ struct WgradFinalizeParams {
 // dW = cvt(alpha * sum of the scratch images + beta * src) for the offsets enabled in mask_filter
 // Four consecutive elements per thread (C is a multiple of 8, so they share their offset).  The first workgroups
 // finish the bias sums of the same backward pass, if there are any: a launch of its own is 4.7 us.
-template <class T>
+template <class T, bool SUMS>
 __global__ __launch_bounds__(256) void wgrad_finalize_kernel(const WgradFinalizeParams p, const ColumnFinalParams sums) {
   using E = Elem<T>;
-  if ((int)blockIdx.x < sums.groups) {
-    column_final<T>(sums, blockIdx.x);
-    return;
+  int64_t block = blockIdx.x;
+  if constexpr (SUMS) {
+    if ((int)blockIdx.x < sums.groups) {
+      column_final<T>(sums, blockIdx.x);
+      return;
+    }
+    block -= sums.groups;
   }
-  const int64_t block = blockIdx.x - sums.groups;
   const int64_t i = (block * 256 + threadIdx.x) * 4;
   if (i >= p.total) return;
   const int r = (int)((i / p.C) % p.kv);
@@ -742,14 +745,17 @@ struct WgradOrderedParams {
   uint32_t slots_bytes;
 };
 
-template <class T>
+template <class T, bool SUMS>
 __global__ __launch_bounds__(256) void wgrad_finalize_ordered_kernel(const WgradOrderedParams p, const ColumnFinalParams sums) {
   using E = Elem<T>;
-  if ((int)blockIdx.x < sums.groups) {
-    column_final<T>(sums, blockIdx.x);
-    return;
+  int64_t block = blockIdx.x;
+  if constexpr (SUMS) {
+    if ((int)blockIdx.x < sums.groups) {
+      column_final<T>(sums, blockIdx.x);
+      return;
+    }
+    block -= sums.groups;
   }
-  const int64_t block = blockIdx.x - sums.groups;
   const int g = threadIdx.x & 7;
   const int64_t i = (block * 32 + (threadIdx.x >> 3)) * 4;
   const bool in_range = i < p.total;
