@@ -810,7 +810,8 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
             else t[x] = SRC ? __builtin_fmaf(p.alpha, a, p.beta * E::to_float(sh[x])) : p.alpha * a;
             t[x] = apply_act(t[x], ACT, p.act_alpha);
           }
-          const v4i outv = round8<T, ACT == 1>(t);      // (a ReLU lets no NaN through)
+          // (a ReLU lets no NaN through; an f16 sum that nothing follows is rounded by the fma itself)
+          const v4i outv = round8<T, ACT == 1, std::is_same_v<T, F16> && ACT == 0 && (SRC || MODE == 4)>(t);
           store_out_b128(outv, rs_c, coff, p.stream_stores != 0);
           outs[g] = outv;
         }
