@@ -243,6 +243,7 @@ class SparseConvGeometry:
     _TABLES = ("indices_fwd", "indices_bwd", "mask_fwd", "order_fwd", "mask_bwd", "order_bwd", "indices_fwd_pos", "indices_bwd_pos")
     _lists = _list_block = None      # (several mask words only)
     _partial = frozenset()           # tables by position that are written only where the launches read them
+    _recorded = False                # built while its stream was recorded: every replay writes the tables anew
     _native = None                   # the geometry as native code has it
 
     def __init__(self, coords: torch.Tensor, spatial_shape: Sequence[int], ksize=(3, 3, 3), stride=None,
@@ -277,6 +278,7 @@ class SparseConvGeometry:
         # memory); backward-weight keeps the table by row
         if ordered:
             self._partial = frozenset(("indices_fwd_pos", "indices_bwd_pos"))
+            self._recorded = torch.cuda.is_current_stream_capturing()
         else:
             self._order_one_by_one()
         if words > 1:
@@ -421,16 +423,23 @@ class SparseConvGeometry:
 
     def _complete(self, name: str) -> None:
         """Whoever looks at a table by position gets all of it: the entries of runs without a pair are written too (the
-        others once more, as they are)."""
-        side, stream = name[8:11], current_stream()
+        others once more, as they are).  Behind the construction, whatever stream and device the reader is on: it
+        needs to be ordered behind that only when it uses the table, as for every other one.  Where a stream is being
+        recorded nothing waits: what is there before a graph, torch has waited for when it begins."""
+        side, lib = name[8:11], _capi.lib()
         n = self.n_out if side == "fwd" else self.n_in
-        if n:
-            self.used_on(stream)
-            _capi.check(_capi.lib().cumm_hip_pairs_by_position(self._ptr["indices_" + side], self._ptr["order_" + side], self.kv, n,
-                                                               self._ptr[name], stream))
-        if not torch.cuda.is_current_stream_capturing():
-            torch.cuda.current_stream().synchronize()      # (it may be read on any stream)
-            self._partial = self._partial - {name}
+        with torch.cuda.device(self._device):
+            stream, recorded = current_stream(), torch.cuda.is_current_stream_capturing()
+            if n:
+                if not recorded and stream != self._stream and not lib.cumm_hip_stream_is_capturing(self._stream):
+                    _capi.check(lib.cumm_hip_stream_synchronize(self._stream))
+                self.used_on(stream)
+                _capi.check(lib.cumm_hip_pairs_by_position(self._ptr["indices_" + side], self._ptr["order_" + side], self.kv, n,
+                                                           self._ptr[name], stream))
+            if not recorded:
+                torch.cuda.current_stream().synchronize()      # (it may be read on any stream)
+                if not self._recorded:
+                    self._partial = self._partial - {name}
 
     def _view(self, name: str) -> tv.Tensor:
         t = self._tensors.get(name)

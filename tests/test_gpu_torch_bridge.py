@@ -352,3 +352,44 @@ def test_tables_by_position_are_whole_for_who_looks(ksize, strided):
         table, order = H.host(getattr(geo, "indices_" + side)), H.host(getattr(geo, "order_" + side))
         np.testing.assert_array_equal(H.host(getattr(geo, "indices_%s_pos" % side)), pairs.pairs_by_position(table, order))
     assert torch.equal(before, tb.sparse_conv(x, w, None, geo))
+
+
+def test_tables_by_position_read_on_another_stream_than_the_building_one():
+    """The building stream is still busy when somebody on another one takes the tables, and is waited for only
+    afterwards; and a geometry that a graph builds anew at every replay."""
+    import torch
+    from cumm_amd import pairs, torch_bridge as tb
+    print("case whole tables, two streams", flush=True)
+    coords, grid = H.small_cloud(3, 30000, grid=(16, 200, 200))
+    coords = torch.as_tensor(coords, device="cuda")
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    busy = torch.randn(4096, 4096, device="cuda")
+
+    def whole(geo, tables):
+        for side, table in tables:
+            by_row, order = H.host(getattr(geo, "indices_" + side)), H.host(getattr(geo, "order_" + side))
+            np.testing.assert_array_equal(H.host(table), pairs.pairs_by_position(by_row, order))
+    torch.cuda.synchronize()
+    with torch.cuda.stream(a):
+        for _ in range(10):
+            busy @ busy
+        geo = tb.SparseConvGeometry(coords, grid)
+    with torch.cuda.stream(b):
+        tables = [(side, getattr(geo, "indices_%s_pos" % side)) for side in ("fwd", "bwd")]
+    b.wait_stream(a)
+    torch.cuda.synchronize()
+    whole(geo, tables)
+
+    # (the same number of sites, elsewhere: runs of positions have other offsets)
+    clouds = [coords] + [torch.as_tensor(H.small_cloud(s, 30000, grid=(16, 200, 200), sigma=30.0)[0], device="cuda") for s in (4, 5)]
+    n = min(len(c) for c in clouds)
+    clouds = [c[:n].contiguous() for c in clouds]
+    now = clouds[0].clone()
+    tb.SparseConvGeometry(now, grid)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        geo = tb.SparseConvGeometry(now, grid)
+    for cloud in clouds:
+        now.copy_(cloud)
+        graph.replay()
+        whole(geo, [(side, getattr(geo, "indices_%s_pos" % side)) for side in ("fwd", "bwd")])

@@ -189,6 +189,71 @@ def test_tables_that_were_handed_out_go_back_when_the_device_has_finished(monkey
     assert waits == []
 
 
+def test_a_table_by_position_is_completed_behind_the_construction(monkeypatch):
+    """Read on another stream than the one that builds it, with another device current: the building stream is waited
+    for, then the launch, on the geometry's device; not where either stream is being recorded.  A geometry that
+    was built while its stream was recorded is completed at every read."""
+    import contextlib
+    from cumm_amd import torch_bridge as tb
+    waited = []
+
+    def fresh(n=1000):
+        g, _, now = _geometry(monkeypatch, tb, n, stream=7)
+        monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: type("S", (), {"synchronize": lambda self: waited.append(now[0])})())
+        g._partial = frozenset(("indices_fwd_pos", "indices_bwd_pos"))
+        now[0] = 9
+        return g, now
+    device, here, building = [None], [False], [False]
+
+    @contextlib.contextmanager
+    def on(d):
+        device[0] = d
+        yield
+        device[0] = None
+    monkeypatch.setattr(torch.cuda, "device", on)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: here[0])
+    log, addresses = [], []
+
+    class Library:
+        def cumm_hip_stream_is_capturing(self, stream):
+            assert stream == 7
+            return building[0]
+
+        def cumm_hip_stream_synchronize(self, stream):
+            log.append(("wait", stream))
+            return 0
+
+        def cumm_hip_pairs_by_position(self, indices, order, kv, n, to, stream):
+            assert device[0] == torch.device("cpu")
+            addresses.append((indices, order, to))
+            log.append(("write", stream))
+            return 0
+    monkeypatch.setattr(_capi, "_lib", Library())
+    g, now = fresh()
+    want = tuple(g._ptr[name] for name in ("indices_fwd", "order_fwd", "indices_fwd_pos"))
+    for _ in range(2):      # (the second read finds it whole)
+        assert g.indices_fwd_pos.byte_pointer() == g._ptr["indices_fwd_pos"]
+        assert log == [("wait", 7), ("write", 9)] and waited == [9] and g._partial == {"indices_bwd_pos"}
+        assert addresses == [want]
+    del log[:], waited[:]
+    g, now = fresh()
+    now[0] = 7
+    g.indices_fwd_pos
+    assert log == [("write", 7)] and waited == [7]
+    for here[0], building[0], left in ((True, False, 2), (False, True, 1)):
+        del log[:], waited[:]
+        g, now = fresh()
+        g.indices_fwd_pos
+        assert log == [("write", 9)] and waited == ([] if here[0] else [9]) and len(g._partial) == left
+    building[0] = False
+    del log[:], waited[:]
+    g, now = fresh()
+    g._recorded = True
+    for trip in (1, 2):
+        g.indices_fwd_pos
+        assert log == [("wait", 7), ("write", 9)] * trip and len(g._partial) == 2
+
+
 def test_pair_lists_wait_only_where_they_were_handed_out(monkeypatch):
     """The lists of a geometry with several mask words: the passes' own go back without a wait (their streams
     are recorded), those that somebody took keep the memory until the device has finished."""
