@@ -119,7 +119,8 @@ __global__ __launch_bounds__(256) void relu_backward_kernel(v4i *dst, const v4i 
 // GATE: 0 = no gate; 1 = the forward output; 2 = its bits, an eighth of the bytes of one of three tensors, the rows
 // then in the order of the positions, in which the bits lie (rows of 128 bytes and more in any order move as
 // fast): 128 channels at 1 M voxels 117 -> 83 us, 797 k rows of 256 channels 195 -> 147; passes forward and
-// backward 716.8 -> 695.1 and 779.1 -> 736.0.
+// backward 716.8 -> 695.1 and 779.1 -> 736.0.  3 = the forward output, the rows in that order too: the sums of 2 for
+// whoever has no bits.
 template <class T, int GATE, bool NT>
 __global__ __launch_bounds__(256) void column_partial_kernel(const ColumnSumParams p, const WgradPrepareParams pre, int pre_blocks) {
   __shared__ float lds[256][9];
@@ -148,23 +149,21 @@ __global__ __launch_bounds__(256) void column_partial_kernel(const ColumnSumPara
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) {
         at[u] = r + u * R < r1 ? r + u * R : r;
-        if constexpr (GATE == 2) {
-          b[u] = bits[at[u] * 8];
-          at[u] = p.order[at[u]];
-        }
+        if constexpr (GATE == 2) b[u] = bits[at[u] * 8];
+        if constexpr (GATE >= 2) at[u] = p.order[at[u]];
         at[u] *= V;
       }
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) {
         g[u] = load_piece<NT>(src + at[u]);
-        if constexpr (GATE == 1) o[u] = load_piece<NT>(out + at[u]);
+        if constexpr (GATE == 1 || GATE == 3) o[u] = load_piece<NT>(out + at[u]);
       }
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) {
         if (r + u * R >= r1) break;
         if constexpr (GATE != 0) {
-          if constexpr (GATE == 1) g[u] = gate8<T>(g[u], o[u]);
-          else g[u] = gate8_bits(g[u], b[u]);
+          if constexpr (GATE == 2) g[u] = gate8_bits(g[u], b[u]);
+          else g[u] = gate8<T>(g[u], o[u]);
           gated[at[u]] = g[u];
         }
         float f[8];
@@ -279,8 +278,9 @@ static void column_partial(const ColumnSumParams &p, const WgradPrepareParams &p
     else hipLaunchKernelGGL((column_partial_kernel<T, GATE, false>), grid, dim3(256), 0, s, p, pre, pre_blocks);
   };
   if (p.gated == nullptr) launch(std::integral_constant<int, 0>{});
-  else if (p.gate == nullptr) launch(std::integral_constant<int, 1>{});
-  else launch(std::integral_constant<int, 2>{});
+  else if (p.gate != nullptr) launch(std::integral_constant<int, 2>{});
+  else if (p.order != nullptr) launch(std::integral_constant<int, 3>{});
+  else launch(std::integral_constant<int, 1>{});
 }
 
 hipError_t launch_column_partial(ColumnSumParams p, const WgradPrepareParams *pre, int pre_blocks, bool bf16, hipStream_t s,

@@ -211,9 +211,9 @@ struct ColumnSumParams {
   void *dst;            // [channels]
   const void *src;      // [rows, channels]
   const void *out;      // [rows, channels] forward output whose positive elements let src through, or
-  const uint8_t *gate;  // a bit for each of them by position (RowGemmParams::gate) and
-  const int32_t *order; // [rows] the row of a position;
+  const uint8_t *gate;  // a bit for each of them by position (RowGemmParams::gate);
   void *gated;          // and the gated rows; NULL all: plain sums
+  const int32_t *order; // [rows] the row of a position, or NULL (not with gate): the order in which rows are added up
   float *partial;       // [blocks, channels] fp32
   int64_t rows, rows_per_block;
   int32_t channels, blocks;

@@ -238,6 +238,11 @@ py::tuple build(const Tensor &coords, const Three &shape, const Three &ksize, co
 }
 
 // ---- a layer
+// Output channels from which the gate of a fused ReLU goes over the gradient in the order of the positions, in which
+// the forward pass leaves its bits - also where there are none (first calls, saved-tensor hooks, compiled autograd: the output
+// is what they have), so that a bias gradient has the same bits whoever computes it.  Rows of 128 bytes (32 channels:
+// 15.2 -> 15.6 us, and 1.6 for the bits; 64: 11.6 -> 10.2 at 120 k rows, 50 -> 46 at 798 k).  torch_bridge.py has the same.
+constexpr int64_t kGateFrom = 64;
 // backward in Python, for calls that are not known here: (geometry, features, weight, out or None, gradient, needed
 // gradients, relu, has_bias, tile_m) -> three gradients
 PyObject *python_backward = nullptr;
@@ -406,12 +411,9 @@ struct SparseConvBackward : public torch::autograd::Node {
     if (relu) {
       gated = at::empty_like(gy);
       sums.gated = gated.data_ptr();
-      if (bits.defined()) {
-        sums.gate = bits.data_ptr();
-        sums.order = g->order_fwd;
-      } else {
-        sums.out = y.data_ptr();
-      }
+      if (bits.defined()) sums.gate = bits.data_ptr();
+      else sums.out = y.data_ptr();
+      if (k_out >= kGateFrom) sums.order = g->order_fwd;
     }
     if (need[2] && !need[1]) check(api.gate_sums(&sums, dtype, s));
     if (!need[2] && relu) check(api.relu_backward(gated.data_ptr(), gy.data_ptr(), y.data_ptr(), (size_t)gy.numel(), dtype, s));
@@ -497,10 +499,8 @@ Tensor run_forward(const Tensor &features, const Tensor &weight, const std::opti
   const bool differentiable =
       at::GradMode::is_enabled() && (features.requires_grad() || weight.requires_grad() || (bias.has_value() && bias->requires_grad()));
   // The gate of the backward pass as bits, which a pass over the gradient reads instead of the output.  Saved-tensor
-  // hooks may hand back another output, which then is what counts.  From rows of 128 bytes on: the pass takes them in the
-  // order of the positions (32 channels: 15.2 -> 15.6 us, and 1.6 for the bits; 64: 11.6 -> 10.2 at 120 k rows, 50 -> 46 at
-  // 798 k).
-  const bool gated = differentiable && relu && weight.size(0) >= 64 && bias.has_value() && bias->requires_grad() &&
+  // hooks may hand back another output, which then is what counts.
+  const bool gated = differentiable && relu && weight.size(0) >= kGateFrom && bias.has_value() && bias->requires_grad() &&
                      !at::SavedTensorDefaultHooks::get_hooks().has_value();
   Tensor x, w, y, gate;
   {

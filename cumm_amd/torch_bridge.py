@@ -214,6 +214,10 @@ def _bytes(n: int, device) -> torch.Tensor:
     return torch.empty(max(int(n), 256), dtype=torch.uint8, device=device)
 
 
+# output channels from which the gradient's gate and sums go by position (torch_native.cpp has the same, and why)
+_GATE_FROM = 64
+
+
 class _HandedOut:
     """What a tv tensor over the block of a geometry keeps alive: its memory goes back to torch's allocator as
     tv's own storage goes back to the driver, when the device has finished with it.  (The operators run
@@ -535,8 +539,9 @@ def _backward(g: SparseConvGeometry, features, weight, out, grad_out, needed, re
         ws = _bytes(need, grad_out.device)
         if relu:
             gated = torch.empty_like(grad_out)
-            _capi.check(lib.cumm_hip_relu_backward_sums(gated.data_ptr(), grad_b.data_ptr(), grad_out.data_ptr(), out.data_ptr(),
-                                                        rows, k_out, dtype, ws.data_ptr(), ws.numel(), stream))
+            sums = _capi.GateSums(gated.data_ptr(), grad_b.data_ptr(), grad_out.data_ptr(), out.data_ptr(), rows, k_out,
+                                  ws.data_ptr(), ws.numel(), None, g._ptr["order_fwd"] if k_out >= _GATE_FROM else None)
+            _capi.check(lib.cumm_hip_gate_sums(ctypes.byref(sums), dtype, stream))
             grad_out = gated
         else:
             _capi.check(lib.cumm_hip_column_sum(grad_b.data_ptr(), grad_out.data_ptr(), rows, k_out, dtype,

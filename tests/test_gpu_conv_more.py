@@ -186,7 +186,7 @@ def test_gate_and_sums_are_of_the_gradient_of_the_call():
 ])
 def test_gate_of_a_forward_pass(dtype, ksize, cin, k_out, tile, n, hint):
     """The bits that a ReLU layer leaves are those of its output; a gradient gated by them is what the output gives, its
-    sums (of whole numbers, exact in any order) too."""
+    sums too: of whole numbers, exact in any order, and in one order of the rows of any numbers."""
     print("case gate", dtype, ksize, cin, k_out, tile, n, hint, flush=True)
     rng, lib = np.random.default_rng(k_out), _capi.lib()
     coords, grid = H.small_cloud(5, n, grid=(20, 90, 90), clusters=12, sigma=6.0)
@@ -215,16 +215,22 @@ def test_gate_of_a_forward_pass(dtype, ksize, cin, k_out, tile, n, hint):
     np.testing.assert_array_equal(got, want)
 
     need = int(lib.cumm_hip_column_sum_workspace(n, k_out))
-    grad = rng.integers(-2, 3, size=(n, k_out)).astype(np.float32)
-    d_grad, ws = H.dev(H.to_storage(grad, dtype), dtype), tv.zeros([need], tv.uint8, 0)
-    both = []
-    for source in ({"out": p.output.byte_pointer()}, {"gate": d_gate.byte_pointer(), "order": p.mask_argsort.byte_pointer()}):
-        gated, sums = tv.zeros([n, k_out], H.TV_DTYPE[dtype], 0), tv.zeros([k_out], H.TV_DTYPE[dtype], 0)
-        gs = _capi.GateSums(gated=gated.byte_pointer(), sums=sums.byte_pointer(), grad=d_grad.byte_pointer(), rows=n, channels=k_out,
-                            workspace=ws.byte_pointer(), workspace_bytes=need, **source)
-        _capi.check(lib.cumm_hip_gate_sums(ctypes.byref(gs), int(H.TV_DTYPE[dtype]), None))
-        _capi.check(lib.cumm_hip_device_synchronize())
-        both.append((H.host(gated).view(np.uint16), H.host(sums).view(np.uint16)))
-    np.testing.assert_array_equal(both[0][0], both[1][0])
-    np.testing.assert_array_equal(both[0][1], both[1][1])
-    np.testing.assert_array_equal(both[0][0] != 0, (H.as_f32(out, dtype) > 0) & (grad != 0))
+    in_order = p.mask_argsort.byte_pointer()
+    sources = ({"out": p.output.byte_pointer()}, {"out": p.output.byte_pointer(), "order": in_order},
+               {"gate": d_gate.byte_pointer(), "order": in_order})
+    for grad in (rng.normal(0, 1, size=(n, k_out)).astype(np.float32), rng.integers(-2, 3, size=(n, k_out)).astype(np.float32)):
+        whole = bool((grad == np.rint(grad)).all())
+        d_grad, ws = H.dev(H.to_storage(grad, dtype), dtype), tv.zeros([need], tv.uint8, 0)
+        got = []
+        for source in sources:
+            gated, sums = tv.zeros([n, k_out], H.TV_DTYPE[dtype], 0), tv.zeros([k_out], H.TV_DTYPE[dtype], 0)
+            gs = _capi.GateSums(gated=gated.byte_pointer(), sums=sums.byte_pointer(), grad=d_grad.byte_pointer(), rows=n, channels=k_out,
+                                workspace=ws.byte_pointer(), workspace_bytes=need, **source)
+            _capi.check(lib.cumm_hip_gate_sums(ctypes.byref(gs), int(H.TV_DTYPE[dtype]), None))
+            _capi.check(lib.cumm_hip_device_synchronize())
+            got.append((H.host(gated).view(np.uint16), H.host(sums).view(np.uint16)))
+        for one, two in ((0, 1), (1, 2)):
+            np.testing.assert_array_equal(got[one][0], got[two][0])
+            if whole or one == 1:
+                np.testing.assert_array_equal(got[one][1], got[two][1])
+        np.testing.assert_array_equal(got[0][0] & 0x7FFF != 0, (H.as_f32(out, dtype) > 0) & (H.to_storage(grad, dtype).view(np.uint16) & 0x7FFF != 0))

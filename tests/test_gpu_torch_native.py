@@ -29,9 +29,10 @@ def _grads(call, x, w, b, g, which=(True, True, True)):
 @pytest.mark.parametrize("ksize,strided,dtype", [(3, False, torch.float16), (3, True, torch.bfloat16), (5, False, torch.bfloat16)])
 @pytest.mark.parametrize("relu", [False, True])
 @pytest.mark.parametrize("with_bias", [False, True])
-def test_same_bits_as_the_python_function(ksize, strided, dtype, relu, with_bias):
-    print("case native", ksize, strided, dtype, relu, with_bias, flush=True)
-    tb, geo, x, w, b, g = _setup(ksize, strided, dtype=dtype)
+@pytest.mark.parametrize("k", [40, 72])      # (from 64 channels on the forward pass leaves its gate as bits)
+def test_same_bits_as_the_python_function(ksize, strided, dtype, relu, with_bias, k):
+    print("case native", ksize, strided, dtype, relu, with_bias, k, flush=True)
+    tb, geo, x, w, b, g = _setup(ksize, strided, k=k, dtype=dtype)
     assert geo._native.tables() == {**geo._ptr, **{"reduced_%d" % w: a for w, a in geo._reduced_at.items()}}
     b = b if with_bias else None
     python = lambda *t: tb._SparseConvFunction.apply(*t, geo, relu)
@@ -72,14 +73,15 @@ def no_python():
 @pytest.mark.parametrize("relu", [False, True])
 @pytest.mark.parametrize("with_bias", [False, True])
 @pytest.mark.parametrize("deterministic", [False, True])
-def test_a_known_backward_pass_stays_native(no_python, ksize, strided, dtype, relu, with_bias, deterministic):
-    print("case stays native", ksize, strided, dtype, relu, with_bias, deterministic, flush=True)
-    tb, geo, x, w, b, g = _setup(ksize, strided, dtype=dtype)
+@pytest.mark.parametrize("k", [40, 64])
+def test_a_known_backward_pass_stays_native(no_python, ksize, strided, dtype, relu, with_bias, deterministic, k):
+    print("case stays native", ksize, strided, dtype, relu, with_bias, deterministic, k, flush=True)
+    tb, geo, x, w, b, g = _setup(ksize, strided, k=k, dtype=dtype)
     b = b if with_bias else None
     torch.use_deterministic_algorithms(deterministic, warn_only=True)
     try:
         want = _grads(lambda *t: tb._SparseConvFunction.apply(*t, geo, relu), x, w, b, g)
-        _, later, *_ = _setup(ksize, strided, dtype=dtype)      # (another geometry of the kind: only what was remembered serves it)
+        _, later, *_ = _setup(ksize, strided, k=k, dtype=dtype)      # (another geometry of the kind: only what was remembered serves it)
         got = _grads(lambda *t: tb._native().forward(*t, later, later._native, relu), x, w, b, g)
         # (the weight gradient's atomics: sums in any order, and one rounding to the type)
         for i, (a, c) in enumerate(zip(got, want)):
@@ -110,8 +112,10 @@ def test_a_gradient_that_nobody_has(no_python):
         assert got.shape == leaf.shape and got.dtype == leaf.dtype and not got.any()
 
 
-def test_what_autograd_keeps():
-    tb, geo, x, w, b, g = _setup()
+@pytest.mark.parametrize("k", [40, 64, 72])
+def test_what_autograd_keeps(k):
+    print("case what autograd keeps", k, flush=True)
+    tb, geo, x, w, b, g = _setup(k=k)
     conv = lambda *t: tb.sparse_conv(*t, geo, True)
     want = _grads(conv, x, w, b, g)
     x, w, b = (t.detach().clone().requires_grad_(True) for t in (x, w, b))
@@ -131,17 +135,48 @@ def test_what_autograd_keeps():
             changed(out)
         with pytest.raises(RuntimeError, match="modified by an inplace operation"):
             torch.autograd.grad(out, (x, w, b), g)
+    # a graph that is kept, without hooks (the weights are others by now)
+    want = _grads(conv, x, w, b, g)
+    out = conv(x, w, b)
+    for keep in (True, False):
+        got = torch.autograd.grad(out, (x, w, b), g, retain_graph=keep)
+        assert all(torch.equal(a, c) for a, c in zip(got[::2], want[1::2]))
+    with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.grad(out, (x, w, b), g)
     # a gradient that nobody computed is zero
     out = conv(x, w, b)
     zero = torch.autograd.grad(out, (x, w, b), torch.zeros_like(out))
     assert all(not t.any() for t in zero)
 
 
-def test_a_node_used_by_two_threads_while_one_frees_it():
+@pytest.mark.parametrize("ksize,strided,k,dtype", [(3, False, 64, torch.float16), (3, True, 72, torch.bfloat16), (5, False, 128, torch.float16),
+                                                   (3, False, 40, torch.float16)])
+def test_a_bias_gradient_is_added_up_in_one_order(ksize, strided, k, dtype):
+    """Gradients of which the large ones cancel, so that another order of the rows gives other bits: the Python
+    function, a native pass with the gate's bits, one whose output went through saved-tensor hooks."""
+    print("case one order of a bias gradient", ksize, strided, k, dtype, flush=True)
+    tb, geo, x, w, b, g = _setup(ksize, strided, k=k, dtype=dtype, n=6000)
+    python = lambda *t: tb._SparseConvFunction.apply(*t, geo, True)
+    native = lambda *t: tb._native().forward(*t, geo, geo._native, True)
+    y = python(x, w, b)
+    turn = (y > 0).cumsum(0) % 4
+    g = torch.where(turn == 1, 1000.0, torch.where(turn == 2, -1000.0, g.float())).to(dtype)
+    want = _grads(python, x, w, b, g)[3]
+    exact = torch.where(y > 0, g, 0).double().sum(0)
+    assert ((want.double() - exact).abs() < 0.02 * exact.abs().max()).all()      # (2000 terms of 1000 in fp32, and one rounding)
+    for _ in range(2):
+        assert torch.equal(_grads(native, x, w, b, g)[3], want)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.clone(), lambda t: t):
+        assert torch.equal(_grads(native, x, w, b, g)[3], want)
+
+
+@pytest.mark.parametrize("k", [40, 64])
+def test_a_node_used_by_two_threads_while_one_frees_it(k):
     """A backward pass that frees the graph, beside calls of the node from another thread: each call has the right
     gradients or the error of a freed graph."""
     import threading
-    tb, geo, x, w, b, g = _setup()
+    print("case two threads", k, flush=True)
+    tb, geo, x, w, b, g = _setup(k=k)
     want = _grads(lambda *t: tb.sparse_conv(*t, geo, True), x, w, b, g)
     leaves = [t.detach().clone().requires_grad_(True) for t in (x, w, b)]
     torch.cuda.synchronize()
@@ -191,8 +226,10 @@ def test_what_is_left_to_python():
         tb.sparse_conv(x, w.cpu(), b, geo)
 
 
-def test_on_another_stream_and_after_the_geometry():
-    tb, geo, x, w, b, g = _setup()
+@pytest.mark.parametrize("k", [40, 64])
+def test_on_another_stream_and_after_the_geometry(k):
+    print("case another stream", k, flush=True)
+    tb, geo, x, w, b, g = _setup(k=k)
     conv = lambda *t: tb.sparse_conv(*t, geo, True)
     want = _grads(conv, x, w, b, g)
     stream = torch.cuda.Stream()
@@ -206,14 +243,15 @@ def test_on_another_stream_and_after_the_geometry():
     assert torch.equal(out.detach(), want[0]) and torch.equal(got[0], want[1]) and torch.equal(got[2], want[3])
 
 
-def test_compiled_autograd():
+@pytest.mark.parametrize("k", [40, 72])
+def test_compiled_autograd(k):
     """A backward pass under torch's compiled autograd (its graph run as it is): the gradients of the ordinary one, also
     where the graph of one layer serves the next - another geometry of the same sizes."""
     from torch._dynamo import compiled_autograd
     for ksize, strided, relu, with_bias in ((3, False, True, True), (3, True, False, False), (5, False, True, False)):
         for seed in (3, 4):
-            print("case compiled autograd", ksize, strided, relu, with_bias, seed, flush=True)
-            tb, geo, x, w, b, g = _setup(ksize, strided, seed=seed)
+            print("case compiled autograd", ksize, strided, relu, with_bias, seed, k, flush=True)
+            tb, geo, x, w, b, g = _setup(ksize, strided, k=k, seed=seed)
             conv = lambda *t: tb.sparse_conv(*t, geo, relu)
             leaves = lambda: [t.detach().clone().requires_grad_(True) for t in ((x, w, b) if with_bias else (x, w))]
             of = lambda ts: tuple(ts) + (() if with_bias else (None,))
@@ -231,15 +269,16 @@ def test_compiled_autograd():
 
 
 @pytest.mark.parametrize("ksize,strided", [(3, False), (3, True), (5, False)])
-def test_without_the_native_half(monkeypatch, ksize, strided):
+@pytest.mark.parametrize("k", [40, 72])
+def test_without_the_native_half(monkeypatch, ksize, strided, k):
     """On a machine without a host compiler the bridge's own functions make every call: the same tables and bits."""
-    print("case without native", ksize, strided, flush=True)
-    tb, geo, x, w, b, g = _setup(ksize, strided)
+    print("case without native", ksize, strided, k, flush=True)
+    tb, geo, x, w, b, g = _setup(ksize, strided, k=k)
     torch.use_deterministic_algorithms(True, warn_only=True)
     try:
         want = _grads(lambda *t: tb.sparse_conv(*t, geo, True), x, w, b, g)
         monkeypatch.setattr(tb, "_native_module", False)
-        _, own, *_ = _setup(ksize, strided)
+        _, own, *_ = _setup(ksize, strided, k=k)
         assert own._native is None and own.out_shape == geo.out_shape and torch.equal(own.out_coords, geo.out_coords)
         for name in tb.SparseConvGeometry._TABLES:
             assert (H.host(getattr(own, name)) == H.host(getattr(geo, name))).all(), name
