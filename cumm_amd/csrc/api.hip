@@ -813,6 +813,7 @@ int sparse_conv_impl(const CummHipConvDesc *desc, const CummHipSparseConvArgs *a
     if (c.op_type != CUMM_HIP_OP_BACKWARD_WEIGHT || fam == 1) return fail(CUMM_HIP_EINVAL, "only backward-weight makes the gate and sums of a gradient");
     if (more->sums->channels != a->K || more->sums->rows != a->rows_out || (more->sums->gated ? more->sums->gated : more->sums->grad) != a->ptr_A)
       return fail(CUMM_HIP_EINVAL, "gate and sums are those of the gradient of this call");
+    if (more->sums->gate && a->N != a->rows_out) return fail(CUMM_HIP_EINVAL, "a gate has a position for every row");
     if (int rc = gate_sums_params(*more->sums, dt, &sums_params)) return rc;
     sums = &sums_params;
   }

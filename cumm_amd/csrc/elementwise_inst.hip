@@ -88,12 +88,13 @@ __device__ __forceinline__ v4i gate8_bits(const v4i &g, uint32_t bits) {
   return r;
 }
 
-// thread: eight channels of a position
-__global__ __launch_bounds__(256) void gate_bits_kernel(uint8_t *gate, const v4i *out, const int32_t *order, int n, int pieces) {
+// thread: eight channels of a position (one that names no row of out is left alone, as by the convolution kernels)
+__global__ __launch_bounds__(256) void gate_bits_kernel(uint8_t *gate, const v4i *out, const int32_t *order, int n, int rows, int pieces) {
   const int64_t total = (int64_t)n * pieces;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
     const int pos = (int)(i / pieces), piece = (int)(i - (int64_t)pos * pieces);
     const int row = order ? order[pos] : pos;
+    if ((uint32_t)row >= (uint32_t)rows) continue;
     gate[((int64_t)(piece >> 3) * n + pos) * 8 + (piece & 7)] = (uint8_t)positive8(out[(int64_t)row * pieces + piece]);
   }
 }
@@ -146,11 +147,16 @@ __global__ __launch_bounds__(256) void column_partial_kernel(const ColumnSumPara
       v4i g[kBatch], o[kBatch];
       int64_t at[kBatch];
       uint32_t b[kBatch];
+      bool none[kBatch];
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) {
         at[u] = r + u * R < r1 ? r + u * R : r;
         if constexpr (GATE == 2) b[u] = bits[at[u] * 8];
-        if constexpr (GATE >= 2) at[u] = p.order[at[u]];
+        if constexpr (GATE >= 2) {      // (a position that names no row: row 0 is loaded and not used)
+          const int64_t row = p.order[at[u]];
+          none[u] = (uint64_t)row >= (uint64_t)p.rows;
+          at[u] = none[u] ? 0 : row;
+        }
         at[u] *= V;
       }
 #pragma unroll
@@ -161,6 +167,7 @@ __global__ __launch_bounds__(256) void column_partial_kernel(const ColumnSumPara
 #pragma unroll
       for (int u = 0; u < kBatch; ++u) {
         if (r + u * R >= r1) break;
+        if (GATE >= 2 && none[u]) continue;
         if constexpr (GATE != 0) {
           if constexpr (GATE == 2) g[u] = gate8_bits(g[u], b[u]);
           else g[u] = gate8<T>(g[u], o[u]);
@@ -216,10 +223,10 @@ hipError_t launch_finish_rows(const FinishRowsParams &p, bool bf16, hipStream_t 
   return hipGetLastError();
 }
 
-hipError_t launch_gate_bits(uint8_t *gate, const void *out, const int32_t *order, int n, int channels, hipStream_t s) {
+hipError_t launch_gate_bits(uint8_t *gate, const void *out, const int32_t *order, int n, int rows, int channels, hipStream_t s) {
   if (n <= 0 || channels <= 0) return hipSuccess;
   const int pieces = channels / 8;
-  hipLaunchKernelGGL(gate_bits_kernel, dim3(grid_for((size_t)n * pieces)), dim3(256), 0, s, gate, reinterpret_cast<const v4i *>(out), order, n, pieces);
+  hipLaunchKernelGGL(gate_bits_kernel, dim3(grid_for((size_t)n * pieces)), dim3(256), 0, s, gate, reinterpret_cast<const v4i *>(out), order, n, rows, pieces);
   return hipGetLastError();
 }
 

@@ -205,7 +205,7 @@ struct FinishRowsParams {
 };
 hipError_t launch_finish_rows(const FinishRowsParams &p, bool bf16, hipStream_t s);
 // RowGemmParams::gate out of the output rows (two-byte elements, not negative) of n positions
-hipError_t launch_gate_bits(uint8_t *gate, const void *out, const int32_t *order, int n, int channels, hipStream_t s);
+hipError_t launch_gate_bits(uint8_t *gate, const void *out, const int32_t *order, int n, int rows, int channels, hipStream_t s);
 hipError_t launch_relu_backward(void *dst, const void *grad, const void *out, size_t vecs, bool bf16, hipStream_t s);
 struct ColumnSumParams {
   void *dst;            // [channels]

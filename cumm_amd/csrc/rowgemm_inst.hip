@@ -220,7 +220,7 @@ static hipError_t launch_one(const RowGemmParams &p, hipStream_t s) {
   }
   err = launch_fallback<T, NW, RB, TN, KS, WT>(p, grid, s);
   if (err != hipSuccess || p.gate == nullptr) return err;
-  return launch_gate_bits(p.gate, p.C, p.out_rows, p.n_pos, p.k_out, s);      // (these kernels leave none)
+  return launch_gate_bits(p.gate, p.C, p.out_rows, p.n_pos, p.rows_c, p.k_out, s);      // (these kernels leave none)
 }
 
 // kernels whose waits the compiler counts

@@ -175,9 +175,10 @@ typedef struct CummHipGateSums {
   void *workspace;                  /* cumm_hip_column_sum_workspace bytes, not shared with the call's own */
   size_t workspace_bytes;
   const void *gate;                 /* instead of out: what the forward call left (CummHipSparseConvMore::gate) */
-  const int32_t *order;             /* that call's mask_argsort_ptr: [rows], every row once.  With gate, and with out where it
-                                       is given, the rows are added up in this order: the same bits from either; NULL:
-                                       out, in the order of the rows */
+  const int32_t *order;             /* that call's mask_argsort_ptr: [rows], every row once (a position that names no row of
+                                       [0, rows) is passed over, and a row that none names left alone).  With gate, and
+                                       with out where it is given, the rows are added up in this order: the same bits from
+                                       either; NULL: out, in the order of the rows */
 } CummHipGateSums;
 
 /* What a training program wants of the same launches beyond the reference's argument block; all zero = nothing. */

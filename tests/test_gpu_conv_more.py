@@ -234,3 +234,80 @@ def test_gate_of_a_forward_pass(dtype, ksize, cin, k_out, tile, n, hint):
             if whole or one == 1:
                 np.testing.assert_array_equal(got[one][1], got[two][1])
         np.testing.assert_array_equal(got[0][0] & 0x7FFF != 0, (H.as_f32(out, dtype) > 0) & (H.to_storage(grad, dtype).view(np.uint16) & 0x7FFF != 0))
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("rows,channels", [(1, 64), (700, 64), (700, 136), (40000, 72)])
+def test_positions_that_name_no_row(dtype, rows, channels):
+    """A few positions of the order lie outside the rows: they are passed over, and the rows that nobody names are left
+    alone."""
+    print("case no row", dtype, rows, channels, flush=True)
+    rng, lib = np.random.default_rng(rows), _capi.lib()
+    order = rng.permutation(rows).astype(np.int32)
+    outside = np.unique(rng.integers(0, rows, size=min(rows, 9)))
+    named = np.ones(rows, bool)
+    named[order[outside]] = False
+    order[outside] = np.resize(np.array([-1, rows, 2 ** 31 - 1, -2 ** 31], np.int32), len(outside))
+    grad, out = (rng.integers(-2, 3, size=(rows, channels)).astype(np.float32) for _ in range(2))
+    want = np.where(named[:, None], np.where(out > 0, grad, np.float32(0)), np.float32(9.0))
+    gate = np.zeros((rows, (channels + 63) // 64 * 64), bool)
+    inside = (order >= 0) & (order < rows)
+    gate[inside, :channels] = out[order[inside]] > 0
+    gate[~inside] = True
+    bits = np.packbits(gate, axis=1, bitorder="little").reshape(rows, -1, 8).transpose(1, 0, 2)
+    d_grad, d_out, d_order = H.dev(H.to_storage(grad, dtype), dtype), H.dev(H.to_storage(out, dtype), dtype), H.dev(order, "i32")
+    d_bits = tv.from_numpy(np.ascontiguousarray(bits)).cuda()
+    need = int(lib.cumm_hip_column_sum_workspace(rows, channels))
+    ws = tv.zeros([need], tv.uint8, 0)
+    for source in ({"out": d_out.byte_pointer()}, {"gate": d_bits.byte_pointer()}):
+        gated, sums = H.dev(H.to_storage(np.full_like(grad, 9.0), dtype), dtype), tv.zeros([channels], H.TV_DTYPE[dtype], 0)
+        gs = _capi.GateSums(gated=gated.byte_pointer(), sums=sums.byte_pointer(), grad=d_grad.byte_pointer(), rows=rows, channels=channels,
+                            workspace=ws.byte_pointer(), workspace_bytes=need, order=d_order.byte_pointer(), **source)
+        _capi.check(lib.cumm_hip_gate_sums(ctypes.byref(gs), int(H.TV_DTYPE[dtype]), None))
+        _capi.check(lib.cumm_hip_device_synchronize())
+        np.testing.assert_array_equal(H.as_f32(H.host(gated), dtype), want)
+        np.testing.assert_array_equal(H.host(sums).view(np.uint16), H.to_storage(want[named].sum(axis=0), dtype).view(np.uint16))
+
+
+@pytest.mark.parametrize("cin,k_out", [(64, 64), (520, 64), (64, 136)])      # (a contraction of 520: the gate is a launch of its own)
+def test_a_gate_of_positions_that_name_no_row(cin, k_out):
+    """The bits of those positions are left alone, the others are what they are."""
+    print("case gate of no row", cin, k_out, flush=True)
+    rng, n = np.random.default_rng(cin + k_out), 300
+    p = ConvParams(3, ConvOpType.Forward)
+    p.conv_algo_desp = H.find_conv_desp("f16", ConvOpType.Forward, 64, 64)
+    order = rng.permutation(n).astype(np.int32)
+    inside = np.ones(n, bool)
+    inside[[0, 7, 128, 299]] = False
+    order[~inside] = [-1, n, 2 ** 31 - 1, -2 ** 31]
+    p.input = H.dev(H.to_storage(rng.normal(0, 1, size=(n, cin)).astype(np.float32), "f16"), "f16")
+    p.weight = H.dev(H.to_storage(rng.normal(0, 0.05, size=(k_out, 1, cin)).astype(np.float32), "f16"), "f16")
+    p.output, p.act_type = tv.zeros([n, k_out], tv.float16, 0), Activation.ReLU
+    p.indices, p.mask, p.mask_argsort = H.dev(np.arange(n, dtype=np.int32)[None], "i32"), H.dev(np.ones(n, np.uint32), "u32"), H.dev(order, "i32")
+    ConvMainUnitTest.implicit_gemm2(p)
+    groups = (k_out + 63) // 64
+    d_gate = tv.from_numpy(np.full((groups, n, 8), 0xA5, np.uint8)).cuda()
+    _again(p, gate=d_gate.byte_pointer())
+    got = H.host(d_gate).transpose(1, 0, 2).reshape(n, groups * 8)[:, :k_out // 8]
+    out = H.as_f32(H.host(p.output), "f16")
+    np.testing.assert_array_equal(got[inside], np.packbits(out[order[inside]] > 0, axis=1, bitorder="little"))
+    assert (got[~inside] == 0xA5).all()
+
+
+def test_a_gate_has_a_position_for_every_row():
+    """The bits of a call with another number of positions are not those of the rows."""
+    n = 64
+    p = ConvParams(3, ConvOpType.BackwardWeight)
+    p.conv_algo_desp = H.find_conv_desp("f16", ConvOpType.BackwardWeight, 64, 64, split_k_parallel=True)
+    p.input, p.output, p.weight = (tv.zeros(shape, tv.float16, 0) for shape in ([n, 64], [n, 64], [64, 1, 64]))
+    p.indices, p.mask, p.mask_argsort = (H.dev(np.arange(n, dtype=np.int32)[None], "i32"), H.dev(np.ones(1, np.uint32), "u32"),
+                                         H.dev(np.arange(n, dtype=np.int32), "i32"))
+    p.mask_width, p.split_k_slices = 64, 4
+    ConvMainUnitTest.implicit_gemm2(p)
+    ws, gate, grad = (tv.zeros([1 << 16], tv.uint8, 0) for _ in range(3))
+    gs = _capi.GateSums(gated=p.output.byte_pointer(), sums=ws.byte_pointer(), grad=grad.byte_pointer(), rows=n, channels=64,
+                        workspace=ws.byte_pointer() + 4096, workspace_bytes=1 << 15, gate=gate.byte_pointer(), order=p.mask_argsort.byte_pointer())
+    _again(p, sums=ctypes.addressof(gs))
+    p.__dict__["_prepared"][5].N = n - 1
+    with pytest.raises(ValueError):
+        _again(p, sums=ctypes.addressof(gs))
