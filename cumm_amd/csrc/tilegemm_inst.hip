@@ -182,11 +182,19 @@ static hipError_t prepare(const WgradPrepareParams &pre, int blocks, const Colum
   return hipGetLastError();
 }
 
+// The table that the unit-walking kernel reads: 1 = by position, 0 = by row (also where a caller has both and only that
+// instantiation holds its counted waits), -1 = neither
+constexpr int units_table(bool by_position, bool by_position_holds, bool by_row_holds) {
+  return by_position && by_position_holds ? 1 : (by_row_holds ? 0 : -1);
+}
+static_assert(units_table(true, true, false) == 1 && units_table(true, false, true) == 0 && units_table(true, false, false) == -1 &&
+              units_table(false, true, true) == 0 && units_table(false, true, false) == -1, "by position only where asked for");
+
 // The unit-walking kernel, for 128 x 128 channels or 64 x 64
 template <class T, bool DET>
-static bool units_ok(bool wide, bool by_position) {
-  if (by_position) return wide ? counted_waits_hold<wgrad_units_kernel<T, 2, 2, 1, DET, true>>() : counted_waits_hold<wgrad_units_kernel<T, 1, 1, 2, DET, true>>();
-  return wide ? counted_waits_hold<wgrad_units_kernel<T, 2, 2, 1, DET>>() : counted_waits_hold<wgrad_units_kernel<T, 1, 1, 2, DET>>();
+static int units_table_of(bool wide, bool by_position) {
+  if (wide) return units_table(by_position, counted_waits_hold<wgrad_units_kernel<T, 2, 2, 1, DET, true>>(), counted_waits_hold<wgrad_units_kernel<T, 2, 2, 1, DET>>());
+  return units_table(by_position, counted_waits_hold<wgrad_units_kernel<T, 1, 1, 2, DET, true>>(), counted_waits_hold<wgrad_units_kernel<T, 1, 1, 2, DET>>());
 }
 template <class T, bool DET>
 static void launch_units(bool wide, const WgradParams &p, dim3 grid, hipStream_t s) {
@@ -210,20 +218,23 @@ hipError_t CUMM_CAT(launch_wgrad_atomic_, CUMM_NAME)(const WgradParams &p, const
   if (groups == 0 || p.kv == 0) return hipSuccess;
   hipError_t e;
   ColumnFinalParams last = {};
-  if (p.live_list != nullptr && !units_ok<T, false>(wide, p.by_position != nullptr)) return hipErrorNotSupported;
   if (p.live_list != nullptr) {
     // lists + zeroed image, then a resident grid that walks the units
-    static int resident_of[2][16] = {};
+    const int table = units_table_of<T, false>(wide, p.by_position != nullptr);
+    if (table < 0) return hipErrorNotSupported;
+    static int resident_of[2][2][16] = {};
     int dev = 0;
     e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
-    int &resident = resident_of[wide ? 1 : 0][dev & 15];
+    int &resident = resident_of[table][wide ? 1 : 0][dev & 15];
     if (resident == 0) {
       int cus = 0, per_cu = 0;
       e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
       if (e == hipSuccess)
-        e = wide ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wgrad_units_kernel<T, 2, 2, 1>, 256, 0)
-                 : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wgrad_units_kernel<T, 1, 1, 2>, 256, 0);
+        e = table == 1 ? (wide ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wgrad_units_kernel<T, 2, 2, 1, false, true>, 256, 0)
+                               : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wgrad_units_kernel<T, 1, 1, 2, false, true>, 256, 0))
+                       : (wide ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wgrad_units_kernel<T, 2, 2, 1>, 256, 0)
+                               : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, wgrad_units_kernel<T, 1, 1, 2>, 256, 0));
       if (e != hipSuccess) return e;
       resident = cus * per_cu > 0 ? cus * per_cu : 1;
     }
@@ -233,6 +244,7 @@ hipError_t CUMM_CAT(launch_wgrad_atomic_, CUMM_NAME)(const WgradParams &p, const
     // inputs) or walks them all on one set of pair lists (the centre offset alone then gives
     // `groups` units: enough when that fills the device).
     WgradParams q = p;
+    if (table == 0) q.by_position = nullptr;
     q.merge_blocks = kblocks * cblocks > 1 && groups >= resident ? 1 : 0;
     // never more workgroups than units can exist
     const long long max_units = ((long long)groups * p.kv + p.kv) * (q.merge_blocks ? 1 : kblocks * cblocks);
@@ -251,7 +263,8 @@ hipError_t CUMM_CAT(launch_wgrad_atomic_, CUMM_NAME)(const WgradParams &p, const
 }
 
 // Fixed-order variant: the same units, a contiguous run per workgroup, partial sums stored into
-// slots and added up in workgroup order.  `max_wgs` = workgroups the caller's slots allow.
+// slots and added up in workgroup order.  `max_wgs` = workgroups the caller's slots allow.  The workgroups of the kernel that
+// reads the table by row, whichever table is read: their number decides the order of the sums.
 int CUMM_CAT(wgrad_ordered_resident_, CUMM_NAME)(bool wide) {
   using T = CUMM_ELEM;
   static int resident_of[2][16] = {};
@@ -275,11 +288,14 @@ hipError_t CUMM_CAT(launch_wgrad_ordered_, CUMM_NAME)(const WgradParams &p, cons
                                                       hipStream_t s) {
   using T = CUMM_ELEM;
   if (p.num_red == 0 || p.kv == 0 || wgs < 1) return hipSuccess;
-  if (!units_ok<T, true>(wide, p.by_position != nullptr)) return hipErrorNotSupported;
+  const int table = units_table_of<T, true>(wide, p.by_position != nullptr);
+  if (table < 0) return hipErrorNotSupported;
+  WgradParams q = p;
+  if (table == 0) q.by_position = nullptr;
   ColumnFinalParams last = {};
   hipError_t e = prepare<T>(pre, p.kv, sums, &last, s);   // lists only: no image to zero
   if (e != hipSuccess) return e;
-  launch_units<T, true>(wide, p, dim3(wgs), s);
+  launch_units<T, true>(wide, q, dim3(wgs), s);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (last.groups > 0) hipLaunchKernelGGL((wgrad_finalize_ordered_kernel<T, true>), dim3((unsigned)((f.total / 4 + 31) / 32) + last.groups), dim3(256), 0, s, f, last);
