@@ -100,6 +100,7 @@ __global__ __launch_bounds__(256) void gate_bits_kernel(uint8_t *gate, const v4i
 }
 
 constexpr size_t kStreamBytes = (size_t)64 << 20;
+constexpr int kNonTemporal = 2;      // of a buffer load: aux bit 1
 
 template <bool NT>
 __device__ __forceinline__ v4i load_piece(const v4i *p) {
@@ -142,41 +143,62 @@ __global__ __launch_bounds__(256) void column_partial_kernel(const ColumnSumPara
     const v4i *src = reinterpret_cast<const v4i *>(p.src) + piece;
     const v4i *out = reinterpret_cast<const v4i *>(p.out) + piece;
     v4i *gated = reinterpret_cast<v4i *>(p.gated) + piece;
-    const uint8_t *bits = p.gate + (int64_t)(piece >> 3) * p.rows * 8 + (piece & 7);
-    for (int64_t r = r0 + lane_row; r < r1; r += kBatch * R) {
-      v4i g[kBatch], o[kBatch];
-      int64_t at[kBatch];
-      uint32_t b[kBatch];
-      bool none[kBatch];
+    // By position (tensors below 2 GiB: checked on the host): nothing branches, a position past the block and one that
+    // names no row lie outside the buffers.
+    if constexpr (GATE >= 2) {
+      const uint32_t row_bytes = (uint32_t)p.channels * 2u, bytes = (uint32_t)p.rows * row_bytes, rows = (uint32_t)p.rows;
+      const __amdgpu_buffer_rsrc_t rs_order = make_rsrc(p.order, rows * 4u), rs_src = make_rsrc(p.src, bytes), rs_to = make_rsrc(p.gated, bytes);
+      const __amdgpu_buffer_rsrc_t rs_gate = GATE == 2 ? make_rsrc(p.gate, (uint32_t)((p.channels + 63) >> 6) * rows * 8u) : make_rsrc(p.out, bytes);
+      const uint32_t plane = (uint32_t)(piece >> 3) * rows * 8u + (uint32_t)(piece & 7);
+      constexpr int kHint = NT ? kNonTemporal : 0;
+      for (uint32_t pos = (uint32_t)r0 + (uint32_t)lane_row; pos < (uint32_t)r1; pos += kBatch * R) {
+        v4i g[kBatch], o[kBatch];
+        uint32_t at[kBatch], b[kBatch];
 #pragma unroll
-      for (int u = 0; u < kBatch; ++u) {
-        at[u] = r + u * R < r1 ? r + u * R : r;
-        if constexpr (GATE == 2) b[u] = bits[at[u] * 8];
-        if constexpr (GATE >= 2) {      // (a position that names no row: row 0 is loaded and not used)
-          const int64_t row = p.order[at[u]];
-          none[u] = (uint64_t)row >= (uint64_t)p.rows;
-          at[u] = none[u] ? 0 : row;
+        for (int u = 0; u < kBatch; ++u) {
+          const uint32_t here = pos + (uint32_t)(u * R);
+          const bool in = here < (uint32_t)r1;
+          at[u] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs_order, here * 4u, 0, 0);
+          if constexpr (GATE == 2) b[u] = __builtin_amdgcn_raw_buffer_load_b8(rs_gate, in ? plane + here * 8u : kOob, 0, 0);
         }
-        at[u] *= V;
-      }
 #pragma unroll
-      for (int u = 0; u < kBatch; ++u) {
-        g[u] = load_piece<NT>(src + at[u]);
-        if constexpr (GATE == 1 || GATE == 3) o[u] = load_piece<NT>(out + at[u]);
-      }
+        for (int u = 0; u < kBatch; ++u) {
+          at[u] = at[u] < rows && pos + (uint32_t)(u * R) < (uint32_t)r1 ? at[u] * row_bytes + (uint32_t)piece * 16u : kOob;
+          g[u] = __builtin_amdgcn_raw_buffer_load_b128(rs_src, at[u], 0, kHint);
+          if constexpr (GATE == 3) o[u] = __builtin_amdgcn_raw_buffer_load_b128(rs_gate, at[u], 0, kHint);
+        }
 #pragma unroll
-      for (int u = 0; u < kBatch; ++u) {
-        if (r + u * R >= r1) break;
-        if (GATE >= 2 && none[u]) continue;
-        if constexpr (GATE != 0) {
+        for (int u = 0; u < kBatch; ++u) {
           if constexpr (GATE == 2) g[u] = gate8_bits(g[u], b[u]);
           else g[u] = gate8<T>(g[u], o[u]);
-          gated[at[u]] = g[u];
-        }
-        float f[8];
-        unpack8<T>(g[u], f);
+          __builtin_amdgcn_raw_buffer_store_b128(g[u], rs_to, at[u], 0, 0);
+          float f[8];
+          unpack8<T>(g[u], f);
 #pragma unroll
-        for (int x = 0; x < 8; ++x) s[x] += f[x];
+          for (int x = 0; x < 8; ++x) s[x] += f[x];
+        }
+      }
+    } else {
+      for (int64_t r = r0 + lane_row; r < r1; r += kBatch * R) {
+        v4i g[kBatch], o[kBatch];
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+          const int64_t at = (r + u * R < r1 ? r + u * R : r) * V;
+          g[u] = load_piece<NT>(src + at);
+          if constexpr (GATE) o[u] = load_piece<NT>(out + at);
+        }
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+          if (r + u * R >= r1) break;
+          if constexpr (GATE) {
+            g[u] = gate8<T>(g[u], o[u]);
+            gated[(r + u * R) * V] = g[u];
+          }
+          float f[8];
+          unpack8<T>(g[u], f);
+#pragma unroll
+          for (int x = 0; x < 8; ++x) s[x] += f[x];
+        }
       }
     }
   }
