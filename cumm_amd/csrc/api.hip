@@ -883,10 +883,8 @@ int sparse_conv_impl(const CummHipConvDesc *desc, const CummHipSparseConvArgs *a
       return fail(CUMM_HIP_ERUNTIME, "your data exceed int32 range.");
     p.gather_bytes = (uint32_t)((int64_t)kv * a->N * 4);
     if (more != nullptr && more->gate != nullptr) {
-      const int64_t bytes = (int64_t)((a->K + 63) / 64) * a->N * 8;
-      if (bytes >= (int64_t)1 << 31) return fail(CUMM_HIP_ERUNTIME, "your data exceed int32 range.");
+      if ((int64_t)((a->K + 63) / 64) * a->N * 8 >= (int64_t)1 << 31) return fail(CUMM_HIP_ERUNTIME, "your data exceed int32 range.");
       p.gate = reinterpret_cast<uint8_t *>(more->gate);
-      p.gate_bytes = (uint32_t)bytes;
     }
     p.stream_stores = p.c_bytes <= kStreamStoreMaxBytes;
     p.small_stages = d.num_stage >= 3;

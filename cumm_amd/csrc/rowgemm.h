@@ -28,12 +28,15 @@
 //   * tiles are handed out heaviest first; each wave owns RB blocks of 16 rows and skips a block
 //     none of whose rows has a pair at offset k (its contribution would be exactly zero).
 #pragma once
+#include <cstddef>
 #include <type_traits>
 
 #include "common.h"
 
 namespace cummhip {
 
+// What every launch reads lies in the first four cache lines: with stream_stores in a fifth a product of 64 channels took
+// 13.9 us for 13.6 (150 k of 200 k rows, rowgemm_wave_kernel).
 struct RowGemmParams {
   const void *A;   // gathered operand, rows of lda elements
   const void *W;   // weights
@@ -52,7 +55,7 @@ struct RowGemmParams {
   int32_t c_in, k_out, kv;
   uint32_t mask_filter;
   int32_t reverse_mask, exit_on_empty, gather_by_pos;
-  float alpha, beta, act_alpha, act_beta;
+  float alpha, beta, act_alpha;
   int32_t act;
   int32_t int8_epilogue;  // scale/bias requantisation instead of alpha/beta
   int32_t read_source;    // D is read (beta != 0)
@@ -67,6 +70,9 @@ struct RowGemmParams {
   // preparation left for this mask array (light_hint_slot in launch.h); a slot that names another
   // array, length or filter says nothing
   const int32_t *hint_slot;
+  // a ReLU layer that will be differentiated, or NULL: a bit for every positive result, by position:
+  // gate[((c / 64) * n_pos + pos) * 8 + c % 64 / 8], bit c % 8
+  uint8_t *gate;
   // 32-bit mask words per position (1; 2 to 4 for kernel volumes above 32: see rowgemm_lds_tile)
   int32_t mask_words;
   // words the caller's mask_out array holds (a tile number beyond it is not written)
@@ -75,10 +81,6 @@ struct RowGemmParams {
   // rows are gated by their pair-table entry alone, cumm/conv/sparse_iters.py:629-631), instead of
   // only in the offsets whose bit its own mask word has
   int32_t ungated_rows;
-  // a ReLU layer that will be differentiated, or NULL: a bit for every positive result, by position:
-  // gate[((c / 64) * n_pos + pos) * 8 + c % 64 / 8], bit c % 8
-  uint8_t *gate;
-  uint32_t gate_bytes;
   // non-zero: the output rows are stored with the non-temporal hint (see kStreamStore)
   int32_t stream_stores;
   // non-zero (descriptors with num_stage 3): a contraction of more than 128 bytes is walked in
@@ -89,7 +91,9 @@ struct RowGemmParams {
   uint32_t even_group[4];      // with four: those of the first and third (first_group: of the first two)
   // non-zero: every row's sum in the one order that all tiles share
   int32_t one_order;
+  float act_beta;
 };
+static_assert(offsetof(RowGemmParams, stream_stores) + sizeof(int32_t) == 256, "four cache lines of arguments");
 
 // An offset no buffer contains: every operand is smaller than 2 GiB (checked on the host), and
 // adding a scalar offset below 2 GiB to it cannot wrap back into range.
@@ -122,6 +126,26 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *p, uint3
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00020000);
 }
 
+// The arguments that an epilogue reads, fetched again where this is called: they hold no scalar registers during the steps.
+// For kernels that would spill some (two or three tile shapes in one: rowgemm_lds_mixed_kernel), and whose first argument is
+// a RowGemmParams; elsewhere the second fetch is 0.15 us.  64 -> 64 channels forward at 120 k voxels, with 31 spills and
+// without: f16 12.0 -> 11.8 us, bf16 12.8 -> 11.9.
+__device__ __forceinline__ RowGemmParams late_params() {
+  typedef const __attribute__((address_space(4))) RowGemmParams *kernarg;
+  kernarg q = (kernarg)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(q));      // (an address that the compiler has not read from)
+  RowGemmParams e;
+  e.C = q->C; e.D = q->D; e.ldc = q->ldc; e.ldd = q->ldd; e.c_bytes = q->c_bytes; e.d_bytes = q->d_bytes;
+  e.n_pos = q->n_pos; e.rows_c = q->rows_c; e.k_out = q->k_out;
+  e.alpha = q->alpha; e.beta = q->beta; e.act_alpha = q->act_alpha; e.act = q->act;
+  e.int8_epilogue = q->int8_epilogue; e.read_source = q->read_source;
+  e.gate = q->gate; e.stream_stores = q->stream_stores;
+  return e;
+}
+
+// (below 2 GiB: checked on the host)
+__device__ __forceinline__ uint32_t gate_bytes(const RowGemmParams &p) { return (uint32_t)((p.k_out + 63) >> 6) * (uint32_t)p.n_pos * 8u; }
+
 // The gate's bits of channels [ch, ch + 8 NG) of a position, from their packed results (channels past the end are
 // zeros).  By position, so that a tile writes whole cache lines (scattered like the output rows, 16 bytes of each, they
 // took 12 us more at 1 M rows of 128 channels).  That launch takes 218 us with the bits, 212 without.
@@ -129,7 +153,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *p, uint3
 template <int NG>
 __device__ __forceinline__ void store_gate(const v4i (&outs)[NG], const RowGemmParams &p, bool ok, int pos, int ch) {
   static_assert(NG == 1 || NG == 2, "a byte, or two");
-  const __amdgpu_buffer_rsrc_t rs = make_rsrc(p.gate, p.gate_bytes);
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc(p.gate, gate_bytes(p));
   uint32_t v = positive8(outs[0]);
   if constexpr (NG == 2) v |= positive8(outs[NG - 1]) << 8;
   // (rows of 16 lanes: {0, 0, 2, 2} and {1, 1, 3, 3}, then {01, 01} and {23, 23})
@@ -151,7 +175,7 @@ __device__ __forceinline__ void store_gate(const v4i (&outs)[NG], const RowGemmP
 template <int N>
 __device__ __forceinline__ void store_gate4(const uint32_t (&bits)[N], const RowGemmParams &p, const bool (&ok)[N], int pos0, int ch) {
   constexpr int B1 = 1 % N, B2 = 2 % N, B3 = 3 % N;      // (named with fewer blocks too, where it is not called)
-  const __amdgpu_buffer_rsrc_t rs = make_rsrc(p.gate, p.gate_bytes);
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc(p.gate, gate_bytes(p));
   const uint32_t lane = threadIdx.x & 63u, block = lane >> 4;      // the row block that this lane stores
   const auto s32 = __builtin_amdgcn_permlane32_swap(bits[0] | bits[B1] << 16, bits[B2] | bits[B3] << 16, false, false);
   const auto lo = __builtin_amdgcn_permlane16_swap(s32[0], s32[0], false, false), hi = __builtin_amdgcn_permlane16_swap(s32[1], s32[1], false, false);

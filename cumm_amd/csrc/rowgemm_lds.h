@@ -79,7 +79,8 @@ struct LdsRing {
 // p.first_group and the second the others (whatever the tile's list: a row's sum does not depend on its
 // neighbours), each with a ring of its own, and at the end they add up their sums in LDS, each of them for
 // half of the row blocks.  Four: by p.even_group too; the first two finish a row block each.
-template <class T, int WM, int WN, int RBW, int NBW, int KS, int NS, bool WT, bool WIDE, bool HALVES, int MW = 1, bool HALF32 = false, int WK = 1>
+// MIXED: one of the tile shapes of rowgemm_lds_mixed_kernel, whose scalar registers are short.
+template <class T, int WM, int WN, int RBW, int NBW, int KS, int NS, bool WT, bool WIDE, bool HALVES, int MW = 1, bool HALF32 = false, int WK = 1, bool MIXED = false>
 __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const int tile, const int col, const LdsRing &lds) {
   static_assert(MW == 1 || MW == 4, "one mask word, or up to four");
   static_assert(MW == 1 || (!HALVES && !HALF32), "the tile shapes of a mixed launch take one mask word");
@@ -559,14 +560,14 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
   };
   typedef int src_vec __attribute__((ext_vector_type(SRC_W)));
   src_vec src_pre[RBW][SRC_N] = {};
-  const bool shared_src = E::kBytes == 2 && p.ldd == 0;      // one row for all (a bias): fetched and converted once
+  constexpr bool SHARED = E::kBytes == 2 && (MIXED || MW > 1 || WK > 1);      // (see MODE 4)
+  const bool shared_src = SHARED && p.ldd == 0;      // one row for all (a bias): converted once
   if (p.read_source && !WIDE) {   // (four-byte outputs read their source in the epilogue)
     const v4i rsw_d = rsrc_words(p.D, p.d_bytes);
 #pragma unroll
     for (int rb = 0; rb < RBW; ++rb) {
-      // (every load is issued, whatever it is for: behind a branch its register could be copied before it lands)
-      const int o = shared_src ? (rb == 0 ? 0 : -1) : out_row[rb];
-      const bool row_ok = o >= 0 && o < p.rows_c;
+      const int o = out_row[rb];
+      const bool row_ok = shared_src || (o >= 0 && o < p.rows_c);      // (one row for all: ldd is zero)
 #pragma unroll
       for (int i = 0; i < SRC_N; ++i) {
         const int ch = piece_channel(i);
@@ -692,6 +693,7 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
     }
   }
 
+  const RowGemmParams e = MIXED && KS == 2 ? late_params() : p;
   wait_vmcnt<0>();   // the loads past the end of the offset list still target this workgroup's LDS
 #pragma unroll
   for (int rb = 0; rb < RBW; ++rb)
@@ -748,17 +750,17 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
   // ---- epilogue: lane (q, m) holds, for each of its rows, channels ch0 .. ch0 + 4*NBW - 1.
   // The activation and the blend mode are lifted out of the element loops (one straight-line
   // copy per combination): tested per element they cost more issue slots than the arithmetic.
-  const __amdgpu_buffer_rsrc_t rs_c = make_rsrc(p.C, p.c_bytes);
+  const __amdgpu_buffer_rsrc_t rs_c = make_rsrc(e.C, e.c_bytes);
   if constexpr (WIDE) {
-    const __amdgpu_buffer_rsrc_t rs_d = make_rsrc(p.D, p.read_source ? p.d_bytes : 0u);
+    const __amdgpu_buffer_rsrc_t rs_d = make_rsrc(e.D, e.read_source ? e.d_bytes : 0u);
 #pragma unroll
     for (int rb = 0; rb < RBW; ++rb) {
       const int o = out_row[rb];
-      const bool row_ok = o >= 0 && o < p.rows_c && mine(rb);
+      const bool row_ok = o >= 0 && o < e.rows_c && mine(rb);
 #pragma unroll
       for (int nb = 0; nb < NBW; ++nb) {
         const int ch = ch0 + nb * 4;
-        store_wide_piece(acc[rb][nb], p, rs_c, rs_d, row_ok && ch < p.k_out, o, ch);
+        store_wide_piece(acc[rb][nb], e, rs_c, rs_d, row_ok && ch < e.k_out, o, ch);
       }
     }
     return;
@@ -769,6 +771,9 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
   // when each was rounded by integer arithmetic and converted the bias again: these were 640 of the 1150
   // instructions of a wave of a 128 x 128 tile with one or two offsets.  bf16 passes forward and backward: 128
   // channels at 1 M voxels 766.6 -> 762.9 us, stride 2, 128 -> 256 at 300 k 825.7 -> 822.2.
+  // MODE 4 only in kernels that serve layers alone (SHARED): 0.1 us of 11.9 in the mixed kernel, nothing in 128 x 128
+  // tiles, and it costs products with rows of their own, in the same kernels, 0.4 - 0.5 us (150 k of 200 k rows, 64 -> 128
+  // channels: f16 23.6 us with it, 23.2 without, bf16 24.0 and 23.5).
   auto store_rows = [&](auto act_c, auto mode_c) {
     constexpr int ACT = decltype(act_c)::value;
     constexpr int MODE = decltype(mode_c)::value;
@@ -785,20 +790,20 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
           const v4i row = __builtin_bit_cast(v4i, src_pre[0][g]);
           const uint16_t *sh = reinterpret_cast<const uint16_t *>(&row);
 #pragma unroll
-          for (int x = 0; x < 8; ++x) shared[g * 8 + x] = p.beta * E::to_float(sh[x]);
+          for (int x = 0; x < 8; ++x) shared[g * 8 + x] = e.beta * E::to_float(sh[x]);
         }
       }
 #pragma unroll
       for (int rb = 0; rb < RBW; ++rb) {
         if (!mine(rb)) continue;
         const int o = out_row[rb];
-        const bool row_ok = o >= 0 && o < p.rows_c;
+        const bool row_ok = o >= 0 && o < e.rows_c;
         v4i outs[NG];
 #pragma unroll
         for (int g = 0; g < NG; ++g) {
           const int ch = ch0 + g * 8;
-          const bool ok = row_ok && ch < p.k_out;
-          const uint32_t coff = ok ? (uint32_t)((int64_t)o * p.ldc + ch) * 2u : kOob;
+          const bool ok = row_ok && ch < e.k_out;
+          const uint32_t coff = ok ? (uint32_t)((int64_t)o * e.ldc + ch) * 2u : kOob;
           v4i src = {0, 0, 0, 0};
           if constexpr (SRC) src = __builtin_bit_cast(v4i, src_pre[rb][g]);
           const uint16_t *sh = reinterpret_cast<const uint16_t *>(&src);
@@ -806,26 +811,26 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
 #pragma unroll
           for (int x = 0; x < 8; ++x) {
             const float a = acc[rb][g * 2 + (x >> 2)][x & 3];
-            if constexpr (MODE == 4) t[x] = __builtin_fmaf(p.alpha, a, shared[g * 8 + x]);
-            else t[x] = SRC ? __builtin_fmaf(p.alpha, a, p.beta * E::to_float(sh[x])) : p.alpha * a;
-            t[x] = apply_act(t[x], ACT, p.act_alpha);
+            if constexpr (MODE == 4) t[x] = __builtin_fmaf(e.alpha, a, shared[g * 8 + x]);
+            else t[x] = SRC ? __builtin_fmaf(e.alpha, a, e.beta * E::to_float(sh[x])) : e.alpha * a;
+            t[x] = apply_act(t[x], ACT, e.act_alpha);
           }
           // (a ReLU lets no NaN through; an f16 sum that nothing follows is rounded by the fma itself)
           const v4i outv = round8<T, ACT == 1, std::is_same_v<T, F16> && ACT == 0 && (SRC || MODE == 4)>(t);
-          store_out_b128(outv, rs_c, coff, p.stream_stores != 0);
+          store_out_b128(outv, rs_c, coff, e.stream_stores != 0);
           outs[g] = outv;
         }
         if constexpr (ACT == 1) {
           if constexpr (GATE4) {
             gate_ok[rb] = row_ok;
-            gate_bits[rb] = p.gate != nullptr ? positive8(outs[0]) | positive8(outs[NG - 1]) << 8 : 0u;
-          } else if (p.gate != nullptr) {
-            store_gate(outs, p, row_ok, pos_base + (wm * RBW + rb) * 16 + m, ch0);
+            gate_bits[rb] = e.gate != nullptr ? positive8(outs[0]) | positive8(outs[NG - 1]) << 8 : 0u;
+          } else if (e.gate != nullptr) {
+            store_gate(outs, e, row_ok, pos_base + (wm * RBW + rb) * 16 + m, ch0);
           }
         }
       }
       if constexpr (GATE4) {
-        if (p.gate != nullptr && n0 + wn * 64 < p.k_out) store_gate4(gate_bits, p, gate_ok, pos_base + wm * 64, n0 + wn * 64);
+        if (e.gate != nullptr && n0 + wn * 64 < e.k_out) store_gate4(gate_bits, e, gate_ok, pos_base + wm * 64, n0 + wn * 64);
       }
     } else {
       // one-byte outputs: the lane's 4*NBW consecutive channels are 8 or 16 bytes of the row.
@@ -836,8 +841,8 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
       for (int rb = 0; rb < RBW; ++rb) {
         if (!mine(rb)) continue;
         const int o = out_row[rb];
-        const bool ok = o >= 0 && o < p.rows_c && ch0 < p.k_out;
-        const uint32_t coff = ok ? (uint32_t)((int64_t)o * p.ldc + ch0) : kOob;
+        const bool ok = o >= 0 && o < e.rows_c && ch0 < e.k_out;
+        const uint32_t coff = ok ? (uint32_t)((int64_t)o * e.ldc + ch0) : kOob;
         vNi src = {};
         if constexpr (SRC) src = __builtin_bit_cast(vNi, src_pre[rb][0]);
         const int8_t *sb = reinterpret_cast<const int8_t *>(&src);
@@ -849,33 +854,33 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
           float t;
           if constexpr (MODE >= 2) {
             t = __builtin_fmaf(scale_v[x], (float)a, bias_v[x]);
-            if constexpr (SRC) t = __builtin_fmaf(p.beta, (float)sb[x], t);
+            if constexpr (SRC) t = __builtin_fmaf(e.beta, (float)sb[x], t);
           } else if constexpr (SRC) {
-            t = __builtin_fmaf(p.alpha, (float)a, p.beta * (float)sb[x]);
+            t = __builtin_fmaf(e.alpha, (float)a, e.beta * (float)sb[x]);
           } else {
-            t = p.alpha * (float)a;
+            t = e.alpha * (float)a;
           }
-          t = apply_act(t, ACT, p.act_alpha);
+          t = apply_act(t, ACT, e.act_alpha);
           ob[x] = f32_to_s8(t);
         }
 #pragma unroll
         for (int g = 0; g < ND; ++g) outv[g] = pack4_bytes(ob[4 * g], ob[4 * g + 1], ob[4 * g + 2], ob[4 * g + 3]);
-        if constexpr (ND == 4) store_out_b128(outv, rs_c, coff, p.stream_stores != 0);
-        else store_out_b64(outv, rs_c, coff, p.stream_stores != 0);
+        if constexpr (ND == 4) store_out_b128(outv, rs_c, coff, e.stream_stores != 0);
+        else store_out_b64(outv, rs_c, coff, e.stream_stores != 0);
       }
     }
   };
   auto with_mode = [&](auto act_c) {
-    const int mode = p.read_source && shared_src ? 4 : (p.read_source ? 1 : 0) | (E::kBytes == 1 && p.int8_epilogue ? 2 : 0);
+    const int mode = e.read_source && shared_src ? 4 : (e.read_source ? 1 : 0) | (E::kBytes == 1 && e.int8_epilogue ? 2 : 0);
     switch (mode) {
     case 0: store_rows(act_c, std::integral_constant<int, 0>{}); break;
     case 1: store_rows(act_c, std::integral_constant<int, 1>{}); break;
-    case 4: if constexpr (E::kBytes == 2) store_rows(act_c, std::integral_constant<int, 4>{}); break;
+    case 4: if constexpr (SHARED) store_rows(act_c, std::integral_constant<int, 4>{}); break;
     case 2: if constexpr (E::kBytes == 1) store_rows(act_c, std::integral_constant<int, 2>{}); break;
     default: if constexpr (E::kBytes == 1) store_rows(act_c, std::integral_constant<int, 3>{}); break;
     }
   };
-  switch (p.act) {
+  switch (e.act) {
   case 1: with_mode(std::integral_constant<int, 1>{}); break;
   case 2: with_mode(std::integral_constant<int, 2>{}); break;
   case 3: with_mode(std::integral_constant<int, 3>{}); break;
@@ -986,14 +991,14 @@ __global__ __launch_bounds__(256) void rowgemm_lds_mixed_kernel(const RowGemmPar
     if constexpr (KS == 2) {
       constexpr int R32 = 32 * 4 * KS;      // 16-byte vectors of 32 rows
       const LdsRing lds = {{st0, st1, st2, nullptr}, {st0 + R32, st1 + R32, st2 + R32, nullptr}, {ix0, ix1, ix2, nullptr}, nullptr};
-      rowgemm_lds_tile<T, 2, 2, 1, 2, KS, 3, WT, false, false, 1, true>(p, 2 * tiles - 1 - rank, 0, lds);
+      rowgemm_lds_tile<T, 2, 2, 1, 2, KS, 3, WT, false, false, 1, true, 1, true>(p, 2 * tiles - 1 - rank, 0, lds);
     }
   } else if (rank - halves < singles) {
     const LdsRing lds = {{st0, st1, st2, nullptr}, {st0 + R64, st1 + R64, st2 + R64, nullptr}, {ix0, ix1, ix2, nullptr}, nullptr};
-    rowgemm_lds_tile<T, 2, 2, 2, 2, KS, 3, WT, false, false>(p, tiles - heavy - 1 - (rank - halves), 0, lds);
+    rowgemm_lds_tile<T, 2, 2, 2, 2, KS, 3, WT, false, false, 1, false, 1, true>(p, tiles - heavy - 1 - (rank - halves), 0, lds);
   } else if (rank - halves - singles < pairs) {
     const LdsRing lds = {{st0, st1, nullptr, nullptr}, {st2, st2 + R64, nullptr, nullptr}, {ix0, ix1, nullptr, nullptr}, nullptr};
-    rowgemm_lds_tile<T, 2, 2, 4, 2, KS, 2, WT, false, true>(p, pairs - 1 - (rank - halves - singles), 0, lds);
+    rowgemm_lds_tile<T, 2, 2, 4, 2, KS, 2, WT, false, true, 1, false, 1, true>(p, pairs - 1 - (rank - halves - singles), 0, lds);
   }
 }
 
