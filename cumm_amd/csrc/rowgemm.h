@@ -28,15 +28,15 @@
 //   * tiles are handed out heaviest first; each wave owns RB blocks of 16 rows and skips a block
 //     none of whose rows has a pair at offset k (its contribution would be exactly zero).
 #pragma once
-#include <cstddef>
 #include <type_traits>
 
 #include "common.h"
 
 namespace cummhip {
 
-// What every launch reads lies in the first four cache lines: with stream_stores in a fifth a product of 64 channels took
-// 13.9 us for 13.6 (150 k of 200 k rows, rowgemm_wave_kernel).
+// (The order of the fields decides which of them are fetched together, and such a group that no longer fits the scalar
+// registers is spilled whole: with the gate between the epilogue's fields and stream_stores behind them a stride-2 s8 layer of
+// 64 -> 64 channels at 300 k voxels took 40.8 us for 34.4, with 58 spills for none.)
 struct RowGemmParams {
   const void *A;   // gathered operand, rows of lda elements
   const void *W;   // weights
@@ -55,7 +55,7 @@ struct RowGemmParams {
   int32_t c_in, k_out, kv;
   uint32_t mask_filter;
   int32_t reverse_mask, exit_on_empty, gather_by_pos;
-  float alpha, beta, act_alpha;
+  float alpha, beta, act_alpha, act_beta;
   int32_t act;
   int32_t int8_epilogue;  // scale/bias requantisation instead of alpha/beta
   int32_t read_source;    // D is read (beta != 0)
@@ -70,9 +70,6 @@ struct RowGemmParams {
   // preparation left for this mask array (light_hint_slot in launch.h); a slot that names another
   // array, length or filter says nothing
   const int32_t *hint_slot;
-  // a ReLU layer that will be differentiated, or NULL: a bit for every positive result, by position:
-  // gate[((c / 64) * n_pos + pos) * 8 + c % 64 / 8], bit c % 8
-  uint8_t *gate;
   // 32-bit mask words per position (1; 2 to 4 for kernel volumes above 32: see rowgemm_lds_tile)
   int32_t mask_words;
   // words the caller's mask_out array holds (a tile number beyond it is not written)
@@ -81,6 +78,9 @@ struct RowGemmParams {
   // rows are gated by their pair-table entry alone, cumm/conv/sparse_iters.py:629-631), instead of
   // only in the offsets whose bit its own mask word has
   int32_t ungated_rows;
+  // a ReLU layer that will be differentiated, or NULL: a bit for every positive result, by position:
+  // gate[((c / 64) * n_pos + pos) * 8 + c % 64 / 8], bit c % 8
+  uint8_t *gate;
   // non-zero: the output rows are stored with the non-temporal hint (see kStreamStore)
   int32_t stream_stores;
   // non-zero (descriptors with num_stage 3): a contraction of more than 128 bytes is walked in
@@ -91,9 +91,7 @@ struct RowGemmParams {
   uint32_t even_group[4];      // with four: those of the first and third (first_group: of the first two)
   // non-zero: every row's sum in the one order that all tiles share
   int32_t one_order;
-  float act_beta;
 };
-static_assert(offsetof(RowGemmParams, stream_stores) + sizeof(int32_t) == 256, "four cache lines of arguments");
 
 // An offset no buffer contains: every operand is smaller than 2 GiB (checked on the host), and
 // adding a scalar offset below 2 GiB to it cannot wrap back into range.
