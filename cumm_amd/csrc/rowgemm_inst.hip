@@ -98,12 +98,20 @@ static void first_group_offsets(int kv, uint32_t (&words)[4], uint32_t (&even)[4
 //   several steps per offset  1024   128 -> 128 channels, 500 workgroups 21.7 / 18.2, 1000 22.3 / 19.6, 2750 23.8 / 34.5
 //   several mask words        1024   5 x 5 x 5, 64 channels, 125 workgroups 62.6 / 44.3, 469 62.1 / 45.3, 938 62.2 / 53.8,
 //                                    1875 66.1 / 69.9
-// Four groups where the device is emptier still: a quarter of the offsets each, one workgroup per CU (136 KB), all
-// sixteen waves of it on four SIMDs, so that a step takes longer; chains of many steps gain.  f16 forward, us, by
-// workgroups, two / four groups; rows of 64 bytes and one step per offset (16 channels) gain nothing:
-//   64 channels       32 9.8 / 9.5, 125 10.0 / 9.7, 250 10.2 / 10.0, 375 10.7 / 10.3
-//   128 -> 128        64 15.8 / 14.3, 250 16.3 / 14.8, 376 16.7 / 15.0, 500 17.0 / 16.9, 750 17.5 / 22.1
-//   5 x 5 x 5         32 33.8 / 29.7, 250 34.0 / 30.7, 500 37.4 / 32.9, 938 46.4 / 56.1; 32 channels: 32 25.5 / 21.8, 375 26.9 / 22.6
+// Four groups, a quarter of the offsets each, where a CU has one tile at most: 136 KB of LDS, and all sixteen waves of it
+// on four SIMDs, so that a step takes longer and only long chains gain - several steps per offset, or several mask
+// words.  One order of the offsets whatever the tile has: a tile of few of them can find most in one group.  us, two / four
+// groups, 64 x 64 tiles; "even" clouds have this many sites per volume:
+//   128 -> 64 channels, bf16   32 - 375 workgroups of a clustered cloud 14.8 - 15.8 / 13.7 - 14.0 (backward-input 15.6 - 16.5 /
+//                              14.1 - 14.3); even ones of 256: 0.05 15.3 / 14.1, 0.4 20.7 / 17.0, 0.002 13.3 / 12.3;
+//                              of 282: 0.05 15.9 / 14.1, but 0.15 17.5 / 17.9 and 0.4 22.1 / 31.7
+//   256 -> 64 channels, s8     64 workgroups 14.9 / 14.0
+//   5 x 5 x 5, 64 channels     250 workgroups of a clustered cloud 32.6 / 28.7 (backward-input 35.1 / 30.7); even ones of 256: 0.05
+//                              33.5 / 30.2, 0.4 40.7 / 34.4, 0.002 21.0 / 21.7; of 282: 0.05 37.2 / 40.2, 0.4 44.7 / 59.7
+//   one step per offset        not taken: 64 channels, 250 workgroups 9.5 / 9.4, but 500 sites, 3 offsets in the heaviest tile,
+//                              4.7 / 6.4, 8000 sites, 17 offsets, 7.3 / 7.8
+// Tiles of few offsets lose: 64 sites with 5 offsets 7.5 / 10.8 (128 channels), 500 sites with 23 of 125 offsets 10.9 / 12.7.
+constexpr unsigned kFourGroups = 256;
 template <class T, int TM, int TN, int KS, bool WT, int MW>
 static bool launch_two_groups(const RowGemmParams &p, dim3 grid, hipStream_t s, hipError_t *err) {
   if constexpr (TM == 64 && TN == 64 && KS <= 2 && !kWide && (!WT || Elem<T>::kBytes == 2)) {
@@ -112,11 +120,13 @@ static bool launch_two_groups(const RowGemmParams &p, dim3 grid, hipStream_t s, 
     if (!counted_waits_hold<rowgemm_lds_kernel<T, 2, 2, 2, 2, KS, 2, WT, false, MW, 2>>()) return false;
     RowGemmParams q = p;
     first_group_offsets(p.kv, q.first_group, q.even_group);
-    const unsigned four = MW > 1 ? 512u : (KS == 2 ? 384u : 0u);
-    if ((uint64_t)grid.x * grid.y <= four && counted_waits_hold<rowgemm_lds_kernel<T, 2, 2, 2, 2, KS, 2, WT, false, MW, 4>>()) {
-      hipLaunchKernelGGL((rowgemm_lds_kernel<T, 2, 2, 2, 2, KS, 2, WT, false, MW, 4>), grid, dim3(1024), 0, s, q);
-      *err = hipGetLastError();
-      return true;
+    if constexpr (MW > 1 || KS == 2) {
+      if ((MW > 1 || p.chunk_shift > 0) && (uint64_t)grid.x * grid.y <= kFourGroups &&
+          counted_waits_hold<rowgemm_lds_kernel<T, 2, 2, 2, 2, KS, 2, WT, false, MW, 4>>()) {
+        hipLaunchKernelGGL((rowgemm_lds_kernel<T, 2, 2, 2, 2, KS, 2, WT, false, MW, 4>), grid, dim3(1024), 0, s, q);
+        *err = hipGetLastError();
+        return true;
+      }
     }
     hipLaunchKernelGGL((rowgemm_lds_kernel<T, 2, 2, 2, 2, KS, 2, WT, false, MW, 2>), grid, dim3(512), 0, s, q);
     *err = hipGetLastError();

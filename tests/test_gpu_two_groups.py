@@ -131,6 +131,32 @@ def test_one_order_on_request(monkeypatch, op, dtype, kv, c, k):
 @pytest.mark.parametrize("op", [ConvOpType.Forward, ConvOpType.BackwardInput])
 @pytest.mark.parametrize("dtype,kv,c,k,n,which", [
     ("f16", 27, 136, 64, 64 * 384, "all"), ("f16", 27, 136, 64, 64 * 384 + 1, "all"), ("bf16", 32, 40, 72, 64 * 192, "all"),
-    ("f16", 125, 32, 64, 64 * 512, "all"), ("bf16", 125, 64, 64, 64 * 512 + 1, "even"), ("bf16", 36, 16, 8, 1, "all")])
+    ("f16", 125, 32, 64, 64 * 512, "all"), ("bf16", 125, 64, 64, 64 * 512 + 1, "even"), ("bf16", 36, 16, 8, 1, "all"),
+    ("bf16", 27, 136, 72, 64 * 128, "all"), ("f16", 27, 136, 64, 64 * 256, "even"), ("bf16", 27, 200, 64, 64 * 256 + 1, "all"),
+    ("f16", 125, 64, 64, 64 * 256, "even"), ("bf16", 125, 32, 64, 64 * 256 + 1, "all")])
 def test_sides_of_the_line_of_four_groups(op, dtype, kv, c, k, n, which):
     test_against_the_sum_over_the_table(op, dtype, kv, c, k, n, which)
+
+
+@pytest.mark.parametrize("c_in,k_out", [(144, 64), (256, 48), (128, 64)])      # (several steps per offset: four groups; one: two)
+def test_s8_of_few_tiles(c_in, k_out):
+    import numpy as np
+    from cumm_amd import pairs, synth
+    from oracle import conv_ref
+    print("case s8 of few tiles", c_in, k_out, flush=True)
+    rng, grid = np.random.default_rng(c_in), (12, 40, 36)
+    pt = pairs.subm_pairs(synth.clustered_voxels(rng, 3000, grid, 6, sigma=3.0), grid)
+    n = pt.indices_fwd.shape[1]
+    x, w = (rng.integers(-20, 21, size=s).astype(np.int8) for s in ((n, c_in), (k_out, 27, c_in)))
+    scale, bias = rng.uniform(0.001, 0.01, size=k_out).astype(np.float32), rng.normal(0, 1, size=k_out).astype(np.float32)
+    ms, order = pairs.sort_by_mask(pt.mask_fwd)
+    out0 = np.zeros((n, k_out), np.int8)
+    p = ConvParams(3, ConvOpType.Forward)
+    p.conv_algo_desp = H.find_conv_desp("s8", ConvOpType.Forward, 64, 64, int8_inference=True)
+    p.input, p.weight, p.output = H.dev(x, "s8"), H.dev(w, "s8"), H.dev(out0, "s8")
+    p.scale, p.bias = H.dev(scale, "f32"), H.dev(bias, "f32")
+    p.indices, p.mask, p.mask_argsort = H.dev(pt.indices_fwd, "i32"), H.dev(ms, "u32"), H.dev(order, "i32")
+    ConvMainUnitTest.implicit_gemm2(p)
+    ref, _ = conv_ref.implicit_gemm_fwd_ref(x, w, out0, pt.indices_fwd, ms, order, tile_m=64, dtype_in="s8", dtype_w="s8", dtype_out="s8",
+                                            scale=scale, bias=bias, int8_inference=True)
+    np.testing.assert_array_equal(H.host(p.output), ref)
