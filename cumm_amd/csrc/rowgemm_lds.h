@@ -560,14 +560,12 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
   };
   typedef int src_vec __attribute__((ext_vector_type(SRC_W)));
   src_vec src_pre[RBW][SRC_N] = {};
-  constexpr bool SHARED = E::kBytes == 2 && (MIXED || MW > 1 || WK > 1);      // (see MODE 4)
-  const bool shared_src = SHARED && p.ldd == 0;      // one row for all (a bias): converted once
   if (p.read_source && !WIDE) {   // (four-byte outputs read their source in the epilogue)
     const v4i rsw_d = rsrc_words(p.D, p.d_bytes);
 #pragma unroll
     for (int rb = 0; rb < RBW; ++rb) {
       const int o = out_row[rb];
-      const bool row_ok = shared_src || (o >= 0 && o < p.rows_c);      // (one row for all: ldd is zero)
+      const bool row_ok = o >= 0 && o < p.rows_c;
 #pragma unroll
       for (int i = 0; i < SRC_N; ++i) {
         const int ch = piece_channel(i);
@@ -765,15 +763,11 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
     }
     return;
   }
-  // MODE: 0 = alpha*acc, 1 = alpha*acc + beta*src, 2 = scale*acc + bias, 3 = ... + beta*src, 4 = as 1 with one
-  // row of src for all.
-  // An element of a ReLU layer with a bias takes 2.5 vector instructions - fma, max, half a conversion - for 9
-  // when each was rounded by integer arithmetic and converted the bias again: these were 640 of the 1150
-  // instructions of a wave of a 128 x 128 tile with one or two offsets.  bf16 passes forward and backward: 128
-  // channels at 1 M voxels 766.6 -> 762.9 us, stride 2, 128 -> 256 at 300 k 825.7 -> 822.2.
-  // MODE 4 only in kernels that serve layers alone (SHARED): 0.1 us of 11.9 in the mixed kernel, nothing in 128 x 128
-  // tiles, and it costs products with rows of their own, in the same kernels, 0.4 - 0.5 us (150 k of 200 k rows, 64 -> 128
-  // channels: f16 23.6 us with it, 23.2 without, bf16 24.0 and 23.5).
+  // MODE: 0 = alpha*acc, 1 = alpha*acc + beta*src, 2 = scale*acc + bias, 3 = ... + beta*src.
+  // (An element of a ReLU layer with a bias takes a fma, a max and half a conversion for each, for 9 vector instructions when
+  // the rounding was integer arithmetic.  A case of its own that converts a bias once for all rows took 0.1 us of 11.9 off a
+  // layer of 120 k voxels and gave products with rows of their own, which share the kernel, 0.4 - 0.5 of 23.2; the compiler
+  // also took other conversions into the fma there, so that tiles rounded differently.)
   auto store_rows = [&](auto act_c, auto mode_c) {
     constexpr int ACT = decltype(act_c)::value;
     constexpr int MODE = decltype(mode_c)::value;
@@ -783,16 +777,6 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
       constexpr bool GATE4 = ACT == 1 && NG == 2 && RBW == 4 && WK == 1;
       uint32_t gate_bits[RBW];
       bool gate_ok[RBW];
-      float shared[MODE == 4 ? CPLW : 1];
-      if constexpr (MODE == 4) {
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-          const v4i row = __builtin_bit_cast(v4i, src_pre[0][g]);
-          const uint16_t *sh = reinterpret_cast<const uint16_t *>(&row);
-#pragma unroll
-          for (int x = 0; x < 8; ++x) shared[g * 8 + x] = e.beta * E::to_float(sh[x]);
-        }
-      }
 #pragma unroll
       for (int rb = 0; rb < RBW; ++rb) {
         if (!mine(rb)) continue;
@@ -811,12 +795,11 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
 #pragma unroll
           for (int x = 0; x < 8; ++x) {
             const float a = acc[rb][g * 2 + (x >> 2)][x & 3];
-            if constexpr (MODE == 4) t[x] = __builtin_fmaf(e.alpha, a, shared[g * 8 + x]);
-            else t[x] = SRC ? __builtin_fmaf(e.alpha, a, e.beta * E::to_float(sh[x])) : e.alpha * a;
+            t[x] = SRC ? __builtin_fmaf(e.alpha, a, e.beta * E::to_float(sh[x])) : e.alpha * a;
             t[x] = apply_act(t[x], ACT, e.act_alpha);
           }
           // (a ReLU lets no NaN through; an f16 sum that nothing follows is rounded by the fma itself)
-          const v4i outv = round8<T, ACT == 1, std::is_same_v<T, F16> && ACT == 0 && (SRC || MODE == 4)>(t);
+          const v4i outv = round8<T, ACT == 1, std::is_same_v<T, F16> && ACT == 0 && SRC>(t);
           store_out_b128(outv, rs_c, coff, e.stream_stores != 0);
           outs[g] = outv;
         }
@@ -871,11 +854,10 @@ __device__ __forceinline__ void rowgemm_lds_tile(const RowGemmParams &p, const i
     }
   };
   auto with_mode = [&](auto act_c) {
-    const int mode = e.read_source && shared_src ? 4 : (e.read_source ? 1 : 0) | (E::kBytes == 1 && e.int8_epilogue ? 2 : 0);
+    const int mode = (e.read_source ? 1 : 0) | (E::kBytes == 1 && e.int8_epilogue ? 2 : 0);
     switch (mode) {
     case 0: store_rows(act_c, std::integral_constant<int, 0>{}); break;
     case 1: store_rows(act_c, std::integral_constant<int, 1>{}); break;
-    case 4: if constexpr (SHARED) store_rows(act_c, std::integral_constant<int, 4>{}); break;
     case 2: if constexpr (E::kBytes == 1) store_rows(act_c, std::integral_constant<int, 2>{}); break;
     default: if constexpr (E::kBytes == 1) store_rows(act_c, std::integral_constant<int, 3>{}); break;
     }

@@ -311,3 +311,78 @@ def test_a_gate_has_a_position_for_every_row():
     p.__dict__["_prepared"][5].N = n - 1
     with pytest.raises(ValueError):
         _again(p, sums=ctypes.addressof(gs))
+
+
+@pytest.mark.parametrize("source", ["rows", "bias"])
+@pytest.mark.parametrize("n", [60000, 9000])      # (one group of waves per tile, and two)
+def test_f16_sums_with_a_source_round_alike_in_every_tile(source, n):
+    """alpha * x + a source without an activation, x an exact sum: every result is one rounding of the exact value or
+    of its fp32 rounding - the compiler takes some conversions into the fma - and the same bits whatever the tile."""
+    print("case rounding with a source", source, n, flush=True)
+    rng, c, alpha = np.random.default_rng(1), 64, 0.33371234
+    x, src = (rng.normal(0, 1, size=(n, c)).astype(np.float16) for _ in range(2))
+    if source == "bias":
+        src = np.repeat(src[:1], n, axis=0)
+    exact = np.float64(np.float32(alpha)) * x + src.astype(np.float64)      # (24 + 11 bits, and 11)
+    one, two = exact.astype(np.float16), exact.astype(np.float32).astype(np.float16)
+    assert (one != two).sum() > 20
+    w = np.zeros((c, 1, c), np.float16)
+    w[np.arange(c), 0, np.arange(c)] = 1
+    rows, first = np.arange(n, dtype=np.int32), None
+    for tile in ((64, 64), (128, 64), (64, 128), (128, 128)):
+        p = ConvParams(3, ConvOpType.Forward)
+        p.conv_algo_desp = H.find_conv_desp("f16", ConvOpType.Forward, *tile)
+        p.input, p.output, p.weight = H.dev(x, "f16"), H.dev(src, "f16"), H.dev(w, "f16")
+        p.indices, p.mask, p.mask_argsort = H.dev(rows[None], "i32"), H.dev(np.ones(n, np.uint32), "u32"), H.dev(rows, "i32")
+        p.alpha, p.beta = alpha, 1.0
+        if source == "bias":
+            p.bias = H.dev(np.ascontiguousarray(src[0]), "f16")
+        for hint in (0, -1):      # (mixed tile shapes, and one)
+            p.light_prefix = hint
+            if source == "rows":
+                p.output = H.dev(src, "f16")
+            ConvMainUnitTest.implicit_gemm2(p)
+            got = H.host(p.output).view(np.uint16)
+            assert ((got == one.view(np.uint16)) | (got == two.view(np.uint16))).all()
+            first = got if first is None else first
+            np.testing.assert_array_equal(got, first)
+
+
+@pytest.mark.parametrize("ksize,channels,k_out,tile,hint", [
+    (5, 64, 64, (64, 64), 0), (5, 136, 40, (128, 128), 0),                       # several mask words
+    (3, 64, 520, (64, 64), 0), (3, 64, 520, (128, 128), 0), (3, 72, 264, (64, 128), -1)])      # kernels whose waits the compiler counts; chunks
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_write_empty_in_every_kernel(dtype, ksize, channels, k_out, tile, hint):
+    """As test_write_empty, in the kernels of several mask words and of long contractions."""
+    print("case write empty", dtype, ksize, channels, k_out, tile, hint, flush=True)
+    rng, grid = np.random.default_rng(12), (12, 40, 36)
+    coords = synth.clustered_voxels(rng, 1500, grid, 6, sigma=3.0)
+    zz, yy = np.meshgrid(np.arange(grid[0]), np.arange(grid[1]), indexing="ij")
+    planes = [np.stack([np.zeros(zz.size, np.int64), zz.ravel(), yy.ravel(), np.full(zz.size, grid[2] - 1)], axis=1)]
+    coords = np.unique(np.concatenate([coords] + planes).astype(np.int32), axis=0)
+    # (a padding that leaves the last plane without an output)
+    pt = pairs.sparse_conv_pairs(coords, grid, ksize=(ksize,) * 3, padding=(0, 0, 0))
+    n_in, n_out, kv = coords.shape[0], pt.indices_fwd.shape[1], ksize ** 3
+    mask = pairs.masks_from_pairs(pt.indices_bwd)
+    none = (mask == 0).all(axis=1)
+    assert none.sum() >= 300
+    w = H.to_storage(rng.normal(0, 0.05, size=(k_out, kv, channels)).astype(np.float32), dtype)
+    dout = H.to_storage(rng.normal(0, 1, size=(n_out, k_out)).astype(np.float32), dtype)
+    p = ConvParams(3, ConvOpType.BackwardInput)
+    p.conv_algo_desp = H.find_conv_desp(dtype, ConvOpType.BackwardInput, *tile, dynamic_mask=kv > 32)
+    p.input = H.dev(H.to_storage(np.full((n_in, channels), 7.0, np.float32), dtype), dtype)
+    p.weight, p.output, p.indices = H.dev(w, dtype), H.dev(dout, dtype), H.dev(pt.indices_bwd, "i32")
+    if kv > 32:
+        p.mask, p.mask_argsort = pairs.sort_by_mask_words_device(H.dev(mask, "u32"))
+        p.mask_int_count = mask.shape[1]
+    else:
+        ms, order = pairs.sort_by_mask(mask[:, 0])
+        p.mask, p.mask_argsort = H.dev(ms, "u32"), H.dev(order, "i32")
+        p.light_prefix = hint
+    ConvMainUnitTest.implicit_gemm2(p)
+    base = H.as_f32(H.host(p.input), dtype)
+    assert (base[none] == 7.0).any()
+    _again(p, write_empty=1)
+    got = H.as_f32(H.host(p.input), dtype)
+    assert (got[none] == 0.0).all()
+    np.testing.assert_array_equal(got[~none], base[~none])

@@ -111,3 +111,19 @@ def test_relu_backward_of_more_pieces_than_a_launch_has_threads():
     assert bool((x[at] == 2.0).all())
     passed = sum(int(torch.count_nonzero(x[i:i + (1 << 31)])) for i in range(0, n, 1 << 31))
     assert passed == len(on)
+
+
+def test_every_fp32_number_rounds_to_bf16_as_by_integers():
+    """All 2^32 bit patterns through the hardware's conversion: to nearest even on bit 16, NaN to 0x7FFF."""
+    lib, chunk = _capi.lib(), 1 << 27
+    for first in range(0, 1 << 32, chunk):
+        bits = torch.arange(first, first + chunk, dtype=torch.int64, device="cuda")
+        acc = (bits - ((bits >> 31) << 32)).to(torch.int32)
+        out = torch.empty(chunk, dtype=torch.int16, device="cuda")
+        _capi.check(lib.cumm_hip_finish_rows(out.data_ptr(), H.TV_DTYPE["bf16"], acc.data_ptr(), None, chunk // 64, 64, 1.0, 0.0,
+                                             onm.ACT_NONE, 0.1, torch.cuda.current_stream().cuda_stream))
+        del acc
+        nan = (bits & 0x7FFFFFFF) > 0x7F800000
+        want = torch.where(nan, 0x7FFF, ((bits + 0x7FFF + ((bits >> 16) & 1)) >> 16) & 0xFFFF)
+        wrong = (out.to(torch.int64) & 0xFFFF) != want
+        assert not bool(wrong.any()), hex(first + int(wrong.nonzero()[0]))
