@@ -27,7 +27,11 @@
 // 1.000 - 1.005 up to 324 k positions, 1.016 at 792 k of a stride-2 table, whose layer (128 -> 256 channels, forward
 // and backward) is none the slower, 851 -> 847 us: rows of one bin stay in their order, neighbours near
 // each other.  At 1 M positions of a submanifold layer it is 1.05 (at 300 k 1.001), and its passes take 791 us for
-// 767: those have two radix passes above 2^19 positions.
+// 767: those have two radix passes above 2^19 positions.  The lines, us with one pass / two, bf16, geometry and then forward
+// of a layer of 64 channels: submanifold, 400 k positions 121 / 137 and 30.4 / 30.3, 500 k 149 / 167 and 36.6 / 36.7, but 600 k
+// 185 / 204 and 47.2 / 45.9, 900 k 258 / 277 and 71.3 / 69.6 (128 channels 185 / 182); stride 2, 541 k sites 113 / 135 and 35.5 /
+// 35.4, 798 k 143 / 165 and 49.5 / 49.4, 922 k 161 / 187 and 56.1 / 56.8; the sums of more than 2^20 positions do not fit a
+// trip of the scan.
 // Chain of kernels: masks, keys and the digits' counts per block of 512 positions - sums of the counts over
 // the blocks - two passes - position.  The first pass knows every chunk's place from the sums, the second
 // looks back (ticket, flagged words); both rank by ballot and are stable.  (Instead of a kernel that clears,

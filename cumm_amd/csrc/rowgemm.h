@@ -126,8 +126,8 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *p, uint3
 
 // The arguments that an epilogue reads, fetched again where this is called: they hold no scalar registers during the steps.
 // For kernels that would spill some (two or three tile shapes in one: rowgemm_lds_mixed_kernel), and whose first argument is
-// a RowGemmParams; elsewhere the second fetch is 0.15 us.  64 -> 64 channels forward at 120 k voxels, with 31 spills and
-// without: f16 12.0 -> 11.8 us, bf16 12.8 -> 11.9.
+// a RowGemmParams; elsewhere the second fetch is 0.15 us.  64 -> 64 channels forward at 120 k voxels, with 19 - 39 spills and
+// without any: bf16 12.5 -> 11.5 us, f16 11.5 either way.
 __device__ __forceinline__ RowGemmParams late_params() {
   typedef const __attribute__((address_space(4))) RowGemmParams *kernarg;
   kernarg q = (kernarg)__builtin_amdgcn_kernarg_segment_ptr();

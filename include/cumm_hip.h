@@ -509,10 +509,15 @@ int cumm_hip_relu_backward(void *dst, const void *grad, const void *out, size_t 
 size_t cumm_hip_column_sum_workspace(int64_t rows, int channels);
 int cumm_hip_column_sum(void *dst, const void *src, int64_t rows, int channels, int dtype, void *workspace,
                         size_t workspace_bytes, void *stream);
+/* Either, as the fields of CummHipGateSums say (dtype f16 or bf16): column sums of grad (gated, out, gate and order NULL), or of
+ * the gated rows, which are written to gated on the way - with out in the order of the rows, or of the positions
+ * where order is given, with gate (and order) always in that of the positions.  The sums are fp32 partial sums per block of
+ * rows, added in block order: the same bits from run to run, and for one order of the rows, whether out or its gate
+ * says which elements pass. */
+int cumm_hip_gate_sums(const CummHipGateSums *g, int dtype, void *stream);
 /* Both at once, reading grad once: gated [rows, channels] = grad where out is positive, else 0, and sums
  * [channels] = the column sums of gated (the input gradient's gate and the bias gradient of a layer with a
  * fused ReLU); the same results as the two calls, workspace as cumm_hip_column_sum. */
-int cumm_hip_gate_sums(const CummHipGateSums *g, int dtype, void *stream);
 int cumm_hip_relu_backward_sums(void *gated, void *sums, const void *grad, const void *out, int64_t rows, int channels,
                                 int dtype, void *workspace, size_t workspace_bytes, void *stream);
 
