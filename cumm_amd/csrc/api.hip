@@ -336,8 +336,8 @@ int gate_sums_params(const CummHipGateSums &g, int dtype, ColumnSumParams *p) {
   if ((g.gated != nullptr) != (g.out != nullptr || g.gate != nullptr) || (g.out && g.gate) || !aligned16(g.gated) || !aligned16(g.out))
     return fail(CUMM_HIP_EINVAL, "gated, grad and out (or gate) must be 16-byte aligned and not empty");
   if (g.gate && !g.order) return fail(CUMM_HIP_EINVAL, "a gate lies in the order of the positions, which must not be empty");
-  if (g.order && !g.gated) return fail(CUMM_HIP_EINVAL, "an order of the rows goes with a gate");
-  if (g.order && g.rows >= ((int64_t)1 << 30) / (g.channels > 0 ? g.channels : 1)) return fail(CUMM_HIP_ERUNTIME, "your data exceed int32 range.");
+  if (g.order && !g.gated && g.rows > 0) return fail(CUMM_HIP_EINVAL, "an order of the rows goes with a gate");
+  if (g.order && g.rows > (((int64_t)1 << 30) - 1) / g.channels) return fail(CUMM_HIP_ERUNTIME, "your data exceed int32 range.");
   const size_t need = sizeof(float) * (size_t)column_sum_blocks(g.rows, g.channels) * (size_t)g.channels;
   if (!g.workspace || g.workspace_bytes < need) return fail(CUMM_HIP_ERUNTIME, "workspace at least %zu bytes.", need);
   if (reinterpret_cast<uintptr_t>(g.workspace) & 3u) return fail(CUMM_HIP_EINVAL, "workspace must be 4-byte aligned");

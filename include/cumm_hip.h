@@ -178,7 +178,8 @@ typedef struct CummHipGateSums {
   const int32_t *order;             /* that call's mask_argsort_ptr: [rows], every row once (a position that names no row of
                                        [0, rows) is passed over, and a row that none names left alone).  With gate, and
                                        with out where it is given, the rows are added up in this order: the same bits from
-                                       either; NULL: out, in the order of the rows */
+                                       either; NULL: out, in the order of the rows.  Below 2^30 elements,
+                                       which every output of a forward call is */
 } CummHipGateSums;
 
 /* What a training program wants of the same launches beyond the reference's argument block; all zero = nothing. */

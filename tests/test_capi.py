@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 from cumm_amd import _capi
+from cumm_amd import tensorview as tv
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -152,3 +153,18 @@ def test_fixed_order_backward_weight_workspace_query():
     args.deterministic = 1     # the field exists (it fills former padding)
     args.light_prefix = 128
     assert ctypes.sizeof(args) == 192
+
+
+def test_the_order_of_a_gradients_rows_is_taken_up_to_the_size_of_a_forward_pass():
+    """Rows of 72 channels below 2 GiB, the last number of them that a forward pass gives out, and the next one."""
+    lib = _capi.lib()
+    channels, last = 72, ((1 << 30) - 1) // 72
+    some = ctypes.create_string_buffer(64)
+    at = (ctypes.addressof(some) + 15) // 16 * 16      # (never read: the workspace is none)
+    for rows, want in ((last, "workspace at least"), (last + 1, "exceed int32 range")):
+        g = _capi.GateSums(gated=at, sums=at, grad=at, out=at, rows=rows, channels=channels, order=at)
+        assert lib.cumm_hip_gate_sums(ctypes.byref(g), int(tv.float16), None) != 0
+        assert want in lib.cumm_hip_last_error().decode()
+    g = _capi.GateSums(sums=at, grad=at, rows=1, channels=channels, order=at)      # an order, and no gate
+    assert lib.cumm_hip_gate_sums(ctypes.byref(g), int(tv.float16), None) != 0
+    assert "goes with a gate" in lib.cumm_hip_last_error().decode()

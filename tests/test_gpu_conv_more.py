@@ -269,6 +269,17 @@ def test_positions_that_name_no_row(dtype, rows, channels):
         np.testing.assert_array_equal(H.host(sums).view(np.uint16), H.to_storage(want[named].sum(axis=0), dtype).view(np.uint16))
 
 
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_sums_of_no_rows_in_an_order(dtype):
+    """No rows, nothing to gate, whatever order they would have: the sums are zeros."""
+    lib, channels = _capi.lib(), 72
+    sums, order, ws = H.dev(H.to_storage(np.full(channels, 3.0, np.float32), dtype), dtype), tv.zeros([64], tv.int32, 0), tv.zeros([4096], tv.uint8, 0)
+    gs = _capi.GateSums(sums=sums.byte_pointer(), rows=0, channels=channels, workspace=ws.byte_pointer(), workspace_bytes=4096, order=order.byte_pointer())
+    _capi.check(lib.cumm_hip_gate_sums(ctypes.byref(gs), int(H.TV_DTYPE[dtype]), None))
+    _capi.check(lib.cumm_hip_device_synchronize())
+    assert not H.host(sums).view(np.uint16).any()
+
+
 @pytest.mark.parametrize("cin,k_out", [(64, 64), (520, 64), (64, 136)])      # (a contraction of 520: the gate is a launch of its own)
 def test_a_gate_of_positions_that_name_no_row(cin, k_out):
     """The bits of those positions are left alone, the others are what they are."""
